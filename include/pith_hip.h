@@ -298,7 +298,7 @@ int pith_cast_f32_bf16(const float* src, void* dst, int64_t n, pith_stream_t str
  * table shared by all batch elements); weight [D] bf16 or fp32. Arithmetic is fp32 with one
  * rounding to bf16 at the end. D must be 8 * a power of two, at most 512; pointers and batch
  * strides must keep 8-byte alignment. `out` may alias x (forward) or dout (backward).
- * Backward: `out` receives dx; with a weight, dweight [D] fp32 is overwritten with the sum over
+ * Backward: `out` receives dx; with a weight, dweight [D] (fp32, or bf16 with dweight_bf16) is overwritten with the sum over
  * all rows, added in a fixed order through `workspace` (size from
  * pith_norm_rope_bwd_workspace_bytes; required then). The forward ignores dout, dweight and the
  * workspace. */
@@ -309,13 +309,15 @@ typedef struct {
   const void* sin;
   const void* dout;
   void* out;
-  float* dweight;
+  void* dweight;
   void* workspace;
   int64_t workspace_bytes;
   int64_t B, S, H, D;
   int64_t x_bs, out_bs, dout_bs, cs_bs; /* batch strides, elements */
   float eps;
   int32_t weight_dtype; /* PITH_BF16 | PITH_F32 */
+  int32_t dweight_bf16; /* != 0: dweight is written as bf16 (the fp32 sum, rounded once) */
+  int32_t reserved0;
 } pith_norm_rope_args;
 
 int pith_norm_rope_fwd(const pith_norm_rope_args* args, pith_stream_t stream);

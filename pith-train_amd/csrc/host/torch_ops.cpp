@@ -1,0 +1,655 @@
+// The operators' host path in native code: torch.library ops with their autograd formulas, and the fast form of
+// the *_into calls, both straight on top of the C ABI (include/pith_hip.h).
+//
+// What bounds a small call is the host, not the GPU: the kernels of a 256-token layer run for 50 us, while checking
+// tensors, filling argument structs and dispatching through Python took 400 us a forward + backward. Everything here
+// therefore works on at::Tensor directly, allocates from torch's caching allocator and enqueues on the current stream.
+//
+// Two layers share each operator. The native one serves the calls of ordinary layout (GPU tensors, the expected dtypes,
+// contiguous per batch element). Whenever a condition fails, or the library rejects the arguments, it has done nothing yet
+// and hands over to the operator's Python body, which accepts every layout (copying where needed) and words the errors.
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+#include <torch/library.h>
+
+#include <array>
+#include <atomic>
+#include <cstdlib>
+
+#include "pith_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ---------------------------------------------------------------------------------------------
+// Python bodies of the ops, registered once at import.
+py::object& bodies() {
+  static py::object* d = new py::object(py::dict());  // never destroyed: the interpreter may be gone by then
+  return *d;
+}
+
+template <typename R, typename... Args>
+R python_body(const char* name, const Args&... args) {
+  py::gil_scoped_acquire gil;
+  return bodies()[name](args...).template cast<R>();
+}
+
+// ---------------------------------------------------------------------------------------------
+// Layout checks, mirroring pithtrain_amd/_C.py. False: not a layout the native path takes.
+
+bool is_gpu_bf16(const Tensor& t, int64_t dim) { return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == dim; }
+bool is_gpu_f32(const Tensor& t, int64_t dim) { return t.is_cuda() && t.scalar_type() == at::kFloat && t.dim() == dim; }
+bool has_shape(const Tensor& t, at::IntArrayRef shape) { return t.sizes() == shape; }
+
+// [B, S, H, D], contiguous within a batch element (a slice along S of a contiguous tensor qualifies)
+bool bshd(const Tensor& t, int64_t* batch_stride) {
+  const auto n = t.sizes();
+  const auto st = t.strides();
+  if (!((n[3] == 1 || st[3] == 1) && (n[2] == 1 || st[2] == n[3]) && (n[1] == 1 || st[1] == n[2] * n[3]))) return false;
+  *batch_stride = n[0] > 1 ? st[0] : n[1] * n[2] * n[3];
+  return true;
+}
+
+// The same for what may be a range of consecutive heads of a wider tensor; heads per row of that tensor come back too.
+bool bshd_heads(const Tensor& t, int64_t* batch_stride, int64_t* row_heads) {
+  const auto n = t.sizes();
+  const auto st = t.strides();
+  const int64_t rh = n[1] == 1 ? n[2] : (n[3] > 0 ? st[1] / n[3] : 0);
+  if (!((n[3] == 1 || st[3] == 1) && (n[2] == 1 || st[2] == n[3]) && (n[1] == 1 || (st[1] % n[3] == 0 && rh >= n[2])))) return false;
+  *batch_stride = n[0] > 1 ? st[0] : n[1] * rh * n[3];
+  *row_heads = rh;
+  return true;
+}
+
+// [B, H, S] with unit stride along S
+bool bhs(const Tensor& t, int64_t* batch_stride, int64_t* head_stride) {
+  const auto n = t.sizes();
+  const auto st = t.strides();
+  if (n[2] != 1 && st[2] != 1) return false;
+  *batch_stride = n[0] > 1 ? st[0] : n[1] * std::max(st[1], n[2]);
+  *head_stride = n[1] > 1 ? st[1] : n[2];
+  return true;
+}
+
+bool dtype_code(const Tensor& t, int32_t* code) {
+  if (t.scalar_type() == at::kBFloat16) *code = PITH_BF16;
+  else if (t.scalar_type() == at::kFloat) *code = PITH_F32;
+  else return false;
+  return true;
+}
+
+bool head_dims_ok(int64_t dq, int64_t dv) { return (dq == 64 && dv == 64) || (dq == 128 && dv == 128) || (dq == 192 && dv == 128); }
+
+pith_stream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+Tensor empty_like_shape(const Tensor& like, at::IntArrayRef shape, at::ScalarType dtype) {
+  return at::empty(shape, like.options().dtype(dtype));
+}
+
+// ---------------------------------------------------------------------------------------------
+// Chunk attention
+
+// The shared rotary key part ([b, s, 64] or [b, s, 1, 64], unit stride along the features).
+bool k_pe_fields(const Tensor& k, const Tensor& k_pe_in, const void** ptr, int64_t* bs, int64_t* rs) {
+  Tensor pe = k_pe_in;
+  if (pe.dim() == 4) {
+    if (pe.size(2) != 1) return false;
+    pe = pe.select(2, 0);
+  }
+  const int64_t b = k.size(0), s = k.size(1);
+  if (!is_gpu_bf16(pe, 3) || pe.device() != k.device() || !has_shape(pe, {b, s, 64}) || pe.stride(2) != 1) return false;
+  *rs = s > 1 ? pe.stride(1) : 64;
+  *bs = b > 1 ? pe.stride(0) : s * *rs;
+  *ptr = pe.data_ptr();
+  return true;
+}
+
+// dtypes, shapes and devices of q, k, v (and k_pe) as the operators require them
+bool qkv_ok(const Tensor& q, const Tensor& k, const Tensor& v, bool causal, bool two_part) {
+  if (!is_gpu_bf16(q, 4) || !is_gpu_bf16(k, 4) || !is_gpu_bf16(v, 4) || k.device() != q.device() || v.device() != q.device()) return false;
+  const int64_t dq = q.size(3), dv = v.size(3);
+  if (!head_dims_ok(dq, dv) || k.size(3) != (two_part ? 128 : dq) || (two_part && (dq != 192 || q.size(2) != k.size(2)))) return false;
+  if (k.size(0) != q.size(0) || v.size(0) != q.size(0) || k.size(1) != v.size(1) || k.size(2) != v.size(2)) return false;
+  return k.size(2) > 0 && q.size(2) % k.size(2) == 0 && (!causal || q.size(1) == k.size(1));
+}
+
+using Rows = std::optional<std::pair<int64_t, int64_t>>;
+
+// o, lse <- attention(q, k, v), see attn_fwd_into in operators/mla/hip.py. False: nothing was launched.
+bool attn_fwd_into(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& o, const Tensor& lse, double scale, bool causal,
+                   const OptTensor& k_pe, const OptTensor& prev_o, const OptTensor& acc_o, const Rows& o_rows, const Rows& acc_o_rows) {
+  if (!qkv_ok(q, k, v, causal, k_pe.has_value())) return false;
+  const int64_t b = q.size(0), sq = q.size(1), hq = q.size(2), dv = v.size(3);
+  const std::array<int64_t, 4> o_shape = {b, sq, hq, dv};
+  pith_attn_fwd_args a = {};
+  if (!is_gpu_f32(lse, 3) || lse.device() != q.device() || !has_shape(lse, {b, hq, sq}) || !bhs(lse, &a.lse_bs, &a.lse_hs)) return false;
+  if (!bshd(q, &a.q_bs) || !bshd(k, &a.k_bs) || !bshd(v, &a.v_bs)) return false;
+  if (o) {
+    if (!is_gpu_bf16(*o, 4) || o->device() != q.device() || !has_shape(*o, o_shape) || !bshd(*o, &a.o_bs)) return false;
+    a.o = o->data_ptr();
+  }
+  if (prev_o) {
+    if (!prev_o->is_cuda() || prev_o->device() != q.device() || prev_o->dim() != 4 || !has_shape(*prev_o, o_shape) || (!o && !acc_o) ||
+        !bshd(*prev_o, &a.prev_o_bs) || !dtype_code(*prev_o, &a.prev_o_dtype))
+      return false;
+    a.prev_o = prev_o->data_ptr();
+    if (acc_o) {
+      if (!is_gpu_f32(*acc_o, 4) || acc_o->device() != q.device() || !has_shape(*acc_o, o_shape) || !bshd(*acc_o, &a.acc_o_bs)) return false;
+      a.acc_o = acc_o->data_ptr<float>();
+    }
+    if (o_rows) a.o_rows[0] = o_rows->first, a.o_rows[1] = o_rows->second;
+    if (acc_o_rows) a.acc_o_rows[0] = acc_o_rows->first, a.acc_o_rows[1] = acc_o_rows->second;
+  } else if (!o || acc_o) {
+    return false;
+  }
+  if (k_pe && !k_pe_fields(k, *k_pe, &a.k_pe, &a.k_pe_bs, &a.k_pe_rs)) return false;
+  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.lse = lse.data_ptr<float>();
+  a.B = b; a.Sq = sq; a.Skv = k.size(1); a.Hq = hq; a.Hkv = k.size(2); a.Dqk = q.size(3); a.Dv = dv;
+  a.scale = (float)scale; a.causal = causal;
+  return pith_attn_fwd(&a, stream_of(q)) == PITH_OK;
+}
+
+bool attn_bwd_delta_into(const Tensor& out, const Tensor& dout, const Tensor& delta) {
+  if (!is_gpu_bf16(out, 4) || !is_gpu_bf16(dout, 4) || dout.device() != out.device() || dout.sizes() != out.sizes()) return false;
+  pith_attn_delta_args a = {};
+  a.B = out.size(0); a.S = out.size(1); a.H = out.size(2); a.D = out.size(3);
+  if (!is_gpu_f32(delta, 3) || delta.device() != out.device() || !has_shape(delta, {a.B, a.H, a.S}) || !bhs(delta, &a.delta_bs, &a.delta_hs) ||
+      !bshd(out, &a.o_bs) || !bshd(dout, &a.dout_bs))
+    return false;
+  a.o = out.data_ptr(); a.dout = dout.data_ptr(); a.delta = delta.data_ptr<float>();
+  return pith_attn_bwd_delta(&a, stream_of(out)) == PITH_OK;
+}
+
+// What both backward calls of a chunk pair share.
+bool bwd_args(pith_attn_bwd_args& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta,
+              double scale, bool causal, const OptTensor& k_pe, const OptTensor& ds) {
+  if (!qkv_ok(q, k, v, causal, k_pe.has_value())) return false;
+  const int64_t b = q.size(0), sq = q.size(1), hq = q.size(2), hkv = k.size(2), dv = v.size(3);
+  if (!is_gpu_bf16(dout, 4) || dout.device() != q.device() || !has_shape(dout, {b, sq, hq, dv})) return false;
+  int64_t d_bs, d_hs, do_rh, v_rh;
+  for (const Tensor* t : {&lse, &delta})
+    if (!is_gpu_f32(*t, 3) || t->device() != q.device() || !has_shape(*t, {b, hq, sq})) return false;
+  if (!bhs(lse, &a.lse_bs, &a.lse_hs) || !bhs(delta, &d_bs, &d_hs) || d_bs != a.lse_bs || d_hs != a.lse_hs) return false;
+  if (!bshd_heads(q, &a.q_bs, &a.q_row_heads) || !bshd_heads(dout, &a.dout_bs, &do_rh) || !bshd_heads(k, &a.k_bs, &a.kv_row_heads) ||
+      !bshd_heads(v, &a.v_bs, &v_rh) || do_rh != a.q_row_heads || v_rh != a.kv_row_heads)
+    return false;
+  if (k_pe && (a.q_row_heads != hq || a.kv_row_heads != hkv || !k_pe_fields(k, *k_pe, &a.k_pe, &a.k_pe_bs, &a.k_pe_rs))) return false;
+  if (ds) {
+    if (!ds->is_cuda() || ds->device() != q.device() || ds->scalar_type() != at::kByte || !ds->is_contiguous() || (uintptr_t)ds->data_ptr() % 256) return false;
+    a.ds = ds->data_ptr();
+    a.ds_bytes = ds->numel();
+  }
+  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.dout = dout.data_ptr();
+  a.lse = lse.data_ptr<float>(); a.delta = delta.data_ptr<float>();
+  a.B = b; a.Sq = sq; a.Skv = k.size(1); a.Hq = hq; a.Hkv = hkv; a.Dqk = q.size(3); a.Dv = dv;
+  a.scale = (float)scale; a.causal = causal;
+  a.dq_dtype = a.dkv_dtype = PITH_BF16;
+  return true;
+}
+
+bool attn_bwd_dkdv_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dk,
+                        const Tensor& dv, double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& dk_pe,
+                        const OptTensor& ds, int64_t zero_tail) {
+  pith_attn_bwd_args a = {};
+  if (!bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds)) return false;
+  if (!dk.is_cuda() || dk.device() != q.device() || dv.device() != q.device() || dk.sizes() != k.sizes() || dv.sizes() != v.sizes() ||
+      dk.scalar_type() != dv.scalar_type() || !dtype_code(dk, &a.dkv_dtype))
+    return false;
+  if (k_pe) {
+    const int64_t b = k.size(0), s = k.size(1);
+    if (!dk_pe || !dk_pe->is_cuda() || dk_pe->device() != q.device() || !has_shape(*dk_pe, {b, s, 64}) || dk_pe->scalar_type() != dk.scalar_type() ||
+        dk_pe->stride(2) != 1 || (s > 1 && dk_pe->stride(1) != 64))
+      return false;
+    a.dk_pe = dk_pe->data_ptr();
+    a.dk_pe_bs = b > 1 ? dk_pe->stride(0) : s * 64;
+  }
+  int64_t dk_rh, dv_rh;
+  if (!bshd_heads(dk, &a.dk_bs, &dk_rh) || !bshd_heads(dv, &a.dv_bs, &dv_rh) || dk_rh != a.kv_row_heads || dv_rh != a.kv_row_heads) return false;
+  a.dk = dk.data_ptr(); a.dv = dv.data_ptr();
+  a.accumulate_dkv = accumulate;
+  a.dkv_zero_tail = zero_tail;
+  Tensor workspace;  // stream order keeps the block alive until the kernels that use it have run
+  const int64_t need = pith_attn_bwd_dkdv_workspace_bytes(&a);
+  if (need > 0) {
+    workspace = empty_like_shape(q, {need}, at::kByte);
+    a.workspace = workspace.data_ptr();
+    a.workspace_bytes = need;
+  }
+  return pith_attn_bwd_dkdv(&a, stream_of(q)) == PITH_OK;
+}
+
+bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
+                      double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& ds, const OptTensor& dq_final,
+                      const Rows& dq_final_rows) {
+  pith_attn_bwd_args a = {};
+  if (!bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds)) return false;
+  int64_t rh;
+  if (!dq.is_cuda() || dq.device() != q.device() || dq.sizes() != q.sizes() || !dtype_code(dq, &a.dq_dtype) || !bshd_heads(dq, &a.dq_bs, &rh) ||
+      rh != a.q_row_heads)
+    return false;
+  a.dq = dq.data_ptr();
+  a.accumulate_dq = accumulate;
+  if (dq_final) {
+    if (!is_gpu_bf16(*dq_final, 4) || dq_final->device() != q.device() || dq_final->sizes() != q.sizes() ||
+        !bshd_heads(*dq_final, &a.dq_final_bs, &rh) || rh != a.q_row_heads)
+      return false;
+    a.dq_final = dq_final->data_ptr();
+    if (dq_final_rows) a.dq_final_rows[0] = dq_final_rows->first, a.dq_final_rows[1] = dq_final_rows->second;
+  }
+  return pith_attn_bwd_dq(&a, stream_of(q)) == PITH_OK;
+}
+
+using Two = std::tuple<Tensor, Tensor>;
+using Three = std::tuple<Tensor, Tensor, Tensor>;
+using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+
+Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+  if (q.is_cuda() && q.dim() == 4 && v.dim() == 4) {
+    Tensor o = at::empty({q.size(0), q.size(1), q.size(2), v.size(3)}, q.options().dtype(at::kBFloat16));
+    Tensor lse = at::empty({q.size(0), q.size(2), q.size(1)}, q.options().dtype(at::kFloat));
+    if (attn_fwd_into(q, k, v, o, lse, scale, causal, {}, {}, {}, {}, {})) return {o, lse};
+  }
+  return python_body<Two>("attn_fwd", q, k, v, scale, causal);
+}
+
+// Compute units of a device, looked up once.
+int64_t compute_units(int device) {
+  static std::array<std::atomic<int>, 64> cached = {};
+  if (device < 0 || device >= 64) return 0;
+  int n = cached[device].load(std::memory_order_relaxed);
+  if (n == 0) {
+    pith_device_info_t info;
+    if (pith_device_info(device, &info) != PITH_OK) return 0;
+    cached[device].store(n = info.compute_units, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
+  // Calls large enough for the dS hand-over (its dQ kernel owns 512 query rows per workgroup) belong to the Python body,
+  // which owns the policy for the hand-over buffer: their kernels outlast its host work many times over.
+  const bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4 &&
+                     !(q.size(3) == 128 && (q.size(1) + 511) / 512 * q.size(2) * q.size(0) >= compute_units(q.device().index()));
+  if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
+    Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    if (attn_bwd_delta_into(o, dout, delta) && attn_bwd_dkdv_into(q, k, v, dout, lse, delta, dk, dv, scale, causal, false, {}, {}, {}, 0) &&
+        attn_bwd_dq_into(q, k, v, dout, lse, delta, dq, scale, causal, false, {}, {}, {}, {}))
+      return {dq, dk, dv};
+  }
+  return python_body<Three>("attn_bwd", q, k, v, o, lse, dout, scale, causal);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Combine
+
+bool combine_into(const Tensor& out1, const Tensor& lse1, const Tensor& out2, const Tensor& lse2, const Tensor& out, const Tensor& lse_out, int64_t base) {
+  pith_combine_args a = {};
+  if (!out1.is_cuda() || out1.dim() != 4) return false;
+  for (const Tensor* t : {&out2, &out})
+    if (t->device() != out1.device() || t->sizes() != out1.sizes()) return false;
+  a.B = out1.size(0); a.S = out1.size(1); a.H = out1.size(2); a.D = out1.size(3);
+  for (const Tensor* t : {&lse1, &lse2, &lse_out})
+    if (!is_gpu_f32(*t, 3) || t->device() != out1.device() || !has_shape(*t, {a.B, a.H, a.S})) return false;
+  if (!bhs(lse1, &a.lse1_bs, &a.lse1_hs) || !bhs(lse2, &a.lse2_bs, &a.lse2_hs) || !bhs(lse_out, &a.lse_out_bs, &a.lse_out_hs)) return false;
+  if (!dtype_code(out1, &a.dtype1) || !dtype_code(out2, &a.dtype2) || !dtype_code(out, &a.dtype_out)) return false;
+  if (!bshd(out1, &a.out1_bs) || !bshd(out2, &a.out2_bs) || !bshd(out, &a.out_bs)) return false;
+  a.out1 = out1.data_ptr(); a.out2 = out2.data_ptr(); a.out = out.data_ptr();
+  a.lse1 = lse1.data_ptr<float>(); a.lse2 = lse2.data_ptr<float>(); a.lse_out = lse_out.data_ptr<float>();
+  a.base = (int32_t)base;
+  return pith_combine(&a, stream_of(out1)) == PITH_OK;
+}
+
+// The reference's calling convention: fresh fp32 outputs. None when the Python body has to take the call.
+std::optional<Two> combine_new(const Tensor& out1, const Tensor& lse1, const Tensor& out2, const Tensor& lse2, int64_t base) {
+  if (!out1.is_cuda() || !lse1.is_cuda() || out1.dim() != 4 || lse1.dim() != 3 || (!lse1.is_contiguous() && lse1.stride(-1) != 1)) return std::nullopt;
+  Tensor out = empty_like_shape(out1, out1.sizes(), at::kFloat), lse = empty_like_shape(lse1, lse1.sizes(), at::kFloat);
+  if (!combine_into(out1, lse1, out2, lse2, out, lse, base)) return std::nullopt;
+  return Two{out, lse};
+}
+
+bool cast_f32_bf16_into(const Tensor& src, const Tensor& dst) {
+  if (!src.is_cuda() || dst.device() != src.device() || src.scalar_type() != at::kFloat || dst.scalar_type() != at::kBFloat16 ||
+      src.numel() != dst.numel() || !src.is_contiguous() || !dst.is_contiguous())
+    return false;
+  return pith_cast_f32_bf16(src.data_ptr<float>(), dst.data_ptr(), src.numel(), stream_of(src)) == PITH_OK;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Per-head RMSNorm + rotary embedding
+
+// Fields that forward and backward share; x and out contiguous.
+bool norm_rope_args(pith_norm_rope_args& a, const Tensor& x, const OptTensor& weight, const Tensor& cos, const Tensor& sin, const Tensor& out, double eps) {
+  if (!is_gpu_bf16(x, 4) || !x.is_contiguous()) return false;
+  a.B = x.size(0); a.S = x.size(1); a.H = x.size(2); a.D = x.size(3);
+  if (!cos.is_cuda() || !sin.is_cuda() || cos.device() != x.device() || sin.device() != x.device() || cos.scalar_type() != at::kBFloat16 ||
+      sin.scalar_type() != at::kBFloat16 || cos.sizes() != sin.sizes() || !cos.is_contiguous() || !sin.is_contiguous())
+    return false;
+  if (cos.dim() == 2) {
+    if (!has_shape(cos, {a.S, a.D})) return false;
+    a.cs_bs = 0;
+  } else {
+    if (cos.dim() != 3 || (cos.size(0) != 1 && cos.size(0) != a.B) || cos.size(1) != a.S || cos.size(2) != a.D) return false;
+    a.cs_bs = cos.size(0) > 1 ? a.S * a.D : 0;
+  }
+  if (weight) {
+    if (!weight->is_cuda() || weight->device() != x.device() || !has_shape(*weight, {a.D}) || !weight->is_contiguous() ||
+        !dtype_code(*weight, &a.weight_dtype))
+      return false;
+    a.weight = weight->data_ptr();
+  }
+  a.x = x.data_ptr(); a.cos = cos.data_ptr(); a.sin = sin.data_ptr(); a.out = out.data_ptr();
+  a.x_bs = a.out_bs = a.S * a.H * a.D;
+  a.eps = (float)eps;
+  return true;
+}
+
+// dout and, with a weight, dweight (in the weight's dtype: the kernel that adds the partial sums rounds it) and the scratch.
+bool norm_rope_bwd_args(pith_norm_rope_args& a, const Tensor& x, const OptTensor& weight, const Tensor& dout, const Tensor& dweight, Tensor& workspace) {
+  if (!is_gpu_bf16(dout, 4) || dout.device() != x.device() || dout.sizes() != x.sizes() || !dout.is_contiguous()) return false;
+  a.dout = dout.data_ptr();
+  a.dout_bs = a.S * a.H * a.D;
+  if (!weight) return true;
+  a.dweight = dweight.data_ptr();
+  a.dweight_bf16 = weight->scalar_type() == at::kBFloat16;
+  a.workspace_bytes = pith_norm_rope_bwd_workspace_bytes(&a);
+  workspace = empty_like_shape(x, {a.workspace_bytes}, at::kByte);
+  a.workspace = workspace.data_ptr();
+  return true;
+}
+
+Tensor dweight_for(const Tensor& x, const OptTensor& weight) {
+  if (weight) return at::empty_like(*weight);
+  return empty_like_shape(x, {0}, at::kFloat);  // placeholder: an op cannot return None
+}
+
+Tensor norm_rope_fwd(const Tensor& x, const OptTensor& weight, const Tensor& cos, const Tensor& sin, double eps) {
+  if (x.is_cuda()) {
+    Tensor out = at::empty_like(x, at::MemoryFormat::Contiguous);
+    pith_norm_rope_args a = {};
+    if (norm_rope_args(a, x, weight, cos, sin, out, eps) && pith_norm_rope_fwd(&a, stream_of(x)) == PITH_OK) return out;
+  }
+  return python_body<Tensor>("norm_rope_fwd", x, weight, cos, sin, eps);
+}
+
+Two norm_rope_bwd(const Tensor& x, const OptTensor& weight, const Tensor& cos, const Tensor& sin, const Tensor& dout, double eps) {
+  if (x.is_cuda()) {
+    Tensor dx = at::empty_like(x, at::MemoryFormat::Contiguous), dw = dweight_for(x, weight), ws;
+    pith_norm_rope_args a = {};
+    if (norm_rope_args(a, x, weight, cos, sin, dx, eps) && norm_rope_bwd_args(a, x, weight, dout, dw, ws) &&
+        pith_norm_rope_bwd(&a, stream_of(x)) == PITH_OK)
+      return {dx, dw};
+  }
+  return python_body<Two>("norm_rope_bwd", x, weight, cos, sin, dout, eps);
+}
+
+Two qk_norm_rope_fwd(const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos, const Tensor& sin, double eps) {
+  if (q.is_cuda() && k.is_cuda()) {
+    Tensor qo = at::empty_like(q, at::MemoryFormat::Contiguous), ko = at::empty_like(k, at::MemoryFormat::Contiguous);
+    pith_norm_rope_args a = {}, b = {};
+    if (k.device() == q.device() && norm_rope_args(a, q, qw, cos, sin, qo, eps) && norm_rope_args(b, k, kw, cos, sin, ko, eps) &&
+        pith_norm_rope_fwd_pair(&a, &b, stream_of(q)) == PITH_OK)
+      return {qo, ko};
+  }
+  return python_body<Two>("qk_norm_rope_fwd", q, k, qw, kw, cos, sin, eps);
+}
+
+Four qk_norm_rope_bwd(const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos, const Tensor& sin, const Tensor& dqo,
+                      const Tensor& dko, double eps) {
+  if (q.is_cuda() && k.is_cuda()) {
+    Tensor dq = at::empty_like(q, at::MemoryFormat::Contiguous), dk = at::empty_like(k, at::MemoryFormat::Contiguous);
+    Tensor dwq = dweight_for(q, qw), dwk = dweight_for(k, kw), ws_q, ws_k;
+    pith_norm_rope_args a = {}, b = {};
+    if (k.device() == q.device() && norm_rope_args(a, q, qw, cos, sin, dq, eps) && norm_rope_args(b, k, kw, cos, sin, dk, eps) &&
+        norm_rope_bwd_args(a, q, qw, dqo, dwq, ws_q) && norm_rope_bwd_args(b, k, kw, dko, dwk, ws_k) &&
+        pith_norm_rope_bwd_pair(&a, &b, stream_of(q)) == PITH_OK)
+      return {dq, dk, dwq, dwk};
+  }
+  return python_body<Four>("qk_norm_rope_bwd", q, k, qw, kw, cos, sin, dqo, dko, eps);
+}
+
+// ---------------------------------------------------------------------------------------------
+// MLA rotary embedding + query / key / value assembly
+
+bool assemble_tables(pith_mla_assemble_args& a, const Tensor& ref, const Tensor& cos, const Tensor& sin, const OptTensor& pos) {
+  for (const Tensor* t : {&cos, &sin})
+    if (!is_gpu_bf16(*t, 2) || t->device() != ref.device() || !t->is_contiguous() || t->size(1) != a.Dr) return false;
+  if (cos.sizes() != sin.sizes()) return false;
+  a.P = cos.size(0);
+  a.cos = cos.data_ptr(); a.sin = sin.data_ptr();
+  if (!pos) return a.P >= a.S;
+  if (std::getenv("PITHTRAIN_AMD_CHECK_POSITIONS") != nullptr) return false;  // the Python body reads the positions back
+  if (!pos->is_cuda() || pos->device() != ref.device() || pos->scalar_type() != at::kLong || pos->dim() != 2 ||
+      (pos->size(0) != 1 && pos->size(0) != a.B) || pos->size(1) != a.S || (a.S > 1 && pos->stride(1) != 1))
+    return false;
+  a.position_ids = pos->data_ptr<int64_t>();
+  a.pos_bs = pos->size(0) > 1 ? pos->stride(0) : 0;
+  return true;
+}
+
+Three mla_assemble_fwd(const Tensor& q, const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin, const OptTensor& pos) {
+  const bool shapes = is_gpu_bf16(q, 4) && is_gpu_bf16(kv, 4) && (is_gpu_bf16(k_pe, 3) || (is_gpu_bf16(k_pe, 4) && k_pe.size(2) == 1)) &&
+                      kv.device() == q.device() && k_pe.device() == q.device();
+  if (shapes && q.is_contiguous() && kv.is_contiguous() && k_pe.stride(-1) == 1) {
+    pith_mla_assemble_args a = {};
+    a.B = q.size(0); a.S = q.size(1); a.H = q.size(2); a.Dr = k_pe.size(-1);
+    a.Dn = q.size(3) - a.Dr;
+    a.Dv = kv.size(3) - a.Dn;
+    if (a.Dn > 0 && a.Dv > 0 && kv.size(0) == a.B && kv.size(1) == a.S && kv.size(2) == a.H && k_pe.size(0) == a.B && k_pe.size(1) == a.S &&
+        assemble_tables(a, q, cos, sin, pos)) {
+      Tensor qo = at::empty_like(q), ko = at::empty_like(q), vo = at::empty({a.B, a.S, a.H, a.Dv}, q.options());
+      a.q = q.data_ptr(); a.kv = kv.data_ptr(); a.k_pe = k_pe.data_ptr();
+      a.q_out = qo.data_ptr(); a.k_out = ko.data_ptr(); a.v_out = vo.data_ptr();
+      a.q_bs = a.S * a.H * (a.Dn + a.Dr);
+      a.kv_bs = a.S * a.H * (a.Dn + a.Dv);
+      a.k_pe_rs = a.S > 1 ? k_pe.stride(1) : a.Dr;
+      a.k_pe_bs = a.B > 1 ? k_pe.stride(0) : a.S * k_pe.stride(1);
+      if (pith_mla_assemble_fwd(&a, stream_of(q)) == PITH_OK) return {qo, ko, vo};
+    }
+  }
+  return python_body<Three>("mla_assemble_fwd", q, kv, k_pe, cos, sin, pos);
+}
+
+Three mla_assemble_bwd(const Tensor& dqo, const Tensor& dko, const Tensor& dvo, const Tensor& cos, const Tensor& sin, const OptTensor& pos, int64_t k_pe_heads) {
+  const bool shapes = is_gpu_bf16(dqo, 4) && is_gpu_bf16(dko, 4) && is_gpu_bf16(dvo, 4) && dko.device() == dqo.device() && dvo.device() == dqo.device() &&
+                      cos.dim() == 2;
+  if (shapes && dqo.is_contiguous() && dko.is_contiguous() && dvo.is_contiguous() && dko.sizes() == dqo.sizes()) {
+    pith_mla_assemble_args a = {};
+    a.B = dqo.size(0); a.S = dqo.size(1); a.H = dqo.size(2); a.Dr = cos.size(1); a.Dv = dvo.size(3);
+    a.Dn = dqo.size(3) - a.Dr;
+    if (a.Dn > 0 && dvo.size(0) == a.B && dvo.size(1) == a.S && dvo.size(2) == a.H && assemble_tables(a, dqo, cos, sin, pos)) {
+      Tensor dq = at::empty_like(dqo), dkv = at::empty({a.B, a.S, a.H, a.Dn + a.Dv}, dqo.options());
+      Tensor dpe = k_pe_heads ? at::empty({a.B, a.S, 1, a.Dr}, dqo.options()) : at::empty({a.B, a.S, a.Dr}, dqo.options());
+      a.dq_out = dqo.data_ptr(); a.dk_out = dko.data_ptr(); a.dv_out = dvo.data_ptr();
+      a.q_out = dq.data_ptr(); a.k_out = dkv.data_ptr(); a.v_out = dpe.data_ptr();
+      if (pith_mla_assemble_bwd(&a, stream_of(dqo)) == PITH_OK) return {dq, dkv, dpe};
+    }
+  }
+  return python_body<Three>("mla_assemble_bwd", dqo, dko, dvo, cos, sin, pos, k_pe_heads);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Autograd. Each formula calls the ops through the dispatcher, below autograd, so that fake tensors, functionalisation and
+// torch.compile see ordinary ops.
+
+template <typename Sig>
+auto op_handle(const char* name) { return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>(); }
+
+bool any_requires_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
+Tensor or_undefined(const OptTensor& t) { return t ? *t : Tensor(); }
+OptTensor or_none(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
+
+Two call_attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+  static const auto op = op_handle<decltype(attn_fwd)>("pithtrain_amd::attn_fwd");
+  return op.call(q, k, v, scale, causal);
+}
+struct AttnFunction : torch::autograd::Function<AttnFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    auto [o, lse] = call_attn_fwd(q, k, v, scale, causal);
+    ctx->save_for_backward({q, k, v, o, lse});
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["causal"] = causal;
+    ctx->mark_non_differentiable({lse});
+    ctx->set_materialize_grads(false);
+    return {o, lse};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static const auto op = op_handle<decltype(attn_bwd)>("pithtrain_amd::attn_bwd");
+    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    const auto s = ctx->get_saved_variables();
+    auto [dq, dk, dv] = op.call(s[0], s[1], s[2], s[3], s[4], grads[0], ctx->saved_data["scale"].toDouble(), ctx->saved_data["causal"].toBool());
+    return {dq, dk, dv, Tensor(), Tensor()};
+  }
+};
+Two attn_fwd_autograd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool causal) {
+  if (!any_requires_grad({&q, &k, &v})) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return call_attn_fwd(q, k, v, scale, causal);
+  }
+  auto r = AttnFunction::apply(q, k, v, scale, causal);
+  return {r[0], r[1]};
+}
+
+Tensor call_norm_rope_fwd(const Tensor& x, const OptTensor& w, const Tensor& cos, const Tensor& sin, double eps) {
+  static const auto op = op_handle<decltype(norm_rope_fwd)>("pithtrain_amd::norm_rope_fwd");
+  return op.call(x, w, cos, sin, eps);
+}
+struct NormRopeFunction : torch::autograd::Function<NormRopeFunction> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const OptTensor& w, const Tensor& cos, const Tensor& sin, double eps) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    ctx->save_for_backward({x, or_undefined(w), cos, sin});
+    ctx->saved_data["eps"] = eps;
+    return call_norm_rope_fwd(x, w, cos, sin, eps);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static const auto op = op_handle<decltype(norm_rope_bwd)>("pithtrain_amd::norm_rope_bwd");
+    const auto s = ctx->get_saved_variables();
+    auto [dx, dw] = op.call(s[0], or_none(s[1]), s[2], s[3], grads[0], ctx->saved_data["eps"].toDouble());
+    return {dx, s[1].defined() ? dw : Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+Tensor norm_rope_fwd_autograd(const Tensor& x, const OptTensor& w, const Tensor& cos, const Tensor& sin, double eps) {
+  const Tensor ww = or_undefined(w);
+  if (any_requires_grad({&x, &ww})) return NormRopeFunction::apply(x, w, cos, sin, eps);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  return call_norm_rope_fwd(x, w, cos, sin, eps);
+}
+
+Two call_qk_norm_rope_fwd(const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos, const Tensor& sin, double eps) {
+  static const auto op = op_handle<decltype(qk_norm_rope_fwd)>("pithtrain_amd::qk_norm_rope_fwd");
+  return op.call(q, k, qw, kw, cos, sin, eps);
+}
+struct QkNormRopeFunction : torch::autograd::Function<QkNormRopeFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos,
+                               const Tensor& sin, double eps) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    ctx->save_for_backward({q, k, or_undefined(qw), or_undefined(kw), cos, sin});
+    ctx->saved_data["eps"] = eps;
+    auto [qo, ko] = call_qk_norm_rope_fwd(q, k, qw, kw, cos, sin, eps);
+    return {qo, ko};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static const auto op = op_handle<decltype(qk_norm_rope_bwd)>("pithtrain_amd::qk_norm_rope_bwd");
+    const auto s = ctx->get_saved_variables();
+    auto [dq, dk, dwq, dwk] = op.call(s[0], s[1], or_none(s[2]), or_none(s[3]), s[4], s[5], grads[0], grads[1], ctx->saved_data["eps"].toDouble());
+    return {dq, dk, s[2].defined() ? dwq : Tensor(), s[3].defined() ? dwk : Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+Two qk_norm_rope_fwd_autograd(const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos, const Tensor& sin, double eps) {
+  const Tensor a = or_undefined(qw), b = or_undefined(kw);
+  if (any_requires_grad({&q, &k, &a, &b})) {
+    auto r = QkNormRopeFunction::apply(q, k, qw, kw, cos, sin, eps);
+    return {r[0], r[1]};
+  }
+  at::AutoDispatchBelowADInplaceOrView guard;
+  return call_qk_norm_rope_fwd(q, k, qw, kw, cos, sin, eps);
+}
+
+Three call_mla_assemble_fwd(const Tensor& q, const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin, const OptTensor& pos) {
+  static const auto op = op_handle<decltype(mla_assemble_fwd)>("pithtrain_amd::mla_assemble_fwd");
+  return op.call(q, kv, k_pe, cos, sin, pos);
+}
+struct MlaAssembleFunction : torch::autograd::Function<MlaAssembleFunction> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin,
+                               const OptTensor& pos) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    ctx->save_for_backward({cos, sin, or_undefined(pos)});
+    ctx->saved_data["k_pe_heads"] = (int64_t)(k_pe.dim() == 4 ? 1 : 0);
+    auto [qo, ko, vo] = call_mla_assemble_fwd(q, kv, k_pe, cos, sin, pos);
+    return {qo, ko, vo};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static const auto op = op_handle<decltype(mla_assemble_bwd)>("pithtrain_amd::mla_assemble_bwd");
+    const auto s = ctx->get_saved_variables();
+    auto [dq, dkv, dpe] = op.call(grads[0], grads[1], grads[2], s[0], s[1], or_none(s[2]), ctx->saved_data["k_pe_heads"].toInt());
+    return {dq, dkv, dpe, Tensor(), Tensor(), Tensor()};
+  }
+};
+Three mla_assemble_fwd_autograd(const Tensor& q, const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin, const OptTensor& pos) {
+  if (any_requires_grad({&q, &kv, &k_pe})) {
+    auto r = MlaAssembleFunction::apply(q, kv, k_pe, cos, sin, pos);
+    return {r[0], r[1], r[2]};
+  }
+  at::AutoDispatchBelowADInplaceOrView guard;
+  return call_mla_assemble_fwd(q, kv, k_pe, cos, sin, pos);
+}
+
+}  // namespace
+
+TORCH_LIBRARY(pithtrain_amd, m) {
+  m.def("attn_fwd(Tensor q, Tensor k, Tensor v, float softmax_scale, bool causal) -> (Tensor, Tensor)");
+  m.def("attn_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor dout, float softmax_scale, bool causal) -> (Tensor, Tensor, Tensor)");
+  m.def("norm_rope_fwd(Tensor x, Tensor? weight, Tensor cos, Tensor sin, float eps) -> Tensor");
+  m.def("norm_rope_bwd(Tensor x, Tensor? weight, Tensor cos, Tensor sin, Tensor dout, float eps) -> (Tensor, Tensor)");
+  m.def("qk_norm_rope_fwd(Tensor q, Tensor k, Tensor? q_weight, Tensor? k_weight, Tensor cos, Tensor sin, float eps) -> (Tensor, Tensor)");
+  m.def("qk_norm_rope_bwd(Tensor q, Tensor k, Tensor? q_weight, Tensor? k_weight, Tensor cos, Tensor sin, Tensor dq_out, Tensor dk_out, float eps) "
+        "-> (Tensor, Tensor, Tensor, Tensor)");
+  m.def("mla_assemble_fwd(Tensor q, Tensor kv, Tensor k_pe, Tensor cos, Tensor sin, Tensor? position_ids) -> (Tensor, Tensor, Tensor)");
+  m.def("mla_assemble_bwd(Tensor dq_out, Tensor dk_out, Tensor dv_out, Tensor cos, Tensor sin, Tensor? position_ids, int k_pe_heads) "
+        "-> (Tensor, Tensor, Tensor)");
+}
+
+// CPU tensors are refused by the Python bodies (there is no CPU path); they reach them through the same functions.
+#define PITH_IMPL(key)                               \
+  TORCH_LIBRARY_IMPL(pithtrain_amd, key, m) {        \
+    m.impl("attn_fwd", &attn_fwd);                   \
+    m.impl("attn_bwd", &attn_bwd);                   \
+    m.impl("norm_rope_fwd", &norm_rope_fwd);         \
+    m.impl("norm_rope_bwd", &norm_rope_bwd);         \
+    m.impl("qk_norm_rope_fwd", &qk_norm_rope_fwd);   \
+    m.impl("qk_norm_rope_bwd", &qk_norm_rope_bwd);   \
+    m.impl("mla_assemble_fwd", &mla_assemble_fwd);   \
+    m.impl("mla_assemble_bwd", &mla_assemble_bwd);   \
+  }
+PITH_IMPL(CUDA)
+PITH_IMPL(CPU)
+#undef PITH_IMPL
+
+TORCH_LIBRARY_IMPL(pithtrain_amd, Autograd, m) {
+  m.impl("attn_fwd", &attn_fwd_autograd);
+  m.impl("norm_rope_fwd", &norm_rope_fwd_autograd);
+  m.impl("qk_norm_rope_fwd", &qk_norm_rope_fwd_autograd);
+  m.impl("mla_assemble_fwd", &mla_assemble_fwd_autograd);
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("set_bodies", [](py::dict d) { bodies().attr("update")(d); }, "Registers the Python bodies of ops (name -> function).");
+  m.def("attn_fwd_into", &attn_fwd_into);
+  m.def("attn_bwd_delta_into", &attn_bwd_delta_into);
+  m.def("attn_bwd_dkdv_into", &attn_bwd_dkdv_into);
+  m.def("attn_bwd_dq_into", &attn_bwd_dq_into);
+  m.def("combine_into", &combine_into);
+  m.def("combine_new", &combine_new);
+  m.def("cast_f32_bf16_into", &cast_f32_bf16_into);
+}

@@ -291,7 +291,8 @@ constexpr int kSumCols = 16;
 
 struct SumParams {
   const float* partial[2];
-  float* dw[2];
+  void* dw[2];
+  int bf16[2];  // dw is bf16: the fp32 sum is rounded here, not by a cast launch behind this one
   int n[2];
   int D[2];
 };
@@ -322,7 +323,8 @@ __global__ __launch_bounds__(kThreads) void sum_partials_kernel(SumParams sp) {
   if (part == 0 && col < D) {
     float total = 0.f;
     for (int i = 0; i < kParts; ++i) total += red[i * kSumCols + c];
-    sp.dw[t][col] = total;
+    if (sp.bf16[t]) reinterpret_cast<__bf16*>(sp.dw[t])[col] = (__bf16)total;
+    else reinterpret_cast<float*>(sp.dw[t])[col] = total;
   }
 }
 
@@ -484,6 +486,7 @@ int launch_bwd(const char* who, const pith_norm_rope_args* a, const pith_norm_ro
   for (int t = 0; t < 2; ++t) {
     sp.partial[t] = pp.t[t].partial;
     sp.dw[t] = both[t]->dweight;
+    sp.bf16[t] = both[t]->dweight_bf16 != 0;
     sp.n[t] = (int)(pp.t[t].grid_x * both[t]->B);
     sp.D[t] = (int)both[t]->D;
     if (both[t]->D > max_d) max_d = both[t]->D;

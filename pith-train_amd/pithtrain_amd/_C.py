@@ -96,7 +96,7 @@ class NormRopeArgs(Structure):
         ("out", c_void_p), ("dweight", c_void_p), ("workspace", c_void_p), ("workspace_bytes", c_int64),
         ("B", c_int64), ("S", c_int64), ("H", c_int64), ("D", c_int64),
         ("x_bs", c_int64), ("out_bs", c_int64), ("dout_bs", c_int64), ("cs_bs", c_int64),
-        ("eps", c_float), ("weight_dtype", c_int32),
+        ("eps", c_float), ("weight_dtype", c_int32), ("dweight_bf16", c_int32), ("reserved0", c_int32),
     ]  # fmt: skip
 
 

@@ -24,6 +24,7 @@ import torch
 import torch.nn as nn
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import define_op, native
 
 SUPPORTED_HEAD_DIMS = ((64, 64), (128, 128), (192, 128))
 
@@ -88,6 +89,8 @@ def attn_fwd_into(
     o (bf16; may be None) and / or acc_o (fp32; may be None); either may be prev_o itself. o_rows / acc_o_rows
     ((begin, end) query rows of this call on multiples of 32, None = all) restrict which rows each output
     receives. Head dims in MERGING_HEAD_DIMS, causal=False only."""
+    if native.attn_fwd_into(q, k, v, o, lse, softmax_scale, causal, k_pe, prev_o, acc_o, o_rows, acc_o_rows):
+        return
     _check_qkv(q, k, v, causal, k_pe)
     _C.require_device(q, lse)
     b, sq, hq, d_q = q.shape
@@ -129,6 +132,8 @@ def attn_fwd_into(
 
 def attn_bwd_delta_into(out: torch.Tensor, dout: torch.Tensor, delta: torch.Tensor) -> None:
     """delta[b, h, s] <- sum_d out * dout (fp32)."""
+    if native.attn_bwd_delta_into(out, dout, delta):
+        return
     _C.require_device(out, dout, delta)
     assert out.dtype == dout.dtype == torch.bfloat16 and out.shape == dout.shape, "out/dout mismatch"
     b, s, h, d_v = out.shape
@@ -214,10 +219,13 @@ def _device_compute_units(device: torch.device) -> int:
     return _compute_units[idx]
 
 
-def _ds_budget_bytes(device: torch.device) -> int:
+def _ds_budget_bytes(device: torch.device, enough: int) -> int:
     """What a hand-over buffer may take right now: the configured limit, and at most a fraction of the
-    memory that is free on the device or cached (unused) by torch's allocator."""
+    memory that is free on the device or cached (unused) by torch's allocator. The allocator's statistics (60 us of
+    host time) are only asked when free memory alone does not already allow the `enough` bytes the caller wants."""
     free, _ = torch.cuda.mem_get_info(device)
+    if min(DS_BUFFER_LIMIT_BYTES, int(free * DS_BUFFER_FREE_FRACTION)) >= enough:
+        return enough
     cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
     return min(DS_BUFFER_LIMIT_BYTES, int((free + max(cached, 0)) * DS_BUFFER_FREE_FRACTION))
 
@@ -227,12 +235,15 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
     or None when both kernels should recompute (no hand-over path for these head dims, the dS-reading dQ
     kernel would have fewer workgroups than the device has compute units, or not even one kv head fits the
     budget)."""
+    b, sq, hq, _ = q.shape
+    hkv = k.shape[2]
+    row_tiles = -(-sq // _DS_ROWS_PER_WORKGROUP)
+    if row_tiles * hq * b < _device_compute_units(q.device):  # no slab can fill the device either
+        return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:
         return None
-    b, sq, hq, _ = q.shape
-    hkv = k.shape[2]
-    budget = _ds_budget_bytes(q.device)
+    budget = _ds_budget_bytes(q.device, need)
     per_kv_head = need // hkv
     heads = hkv
     while heads > 1 and per_kv_head * heads > budget:
@@ -241,7 +252,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
             heads -= 1
     if per_kv_head * heads > budget:
         return None
-    if -(-sq // _DS_ROWS_PER_WORKGROUP) * (hq // hkv) * heads * b < _device_compute_units(q.device):
+    if row_tiles * (hq // hkv) * heads * b < _device_compute_units(q.device):
         return None
     return heads, per_kv_head * heads
 
@@ -305,6 +316,8 @@ def attn_bwd_dkdv_into(
     same dtype as dk) receives the gradient of k_pe, summed over heads in head order.
     ds: uint8 buffer of attn_bwd_ds_bytes(q, k, v, causal) bytes; the kernel leaves its dS tiles there for an
     attn_bwd_dq_into call on the same chunk pair with the same buffer."""
+    if native.attn_bwd_dkdv_into(q, k, v, dout, lse, delta, dk, dv, softmax_scale, causal, accumulate, k_pe, dk_pe, ds, zero_tail):
+        return
     args = _bwd_args(q, k, v, dout, lse, delta, softmax_scale, causal, k_pe)
     _set_ds(args, ds, q)
     _C.require_device(q, dk, dv)
@@ -343,6 +356,8 @@ def attn_bwd_dq_into(
     rounded to bf16 in dq_final instead of dq.
     ds: the buffer an attn_bwd_dkdv_into call on the same chunk pair has just filled; dq is then
     computed from those dS tiles without recomputing the scores."""
+    if native.attn_bwd_dq_into(q, k, v, dout, lse, delta, dq, softmax_scale, causal, accumulate, k_pe, ds, dq_final, dq_final_rows):
+        return
     args = _bwd_args(q, k, v, dout, lse, delta, softmax_scale, causal, k_pe)
     _set_ds(args, ds, q)
     _C.require_device(q, dq)
@@ -411,28 +426,23 @@ def _mla_bwd_dq(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, dout: torch.T
 
 
 # ---------------------------------------------------------------------------------------------
-# Single-device attention as torch.library custom ops, so that layers compiled with
+# Single-device attention as torch.library ops, so that layers compiled with
 # torch.compile(fullgraph=True) keep working: the reference wraps its Triton launches the same
-# way (pithtrain/operators/mla/triton.py:445-508). Two ops (forward, backward), fake
-# implementations that only produce shapes, and an autograd formula tying them together.
+# way (pithtrain/operators/mla/triton.py:445-508). Two ops (forward, backward) and the autograd
+# formula that ties them together live in the native host path; here are the bodies for calls of
+# unusual layout, and the fake implementations that only produce shapes.
 
 
-@torch.library.custom_op("pithtrain_amd::attn_fwd", mutates_args=())
-def _attn_fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float,
-                 causal: bool) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
+def _attn_fwd_body(q, k, v, softmax_scale, causal):
     return _mla_fwd(q.contiguous(), k.contiguous(), v.contiguous(), softmax_scale, causal)
 
 
-@_attn_fwd_op.register_fake
-def _(q, k, v, softmax_scale, causal):
+def _attn_fwd_fake(q, k, v, softmax_scale, causal):
     b, sq, hq, _ = q.shape
     return q.new_empty((b, sq, hq, v.shape[-1])), q.new_empty((b, hq, sq), dtype=torch.float32)
 
 
-@torch.library.custom_op("pithtrain_amd::attn_bwd", mutates_args=())
-def _attn_bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
-                 dout: torch.Tensor, softmax_scale: float,
-                 causal: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:  # fmt: skip
+def _attn_bwd_body(q, k, v, o, lse, dout, softmax_scale, causal):
     q, k, v, o, dout = q.contiguous(), k.contiguous(), v.contiguous(), o.contiguous(), dout.contiguous()
     delta = _mla_bwd_preprocess(o, dout)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
@@ -440,26 +450,12 @@ def _attn_bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Ten
     return dq, dk, dv
 
 
-@_attn_bwd_op.register_fake
-def _(q, k, v, o, lse, dout, softmax_scale, causal):
+def _attn_bwd_fake(q, k, v, o, lse, dout, softmax_scale, causal):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
 
 
-def _attn_setup_context(ctx, inputs, output):
-    q, k, v, softmax_scale, causal = inputs
-    o, lse = output
-    ctx.save_for_backward(q, k, v, o, lse)
-    ctx.softmax_scale = softmax_scale
-    ctx.causal = causal
-
-
-def _attn_backward(ctx, grad_o, grad_lse):
-    q, k, v, o, lse = ctx.saved_tensors
-    dq, dk, dv = _attn_bwd_op(q, k, v, o, lse, grad_o, ctx.softmax_scale, ctx.causal)
-    return dq, dk, dv, None, None
-
-
-_attn_fwd_op.register_autograd(_attn_backward, setup_context=_attn_setup_context)
+_attn_fwd_op = define_op("attn_fwd", _attn_fwd_body, _attn_fwd_fake)
+_attn_bwd_op = define_op("attn_bwd", _attn_bwd_body, _attn_bwd_fake)
 
 
 def attention_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float | None = None,

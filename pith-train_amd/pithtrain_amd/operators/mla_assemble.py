@@ -27,6 +27,7 @@ from typing import Optional, Tuple
 import torch
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import define_op
 
 
 def _tables(cos: torch.Tensor, sin: torch.Tensor, dr: int) -> int:
@@ -110,9 +111,11 @@ def mla_assemble_bwd_into(dq_out, dk_out, dv_out, cos, sin, position_ids, dq, dk
     _C.check(_C.lib().pith_mla_assemble_bwd(_C.byref(args), _C.current_stream(dq_out)))
 
 
-@torch.library.custom_op("pithtrain_amd::mla_assemble_fwd", mutates_args=())
-def _mla_assemble_fwd_op(q: torch.Tensor, kv: torch.Tensor, k_pe: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                         position_ids: Optional[torch.Tensor]) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:  # fmt: skip
+# Bodies of the ops for calls of unusual layout, and their fake (shape) implementations; the ordinary calls and the
+# autograd formula are native.
+
+
+def _mla_assemble_fwd_body(q, kv, k_pe, cos, sin, position_ids):
     b, s, h, dqk = q.shape
     dv = kv.shape[-1] - (dqk - k_pe.shape[-1])
     q_out = q.new_empty((b, s, h, dqk))
@@ -122,17 +125,13 @@ def _mla_assemble_fwd_op(q: torch.Tensor, kv: torch.Tensor, k_pe: torch.Tensor, 
     return q_out, k_out, v_out
 
 
-@_mla_assemble_fwd_op.register_fake
-def _(q, kv, k_pe, cos, sin, position_ids):
+def _mla_assemble_fwd_fake(q, kv, k_pe, cos, sin, position_ids):
     b, s, h, dqk = q.shape
     dv = kv.shape[-1] - (dqk - k_pe.shape[-1])
     return q.new_empty((b, s, h, dqk)), q.new_empty((b, s, h, dqk)), q.new_empty((b, s, h, dv))
 
 
-@torch.library.custom_op("pithtrain_amd::mla_assemble_bwd", mutates_args=())
-def _mla_assemble_bwd_op(dq_out: torch.Tensor, dk_out: torch.Tensor, dv_out: torch.Tensor, cos: torch.Tensor,
-                         sin: torch.Tensor, position_ids: Optional[torch.Tensor],
-                         k_pe_heads: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:  # fmt: skip
+def _mla_assemble_bwd_body(dq_out, dk_out, dv_out, cos, sin, position_ids, k_pe_heads):
     b, s, h, dqk = dq_out.shape
     dr, dv = cos.shape[1], dv_out.shape[-1]
     dq = dq_out.new_empty((b, s, h, dqk))
@@ -143,27 +142,15 @@ def _mla_assemble_bwd_op(dq_out: torch.Tensor, dk_out: torch.Tensor, dv_out: tor
     return dq, dkv, (dk_pe.unsqueeze(2) if k_pe_heads else dk_pe)
 
 
-@_mla_assemble_bwd_op.register_fake
-def _(dq_out, dk_out, dv_out, cos, sin, position_ids, k_pe_heads):
+def _mla_assemble_bwd_fake(dq_out, dk_out, dv_out, cos, sin, position_ids, k_pe_heads):
     b, s, h, dqk = dq_out.shape
     dr, dv = cos.shape[1], dv_out.shape[-1]
     dk_pe = dq_out.new_empty((b, s, 1, dr) if k_pe_heads else (b, s, dr))
     return dq_out.new_empty((b, s, h, dqk)), dq_out.new_empty((b, s, h, dqk - dr + dv)), dk_pe
 
 
-def _setup_context(ctx, inputs, output):
-    q, kv, k_pe, cos, sin, position_ids = inputs
-    ctx.save_for_backward(cos, sin, position_ids)
-    ctx.k_pe_heads = 1 if k_pe.dim() == 4 else 0
-
-
-def _backward(ctx, dq_out, dk_out, dv_out):
-    cos, sin, position_ids = ctx.saved_tensors
-    dq, dkv, dk_pe = _mla_assemble_bwd_op(dq_out, dk_out, dv_out, cos, sin, position_ids, ctx.k_pe_heads)
-    return dq, dkv, dk_pe, None, None, None
-
-
-_mla_assemble_fwd_op.register_autograd(_backward, setup_context=_setup_context)
+_mla_assemble_fwd_op = define_op("mla_assemble_fwd", _mla_assemble_fwd_body, _mla_assemble_fwd_fake)
+_mla_assemble_bwd_op = define_op("mla_assemble_bwd", _mla_assemble_bwd_body, _mla_assemble_bwd_fake)
 
 
 def mla_assemble_qkv(q: torch.Tensor, kv: torch.Tensor, k_pe: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

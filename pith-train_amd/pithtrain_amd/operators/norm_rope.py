@@ -15,8 +15,8 @@ with  `qk_norm_rope(query_states, key_states, self.q_norm.weight, self.k_norm.we
  b : batch size, s : sequence length, h : heads, d : head dim.
 x [b, s, h, d] bf16; cos, sin [b, s, d] (or [1, s, d] / [s, d], shared by the batch) bf16;
 weight [d] bf16 or fp32. Arithmetic is fp32 with a single rounding to bf16 (the reference's eager
-bf16 expression rounds after every elementwise op). Wrapped as torch.library custom ops with fake
-implementations and an autograd formula, so compiled layers keep working.
+bf16 expression rounds after every elementwise op). torch.library ops with fake implementations and an
+autograd formula, so compiled layers keep working.
 """
 
 from typing import Optional, Tuple
@@ -24,6 +24,7 @@ from typing import Optional, Tuple
 import torch
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import define_op
 
 
 def _cos_sin_stride(cos: torch.Tensor, sin: torch.Tensor, b: int, s: int, d: int) -> int:
@@ -86,51 +87,43 @@ def norm_rope_bwd_into(x: torch.Tensor, weight: Optional[torch.Tensor], cos: tor
     _C.check(_C.lib().pith_norm_rope_bwd(_C.byref(args), _C.current_stream(x)))
 
 
-@torch.library.custom_op("pithtrain_amd::norm_rope_fwd", mutates_args=())
-def _norm_rope_fwd_op(x: torch.Tensor, weight: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
-                      eps: float) -> torch.Tensor:  # fmt: skip
+# Bodies of the ops for calls of unusual layout, and their fake (shape) implementations; the ordinary calls and the
+# autograd formulas are native.
+
+
+def _dweight_like(x: torch.Tensor, weight: Optional[torch.Tensor]) -> torch.Tensor:
+    """Result of an op for the weight gradient, in the weight's dtype; an op cannot return None, hence the placeholder."""
+    return x.new_empty((0,), dtype=torch.float32) if weight is None else torch.empty_like(weight)
+
+
+def _norm_rope_fwd_body(x, weight, cos, sin, eps):
     x = x.contiguous()
     out = torch.empty_like(x)
     norm_rope_fwd_into(x, weight, cos.contiguous(), sin.contiguous(), out, eps)
     return out
 
 
-@_norm_rope_fwd_op.register_fake
-def _(x, weight, cos, sin, eps):
+def _norm_rope_fwd_fake(x, weight, cos, sin, eps):
     return torch.empty_like(x, memory_format=torch.contiguous_format)
 
 
-@torch.library.custom_op("pithtrain_amd::norm_rope_bwd", mutates_args=())
-def _norm_rope_bwd_op(x: torch.Tensor, weight: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
-                      dout: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
+def _norm_rope_bwd_body(x, weight, cos, sin, dout, eps):
     x, dout = x.contiguous(), dout.contiguous()
     dx = torch.empty_like(x)
-    # without a weight the second result is an empty placeholder (custom ops cannot return None)
-    dweight = x.new_empty((x.shape[-1] if weight is not None else 0,), dtype=torch.float32)
-    norm_rope_bwd_into(x, weight, cos.contiguous(), sin.contiguous(), dout, dx,
-                       dweight if weight is not None else None, eps)  # fmt: skip
-    return dx, dweight
+    if weight is None:
+        norm_rope_bwd_into(x, None, cos.contiguous(), sin.contiguous(), dout, dx, None, eps)
+        return dx, _dweight_like(x, None)
+    dweight = x.new_empty((x.shape[-1],), dtype=torch.float32)
+    norm_rope_bwd_into(x, weight, cos.contiguous(), sin.contiguous(), dout, dx, dweight, eps)
+    return dx, dweight.to(weight.dtype)
 
 
-@_norm_rope_bwd_op.register_fake
-def _(x, weight, cos, sin, dout, eps):
-    dx = torch.empty_like(x, memory_format=torch.contiguous_format)
-    return dx, x.new_empty((x.shape[-1] if weight is not None else 0,), dtype=torch.float32)
+def _norm_rope_bwd_fake(x, weight, cos, sin, dout, eps):
+    return torch.empty_like(x, memory_format=torch.contiguous_format), _dweight_like(x, weight)
 
 
-def _setup_context(ctx, inputs, output):
-    x, weight, cos, sin, eps = inputs
-    ctx.save_for_backward(x, weight, cos, sin)
-    ctx.eps = eps
-
-
-def _backward(ctx, grad_out):
-    x, weight, cos, sin = ctx.saved_tensors
-    dx, dweight = _norm_rope_bwd_op(x, weight, cos, sin, grad_out, ctx.eps)
-    return dx, (None if weight is None else dweight.to(weight.dtype)), None, None, None
-
-
-_norm_rope_fwd_op.register_autograd(_backward, setup_context=_setup_context)
+_norm_rope_fwd_op = define_op("norm_rope_fwd", _norm_rope_fwd_body, _norm_rope_fwd_fake)
+_norm_rope_bwd_op = define_op("norm_rope_bwd", _norm_rope_bwd_body, _norm_rope_bwd_fake)
 
 
 def norm_rope(x: torch.Tensor, weight: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
@@ -180,60 +173,34 @@ def qk_norm_rope_bwd_into(q, k, q_weight, k_weight, cos, sin, dq_out, dk_out, dq
     _C.check(_C.lib().pith_norm_rope_bwd_pair(_C.byref(a), _C.byref(b), _C.current_stream(q)))
 
 
-@torch.library.custom_op("pithtrain_amd::qk_norm_rope_fwd", mutates_args=())
-def _qk_norm_rope_fwd_op(q: torch.Tensor, k: torch.Tensor, q_weight: Optional[torch.Tensor],
-                         k_weight: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
-                         eps: float) -> Tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
+def _qk_norm_rope_fwd_body(q, k, q_weight, k_weight, cos, sin, eps):
     q, k = q.contiguous(), k.contiguous()
     q_out, k_out = torch.empty_like(q), torch.empty_like(k)
     qk_norm_rope_fwd_into(q, k, q_weight, k_weight, cos.contiguous(), sin.contiguous(), q_out, k_out, eps)
     return q_out, k_out
 
 
-@_qk_norm_rope_fwd_op.register_fake
-def _(q, k, q_weight, k_weight, cos, sin, eps):
+def _qk_norm_rope_fwd_fake(q, k, q_weight, k_weight, cos, sin, eps):
     fmt = torch.contiguous_format
     return torch.empty_like(q, memory_format=fmt), torch.empty_like(k, memory_format=fmt)
 
 
-@torch.library.custom_op("pithtrain_amd::qk_norm_rope_bwd", mutates_args=())
-def _qk_norm_rope_bwd_op(q: torch.Tensor, k: torch.Tensor, q_weight: Optional[torch.Tensor],
-                         k_weight: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor,
-                         dq_out: torch.Tensor, dk_out: torch.Tensor,
-                         eps: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:  # fmt: skip
+def _qk_norm_rope_bwd_body(q, k, q_weight, k_weight, cos, sin, dq_out, dk_out, eps):
     q, k, dq_out, dk_out = q.contiguous(), k.contiguous(), dq_out.contiguous(), dk_out.contiguous()
     dq, dk = torch.empty_like(q), torch.empty_like(k)
-    # without weights the last two results are empty placeholders (custom ops cannot return None)
-    n = q.shape[-1] if q_weight is not None else 0
-    dwq, dwk = q.new_empty((n,), dtype=torch.float32), q.new_empty((n,), dtype=torch.float32)
-    qk_norm_rope_bwd_into(q, k, q_weight, k_weight, cos.contiguous(), sin.contiguous(), dq_out, dk_out, dq, dk,
-                          dwq if n else None, dwk if n else None, eps)  # fmt: skip
-    return dq, dk, dwq, dwk
+    dws = [None if w is None else q.new_empty((q.shape[-1],), dtype=torch.float32) for w in (q_weight, k_weight)]
+    qk_norm_rope_bwd_into(q, k, q_weight, k_weight, cos.contiguous(), sin.contiguous(), dq_out, dk_out, dq, dk, *dws, eps)
+    return dq, dk, *(_dweight_like(q, None) if w is None else dw.to(w.dtype) for w, dw in zip((q_weight, k_weight), dws))
 
 
-@_qk_norm_rope_bwd_op.register_fake
-def _(q, k, q_weight, k_weight, cos, sin, dq_out, dk_out, eps):
+def _qk_norm_rope_bwd_fake(q, k, q_weight, k_weight, cos, sin, dq_out, dk_out, eps):
     fmt = torch.contiguous_format
-    n = q.shape[-1] if q_weight is not None else 0
     return (torch.empty_like(q, memory_format=fmt), torch.empty_like(k, memory_format=fmt),
-            q.new_empty((n,), dtype=torch.float32), q.new_empty((n,), dtype=torch.float32))  # fmt: skip
+            _dweight_like(q, q_weight), _dweight_like(q, k_weight))  # fmt: skip
 
 
-def _qk_setup_context(ctx, inputs, output):
-    q, k, q_weight, k_weight, cos, sin, eps = inputs
-    ctx.save_for_backward(q, k, q_weight, k_weight, cos, sin)
-    ctx.eps = eps
-
-
-def _qk_backward(ctx, grad_q, grad_k):
-    q, k, q_weight, k_weight, cos, sin = ctx.saved_tensors
-    dq, dk, dwq, dwk = _qk_norm_rope_bwd_op(q, k, q_weight, k_weight, cos, sin, grad_q, grad_k, ctx.eps)
-    if q_weight is None:
-        return dq, dk, None, None, None, None, None
-    return dq, dk, dwq.to(q_weight.dtype), dwk.to(k_weight.dtype), None, None, None
-
-
-_qk_norm_rope_fwd_op.register_autograd(_qk_backward, setup_context=_qk_setup_context)
+_qk_norm_rope_fwd_op = define_op("qk_norm_rope_fwd", _qk_norm_rope_fwd_body, _qk_norm_rope_fwd_fake)
+_qk_norm_rope_bwd_op = define_op("qk_norm_rope_bwd", _qk_norm_rope_bwd_body, _qk_norm_rope_bwd_fake)
 
 
 def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor,

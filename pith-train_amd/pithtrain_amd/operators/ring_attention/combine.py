@@ -8,6 +8,7 @@ pithtrain/operators/ring_attention/standard.py:53-66.
 import torch
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import native
 
 
 def combine_into(
@@ -20,6 +21,8 @@ def combine_into(
     along S of larger contiguous tensors. `out` may be out1 or out2 itself when dtypes match, and
     lse_out may be lse1 or lse2 (every element is read before it is written by the same thread).
     """
+    if native.combine_into(out1, lse1, out2, lse2, out, lse_out, base):
+        return
     _C.require_device(out1, lse1, out2, lse2, out, lse_out)
     b, s, h, d = out1.shape
     assert out2.shape == out1.shape and out.shape == out1.shape, "out tensors disagree on shape"
@@ -40,6 +43,9 @@ def combine_into(
 
 def _combine_new(out1, lse1, out2, lse2, base):
     """Reference calling convention: fresh fp32 outputs whatever the input dtypes."""
+    made = native.combine_new(out1, lse1, out2, lse2, base)
+    if made is not None:
+        return made
     assert lse1.is_contiguous() or lse1.stride(-1) == 1
     new_out = torch.empty(out1.shape, dtype=torch.float32, device=out1.device)
     new_lse = torch.empty(lse1.shape, dtype=torch.float32, device=lse1.device)
@@ -49,6 +55,8 @@ def _combine_new(out1, lse1, out2, lse2, base):
 
 def cast_f32_bf16_into(src: torch.Tensor, dst: torch.Tensor) -> None:
     """dst <- bf16(src), both contiguous with the same number of elements."""
+    if native.cast_f32_bf16_into(src, dst):
+        return
     _C.require_device(src, dst)
     assert src.dtype == torch.float32 and dst.dtype == torch.bfloat16 and src.numel() == dst.numel()
     assert src.is_contiguous() and dst.is_contiguous()
