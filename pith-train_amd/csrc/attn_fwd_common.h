@@ -6,8 +6,7 @@
 namespace pith {
 
 constexpr int kFwdBlockN = 64;            // keys per LDS tile
-constexpr float kRescaleThreshold = 8.f;  // log2 units, see attn_fwd.hip
-constexpr float kRescaleLimit = 256.f;    // = 2^kRescaleThreshold: the same bound on a P value, tested on row sums (attn_fwd_direct.hip)
+constexpr float kRescaleLimit = 256.f;    // bound on a P value before the running maximum is refreshed, tested on row sums
 
 struct FwdParams {
   const __bf16* q;
@@ -34,9 +33,11 @@ struct FwdParams {
   int o_r0, o_r1, acc_r0, acc_r1;  // query rows [r0, r1) that receive o / acc_o when merging (multiples of 32, or Sq)
 };
 
-// Forward for head dims (128, 128) and (192, 128) with tiles loaded global -> LDS directly:
-// attn_fwd_direct.hip. dqk = 128 or 192; half = workgroups of 128 query rows whose wave pairs split
-// the keys of every tile (see there) instead of 256-row workgroups.
+// Forward with one 8-wave workgroup per compute unit: attn_fwd_direct.hip. dqk = 128, or 192 with half; half = workgroups
+// of 128 query rows whose wave pairs split the keys of every tile (see there) instead of 256-row workgroups.
 void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipStream_t stream);
+
+// Forward with two (64 features: three) 4-wave workgroups of 128 query rows per compute unit: attn_fwd_duo.hip.
+void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t stream);
 
 }  // namespace pith

@@ -1,5 +1,5 @@
 // Chunk attention forward for head dims (128, 128) and (192, 128) on gfx950. Same function and
-// numerics as the general kernel in attn_fwd.hip (pithtrain/operators/mla/triton.py:32-93,
+// numerics as stated in attn_fwd.hip (pithtrain/operators/mla/triton.py:32-93,
 // :274-323: fp32 scores from bf16 MFMA, P = exp2(kappa*(s - m)) in fp32, row sum from the fp32 P,
 // P rounded to bf16 for P V, base-2 LSE, lazily refreshed running maximum), organised around two
 // facts measured on the device:
@@ -52,8 +52,7 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
   constexpr int KVB = HALF ? 1 : 2;          // 32-key blocks of a tile this wave owns
   constexpr int kBM = HALF ? 128 : 256;      // query rows per workgroup
   constexpr int kKTile = kTile + (DQK == 192 ? kExtraTile : 0);
-  static_assert(DQK == 128 || DQK == 192, "head dims");
-  constexpr bool kSumTest = !(DQK == 192 && !HALF);  // how the softmax decides to refresh its running maximum
+  static_assert(DQK == 128 || (DQK == 192 && HALF), "head dims");
   // the tile rings; the epilogue reuses them to turn the output tile (one area per storing wave)
   constexpr int kRings = kSlots * (kKTile + kTile), kTurn = (HALF ? kWaves / 2 : kWaves) * kRowsViaLdsBytes<DVB>;
   // 256-row workgroups for 128 features fetch their query block through LDS as well (four 64-row tiles into the three
@@ -163,13 +162,12 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
   int x_base = kTile + straight_offset128(c, g + 8 * kvb0);
   int v_base[2] = {transposed_offset128(0, 0, 0, lane) + kvb0 * 32 * kRowBytes128,
                    transposed_offset128(0, 1, 0, lane) + kvb0 * 32 * kRowBytes128};
-  // Only the variants that would spill otherwise pay the extra XOR per read (the 256-row causal kernels); the
+  // Only the variant that would spill otherwise pays the extra XOR per read (the 256-row causal kernel); the
   // others let the compiler keep every derived offset in a register.
   constexpr bool kDeriveOffsets = !HALF && CAUSAL;
   auto refresh_offsets = [&]() __attribute__((always_inline)) {
     if constexpr (kDeriveOffsets) {
       asm volatile("" : "+v"(k_base), "+v"(v_base[0]), "+v"(v_base[1]));
-      if constexpr (DQK == 192) asm volatile("" : "+v"(x_base));
     }
   };
   auto k_off = [&](int ks) __attribute__((always_inline)) { return ks < 8 ? k_base ^ (ks << 5) : x_base ^ ((ks - 8) << 5); };
@@ -218,66 +216,37 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
     }
     f32x16 e[KVB];
     float rs = 0.f;
-    if constexpr (kSumTest) {
-      // The running maximum is refreshed lazily, and whether a refresh is due is read off the row sum instead of a
-      // maximum over the tile: every term of the sum is >= 0, so a lane's partial sum within kRescaleLimit means that
-      // none of its P values exceeds kRescaleLimit either. The common tile then costs no maximum at all (24 of the
-      // ~140 vector instructions per tile); a tile that fails the test (the first tile of a row, tiles where the scores
-      // still climb, and any overflow or NaN) is redone from the scores, which are kept until the test has passed.
-      const bool fresh = m_run == -INFINITY;
-      float mk = fresh ? 0.f : m_run * p.kappa;
+    // The running maximum is refreshed lazily, and whether a refresh is due is read off the row sum instead of a
+    // maximum over the tile: every term of the sum is >= 0, so a lane's partial sum within kRescaleLimit means that
+    // none of its P values exceeds kRescaleLimit either. The common tile then costs no maximum at all (24 of the
+    // ~140 vector instructions per tile); a tile that fails the test (the first tile of a row, tiles where the scores
+    // still climb, and any overflow or NaN) is redone from the scores, which are kept until the test has passed.
+    const bool fresh = m_run == -INFINITY;
+    float mk = fresh ? 0.f : m_run * p.kappa;
 #pragma unroll
-      for (int kvb = 0; kvb < KVB; ++kvb)
+    for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          e[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - mk);
-          rs += e[kvb][v];
-        }
-      if (__builtin_amdgcn_ballot_w64(fresh || !(rs <= kRescaleLimit)) != 0) {  // wave-uniform, rare
-        float x = s[0][0];
-#pragma unroll
-        for (int kvb = 0; kvb < KVB; ++kvb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) x = fmaxf(x, s[kvb][v]);
-        const float m_new = fmaxf(m_run, pair_max(x));
-        // a row with no visible key so far keeps m = -inf; exp2 of (-inf - -inf) is avoided
-        const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
-        m_run = m_new;
-        l_run *= alpha;
-#pragma unroll
-        for (int i = 0; i < DVB; ++i)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) oacc[i][v] *= alpha;
-        mk = (m_run == -INFINITY) ? 0.f : m_run * p.kappa;
-        rs = 0.f;
-#pragma unroll
-        for (int kvb = 0; kvb < KVB; ++kvb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            e[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - mk);
-            rs += e[kvb][v];
-          }
+      for (int v = 0; v < 16; ++v) {
+        e[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - mk);
+        rs += e[kvb][v];
       }
-    } else {
-      // the 256-row kernels for 192-feature keys have no registers for a second score tile: tile maximum first
+    if (__builtin_amdgcn_ballot_w64(fresh || !(rs <= kRescaleLimit)) != 0) {  // wave-uniform, rare
       float x = s[0][0];
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) x = fmaxf(x, s[kvb][v]);
-      const float mx = pair_max(x);
-      const bool refresh = (mx - m_run) * p.kappa > kRescaleThreshold;  // true on the first tile (m = -inf)
-      if (__builtin_amdgcn_ballot_w64(refresh) != 0) {                   // wave-uniform
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
-        m_run = m_new;
-        l_run *= alpha;
+      const float m_new = fmaxf(m_run, pair_max(x));
+      // a row with no visible key so far keeps m = -inf; exp2 of (-inf - -inf) is avoided
+      const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
+      m_run = m_new;
+      l_run *= alpha;
 #pragma unroll
-        for (int i = 0; i < DVB; ++i)
+      for (int i = 0; i < DVB; ++i)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) oacc[i][v] *= alpha;
-      }
-      const float mk = (m_run == -INFINITY) ? 0.f : m_run * p.kappa;
+        for (int v = 0; v < 16; ++v) oacc[i][v] *= alpha;
+      mk = (m_run == -INFINITY) ? 0.f : m_run * p.kappa;
+      rs = 0.f;
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
@@ -437,13 +406,10 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
     using Full = std::true_type;
     using Part = std::false_type;
     int i = 0;
-    // the pair as one loop body (no parity tests, the odd interval without request code) wherever two copies of the
-    // interval still fit the registers
-    if constexpr (!(DQK == 192 && !HALF)) {
-      for (; i + 2 < n_tiles_wave; i += 2) {
-        interval(i, late_tag, Full{}, std::integral_constant<int, 1>{});
-        interval(i + 1, late_tag, Full{}, std::integral_constant<int, 2>{});
-      }
+    // the pair as one loop body: no parity tests, the odd interval without request code
+    for (; i + 2 < n_tiles_wave; i += 2) {
+      interval(i, late_tag, Full{}, std::integral_constant<int, 1>{});
+      interval(i + 1, late_tag, Full{}, std::integral_constant<int, 2>{});
     }
     if constexpr (kQViaLds && !CAUSAL) warm_previous_rows();
     for (; i + 1 < n_tiles_wave; ++i) interval(i, late_tag, Full{}, std::integral_constant<int, 0>{});
@@ -522,23 +488,8 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
   }
   // O^T sits in the accumulators (a lane owns one query row): turned through LDS so that the stores
   // cover whole rows. Every wave is past the barrier behind the last tile read (HALF: past the merge).
-  // (Not in the 256-row causal kernel for 192-feature keys, which has no register to spare: the extra
-  // live values of the turned epilogue push spills into its main loop.)
-  if constexpr (!(DQK == 192 && !HALF && CAUSAL)) {
-    char* const turn = smem + (HALF ? (wave & 3) : wave) * kRowsViaLdsBytes<DVB>;
-    store_rows32_via_lds<__bf16, DVB>(turn, oh + q_wave0 * o_row_stride, o_row_stride, p.Sq - q_wave0, oacc, inv, false, lane);
-  } else if (qrow < p.Sq) {
-    __bf16* dst = oh + qrow * o_row_stride;
-#pragma unroll
-    for (int i = 0; i < DVB; ++i)
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        u32x2 w;
-        w[0] = pack_bf16x2(oacc[i][4 * b4] * inv, oacc[i][4 * b4 + 1] * inv);
-        w[1] = pack_bf16x2(oacc[i][4 * b4 + 2] * inv, oacc[i][4 * b4 + 3] * inv);
-        *reinterpret_cast<u32x2*>(dst + 32 * i + 8 * b4 + 4 * g) = w;
-      }
-  }
+  char* const turn = smem + (HALF ? (wave & 3) : wave) * kRowsViaLdsBytes<DVB>;
+  store_rows32_via_lds<__bf16, DVB>(turn, oh + q_wave0 * o_row_stride, o_row_stride, p.Sq - q_wave0, oacc, inv, false, lane);
   if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
@@ -558,8 +509,7 @@ void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipS
     if (half) launch_one<128, true>(p, causal, st);
     else launch_one<128, false>(p, causal, st);
   } else {
-    if (half) launch_one<192, true>(p, causal, st);
-    else launch_one<192, false>(p, causal, st);
+    launch_one<192, true>(p, causal, st);
   }
 }
 

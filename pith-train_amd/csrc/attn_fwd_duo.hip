@@ -1,0 +1,338 @@
+// Chunk attention forward for head dims (64, 64), (128, 128) and (192, 128) on gfx950 with SMALL workgroups: 4 wavefronts,
+// 128 query rows, two of them per compute unit (three at 64 features). Same function, numerics and tile layouts as
+// attn_fwd_direct.hip (pithtrain/operators/mla/triton.py:32-93, :274-323): a wave owns 32 query rows and all 64 keys of a
+// tile, per interval one matrix block [O^T += V(i)^T P(i)^T ; S(i+1)^T = K(i+1) Q^T] and one softmax.
+//
+// What bounds launches of a few rounds of workgroups is not the loop but everything around it: with one 8-wave workgroup
+// per compute unit nothing runs while it fetches its first tiles, waits for its slowest wave at the diagonal and writes its
+// rows (9-15 us per round). Two independent workgroups hide each other's: 3 x 1999 rows x 32 heads causal 131 -> 105 us
+// (128-row workgroups with split keys before), 8 x 512 x 32 47 -> 32 us, 2 x 2048 x 16 heads of 64 features 42 -> 31 us.
+// The waves that share a SIMD belong to different workgroups, so no role split keeps their matrix and vector phases apart;
+// measured, the workgroups drift apart by themselves: fixed or alternating wave priorities by wave slot were 2-10 %
+// slower, and so was asking for the tiles behind the matrix block (0-4 %).
+// 64 features: a K or V tile packs two rows per 256-byte LDS row (see DirectPaired64), and the softmax of 32 x 64 scores
+// costs as much vector time as its products cost matrix time, so three workgroups per compute unit share the pipes.
+//
+// LDS: rings of two K and two V tiles; interval i reads V(i) and K(i+1) while V(i+1) and K(i+2) land in the slots that
+// interval i-1 released.
+#include "attn_fwd_common.h"
+
+namespace pith {
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * 64;
+constexpr int kBM = 32 * kWaves;  // query rows per workgroup
+constexpr int kBN = kFwdBlockN;   // keys per tile
+constexpr int kAhead = 4;         // fragment reads run this many products ahead in the matrix block
+
+template <int DQK>
+struct DuoLayout {
+  static constexpr int kDv = DQK == 64 ? 64 : 128;
+  static constexpr int kKTile = DQK == 64 ? kExtraTileBytes : DQK == 128 ? kBN * kRowBytes128 : kBN * kRowBytes128 + kExtraTileBytes;
+  static constexpr int kVTile = kDv == 64 ? kExtraTileBytes : kBN * kRowBytes128;
+  static constexpr int kRings = 2 * (kKTile + kVTile);
+  static constexpr int kTurn = kWaves * kRowsViaLdsBytes<kDv / 32>;
+  static constexpr int kSmem = kRings > kTurn ? kRings : kTurn;
+};
+
+template <int DQK, bool CAUSAL>
+__global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) {
+  using L = DuoLayout<DQK>;
+  constexpr int kDv = L::kDv, KS = DQK / 16, DVB = kDv / 32, KVB = 2;
+  constexpr bool kPaired = DQK == 64;  // tiles hold two rows per 256-byte LDS row
+  constexpr int kTile = kBN * kRowBytes128;
+  __shared__ __attribute__((aligned(1024))) char smem[L::kSmem];
+  char* const kbuf = smem;
+  char* const vbuf = smem + 2 * L::kKTile;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, g = lane >> 5;
+
+  int m_tile, h, b;
+  decode_block(blockIdx.x, p.Hq, p.B, p.m_tiles, p.group, m_tile, h, b);
+  const int hk = h / p.group;
+  const int m0 = m_tile * kBM;
+  const int q_wave0 = m0 + wave * 32;
+  const int qrow = q_wave0 + c;
+
+  const int64_t q_row_stride = (int64_t)p.Hq * DQK;
+  const int64_t o_row_stride = (int64_t)p.Hq * kDv;
+  // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
+  const bool two_part = DQK == 192 && p.k_pe != nullptr;
+  const int k_head_elems = two_part ? 128 : DQK;
+  const int k_row_bytes = p.Hkv * k_head_elems * 2, v_row_bytes = p.Hkv * kDv * 2;
+  const __bf16* qh = p.q + b * p.q_bs + (int64_t)h * DQK;
+  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
+  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;
+  const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
+  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
+
+  // Number of key tiles this workgroup / this wavefront has to visit.
+  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
+  int n_tiles_wg = n_tiles_all, n_tiles_wave = n_tiles_all;
+  if (CAUSAL) {
+    n_tiles_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
+    n_tiles_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
+  }
+
+  DirectTile128<kBN, kThreads> vmover, kmover;
+  DirectPaired64<kThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
+  if constexpr (kPaired) {
+    vpmover.init(v_row_bytes, 0, wave, lane);
+    kpmover.init(k_row_bytes, 0, wave, lane);
+  } else {
+    vmover.init(v_row_bytes, wave, lane);
+    kmover.init(k_row_bytes, wave, lane);
+    if constexpr (DQK == 192) kpmover.init(kx_row_bytes, two_part ? 0 : 256, wave, lane);
+  }
+  auto issue_k = [&](int t) __attribute__((always_inline)) {
+    char* slot = kbuf + (t & 1) * L::kKTile;
+    const char* src = kh + (int64_t)t * kBN * k_row_bytes;
+    if constexpr (kPaired) {
+      kpmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+    } else {
+      kmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+      if constexpr (DQK == 192) kpmover.issue(kx + (int64_t)t * kBN * kx_row_bytes, p.Skv - t * kBN, slot + kTile, wave, lane);
+    }
+  };
+  auto issue_v = [&](int t) __attribute__((always_inline)) {
+    char* slot = vbuf + (t & 1) * L::kVTile;
+    const char* src = vh + (int64_t)t * kBN * v_row_bytes;
+    if constexpr (kPaired) vpmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+    else vmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+  };
+  issue_k(0);
+  issue_v(0);
+  if (n_tiles_wg > 1) issue_k(1);
+
+  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features.
+  bf16x8 qf[KS];
+  {
+    const int row = qrow < p.Sq ? qrow : p.Sq - 1;
+    const __bf16* src = qh + row * q_row_stride + g * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
+  }
+
+  // per-lane read offsets (see attn_fwd_direct.hip): one base per tile part, the rest by XOR
+  int k_base = straight_offset128(c, g);
+  int v_base[2] = {transposed_offset128(0, 0, 0, lane), transposed_offset128(0, 1, 0, lane)};
+  auto k_frag = [&](const char* ktile, int ks, int kvb) __attribute__((always_inline)) {
+    int off;
+    if (kPaired) off = k_base ^ (ks << 5) ^ (kvb << 7);
+    else if (ks < 8) off = (k_base ^ (ks << 5)) + kvb * 32 * kRowBytes128;
+    else off = kTile + (k_base ^ ((ks - 8) << 5) ^ (kvb << 7));
+    return *reinterpret_cast<const bf16x8*>(ktile + off);
+  };
+  // 16 keys j, feature block i
+  auto v_frag = [&](const char* vtile, int j, int i) __attribute__((always_inline)) {
+    const int add = kPaired ? (j & 1) * 16 * kRowBytes128 : j * 16 * kRowBytes128;
+    const int flip = kPaired ? (i << 6) | ((j >> 1) << 7) : i << 6;
+    return lds_read_transposed_at(vtile + (v_base[0] ^ flip) + add, vtile + (v_base[1] ^ flip) + add);
+  };
+
+  f32x16 oacc[DVB];
+#pragma unroll
+  for (int i = 0; i < DVB; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
+  float m_run = -INFINITY;
+  float l_run = 0.f;  // this lane's share of the row sum (the partner lane holds the rest)
+  f32x16 s[KVB];       // S^T of one tile: 32 x 32 tiles [keys] x [queries]
+  bf16x8 pf[2 * KVB];  // P^T as B operand, one fragment per 16 keys
+
+  // ---- S^T = K Q^T
+  auto scores = [&](const char* ktile) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[kvb][v] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb) s[kvb] = mfma32(k_frag(ktile, ks, kvb), qf[ks], s[kvb]);
+  };
+
+  // ---- mask, online softmax (one query column per lane pair), P^T fragments
+  auto softmax = [&](int t) __attribute__((always_inline)) {
+    const int n0 = t * kBN;
+    if ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv)) {
+      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int key = n0 + kvb * 32 + acc_row(v, g);
+          if (key > limit) s[kvb][v] = -INFINITY;
+        }
+    }
+    f32x16 e[KVB];
+    float rs = 0.f;
+    // lazily refreshed running maximum, tested on the row sum (attn_fwd_direct.hip)
+    const bool fresh = m_run == -INFINITY;
+    float mk = fresh ? 0.f : m_run * p.kappa;
+#pragma unroll
+    for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        e[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - mk);
+        rs += e[kvb][v];
+      }
+    if (__builtin_amdgcn_ballot_w64(fresh || !(rs <= kRescaleLimit)) != 0) {
+      float x = s[0][0];
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) x = fmaxf(x, s[kvb][v]);
+      const float m_new = fmaxf(m_run, pair_max(x));
+      const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < DVB; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[i][v] *= alpha;
+      mk = (m_run == -INFINITY) ? 0.f : m_run * p.kappa;
+      rs = 0.f;
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          e[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - mk);
+          rs += e[kvb][v];
+        }
+    }
+    l_run += rs;
+#pragma unroll
+    for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) {
+        const f32x16& x16 = e[kvb];
+        pf[2 * kvb + jj] = to_bf16x8(x16[8 * jj], x16[8 * jj + 1], x16[8 * jj + 2], x16[8 * jj + 3], x16[8 * jj + 4],
+                                     x16[8 * jj + 5], x16[8 * jj + 6], x16[8 * jj + 7]);
+      }
+  };
+
+  // ---- O^T += V^T P^T
+  auto accumulate = [&](const char* vtile) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 2 * KVB; ++j)
+#pragma unroll
+      for (int i = 0; i < DVB; ++i) oacc[i] = mfma32(v_frag(vtile, j, i), pf[j], oacc[i]);
+  };
+
+  // both products of an interval, with the fragment reads pinned kAhead products ahead of their use
+  auto matrix_block = [&](const char* vtile, const char* ktile) __attribute__((always_inline)) {
+    constexpr int NPV = 2 * KVB * DVB, NQK = KVB * KS;
+    __builtin_amdgcn_s_setprio(2);
+    bf16x8 av[2 * KVB][DVB], ak[KS][KVB];
+#pragma unroll
+    for (int j = 0; j < 2 * KVB; ++j)
+#pragma unroll
+      for (int i = 0; i < DVB; ++i) av[j][i] = v_frag(vtile, j, i);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb) ak[ks][kvb] = k_frag(ktile, ks, kvb);
+#pragma unroll
+    for (int j = 0; j < 2 * KVB; ++j)
+#pragma unroll
+      for (int i = 0; i < DVB; ++i) oacc[i] = mfma32(av[j][i], pf[j], oacc[i]);
+#pragma unroll
+    for (int kvb = 0; kvb < KVB; ++kvb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[kvb][v] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kvb = 0; kvb < KVB; ++kvb) s[kvb] = mfma32(ak[ks][kvb], qf[ks], s[kvb]);
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAhead, 0);
+#pragma unroll
+    for (int m = 0; m < NPV - kAhead; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < NQK; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  scores(kbuf);
+  softmax(0);
+  __syncthreads();  // K tile 0 has been read: its slot may be refilled
+
+  // interval i: O += V(i)^T P(i), S(i+1) = K(i+1) Q^T, P(i+1); K(i+2) and V(i+1) are requested meanwhile
+  int i = 0;
+  for (; i + 1 < n_tiles_wave; ++i) {
+    if (i + 2 < n_tiles_wg) issue_k(i + 2);
+    issue_v(i + 1);
+    matrix_block(vbuf + (i & 1) * L::kVTile, kbuf + ((i + 1) & 1) * L::kKTile);
+    softmax(i + 1);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+  }
+  for (; i < n_tiles_wg; ++i) {
+    if (i + 2 < n_tiles_wg) issue_k(i + 2);
+    if (i + 1 < n_tiles_wg) issue_v(i + 1);
+    if (i < n_tiles_wave) accumulate(vbuf + (i & 1) * L::kVTile);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+  }
+
+  // ---- epilogue: normalise, store O (bf16) and LSE2; the rings are free (every wave passed the last barrier)
+  __bf16* oh = p.o + b * p.o_bs + (int64_t)h * kDv;
+  float* lse = p.lse + b * p.lse_bs + (int64_t)h * p.lse_hs;
+  const float l = pair_sum(l_run);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  char* const turn = smem + wave * kRowsViaLdsBytes<DVB>;
+  if constexpr (!CAUSAL && kDv == 128) {
+    if (p.prev_o != nullptr) {  // merge with the running result of the rows, as in attn_fwd_direct.hip
+      const float lse_new = l > 0.f ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
+      const float lse_old = qrow < p.Sq ? lse[qrow] : -INFINITY;
+      const float big = fmaxf(lse_old, lse_new);
+      const float w_old = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_old - big);
+      const float w_new = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_new - big);
+      const float den = w_old + w_new;
+      const float rden = den > 0.f ? 1.f / den : 0.f;
+      const int64_t prev_rs = o_row_stride;
+      const char* prev = reinterpret_cast<const char*>(p.prev_o) +
+                         (b * p.prev_bs + (int64_t)h * kDv + q_wave0 * prev_rs) * (p.prev_f32 ? 4 : 2);
+      const bool to_o = p.o && q_wave0 >= p.o_r0 && q_wave0 < p.o_r1;
+      const bool to_acc = p.acc_o && q_wave0 >= p.acc_r0 && q_wave0 < p.acc_r1;
+      merge_rows32_via_lds<DVB>(turn, prev, p.prev_f32 != 0, prev_rs, to_o ? oh + q_wave0 * o_row_stride : nullptr, o_row_stride,
+                                to_acc ? p.acc_o + b * p.acc_bs + (int64_t)h * kDv + q_wave0 * o_row_stride : nullptr,
+                                o_row_stride, p.Sq - q_wave0, oacc, w_new * inv * rden, w_old * rden, lane);
+      if (qrow < p.Sq && g == 0) lse[qrow] = den > 0.f ? big + __builtin_amdgcn_logf(den) : -INFINITY;
+      return;
+    }
+  }
+  store_rows32_via_lds<__bf16, DVB>(turn, oh + q_wave0 * o_row_stride, o_row_stride, p.Sq - q_wave0, oacc, inv, false, lane);
+  if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
+}
+
+template <int DQK>
+void launch_one(FwdParams p, bool causal, hipStream_t st) {
+  p.m_tiles = (p.Sq + kBM - 1) / kBM;
+  const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
+  if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false>), grid, block, 0, st, p);
+}
+
+}  // namespace
+
+void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t st) {
+  if (dqk == 64) launch_one<64>(p, causal, st);
+  else if (dqk == 128) launch_one<128>(p, causal, st);
+  else launch_one<192>(p, causal, st);
+}
+
+}  // namespace pith

@@ -280,6 +280,35 @@ struct DirectExtra64 {
   }
 };
 
+// The same for a workgroup of THREADS threads, and for whole 64-feature operands: wave w fills LDS rows
+// 4w + 4*WAVES*n .. +3, and with 4 * WAVES a multiple of 16 the swizzle (hence the source offset) of a lane does not
+// depend on n.
+template <int THREADS>
+struct DirectPaired64 {
+  static constexpr int kWaves = THREADS / 64;
+  static constexpr int kPerThread = 32 / (4 * kWaves);
+  static_assert(32 % (4 * kWaves) == 0 && (4 * kWaves) % 16 == 0, "rows of successive pieces must share their swizzle");
+  int src_off, row_bytes, col_bytes;
+  __device__ __forceinline__ void init(int row_bytes_, int col_bytes_, int wave, int lane) {
+    row_bytes = row_bytes_;
+    col_bytes = col_bytes_;
+    src_off = DirectExtra64::source(row_bytes_, col_bytes_, wave, lane, 64);
+  }
+  __device__ __forceinline__ void issue(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
+    if (rows_left >= 64) {
+      int off = src_off;
+      asm volatile("" : "+v"(off));  // pinned before the first load, see DirectTile128::issue
+#pragma unroll
+      for (int n = 0; n < kPerThread; ++n)
+        load_lds16(tile_src + (int64_t)n * 4 * kWaves * row_bytes, off, slot + (n * kWaves + wave) * 1024);
+    } else {
+#pragma unroll
+      for (int n = 0; n < kPerThread; ++n)
+        load_lds16(tile_src, DirectExtra64::source(row_bytes, col_bytes, n * kWaves + wave, lane, rows_left), slot + (n * kWaves + wave) * 1024);
+    }
+  }
+};
+
 // Per-lane offsets for reading a packed swizzled tile.
 // straight_offset(c, piece): fragment of row c (+ a multiple of 16 rows added by the caller as
 // rows * 256 bytes), features 8*piece .. 8*piece+7.

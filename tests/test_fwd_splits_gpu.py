@@ -1,0 +1,45 @@
+"""The forward's work splits on both sides of every line of its dispatch, and at the edges of the two-workgroup kernel's tiles,
+against plain fp32 PyTorch."""
+
+import pytest
+import torch
+
+from helpers import check_bf16_result, check_lse
+from pithtrain_amd.operators.mla.hip import _mla_fwd
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, scale, causal):
+    """O and base-2 LSE in fp32, one query head at a time."""
+    b, sq, hq, _ = q.shape
+    group = hq // k.shape[2]
+    o = torch.empty(b, sq, hq, v.shape[-1], device=q.device)
+    lse = torch.empty(b, hq, sq, device=q.device)
+    mask = torch.ones(sq, k.shape[1], dtype=torch.bool, device=q.device).triu(1) if causal else None
+    for bi in range(b):
+        for h in range(hq):
+            s = (q[bi, :, h].float() @ k[bi, :, h // group].float().t().contiguous()) * scale
+            if causal:
+                s.masked_fill_(mask, float("-inf"))
+            lse[bi, h] = torch.logsumexp(s, -1) / 0.6931471805599453
+            o[bi, :, h] = torch.softmax(s, -1) @ v[bi, :, h // group].float()
+    return o, lse
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D,causal", [
+    # two-workgroup kernel: one row, tile and wave edges, ragged keys
+    (1, 1, 1, 2, 1, 64, True), (1, 33, 33, 2, 2, 64, True), (2, 129, 129, 4, 2, 64, True), (1, 70, 200, 4, 1, 64, False),
+    (1, 640, 640, 4, 4, 64, True), (1, 127, 127, 2, 1, 128, True), (1, 65, 257, 4, 2, 128, False), (1, 512, 512, 2, 2, 192, True),
+    # 256 / 257 and 512 / 513 workgroups of 128 rows; streams of 512 / 513, 1024 / 1025, 1535 / 1536 keys
+    (1, 512, 512, 16, 4, 128, False), (1, 513, 513, 16, 4, 128, False), (1, 520, 520, 52, 4, 128, True), (1, 896, 1025, 37, 37, 128, False),
+    (1, 896, 1024, 37, 37, 128, False), (1, 1535, 1535, 42, 2, 192, True), (1, 1536, 1536, 42, 2, 192, True), (1, 3072, 3072, 22, 2, 128, True),
+])  # fmt: skip
+def test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+    g = torch.Generator(device=gpu).manual_seed(9)
+    mk = lambda s, h, d: torch.randn(B, s, h, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(Sq, Hq, D), mk(Skv, Hkv, D), mk(Skv, Hkv, min(D, 128))
+    o, lse = _mla_fwd(q, k, v, D**-0.5, causal)
+    ref_o, ref_lse = _reference(q, k, v, D**-0.5, causal)
+    check_bf16_result(o, ref_o, "O")
+    check_lse(lse, ref_lse, "LSE2")
