@@ -181,18 +181,21 @@ __device__ __forceinline__ void decode_dkdv_block(int linear, int per_level, int
 
 // dK/dV kernels: a workgroup owns kDkdvBlockN key rows (the grid and the head split depend on it).
 constexpr int kDkdvBlockN = 128;
+// dK/dV for head dims (64, 64): attn_bwd_dkdv_d64.hip. Conventions as below.
+void launch_dkdv_d64(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
+
 // dK/dV for head dims (128, 128): attn_bwd_dkdv_d128.hip. p.tiles, p.split, p.ws_* are set by the caller.
 void launch_dkdv_d128(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
 
 // dK/dV for head dims (192, 128): attn_bwd_dkdv_d192.hip. Same conventions.
 void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
 
-// dQ for head dims (128, 128): attn_bwd_dq_d128.hip. p.tiles = number of 256-row query tiles.
-void launch_dq_d128(const BwdParams& p, bool causal, bool f32_out, hipStream_t stream);
-
-// dQ for head dims (128, 128) and (192, 128) with 128-row workgroups, early / late wave roles:
-// attn_bwd_dq_direct.hip. p.tiles = number of 128-row query tiles.
+// dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
+// split every tile's keys: attn_bwd_dq_direct.hip.
 void launch_dq_direct(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t stream);
+
+// dQ with two 4-wave workgroups of 128 query rows per compute unit, all head dims: attn_bwd_dq_duo.hip.
+void launch_dq_duo(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t stream);
 
 // dQ for head dims (128, 128) from the dS images the dK/dV kernel left in p.ds: attn_bwd_dq_ds.hip.
 // p.tiles = number of 512-row query tiles.

@@ -1,27 +1,6 @@
-// Key/value-gradient kernel of one chunk attention backward for gfx950 with register-staged tiles
-// (used for head dims 64/64; 128/128 and 192/128 have direct-load kernels of their own), the entry
-// points of the dK/dV step and the reduction kernel of the head split; against an external
-// (ring-combined) base-2 LSE and delta = rowsum(O*dO). Follows
-// pithtrain/operators/mla/triton.py:130-197 (non-causal :331-384): P = exp2(kappa*s - lse2) in
-// fp32, masked entries 0, P rounded to bf16 for dV += P^T dO, dS = P*(dP - delta)*scale rounded
-// to bf16 for dK += dS^T Q, fp32 accumulation.
-//
-// Work split. A workgroup of 8 wavefronts owns 128 key rows of one (batch, kv head) and loops
-// over query tiles of 32 rows of the query heads assigned to it. The 8 wavefronts form 4 PAIRS,
-// one per 32 key rows; the two waves of a pair share a SIMD and split the work so that each
-// stays below 256 registers (two waves per SIMD, no accumulator spills):
-//     wave A:  S = Q K^T  ->  P = exp2(kappa*S - lse)  ->  dV^T += dO^T P      (holds K, dV)
-//     wave B:  dP = dO V^T ->  dS = P o (dP - delta) * scale -> dK^T += Q^T dS (holds V, dK)
-// B needs A's P: A leaves the fp32 P tile (32 x 32) in an LDS exchange buffer, in the lane order
-// both waves share, and B picks it up after the iteration's only barrier. Both waves issue the
-// same number of MFMAs.
-// The stationary side (K or V rows) sits in registers as B operands, so score tiles have the key
-// index as their column; P / dS then feed the products that contract over queries straight from
-// registers (slot order, see attn_tiles.h) with dO^T / Q^T read transposed from LDS.
-//
-// Query tiles stream through a 3-deep LDS ring: the tile for iteration i+1 is committed while
-// iteration i computes and becomes visible at iteration i's barrier, its buffer having been
-// released by the previous barrier. Global loads run two tiles ahead.
+// Entry points of the key/value-gradient step of one chunk attention backward for gfx950, against an external
+// (ring-combined) base-2 LSE and delta = rowsum(O*dO): argument checks, the head split and its reduction kernel. The
+// kernels are attn_bwd_dkdv_d64.hip, attn_bwd_dkdv_d128.hip and attn_bwd_dkdv_d192.hip.
 //
 // With grouped-query attention the heads of a group may be cut into `split` parts handled by
 // different workgroups (more parallelism when there are few key tiles); the parts leave fp32
@@ -34,245 +13,7 @@
 namespace pith {
 namespace {
 
-constexpr int kThreads = 512;
-constexpr int kBM = 32;    // query rows per tile
 constexpr int kBN = kDkdvBlockN;  // key rows per workgroup
-constexpr int kStages = 3;
-
-template <int DQK, int DV>
-struct DkdvLayout {
-  static constexpr int QP = DQK * 2 + 80;  // tiles are read straight by one wave of a pair, transposed by the other
-  static constexpr int OP = DV * 2 + 80;
-  static constexpr int kQTile = kBM * QP;
-  static constexpr int kOTile = kBM * OP;
-  static constexpr int kStat = 2 * kBM * 4;  // lse[32], delta[32]
-  static constexpr int kStage = kQTile + kOTile + kStat;
-  static constexpr int kExch = 4 * 2 * 4096;  // [pair][parity][32 x 32 fp32]
-  static constexpr int kTotal = kStages * kStage + kExch;
-};
-
-// One wave's loop. ROLE_B = false: wave A (T1 = Q tile, stationary K, out dV). ROLE_B = true:
-// wave B (T1 = dO tile, stationary V, out dK). KDIM = contraction length of the score-type
-// product, ODIM = feature length of the gradient this wave accumulates.
-template <int DQK, int DV, bool CAUSAL, bool ROLE_B, typename Fetch, typename Commit>
-__device__ __forceinline__ void dkdv_wave_loop(const BwdParams& p, char* smem, int lane, int pair, int kv_pair0, int n_iter,
-                                               int m_end, int m_start_wg, const bf16x8* stat,
-                                               f32x16* acc, Fetch& fetch, Commit& commit) {
-  using L = DkdvLayout<DQK, DV>;
-  constexpr int KDIM = ROLE_B ? DV : DQK;
-  constexpr int ODIM = ROLE_B ? DQK : DV;
-  constexpr int T1P = ROLE_B ? L::OP : L::QP;   // pitch of the tile read straight
-  constexpr int T2P = ROLE_B ? L::QP : L::OP;   // pitch of the tile read transposed
-  constexpr int T1_OFF = ROLE_B ? L::kQTile : 0;
-  constexpr int T2_OFF = ROLE_B ? 0 : L::kQTile;
-  const int c = lane & 31, g = lane >> 5;
-  const int key = kv_pair0 + c;
-  const int m_start_pair = CAUSAL ? kv_pair0 / kBM : 0;
-  char* exch = smem + kStages * L::kStage + pair * 8192;
-
-  // Ring stages rotate (prev <- cur <- next <- prev) and the tile position advances by increments:
-  // no division or modulo in the loop. The body has no branch around its matrix instructions (a
-  // tile entirely above this pair's diagonal is processed like any other, its P is all zeros), so
-  // the accumulators stay in place from one iteration to the next.
-  int off_prev = 2 * L::kStage, off_cur = 0, off_next = L::kStage;
-  int mt = m_start_wg;
-  for (int i = 0; i < n_iter; ++i) {
-    if (i + 1 < n_iter) commit(off_next);
-    if (i + 2 < n_iter) fetch();
-    const char* stage = smem + off_cur;
-    const float* stats = reinterpret_cast<const float*>(stage + L::kQTile + L::kOTile);
-    const int q0 = mt * kBM;
-
-    f32x16 x;
-    bf16x8 frag[2];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) x[v] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KDIM / 16; ++ks) {
-      const bf16x8 a = lds_read_straight(stage + T1_OFF, T1P, c, ks * 16 + g * 8);
-      x = mfma32(a, stat[ks], x);
-    }
-    if (!ROLE_B) {
-      // rows of the tile are queries q0 + acc_row(v, g); this lane's column is `key`
-      f32x4 l4[4];
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) l4[b4] = *reinterpret_cast<const f32x4*>(stats + 8 * b4 + 4 * g);
-#pragma unroll
-      for (int v = 0; v < 16; ++v) x[v] = __builtin_amdgcn_exp2f(x[v] * p.kappa - l4[v >> 2][v & 3]);
-      if ((CAUSAL && mt <= m_start_pair) || (q0 + kBM > p.Sq)) {  // wave-uniform
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int qrow = q0 + acc_row(v, g);
-          if ((CAUSAL && key > qrow) || qrow >= p.Sq) x[v] = 0.f;
-        }
-      }
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        const f32x4 pr = {x[4 * b4], x[4 * b4 + 1], x[4 * b4 + 2], x[4 * b4 + 3]};
-        *reinterpret_cast<f32x4*>(exch + (i & 1) * 4096 + (b4 * 64 + lane) * 16) = pr;
-      }
-    }
-    __syncthreads();
-    if (ROLE_B) {
-      const float* delta_s = stats + kBM;
-      f32x4 pr[4], d4[4];
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        pr[b4] = *reinterpret_cast<const f32x4*>(exch + (i & 1) * 4096 + (b4 * 64 + lane) * 16);
-        d4[b4] = *reinterpret_cast<const f32x4*>(delta_s + 8 * b4 + 4 * g);
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) x[v] = pr[v >> 2][v & 3] * (x[v] - d4[v >> 2][v & 3]) * p.scale;
-    }
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-      frag[jj] = to_bf16x8(x[8 * jj], x[8 * jj + 1], x[8 * jj + 2], x[8 * jj + 3], x[8 * jj + 4], x[8 * jj + 5],
-                           x[8 * jj + 6], x[8 * jj + 7]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int o = 0; o < ODIM / 32; ++o) {
-        const bf16x8 a = lds_read_transposed(stage + T2_OFF, T2P, 16 * j, 32 * o, lane);
-        acc[o] = mfma32(a, frag[j], acc[o]);
-      }
-    const int t = off_prev;
-    off_prev = off_cur;
-    off_cur = off_next;
-    off_next = t;
-    if (++mt == m_end) mt = m_start_wg;
-  }
-}
-
-template <int DQK, int DV, bool CAUSAL, typename OutT>
-__global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_kernel(BwdParams p) {
-  using L = DkdvLayout<DQK, DV>;
-  constexpr int KS = DQK / 16, VS = DV / 16, DB = DQK / 32, DVB = DV / 32;
-  constexpr int NSTAT = KS > VS ? KS : VS, NACC = DB > DVB ? DB : DVB;
-  __shared__ __attribute__((aligned(16))) char smem[L::kTotal];
-
-  const int tid = threadIdx.x;
-  if ((int)blockIdx.x >= p.main_blocks) {  // workgroups appended to the grid: clear the rows behind the chunk's visible part
-    zero_tail_block<OutT>(p, (int)blockIdx.x - p.main_blocks, DQK, DV, tid, kThreads);
-    return;
-  }
-  const int lane = tid & 63, wave = tid >> 6;
-  const int c = lane & 31, g = lane >> 5;
-  const int pair = wave & 3;
-  const bool role_b = wave >= 4;
-
-  // linear block id -> (key tile, kv head, batch, head part)
-  const int per_level = p.Hkv * p.B * p.split;
-  int n_tile, pos;
-  decode_dkdv_block(blockIdx.x, per_level, p.tiles, n_tile, pos);
-  const int part = pos % p.split;
-  pos /= p.split;
-  const int hk = pos % p.Hkv, b = pos / p.Hkv;
-  const int heads_per_part = p.group / p.split;
-  const int hq0 = hk * p.group + part * heads_per_part;
-
-  const int kv_wg0 = n_tile * kBN;
-  const int kv_pair0 = kv_wg0 + pair * 32;
-  const int key = kv_pair0 + c;
-
-  const int64_t q_row_stride = (int64_t)p.HqT * DQK;
-  const int64_t do_row_stride = (int64_t)p.HqT * DV;
-  const int k_head = DQK;
-  const int64_t k_row_stride = (int64_t)p.HkvT * k_head;
-  const int64_t v_row_stride = (int64_t)p.HkvT * DV;
-
-  // stationary fragments: K rows for wave A, V rows for wave B
-  bf16x8 stat[NSTAT];
-  {
-    const int row = key < p.Skv ? key : p.Skv - 1;
-    if (!role_b) {
-      const __bf16* src = p.k + b * p.k_bs + row * k_row_stride + (int64_t)hk * k_head + g * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) stat[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    } else {
-      const __bf16* src = p.v + b * p.v_bs + row * v_row_stride + (int64_t)hk * DV + g * 8;
-#pragma unroll
-      for (int ks = 0; ks < VS; ++ks) stat[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    }
-  }
-  f32x16 acc[NACC];
-#pragma unroll
-  for (int i = 0; i < NACC; ++i)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
-
-  // Query tiles to visit: all of them, or from the diagonal down under the causal mask.
-  const int m_tiles_all = (p.Sq + kBM - 1) / kBM;
-  const int m_start_wg = CAUSAL ? min(kv_wg0 / kBM, m_tiles_all) : 0;
-  const int n_m = m_tiles_all - m_start_wg;
-  const int n_iter = n_m * heads_per_part;
-
-  TileCopy<kBM, DQK, L::QP, kThreads> qcopy;
-  TileCopy<kBM, DV, L::OP, kThreads> ocopy;
-  float stat_val = 0.f;  // threads 0..31 carry lse, 32..63 carry delta of the tile's rows
-  int fetch_hq = hq0, fetch_mt = m_start_wg;  // position of the next tile to fetch
-  auto fetch = [&]() {
-    const int hq = fetch_hq, mt = fetch_mt;
-    if (++fetch_mt == m_tiles_all) {
-      fetch_mt = m_start_wg;
-      ++fetch_hq;
-    }
-    qcopy.fetch(p.q + b * p.q_bs + (int64_t)hq * DQK, q_row_stride, mt * kBM, p.Sq, tid);
-    ocopy.fetch(p.dout + b * p.dout_bs + (int64_t)hq * DV, do_row_stride, mt * kBM, p.Sq, tid);
-    if (tid < 2 * kBM) {
-      int row = mt * kBM + (tid & (kBM - 1));
-      row = row < p.Sq ? row : p.Sq - 1;
-      const float* src = (tid < kBM ? p.lse : p.delta) + b * p.lse_bs + (int64_t)hq * p.lse_hs;
-      stat_val = src[row];
-    }
-  };
-  auto commit = [&](int stage_off) {
-    char* base = smem + stage_off;
-    qcopy.commit(base, tid);
-    ocopy.commit(base + L::kQTile, tid);
-    if (tid < 2 * kBM) reinterpret_cast<float*>(base + L::kQTile + L::kOTile)[tid] = stat_val;
-  };
-
-  if (n_iter > 0) {
-    fetch();
-    commit(0);
-    if (n_iter > 1) fetch();
-  }
-  wait_all_vector_loads();
-  __syncthreads();
-
-  if (!role_b)
-    dkdv_wave_loop<DQK, DV, CAUSAL, false>(p, smem, lane, pair, kv_pair0, n_iter, m_tiles_all, m_start_wg, stat, acc, fetch, commit);
-  else
-    dkdv_wave_loop<DQK, DV, CAUSAL, true>(p, smem, lane, pair, kv_pair0, n_iter, m_tiles_all, m_start_wg, stat, acc, fetch, commit);
-
-  // ---- epilogue: wave A stores dV, wave B stores dK, for key row `key`, features 32*o + 8*b4 + 4*g ..+3
-  if (key < p.Skv) {
-    const int d = role_b ? k_head : DV;
-    const int nblk = role_b ? k_head / 32 : DVB;
-    const int64_t row_stride = role_b ? k_row_stride : v_row_stride;
-    if (p.split > 1) {
-      float* ws = (role_b ? p.ws_dk : p.ws_dv) +
-                  (((int64_t)part * p.B + b) * p.Skv + key) * ((int64_t)p.Hkv * d) + (int64_t)hk * d;  // partials are packed
-#pragma unroll
-      for (int o = 0; o < NACC; ++o)
-        if (o < nblk)
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4)
-            store4<float>(ws + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4], acc[o][4 * b4 + 1], acc[o][4 * b4 + 2],
-                          acc[o][4 * b4 + 3], false);
-    } else {
-      OutT* out = reinterpret_cast<OutT*>(role_b ? p.dk : p.dv) + b * (role_b ? p.dk_bs : p.dv_bs) + key * row_stride +
-                  (int64_t)hk * d;
-#pragma unroll
-      for (int o = 0; o < NACC; ++o)
-        if (o < nblk)
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4)
-            store4<OutT>(out + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4], acc[o][4 * b4 + 1], acc[o][4 * b4 + 2],
-                         acc[o][4 * b4 + 3], p.accumulate != 0);
-    }
-  }
-}
 
 // out[b, s, h, :] (+)= sum over parts of ws[part][b][s][h][:], parts added in index order; dK
 // (blockIdx.y = 0) and dV (blockIdx.y = 1) in one launch.
@@ -308,9 +49,11 @@ int pick_split(const pith_attn_bwd_args* a) {
   const int64_t group = a->Hq / a->Hkv;
   const int64_t base = ((a->Skv + kBN - 1) / kBN) * a->Hkv * a->B;
   int split = 1;
-  // one workgroup per compute unit is resident; without a causal mask all workgroups carry the same
-  // work, so one full round is ideal; under the mask two rounds (heaviest first) balance better
-  const int64_t want = (a->causal ? 2 : 1) * (int64_t)compute_units_or_default();
+  // Workgroups wanted. Without a causal mask all of them carry the same work, so one full round is ideal; under the mask
+  // two rounds (heaviest first) balance better. At 64 features two workgroups share a compute unit and twice as many are
+  // wanted (8192 rows x 32 heads causal: 757 us with 512 workgroups, 560 us with 1024; without a mask 512 and 1024 are
+  // within 2 %).
+  const int64_t want = (a->causal ? 2 : 1) * (a->Dqk == 64 ? 2 : 1) * (int64_t)compute_units_or_default();
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
   return split;
 }
@@ -334,22 +77,16 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, hipStream_t st) {
   p.accumulate = a->accumulate_dkv;
   p.main_blocks = (int)(p.tiles * a->Hkv * a->B * p.split);
   p.zero_tail = a->accumulate_dkv ? 0 : (int)a->dkv_zero_tail;  // rows that are added to keep what they hold
-  const dim3 grid((unsigned)(p.main_blocks + (p.zero_tail + kZeroTailRows - 1) / kZeroTailRows)), block(kThreads);
+  const unsigned grid = (unsigned)(p.main_blocks + (p.zero_tail + kZeroTailRows - 1) / kZeroTailRows);
   const bool f32 = a->dkv_dtype == PITH_F32;
   if constexpr (DQK == 128 && DV == 128) {
     // descending walk under the mask when Q and dO together exceed what the last-level cache (256 MB) keeps
     p.walk_desc = a->causal != 0 && (int64_t)a->B * a->Sq * a->Hq * (DQK + DV) * 2 > kWalkDescBytes;
-    launch_dkdv_d128(p, a->causal != 0, f32, grid.x, st);
+    launch_dkdv_d128(p, a->causal != 0, f32, grid, st);
   } else if constexpr (DQK == 192 && DV == 128) {
-    launch_dkdv_d192(p, a->causal != 0, f32, grid.x, st);
+    launch_dkdv_d192(p, a->causal != 0, f32, grid, st);
   } else {
-    if (a->causal) {
-      if (f32) hipLaunchKernelGGL((attn_bwd_dkdv_kernel<DQK, DV, true, float>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((attn_bwd_dkdv_kernel<DQK, DV, true, __bf16>), grid, block, 0, st, p);
-    } else {
-      if (f32) hipLaunchKernelGGL((attn_bwd_dkdv_kernel<DQK, DV, false, float>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((attn_bwd_dkdv_kernel<DQK, DV, false, __bf16>), grid, block, 0, st, p);
-    }
+    launch_dkdv_d64(p, a->causal != 0, f32, grid, st);
   }
   if (p.k_pe) {  // dk_pe (+)= sum over heads, in head order
     ReduceParams r;

@@ -1,234 +1,27 @@
-// Query-gradient kernel of one chunk attention backward for gfx950, against an external
-// (ring-combined) base-2 LSE and delta = rowsum(O*dO); plus the argument checks shared with the
-// dK/dV kernel. Follows pithtrain/operators/mla/triton.py:205-266 (non-causal :392-441):
-// P = exp2(kappa*s - lse2) in fp32, masked entries 0, dS = P*(dP - delta)*scale rounded to bf16,
-// fp32 accumulation of dQ += dS K.
-//
-// The query side is stationary in registers as B operands (a lane owns one query row), K/V tiles
-// stream through LDS as A operands, and the score tile is produced with the query index as its
-// COLUMN: lse and delta are then per-lane scalars and dS^T feeds dQ^T += K^T dS^T from registers
-// (slot order, see attn_tiles.h) with K^T coming from transposing LDS reads.
+// Entry point of the query-gradient step of one chunk attention backward for gfx950 (against an external, ring-combined
+// base-2 LSE and delta = rowsum(O*dO)): argument checks shared with the dK/dV step and the choice of a kernel. Numerics of
+// all kernels follow pithtrain/operators/mla/triton.py:205-266 (non-causal :392-441).
 #include "attn_bwd_common.h"
 
 namespace pith {
 namespace {
 
-// =============================================================================================
-// dQ kernel. Workgroup = WAVES wavefronts x (32*QB) query rows of one (batch, head); key tiles of
-// 32*NB keys. With QB = NB = 1 a wavefront stays below 256 registers and two share a SIMD. Per tile: S^T = K Q^T, dP^T = V dO^T, dS^T = P^T o (dP^T - delta) * scale,
-// dQ^T += K^T dS^T.
-template <int DQK, int DV, bool CAUSAL, int QB, int NB, int WAVES, typename OutT>
-__global__ __launch_bounds__(WAVES * 64) void attn_bwd_dq_kernel(BwdParams p) {
-  constexpr int THREADS = WAVES * 64;
-  constexpr int KS = DQK / 16, VS = DV / 16, DB = DQK / 32;
-  constexpr int BN = 32 * NB;
-  constexpr int ROWS_WAVE = 32 * QB, BM = WAVES * ROWS_WAVE;
-  constexpr int KP = DQK * 2 + 80;  // read straight and transposed
-  constexpr int VP = DV * 2 + 16;   // read straight only
-  constexpr int kKTile = BN * KP, kVTile = BN * VP;
-  __shared__ __attribute__((aligned(16))) char smem[2 * (kKTile + kVTile)];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int c = lane & 31, g = lane >> 5;
-  int m_tile, h, b;
-  decode_block(blockIdx.x, p.Hq, p.B, p.tiles, p.group, m_tile, h, b);
-  const int hk = h / p.group;
-  const int m0 = m_tile * BM;
-  const int q_wave0 = m0 + wave * ROWS_WAVE;
-
-  const int64_t q_row_stride = (int64_t)p.HqT * DQK;
-  const int64_t do_row_stride = (int64_t)p.HqT * DV;
-  const int64_t k_row_stride = (int64_t)p.HkvT * DQK;
-  const int64_t v_row_stride = (int64_t)p.HkvT * DV;
-  const __bf16* qh = p.q + b * p.q_bs + (int64_t)h * DQK;
-  const __bf16* doh = p.dout + b * p.dout_bs + (int64_t)h * DV;
-  const __bf16* kh = p.k + b * p.k_bs + (int64_t)hk * DQK;
-  const __bf16* vh = p.v + b * p.v_bs + (int64_t)hk * DV;
-  const float* lse = p.lse + b * p.lse_bs + (int64_t)h * p.lse_hs;
-  const float* delta = p.delta + b * p.lse_bs + (int64_t)h * p.lse_hs;
-
-  bf16x8 qf[QB][KS], dof[QB][VS];
-  float lse_q[QB], delta_q[QB];
-#pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    int row = q_wave0 + qb * 32 + c;
-    row = row < p.Sq ? row : p.Sq - 1;
-    const __bf16* src = qh + row * q_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    const __bf16* dsrc = doh + row * do_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < VS; ++ks) dof[qb][ks] = *reinterpret_cast<const bf16x8*>(dsrc + ks * 16);
-    lse_q[qb] = lse[row];
-    delta_q[qb] = delta[row];
-  }
-
-  f32x16 acc[DB][QB];
-#pragma unroll
-  for (int i = 0; i < DB; ++i)
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][qb][v] = 0.f;
-
-  const int n_tiles_all = (p.Skv + BN - 1) / BN;
-  int n_tiles_wg = n_tiles_all;
-  if (CAUSAL) n_tiles_wg = min(n_tiles_all, (m0 + BM - 1) / BN + 1);
-
-  TileCopy<BN, DQK, KP, THREADS> kcopy;
-  TileCopy<BN, DV, VP, THREADS> vcopy;
-  kcopy.fetch(kh, k_row_stride, 0, p.Skv, tid);
-  vcopy.fetch(vh, v_row_stride, 0, p.Skv, tid);
-  kcopy.commit(smem, tid);
-  vcopy.commit(smem + kKTile, tid);
-  wait_all_vector_loads();
-  __syncthreads();
-
-  for (int t = 0; t < n_tiles_wg; ++t) {
-    const char* ktile = smem + (t & 1) * (kKTile + kVTile);
-    const char* vtile = ktile + kKTile;
-    const bool have_next = t + 1 < n_tiles_wg;
-    if (have_next) {
-      kcopy.fetch(kh, k_row_stride, (t + 1) * BN, p.Skv, tid);
-      vcopy.fetch(vh, v_row_stride, (t + 1) * BN, p.Skv, tid);
-    }
-
-    // No branch around the matrix instructions: a wave whose rows lie entirely above this tile
-    // under the causal mask processes it like any other (its P is all zeros), which keeps the
-    // accumulators in place across iterations; the workgroup waits for its last wave anyway.
-    {
-      f32x16 s[NB][QB], dp[NB][QB];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            s[nb][qb][v] = 0.f;
-            dp[nb][qb][v] = 0.f;
-          }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const bf16x8 a = lds_read_straight(ktile, KP, nb * 32 + c, ks * 16 + g * 8);
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) s[nb][qb] = mfma32(a, qf[qb][ks], s[nb][qb]);
-        }
-#pragma unroll
-      for (int ks = 0; ks < VS; ++ks)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const bf16x8 a = lds_read_straight(vtile, VP, nb * 32 + c, ks * 16 + g * 8);
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) dp[nb][qb] = mfma32(a, dof[qb][ks], dp[nb][qb]);
-        }
-
-      const int n0 = t * BN;
-      const bool masked = (CAUSAL && (n0 + BN - 1 > q_wave0)) || (n0 + BN > p.Skv);  // wave-uniform
-      bf16x8 dsf[QB][2 * NB];
-      // With registers to spare (small head dims) the mask is a pass of its own under the
-      // wave-uniform branch, which saves a compare and a select per element on unmasked tiles;
-      // at 192/128 that version spills, and the test stays inside the element loop.
-      constexpr bool kMaskPass = DQK + DV <= 192;
-      if (kMaskPass) {
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) s[nb][qb][v] = __builtin_amdgcn_exp2f(s[nb][qb][v] * p.kappa - lse_q[qb]);
-        if (masked) {
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            const int qrow = q_wave0 + qb * 32 + c;
-            const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-              for (int v = 0; v < 16; ++v)
-                if (n0 + nb * 32 + acc_row(v, g) > limit) s[nb][qb][v] = 0.f;
-          }
-        }
-      }
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        const int qrow = q_wave0 + qb * 32 + c;
-        const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            float pr = s[nb][qb][v];
-            if (!kMaskPass) {
-              pr = __builtin_amdgcn_exp2f(pr * p.kappa - lse_q[qb]);
-              if (masked && (n0 + nb * 32 + acc_row(v, g) > limit)) pr = 0.f;
-            }
-            s[nb][qb][v] = pr * (dp[nb][qb][v] - delta_q[qb]) * p.scale;
-          }
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) {
-            const f32x16& x = s[nb][qb];
-            dsf[qb][2 * nb + jj] = to_bf16x8(x[8 * jj], x[8 * jj + 1], x[8 * jj + 2], x[8 * jj + 3], x[8 * jj + 4],
-                                             x[8 * jj + 5], x[8 * jj + 6], x[8 * jj + 7]);
-          }
-        }
-      }
-
-#pragma unroll
-      for (int j = 0; j < 2 * NB; ++j)
-#pragma unroll
-        for (int i = 0; i < DB; ++i) {
-          const bf16x8 a = lds_read_transposed(ktile, KP, 16 * j, 32 * i, lane);
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) acc[i][qb] = mfma32(a, dsf[qb][j], acc[i][qb]);
-        }
-    }
-
-    if (have_next) {
-      char* nk = smem + ((t + 1) & 1) * (kKTile + kVTile);
-      kcopy.commit(nk, tid);
-      vcopy.commit(nk + kKTile, tid);
-    }
-    __syncthreads();
-  }
-
-  OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK;
-#pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    const int qrow = q_wave0 + qb * 32 + c;
-    if (qrow < p.Sq) {
-      OutT* dst = dqh + qrow * q_row_stride;
-#pragma unroll
-      for (int i = 0; i < DB; ++i)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4)
-          store4<OutT>(dst + 32 * i + 8 * b4 + 4 * g, acc[i][qb][4 * b4], acc[i][qb][4 * b4 + 1],
-                       acc[i][qb][4 * b4 + 2], acc[i][qb][4 * b4 + 3], p.accumulate != 0);
-    }
-  }
-}
-
-template <int DQK, int DV, int QB, int NB, int WAVES>
-void launch_dq(BwdParams p, const pith_attn_bwd_args* a, hipStream_t st) {
-  constexpr int BM = WAVES * 32 * QB;
-  p.tiles = (int)((a->Sq + BM - 1) / BM);
-  p.accumulate = a->accumulate_dq;
-  const dim3 grid((unsigned)(p.tiles * a->Hq * a->B)), block(WAVES * 64);
-  const bool f32 = a->dq_dtype == PITH_F32;
-  if constexpr (DQK == 128 && DV == 128) {
-    static_assert(BM == 256, "the 128-dim kernel owns 256 query rows per workgroup");
-    launch_dq_d128(p, a->causal != 0, f32, st);
-  } else {
-    if (a->causal) {
-      if (f32) hipLaunchKernelGGL((attn_bwd_dq_kernel<DQK, DV, true, QB, NB, WAVES, float>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((attn_bwd_dq_kernel<DQK, DV, true, QB, NB, WAVES, __bf16>), grid, block, 0, st, p);
-    } else {
-      if (f32) hipLaunchKernelGGL((attn_bwd_dq_kernel<DQK, DV, false, QB, NB, WAVES, float>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((attn_bwd_dq_kernel<DQK, DV, false, QB, NB, WAVES, __bf16>), grid, block, 0, st, p);
-    }
-  }
+// Recomputing dQ kernels: 128-row workgroups either way. Two 4-wave workgroups per compute unit (attn_bwd_dq_duo.hip), or
+// one of 8 waves whose pairs split every tile's keys (attn_bwd_dq_direct.hip, "half"). Measured, microseconds:
+//                                              duo    half
+//   d128  1 x 4096 x 32 heads causal           176    197        d192  1 x 4096 x 128 heads causal     1105   1210
+//         1 x 2048 x 32, 512 WGs, causal       65     58               1 x 4096 x 16, 512 WGs, causal  179    136
+//         1 x 1024 x 32, 256 WGs, no mask      32     30               2048 x 4096 x 16, 256 WGs       139    120
+//         1 x 1536 x 32, 384 WGs, no mask      56     69               4096 x 2048 x 16, 512 WGs       119    130
+//         1 x 256 x 32                         12.1   12.7             1 x 256 x 16                    15.9   16.4
+// So the split keys pay where a workgroup has its compute unit to itself: grids of up to one workgroup per unit, and under
+// the mask, where the heavy half of the workgroups ends up alone, of up to two for long streams (the same lines as in the
+// forward). 64 features always use duo (three workgroups fit a unit; no split-key kernel exists).
+bool use_split_keys(const pith_attn_bwd_args* a) {
+  if (a->Dqk == 64) return false;
+  const int64_t cus = compute_units_or_default();
+  const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
+  return wgs <= cus ? a->Skv > 256 : a->causal && wgs <= 2 * cus && a->Skv >= 1536;
 }
 
 }  // namespace
@@ -354,23 +147,10 @@ extern "C" int pith_attn_bwd_dq(const pith_attn_bwd_args* a, pith_stream_t strea
     launch_dq_from_ds(q, a->causal != 0, a->dq_dtype == PITH_F32, st);
     return check_launch("pith_attn_bwd_dq");
   }
-  const bool half = a->Dqk == 192 || prefer_half_rows(a->Sq, a->Hq, a->B, a->causal != 0);
-  if (a->Dqk == 192 || (a->Dqk == 128 && half)) {
-    // early / late wave roles with 128-row workgroups whose wave pairs split every tile's keys: the
-    // only direct-load form for 192-feature queries, and the better one for 128 features when
-    // 256-row workgroups would leave compute units idle
-    BwdParams q = p;
-    q.tiles = (int)((a->Sq + 127) / 128);
-    q.accumulate = a->accumulate_dq;
-    launch_dq_direct(q, (int)a->Dqk, a->causal != 0, a->dq_dtype == PITH_F32, st);
-  } else if (a->Dqk == 128) {
-    launch_dq<128, 128, 1, 2, 8>(p, a, st);
-  } else {
-    // short query ranges: workgroups of 4 wavefronts x 32 rows, so that no compute unit idles
-    const bool few = ((a->Sq + 255) / 256) * a->Hq * a->B * 4 < 3 * (int64_t)compute_units_or_default();
-    if (few) launch_dq<64, 64, 1, 1, 4>(p, a, st);
-    else launch_dq<64, 64, 1, 1, 8>(p, a, st);
-  }
+  p.accumulate = a->accumulate_dq;
+  const bool f32 = a->dq_dtype == PITH_F32;
+  if (use_split_keys(a)) launch_dq_direct(p, (int)a->Dqk, a->causal != 0, f32, st);
+  else launch_dq_duo(p, (int)a->Dqk, a->causal != 0, f32, st);
   return check_launch("pith_attn_bwd_dq");
 }
 

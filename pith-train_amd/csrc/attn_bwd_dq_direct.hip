@@ -1,5 +1,5 @@
 // Query-gradient kernel for head dims (128, 128) and (192, 128) on gfx950, organised like the
-// direct-load forward kernel (256-row workgroups, or 128-row ones whose wave pairs split the keys).
+// direct-load forward kernel with 128-row workgroups whose wave pairs split the keys.
 // Same function and numerics as the other dQ kernels (pithtrain/operators/mla/triton.py:205-266,
 // :392-441: P = exp2(kappa*s - lse2) in fp32, masked entries 0, dS = P*(dP - delta)*scale rounded
 // to bf16, fp32 accumulation of dQ += dS K; `scale` is applied once to the accumulated dQ).
@@ -11,10 +11,7 @@
 // and one vector block  dS(i+1) = P o (dP - delta);  early waves (0-3) run matrix then vector, late
 // waves (4-7) vector then matrix, so that on every SIMD one wave's MFMAs coincide with the other's
 // arithmetic. Q^T and dO^T fragments, lse and delta of a wave's 32 query rows are stationary.
-// FULL: a workgroup owns 256 query rows, every wave 32 of them and all 64 keys of each tile (48
-// matrix instructions per wave and interval against some 110 vector instructions: the vector block
-// hides completely behind the sibling's matrix block).
-// HALF: a workgroup owns 128 query rows; wave w and w + 4 own the SAME 32 rows, the early wave keys
+// A workgroup owns 128 query rows; wave w and w + 4 own the SAME 32 rows, the early wave keys
 // 0-31 and the late wave keys 32-63 of every tile; at the end the late wave hands its partial dQ to
 // the early wave through LDS.
 //
@@ -43,11 +40,11 @@ constexpr int kSlots = 4;  // K ring depth (tiles i, i+1 in use, later ones land
 constexpr int kAhead = 4;  // fragment reads run this many products ahead in the matrix block
 constexpr int kTile = kBN * kRowBytes128;
 
-template <int DQK, bool HALF, bool CAUSAL, typename OutT>
+template <int DQK, bool CAUSAL, typename OutT>
 __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams p) {
-  static_assert(DQK == 128 || (DQK == 192 && HALF), "head dims (192-feature queries need the HALF form)");
-  constexpr int KVB = HALF ? 1 : 2;      // 32-key blocks of a tile this wave owns
-  constexpr int kBM = HALF ? 128 : 256;  // query rows per workgroup
+  static_assert(DQK == 128 || DQK == 192, "head dims");
+  constexpr int KVB = 1;    // 32-key blocks of a tile this wave owns
+  constexpr int kBM = 128;  // query rows per workgroup
   // kDist: a tile is requested kDist intervals before the interval that first reads it.
   // kLdsQ / kLdsDo: trailing Q^T / dO^T fragments kept in LDS instead of registers.
   constexpr int kDist = DQK == 192 ? 1 : 2;
@@ -67,13 +64,13 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
   const bool late = wave >= kWaves / 2;
-  const int kvb0 = HALF ? wave >> 2 : 0;  // the first 32-key block of every tile this wave owns
+  const int kvb0 = wave >> 2;  // the 32-key block of every tile this wave owns
 
   int m_tile, h, b;
   decode_block(blockIdx.x, p.Hq, p.B, p.tiles, p.group, m_tile, h, b);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
-  const int q_wave0 = m0 + (HALF ? (wave & 3) : wave) * 32;
+  const int q_wave0 = m0 + (wave & 3) * 32;
   const int qrow = q_wave0 + c;
 
   const int64_t q_row_stride = (int64_t)p.HqT * DQK;
@@ -168,7 +165,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   // would compute all derived offsets once, keep them in registers across the loop and spill others.
   auto refresh_offsets = [&]() __attribute__((always_inline)) {
     if constexpr (DQK == 192) asm volatile("" : "+v"(s_base), "+v"(sx_base), "+v"(t_base[0]), "+v"(t_base[1]), "+v"(tx_base[0]), "+v"(tx_base[1]));
-    else if constexpr (!HALF) asm volatile("" : "+v"(s_base), "+v"(t_base[0]), "+v"(t_base[1]));
   };
   auto s_off = [&](int ks) __attribute__((always_inline)) { return ks < 8 ? s_base ^ (ks << 5) : sx_base ^ ((ks - 8) << 5); };
   auto t_off = [&](int o, int hh) __attribute__((always_inline)) {
@@ -184,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   f32x16 s[KVB], dp[KVB];  // S^T and dP^T of this wave's keys of one tile: 32 x 32 tiles [keys] x [queries]
   bf16x8 dsf[2 * KVB];     // dS^T / scale of the same keys as B operand, one fragment per 16 keys
   // straight fragment of key block kvb: the 128-feature tile steps 32 rows on, the extra tile (192
-  // features, HALF only) is never asked for a second block
+  // features) is never asked for a second block
   auto a_frag = [&](const char* tile, int ks, int kvb) __attribute__((always_inline)) {
     return *reinterpret_cast<const bf16x8*>(tile + s_off(ks) + kvb * 32 * kRowBytes128);
   };
@@ -223,7 +219,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   auto matrix_block = [&](const char* kprev, const char* ktile, const char* vtile) __attribute__((always_inline)) {
     constexpr int NT = 2 * KVB * DB, N1 = KVB * (KSR + VSR), N2 = kLdsQ + kLdsDo;
     static_assert(kAhead <= NT && kAhead <= N1 && (N2 == 0 || kAhead <= N2), "look-ahead segments");
-    static_assert(N2 == 0 || KVB == 1, "LDS-resident B operands only in the HALF form");
     bf16x8 at[2 * KVB][DB], ak[KS][KVB], av[VS][KVB], bq[kLdsQ + 1], bd[kLdsDo + 1];
 #pragma unroll
     for (int j = 0; j < 2 * KVB; ++j)
@@ -397,19 +392,6 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   constexpr int kExch = kTurn ? kRowsViaLdsBytes<DB> : DB * 4 * 64 * 16;
   static_assert(kExch >= DB * 4 * 64 * 16 && 4 * kExch <= (int)sizeof(smem), "exchange area");
   char* const exch = smem + (wave & 3) * kExch;
-  if constexpr (!HALF) {
-    OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK;
-    if (qrow < p.Sq) {
-      OutT* dst = dqh + qrow * q_row_stride;
-#pragma unroll
-      for (int o = 0; o < DB; ++o)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4)
-          store4<OutT>(dst + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4] * p.scale, acc[o][4 * b4 + 1] * p.scale,
-                       acc[o][4 * b4 + 2] * p.scale, acc[o][4 * b4 + 3] * p.scale, p.accumulate != 0);
-    }
-    return;
-  }
   if (late) {
 #pragma unroll
     for (int o = 0; o < DB; ++o)
@@ -462,25 +444,24 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_direct_kernel(BwdParams 
   }
 }
 
-template <int DQK, bool HALF>
-void launch_one(const BwdParams& p, bool causal, bool f32_out, hipStream_t st) {
+template <int DQK>
+void launch_one(BwdParams p, bool causal, bool f32_out, hipStream_t st) {
+  p.tiles = (p.Sq + 127) / 128;
   const dim3 grid((unsigned)(p.tiles * p.Hq * p.B)), block(kThreads);
   if (causal) {
-    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, HALF, true, float>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, HALF, true, __bf16>), grid, block, 0, st, p);
+    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, true, float>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, true, __bf16>), grid, block, 0, st, p);
   } else {
-    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, HALF, false, float>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, HALF, false, __bf16>), grid, block, 0, st, p);
+    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, false, float>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((attn_bwd_dq_direct_kernel<DQK, false, __bf16>), grid, block, 0, st, p);
   }
 }
 
 }  // namespace
 
 void launch_dq_direct(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t st) {
-  // only the HALF form is built: with all 64 keys of a tile per wave this organisation needs some 300
-  // registers (the 256-row kernel for 128 features is attn_bwd_dq_d128.hip, organised differently)
-  if (dqk == 192) launch_one<192, true>(p, causal, f32_out, st);
-  else launch_one<128, true>(p, causal, f32_out, st);
+  if (dqk == 192) launch_one<192>(p, causal, f32_out, st);
+  else launch_one<128>(p, causal, f32_out, st);
 }
 
 }  // namespace pith

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) 
   }
 
   DirectTile128<kBN, kThreads> vmover, kmover;
-  DirectPaired64<kThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
+  DirectPaired64<kBN, kThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
   if constexpr (kPaired) {
     vpmover.init(v_row_bytes, 0, wave, lane);
     kpmover.init(k_row_bytes, 0, wave, lane);

@@ -235,13 +235,18 @@ struct DirectTile128 {
       for (int n = 0; n < kPerThread; ++n)
         load_lds16(tile_src + (int64_t)n * 4 * kWaves * row_bytes, off, slot + (n * kWaves + wave) * 1024);
     } else {
+      issue_clamped(tile_src, rows_left, slot, wave, lane);
+    }
+  }
+  // The same for any rows_left, source offsets formed on the spot: a few more vector instructions, but no per-lane
+  // register lives from one tile to the next (for kernels that would spill it).
+  __device__ __forceinline__ void issue_clamped(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
 #pragma unroll
-      for (int n = 0; n < kPerThread; ++n) {
-        const int row = 4 * (n * kWaves + wave) + (lane >> 4);
-        const int src_row = row < rows_left ? row : rows_left - 1;
-        load_lds16(tile_src, src_row * row_bytes + (((lane & 15) ^ tile_swizzle(row)) << 4),
-                   slot + (n * kWaves + wave) * 1024);
-      }
+    for (int n = 0; n < kPerThread; ++n) {
+      const int row = 4 * (n * kWaves + wave) + (lane >> 4);
+      const int src_row = row < rows_left ? row : rows_left - 1;
+      load_lds16(tile_src, src_row * row_bytes + (((lane & 15) ^ tile_swizzle(row)) << 4),
+                 slot + (n * kWaves + wave) * 1024);
     }
   }
 };
@@ -280,32 +285,43 @@ struct DirectExtra64 {
   }
 };
 
-// The same for a workgroup of THREADS threads, and for whole 64-feature operands: wave w fills LDS rows
-// 4w + 4*WAVES*n .. +3, and with 4 * WAVES a multiple of 16 the swizzle (hence the source offset) of a lane does not
-// depend on n.
-template <int THREADS>
+// The same for tiles of KEYS rows and workgroups of THREADS threads, and for whole 64-feature operands: LDS row r holds
+// tile rows r and r + KEYS/2. Wave w fills LDS rows 4w + 4*WAVES*n .. +3, and with 4 * WAVES a multiple of 16 the swizzle
+// (hence the source offset) of a lane does not depend on n.
+template <int KEYS, int THREADS>
 struct DirectPaired64 {
   static constexpr int kWaves = THREADS / 64;
-  static constexpr int kPerThread = 32 / (4 * kWaves);
-  static_assert(32 % (4 * kWaves) == 0 && (4 * kWaves) % 16 == 0, "rows of successive pieces must share their swizzle");
+  static constexpr int kPerThread = KEYS / 2 / (4 * kWaves);
+  static_assert(KEYS / 2 % (4 * kWaves) == 0 && (4 * kWaves) % 16 == 0, "rows of successive pieces must share their swizzle");
+  static constexpr int kTileBytes = KEYS / 2 * kRowBytes128;
   int src_off, row_bytes, col_bytes;
+  __device__ __forceinline__ static int source(int row_bytes, int col_bytes, int row, int lane, int rows_left) {
+    const int piece = (lane & 15) ^ tile_swizzle(row);
+    int key = row + KEYS / 2 * (piece >> 3);
+    key = key < rows_left ? key : rows_left - 1;
+    return key * row_bytes + col_bytes + ((piece & 7) << 4);
+  }
   __device__ __forceinline__ void init(int row_bytes_, int col_bytes_, int wave, int lane) {
     row_bytes = row_bytes_;
     col_bytes = col_bytes_;
-    src_off = DirectExtra64::source(row_bytes_, col_bytes_, wave, lane, 64);
+    src_off = source(row_bytes_, col_bytes_, 4 * wave + (lane >> 4), lane, KEYS);
   }
   __device__ __forceinline__ void issue(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
-    if (rows_left >= 64) {
+    if (rows_left >= KEYS) {
       int off = src_off;
       asm volatile("" : "+v"(off));  // pinned before the first load, see DirectTile128::issue
 #pragma unroll
       for (int n = 0; n < kPerThread; ++n)
         load_lds16(tile_src + (int64_t)n * 4 * kWaves * row_bytes, off, slot + (n * kWaves + wave) * 1024);
     } else {
-#pragma unroll
-      for (int n = 0; n < kPerThread; ++n)
-        load_lds16(tile_src, DirectExtra64::source(row_bytes, col_bytes, n * kWaves + wave, lane, rows_left), slot + (n * kWaves + wave) * 1024);
+      issue_clamped(tile_src, rows_left, slot, wave, lane);
     }
+  }
+  __device__ __forceinline__ void issue_clamped(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
+#pragma unroll
+    for (int n = 0; n < kPerThread; ++n)
+      load_lds16(tile_src, source(row_bytes, col_bytes, 4 * (n * kWaves + wave) + (lane >> 4), lane, rows_left),
+                 slot + (n * kWaves + wave) * 1024);
   }
 };
 

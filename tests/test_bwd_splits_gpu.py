@@ -1,0 +1,60 @@
+"""The backward's kernels at the edges of their tiles and on both sides of the lines between them, against plain fp32 PyTorch."""
+
+import pytest
+import torch
+
+from helpers import check_bf16_result
+from pithtrain_amd.operators.mla.hip import _mla_bwd_dk_dv, _mla_bwd_dq, _mla_bwd_preprocess, _mla_fwd, attn_bwd_pair_into
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, dout, scale, causal):
+    """dQ, dK, dV in fp32, one query head at a time."""
+    b, sq, hq, _ = q.shape
+    group = hq // k.shape[2]
+    dq, dk, dv = (torch.zeros(t.shape, device=t.device) for t in (q, k, v))
+    mask = torch.ones(sq, k.shape[1], dtype=torch.bool, device=q.device).triu(1) if causal else None
+    for bi in range(b):
+        for h in range(hq):
+            qh, kh, vh, do = q[bi, :, h].float(), k[bi, :, h // group].float(), v[bi, :, h // group].float(), dout[bi, :, h].float()
+            s = (qh @ kh.t().contiguous()) * scale
+            if causal:
+                s.masked_fill_(mask, float("-inf"))
+            p = torch.softmax(s, -1)
+            dp = do @ vh.t().contiguous()
+            ds = p * (dp - (dp * p).sum(-1, keepdim=True)) * scale
+            dq[bi, :, h] = ds @ kh
+            dk[bi, :, h // group] += ds.t().contiguous() @ qh
+            dv[bi, :, h // group] += p.t().contiguous() @ do
+    return dq, dk, dv
+
+
+CASES = [
+    # one row; 32-row tiles and 128-row workgroups minus / plus one; ragged keys against ragged queries
+    (1, 1, 1, 2, 1, 64, True), (1, 33, 33, 2, 2, 64, True), (2, 129, 129, 4, 2, 64, True), (1, 70, 200, 4, 1, 64, False),
+    (1, 200, 70, 4, 2, 64, False), (1, 640, 640, 8, 4, 64, True), (1, 127, 127, 2, 1, 128, True), (1, 65, 257, 4, 2, 128, False),
+    (1, 31, 256, 3, 3, 192, False), (1, 256, 256, 2, 2, 192, True), (1, 97, 33, 2, 2, 192, False),
+    # 256 / 257 and 512 / 513 workgroups of 128 query rows, streams of 1535 / 1536 keys
+    (1, 512, 512, 16, 4, 128, False), (1, 257, 300, 86, 86, 192, False), (1, 896, 300, 37, 37, 192, False), (1, 1535, 1535, 42, 2, 128, True),
+    (1, 1536, 1536, 42, 42, 192, True), (1, 1664, 1664, 42, 2, 128, True),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D,causal", CASES)
+def test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+    g = torch.Generator(device=gpu).manual_seed(13)
+    mk = lambda s, h, d: torch.randn(B, s, h, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    dv_dim, scale = min(D, 128), D**-0.5
+    q, k, v, dout = mk(Sq, Hq, D), mk(Skv, Hkv, D), mk(Skv, Hkv, dv_dim), mk(Sq, Hq, dv_dim)
+    o, lse = _mla_fwd(q, k, v, scale, causal)
+    delta = _mla_bwd_preprocess(o, dout)
+    dq = _mla_bwd_dq(q, k, v, dout, lse, delta, scale, causal)
+    dk, dv = _mla_bwd_dk_dv(q, k, v, dout, lse, delta, scale, causal)
+    refs = _reference(q, k, v, dout, scale, causal)
+    for name, got, want in zip(("dQ", "dK", "dV"), (dq, dk, dv), refs):
+        check_bf16_result(got, want, name, otol=1e-3)
+    pair = [torch.empty_like(t) for t in (q, k, v)]
+    attn_bwd_pair_into(q, k, v, dout, lse, delta, *pair, scale, causal)
+    for name, got, want in zip(("dQ", "dK", "dV"), pair, refs):
+        check_bf16_result(got, want, name + " of the pair", otol=1e-3)
