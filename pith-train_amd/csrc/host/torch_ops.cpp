@@ -269,11 +269,22 @@ int64_t compute_units(int device) {
   return n;
 }
 
+// Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill
+// the device, and under the mask one round of workgroups will not do, because the heaviest of them carries almost twice
+// the average work (1 x 4096 rows x 32 heads: pair of kernels 445 us handing over, 428 us recomputing; 2 x 2048 x 32: 252
+// and 238 us), unless the sequence is so short (two tiles) that there is nothing to balance.
+bool ds_handover_pays(int64_t workgroups, int64_t row_tiles, bool causal, int64_t cus) {
+  return workgroups >= cus && !(causal && row_tiles > 2 && workgroups <= cus);
+}
+
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
-  // Calls large enough for the dS hand-over (its dQ kernel owns 512 query rows per workgroup) belong to the Python body,
-  // which owns the policy for the hand-over buffer: their kernels outlast its host work many times over.
-  const bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4 &&
-                     !(q.size(3) == 128 && (q.size(1) + 511) / 512 * q.size(2) * q.size(0) >= compute_units(q.device().index()));
+  // Calls large enough for the dS hand-over belong to the Python body, which owns the policy for the hand-over buffer: their
+  // kernels outlast its host work many times over.
+  bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4;
+  if (small && q.size(3) == 128) {
+    const int64_t row_tiles = (q.size(1) + 511) / 512;
+    small = !ds_handover_pays(row_tiles * q.size(2) * q.size(0), row_tiles, causal, compute_units(q.device().index()));
+  }
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
@@ -652,4 +663,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("combine_into", &combine_into);
   m.def("combine_new", &combine_new);
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into);
+  m.def("ds_handover_pays", &ds_handover_pays);
 }

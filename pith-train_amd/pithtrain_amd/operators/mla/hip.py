@@ -197,7 +197,7 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
     args.ds, args.ds_bytes = ds.data_ptr(), ds.numel()
 
 
-# The dS hand-over (head dims 128/128) makes the backward of a chunk pair 3-6 % faster at the price of a
+# The dS hand-over (head dims 128/128) makes the backward of a chunk pair 3-5 % faster at the price of a
 # transient buffer of Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask).
 # Policy: the buffer never exceeds DS_BUFFER_LIMIT_BYTES nor DS_BUFFER_FREE_FRACTION of the device memory that is
 # free right now; a chunk pair that needs more is processed one group of kv heads (with their query heads) after
@@ -238,7 +238,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
     b, sq, hq, _ = q.shape
     hkv = k.shape[2]
     row_tiles = -(-sq // _DS_ROWS_PER_WORKGROUP)
-    if row_tiles * hq * b < _device_compute_units(q.device):  # no slab can fill the device either
+    if not native.ds_handover_pays(row_tiles * hq * b, row_tiles, causal, _device_compute_units(q.device)):  # nor for any slab
         return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:
