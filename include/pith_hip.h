@@ -244,6 +244,10 @@ typedef struct {
 
 int pith_attn_bwd_dkdv(const pith_attn_bwd_args* args, pith_stream_t stream);
 int pith_attn_bwd_dq(const pith_attn_bwd_args* args, pith_stream_t stream);
+/* Both of them for one chunk pair (dk, dv and dq all set), with the results of pith_attn_bwd_dkdv followed by pith_attn_bwd_dq.
+ * Without a usable `ds` the two do not depend on each other, and where that pays (grids that do not fill the
+ * device many times over) they run as one grid instead of one after the other. */
+int pith_attn_bwd(const pith_attn_bwd_args* args, pith_stream_t stream);
 
 /* Scratch size with which pith_attn_bwd_dkdv runs fastest for these shapes (0 = none needed).
  * With grouped-query attention and few key rows the kernel spreads the query heads of a group

@@ -19,10 +19,10 @@ struct BwdParams {
   // heads per ROW of the query-side tensors (q, dout, dq) and of the key-side tensors (k, v, dk, dv): Hq / Hkv for
   // tensors that hold exactly the heads of this call, larger when the call works on a head range of wider tensors
   int HqT, HkvT;
-  int tiles;  // query tiles (dQ kernel) or key tiles (dK/dV kernel) in the grid's x dimension
+  int tiles, q_tiles;  // key tiles of the dK/dV kernels' grid, query tiles of the dQ kernels'
   int64_t q_bs, k_bs, v_bs, dout_bs, dq_bs, dk_bs, dv_bs, lse_bs, lse_hs;
   float kappa, scale;
-  int accumulate;
+  int accumulate, accumulate_dq;  // dK/dV and dQ kernels: add to what the outputs hold
   int split;        // dK/dV kernel: query-head groups are cut into `split` parts handled by different workgroups
   float* ws_dk;     // dK/dV kernel, split > 1: fp32 partial results [split][B][Skv][Hkv][D]
   float* ws_dv;
@@ -190,6 +190,11 @@ void launch_dkdv_d128(const BwdParams& p, bool causal, bool f32_out, unsigned gr
 // dK/dV for head dims (192, 128): attn_bwd_dkdv_d192.hip. Same conventions.
 void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
 
+// dK/dV and recomputing dQ of one chunk pair as ONE grid (the dK/dV workgroups first): attn_bwd_pair.hip. dkdv_blocks = the
+// dK/dV kernel's grid; everything else as for the separate launches. Head dims (128, 128) and (192, 128) use the split-key
+// dQ workgroups. False: no such kernel for these output types.
+bool launch_bwd_pair(const BwdParams& p, int dqk, bool causal, bool dkdv_f32, bool dq_f32, unsigned dkdv_blocks, hipStream_t stream);
+
 // dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
 // split every tile's keys: attn_bwd_dq_direct.hip.
 void launch_dq_direct(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t stream);
@@ -198,10 +203,14 @@ void launch_dq_direct(const BwdParams& p, int dqk, bool causal, bool f32_out, hi
 void launch_dq_duo(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t stream);
 
 // dQ for head dims (128, 128) from the dS images the dK/dV kernel left in p.ds: attn_bwd_dq_ds.hip.
-// p.tiles = number of 512-row query tiles.
+// p.q_tiles = number of 512-row query tiles.
 void launch_dq_from_ds(const BwdParams& p, bool causal, bool f32_out, hipStream_t stream);
-// Bytes of dS images for a shape (0: the shape has no hand-over path).
+// Bytes of dS images for a shape (0: the shape has no hand-over path), and whether the call brings a buffer for them.
 int64_t ds_bytes_for(const pith_attn_bwd_args* a);
+bool ds_usable(const pith_attn_bwd_args* a);
+// Whether a recomputing dQ call uses the split-key workgroups, and its share of the parameters (attn_bwd_dq.hip).
+bool dq_split_keys(const pith_attn_bwd_args* a);
+int prepare_dq(const pith_attn_bwd_args* a, BwdParams* p, const char* who);
 
 // Argument checks common to both entry points; returns PITH_OK or records the error.
 int validate_bwd(const pith_attn_bwd_args* a, const char* who, bool need_dq, bool need_dkv);

@@ -71,15 +71,18 @@ int64_t workspace_bytes_for(const pith_attn_bwd_args* a, int split) { return spl
 
 constexpr int64_t kWalkDescBytes = 192ll << 20;
 
+// with_dq: dQ of the pair in the same grid (p prepared for it)
 template <int DQK, int DV>
-void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, hipStream_t st) {
+void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, bool with_dq, hipStream_t st) {
   p.tiles = (int)((a->Skv + kBN - 1) / kBN);
   p.accumulate = a->accumulate_dkv;
   p.main_blocks = (int)(p.tiles * a->Hkv * a->B * p.split);
   p.zero_tail = a->accumulate_dkv ? 0 : (int)a->dkv_zero_tail;  // rows that are added to keep what they hold
   const unsigned grid = (unsigned)(p.main_blocks + (p.zero_tail + kZeroTailRows - 1) / kZeroTailRows);
   const bool f32 = a->dkv_dtype == PITH_F32;
-  if constexpr (DQK == 128 && DV == 128) {
+  if (with_dq) {
+    launch_bwd_pair(p, DQK, a->causal != 0, f32, a->dq_dtype == PITH_F32, grid, st);
+  } else if constexpr (DQK == 128 && DV == 128) {
     // descending walk under the mask when Q and dO together exceed what the last-level cache (256 MB) keeps
     p.walk_desc = a->causal != 0 && (int64_t)a->B * a->Sq * a->Hq * (DQK + DV) * 2 > kWalkDescBytes;
     launch_dkdv_d128(p, a->causal != 0, f32, grid, st);
@@ -143,12 +146,14 @@ extern "C" int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* 
 namespace {
 
 // Runs the kernels with the head-split partials in `workspace` (NULL: no head split).
-int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_t st, const char* who) {
+int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_t st, const char* who, bool with_dq = false) {
   // the grid of this kernel runs over key tiles (validate_bwd bounded the query-side grid)
   if (((a->Skv + kBN - 1) / kBN) * a->Hkv * a->B * (int64_t)split > 0x7fffffffLL)
     return fail(PITH_ERR_UNSUPPORTED, "%s: Skv=%lld x Hkv=%lld x B=%lld exceeds the launch grid limit", who,
                 (long long)a->Skv, (long long)a->Hkv, (long long)a->B);
   BwdParams p = make_bwd_params(a);
+  if (with_dq)
+    if (const int rc = prepare_dq(a, &p, who)) return rc;
   if (a->k_pe) {
     if (a->Hq != a->Hkv)
       return fail(PITH_ERR_UNSUPPORTED, "%s: keys in two parts need Hq == Hkv (got %lld, %lld)", who, (long long)a->Hq, (long long)a->Hkv);
@@ -164,13 +169,13 @@ int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_
     p.ws_dv = p.ws_dk + (int64_t)split * a->B * a->Skv * a->Hkv * a->Dqk;
   }
   // dS hand-over to the dQ call: only when the buffer is usable (otherwise the call behaves as without it)
-  if (a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a)) {
+  if (ds_usable(a)) {
     if ((uintptr_t)a->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
     p.ds = reinterpret_cast<char*>(a->ds);
   }
-  if (a->Dqk == 128) launch_dkdv<128, 128>(p, a, st);
-  else if (a->Dqk == 192) launch_dkdv<192, 128>(p, a, st);
-  else launch_dkdv<64, 64>(p, a, st);
+  if (a->Dqk == 128) launch_dkdv<128, 128>(p, a, with_dq, st);
+  else if (a->Dqk == 192) launch_dkdv<192, 128>(p, a, with_dq, st);
+  else launch_dkdv<64, 64>(p, a, with_dq, st);
   return check_launch(who);
 }
 
@@ -204,17 +209,44 @@ int static_scratch(void** out, const char* who) {
 
 }  // namespace
 
-extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream) {
-  const int rc = validate_bwd(a, "pith_attn_bwd_dkdv", false, true);
+namespace {
+
+int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who, bool with_dq) {
+  const int rc = validate_bwd(a, who, false, true);
   if (rc != PITH_OK) return rc;
   // Head groups are split only when the caller brought a workspace that is large enough.
   int split = pick_split(a);
   if (!(split > 1 && a->workspace && a->workspace_bytes >= workspace_bytes_for(a, split))) split = 1;
-  if (a->workspace && !aligned16(a->workspace)) return fail(PITH_ERR_MISALIGNED, "pith_attn_bwd_dkdv: workspace must be 16-byte aligned");
+  if (a->workspace && !aligned16(a->workspace)) return fail(PITH_ERR_MISALIGNED, "%s: workspace must be 16-byte aligned", who);
   if (a->k_pe && (!a->workspace || a->workspace_bytes < workspace_bytes_for(a, split)))
-    return fail(PITH_ERR_BAD_SHAPE, "pith_attn_bwd_dkdv: keys in two parts need a workspace of %lld bytes, %lld given",
+    return fail(PITH_ERR_BAD_SHAPE, "%s: keys in two parts need a workspace of %lld bytes, %lld given", who,
                 (long long)workspace_bytes_for(a, split), (long long)(a->workspace ? a->workspace_bytes : 0));
-  return run_dkdv(a, split, a->workspace, (hipStream_t)stream, "pith_attn_bwd_dkdv");
+  return run_dkdv(a, split, a->workspace, (hipStream_t)stream, who, with_dq);
+}
+
+// Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
+// split-key ones (the two kernels must agree on the workgroup size), which is what grids of up to one workgroup per compute
+// unit want anyway; larger ones fill the device with either kernel and gain nothing (1 x 4096 x 16 heads of 192 features,
+// 512 + 512 workgroups: 293 us apart, 298 us together). At 64 features one kernel costs dQ its third workgroup per compute
+// unit (186 instead of 150 registers), which only grids of a few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us,
+// 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16 474 -> 483 us).
+bool one_grid(const pith_attn_bwd_args* a) {
+  if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
+  const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
+  return q_wgs <= (a->Dqk == 64 ? 4 : 1) * (int64_t)compute_units_or_default();
+}
+
+}  // namespace
+
+extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream) {
+  return bwd_dkdv(a, stream, "pith_attn_bwd_dkdv", false);
+}
+
+extern "C" int pith_attn_bwd(const pith_attn_bwd_args* a, pith_stream_t stream) {
+  if (const int rc = validate_bwd(a, "pith_attn_bwd", true, true)) return rc;
+  if (one_grid(a)) return bwd_dkdv(a, stream, "pith_attn_bwd", true);
+  if (const int rc = pith_attn_bwd_dkdv(a, stream)) return rc;
+  return pith_attn_bwd_dq(a, stream);
 }
 
 extern "C" int pith_attn_bwd_dkdv_static(const pith_attn_bwd_args* a, pith_stream_t stream) {

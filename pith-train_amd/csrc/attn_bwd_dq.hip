@@ -4,8 +4,6 @@
 #include "attn_bwd_common.h"
 
 namespace pith {
-namespace {
-
 // Recomputing dQ kernels: 128-row workgroups either way. Two 4-wave workgroups per compute unit (attn_bwd_dq_duo.hip), or
 // one of 8 waves whose pairs split every tile's keys (attn_bwd_dq_direct.hip, "half"). Measured, microseconds:
 //                                              duo    half
@@ -17,14 +15,14 @@ namespace {
 // So the split keys pay where a workgroup has its compute unit to itself: grids of up to one workgroup per unit, and under
 // the mask, where the heavy half of the workgroups ends up alone, of up to two for long streams (the same lines as in the
 // forward). 64 features always use duo (three workgroups fit a unit; no split-key kernel exists).
-bool use_split_keys(const pith_attn_bwd_args* a) {
+bool dq_split_keys(const pith_attn_bwd_args* a) {
   if (a->Dqk == 64) return false;
   const int64_t cus = compute_units_or_default();
   const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
   return wgs <= cus ? a->Skv > 256 : a->causal && wgs <= 2 * cus && a->Skv >= 1536;
 }
 
-}  // namespace
+bool ds_usable(const pith_attn_bwd_args* a) { return a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a); }
 
 int validate_bwd(const pith_attn_bwd_args* a, const char* who, bool need_dq, bool need_dkv) {
   if (!a) return fail(PITH_ERR_NULL_POINTER, "%s: args is NULL", who);
@@ -82,12 +80,12 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
   p.Sq = (int)a->Sq; p.Skv = (int)a->Skv; p.Hq = (int)a->Hq; p.Hkv = (int)a->Hkv; p.group = (int)(a->Hq / a->Hkv); p.B = (int)a->B;
   p.HqT = (int)(a->q_row_heads ? a->q_row_heads : a->Hq);
   p.HkvT = (int)(a->kv_row_heads ? a->kv_row_heads : a->Hkv);
-  p.tiles = 0;
+  p.tiles = p.q_tiles = 0;
   p.q_bs = a->q_bs; p.k_bs = a->k_bs; p.v_bs = a->v_bs; p.dout_bs = a->dout_bs;
   p.dq_bs = a->dq_bs; p.dk_bs = a->dk_bs; p.dv_bs = a->dv_bs; p.lse_bs = a->lse_bs; p.lse_hs = a->lse_hs;
   p.scale = a->scale;
   p.kappa = a->scale * 1.44269504088896340736f;
-  p.accumulate = 0;
+  p.accumulate = p.accumulate_dq = 0;
   p.split = 1;
   p.ws_dk = nullptr;
   p.ws_dv = nullptr;
@@ -116,41 +114,48 @@ using namespace pith;
 
 extern "C" int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* a) { return ds_bytes_for(a); }
 
-extern "C" int pith_attn_bwd_dq(const pith_attn_bwd_args* a, pith_stream_t stream) {
-  const int rc = validate_bwd(a, "pith_attn_bwd_dq", true, false);
-  if (rc != PITH_OK) return rc;
-  BwdParams p = make_bwd_params(a);
-  if (a->dq_final) {
-    if (a->dq_dtype != PITH_F32 || a->Dv != 128 || (a->Dqk != 128 && a->Dqk != 192))
-      return fail(PITH_ERR_UNSUPPORTED, "pith_attn_bwd_dq: dq_final needs an fp32 dq and head dims (128,128) or (192,128)");
-    if (!aligned16(a->dq_final) || a->dq_final_bs % 8)
-      return fail(PITH_ERR_MISALIGNED, "pith_attn_bwd_dq: dq_final pointer / batch stride must keep 16-byte alignment");
-    int64_t r0 = a->dq_final_rows[0], r1 = a->dq_final_rows[1];
-    if (r0 == 0 && r1 == 0) r1 = a->Sq;
-    if (r0 < 0 || r1 < r0 || r1 > a->Sq || r0 % 32 || (r1 % 32 && r1 != a->Sq))
-      return fail(PITH_ERR_BAD_SHAPE, "pith_attn_bwd_dq: dq_final_rows = [%lld, %lld) must lie within the %lld query rows on multiples of 32",
-                  (long long)a->dq_final_rows[0], (long long)a->dq_final_rows[1], (long long)a->Sq);
-    p.dq_final = reinterpret_cast<__bf16*>(a->dq_final);
-    p.dq_final_bs = a->dq_final_bs;
-    p.final_r0 = (int)r0;
-    p.final_r1 = (int)r1;
-  }
-  hipStream_t st = (hipStream_t)stream;
-  begin_launch();
-  if (a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a)) {
-    // dS was left by the dK/dV call of the same chunk: one product instead of three
-    if ((uintptr_t)a->ds % 256) return fail(PITH_ERR_MISALIGNED, "pith_attn_bwd_dq: ds must be 256-byte aligned");
-    BwdParams q = p;
-    q.ds = reinterpret_cast<char*>(a->ds);
-    q.tiles = (int)((a->Sq + 511) / 512);
-    q.accumulate = a->accumulate_dq;
-    launch_dq_from_ds(q, a->causal != 0, a->dq_dtype == PITH_F32, st);
-    return check_launch("pith_attn_bwd_dq");
-  }
-  p.accumulate = a->accumulate_dq;
-  const bool f32 = a->dq_dtype == PITH_F32;
-  if (use_split_keys(a)) launch_dq_direct(p, (int)a->Dqk, a->causal != 0, f32, st);
-  else launch_dq_duo(p, (int)a->Dqk, a->causal != 0, f32, st);
-  return check_launch("pith_attn_bwd_dq");
+namespace pith {
+
+// What the dQ call adds to the shared parameters: its accumulation and the rows it finishes.
+int prepare_dq(const pith_attn_bwd_args* a, BwdParams* p, const char* who) {
+  p->accumulate_dq = a->accumulate_dq;
+  if (!a->dq_final) return PITH_OK;
+  if (a->dq_dtype != PITH_F32 || a->Dv != 128 || (a->Dqk != 128 && a->Dqk != 192))
+    return fail(PITH_ERR_UNSUPPORTED, "%s: dq_final needs an fp32 dq and head dims (128,128) or (192,128)", who);
+  if (!aligned16(a->dq_final) || a->dq_final_bs % 8)
+    return fail(PITH_ERR_MISALIGNED, "%s: dq_final pointer / batch stride must keep 16-byte alignment", who);
+  int64_t r0 = a->dq_final_rows[0], r1 = a->dq_final_rows[1];
+  if (r0 == 0 && r1 == 0) r1 = a->Sq;
+  if (r0 < 0 || r1 < r0 || r1 > a->Sq || r0 % 32 || (r1 % 32 && r1 != a->Sq))
+    return fail(PITH_ERR_BAD_SHAPE, "%s: dq_final_rows = [%lld, %lld) must lie within the %lld query rows on multiples of 32", who,
+                (long long)a->dq_final_rows[0], (long long)a->dq_final_rows[1], (long long)a->Sq);
+  p->dq_final = reinterpret_cast<__bf16*>(a->dq_final);
+  p->dq_final_bs = a->dq_final_bs;
+  p->final_r0 = (int)r0;
+  p->final_r1 = (int)r1;
+  return PITH_OK;
 }
 
+}  // namespace pith
+
+extern "C" int pith_attn_bwd_dq(const pith_attn_bwd_args* a, pith_stream_t stream) {
+  const char* who = "pith_attn_bwd_dq";
+  if (const int rc = validate_bwd(a, who, true, false)) return rc;
+  BwdParams p = make_bwd_params(a);
+  if (const int rc = prepare_dq(a, &p, who)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const bool f32 = a->dq_dtype == PITH_F32;
+  begin_launch();
+  if (ds_usable(a)) {
+    // dS was left by the dK/dV call of the same chunk: one product instead of three
+    if ((uintptr_t)a->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
+    p.ds = reinterpret_cast<char*>(a->ds);
+    p.q_tiles = (int)((a->Sq + 511) / 512);
+    launch_dq_from_ds(p, a->causal != 0, f32, st);
+  } else if (dq_split_keys(a)) {
+    launch_dq_direct(p, (int)a->Dqk, a->causal != 0, f32, st);
+  } else {
+    launch_dq_duo(p, (int)a->Dqk, a->causal != 0, f32, st);
+  }
+  return check_launch(who);
+}

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
   int m_tile, h, b;
-  decode_block(blockIdx.x, p.Hq, p.B, p.tiles, p.group, m_tile, h, b);
+  decode_block(blockIdx.x, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
   const int q_wave0 = m0 + wave * QW;
@@ -234,14 +234,14 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
     __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
     if (p.dq_final != nullptr && row0 >= p.final_r0 && row0 < p.final_r1)
       fin = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + row0 * row_stride;
-    store_rows32<OutT, DB>(dqh + row0 * row_stride, row_stride, p.Sq - row0, acc[rb], sc, p.accumulate != 0, c, g, fin);
+    store_rows32<OutT, DB>(dqh + row0 * row_stride, row_stride, p.Sq - row0, acc[rb], sc, p.accumulate_dq != 0, c, g, fin);
   }
 }
 
 }  // namespace
 
 void launch_dq_from_ds(const BwdParams& p, bool causal, bool f32_out, hipStream_t st) {
-  const dim3 grid((unsigned)(p.tiles * p.Hq * p.B)), block(kThreads);
+  const dim3 grid((unsigned)(p.q_tiles * p.Hq * p.B)), block(kThreads);
   if (causal) {
     if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<true, float>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<true, __bf16>), grid, block, 0, st, p);

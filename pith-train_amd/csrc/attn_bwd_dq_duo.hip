@@ -1,284 +1,20 @@
-// Query-gradient kernel for head dims (64, 64), (128, 128) and (192, 128) on gfx950 with SMALL workgroups: 4 wavefronts,
-// 128 query rows, two of them per compute unit (three at 64 features). Same function and numerics as
-// attn_bwd_dq_direct.hip (pithtrain/operators/mla/triton.py:205-266, :392-441: P = exp2(kappa*s - lse2) in fp32, masked
-// entries 0, dS = P*(dP - delta) rounded to bf16, fp32 accumulation of dQ += dS K, `scale` applied once at the end).
-//
-// A wave owns 32 query rows (Q^T, dO^T, lse and delta stationary) and walks key tiles of 32; per interval one matrix block
-//     dQ^T += K(i-1)^T dS(i-1)^T ;  S(i)^T = K(i) Q^T ;  dP(i)^T = V(i) dO^T
-// and one vector block dS(i). Nothing inside a wave overlaps the two; the two workgroups of a compute unit do (each SIMD
-// holds one wave of either), and they also hide each other's first tiles, diagonal and epilogue. Tiles of 32 keys keep S,
-// dP and dS at 40 registers, which is what lets 192 features fit; they are requested two intervals ahead into rings of
-// four, and the wait that ends an interval counts: it lets exactly the loads of that interval stay in flight.
-// Bound by the matrix pipe (three products executed for the one that counts). Measured, executed products: 8192 x 8192 x
-// 32 heads of 128 features 1284 TFLOP/s (1242 for the 256-row kernel with interleaved halves it replaces), 2 x 4096 x 16 of 64
-// features 1033 (915 register-staged), 4096 x 4096 x 16 of 192 features 1219 (1156 with 128-row workgroups splitting keys).
+// dQ launches of the kernel in attn_bwd_dq_duo.h.
 #include "attn_bwd_common.h"
+#include "attn_bwd_dq_duo.h"
 
 namespace pith {
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
-constexpr int kBM = 32 * kWaves;  // query rows per workgroup
-constexpr int kBN = 32;           // keys per tile
-constexpr int kSlots = 4;         // tiles i-1 and i (in use), i+1 and i+2 (landing); a power of two
-
-template <int DQK>
-struct DqDuoLayout {
-  static constexpr int kDv = DQK == 64 ? 64 : 128;
-  static constexpr int kPair = kBN / 2 * kRowBytes128, kFull = kBN * kRowBytes128;  // 64- and 128-feature tiles
-  static constexpr int kKTile = DQK == 64 ? kPair : DQK == 128 ? kFull : kFull + kPair;
-  static constexpr int kVTile = kDv == 64 ? kPair : kFull;
-  static constexpr int kRings = kSlots * (kKTile + kVTile);
-  static constexpr int kTurnBlocks = DQK == 192 ? 3 : DQK / 32;  // feature blocks the epilogue turns at a time
-  static constexpr int kTurn = kWaves * kRowsViaLdsBytes<kTurnBlocks>;
-  static constexpr int kSmem = kRings > kTurn ? kRings : kTurn;
-  static constexpr int kLoads = (DQK == 64 ? 1 : DQK == 128 ? 2 : 3) + (kDv == 64 ? 1 : 2);  // load instructions per wave and tile
-};
-
 template <int DQK, bool CAUSAL, typename OutT>
-__global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_duo_kernel(BwdParams p) {
-  using L = DqDuoLayout<DQK>;
-  constexpr int kDv = L::kDv, KS = DQK / 16, VS = kDv / 16, DB = DQK / 32;
-  constexpr bool kPaired = DQK == 64;
-  constexpr int kAhead = DQK == 192 ? 3 : 4;  // fragment reads run this many products ahead in the matrix block
-  __shared__ __attribute__((aligned(1024))) char smem[L::kSmem];
-  char* const kbuf = smem;
-  char* const vbuf = smem + kSlots * L::kKTile;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 31, g = lane >> 5;
-
-  int m_tile, h, b;
-  decode_block(blockIdx.x, p.Hq, p.B, p.tiles, p.group, m_tile, h, b);
-  const int hk = h / p.group;
-  const int m0 = m_tile * kBM;
-  const int q_wave0 = m0 + wave * 32;
-  const int qrow = q_wave0 + c;
-
-  const int64_t q_row_stride = (int64_t)p.HqT * DQK;
-  const int64_t do_row_stride = (int64_t)p.HqT * kDv;
-  // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
-  const bool two_part = DQK == 192 && p.k_pe != nullptr;
-  const int k_head_elems = two_part ? 128 : DQK;
-  const int k_row_bytes = p.HkvT * k_head_elems * 2, v_row_bytes = p.HkvT * kDv * 2;
-  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
-  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;
-  const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
-  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
-
-  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
-  int n_wg = n_tiles_all, n_wave = n_tiles_all;  // key tiles this workgroup / this wave visits
-  if (CAUSAL) {
-    n_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
-    n_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
-  }
-
-  DirectTile128<kBN, kThreads> vmover, kmover;
-  DirectPaired64<kBN, kThreads> vpmover, kpmover;
-  if constexpr (kPaired) {
-    vpmover.init(v_row_bytes, 0, wave, lane);
-    kpmover.init(k_row_bytes, 0, wave, lane);
-  } else {
-    vmover.init(v_row_bytes, wave, lane);
-    kmover.init(k_row_bytes, wave, lane);
-    if constexpr (DQK == 192) kpmover.init(kx_row_bytes, two_part ? 0 : 256, wave, lane);
-  }
-  auto request = [&](int t) __attribute__((always_inline)) {
-    char* const ks = kbuf + (t & (kSlots - 1)) * L::kKTile;
-    char* const vs = vbuf + (t & (kSlots - 1)) * L::kVTile;
-    const char* ksrc = kh + (int64_t)t * kBN * k_row_bytes;
-    const char* vsrc = vh + (int64_t)t * kBN * v_row_bytes;
-    const int left = p.Skv - t * kBN;
-    if constexpr (kPaired) {
-      kpmover.issue(ksrc, left, ks, wave, lane);
-      vpmover.issue(vsrc, left, vs, wave, lane);
-    } else if constexpr (DQK == 128) {
-      kmover.issue(ksrc, left, ks, wave, lane);
-      vmover.issue(vsrc, left, vs, wave, lane);
-    } else {  // no register to spare for source offsets: reloading a spilled one would wait for the tiles in flight
-      kmover.issue_clamped(ksrc, left, ks, wave, lane);
-      kpmover.issue_clamped(kx + (int64_t)t * kBN * kx_row_bytes, left, ks + L::kFull, wave, lane);
-      vmover.issue_clamped(vsrc, left, vs, wave, lane);
-    }
-  };
-  request(0);
-  if (n_wg > 1) request(1);
-  if (n_wg > 2) request(2);
-
-  // stationary B operands (column = query row), lse and delta of this lane's row
-  bf16x8 qf[KS], dof[VS];
-  float lse_q, delta_q;
-  {
-    const int row = qrow < p.Sq ? qrow : p.Sq - 1;
-    const __bf16* src = p.q + b * p.q_bs + (int64_t)h * DQK + row * q_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    const __bf16* dsrc = p.dout + b * p.dout_bs + (int64_t)h * kDv + row * do_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < VS; ++ks) dof[ks] = *reinterpret_cast<const bf16x8*>(dsrc + ks * 16);
-    lse_q = p.lse[b * p.lse_bs + (int64_t)h * p.lse_hs + row];
-    delta_q = p.delta[b * p.lse_bs + (int64_t)h * p.lse_hs + row];
-  }
-
-  // per-lane read offsets. Straight fragment of the tile's 32 keys, contraction step ks; transposed fragment of keys
-  // 16j..16j+15, feature block i. A 64-feature tile holds key r in pieces 0-7 and key r + 16 in pieces 8-15 of LDS row r.
-  int s_base = straight_offset128(c, g);
-  int x_base = straight_offset128(c & 15, g + 8 * (c >> 4));
-  int t_base[2] = {transposed_offset128(0, 0, 0, lane), transposed_offset128(0, 1, 0, lane)};
-  // 192 features: one base per tile part lives across the loop, the derived offsets are formed anew in every interval
-  // (hoisted out of it they would push accumulators into scratch memory)
-  auto refresh_offsets = [&]() __attribute__((always_inline)) {
-    if constexpr (DQK == 192) asm volatile("" : "+v"(s_base), "+v"(x_base), "+v"(t_base[0]), "+v"(t_base[1]));
-  };
-  auto k_frag = [&](const char* kt, int ks) __attribute__((always_inline)) {
-    const int off = kPaired ? x_base ^ (ks << 5) : ks < 8 ? s_base ^ (ks << 5) : L::kFull + (x_base ^ ((ks - 8) << 5));
-    return *reinterpret_cast<const bf16x8*>(kt + off);
-  };
-  auto v_frag = [&](const char* vt, int ks) __attribute__((always_inline)) {
-    return *reinterpret_cast<const bf16x8*>(vt + ((kPaired ? x_base : s_base) ^ (ks << 5)));
-  };
-  auto kt_frag = [&](const char* kt, int j, int i) __attribute__((always_inline)) {
-    int flip, add;
-    if (kPaired) { flip = (i << 6) | (j << 7); add = 0; }
-    else if (i < 4) { flip = i << 6; add = j * 16 * kRowBytes128; }
-    else { flip = ((i - 4) << 6) | (j << 7); add = L::kFull; }
-    return lds_read_transposed_at(kt + (t_base[0] ^ flip) + add, kt + (t_base[1] ^ flip) + add);
-  };
-
-  f32x16 acc[DB];
-#pragma unroll
-  for (int o = 0; o < DB; ++o)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[o][v] = 0.f;
-  f32x16 s, dp;
-  bf16x8 dsf[2];
-
-  auto start = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      s[v] = 0.f;
-      dp[v] = -delta_q;  // dP starts from -delta: dS = P * (dP - delta) without a subtraction per element
-    }
-  };
-  auto scores = [&](const char* kt, const char* vt) __attribute__((always_inline)) {
-    start();
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      s = mfma32(k_frag(kt, ks), qf[ks], s);
-      if (ks < VS) dp = mfma32(v_frag(vt, ks), dof[ks], dp);
-    }
-  };
-  auto accumulate = [&](const char* kt) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int o = 0; o < DB; ++o) acc[o] = mfma32(kt_frag(kt, j, o), dsf[j], acc[o]);
-  };
-  // dQ^T += K(prev)^T dS(prev)^T, then S^T and dP^T of the next tile, fragment reads kAhead products ahead
-  auto matrix_block = [&](const char* kprev, const char* kt, const char* vt) __attribute__((always_inline)) {
-    constexpr int NT = 2 * DB, NS = KS + VS;
-    __builtin_amdgcn_s_setprio(2);
-    bf16x8 at[2][DB], ak[KS], av[VS];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int o = 0; o < DB; ++o) at[j][o] = kt_frag(kprev, j, o);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      ak[ks] = k_frag(kt, ks);
-      if (ks < VS) av[ks] = v_frag(vt, ks);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int o = 0; o < DB; ++o) acc[o] = mfma32(at[j][o], dsf[j], acc[o]);
-    start();
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      s = mfma32(ak[ks], qf[ks], s);
-      if (ks < VS) dp = mfma32(av[ks], dof[ks], dp);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAhead, 0);
-#pragma unroll
-    for (int m = 0; m < NT - kAhead; ++m) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-#pragma unroll
-    for (int m = 0; m < NS; ++m) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-  // P = exp2(kappa s - lse), masked entries 0, dS = P * (dP - delta) -> bf16
-  auto make_ds = [&](int t) __attribute__((always_inline)) {
-    const int n0 = t * kBN;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) s[v] = __builtin_amdgcn_exp2f(s[v] * p.kappa - lse_q);
-    if ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv)) {  // wave-uniform
-      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if (n0 + acc_row(v, g) > limit) s[v] = 0.f;
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) s[v] *= dp[v];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      dsf[j] = to_bf16x8(s[8 * j], s[8 * j + 1], s[8 * j + 2], s[8 * j + 3], s[8 * j + 4], s[8 * j + 5], s[8 * j + 6], s[8 * j + 7]);
-  };
-
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  __syncthreads();
-  scores(kbuf, vbuf);
-  make_ds(0);
-
-  int i = 1;
-  for (; i < n_wave; ++i) {
-    const bool more = i + 2 < n_wg;
-    refresh_offsets();
-    if (more) request(i + 2);
-    matrix_block(kbuf + ((i - 1) & (kSlots - 1)) * L::kKTile, kbuf + (i & (kSlots - 1)) * L::kKTile, vbuf + (i & (kSlots - 1)) * L::kVTile);
-    make_ds(i);
-    // tile i + 1 has landed; the loads just requested may stay in flight (they are the wave's last memory operations)
-    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  }
-  accumulate(kbuf + ((n_wave - 1) & (kSlots - 1)) * L::kKTile);
-  for (; i < n_wg; ++i) {  // waves above the workgroup's last diagonal block keep moving tiles for the others
-    const bool more = i + 2 < n_wg;
-    if (more) request(i + 2);
-    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  }
-  __syncthreads();  // every wave is done with the rings
-
-  OutT* block = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK + q_wave0 * q_row_stride;
-  __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
-  if (sizeof(OutT) == 4 && p.dq_final != nullptr && q_wave0 >= p.final_r0 && q_wave0 < p.final_r1)
-    fin = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + q_wave0 * q_row_stride;
-  char* const turn = smem + wave * kRowsViaLdsBytes<L::kTurnBlocks>;
-#pragma unroll
-  for (int o0 = 0; o0 < DB; o0 += L::kTurnBlocks) {
-    f32x16 part[L::kTurnBlocks];
-#pragma unroll
-    for (int o = 0; o < L::kTurnBlocks; ++o) part[o] = acc[o0 + o];
-    store_rows32_via_lds<OutT, L::kTurnBlocks>(turn, block + 32 * o0, q_row_stride, p.Sq - q_wave0, part, p.scale, p.accumulate != 0, lane,
-                                               fin == nullptr ? nullptr : fin + 32 * o0);
-  }
+__global__ __launch_bounds__(dq_duo::kThreads, 2) void attn_bwd_dq_duo_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[dq_duo::kSmem<DQK>];
+  dq_duo::body<DQK, CAUSAL, OutT>(p, smem, blockIdx.x);
 }
 
 template <int DQK>
 void launch_one(BwdParams p, bool causal, bool f32_out, hipStream_t st) {
-  p.tiles = (p.Sq + kBM - 1) / kBM;
-  const dim3 grid((unsigned)(p.tiles * p.Hq * p.B)), block(kThreads);
+  p.q_tiles = (p.Sq + 127) / 128;
+  const dim3 grid((unsigned)(p.q_tiles * p.Hq * p.B)), block(dq_duo::kThreads);
   if (causal) {
     if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_duo_kernel<DQK, true, float>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((attn_bwd_dq_duo_kernel<DQK, true, __bf16>), grid, block, 0, st, p);

@@ -191,11 +191,10 @@ bool bwd_args(pith_attn_bwd_args& a, const Tensor& q, const Tensor& k, const Ten
   return true;
 }
 
-bool attn_bwd_dkdv_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dk,
-                        const Tensor& dv, double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& dk_pe,
-                        const OptTensor& ds, int64_t zero_tail) {
-  pith_attn_bwd_args a = {};
-  if (!bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds)) return false;
+// dK/dV side of a backward call: outputs and, in `workspace`, the scratch (stream order keeps the block alive until the
+// kernels that use it have run).
+bool dkdv_args(pith_attn_bwd_args& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dk, const Tensor& dv, bool accumulate,
+               const OptTensor& k_pe, const OptTensor& dk_pe, int64_t zero_tail, Tensor& workspace) {
   if (!dk.is_cuda() || dk.device() != q.device() || dv.device() != q.device() || dk.sizes() != k.sizes() || dv.sizes() != v.sizes() ||
       dk.scalar_type() != dv.scalar_type() || !dtype_code(dk, &a.dkv_dtype))
     return false;
@@ -212,21 +211,16 @@ bool attn_bwd_dkdv_into(const Tensor& q, const Tensor& k, const Tensor& v, const
   a.dk = dk.data_ptr(); a.dv = dv.data_ptr();
   a.accumulate_dkv = accumulate;
   a.dkv_zero_tail = zero_tail;
-  Tensor workspace;  // stream order keeps the block alive until the kernels that use it have run
   const int64_t need = pith_attn_bwd_dkdv_workspace_bytes(&a);
   if (need > 0) {
     workspace = empty_like_shape(q, {need}, at::kByte);
     a.workspace = workspace.data_ptr();
     a.workspace_bytes = need;
   }
-  return pith_attn_bwd_dkdv(&a, stream_of(q)) == PITH_OK;
+  return true;
 }
 
-bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
-                      double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& ds, const OptTensor& dq_final,
-                      const Rows& dq_final_rows) {
-  pith_attn_bwd_args a = {};
-  if (!bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds)) return false;
+bool dq_args(pith_attn_bwd_args& a, const Tensor& q, const Tensor& dq, bool accumulate, const OptTensor& dq_final, const Rows& dq_final_rows) {
   int64_t rh;
   if (!dq.is_cuda() || dq.device() != q.device() || dq.sizes() != q.sizes() || !dtype_code(dq, &a.dq_dtype) || !bshd_heads(dq, &a.dq_bs, &rh) ||
       rh != a.q_row_heads)
@@ -240,7 +234,35 @@ bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const T
     a.dq_final = dq_final->data_ptr();
     if (dq_final_rows) a.dq_final_rows[0] = dq_final_rows->first, a.dq_final_rows[1] = dq_final_rows->second;
   }
-  return pith_attn_bwd_dq(&a, stream_of(q)) == PITH_OK;
+  return true;
+}
+
+bool attn_bwd_dkdv_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dk,
+                        const Tensor& dv, double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& dk_pe,
+                        const OptTensor& ds, int64_t zero_tail) {
+  pith_attn_bwd_args a = {};
+  Tensor workspace;
+  return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) && dkdv_args(a, q, k, v, dk, dv, accumulate, k_pe, dk_pe, zero_tail, workspace) &&
+         pith_attn_bwd_dkdv(&a, stream_of(q)) == PITH_OK;
+}
+
+bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
+                      double scale, bool causal, bool accumulate, const OptTensor& k_pe, const OptTensor& ds, const OptTensor& dq_final,
+                      const Rows& dq_final_rows) {
+  pith_attn_bwd_args a = {};
+  return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) && dq_args(a, q, dq, accumulate, dq_final, dq_final_rows) &&
+         pith_attn_bwd_dq(&a, stream_of(q)) == PITH_OK;
+}
+
+// Both of them; `ds` is the hand-over buffer between the two, if any.
+bool attn_bwd_pair_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
+                        const Tensor& dk, const Tensor& dv, double scale, bool causal, bool accumulate_dq, bool accumulate_dkv, const OptTensor& k_pe,
+                        const OptTensor& dk_pe, const OptTensor& ds, int64_t zero_tail, const OptTensor& dq_final, const Rows& dq_final_rows) {
+  pith_attn_bwd_args a = {};
+  Tensor workspace;
+  return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) &&
+         dkdv_args(a, q, k, v, dk, dv, accumulate_dkv, k_pe, dk_pe, zero_tail, workspace) && dq_args(a, q, dq, accumulate_dq, dq_final, dq_final_rows) &&
+         pith_attn_bwd(&a, stream_of(q)) == PITH_OK;
 }
 
 using Two = std::tuple<Tensor, Tensor>;
@@ -288,8 +310,8 @@ Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& 
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    if (attn_bwd_delta_into(o, dout, delta) && attn_bwd_dkdv_into(q, k, v, dout, lse, delta, dk, dv, scale, causal, false, {}, {}, {}, 0) &&
-        attn_bwd_dq_into(q, k, v, dout, lse, delta, dq, scale, causal, false, {}, {}, {}, {}))
+    if (attn_bwd_delta_into(o, dout, delta) &&
+        attn_bwd_pair_into(q, k, v, dout, lse, delta, dq, dk, dv, scale, causal, false, false, {}, {}, {}, 0, {}, {}))
       return {dq, dk, dv};
   }
   return python_body<Three>("attn_bwd", q, k, v, o, lse, dout, scale, causal);
@@ -660,6 +682,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_bwd_delta_into", &attn_bwd_delta_into);
   m.def("attn_bwd_dkdv_into", &attn_bwd_dkdv_into);
   m.def("attn_bwd_dq_into", &attn_bwd_dq_into);
+  m.def("attn_bwd_pair_into", &attn_bwd_pair_into);
   m.def("combine_into", &combine_into);
   m.def("combine_new", &combine_new);
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into);

@@ -129,6 +129,7 @@ SYMBOLS = {
     "pith_attn_bwd_delta": (c_int, [POINTER(AttnDeltaArgs), c_void_p]),
     "pith_attn_bwd_dkdv": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dq": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
+    "pith_attn_bwd": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dkdv_static": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dkdv_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
     "pith_attn_bwd_ds_bytes": (c_int64, [POINTER(AttnBwdArgs)]),

@@ -285,6 +285,9 @@ def attn_bwd_pair_into(
     buf = _try_alloc(plan[1], q.device) if plan is not None else None
     hkv = k.shape[2]
     if buf is None or plan[0] == hkv:
+        if native.attn_bwd_pair_into(q, k, v, dout, lse, delta, dq, dk, dv, softmax_scale, causal, accumulate_dq, accumulate_dkv,
+                                     k_pe, dk_pe, buf, zero_tail, dq_final, dq_final_rows):  # fmt: skip
+            return 0 if buf is None else buf.numel()
         attn_bwd_dkdv_into(q, k, v, dout, lse, delta, dk, dv, softmax_scale, causal, accumulate=accumulate_dkv,
                            k_pe=k_pe, dk_pe=dk_pe, ds=buf, zero_tail=zero_tail)  # fmt: skip
         attn_bwd_dq_into(q, k, v, dout, lse, delta, dq, softmax_scale, causal, accumulate=accumulate_dq, k_pe=k_pe, ds=buf,
