@@ -156,6 +156,29 @@ typedef struct {
 int pith_attn_fwd(const pith_attn_fwd_args* args, pith_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
+ * The same against several key/value chunks at once: softmax over the union of their keys, in one
+ * launch (a ring share whose chunks are all at hand: no partial results, no merges).
+ * args describes the queries, the outputs and what the chunks share (head counts and dims, batch
+ * strides, scale); its k, v, k_pe and Skv are ignored. Chunk i holds `rows` keys that query rows
+ * q_row0 .. Sq-1 see. At most PITH_MAX_CHUNKS of them, sorted by q_row0; with args->causal the LAST
+ * one is the queries' own chunk (rows == Sq, q_row0 = 0), seen under the causal mask. Without it the
+ * first has q_row0 = 0. k_pe is given for all chunks or for none.
+ * The backward call additionally writes dk, dv (and dk_pe) of every chunk: its `rows` first rows, and
+ * zeros in the `zero_tail` rows behind them. */
+#define PITH_MAX_CHUNKS 16
+typedef struct {
+  const void* k;
+  const void* v;
+  const void* k_pe;
+  void* dk;
+  void* dv;
+  void* dk_pe;
+  int64_t rows, q_row0, zero_tail;
+} pith_key_chunk;
+
+int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream);
+
+/* ------------------------------------------------------------------------------------------
  * delta[b,h,s] = sum_d fp32(o[b,s,h,d]) * fp32(dout[b,s,h,d]).
  * Replaces _mla_bwd_preprocess (mla/triton.py:566-574; kernel :101-122). */
 typedef struct {

@@ -1,6 +1,8 @@
 // Declarations shared by the forward kernels.
 #pragma once
 
+#include <type_traits>
+
 #include "attn_tiles.h"
 
 namespace pith {
@@ -33,11 +35,26 @@ struct FwdParams {
   int o_r0, o_r1, acc_r0, acc_r1;  // query rows [r0, r1) that receive o / acc_o when merging (multiples of 32, or Sq)
 };
 
+// The same over several chunks of keys: k, v, k_pe and Skv of the base are unused, its batch strides hold for every chunk.
+struct FwdChunkParams : FwdParams {
+  int n_chunks;
+  KeyChunk chunk[kMaxChunks];
+};
+
+template <bool MULTI>
+using FwdArgs = std::conditional_t<MULTI, FwdChunkParams, FwdParams>;
+__device__ __forceinline__ KeyChunk chunk_of(const FwdParams& p, int) { return KeyChunk{p.k, p.v, p.k_pe, p.Skv, 0}; }
+__device__ __forceinline__ const KeyChunk& chunk_of(const FwdChunkParams& p, int i) { return p.chunk[i]; }
+__device__ __forceinline__ int chunk_count(const FwdParams&) { return 1; }
+__device__ __forceinline__ int chunk_count(const FwdChunkParams& p) { return p.n_chunks; }
+
 // Forward with one 8-wave workgroup per compute unit: attn_fwd_direct.hip. dqk = 128, or 192 with half; half = workgroups
 // of 128 query rows whose wave pairs split the keys of every tile (see there) instead of 256-row workgroups.
 void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipStream_t stream);
+void launch_fwd_direct(const FwdChunkParams& p, int dqk, bool causal, bool half, hipStream_t stream);
 
 // Forward with two (64 features: three) 4-wave workgroups of 128 query rows per compute unit: attn_fwd_duo.hip.
 void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t stream);
+void launch_fwd_duo(const FwdChunkParams& p, int dqk, bool causal, hipStream_t stream);
 
 }  // namespace pith

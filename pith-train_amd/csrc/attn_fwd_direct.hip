@@ -27,8 +27,6 @@
 // workgroups (for launches that would leave compute units idle or badly balanced under the
 // causal mask) and halves the registers per wave that depend on the tile width, at the price of
 // half as many matrix instructions between two barriers.
-#include <type_traits>
-
 #include "attn_fwd_common.h"
 
 namespace pith {
@@ -45,8 +43,8 @@ constexpr int kAhead = 4;  // fragment reads run this many products ahead in the
 constexpr int kTile = kBN * kRowBytes128;  // a packed 128-feature tile of 64 rows
 constexpr int kExtraTile = kExtraTileBytes;  // features 128..191 of 64 keys, two keys per row
 
-template <int DQK, bool HALF, bool CAUSAL>
-__global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) {
+template <int DQK, bool HALF, bool CAUSAL, bool MULTI>
+__global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI> p) {
   constexpr int KS = DQK / 16;    // contraction steps of Q K^T
   constexpr int DVB = kDv / 32;   // 32-row blocks of O^T
   constexpr int KVB = HALF ? 1 : 2;          // 32-key blocks of a tile this wave owns
@@ -81,22 +79,33 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
   const int64_t q_row_stride = (int64_t)p.Hq * DQK;
   const int64_t o_row_stride = (int64_t)p.Hq * kDv;
   // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
-  const bool two_part = DQK == 192 && p.k_pe != nullptr;
+  const bool two_part = DQK == 192 && chunk_of(p, 0).k_pe != nullptr;
   const int k_head_elems = two_part ? 128 : DQK;
   const int k_row_bytes = p.Hkv * k_head_elems * 2, v_row_bytes = p.Hkv * kDv * 2;
   const __bf16* qh = p.q + b * p.q_bs + (int64_t)h * DQK;
-  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
-  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;  // source of features 128..
   const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
-  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
+  // a chunk's first row in K, in the source of features 128.. and in V
+  auto k_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).k + b * p.k_bs + (int64_t)hk * k_head_elems);
+  };
+  auto kx_rows = [&](int id) __attribute__((always_inline)) {
+    return two_part ? reinterpret_cast<const char*>(chunk_of(p, id).k_pe + b * p.k_pe_bs) : k_rows(id);
+  };
+  auto v_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).v + b * p.v_bs + (int64_t)hk * kDv);
+  };
 
   // Number of key tiles this workgroup / this wavefront has to visit.
-  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
-  int n_tiles_wg = n_tiles_all, n_tiles_wave = n_tiles_all;
+  const ChunkRange<MULTI, CAUSAL, kBN> range(p, m0 + kBM);
+  int n_tiles_wg = range.tiles_full, n_tiles_wave = range.tiles_full;
   if (CAUSAL) {
-    n_tiles_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
-    n_tiles_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
+    const int tiles = (chunk_of(p, range.last).rows + kBN - 1) / kBN;
+    n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
+    n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
+  TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows),
+      v_src(p, range, v_row_bytes, v_rows);
+  TileMask<MULTI, CAUSAL, kBN> mask(p, range);
 
   DirectTile128<kBN, kThreads> mover, kmover;  // V tiles (and K tiles when the row pitches agree); K tiles otherwise
   DirectExtra64 xmover;
@@ -105,18 +114,21 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
     kmover.init(k_row_bytes, wave, lane);
     xmover.init(kx_row_bytes, two_part ? 0 : 256, wave, lane);
   }
+  // (tiles are requested strictly in order, so the sources just move on)
   auto issue_k = [&](int t) __attribute__((always_inline)) {
     char* slot = kbuf + (t & (kSlots - 1)) * kKTile;
-    const char* src = kh + (int64_t)t * kBN * k_row_bytes;
     if constexpr (DQK != kDv) {
-      kmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
-      xmover.issue(kx + (int64_t)t * kBN * kx_row_bytes, p.Skv - t * kBN, slot + kTile, wave, lane);
+      kmover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
+      xmover.issue(kx_src.src(t), kx_src.left(t), slot + kTile, wave, lane);
+      kx_src.advance(p, range, kx_rows);
     } else {
-      mover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+      mover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
     }
+    k_src.advance(p, range, k_rows);
   };
   auto issue_v = [&](int t) __attribute__((always_inline)) {
-    mover.issue(vh + (int64_t)t * kBN * v_row_bytes, p.Skv - t * kBN, vbuf + (t & (kSlots - 1)) * kTile, wave, lane);
+    mover.issue(v_src.src(t), v_src.left(t), vbuf + (t & (kSlots - 1)) * kTile, wave, lane);
+    v_src.advance(p, range, v_rows);
   };
   // tiles needed by the prologue (K 0), interval 0 (K 1, V 0) and interval 1 (K 2, V 1)
   issue_k(0);
@@ -200,20 +212,19 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
       for (int kvb = 0; kvb < KVB; ++kvb) s[kvb] = mfma32(k_frag(ktile, ks, kvb), qf[ks], s[kvb]);
   };
 
-  // ---- mask, online softmax (one query column per lane pair), P^T fragments
+  // ---- mask, online softmax of the next tile in order (one query column per lane pair), P^T fragments
   auto softmax = [&](int t) __attribute__((always_inline)) {
-    const int n0 = t * kBN;
-    if ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv)) {
-      // tile crossing the diagonal of a causal chunk, or a ragged last tile
-      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;  // last visible key
+    if (mask.partial(range, t, q_wave0)) {
+      const int limit = mask.limit(range, qrow);
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int key = n0 + (kvb0 + kvb) * 32 + acc_row(v, g);
+          const int key = mask.key0(t) + (kvb0 + kvb) * 32 + acc_row(v, g);
           if (key > limit) s[kvb][v] = -INFINITY;
         }
     }
+    mask.advance(p, range);
     f32x16 e[KVB];
     float rs = 0.f;
     // The running maximum is refreshed lazily, and whether a refresh is due is read off the row sum instead of a
@@ -493,24 +504,30 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdParams p) 
   if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
-template <int DQK, bool HALF>
-void launch_one(FwdParams p, bool causal, hipStream_t st) {
+template <int DQK, bool HALF, bool MULTI>
+void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   constexpr int kBM = HALF ? 128 : 256;
   p.m_tiles = (p.Sq + kBM - 1) / kBM;
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
-  if (causal) hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false>), grid, block, 0, st, p);
+  if (causal) hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, MULTI>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false, MULTI>), grid, block, 0, st, p);
+}
+
+template <bool MULTI>
+void launch_split(const FwdArgs<MULTI>& p, int dqk, bool causal, bool half, hipStream_t st) {
+  if (dqk == 192) launch_one<192, true, MULTI>(p, causal, st);
+  else if (half) launch_one<128, true, MULTI>(p, causal, st);
+  else launch_one<128, false, MULTI>(p, causal, st);
 }
 
 }  // namespace
 
 void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipStream_t st) {
-  if (dqk == 128) {
-    if (half) launch_one<128, true>(p, causal, st);
-    else launch_one<128, false>(p, causal, st);
-  } else {
-    launch_one<192, true>(p, causal, st);
-  }
+  launch_split<false>(p, dqk, causal, half, st);
+}
+
+void launch_fwd_direct(const FwdChunkParams& p, int dqk, bool causal, bool half, hipStream_t st) {
+  launch_split<true>(p, dqk, causal, half, st);
 }
 
 }  // namespace pith

@@ -36,8 +36,8 @@ struct DuoLayout {
   static constexpr int kSmem = kRings > kTurn ? kRings : kTurn;
 };
 
-template <int DQK, bool CAUSAL>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) {
+template <int DQK, bool CAUSAL, bool MULTI>
+__global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI> p) {
   using L = DuoLayout<DQK>;
   constexpr int kDv = L::kDv, KS = DQK / 16, DVB = kDv / 32, KVB = 2;
   constexpr bool kPaired = DQK == 64;  // tiles hold two rows per 256-byte LDS row
@@ -60,22 +60,33 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) 
   const int64_t q_row_stride = (int64_t)p.Hq * DQK;
   const int64_t o_row_stride = (int64_t)p.Hq * kDv;
   // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
-  const bool two_part = DQK == 192 && p.k_pe != nullptr;
+  const bool two_part = DQK == 192 && chunk_of(p, 0).k_pe != nullptr;
   const int k_head_elems = two_part ? 128 : DQK;
   const int k_row_bytes = p.Hkv * k_head_elems * 2, v_row_bytes = p.Hkv * kDv * 2;
   const __bf16* qh = p.q + b * p.q_bs + (int64_t)h * DQK;
-  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
-  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;
   const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
-  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
+  // a chunk's first row in K, in the source of features 128.. and in V
+  auto k_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).k + b * p.k_bs + (int64_t)hk * k_head_elems);
+  };
+  auto kx_rows = [&](int id) __attribute__((always_inline)) {
+    return two_part ? reinterpret_cast<const char*>(chunk_of(p, id).k_pe + b * p.k_pe_bs) : k_rows(id);
+  };
+  auto v_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).v + b * p.v_bs + (int64_t)hk * kDv);
+  };
 
   // Number of key tiles this workgroup / this wavefront has to visit.
-  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
-  int n_tiles_wg = n_tiles_all, n_tiles_wave = n_tiles_all;
+  const ChunkRange<MULTI, CAUSAL, kBN> range(p, m0 + kBM);
+  int n_tiles_wg = range.tiles_full, n_tiles_wave = range.tiles_full;
   if (CAUSAL) {
-    n_tiles_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
-    n_tiles_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
+    const int tiles = (chunk_of(p, range.last).rows + kBN - 1) / kBN;
+    n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
+    n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
+  TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows),
+      v_src(p, range, v_row_bytes, v_rows);
+  TileMask<MULTI, CAUSAL, kBN> mask(p, range);
 
   DirectTile128<kBN, kThreads> vmover, kmover;
   DirectPaired64<kBN, kThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
@@ -87,21 +98,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) 
     kmover.init(k_row_bytes, wave, lane);
     if constexpr (DQK == 192) kpmover.init(kx_row_bytes, two_part ? 0 : 256, wave, lane);
   }
+  // (tiles are requested strictly in order, so the sources just move on)
   auto issue_k = [&](int t) __attribute__((always_inline)) {
     char* slot = kbuf + (t & 1) * L::kKTile;
-    const char* src = kh + (int64_t)t * kBN * k_row_bytes;
     if constexpr (kPaired) {
-      kpmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+      kpmover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
     } else {
-      kmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
-      if constexpr (DQK == 192) kpmover.issue(kx + (int64_t)t * kBN * kx_row_bytes, p.Skv - t * kBN, slot + kTile, wave, lane);
+      kmover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
+      if constexpr (DQK == 192) {
+        kpmover.issue(kx_src.src(t), kx_src.left(t), slot + kTile, wave, lane);
+        kx_src.advance(p, range, kx_rows);
+      }
     }
+    k_src.advance(p, range, k_rows);
   };
   auto issue_v = [&](int t) __attribute__((always_inline)) {
     char* slot = vbuf + (t & 1) * L::kVTile;
-    const char* src = vh + (int64_t)t * kBN * v_row_bytes;
-    if constexpr (kPaired) vpmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
-    else vmover.issue(src, p.Skv - t * kBN, slot, wave, lane);
+    if constexpr (kPaired) vpmover.issue(v_src.src(t), v_src.left(t), slot, wave, lane);
+    else vmover.issue(v_src.src(t), v_src.left(t), slot, wave, lane);
+    v_src.advance(p, range, v_rows);
   };
   issue_k(0);
   issue_v(0);
@@ -155,19 +170,19 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) 
       for (int kvb = 0; kvb < KVB; ++kvb) s[kvb] = mfma32(k_frag(ktile, ks, kvb), qf[ks], s[kvb]);
   };
 
-  // ---- mask, online softmax (one query column per lane pair), P^T fragments
+  // ---- mask, online softmax of the next tile in order (one query column per lane pair), P^T fragments
   auto softmax = [&](int t) __attribute__((always_inline)) {
-    const int n0 = t * kBN;
-    if ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv)) {
-      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
+    if (mask.partial(range, t, q_wave0)) {
+      const int limit = mask.limit(range, qrow);
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int key = n0 + kvb * 32 + acc_row(v, g);
+          const int key = mask.key0(t) + kvb * 32 + acc_row(v, g);
           if (key > limit) s[kvb][v] = -INFINITY;
         }
     }
+    mask.advance(p, range);
     f32x16 e[KVB];
     float rs = 0.f;
     // lazily refreshed running maximum, tested on the row sum (attn_fwd_direct.hip)
@@ -319,20 +334,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdParams p) 
   if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
-template <int DQK>
-void launch_one(FwdParams p, bool causal, hipStream_t st) {
+template <int DQK, bool MULTI>
+void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   p.m_tiles = (p.Sq + kBM - 1) / kBM;
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
-  if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false>), grid, block, 0, st, p);
+  if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, MULTI>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false, MULTI>), grid, block, 0, st, p);
+}
+
+template <bool MULTI>
+void launch_dim(const FwdArgs<MULTI>& p, int dqk, bool causal, hipStream_t st) {
+  if (dqk == 64) launch_one<64, MULTI>(p, causal, st);
+  else if (dqk == 128) launch_one<128, MULTI>(p, causal, st);
+  else launch_one<192, MULTI>(p, causal, st);
 }
 
 }  // namespace
 
-void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t st) {
-  if (dqk == 64) launch_one<64>(p, causal, st);
-  else if (dqk == 128) launch_one<128>(p, causal, st);
-  else launch_one<192>(p, causal, st);
-}
+void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t st) { launch_dim<false>(p, dqk, causal, st); }
+
+void launch_fwd_duo(const FwdChunkParams& p, int dqk, bool causal, hipStream_t st) { launch_dim<true>(p, dqk, causal, st); }
 
 }  // namespace pith

@@ -10,7 +10,7 @@
 // row 16*j + 8*(e/4) + 4*g + e%4 of the tile ("slot order"). The other operand of that product
 // is fetched from LDS in the same slot order.
 //
-// Tiles streamed through LDS are row-major [row][col] bf16 with a padded pitch. They are read
+// Tiles streamed through LDS are packed, swizzled rows (see below). They are read
 //   - "straight": lane takes 8 consecutive columns of row c            (one ds_read_b128), or
 //   - "transposed": lane takes column c at 8 rows in slot order         (two ds_read_b64_tr_b16).
 #pragma once
@@ -25,32 +25,11 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Straight A/B fragment: row `row`, columns col0 .. col0+7 (col0 multiple of 8).
-__device__ __forceinline__ bf16x8 lds_read_straight(const char* tile, int pitch, int row, int col0) {
-  return *reinterpret_cast<const bf16x8*>(tile + row * pitch + col0 * 2);
-}
-
-// Transposed fragment in slot order. For a wavefront the result is the A (or B) operand whose
-// non-contracted index is the tile COLUMN col_base + c and whose contraction slots (g, e) are
-// the tile ROWS row_base + 8*(e/4) + 4*g + e%4.
-// ds_read_b64_tr_b16 works on blocks of 16 lanes: lane r of a block supplies the address of 4
+// Transposed fragments in slot order: for a wavefront the A (or B) operand whose non-contracted index is the tile COLUMN
+// col_base + c and whose contraction slots (g, e) are the tile ROWS row_base + 8*(e/4) + 4*g + e%4 (lds_read_transposed_at
+// below). ds_read_b64_tr_b16 works on blocks of 16 lanes: lane r of a block supplies the address of 4
 // consecutive columns; lanes 4i..4i+3 of the block must cover 16 consecutive columns of row i;
 // lane r then receives column r of rows 0..3 of the block.
-__device__ __forceinline__ bf16x8 lds_read_transposed(const char* tile, int pitch, int row_base, int col_base,
-                                                      int lane) {
-  const int r = lane & 15, blk = lane >> 4;
-  const int row = row_base + 4 * (blk >> 1) + (r >> 2);
-  const int col = col_base + 16 * (blk & 1) + 4 * (r & 3);
-  const char* p = tile + row * pitch + col * 2;
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 8 * pitch));
-  typedef __attribute__((ext_vector_type(8))) short s16x8;
-  s16x8 v;
-  v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-  v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-  return __builtin_bit_cast(bf16x8, v);
-}
 
 // Row index (0..31) inside a 32x32 result tile of accumulator element v for lane group g.
 __device__ __forceinline__ int acc_row(int v, int g) { return 8 * (v >> 2) + 4 * g + (v & 3); }
@@ -74,14 +53,6 @@ __device__ __forceinline__ bf16x8 to_bf16x8(float a0, float a1, float a2, float 
   r[0] = (__bf16)a0; r[1] = (__bf16)a1; r[2] = (__bf16)a2; r[3] = (__bf16)a3;
   r[4] = (__bf16)a4; r[5] = (__bf16)a5; r[6] = (__bf16)a6; r[7] = (__bf16)a7;
   return r;
-}
-
-// Waits until every vector-memory load issued so far has returned. Placed once before a main
-// loop, after the loop-invariant fragments were fetched: otherwise the compiler keeps the waits
-// for those fragments inside the loop, where they also wait for the loads that prefetch the next
-// tile and so expose the global-memory latency in every iteration.
-__device__ __forceinline__ void wait_all_vector_loads() {
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), expcnt and lgkmcnt left at their maxima
 }
 
 // Maps a linear workgroup id to (tile, head, batch) so that
@@ -118,40 +89,110 @@ __device__ __forceinline__ void decode_block(int linear, int heads, int batch, i
   h = pos - b * heads;
 }
 
-// Cooperative copy of a [ROWS x COLS] bf16 tile between global memory and LDS by THREADS threads,
-// split into a "fetch to registers" half and a "store to LDS" half so that the global loads of
-// the next tile can be in flight while the current tile is consumed.
-template <int ROWS, int COLS, int PITCH, int THREADS>
-struct TileCopy {
-  static constexpr int kChunksPerRow = COLS / 8;
-  static constexpr int kChunks = ROWS * kChunksPerRow;
-  static constexpr int kPerThread = (kChunks + THREADS - 1) / THREADS;
-  u32x4 regs[kPerThread];
+// ---------------------------------------------------------------------------------------------
+// Several K/V chunks in one launch. A ring share attends its queries to one chunk per ring step; where all of them are at
+// hand, a query-stationary workgroup simply walks the key tiles of every chunk its rows can see as one stream: no partial
+// results, no merges, one set of first tiles and one epilogue. The chunks come sorted: those without a causal mask by the
+// first query row that sees them, then (CAUSAL kernels) the chunk that holds the queries' own keys, under the mask.
+constexpr int kMaxChunks = PITH_MAX_CHUNKS;
+struct KeyChunk {
+  const __bf16* k;
+  const __bf16* v;
+  const __bf16* k_pe;  // keys in two parts (the same for all chunks: all or none)
+  int rows;            // keys of the chunk
+  int q_row0;          // query rows below do not see it
+};
 
-  // src: address of element [row 0][col 0] of the tile's head slice; row_stride in elements;
-  // rows at or beyond `valid_rows` are read from the last valid row (their values are masked
-  // or discarded by the caller).
-  __device__ __forceinline__ void fetch(const __bf16* src, int64_t row_stride, int row0, int valid_rows, int tid) {
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      const int c = tid + i * THREADS;
-      if (kChunks % THREADS == 0 || c < kChunks) {
-        const int row = c / kChunksPerRow, col = c - row * kChunksPerRow;
-        int grow = row0 + row;
-        grow = grow < valid_rows ? grow : valid_rows - 1;
-        regs[i] = *reinterpret_cast<const u32x4*>(src + grow * row_stride + col * 8);
+// How a workgroup walks its stream. MULTI = false: one chunk, addressed by the tile number, which costs nothing beyond what
+// a kernel without chunks costs; MULTI = true: several, tiles taken strictly in order (the scalar state of three walks
+// measured 1 us per launch and 1-4 % in the loops: worth it only where it saves launches and merges). The kernels'
+// parameters P come with chunk_of(p, id) and chunk_count(p).
+//
+// The chunks that query rows below row_end see: ids 0 .. n_full-1 and, CAUSAL, the last one.
+template <bool MULTI, bool CAUSAL, int BN>
+struct ChunkRange {
+  int n_full, last, tiles_full;
+  template <typename P>
+  __device__ __forceinline__ ChunkRange(const P& p, int row_end) {
+    if constexpr (MULTI) {
+      last = chunk_count(p) - 1;
+      n_full = tiles_full = 0;
+      const int most = CAUSAL ? last : last + 1;
+      while (n_full < most && chunk_of(p, n_full).q_row0 < row_end) {
+        tiles_full += (chunk_of(p, n_full).rows + BN - 1) / BN;
+        ++n_full;
+      }
+    } else {
+      last = 0;
+      n_full = CAUSAL ? 0 : 1;
+      tiles_full = CAUSAL ? 0 : (chunk_of(p, 0).rows + BN - 1) / BN;
+    }
+  }
+  // the chunk behind chunk i of the stream
+  __device__ __forceinline__ int next(int i) const { return i + 1 < n_full ? i + 1 : last; }
+  __device__ __forceinline__ int first() const { return MULTI && n_full == 0 ? last : 0; }
+};
+
+// Where the requests for one operand stand: address of a tile's first row (`base(chunk id)` gives the chunk's) and rows left
+// from it on. Wave-uniform.
+template <bool MULTI, bool CAUSAL, int BN>
+struct TileSource {
+  int id, rows_left, row_bytes;
+  const char* at;
+  template <typename P, typename Base>
+  __device__ __forceinline__ TileSource(const P& p, const ChunkRange<MULTI, CAUSAL, BN>& r, int row_bytes_, Base base) {
+    id = r.first();
+    rows_left = chunk_of(p, id).rows;
+    row_bytes = row_bytes_;
+    at = base(id);
+  }
+  __device__ __forceinline__ const char* src(int t) const { return MULTI ? at : at + (int64_t)t * BN * row_bytes; }
+  __device__ __forceinline__ int left(int t) const { return MULTI ? rows_left : rows_left - t * BN; }
+  template <typename P, typename Base>
+  __device__ __forceinline__ void advance(const P& p, const ChunkRange<MULTI, CAUSAL, BN>& r, Base base) {
+    if constexpr (MULTI) {
+      rows_left -= BN;
+      at += BN * row_bytes;
+      if (rows_left <= 0) {
+        id = r.next(id);
+        rows_left = chunk_of(p, id).rows;
+        at = base(id);
       }
     }
   }
-  __device__ __forceinline__ void commit(char* tile, int tid) const {
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      const int c = tid + i * THREADS;
-      if (kChunks % THREADS == 0 || c < kChunks) {
-        const int row = c / kChunksPerRow, col = c - row * kChunksPerRow;
-        *reinterpret_cast<u32x4*>(tile + row * PITCH + col * 16) = regs[i];
-      }
+};
+
+// Where the softmax stands: which keys of its tile a query row may see.
+template <bool MULTI, bool CAUSAL, int BN>
+struct TileMask {
+  int id, first_key, rows, q_row0;
+  template <typename P>
+  __device__ __forceinline__ void enter(const P& p, int i) {
+    id = i;
+    first_key = 0;
+    rows = chunk_of(p, i).rows;
+    q_row0 = MULTI ? chunk_of(p, i).q_row0 : 0;
+  }
+  template <typename P>
+  __device__ __forceinline__ TileMask(const P& p, const ChunkRange<MULTI, CAUSAL, BN>& r) { enter(p, r.first()); }
+  template <typename P>
+  __device__ __forceinline__ void advance(const P& p, const ChunkRange<MULTI, CAUSAL, BN>& r) {
+    if constexpr (MULTI) {
+      first_key += BN;
+      if (first_key >= rows) enter(p, r.next(id));
     }
+  }
+  __device__ __forceinline__ int key0(int t) const { return MULTI ? first_key : t * BN; }
+  __device__ __forceinline__ bool diagonal(const ChunkRange<MULTI, CAUSAL, BN>& r) const { return CAUSAL && (!MULTI || id == r.last); }
+  // whether some of the wave's query rows from q0 on do not see the whole tile: it crosses the diagonal, is a chunk's ragged
+  // last one, or belongs to a chunk that only later rows see
+  __device__ __forceinline__ bool partial(const ChunkRange<MULTI, CAUSAL, BN>& r, int t, int q0) const {
+    return (diagonal(r) && key0(t) + BN - 1 > q0) || key0(t) + BN > rows || (MULTI && q0 < q_row0);
+  }
+  // last key of the chunk that row `qrow` sees (-1: none)
+  __device__ __forceinline__ int limit(const ChunkRange<MULTI, CAUSAL, BN>& r, int qrow) const {
+    const int l = diagonal(r) ? min(qrow, rows - 1) : rows - 1;
+    return MULTI && qrow < q_row0 ? -1 : l;
   }
 };
 
@@ -330,7 +371,7 @@ struct DirectPaired64 {
 // rows * 256 bytes), features 8*piece .. 8*piece+7.
 __device__ __forceinline__ int straight_offset128(int row, int piece) { return swizzled_offset(row, piece); }
 
-// Offset for one ds_read_b64_tr_b16 of a transposed fragment (see lds_read_transposed): tile
+// Offset for one ds_read_b64_tr_b16 of a transposed fragment: tile
 // rows row_base + 8*half + 4*(blk>>1) + (r>>2), features col_base + 16*(blk&1) + 4*(r&3) .. +3.
 // row_base must be a multiple of 16, col_base a multiple of 32.
 __device__ __forceinline__ int transposed_offset128(int row_base, int half, int col_base, int lane) {

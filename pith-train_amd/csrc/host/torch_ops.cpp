@@ -265,6 +265,66 @@ bool attn_bwd_pair_into(const Tensor& q, const Tensor& k, const Tensor& v, const
          pith_attn_bwd(&a, stream_of(q)) == PITH_OK;
 }
 
+// ---------------------------------------------------------------------------------------------
+// One rank's ring share with all of its chunks at hand (operators/ring_attention/local.py): every chunk in one launch.
+
+struct RingChunks {
+  std::vector<pith_key_chunk> chunk;  // as pith_attn_fwd_chunks wants them: the own chunk, under the mask, last
+  std::vector<int64_t> rank;          // owner of each
+};
+
+// The chunks rank `rank` of `cp` visits, in ring order, and in `a` what they share. False: not a case for the chunk calls.
+template <typename Args>
+bool ring_chunks(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes,
+                 int64_t rank, int64_t cp, bool zigzag, Args& a, RingChunks& r) {
+  if (!is_gpu_bf16(q, 4) || !q.is_contiguous() || rank < 0 || rank >= cp || (int64_t)ks.size() != cp || (int64_t)vs.size() != cp || (pes && (int64_t)pes->size() != cp))
+    return false;
+  const int64_t s = q.size(1);
+  if (zigzag && s % 2) return false;
+  for (int64_t step = 1; step <= cp; ++step) {
+    const int64_t j = (rank - step + cp) % cp;  // the own chunk comes last
+    if (!zigzag && j > rank) continue;
+    if (!ks[j] || !vs[j] || (pes && !(*pes)[j])) return false;
+    const Tensor &k = *ks[j], &v = *vs[j];
+    if (!qkv_ok(q, k, v, true, pes.has_value()) || !k.is_contiguous() || !v.is_contiguous() || k.size(2) != ks[rank]->size(2)) return false;
+    pith_key_chunk c = {};
+    c.k = k.data_ptr(); c.v = v.data_ptr();
+    c.rows = zigzag && j < rank ? s / 2 : s;
+    c.q_row0 = j > rank ? s / 2 : 0;
+    c.zero_tail = s - c.rows;
+    int64_t pe_bs = 0, pe_rs = 0;
+    if (pes && !k_pe_fields(k, *(*pes)[j], &c.k_pe, &pe_bs, &pe_rs)) return false;
+    if (!r.chunk.empty() && (pe_bs != a.k_pe_bs || pe_rs != a.k_pe_rs)) return false;
+    a.k_pe_bs = pe_bs; a.k_pe_rs = pe_rs;
+    r.chunk.push_back(c);
+    r.rank.push_back(j);
+  }
+  if (r.chunk.size() > PITH_MAX_CHUNKS) return false;
+  const Tensor &k = *ks[rank], &v = *vs[rank];
+  a.q = q.data_ptr();
+  a.B = q.size(0); a.Sq = s; a.Hq = q.size(2); a.Hkv = k.size(2); a.Dqk = q.size(3); a.Dv = v.size(3);
+  a.q_bs = s * a.Hq * a.Dqk; a.k_bs = s * a.Hkv * k.size(3); a.v_bs = s * a.Hkv * a.Dv;
+  a.lse_bs = a.Hq * s; a.lse_hs = s;
+  a.causal = 1;
+  return true;
+}
+
+// (out, lse), or None when the steps have to run one by one.
+std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs,
+                                                       const std::optional<std::vector<OptTensor>>& pes, double scale, int64_t rank, int64_t cp,
+                                                       bool zigzag) {
+  pith_attn_fwd_args a = {};
+  RingChunks r;
+  if (!ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r)) return std::nullopt;
+  Tensor o = at::empty({a.B, a.Sq, a.Hq, a.Dv}, q.options());
+  Tensor lse = empty_like_shape(q, {a.B, a.Hq, a.Sq}, at::kFloat);
+  a.o = o.data_ptr(); a.lse = lse.data_ptr<float>();
+  a.o_bs = a.Sq * a.Hq * a.Dv;
+  a.scale = (float)scale;
+  if (pith_attn_fwd_chunks(&a, r.chunk.data(), (int64_t)r.chunk.size(), stream_of(q)) != PITH_OK) return std::nullopt;
+  return std::make_tuple(o, lse);
+}
+
 using Two = std::tuple<Tensor, Tensor>;
 using Three = std::tuple<Tensor, Tensor, Tensor>;
 using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
@@ -683,6 +743,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_bwd_dkdv_into", &attn_bwd_dkdv_into);
   m.def("attn_bwd_dq_into", &attn_bwd_dq_into);
   m.def("attn_bwd_pair_into", &attn_bwd_pair_into);
+  m.def("ring_forward", &ring_forward);
   m.def("combine_into", &combine_into);
   m.def("combine_new", &combine_new);
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into);

@@ -61,6 +61,13 @@ class AttnFwdArgs(Structure):
     ]  # fmt: skip
 
 
+class KeyChunk(Structure):
+    _fields_ = [
+        ("k", c_void_p), ("v", c_void_p), ("k_pe", c_void_p), ("dk", c_void_p), ("dv", c_void_p), ("dk_pe", c_void_p),
+        ("rows", c_int64), ("q_row0", c_int64), ("zero_tail", c_int64),
+    ]  # fmt: skip
+
+
 class AttnDeltaArgs(Structure):
     _fields_ = [
         ("o", c_void_p), ("dout", c_void_p), ("delta", c_void_p),
@@ -126,6 +133,7 @@ SYMBOLS = {
     "pith_device_info": (c_int, [c_int, POINTER(DeviceInfo)]),
     "pith_combine": (c_int, [POINTER(CombineArgs), c_void_p]),
     "pith_attn_fwd": (c_int, [POINTER(AttnFwdArgs), c_void_p]),
+    "pith_attn_fwd_chunks": (c_int, [POINTER(AttnFwdArgs), POINTER(KeyChunk), c_int64, c_void_p]),
     "pith_attn_bwd_delta": (c_int, [POINTER(AttnDeltaArgs), c_void_p]),
     "pith_attn_bwd_dkdv": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dq": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
@@ -223,6 +231,6 @@ def bhs_strides(t: torch.Tensor, what: str):
 
 
 __all__ = [
-    "lib", "check", "PithError", "CombineArgs", "AttnFwdArgs", "AttnDeltaArgs", "AttnBwdArgs", "NormRopeArgs", "MlaAssembleArgs", "DeviceInfo", "SYMBOLS",
+    "lib", "check", "PithError", "CombineArgs", "AttnFwdArgs", "KeyChunk", "AttnDeltaArgs", "AttnBwdArgs", "NormRopeArgs", "MlaAssembleArgs", "DeviceInfo", "SYMBOLS",
     "dtype_code", "current_stream", "require_device", "bshd_batch_stride", "bshd_head_range_strides", "bhs_strides", "byref",
 ]  # fmt: skip

@@ -41,6 +41,7 @@ from typing import List, Sequence, Tuple
 import torch
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import native
 from pithtrain_amd.operators.mla.hip import (
     FINAL_DQ_HEAD_DIMS,
     MERGING_HEAD_DIMS,
@@ -51,6 +52,9 @@ from pithtrain_amd.operators.mla.hip import (
 from pithtrain_amd.operators.ring_attention.combine import cast_f32_bf16_into, combine_into
 
 LAYOUTS = ("contiguous", "zigzag")
+# A share whose chunks are all at hand runs as one launch over all of them; False restores one launch per step (what a
+# share has to do whose chunks arrive one by one; kept for comparison runs).
+FUSE_CHUNKS = True
 # Ring steps after the first merge inside the forward kernel (one launch per step) where the kernels support it;
 # False restores chunk forward + combine launch per step (kept for comparison runs).
 FUSE_MERGE = True
@@ -358,6 +362,10 @@ def ring_forward_local(
 
     k_chunks[j] / v_chunks[j] are the K/V chunks owned by rank j (entries the schedule never
     visits may be None); with k_pe_chunks the keys come in two parts (k_chunks = k_nope)."""
+    if layout in LAYOUTS and FUSE_CHUNKS:
+        done = native.ring_forward(q, k_chunks, v_chunks, k_pe_chunks, softmax_scale, cp_rank, cp_size, layout == "zigzag")
+        if done is not None:
+            return done
     steps = ring_schedule(cp_rank, cp_size, q.shape[1], layout)
     fwd = RingForward(q, v_chunks[cp_rank].shape[-1], softmax_scale, steps, layout)
     for st in steps:
