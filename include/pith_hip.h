@@ -159,10 +159,9 @@ int pith_attn_fwd(const pith_attn_fwd_args* args, pith_stream_t stream);
  * The same against several key/value chunks at once: softmax over the union of their keys, in one
  * launch (a ring share whose chunks are all at hand: no partial results, no merges).
  * args describes the queries, the outputs and what the chunks share (head counts and dims, batch
- * strides, scale); its k, v, k_pe and Skv are ignored. Chunk i holds `rows` keys that query rows
- * q_row0 .. Sq-1 see. At most PITH_MAX_CHUNKS of them, sorted by q_row0; with args->causal the LAST
- * one is the queries' own chunk (rows == Sq, q_row0 = 0), seen under the causal mask. Without it the
- * first has q_row0 = 0. k_pe is given for all chunks or for none.
+ * strides, scale); its k, v, k_pe, Skv and causal are ignored. Chunk i holds `rows` keys that query rows
+ * q_row0 .. Sq-1 see. At most PITH_MAX_CHUNKS of them, sorted by q_row0, and LAST the queries' own
+ * chunk (rows == Sq, q_row0 = 0), seen under the causal mask. k_pe is given for all chunks or for none.
  * The backward call additionally writes dk, dv (and dk_pe) of every chunk: its `rows` first rows, and
  * zeros in the `zero_tail` rows behind them. */
 #define PITH_MAX_CHUNKS 16
@@ -271,6 +270,13 @@ int pith_attn_bwd_dq(const pith_attn_bwd_args* args, pith_stream_t stream);
  * Without a usable `ds` the two do not depend on each other, and where that pays (grids that do not fill the
  * device many times over) they run as one grid instead of one after the other. */
 int pith_attn_bwd(const pith_attn_bwd_args* args, pith_stream_t stream);
+
+/* The same against several chunks at once (pith_key_chunk, conventions of pith_attn_fwd_chunks): dq is written once, over
+ * all chunks, and dk, dv (dk_pe) of every chunk. args describes the query side and what the chunks share; its k, v, k_pe,
+ * Skv, causal, dk, dv, dk_pe, dkv_zero_tail and ds are ignored. Gradients are bf16, nothing is accumulated. The workspace is
+ * required wherever pith_attn_bwd_chunks_workspace_bytes is not 0. */
+int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n);
+int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream);
 
 /* Scratch size with which pith_attn_bwd_dkdv runs fastest for these shapes (0 = none needed).
  * With grouped-query attention and few key rows the kernel spreads the query heads of a group

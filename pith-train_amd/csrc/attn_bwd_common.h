@@ -1,6 +1,8 @@
 // Declarations shared by the two backward kernels (dQ and dK/dV).
 #pragma once
 
+#include <type_traits>
+
 #include "attn_tiles.h"
 
 namespace pith {
@@ -45,11 +47,66 @@ struct BwdParams {
   __bf16* dq_final;
   int64_t dq_final_bs;
   int final_r0, final_r1;
-  // dK/dV kernels: blocks main_blocks .. of the grid clear rows [Skv, Skv + zero_tail) of dk and dv
+  // dK/dV kernels: blocks main_blocks .. of the grid clear rows [Skv, Skv + zero_tail) of dk and dv, and of dk_pe if
+  // that is given (a chunk call; rows of 64 features)
   int zero_tail, main_blocks;
+  __bf16* dk_pe;
+  int64_t dk_pe_bs;
   // dK/dV for head dims (128, 128), causal: launch the instance that visits the query tiles from the last one down
   int walk_desc;
 };
+
+// The backward over several chunks of keys in one launch (bf16 gradients, the last chunk under the causal mask). Of the base,
+// the query side, the strides and the split hold for every chunk; the dK/dV workgroups replace the rest by their chunk's.
+struct BwdChunk {
+  KeyChunk key;
+  __bf16* dk;
+  __bf16* dv;
+  __bf16* dk_pe;
+  int tiles, zero_tail;   // as in BwdParams
+  int first_block;        // of the dK/dV grid
+  int rows_before;        // keys of the chunks in front: where the chunk's part of the workspaces lies
+};
+struct BwdChunkParams : BwdParams {
+  int n_chunks;
+  BwdChunk chunk[kMaxChunks];
+};
+
+template <bool MULTI>
+using BwdArgs = std::conditional_t<MULTI, BwdChunkParams, BwdParams>;
+__device__ __forceinline__ KeyChunk chunk_of(const BwdParams& p, int) { return KeyChunk{p.k, p.v, p.k_pe, p.Skv, 0}; }
+__device__ __forceinline__ const KeyChunk& chunk_of(const BwdChunkParams& p, int i) { return p.chunk[i].key; }
+__device__ __forceinline__ int chunk_count(const BwdParams&) { return 1; }
+__device__ __forceinline__ int chunk_count(const BwdChunkParams& p) { return p.n_chunks; }
+
+// dK/dV of chunk calls: keys of the chunks that every query row from q_row0 on sees in full stand at positions below 0 for
+// the causal mask; the bodies subtract this from their key positions.
+constexpr int kFullyVisible = 1 << 28;
+
+// The dK/dV view of the chunk that block `block` belongs to: `block` becomes the block's number within the chunk.
+template <int DQK, int DV>
+__device__ __forceinline__ BwdParams dkdv_chunk_params(const BwdChunkParams& p, int& block, int& key_shift) {
+  int i = 0;
+  while (i + 1 < p.n_chunks && block >= p.chunk[i + 1].first_block) ++i;
+  const BwdChunk& ch = p.chunk[i];
+  block -= ch.first_block;
+  key_shift = i + 1 < p.n_chunks ? kFullyVisible : 0;
+  BwdParams r = p;
+  r.k = ch.key.k; r.v = ch.key.v; r.k_pe = ch.key.k_pe; r.Skv = ch.key.rows;
+  r.dk = ch.dk; r.dv = ch.dv; r.dk_pe = ch.dk_pe;
+  r.q += (int64_t)ch.key.q_row0 * p.HqT * DQK;
+  r.dout += (int64_t)ch.key.q_row0 * p.HqT * DV;
+  r.lse += ch.key.q_row0;
+  r.delta += ch.key.q_row0;
+  r.Sq -= ch.key.q_row0;
+  r.tiles = ch.tiles; r.zero_tail = ch.zero_tail;
+  r.main_blocks = ch.tiles * p.Hkv * p.B * p.split;
+  const int64_t row_parts = (int64_t)ch.rows_before * p.B * p.Hkv;
+  r.ws_dk += row_parts * p.split * DQK;
+  r.ws_dv += row_parts * p.split * DV;
+  r.ws_dkpe += row_parts * 64;
+  return r;
+}
 
 constexpr int kZeroTailRows = 32;  // rows one such block clears
 
@@ -57,25 +114,26 @@ constexpr int kZeroTailRows = 32;  // rows one such block clears
 // call computes (a ring step that sees only the first rows of a chunk owes the others a zero gradient).
 // dk_feats: features per head of dk (128 when the keys come in two parts).
 template <typename OutT>
+__device__ __forceinline__ void clear_rows(OutT* base, int64_t bs, int64_t row_stride, int row_elems, int B, int r0, int rows, int tid, int threads) {
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  constexpr int kPer16 = 16 / (int)sizeof(OutT);  // elements per 16-byte piece
+  const int pieces = row_elems / kPer16;
+  const int total = B * rows * pieces;
+  for (int i = tid; i < total; i += threads) {
+    const int piece = i % pieces, rb = i / pieces;
+    const int row = r0 + rb % rows, b = rb / rows;
+    *reinterpret_cast<u32x4*>(base + b * bs + row * row_stride + (int64_t)piece * kPer16) = zero;
+  }
+}
+
+template <typename OutT>
 __device__ __forceinline__ void zero_tail_block(const BwdParams& p, int idx, int dk_feats, int dv_feats, int tid, int threads) {
   const int r0 = p.Skv + idx * kZeroTailRows;
   const int rows = min(kZeroTailRows, p.Skv + p.zero_tail - r0);
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  constexpr int kPer16 = 16 / (int)sizeof(OutT);  // elements per 16-byte piece
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    OutT* base = reinterpret_cast<OutT*>(t == 0 ? p.dk : p.dv);
-    const int64_t bs = t == 0 ? p.dk_bs : p.dv_bs;
-    const int feats = t == 0 ? dk_feats : dv_feats;
-    const int64_t row_stride = (int64_t)p.HkvT * feats;  // a row holds HkvT heads, Hkv of them belong to this call
-    const int pieces = p.Hkv * feats / kPer16;
-    const int total = p.B * rows * pieces;
-    for (int i = tid; i < total; i += threads) {
-      const int piece = i % pieces, rb = i / pieces;
-      const int row = r0 + rb % rows, b = rb / rows;
-      *reinterpret_cast<u32x4*>(base + b * bs + row * row_stride + (int64_t)piece * kPer16) = zero;
-    }
-  }
+  // a row holds HkvT heads, Hkv of them belong to this call
+  clear_rows(reinterpret_cast<OutT*>(p.dk), p.dk_bs, (int64_t)p.HkvT * dk_feats, p.Hkv * dk_feats, p.B, r0, rows, tid, threads);
+  clear_rows(reinterpret_cast<OutT*>(p.dv), p.dv_bs, (int64_t)p.HkvT * dv_feats, p.Hkv * dv_feats, p.B, r0, rows, tid, threads);
+  if (p.dk_pe != nullptr) clear_rows(p.dk_pe, p.dk_pe_bs, 64, 64, p.B, r0, rows, tid, threads);
 }
 
 constexpr int kDsBlockBytes = 4 * 4096;  // one (query tile, key block): four wave-pair images
@@ -194,6 +252,10 @@ void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned gr
 // dK/dV kernel's grid; everything else as for the separate launches. Head dims (128, 128) and (192, 128) use the split-key
 // dQ workgroups. False: no such kernel for these output types.
 bool launch_bwd_pair(const BwdParams& p, int dqk, bool causal, bool dkdv_f32, bool dq_f32, unsigned dkdv_blocks, hipStream_t stream);
+
+// The backward of a chunk call: attn_bwd_chunks.hip. dkdv_blocks = the dK/dV grid; p.q_tiles = 128-row query tiles; split_keys
+// as for launch_dq_direct / launch_dq_duo (one_grid implies it at 128 and 192 features).
+void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool split_keys, unsigned dkdv_blocks, hipStream_t stream);
 
 // dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
 // split every tile's keys: attn_bwd_dq_direct.hip.

@@ -15,39 +15,69 @@ namespace {
 
 constexpr int kBN = kDkdvBlockN;  // key rows per workgroup
 
-// out[b, s, h, :] (+)= sum over parts of ws[part][b][s][h][:], parts added in index order; dK
-// (blockIdx.y = 0) and dV (blockIdx.y = 1) in one launch.
-struct ReduceParams {
-  const float* ws[2];
-  void* out[2];
-  int64_t part_stride[2], row_elems[2], out_bs[2], n4[2];
-  int64_t out_row_elems[2];  // elements between consecutive rows of `out` (>= row_elems: a head range of a wider tensor)
+// out[b, s, h, :] (+)= sum over parts of ws[part][b][s][h][:], parts added in index order; blockIdx.y picks the item (dK and
+// dV of a call, or those of all its chunks).
+struct ReduceItem {
+  const float* ws;
+  void* out;
+  int64_t part_stride, row_elems, out_bs, n4;
+  int64_t out_row_elems;  // elements between consecutive rows of `out` (>= row_elems: a head range of a wider tensor)
   int64_t rows_per_batch;
+};
+template <int N>
+struct ReduceParams {
+  ReduceItem item[N];
   int parts, accumulate;
 };
 
-template <typename OutT>
-__global__ __launch_bounds__(256) void reduce_parts_kernel(ReduceParams r) {
-  const int t = blockIdx.y;
-  const float* __restrict__ ws = r.ws[t];
-  OutT* out = reinterpret_cast<OutT*>(r.out[t]);
-  const int64_t part_stride = r.part_stride[t], n4 = r.n4[t];
-  const int64_t per_batch = r.rows_per_batch * r.row_elems[t];
+template <typename OutT, int N>
+__global__ __launch_bounds__(256) void reduce_parts_kernel(ReduceParams<N> p) {
+  const ReduceItem& r = p.item[blockIdx.y];
+  const float* __restrict__ ws = r.ws;
+  OutT* out = reinterpret_cast<OutT*>(r.out);
+  const int64_t part_stride = r.part_stride, n4 = r.n4;
+  const int64_t per_batch = r.rows_per_batch * r.row_elems;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t e = i * 4;
     f32x4 s = *reinterpret_cast<const f32x4*>(ws + e);
-    for (int pidx = 1; pidx < r.parts; ++pidx) s += *reinterpret_cast<const f32x4*>(ws + pidx * part_stride + e);
+    for (int pidx = 1; pidx < p.parts; ++pidx) s += *reinterpret_cast<const f32x4*>(ws + pidx * part_stride + e);
     const int64_t bb = e / per_batch;
     const int64_t in_batch = e - bb * per_batch;
-    const int64_t row = in_batch / r.row_elems[t];
-    OutT* dst = out + bb * r.out_bs[t] + row * r.out_row_elems[t] + (in_batch - row * r.row_elems[t]);
-    store4<OutT>(dst, s[0], s[1], s[2], s[3], r.accumulate != 0);
+    const int64_t row = in_batch / r.row_elems;
+    OutT* dst = out + bb * r.out_bs + row * r.out_row_elems + (in_batch - row * r.row_elems);
+    store4<OutT>(dst, s[0], s[1], s[2], s[3], p.accumulate != 0);
   }
 }
 
-int pick_split(const pith_attn_bwd_args* a) {
+// A launch of the above, item by item.
+template <int N>
+struct Reduction {
+  ReduceParams<N> p;
+  int n = 0;
+  int64_t max_n4 = 0;
+
+  void add(const float* ws, void* out, int64_t out_bs, int64_t batch, int64_t rows, int64_t row_elems, int64_t out_row_elems) {
+    ReduceItem& r = p.item[n++];
+    r.ws = ws; r.out = out; r.out_bs = out_bs;
+    r.row_elems = row_elems; r.out_row_elems = out_row_elems; r.rows_per_batch = rows;
+    r.part_stride = batch * rows * row_elems;
+    r.n4 = r.part_stride / 4;
+    if (r.n4 > max_n4) max_n4 = r.n4;
+  }
+  void launch(int parts, bool accumulate, bool f32, hipStream_t st) {
+    p.parts = parts;
+    p.accumulate = accumulate;
+    const int64_t blocks = (max_n4 + 255) / 256;
+    const dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192), n);
+    if (f32) hipLaunchKernelGGL((reduce_parts_kernel<float, N>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((reduce_parts_kernel<__bf16, N>), grid, dim3(256), 0, st, p);
+  }
+};
+
+// tiles: key tiles of the launch, over all of its chunks
+int pick_split(const pith_attn_bwd_args* a, int64_t tiles) {
   const int64_t group = a->Hq / a->Hkv;
-  const int64_t base = ((a->Skv + kBN - 1) / kBN) * a->Hkv * a->B;
+  const int64_t base = tiles * a->Hkv * a->B;
   int split = 1;
   // Workgroups wanted. Without a causal mask all of them carry the same work, so one full round is ideal; under the mask
   // two rounds (heaviest first) balance better. At 64 features two workgroups share a compute unit and twice as many are
@@ -57,6 +87,7 @@ int pick_split(const pith_attn_bwd_args* a) {
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
   return split;
 }
+int pick_split(const pith_attn_bwd_args* a) { return pick_split(a, (a->Skv + kBN - 1) / kBN); }
 
 // Workspace layout: [head-split partial dK | partial dV] (split > 1), then the per-head gradients of a
 // shared k_pe [Hkv][B][Skv][64] (keys in two parts).
@@ -92,44 +123,15 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, bool with_dq, hipStre
     launch_dkdv_d64(p, a->causal != 0, f32, grid, st);
   }
   if (p.k_pe) {  // dk_pe (+)= sum over heads, in head order
-    ReduceParams r;
-    r.row_elems[0] = r.out_row_elems[0] = 64;
-    r.part_stride[0] = a->B * a->Skv * 64;
-    r.n4[0] = r.part_stride[0] / 4;
-    r.ws[0] = p.ws_dkpe;
-    r.out[0] = a->dk_pe;
-    r.out_bs[0] = a->dk_pe_bs;
-    r.row_elems[1] = r.out_row_elems[1] = r.part_stride[1] = r.n4[1] = r.out_bs[1] = 0;
-    r.ws[1] = nullptr;
-    r.out[1] = nullptr;
-    r.rows_per_batch = a->Skv;
-    r.parts = (int)a->Hkv;
-    r.accumulate = a->accumulate_dkv;
-    const int64_t blocks = (r.n4[0] + 255) / 256;
-    const dim3 rgrid((unsigned)(blocks < 8192 ? blocks : 8192), 1);
-    if (f32) hipLaunchKernelGGL((reduce_parts_kernel<float>), rgrid, dim3(256), 0, st, r);
-    else hipLaunchKernelGGL((reduce_parts_kernel<__bf16>), rgrid, dim3(256), 0, st, r);
+    Reduction<2> r;
+    r.add(p.ws_dkpe, a->dk_pe, a->dk_pe_bs, a->B, a->Skv, 64, 64);
+    r.launch((int)a->Hkv, a->accumulate_dkv, f32, st);
   }
   if (p.split > 1) {
-    ReduceParams r;
-    int64_t max_n4 = 0;
-    for (int which = 0; which < 2; ++which) {
-      const int64_t d = which == 0 ? a->Dqk : a->Dv;
-      r.row_elems[which] = a->Hkv * d;
-      r.out_row_elems[which] = p.HkvT * d;
-      r.part_stride[which] = a->B * a->Skv * r.row_elems[which];
-      r.n4[which] = r.part_stride[which] / 4;
-      r.ws[which] = which == 0 ? p.ws_dk : p.ws_dv;
-      r.out[which] = which == 0 ? a->dk : a->dv;
-      r.out_bs[which] = which == 0 ? a->dk_bs : a->dv_bs;
-      if (r.n4[which] > max_n4) max_n4 = r.n4[which];
-    }
-    r.rows_per_batch = a->Skv;
-    r.parts = p.split;
-    r.accumulate = a->accumulate_dkv;
-    const dim3 rgrid((unsigned)((max_n4 + 255) / 256 < 8192 ? (max_n4 + 255) / 256 : 8192), 2);
-    if (f32) hipLaunchKernelGGL((reduce_parts_kernel<float>), rgrid, dim3(256), 0, st, r);
-    else hipLaunchKernelGGL((reduce_parts_kernel<__bf16>), rgrid, dim3(256), 0, st, r);
+    Reduction<2> r;
+    r.add(p.ws_dk, a->dk, a->dk_bs, a->B, a->Skv, a->Hkv * a->Dqk, p.HkvT * a->Dqk);
+    r.add(p.ws_dv, a->dv, a->dv_bs, a->B, a->Skv, a->Hkv * a->Dv, p.HkvT * a->Dv);
+    r.launch(p.split, a->accumulate_dkv, f32, st);
   }
 }
 
@@ -145,6 +147,16 @@ extern "C" int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* 
 
 namespace {
 
+// Keys in two parts: what the dK/dV side asks of them.
+int validate_dk_pe(const pith_attn_bwd_args* a, const char* who) {
+  if (!a->k_pe) return PITH_OK;
+  if (a->Hq != a->Hkv)
+    return fail(PITH_ERR_UNSUPPORTED, "%s: keys in two parts need Hq == Hkv (got %lld, %lld)", who, (long long)a->Hq, (long long)a->Hkv);
+  if (!a->dk_pe) return fail(PITH_ERR_NULL_POINTER, "%s: dk_pe is NULL", who);
+  if (!aligned16(a->dk_pe) || a->dk_pe_bs % 8) return fail(PITH_ERR_MISALIGNED, "%s: dk_pe pointer / batch stride must keep 16-byte alignment", who);
+  return PITH_OK;
+}
+
 // Runs the kernels with the head-split partials in `workspace` (NULL: no head split).
 int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_t st, const char* who, bool with_dq = false) {
   // the grid of this kernel runs over key tiles (validate_bwd bounded the query-side grid)
@@ -155,10 +167,7 @@ int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_
   if (with_dq)
     if (const int rc = prepare_dq(a, &p, who)) return rc;
   if (a->k_pe) {
-    if (a->Hq != a->Hkv)
-      return fail(PITH_ERR_UNSUPPORTED, "%s: keys in two parts need Hq == Hkv (got %lld, %lld)", who, (long long)a->Hq, (long long)a->Hkv);
-    if (!a->dk_pe) return fail(PITH_ERR_NULL_POINTER, "%s: dk_pe is NULL", who);
-    if (!aligned16(a->dk_pe) || a->dk_pe_bs % 8) return fail(PITH_ERR_MISALIGNED, "%s: dk_pe pointer / batch stride must keep 16-byte alignment", who);
+    if (const int rc = validate_dk_pe(a, who)) return rc;
     if (!workspace) return fail(PITH_ERR_BAD_SHAPE, "%s: keys in two parts need a workspace of %lld bytes", who, (long long)dkpe_bytes_for(a));
     p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + split_bytes_for(a, split));
   }
@@ -266,4 +275,117 @@ extern "C" int pith_attn_bwd_dkdv_static(const pith_attn_bwd_args* a, pith_strea
     if (src != PITH_OK) return src;
   }
   return run_dkdv(a, split, ws, (hipStream_t)stream, who);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Several chunks of keys in one call
+
+namespace {
+
+// The call as one against all keys of its chunks together: what the rules for launches look at. False: malformed.
+bool merged_call(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_attn_bwd_args* a, int64_t* tiles) {
+  if (!args || !chunks || n < 1 || n > kMaxChunks) return false;
+  *a = *args;
+  a->Skv = 0;
+  *tiles = 0;
+  int64_t seen = 0;  // (query row, key) pairs
+  for (int64_t i = 0; i < n; ++i) {
+    const pith_key_chunk& c = chunks[i];
+    if (c.rows <= 0 || c.rows > (1 << 24) || c.q_row0 < 0 || c.q_row0 >= args->Sq) return false;
+    a->Skv += c.rows;
+    *tiles += (c.rows + kBN - 1) / kBN;
+    seen += i == n - 1 ? c.rows * args->Sq / 2 : c.rows * (args->Sq - c.q_row0);
+  }
+  a->k_pe = chunks[0].k_pe;
+  a->ds = nullptr;
+  a->causal = 10 * seen <= 7 * a->Skv * args->Sq;  // rows as unequal as under a mask (see pith_attn_fwd_chunks)
+  return a->B > 0 && a->Hkv > 0 && a->Hq > 0 && a->Hq % a->Hkv == 0;
+}
+
+int pick_chunks_split(pith_attn_bwd_args a, int64_t tiles) {
+  a.causal = 1;  // the chunks' workgroups are unequal in any case
+  return pick_split(&a, tiles);
+}
+
+}  // namespace
+
+extern "C" int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n) {
+  pith_attn_bwd_args a;
+  int64_t tiles;
+  if (!merged_call(args, chunks, n, &a, &tiles)) return 0;
+  return workspace_bytes_for(&a, pick_chunks_split(a, tiles));
+}
+
+extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
+  const char* who = "pith_attn_bwd_chunks";
+  if (!args || !chunks) return fail(PITH_ERR_NULL_POINTER, "%s: args or chunks is NULL", who);
+  pith_attn_bwd_args all;
+  int64_t tiles;
+  if (!merged_call(args, chunks, n, &all, &tiles))
+    return fail(PITH_ERR_BAD_SHAPE, "%s: 1..%d chunks, each of 1..2^24 rows and seen from a query row on, and Hq a multiple of Hkv", who, kMaxChunks);
+  if (args->dq_dtype != PITH_BF16 || args->dkv_dtype != PITH_BF16 || args->accumulate_dq || args->accumulate_dkv || args->dq_final)
+    return fail(PITH_ERR_UNSUPPORTED, "%s: gradients are written, once, in bf16", who);
+  if (n == 1) {
+    pith_attn_bwd_args a = *args;
+    const pith_key_chunk& c = chunks[0];
+    a.k = c.k; a.v = c.v; a.k_pe = c.k_pe; a.dk = c.dk; a.dv = c.dv; a.dk_pe = c.dk_pe;
+    a.Skv = c.rows; a.causal = 1; a.dkv_zero_tail = c.zero_tail; a.ds = nullptr;
+    return pith_attn_bwd(&a, stream);
+  }
+  const int split = pick_chunks_split(all, tiles);
+  const int64_t need = workspace_bytes_for(&all, split);
+  if (need > 0 && (!args->workspace || args->workspace_bytes < need || !aligned16(args->workspace)))
+    return fail(PITH_ERR_BAD_SHAPE, "%s: a 16-byte aligned workspace of %lld bytes is needed", who, (long long)need);
+  BwdChunkParams p;
+  unsigned blocks = 0;
+  int64_t rows_before = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const pith_key_chunk& c = chunks[i];
+    const bool diagonal = i == n - 1;
+    if ((diagonal && c.q_row0) || (i > 0 && !diagonal && c.q_row0 < chunks[i - 1].q_row0))
+      return fail(PITH_ERR_BAD_SHAPE, "%s: chunk %lld: q_row0=%lld (chunks sorted by it, the queries' own, 0, last)", who, (long long)i, (long long)c.q_row0);
+    pith_attn_bwd_args a = *args;
+    a.k = c.k; a.v = c.v; a.k_pe = c.k_pe; a.dk = c.dk; a.dv = c.dv; a.dk_pe = c.dk_pe;
+    a.Skv = c.rows; a.causal = diagonal; a.dkv_zero_tail = c.zero_tail; a.ds = nullptr;
+    if (!c.k_pe != !chunks[0].k_pe) return fail(PITH_ERR_UNSUPPORTED, "%s: keys in two parts in some chunks only", who);
+    if (const int rc = validate_bwd(&a, who, true, true)) return rc;
+    if (const int rc = validate_dk_pe(&a, who)) return rc;
+    if (i == 0) static_cast<BwdParams&>(p) = make_bwd_params(&a);
+    BwdChunk& ch = p.chunk[i];
+    ch.key = KeyChunk{(const __bf16*)c.k, (const __bf16*)c.v, (const __bf16*)c.k_pe, (int)c.rows, (int)c.q_row0};
+    ch.dk = (__bf16*)c.dk; ch.dv = (__bf16*)c.dv; ch.dk_pe = (__bf16*)c.dk_pe;
+    ch.tiles = (int)((c.rows + kBN - 1) / kBN);
+    ch.zero_tail = (int)c.zero_tail;
+    ch.first_block = (int)blocks;
+    ch.rows_before = (int)rows_before;
+    const int64_t next = blocks + (int64_t)ch.tiles * a.Hkv * a.B * split + (c.zero_tail + kZeroTailRows - 1) / kZeroTailRows;
+    rows_before += c.rows;
+    if (next > 0x3fffffff || rows_before > 0x3fffffff) return fail(PITH_ERR_UNSUPPORTED, "%s: the chunks exceed the launch grid limit", who);
+    blocks = (unsigned)next;
+  }
+  p.n_chunks = (int)n;
+  p.dk_pe_bs = args->dk_pe_bs;
+  p.split = split;
+  p.q_tiles = (p.Sq + 127) / 128;
+  p.ws_dk = reinterpret_cast<float*>(need > 0 ? args->workspace : nullptr);
+  p.ws_dv = p.ws_dk + (split > 1 ? (int64_t)split * all.B * all.Skv * all.Hkv * all.Dqk : 0);
+  p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));
+  hipStream_t st = (hipStream_t)stream;
+  begin_launch();
+  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all), dq_split_keys(&all), blocks, st);
+  if (all.k_pe || split > 1) {  // (never both: keys in two parts have no head groups to split)
+    Reduction<2 * kMaxChunks> r;
+    for (int64_t i = 0; i < n; ++i) {
+      const pith_key_chunk& c = chunks[i];
+      const int64_t at = p.chunk[i].rows_before * all.B * all.Hkv;
+      if (all.k_pe) {
+        r.add(p.ws_dkpe + at * 64, c.dk_pe, args->dk_pe_bs, all.B, c.rows, 64, 64);
+      } else {
+        r.add(p.ws_dk + at * split * all.Dqk, c.dk, args->dk_bs, all.B, c.rows, all.Hkv * all.Dqk, p.HkvT * all.Dqk);
+        r.add(p.ws_dv + at * split * all.Dv, c.dv, args->dv_bs, all.B, c.rows, all.Hkv * all.Dv, p.HkvT * all.Dv);
+      }
+    }
+    r.launch(all.k_pe ? (int)all.Hkv : split, false, false, st);
+  }
+  return check_launch(who);
 }

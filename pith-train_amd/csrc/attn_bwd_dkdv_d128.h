@@ -80,7 +80,7 @@ struct TileCursor {
 // XOR terms make the reader's transposing LDS reads conflict-free). Keys at or beyond Skv hold 0
 // (their P is masked to 0).
 template <bool CAUSAL, typename OutT, bool EMIT_DS, bool DESC = false>
-__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) {
+__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, int key_shift = 0) {
   constexpr int KS = kD / 16, DB = kD / 32;
 
   const int tid = threadIdx.x;
@@ -112,7 +112,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
 
   // Query tiles to visit: all of them, or from the diagonal down under the causal mask.
   const int m_end = (p.Sq + kBM - 1) / kBM;
-  const int m_first = CAUSAL ? min(kv_wg0 / kBM, m_end) : 0;
+  const int m_first = CAUSAL ? min(max(kv_wg0 - key_shift, 0) / kBM, m_end) : 0;
   const int n_iter = (m_end - m_first) * heads_per_part;
 
   // ---- requests: issued by the four B waves only (their vector block, dS, is the shorter one: measured
@@ -280,7 +280,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) x[rb][v] = __builtin_amdgcn_exp2f(x[rb][v] * p.kappa - l4[rb][v >> 2][v & 3]);
-    if ((CAUSAL && q0 < kv_pair0 + 31) || (q0 + kBM > p.Sq) || (EMIT_DS && kv_pair0 + 32 > p.Skv)) {
+    if ((CAUSAL && q0 < kv_pair0 - key_shift + 31) || (q0 + kBM > p.Sq) || (EMIT_DS && kv_pair0 + 32 > p.Skv)) {
       // tile on the diagonal of a causal chunk, a ragged last tile, or (when dS is handed on, where
       // nonexistent keys must read 0) the ragged last key block (wave-uniform branch)
 #pragma unroll
@@ -288,7 +288,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int qrow = q0 + 32 * rb + acc_row(v, g);
-          if ((CAUSAL && key > qrow) || qrow >= p.Sq || (EMIT_DS && key >= p.Skv)) x[rb][v] = 0.f;
+          if ((CAUSAL && key - key_shift > qrow) || qrow >= p.Sq || (EMIT_DS && key >= p.Skv)) x[rb][v] = 0.f;
         }
     }
 #pragma unroll

@@ -89,7 +89,7 @@ constexpr int kTB = 2;  // 64-row query tiles (32-row tiles, 1, measured 3 % slo
 constexpr int kSmem = Layout<kTB>::kSmem;
 
 template <bool CAUSAL, typename OutT, int TB = kTB>
-__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) {
+__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, int key_shift = 0) {
   using L = Layout<TB>;
   constexpr int kBM = L::kBM, kStage = L::kStage, kOffExtra = L::kOffExtra, kOffO = L::kOffO, kOffStat = L::kOffStat;
   constexpr int kExchPair = L::kExchPair;
@@ -127,7 +127,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
 
   // Query tiles to visit: all of them, or from the diagonal down under the causal mask.
   const int m_end = (p.Sq + kBM - 1) / kBM;
-  const int m_first = CAUSAL ? min(kv_wg0 / kBM, m_end) : 0;
+  const int m_first = CAUSAL ? min(max(kv_wg0 - key_shift, 0) / kBM, m_end) : 0;
   const int n_iter = (m_end - m_first) * heads_per_part;
 
   // ---- requests: issued by the four B waves only (their vector block, dS, is the shorter one)
@@ -309,7 +309,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   auto make_p = [&](const char* stage, int mt) __attribute__((always_inline)) {
     const float* lse_s = reinterpret_cast<const float*>(stage + kOffStat);
     const int q0 = mt * kBM;
-    const bool masked = (CAUSAL && q0 < kv_pair0 + 31) || (q0 + kBM > p.Sq);  // wave-uniform: diagonal or ragged tile
+    const bool masked = (CAUSAL && q0 < kv_pair0 - key_shift + 31) || (q0 + kBM > p.Sq);  // wave-uniform: diagonal or ragged tile
 #pragma unroll
     for (int rb = 0; rb < TB; ++rb) {
       f32x4 l4[4];
@@ -321,7 +321,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int qrow = q0 + 32 * rb + acc_row(v, g);
-          if ((CAUSAL && key > qrow) || qrow >= p.Sq) x[rb][v] = 0.f;
+          if ((CAUSAL && key - key_shift > qrow) || qrow >= p.Sq) x[rb][v] = 0.f;
         }
       }
 #pragma unroll

@@ -35,7 +35,7 @@ constexpr int kSmem = kSlots * kSlot > kTurn ? kSlots * kSlot : kTurn;
 constexpr int kLoads = 3;                       // load instructions per wave and tile
 
 template <bool CAUSAL, typename OutT>
-__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) {
+__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, int key_shift = 0) {
   constexpr int KS = kD / 16, DB = kD / 32;
 
   const int tid = threadIdx.x;
@@ -64,7 +64,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
 
   // Query tiles to visit: all of them, or from the workgroup's diagonal down under the causal mask, head by head.
   const int m_end = (p.Sq + kBM - 1) / kBM;
-  const int m_first = CAUSAL ? min(kv_wg0 / kBM, m_end) : 0;
+  const int m_first = CAUSAL ? min(max(kv_wg0 - key_shift, 0) / kBM, m_end) : 0;
   const int n_iter = (m_end - m_first) * heads_per_part;
 
   DirectPaired64<kBM, kThreads> mover;
@@ -207,11 +207,11 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
     const int q0 = m_tile * kBM;
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] = __builtin_amdgcn_exp2f(s[v] * p.kappa - lse4[v >> 2][v & 3]);
-    if ((CAUSAL && q0 < kv_wave0 + 31) || q0 + kBM > p.Sq) {  // wave-uniform: diagonal or ragged tile
+    if ((CAUSAL && q0 < kv_wave0 - key_shift + 31) || q0 + kBM > p.Sq) {  // wave-uniform: diagonal or ragged tile
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int qrow = q0 + acc_row(v, g);
-        if ((CAUSAL && key > qrow) || qrow >= p.Sq) s[v] = 0.f;
+        if ((CAUSAL && key - key_shift > qrow) || qrow >= p.Sq) s[v] = 0.f;
       }
     }
 #pragma unroll

@@ -96,7 +96,7 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
   p.ds_kb = (int)((a->Skv + kDkdvBlockN - 1) / kDkdvBlockN);
   p.ds_hs = (a->causal ? ds_tile_start<true>(p.ds_qt, p.ds_kb) : ds_tile_start<false>(p.ds_qt, p.ds_kb)) * kDsBlockBytes;
   p.dq_final = nullptr; p.dq_final_bs = 0; p.final_r0 = p.final_r1 = 0;
-  p.zero_tail = 0; p.main_blocks = 0x7fffffff; p.walk_desc = 0;
+  p.zero_tail = 0; p.main_blocks = 0x7fffffff; p.dk_pe = nullptr; p.dk_pe_bs = 0; p.walk_desc = 0;
   return p;
 }
 

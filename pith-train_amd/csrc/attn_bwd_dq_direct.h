@@ -46,8 +46,8 @@ constexpr int kTile = kBN * kRowBytes128;
 template <int DQK>
 constexpr int kSmem = DQK == 192 ? kSlots * (kTile + kExtraTileBytes) + 2 * kTile + 4 * 8192 : 2 * kSlots * kTile;
 
-template <int DQK, bool CAUSAL, typename OutT>
-__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) {
+template <int DQK, bool CAUSAL, typename OutT, bool MULTI = false>
+__device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int block) {
   static_assert(DQK == 128 || DQK == 192, "head dims");
   constexpr int KVB = 1;    // 32-key blocks of a tile this wave owns
   constexpr int kBM = 128;  // query rows per workgroup
@@ -82,20 +82,30 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   const int64_t q_row_stride = (int64_t)p.HqT * DQK;
   const int64_t do_row_stride = (int64_t)p.HqT * kDv;
   // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
-  const bool two_part = DQK == 192 && p.k_pe != nullptr;
+  const bool two_part = DQK == 192 && chunk_of(p, 0).k_pe != nullptr;
   const int k_head_elems = two_part ? 128 : DQK;
   const int k_row_bytes = p.HkvT * k_head_elems * 2, v_row_bytes = p.HkvT * kDv * 2;
-  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
-  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;  // source of features 128..
   const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
-  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
+  // a chunk's first row in K, in the source of features 128.. and in V
+  auto k_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).k + b * p.k_bs + (int64_t)hk * k_head_elems);
+  };
+  auto kx_rows = [&](int id) __attribute__((always_inline)) {
+    return two_part ? reinterpret_cast<const char*>(chunk_of(p, id).k_pe + b * p.k_pe_bs) : k_rows(id);
+  };
+  auto v_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).v + b * p.v_bs + (int64_t)hk * kDv);
+  };
 
-  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
-  int n_tiles_wg = n_tiles_all, n_tiles_wave = n_tiles_all;
+  const ChunkRange<MULTI, CAUSAL, kBN> range(p, m0 + kBM);
+  int n_tiles_wg = range.tiles_full, n_tiles_wave = range.tiles_full;
   if (CAUSAL) {
-    n_tiles_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
-    n_tiles_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
+    const int tiles = (chunk_of(p, range.last).rows + kBN - 1) / kBN;
+    n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
+    n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
+  TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows), v_src(p, range, v_row_bytes, v_rows);
+  TileMask<MULTI, CAUSAL, kBN> mask(p, range);
 
   DirectTile128<kBN, kThreads> mover, kmover;  // V tiles (and K tiles when the row pitches agree); K tiles otherwise
   DirectExtra64 xmover;
@@ -106,14 +116,16 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   }
   auto request = [&](int t) __attribute__((always_inline)) {
     char* kslot = kbuf + (t & (kSlots - 1)) * kKTile;
-    const char* ksrc = kh + (int64_t)t * kBN * k_row_bytes;
     if constexpr (DQK != kDv) {
-      kmover.issue(ksrc, p.Skv - t * kBN, kslot, wave, lane);
-      xmover.issue(kx + (int64_t)t * kBN * kx_row_bytes, p.Skv - t * kBN, kslot + kTile, wave, lane);
+      kmover.issue(k_src.src(t), k_src.left(t), kslot, wave, lane);
+      xmover.issue(kx_src.src(t), k_src.left(t), kslot + kTile, wave, lane);
+      kx_src.advance(p, range, kx_rows);
     } else {
-      mover.issue(ksrc, p.Skv - t * kBN, kslot, wave, lane);
+      mover.issue(k_src.src(t), k_src.left(t), kslot, wave, lane);
     }
-    mover.issue(vh + (int64_t)t * kBN * v_row_bytes, p.Skv - t * kBN, vbuf + (t & (kVSlots - 1)) * kTile, wave, lane);
+    mover.issue(v_src.src(t), k_src.left(t), vbuf + (t & (kVSlots - 1)) * kTile, wave, lane);
+    k_src.advance(p, range, k_rows);
+    v_src.advance(p, range, v_rows);
   };
   // tiles of the prologue (0) and of the first kDist intervals
 #pragma unroll
@@ -299,20 +311,19 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   // the key range (no mask code, and nothing it needs stays live in the loop that uses it)
   auto make_ds = [&](int t, auto masked_tag) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
-    const int n0 = t * kBN;
 #pragma unroll
     for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) s[kvb][v] = __builtin_amdgcn_exp2f(s[kvb][v] * p.kappa - lse_q);
-    if (MASKED && ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv))) {
-      // tile crossing the diagonal of a causal chunk, or a ragged last tile (wave-uniform branch)
-      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;  // last visible key
+    if (MASKED && mask.partial(range, t, q_wave0)) {  // wave-uniform branch
+      const int limit = mask.limit(range, qrow), n0 = mask.key0(t);
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
           if (n0 + (kvb0 + kvb) * 32 + acc_row(v, g) > limit) s[kvb][v] = 0.f;
     }
+    mask.advance(p, range);
 #pragma unroll
     for (int kvb = 0; kvb < KVB; ++kvb) {
 #pragma unroll
@@ -372,9 +383,10 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
     }
     land_and_sync(will_request);
   };
-  // tiles [0, first_masked) need no mask for this wave: they lie below its diagonal and inside Skv
-  int first_masked = p.Skv / kBN;
-  if (CAUSAL) first_masked = min(first_masked, q_wave0 >= kBN - 1 ? (q_wave0 - (kBN - 1)) / kBN + 1 : 0);
+  // tiles [0, first_masked) need no mask for this wave: they lie below its diagonal and inside Skv (several chunks: any of
+  // their last tiles may be ragged, and the mask is always there)
+  int first_masked = MULTI ? 0 : p.Skv / kBN;
+  if (CAUSAL && !MULTI) first_masked = min(first_masked, q_wave0 >= kBN - 1 ? (q_wave0 - (kBN - 1)) / kBN + 1 : 0);
   constexpr std::false_type no;
   constexpr std::true_type yes;
   if (!late) {

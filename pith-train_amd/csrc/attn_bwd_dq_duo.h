@@ -41,8 +41,8 @@ struct DqDuoLayout {
 template <int DQK>
 constexpr int kSmem = DqDuoLayout<DQK>::kSmem;
 
-template <int DQK, bool CAUSAL, typename OutT>
-__device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) {
+template <int DQK, bool CAUSAL, typename OutT, bool MULTI = false>
+__device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int block) {
   using L = DqDuoLayout<DQK>;
   constexpr int kDv = L::kDv, KS = DQK / 16, VS = kDv / 16, DB = DQK / 32;
   constexpr bool kPaired = DQK == 64;
@@ -64,20 +64,30 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   const int64_t q_row_stride = (int64_t)p.HqT * DQK;
   const int64_t do_row_stride = (int64_t)p.HqT * kDv;
   // keys in two parts: K rows hold 128 features per head, the last 64 come from k_pe (no head offset)
-  const bool two_part = DQK == 192 && p.k_pe != nullptr;
+  const bool two_part = DQK == 192 && chunk_of(p, 0).k_pe != nullptr;
   const int k_head_elems = two_part ? 128 : DQK;
   const int k_row_bytes = p.HkvT * k_head_elems * 2, v_row_bytes = p.HkvT * kDv * 2;
-  const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head_elems);
-  const char* kx = two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : kh;
   const int kx_row_bytes = two_part ? (int)p.k_pe_rs * 2 : k_row_bytes;
-  const char* vh = reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDv);
+  // a chunk's first row in K, in the source of features 128.. and in V
+  auto k_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).k + b * p.k_bs + (int64_t)hk * k_head_elems);
+  };
+  auto kx_rows = [&](int id) __attribute__((always_inline)) {
+    return two_part ? reinterpret_cast<const char*>(chunk_of(p, id).k_pe + b * p.k_pe_bs) : k_rows(id);
+  };
+  auto v_rows = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(chunk_of(p, id).v + b * p.v_bs + (int64_t)hk * kDv);
+  };
 
-  const int n_tiles_all = (p.Skv + kBN - 1) / kBN;
-  int n_wg = n_tiles_all, n_wave = n_tiles_all;  // key tiles this workgroup / this wave visits
+  const ChunkRange<MULTI, CAUSAL, kBN> range(p, m0 + kBM);
+  int n_wg = range.tiles_full, n_wave = range.tiles_full;  // key tiles this workgroup / this wave visits
   if (CAUSAL) {
-    n_wg = min(n_tiles_all, (m0 + kBM - 1) / kBN + 1);
-    n_wave = min(n_tiles_all, (q_wave0 + 31) / kBN + 1);
+    const int tiles = (chunk_of(p, range.last).rows + kBN - 1) / kBN;
+    n_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
+    n_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
+  TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows), v_src(p, range, v_row_bytes, v_rows);
+  TileMask<MULTI, CAUSAL, kBN> mask(p, range);
 
   DirectTile128<kBN, kThreads> vmover, kmover;
   DirectPaired64<kBN, kThreads> vpmover, kpmover;
@@ -92,9 +102,9 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   auto request = [&](int t) __attribute__((always_inline)) {
     char* const ks = kbuf + (t & (kSlots - 1)) * L::kKTile;
     char* const vs = vbuf + (t & (kSlots - 1)) * L::kVTile;
-    const char* ksrc = kh + (int64_t)t * kBN * k_row_bytes;
-    const char* vsrc = vh + (int64_t)t * kBN * v_row_bytes;
-    const int left = p.Skv - t * kBN;
+    const char* const ksrc = k_src.src(t);
+    const char* const vsrc = v_src.src(t);
+    const int left = k_src.left(t);
     if constexpr (kPaired) {
       kpmover.issue(ksrc, left, ks, wave, lane);
       vpmover.issue(vsrc, left, vs, wave, lane);
@@ -103,9 +113,12 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
       vmover.issue(vsrc, left, vs, wave, lane);
     } else {  // no register to spare for source offsets: reloading a spilled one would wait for the tiles in flight
       kmover.issue_clamped(ksrc, left, ks, wave, lane);
-      kpmover.issue_clamped(kx + (int64_t)t * kBN * kx_row_bytes, left, ks + L::kFull, wave, lane);
+      kpmover.issue_clamped(kx_src.src(t), left, ks + L::kFull, wave, lane);
       vmover.issue_clamped(vsrc, left, vs, wave, lane);
+      kx_src.advance(p, range, kx_rows);
     }
+    k_src.advance(p, range, k_rows);
+    v_src.advance(p, range, v_rows);
   };
   request(0);
   if (n_wg > 1) request(1);
@@ -221,15 +234,15 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
   };
   // P = exp2(kappa s - lse), masked entries 0, dS = P * (dP - delta) -> bf16
   auto make_ds = [&](int t) __attribute__((always_inline)) {
-    const int n0 = t * kBN;
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] = __builtin_amdgcn_exp2f(s[v] * p.kappa - lse_q);
-    if ((CAUSAL && (n0 + kBN - 1 > q_wave0)) || (n0 + kBN > p.Skv)) {  // wave-uniform
-      const int limit = CAUSAL ? min(qrow, p.Skv - 1) : p.Skv - 1;
+    if (mask.partial(range, t, q_wave0)) {  // wave-uniform
+      const int limit = mask.limit(range, qrow), n0 = mask.key0(t);
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         if (n0 + acc_row(v, g) > limit) s[v] = 0.f;
     }
+    mask.advance(p, range);
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] *= dp[v];
 #pragma unroll

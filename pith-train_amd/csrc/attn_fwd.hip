@@ -142,10 +142,9 @@ extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_k
   int64_t keys = 0, seen = 0;  // in the chunks; (query row, key) pairs
   for (int64_t i = 0; i < n; ++i) {
     const pith_key_chunk& c = chunks[i];
-    const bool diagonal = args->causal && i == n - 1;
-    if (c.q_row0 < 0 || c.q_row0 >= args->Sq || (i > 0 && !diagonal && c.q_row0 < chunks[i - 1].q_row0) || ((diagonal || n == 1) && c.q_row0) ||
-        (i == 0 && c.q_row0 && !args->causal))
-      return fail(PITH_ERR_BAD_SHAPE, "%s: chunk %lld: q_row0=%lld (chunks sorted by it; every query row sees one)", who, (long long)i, (long long)c.q_row0);
+    const bool diagonal = i == n - 1;
+    if (c.q_row0 < 0 || c.q_row0 >= args->Sq || (diagonal && c.q_row0) || (i > 0 && !diagonal && c.q_row0 < chunks[i - 1].q_row0))
+      return fail(PITH_ERR_BAD_SHAPE, "%s: chunk %lld: q_row0=%lld (chunks sorted by it, the queries' own, 0, last)", who, (long long)i, (long long)c.q_row0);
     a.k = c.k; a.v = c.v; a.k_pe = c.k_pe; a.Skv = c.rows; a.causal = diagonal;
     if (!c.k_pe != !chunks[0].k_pe) return fail(PITH_ERR_UNSUPPORTED, "%s: keys in two parts in some chunks only", who);
     if (const int rc = prepare(&a, p)) return rc;
@@ -160,7 +159,7 @@ extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_k
   a.Skv = keys;
   a.causal = 10 * seen <= 7 * keys * args->Sq;
   const Split split = pick_split(&a);
-  a.causal = args->causal;
+  a.causal = 1;
   if (n == 1) return launch<FwdParams>(p, &a, split, stream, who);
   return launch(p, &a, split, stream, who);
 }

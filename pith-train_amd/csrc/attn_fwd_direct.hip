@@ -509,8 +509,12 @@ void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   constexpr int kBM = HALF ? 128 : 256;
   p.m_tiles = (p.Sq + kBM - 1) / kBM;
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
-  if (causal) hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, MULTI>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false, MULTI>), grid, block, 0, st, p);
+  if constexpr (MULTI) {  // the last chunk is seen under the mask
+    hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, true>), grid, block, 0, st, p);
+  } else {
+    if (causal) hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false, false>), grid, block, 0, st, p);
+  }
 }
 
 template <bool MULTI>

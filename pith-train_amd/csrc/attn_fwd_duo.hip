@@ -338,8 +338,12 @@ template <int DQK, bool MULTI>
 void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   p.m_tiles = (p.Sq + kBM - 1) / kBM;
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
-  if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, MULTI>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false, MULTI>), grid, block, 0, st, p);
+  if constexpr (MULTI) {  // the last chunk is seen under the mask
+    hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, true>), grid, block, 0, st, p);
+  } else {
+    if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false, false>), grid, block, 0, st, p);
+  }
 }
 
 template <bool MULTI>

@@ -325,6 +325,51 @@ std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const st
   return std::make_tuple(o, lse);
 }
 
+// (dq, dk list, dv list, dk_pe list or empty); the lists hold a tensor per visited chunk. None as above. The policy for the
+// dS hand-over is the caller's: this call recomputes.
+using RingGrads = std::tuple<Tensor, std::vector<OptTensor>, std::vector<OptTensor>, std::vector<OptTensor>>;
+std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, const Tensor& out, const Tensor& lse, const std::vector<OptTensor>& ks,
+                                       const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes, double scale, int64_t rank,
+                                       int64_t cp, bool zigzag) {
+  pith_attn_bwd_args a = {};
+  RingChunks r;
+  if (!ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r)) return std::nullopt;
+  if (!is_gpu_bf16(dout_in, 4) || !is_gpu_bf16(out, 4) || !out.is_contiguous() || !is_gpu_f32(lse, 3) || !lse.is_contiguous() ||
+      dout_in.device() != q.device() || out.device() != q.device() || lse.device() != q.device() || !has_shape(dout_in, {a.B, a.Sq, a.Hq, a.Dv}) ||
+      !has_shape(out, {a.B, a.Sq, a.Hq, a.Dv}) || !has_shape(lse, {a.B, a.Hq, a.Sq}))
+    return std::nullopt;
+  const Tensor dout = dout_in.contiguous();
+  Tensor delta = empty_like_shape(q, {a.B, a.Hq, a.Sq}, at::kFloat), dq = at::empty_like(q), workspace;
+  if (!attn_bwd_delta_into(out, dout, delta)) return std::nullopt;
+  a.dout = dout.data_ptr(); a.lse = lse.data_ptr<float>(); a.delta = delta.data_ptr<float>(); a.dq = dq.data_ptr();
+  a.dout_bs = a.Sq * a.Hq * a.Dv;
+  a.dq_bs = a.q_bs; a.dk_bs = a.k_bs; a.dv_bs = a.v_bs;
+  a.dk_pe_bs = a.Sq * 64;
+  a.dq_dtype = a.dkv_dtype = PITH_BF16;
+  a.scale = (float)scale;
+  RingGrads g = {dq, std::vector<OptTensor>(cp), std::vector<OptTensor>(cp), std::vector<OptTensor>(pes ? cp : 0)};
+  for (size_t i = 0; i < r.chunk.size(); ++i) {
+    const int64_t j = r.rank[i];
+    Tensor dk = at::empty_like(*ks[j]), dv = at::empty_like(*vs[j]);
+    r.chunk[i].dk = dk.data_ptr(); r.chunk[i].dv = dv.data_ptr();
+    std::get<1>(g)[j] = dk;
+    std::get<2>(g)[j] = dv;
+    if (pes) {
+      Tensor dk_pe = at::empty({a.B, a.Sq, 64}, q.options());
+      r.chunk[i].dk_pe = dk_pe.data_ptr();
+      std::get<3>(g)[j] = dk_pe;
+    }
+  }
+  const int64_t n = (int64_t)r.chunk.size(), need = pith_attn_bwd_chunks_workspace_bytes(&a, r.chunk.data(), n);
+  if (need > 0) {
+    workspace = empty_like_shape(q, {need}, at::kByte);
+    a.workspace = workspace.data_ptr();
+    a.workspace_bytes = need;
+  }
+  if (pith_attn_bwd_chunks(&a, r.chunk.data(), n, stream_of(q)) != PITH_OK) return std::nullopt;
+  return g;
+}
+
 using Two = std::tuple<Tensor, Tensor>;
 using Three = std::tuple<Tensor, Tensor, Tensor>;
 using Four = std::tuple<Tensor, Tensor, Tensor, Tensor>;
@@ -744,6 +789,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_bwd_dq_into", &attn_bwd_dq_into);
   m.def("attn_bwd_pair_into", &attn_bwd_pair_into);
   m.def("ring_forward", &ring_forward);
+  m.def("ring_backward", &ring_backward);
   m.def("combine_into", &combine_into);
   m.def("combine_new", &combine_new);
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into);

@@ -138,6 +138,8 @@ SYMBOLS = {
     "pith_attn_bwd_dkdv": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dq": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
+    "pith_attn_bwd_chunks": (c_int, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64, c_void_p]),
+    "pith_attn_bwd_chunks_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64]),
     "pith_attn_bwd_dkdv_static": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dkdv_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
     "pith_attn_bwd_ds_bytes": (c_int64, [POINTER(AttnBwdArgs)]),

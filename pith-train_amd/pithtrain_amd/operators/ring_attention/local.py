@@ -42,6 +42,7 @@ import torch
 
 from pithtrain_amd import _C
 from pithtrain_amd._ext import native
+from pithtrain_amd.operators.mla import hip
 from pithtrain_amd.operators.mla.hip import (
     FINAL_DQ_HEAD_DIMS,
     MERGING_HEAD_DIMS,
@@ -353,6 +354,18 @@ class RingBackward:
         return self.dq
 
 
+def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunks) -> bool:
+    """Whether some step of the share would hand dS from its dK/dV to its dQ kernel: 5 matrix products instead of 7, which is
+    worth more than one launch over all chunks saves (8192 rows x 32 heads, four ranks: 6.1 ms in steps, 6.6 ms in one launch;
+    4096 rows: 1645 and 1705 us)."""
+    if q.shape[-1] != 128:
+        return False
+    return any(
+        hip.ds_plan(_rows(q, st.q_rows), _rows(k_chunks[st.kv_rank], st.kv_rows), _rows(v_chunks[st.kv_rank], st.kv_rows), st.causal) is not None
+        for st in steps
+    )
+
+
 def ring_forward_local(
     q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
     softmax_scale: float, cp_rank: int, cp_size: int, layout: str = "contiguous",
@@ -384,6 +397,10 @@ def ring_backward_local(
     dv_list[j] are this rank's contribution to the gradients of chunk j (None if never visited).
     With k_pe_chunks (keys in two parts) a fourth list holds the contributions to every k_pe chunk."""
     steps = ring_schedule(cp_rank, cp_size, q.shape[1], layout)
+    if FUSE_CHUNKS and not _handover_pays(steps, q, k_chunks, v_chunks):
+        done = native.ring_backward(dout, q, out, lse, k_chunks, v_chunks, k_pe_chunks, softmax_scale, cp_rank, cp_size, layout == "zigzag")
+        if done is not None:
+            return done if k_pe_chunks is not None else done[:3]
     bwd = RingBackward(dout, q, out, lse, softmax_scale, steps)
     dk_list: List[torch.Tensor] = [None] * cp_size
     dv_list: List[torch.Tensor] = [None] * cp_size

@@ -11,14 +11,6 @@ from pithtrain_amd.operators.ring_attention import local as L
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True)
-def no_stepwise_path(monkeypatch):
-    def used(*args, **kwargs):
-        raise AssertionError("the share was not taken by the chunk calls")
-
-    monkeypatch.setattr(L, "RingForward", used)
-
-
 CASES = [  # B, S_l, Hq, Hkv, D, C, rank, layout, keys in two parts
     (2, 2, 2, 1, 64, 2, 0, "zigzag", False), (1, 66, 4, 2, 64, 3, 1, "zigzag", False), (1, 257, 4, 4, 64, 2, 1, "contiguous", False),
     (1, 1, 2, 1, 128, 2, 1, "contiguous", False), (2, 130, 4, 2, 128, 3, 0, "zigzag", False), (1, 258, 4, 2, 128, 3, 2, "zigzag", False),
@@ -28,8 +20,16 @@ CASES = [  # B, S_l, Hq, Hkv, D, C, rank, layout, keys in two parts
 ]  # fmt: skip
 
 
-@pytest.mark.parametrize("B,S,Hq,Hkv,D,C,rank,layout,two_part", CASES)
-def test_share(gpu, B, S, Hq, Hkv, D, C, rank, layout, two_part):
+def _not_used(*args, **kwargs):
+    raise AssertionError("the other path took the call")
+
+
+# (step by step: what a ring does whose chunks arrive one after the other)
+@pytest.mark.parametrize("one_launch,B,S,Hq,Hkv,D,C,rank,layout,two_part", [(True, *c) for c in CASES] + [(False, *c) for c in CASES[3:6] + CASES[9:12]])
+def test_share(gpu, monkeypatch, one_launch, B, S, Hq, Hkv, D, C, rank, layout, two_part):
+    monkeypatch.setattr(L, "FUSE_CHUNKS", one_launch)
+    for name in ("RingForward", "RingBackward") if one_launch else ("native",):
+        monkeypatch.setattr(L, name, _not_used)
     g = torch.Generator().manual_seed(5)
     mk = lambda h, d: torch.randn(B, S, h, d, generator=g).to(torch.bfloat16)  # noqa: E731
     scale, dv = D**-0.5, min(D, 128)
@@ -43,3 +43,19 @@ def test_share(gpu, B, S, Hq, Hkv, D, C, rank, layout, two_part):
     out, lse = L.ring_forward_local(q.to(gpu), on_gpu(ks), on_gpu(vs), scale, rank, C, layout, on_gpu(pes))
     check_bf16_result(out, ref_o, "O")
     check_lse(lse, ref_lse, "LSE2")
+
+    # Both sides take O as the operator has it, in bf16: delta = rowsum(dO * O) inherits its rounding (2^-9 of each |O dO|),
+    # which a row with one or two keys and a saturated softmax does not average out.
+    dout, o = mk(Hq, dv), ref_o.to(torch.bfloat16)
+    ref_dq, ref_dk, ref_dv = R.ring_backward(dout, q, o, ref_lse, full_ks, vs, scale, rank, C, layout)
+    dq, dk, dv_, *dpe = L.ring_backward_local(dout.to(gpu), q.to(gpu), o.to(gpu), ref_lse.to(gpu, torch.float32), on_gpu(ks),
+                                              on_gpu(vs), scale, rank, C, layout, on_gpu(pes))  # fmt: skip
+    check_bf16_result(dq, ref_dq, "dQ", otol=1e-3)
+    for j in range(C):
+        assert (dk[j] is None) == (ref_dk[j] is None)
+        if ref_dk[j] is None:
+            continue
+        check_bf16_result(dk[j], ref_dk[j][..., : dk[j].shape[-1]], f"chunk {j} dK", otol=1e-3)
+        check_bf16_result(dv_[j], ref_dv[j], f"chunk {j} dV", otol=1e-3)
+        if two_part:
+            check_bf16_result(dpe[0][j], ref_dk[j][..., 128:].sum(2), f"chunk {j} dk_pe", otol=1e-3)
