@@ -743,6 +743,55 @@ Three mla_assemble_fwd_autograd(const Tensor& q, const Tensor& kv, const Tensor&
   return call_mla_assemble_fwd(q, kv, k_pe, cos, sin, pos);
 }
 
+// The backward ops have no derivative of their own: under create_graph their results carry a node that raises when somebody
+// differentiates through it (without one the dispatcher would only warn and leave the second-order part out).
+struct NoSecondDerivative : torch::autograd::Function<NoSecondDerivative> {
+  static variable_list forward(AutogradContext*, at::TensorList, const std::function<variable_list()>& call) { return call(); }
+  static variable_list backward(AutogradContext*, variable_list) {
+    TORCH_CHECK(false, "Trying to backward through the backward of a pithtrain_amd operator: second derivatives are not implemented");
+  }
+};
+
+void collect(variable_list& l, const Tensor& t) {
+  if (t.defined()) l.push_back(t);
+}
+void collect(variable_list& l, const OptTensor& t) { collect(l, or_undefined(t)); }
+template <typename T>
+std::enable_if_t<std::is_arithmetic_v<T>> collect(variable_list&, T) {}
+
+template <typename... Tensors>
+std::tuple<Tensors...> as_tuple(const variable_list& l) {
+  size_t i = 0;
+  return std::tuple<Tensors...>{(Tensors)l[i++]...};
+}
+
+template <auto BODY>
+struct BackwardOp;
+template <typename... Tensors, typename... Args, std::tuple<Tensors...> (*BODY)(Args...)>
+struct BackwardOp<BODY> {
+  template <const char* NAME>
+  static std::tuple<Tensors...> call(Args... args) {
+    static const auto op = op_handle<std::tuple<Tensors...>(Args...)>(NAME);
+    bool recorded = false;
+    variable_list inputs;
+    if (at::GradMode::is_enabled()) {
+      (collect(inputs, args), ...);
+      for (const Tensor& t : inputs) recorded |= t.requires_grad();
+    }
+    const auto below = [&] {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      return op.call(args...);
+    };
+    if (!recorded) return below();
+    return as_tuple<Tensors...>(NoSecondDerivative::apply(at::TensorList(inputs), std::function<variable_list()>([&] {
+      return std::apply([](const auto&... t) { return variable_list{t...}; }, below());
+    })));
+  }
+};
+
+constexpr char kAttnBwd[] = "pithtrain_amd::attn_bwd", kNormRopeBwd[] = "pithtrain_amd::norm_rope_bwd",
+               kQkNormRopeBwd[] = "pithtrain_amd::qk_norm_rope_bwd", kMlaAssembleBwd[] = "pithtrain_amd::mla_assemble_bwd";
+
 }  // namespace
 
 TORCH_LIBRARY(pithtrain_amd, m) {
@@ -779,6 +828,10 @@ TORCH_LIBRARY_IMPL(pithtrain_amd, Autograd, m) {
   m.impl("norm_rope_fwd", &norm_rope_fwd_autograd);
   m.impl("qk_norm_rope_fwd", &qk_norm_rope_fwd_autograd);
   m.impl("mla_assemble_fwd", &mla_assemble_fwd_autograd);
+  m.impl("attn_bwd", &BackwardOp<&attn_bwd>::call<kAttnBwd>);
+  m.impl("norm_rope_bwd", &BackwardOp<&norm_rope_bwd>::call<kNormRopeBwd>);
+  m.impl("qk_norm_rope_bwd", &BackwardOp<&qk_norm_rope_bwd>::call<kQkNormRopeBwd>);
+  m.impl("mla_assemble_bwd", &BackwardOp<&mla_assemble_bwd>::call<kMlaAssembleBwd>);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
