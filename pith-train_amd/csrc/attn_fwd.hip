@@ -10,34 +10,52 @@
 namespace pith {
 namespace {
 
-// Three work splits (attn_fwd_direct.hip, attn_fwd_duo.hip), measured on one box, microseconds:
-//   FULL  one 256-row workgroup of 8 waves per compute unit: the fewest K/V tile requests per product;
-//   DUO   two 128-row workgroups of 4 waves per compute unit: twice the requests, but one's prologue, epilogue and last
-//         tiles overlap the other's loop, and the diagonal wastes half as much;
-//   HALF  one 128-row workgroup of 8 waves per compute unit, wave pairs splitting the keys of every tile: the shortest
-//         time per tile for a workgroup that has its compute unit to itself.
-//                                                FULL   DUO    HALF
-//   d128 causal  1 x 16384 x 8 heads             448    462    498
-//                3 x 1999 x 32                   105.6  105.0  131.4
-//                8 x 512 x 32                    35.8   32.2   46.7
-//                1 x 4096 x 8 (256 WGs of 128)   77.6   71.2   53.8
-//   d192 causal  1 x 32768 x 16                  4438   4376   4959
-//                1 x 4096 x 128                  694    663    810
-//                1 x 2048 x 16 (256 WGs of 128)  57.7   46.3   40.1
-// HALF: grids that leave DUO one workgroup per compute unit, unless the stream is so short (8 tiles) that the merge of the
-// halves costs more than it gives; under the mask also up to two per compute unit for longer streams, where the
-// heaviest workgroups run alone in DUO's second half. FULL: 128 features with enough rows that its coarser diagonal and
-// its rounds of workgroups no longer show; at 192 features it never won (the register budget of 256 rows forced a tile
-// maximum into every softmax) and does not exist. 64 features always use DUO (three workgroups fit there).
-enum class Split { kFull, kDuo, kHalf };
+// Work splits (attn_fwd_direct.hip, attn_fwd_duo.hip), kernels measured on one box, microseconds:
+//   FULL   one 256-row workgroup of 8 waves per compute unit: the fewest K/V tile requests per product;
+//   DUO    two 128-row workgroups of 4 waves per compute unit: twice the requests, but one's prologue, epilogue and last
+//          tiles overlap the other's loop, and the diagonal wastes half as much;
+//   HALF   one 128-row workgroup of 8 waves per compute unit, wave pairs splitting the keys of every tile;
+//   TEAMS  one 128-row workgroup of 8 waves per compute unit, two teams of 4 waves taking every second tile;
+//   QUARTER  one 64-row workgroup of 8 waves: two teams, and wave pairs of a team splitting the keys of its tile.
+// FULL and DUO when every compute unit has work for its whole time; the others, from left to right more of the device per
+// row, when workgroups are few or (under the mask) so unequal that a heavy one would run alone on its unit.
+//                                                       FULL    DUO   HALF  TEAMS QUARTER
+//   d128 causal   1 x 16384 x 8 heads                    454    470    507    515    643
+//                 3 x 1999 x 32                          109    107    133    131    187
+//                 1 x 4096 x 8  (256 WGs of 128 rows)     78     70   55.4   58.8   52.3
+//                 1 x 2048 x 16 (256 WGs)               44.8   40.2   33.5   35.0   34.9
+//                 1 x 2048 x 8  (128 WGs)               42.9   37.4   29.7   32.9   25.6
+//                 1 x 384 x 8 / 320 x 8                        11.2 / 9.5           10.9 / 10.3
+//   d192 causal   1 x 8192 x 16 (1024 WGs)                      298    339    331    430
+//                 1 x 4096 x 16 (512 WGs)                       100   94.7   92.4    125
+//                 1 x 4096 x 8  (256 WGs)                      82.4   71.4   72.0   63.7
+//                 1 x 1021 x 16 (128 WGs)                      24.9   23.5   22.5   19.2
+//        full     1 x 4096 x 8  (256 WGs)                      92.5   81.2   82.5    111
+//   d64  causal   1 x 4096 x 20 (640 WGs)                      62.4          69.7   78.0
+//                 1 x 4096 x 16 (512 WGs)                      60.5          52.6   63.4
+//                 1 x 4096 x 8  (256 WGs)                      51.0          42.1   33.0
+//                 1 x 1024 x 16 (128 WGs)                      16.2          15.1   11.7
+//        full     1 x 2048 x 16 / 32 (256 / 512 WGs)           30.9 / 38.9   27.7 / 48.8   33.6 / 62.3
+//   ring shares, 4 ranks, zigzag, d192: 4096 rows x 16 rank 0 / 3   357 / 315   329 / 332   312 / 314   430 / 423
+//                                       2048 rows x 16 rank 1 / 2   149 / 129   125 / 111   116 / 105   117 / 116
+// (d192 FULL never won: the register budget of 256 rows forced a tile maximum into every softmax.)
+enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter };
 
-Split pick_split(const pith_attn_fwd_args* a) {
-  if (a->Dqk == 64) return Split::kDuo;
+// `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50). At 192 features
+// TEAMS stands in for HALF except on a full (unmasked) chunk, where HALF is 1.5 % faster.
+Split pick_split(const pith_attn_fwd_args* a, int mean, bool full_chunk) {
   const int64_t cus = compute_units_or_default();
-  const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;  // workgroups of 128 rows
-  if (a->Skv > 512 && wgs <= cus) return Split::kHalf;
-  if (a->causal && a->Skv >= 1536 && wgs <= 2 * cus) return Split::kHalf;
-  if (a->Dqk == 128 && (a->causal ? a->Sq >= 3072 && wgs > 2 * cus : a->Skv > 1024 && wgs > cus)) return Split::kFull;
+  const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B, wgs64 = ((a->Sq + 63) / 64) * a->Hq * a->B;  // of 128 and 64 rows
+  const bool unequal = mean <= 70;
+  const Split key_split = a->Dqk == 64 || (a->Dqk == 192 && !full_chunk) ? Split::kTeams : Split::kHalf;
+  // few rows: below 6 tiles (64 features: 5) the merge costs more than the shorter streams save
+  if (wgs64 <= cus && a->Skv > (a->Dqk == 64 ? 256 : 320)) return Split::kQuarter;
+  // two 64-row workgroups per compute unit one after the other, a heavy one and a light one
+  if (unequal && wgs64 <= 2 * cus && a->Skv >= (a->Dqk == 64 ? 2048 : 4096)) return Split::kQuarter;
+  if (wgs <= cus && a->Skv > (a->Dqk == 64 ? 1024 : 512)) return key_split;
+  // at 0.8 (zigzag, last rank) TEAMS still ties with DUO or wins by 3 %, HALF is 5-10 % slower above 0.7
+  if (wgs <= 2 * cus && a->Skv >= 1536 && mean <= (a->Dqk == 192 ? 80 : 70)) return key_split;
+  if (a->Dqk == 128 && (unequal ? a->Sq >= 3072 && wgs > 2 * cus : a->Skv > 1024 && wgs > cus)) return Split::kFull;
   return Split::kDuo;
 }
 
@@ -119,8 +137,10 @@ template <typename P>
 int launch(const P& p, const pith_attn_fwd_args* a, Split split, pith_stream_t stream, const char* who) {
   hipStream_t st = (hipStream_t)stream;
   begin_launch();
-  if (split == Split::kDuo) launch_fwd_duo(p, (int)a->Dqk, a->causal != 0, st);
-  else launch_fwd_direct(p, (int)a->Dqk, a->causal != 0, split == Split::kHalf, st);
+  const int dqk = (int)a->Dqk;
+  const bool causal = a->causal != 0;
+  if (split == Split::kFull || split == Split::kHalf) launch_fwd_direct(p, dqk, causal, split == Split::kHalf, st);
+  else launch_fwd_duo(p, dqk, split == Split::kDuo ? 1 : split == Split::kTeams ? 2 : 4, causal, st);
   return check_launch(who);
 }
 
@@ -129,7 +149,7 @@ int launch(const P& p, const pith_attn_fwd_args* a, Split split, pith_stream_t s
 extern "C" int pith_attn_fwd(const pith_attn_fwd_args* a, pith_stream_t stream) {
   FwdParams p;
   if (const int rc = prepare(a, p)) return rc;
-  return launch(p, a, pick_split(a), stream, "pith_attn_fwd");
+  return launch(p, a, pick_split(a, a->causal ? 50 : 100, !a->causal), stream, "pith_attn_fwd");
 }
 
 extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
@@ -153,12 +173,9 @@ extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_k
     seen += diagonal ? c.rows * args->Sq / 2 : c.rows * (args->Sq - c.q_row0);
   }
   p.n_chunks = (int)n;
-  // The split goes by the whole stream, taken for a masked one when its rows are as unequal as those under a mask are: on
-  // two workgroups per compute unit HALF is 6-9 % faster where the mean stream is at most 0.6 of the longest (zigzag, low
-  // ranks), 2 % at 0.67, 3 % slower at 0.75 and 5-10 % above.
+  // The split goes by the whole stream and by how unequal the rows' streams are.
   a.Skv = keys;
-  a.causal = 10 * seen <= 7 * keys * args->Sq;
-  const Split split = pick_split(&a);
+  const Split split = pick_split(&a, (int)(100 * seen / (keys * args->Sq)), false);
   a.causal = 1;
   if (n == 1) return launch<FwdParams>(p, &a, split, stream, who);
   return launch(p, &a, split, stream, who);

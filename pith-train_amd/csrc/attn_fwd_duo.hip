@@ -1,5 +1,5 @@
 // Chunk attention forward for head dims (64, 64), (128, 128) and (192, 128) on gfx950 with SMALL workgroups: 4 wavefronts,
-// 128 query rows, two of them per compute unit (three at 64 features). Same function, numerics and tile layouts as
+// 128 query rows (PARTS = 1), two of them per compute unit (three at 64 features). Same function, numerics and tile layouts as
 // attn_fwd_direct.hip (pithtrain/operators/mla/triton.py:32-93, :274-323): a wave owns 32 query rows and all 64 keys of a
 // tile, per interval one matrix block [O^T += V(i)^T P(i)^T ; S(i+1)^T = K(i+1) Q^T] and one softmax.
 //
@@ -13,6 +13,14 @@
 // 64 features: a K or V tile packs two rows per 256-byte LDS row (see DirectPaired64), and the softmax of 32 x 64 scores
 // costs as much vector time as its products cost matrix time, so three workgroups per compute unit share the pipes.
 //
+// PARTS > 1: two such teams of 4 waves in one workgroup, each with its own rings, taking every second tile; the results are
+// merged through LDS. For grids that leave units idle or a heavy workgroup alone on its unit, where the length of a stream
+// counts. PARTS = 2: 128 rows as above. PARTS = 4: 64 rows, the two waves of a team that share rows take half a tile's keys
+// each: twice the requests per product, on units that have nothing else to do. Measured against the split-key workgroups of
+// attn_fwd_direct.hip (64 features: against one team): 1 x 1021 x 16 heads of 192 23.5 -> 19.2 us, its ring share of 3
+// chunks 55.4 -> 46.6, 1 x 4096 x 4 of 192 69 -> 52, 1 x 2048 x 8 of 128 29.7 -> 25.6, 1 x 8192 x 4 of 64 97 -> 58 (4
+// parts); 4096 x 16 of 192, ring share of 4 ranks 330 -> 314, 1 x 4096 x 16 of 64 61 -> 53 (2 parts). More at pick_split.
+//
 // LDS: rings of two K and two V tiles; interval i reads V(i) and K(i+1) while V(i+1) and K(i+2) land in the slots that
 // interval i-1 released.
 #include "attn_fwd_common.h"
@@ -20,41 +28,49 @@
 namespace pith {
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
-constexpr int kBM = 32 * kWaves;  // query rows per workgroup
+constexpr int kTeamWaves = 4;                 // waves that share a stream of tiles
+constexpr int kTeamThreads = kTeamWaves * 64;
 constexpr int kBN = kFwdBlockN;   // keys per tile
 constexpr int kAhead = 4;         // fragment reads run this many products ahead in the matrix block
 
-template <int DQK>
+template <int DQK, int PARTS>
 struct DuoLayout {
+  static constexpr int kTeams = PARTS == 1 ? 1 : 2;
+  static constexpr int kThreads = kTeams * kTeamThreads;
+  static constexpr int kRowBlocks = PARTS == 4 ? 2 : 4;  // of 32 query rows
+  static constexpr int kBM = 32 * kRowBlocks;            // query rows per workgroup
   static constexpr int kDv = DQK == 64 ? 64 : 128;
   static constexpr int kKTile = DQK == 64 ? kExtraTileBytes : DQK == 128 ? kBN * kRowBytes128 : kBN * kRowBytes128 + kExtraTileBytes;
   static constexpr int kVTile = kDv == 64 ? kExtraTileBytes : kBN * kRowBytes128;
-  static constexpr int kRings = 2 * (kKTile + kVTile);
-  static constexpr int kTurn = kWaves * kRowsViaLdsBytes<kDv / 32>;
-  static constexpr int kSmem = kRings > kTurn ? kRings : kTurn;
+  static constexpr int kRings = 2 * (kKTile + kVTile);   // of one team
+  static constexpr int kTurn = kRowsViaLdsBytes<kDv / 32>;
+  static constexpr int kAfter = kRowBlocks * (PARTS == 1 ? 1 : PARTS - 1) * kTurn;  // the epilogue's use of the rings
+  static constexpr int kSmem = kTeams * kRings > kAfter ? kTeams * kRings : kAfter;
 };
 
-template <int DQK, bool CAUSAL, bool MULTI>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI> p) {
-  using L = DuoLayout<DQK>;
-  constexpr int kDv = L::kDv, KS = DQK / 16, DVB = kDv / 32, KVB = 2;
+template <int DQK, int PARTS, bool CAUSAL, bool MULTI>
+__global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd_duo_kernel(FwdArgs<MULTI> p) {
+  using L = DuoLayout<DQK, PARTS>;
+  constexpr int kDv = L::kDv, KS = DQK / 16, DVB = kDv / 32, kBM = L::kBM, kTeams = L::kTeams;
+  constexpr int KVB = PARTS == 4 ? 1 : 2;  // 32-key blocks of a tile this wave owns
   constexpr bool kPaired = DQK == 64;  // tiles hold two rows per 256-byte LDS row
   constexpr int kTile = kBN * kRowBytes128;
   __shared__ __attribute__((aligned(1024))) char smem[L::kSmem];
-  char* const kbuf = smem;
-  char* const vbuf = smem + 2 * L::kKTile;
-
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, wg_wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wg_wave & (kTeamWaves - 1);              // within its team
+  const int team = kTeams == 1 ? 0 : wg_wave / kTeamWaves;  // takes the tiles t with t % kTeams == team
+  const int row_block = wave & (L::kRowBlocks - 1);
+  const int kvb0 = PARTS == 4 ? wave >> 1 : 0;              // first 32-key block of a tile this wave owns
+  char* const kbuf = smem + team * L::kRings;
+  char* const vbuf = kbuf + 2 * L::kKTile;
   const int c = lane & 31, g = lane >> 5;
 
   int m_tile, h, b;
   decode_block(blockIdx.x, p.Hq, p.B, p.m_tiles, p.group, m_tile, h, b);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
-  const int q_wave0 = m0 + wave * 32;
+  const int q_wave0 = m0 + row_block * 32;
   const int qrow = q_wave0 + c;
 
   const int64_t q_row_stride = (int64_t)p.Hq * DQK;
@@ -84,12 +100,24 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
     n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
     n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
+  const int intervals = (n_tiles_wg + kTeams - 1) / kTeams;  // of the workgroup
+  if constexpr (kTeams > 1) {  // from here on a team's own tiles (the second team of a single tile has none)
+    n_tiles_wg = (n_tiles_wg + 1 - team) >> 1;
+    n_tiles_wave = (n_tiles_wave + 1 - team) >> 1;
+  }
+  auto tile = [&](int t) __attribute__((always_inline)) { return kTeams * t + team; };  // in the workgroup's stream
   TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows),
       v_src(p, range, v_row_bytes, v_rows);
   TileMask<MULTI, CAUSAL, kBN> mask(p, range);
+  if (team == 1) {
+    k_src.advance(p, range, k_rows);
+    if constexpr (DQK == 192) kx_src.advance(p, range, kx_rows);
+    v_src.advance(p, range, v_rows);
+    mask.advance(p, range);
+  }
 
-  DirectTile128<kBN, kThreads> vmover, kmover;
-  DirectPaired64<kBN, kThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
+  DirectTile128<kBN, kTeamThreads> vmover, kmover;
+  DirectPaired64<kBN, kTeamThreads> vpmover, kpmover;  // 64-feature tiles, and features 128..191 of a 192-feature key
   if constexpr (kPaired) {
     vpmover.init(v_row_bytes, 0, wave, lane);
     kpmover.init(k_row_bytes, 0, wave, lane);
@@ -101,25 +129,29 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
   // (tiles are requested strictly in order, so the sources just move on)
   auto issue_k = [&](int t) __attribute__((always_inline)) {
     char* slot = kbuf + (t & 1) * L::kKTile;
+    const int at = tile(t);
     if constexpr (kPaired) {
-      kpmover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
+      kpmover.issue(k_src.src(at), k_src.left(at), slot, wave, lane);
     } else {
-      kmover.issue(k_src.src(t), k_src.left(t), slot, wave, lane);
+      kmover.issue(k_src.src(at), k_src.left(at), slot, wave, lane);
       if constexpr (DQK == 192) {
-        kpmover.issue(kx_src.src(t), kx_src.left(t), slot + kTile, wave, lane);
-        kx_src.advance(p, range, kx_rows);
+        kpmover.issue(kx_src.src(at), kx_src.left(at), slot + kTile, wave, lane);
+        for (int n = 0; n < kTeams; ++n) kx_src.advance(p, range, kx_rows);
       }
     }
-    k_src.advance(p, range, k_rows);
+    for (int n = 0; n < kTeams; ++n) k_src.advance(p, range, k_rows);
   };
   auto issue_v = [&](int t) __attribute__((always_inline)) {
     char* slot = vbuf + (t & 1) * L::kVTile;
-    if constexpr (kPaired) vpmover.issue(v_src.src(t), v_src.left(t), slot, wave, lane);
-    else vmover.issue(v_src.src(t), v_src.left(t), slot, wave, lane);
-    v_src.advance(p, range, v_rows);
+    const int at = tile(t);
+    if constexpr (kPaired) vpmover.issue(v_src.src(at), v_src.left(at), slot, wave, lane);
+    else vmover.issue(v_src.src(at), v_src.left(at), slot, wave, lane);
+    for (int n = 0; n < kTeams; ++n) v_src.advance(p, range, v_rows);
   };
-  issue_k(0);
-  issue_v(0);
+  if (kTeams == 1 || n_tiles_wg > 0) {
+    issue_k(0);
+    issue_v(0);
+  }
   if (n_tiles_wg > 1) issue_k(1);
 
   // Q^T fragments (B operand): column = query row, slots = 8 consecutive features.
@@ -132,16 +164,18 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
   }
 
   // per-lane read offsets (see attn_fwd_direct.hip): one base per tile part, the rest by XOR
-  int k_base = straight_offset128(c, g);
+  // (KVB = 1: the wave's key block sits in the bases)
+  const int k_base = straight_offset128(c, g) + kvb0 * 32 * kRowBytes128, x_base = straight_offset128(c, g) ^ (kvb0 << 7);
   int v_base[2] = {transposed_offset128(0, 0, 0, lane), transposed_offset128(0, 1, 0, lane)};
+  for (int& v : v_base) v = kPaired ? v ^ (kvb0 << 7) : v + kvb0 * 32 * kRowBytes128;
   auto k_frag = [&](const char* ktile, int ks, int kvb) __attribute__((always_inline)) {
     int off;
-    if (kPaired) off = k_base ^ (ks << 5) ^ (kvb << 7);
+    if (kPaired) off = x_base ^ (ks << 5) ^ (kvb << 7);
     else if (ks < 8) off = (k_base ^ (ks << 5)) + kvb * 32 * kRowBytes128;
-    else off = kTile + (k_base ^ ((ks - 8) << 5) ^ (kvb << 7));
+    else off = kTile + (x_base ^ ((ks - 8) << 5) ^ (kvb << 7));
     return *reinterpret_cast<const bf16x8*>(ktile + off);
   };
-  // 16 keys j, feature block i
+  // 16 keys j of the wave's, feature block i
   auto v_frag = [&](const char* vtile, int j, int i) __attribute__((always_inline)) {
     const int add = kPaired ? (j & 1) * 16 * kRowBytes128 : j * 16 * kRowBytes128;
     const int flip = kPaired ? (i << 6) | ((j >> 1) << 7) : i << 6;
@@ -172,17 +206,18 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
 
   // ---- mask, online softmax of the next tile in order (one query column per lane pair), P^T fragments
   auto softmax = [&](int t) __attribute__((always_inline)) {
-    if (mask.partial(range, t, q_wave0)) {
+    const int at = tile(t);
+    if (mask.partial(range, at, q_wave0)) {
       const int limit = mask.limit(range, qrow);
 #pragma unroll
       for (int kvb = 0; kvb < KVB; ++kvb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int key = mask.key0(t) + kvb * 32 + acc_row(v, g);
+          const int key = mask.key0(at) + (kvb0 + kvb) * 32 + acc_row(v, g);
           if (key > limit) s[kvb][v] = -INFINITY;
         }
     }
-    mask.advance(p, range);
+    for (int n = 0; n < kTeams; ++n) mask.advance(p, range);
     f32x16 e[KVB];
     float rs = 0.f;
     // lazily refreshed running maximum, tested on the row sum (attn_fwd_direct.hip)
@@ -281,26 +316,91 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
 
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
-  scores(kbuf);
-  softmax(0);
+  const bool any = kTeams == 1 || n_tiles_wave > 0;
+  if (any) scores(kbuf);
+  if (team == 0) softmax(0);
   __syncthreads();  // K tile 0 has been read: its slot may be refilled
 
-  // interval i: O += V(i)^T P(i), S(i+1) = K(i+1) Q^T, P(i+1); K(i+2) and V(i+1) are requested meanwhile
-  int i = 0;
-  for (; i + 1 < n_tiles_wave; ++i) {
-    if (i + 2 < n_tiles_wg) issue_k(i + 2);
-    issue_v(i + 1);
-    matrix_block(vbuf + (i & 1) * L::kVTile, kbuf + ((i + 1) & 1) * L::kKTile);
-    softmax(i + 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+  // interval i: O += V(i)^T P(i), S(i+1) = K(i+1) Q^T, P(i+1); K(i+2) and V(i+1) are requested meanwhile. The second team
+  // takes the softmax first (of S(i)): the two waves of a SIMD are in different phases.
+  auto run = [&](auto second_tag) __attribute__((always_inline)) {
+    constexpr bool SECOND = decltype(second_tag)::value;
+    int i = 0;
+    for (; i + 1 < n_tiles_wave; ++i) {
+      if (i + 2 < n_tiles_wg) issue_k(i + 2);
+      issue_v(i + 1);
+      if constexpr (SECOND) {
+        softmax(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      matrix_block(vbuf + (i & 1) * L::kVTile, kbuf + ((i + 1) & 1) * L::kKTile);
+      if constexpr (!SECOND) softmax(i + 1);
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+    for (; i < intervals; ++i) {
+      if (i + 2 < n_tiles_wg) issue_k(i + 2);
+      if (i + 1 < n_tiles_wg) issue_v(i + 1);
+      if (i < n_tiles_wave) {
+        if constexpr (SECOND) softmax(i);
+        accumulate(vbuf + (i & 1) * L::kVTile);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+  };
+  if (kTeams == 1 || team == 0) run(std::false_type{});
+  else run(std::true_type{});
+
+  // ---- several parts: the other waves of a row block hand accumulator, maximum and sum to its first one, which rescales
+  // all to the common maximum and adds them. The rings are free (every wave passed the barrier behind the last interval).
+  if constexpr (PARTS > 1) {
+    constexpr int kExch = L::kTurn;  // DVB * 16 accumulator values and (m, l) per lane
+    static_assert(kExch == DVB * 4 * 64 * 16 + 64 * 8, "exchange area");
+    const int part = PARTS == 4 ? 2 * team + kvb0 : team;
+    auto area = [&](int from) __attribute__((always_inline)) { return smem + ((from - 1) * L::kRowBlocks + row_block) * kExch; };
+    if (part > 0) {
+      char* const exch = area(part);
+#pragma unroll
+      for (int i = 0; i < DVB; ++i)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x4 v4 = {oacc[i][4 * b4], oacc[i][4 * b4 + 1], oacc[i][4 * b4 + 2], oacc[i][4 * b4 + 3]};
+          *reinterpret_cast<f32x4*>(exch + ((i * 4 + b4) * 64 + lane) * 16) = v4;
+        }
+      const f32x2 ml = {m_run, l_run};
+      *reinterpret_cast<f32x2*>(exch + DVB * 4 * 64 * 16 + lane * 8) = ml;
+    }
     __syncthreads();
-  }
-  for (; i < n_tiles_wg; ++i) {
-    if (i + 2 < n_tiles_wg) issue_k(i + 2);
-    if (i + 1 < n_tiles_wg) issue_v(i + 1);
-    if (i < n_tiles_wave) accumulate(vbuf + (i & 1) * L::kVTile);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    if (part > 0) return;
+    f32x2 ml[PARTS - 1];
+    float m_new = m_run;
+#pragma unroll
+    for (int n = 0; n < PARTS - 1; ++n) {
+      ml[n] = *reinterpret_cast<const f32x2*>(area(n + 1) + DVB * 4 * 64 * 16 + lane * 8);
+      m_new = fmaxf(m_new, ml[n][0]);
+    }
+    // a part that saw no key has m = -inf, l = 0 and a zero accumulator: weight 0
+    const float w0 = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
+    m_run = m_new;
+    l_run *= w0;
+#pragma unroll
+    for (int i = 0; i < DVB; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) oacc[i][v] *= w0;
+#pragma unroll
+    for (int n = 0; n < PARTS - 1; ++n) {
+      const float w = (ml[n][0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((ml[n][0] - m_new) * p.kappa);
+      l_run += ml[n][1] * w;
+#pragma unroll
+      for (int i = 0; i < DVB; ++i)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x4 v4 = *reinterpret_cast<const f32x4*>(area(n + 1) + ((i * 4 + b4) * 64 + lane) * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[i][4 * b4 + e] += v4[e] * w;
+        }
+    }
   }
 
   // ---- epilogue: normalise, store O (bf16) and LSE2; the rings are free (every wave passed the last barrier)
@@ -308,7 +408,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
   float* lse = p.lse + b * p.lse_bs + (int64_t)h * p.lse_hs;
   const float l = pair_sum(l_run);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  char* const turn = smem + wave * kRowsViaLdsBytes<DVB>;
+  char* const turn = smem + row_block * L::kTurn;
   if constexpr (!CAUSAL && kDv == 128) {
     if (p.prev_o != nullptr) {  // merge with the running result of the rows, as in attn_fwd_direct.hip
       const float lse_new = l > 0.f ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
@@ -334,29 +434,37 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_duo_kernel(FwdArgs<MULTI
   if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
-template <int DQK, bool MULTI>
+template <int DQK, int PARTS, bool MULTI>
 void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
-  p.m_tiles = (p.Sq + kBM - 1) / kBM;
-  const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
+  using L = DuoLayout<DQK, PARTS>;
+  p.m_tiles = (p.Sq + L::kBM - 1) / L::kBM;
+  const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(L::kThreads);
   if constexpr (MULTI) {  // the last chunk is seen under the mask
-    hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, true>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, PARTS, true, true>), grid, block, 0, st, p);
   } else {
-    if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, true, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, false, false>), grid, block, 0, st, p);
+    if (causal) hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, PARTS, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, PARTS, false, false>), grid, block, 0, st, p);
   }
 }
 
+template <int DQK, bool MULTI>
+void launch_parts(const FwdArgs<MULTI>& p, int parts, bool causal, hipStream_t st) {
+  if (parts == 1) launch_one<DQK, 1, MULTI>(p, causal, st);
+  else if (parts == 2) launch_one<DQK, 2, MULTI>(p, causal, st);
+  else launch_one<DQK, 4, MULTI>(p, causal, st);
+}
+
 template <bool MULTI>
-void launch_dim(const FwdArgs<MULTI>& p, int dqk, bool causal, hipStream_t st) {
-  if (dqk == 64) launch_one<64, MULTI>(p, causal, st);
-  else if (dqk == 128) launch_one<128, MULTI>(p, causal, st);
-  else launch_one<192, MULTI>(p, causal, st);
+void launch_dim(const FwdArgs<MULTI>& p, int dqk, int parts, bool causal, hipStream_t st) {
+  if (dqk == 64) launch_parts<64, MULTI>(p, parts, causal, st);
+  else if (dqk == 128) launch_parts<128, MULTI>(p, parts, causal, st);
+  else launch_parts<192, MULTI>(p, parts, causal, st);
 }
 
 }  // namespace
 
-void launch_fwd_duo(const FwdParams& p, int dqk, bool causal, hipStream_t st) { launch_dim<false>(p, dqk, causal, st); }
+void launch_fwd_duo(const FwdParams& p, int dqk, int parts, bool causal, hipStream_t st) { launch_dim<false>(p, dqk, parts, causal, st); }
 
-void launch_fwd_duo(const FwdChunkParams& p, int dqk, bool causal, hipStream_t st) { launch_dim<true>(p, dqk, causal, st); }
+void launch_fwd_duo(const FwdChunkParams& p, int dqk, int parts, bool causal, hipStream_t st) { launch_dim<true>(p, dqk, parts, causal, st); }
 
 }  // namespace pith

@@ -59,3 +59,8 @@ def test_share(gpu, monkeypatch, one_launch, B, S, Hq, Hkv, D, C, rank, layout, 
         check_bf16_result(dv_[j], ref_dv[j], f"chunk {j} dV", otol=1e-3)
         if two_part:
             check_bf16_result(dpe[0][j], ref_dk[j][..., 128:].sum(2), f"chunk {j} dk_pe", otol=1e-3)
+
+
+def test_share_of_unequal_rows_64_features(gpu, monkeypatch):
+    """The two-team forward over several chunks."""
+    test_share(gpu, monkeypatch, True, 1, 1022, 36, 36, 64, 2, 0, "zigzag", False)
