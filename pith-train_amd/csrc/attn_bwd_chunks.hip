@@ -4,7 +4,10 @@
 //          call; in chunks without a mask all key positions lie below the first query row.
 //   dQ     a workgroup walks the key tiles of every chunk its rows see as one stream, dQ stays in registers throughout and is
 //          written once, as bf16 (no fp32 accumulator that every ring step reads and writes, no cast at the end).
-// As for chunk pairs, small launches put both into one grid (attn_bwd_pair.hip).
+// As for chunk pairs, small launches put both into one grid (attn_bwd_pair.hip), here with the longer kind first: dQ
+// workgroups walk all chunks, and started behind the dK/dV ones of every chunk they are what the launch ends on. Measured,
+// dK/dV first against dQ first: 1021 rows x 16 heads of 192, 4 ranks, contiguous 135 -> 122 us; 1024 x 16 of 192, zigzag
+// 118 -> 96; 1024 x 8/2 of 128, rank 0 102 -> 85; 2 x 1536 x 16/4 of 64 207 -> 179; 2048 x 4 of 192, 8 ranks 290 -> 245.
 #include "attn_bwd_common.h"
 #include "attn_bwd_dkdv_d128.h"
 #include "attn_bwd_dkdv_d192.h"
@@ -50,8 +53,9 @@ __global__ __launch_bounds__(dq_direct::kThreads) void attn_bwd_dq_direct_chunks
 }
 
 template <int DQK>
-__global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_pair_chunks_kernel(BwdChunkParams p, int dkdv_blocks) {
-  const int block = blockIdx.x;
+__global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_pair_chunks_kernel(BwdChunkParams p, int dkdv_blocks, int dq_first) {
+  const int dq_blocks = gridDim.x - dkdv_blocks;
+  const int block = dq_first ? ((int)blockIdx.x < dq_blocks ? dkdv_blocks + blockIdx.x : blockIdx.x - dq_blocks) : blockIdx.x;
   if constexpr (DQK == 64) {
     __shared__ __attribute__((aligned(1024))) char smem[larger(kDkdvSmem<64>, dq_duo::kSmem<64>)];
     if (block < dkdv_blocks) dkdv_body<64>(p, smem, block);
@@ -64,10 +68,10 @@ __global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_pair_chunks_ker
 }
 
 template <int DQK>
-void launch_dim(const BwdChunkParams& p, bool one_grid, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
+void launch_dim(const BwdChunkParams& p, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
   const unsigned dq_blocks = (unsigned)(p.q_tiles * p.Hq * p.B);
   if (one_grid) {
-    hipLaunchKernelGGL((attn_bwd_pair_chunks_kernel<DQK>), dim3(dkdv_blocks + dq_blocks), dim3(kDkdvThreads<DQK>), 0, st, p, (int)dkdv_blocks);
+    hipLaunchKernelGGL((attn_bwd_pair_chunks_kernel<DQK>), dim3(dkdv_blocks + dq_blocks), dim3(kDkdvThreads<DQK>), 0, st, p, (int)dkdv_blocks, (int)dq_first);
     return;
   }
   hipLaunchKernelGGL((attn_bwd_dkdv_chunks_kernel<DQK>), dim3(dkdv_blocks), dim3(kDkdvThreads<DQK>), 0, st, p);
@@ -82,10 +86,10 @@ void launch_dim(const BwdChunkParams& p, bool one_grid, bool split_keys, unsigne
 
 }  // namespace
 
-void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
-  if (dqk == 64) launch_dim<64>(p, one_grid, split_keys, dkdv_blocks, st);
-  else if (dqk == 128) launch_dim<128>(p, one_grid, split_keys, dkdv_blocks, st);
-  else launch_dim<192>(p, one_grid, split_keys, dkdv_blocks, st);
+void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
+  if (dqk == 64) launch_dim<64>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
+  else if (dqk == 128) launch_dim<128>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
+  else launch_dim<192>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
 }
 
 }  // namespace pith

@@ -254,8 +254,8 @@ void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned gr
 bool launch_bwd_pair(const BwdParams& p, int dqk, bool causal, bool dkdv_f32, bool dq_f32, unsigned dkdv_blocks, hipStream_t stream);
 
 // The backward of a chunk call: attn_bwd_chunks.hip. dkdv_blocks = the dK/dV grid; p.q_tiles = 128-row query tiles; split_keys
-// as for launch_dq_direct / launch_dq_duo (one_grid implies it at 128 and 192 features).
-void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool split_keys, unsigned dkdv_blocks, hipStream_t stream);
+// as for launch_dq_direct / launch_dq_duo (one_grid implies it at 128 and 192 features); dq_first: one grid starts with dQ.
+void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t stream);
 
 // dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
 // split every tile's keys: attn_bwd_dq_direct.hip.

@@ -235,14 +235,15 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
 
 // Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
 // split-key ones (the two kernels must agree on the workgroup size), which is what grids of up to one workgroup per compute
-// unit want anyway; larger ones fill the device with either kernel and gain nothing (1 x 4096 x 16 heads of 192 features,
-// 512 + 512 workgroups: 293 us apart, 298 us together). At 64 features one kernel costs dQ its third workgroup per compute
-// unit (186 instead of 150 registers), which only grids of a few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us,
-// 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16 474 -> 483 us).
-bool one_grid(const pith_attn_bwd_args* a) {
+// unit want anyway. With two per unit a chunk pair gains nothing (1 x 4096 x 16 heads of 192 features: 293 us apart, 298 us
+// together), several chunks, whose dK/dV workgroups are more unequal, 1-5 % (2048 x 32/4 of 128, 4 ranks, zigzag, rank 0:
+// 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081); with three it loses (6144 x 16 of 192: 2385 -> 2413). At 64
+// features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only grids of a
+// few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us, 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16 474 -> 483 us).
+bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
   if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
   const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
-  return q_wgs <= (a->Dqk == 64 ? 4 : 1) * (int64_t)compute_units_or_default();
+  return q_wgs <= (a->Dqk == 64 ? 4 : chunks ? 2 : 1) * (int64_t)compute_units_or_default();
 }
 
 }  // namespace
@@ -253,7 +254,7 @@ extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t str
 
 extern "C" int pith_attn_bwd(const pith_attn_bwd_args* a, pith_stream_t stream) {
   if (const int rc = validate_bwd(a, "pith_attn_bwd", true, true)) return rc;
-  if (one_grid(a)) return bwd_dkdv(a, stream, "pith_attn_bwd", true);
+  if (one_grid(a, false)) return bwd_dkdv(a, stream, "pith_attn_bwd", true);
   if (const int rc = pith_attn_bwd_dkdv(a, stream)) return rc;
   return pith_attn_bwd_dq(a, stream);
 }
@@ -372,7 +373,12 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));
   hipStream_t st = (hipStream_t)stream;
   begin_launch();
-  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all), dq_split_keys(&all), blocks, st);
+  // In one grid the longer workgroups go first: dQ's cost 3 products per key of all chunks, dK/dV's 4 per query row and head
+  // of the part. With more than a workgroup of either per compute unit the dK/dV ones, unequal over the chunks, come first in
+  // any case (128 and 192 features): 2048 x 32/4 of 128, rank 0: 498 us, dQ first 518; 4096 x 16 of 192, rank 3: 1081 and 1084.
+  const bool few = all.Dqk == 64 || ((all.Sq + 127) / 128) * all.Hq * all.B <= (int64_t)compute_units_or_default();
+  const bool dq_first = few && 3 * all.Skv > 4 * all.Sq * (all.Hq / all.Hkv / split);
+  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, true), dq_first, dq_split_keys(&all), blocks, st);
   if (all.k_pe || split > 1) {  // (never both: keys in two parts have no head groups to split)
     Reduction<2 * kMaxChunks> r;
     for (int64_t i = 0; i < n; ++i) {
