@@ -10,51 +10,53 @@
 namespace pith {
 namespace {
 
-// Work splits (attn_fwd_direct.hip, attn_fwd_duo.hip), kernels measured on one box, microseconds:
+// Work splits (attn_fwd_direct.hip, attn_fwd_duo.hip):
 //   FULL   one 256-row workgroup of 8 waves per compute unit: the fewest K/V tile requests per product;
 //   DUO    two 128-row workgroups of 4 waves per compute unit: twice the requests, but one's prologue, epilogue and last
 //          tiles overlap the other's loop, and the diagonal wastes half as much;
 //   HALF   one 128-row workgroup of 8 waves per compute unit, wave pairs splitting the keys of every tile;
-//   TEAMS  one 128-row workgroup of 8 waves per compute unit, two teams of 4 waves taking every second tile;
+//   TEAMS  one 128-row workgroup of 8 waves per compute unit, two teams of 4 waves taking every second tile (64 features);
 //   QUARTER  one 64-row workgroup of 8 waves: two teams, and wave pairs of a team splitting the keys of its tile.
-// FULL and DUO when every compute unit has work for its whole time; the others, from left to right more of the device per
-// row, when workgroups are few or (under the mask) so unequal that a heavy one would run alone on its unit.
+// FULL and DUO when every compute unit has work for its whole time; the others when workgroups are few or (under the mask)
+// so unequal that a heavy one would run alone on its unit. Kernels measured on one box, microseconds, with inputs that
+// rotate over 500 MB (the tiles come from memory, as in a training step; the prefetch depth counts then: TEAMS at 192
+// features, two tiles per ring, beat HALF by 2-8 % on inputs in the last-level cache and lost 4-9 % here):
 //                                                       FULL    DUO   HALF  TEAMS QUARTER
-//   d128 causal   1 x 16384 x 8 heads                    454    470    507    515    643
-//                 3 x 1999 x 32                          109    107    133    131    187
-//                 1 x 4096 x 8  (256 WGs of 128 rows)     78     70   55.4   58.8   52.3
-//                 1 x 2048 x 16 (256 WGs)               44.8   40.2   33.5   35.0   34.9
-//                 1 x 2048 x 8  (128 WGs)               42.9   37.4   29.7   32.9   25.6
-//                 1 x 384 x 8 / 320 x 8                        11.2 / 9.5           10.9 / 10.3
-//   d192 causal   1 x 8192 x 16 (1024 WGs)                      298    339    331    430
-//                 1 x 4096 x 16 (512 WGs)                       100   94.7   92.4    125
-//                 1 x 4096 x 8  (256 WGs)                      82.4   71.4   72.0   63.7
-//                 1 x 1021 x 16 (128 WGs)                      24.9   23.5   22.5   19.2
-//        full     1 x 4096 x 8  (256 WGs)                      92.5   81.2   82.5    111
-//   d64  causal   1 x 4096 x 20 (640 WGs)                      62.4          69.7   78.0
-//                 1 x 4096 x 16 (512 WGs)                      60.5          52.6   63.4
-//                 1 x 4096 x 8  (256 WGs)                      51.0          42.1   33.0
-//                 1 x 1024 x 16 (128 WGs)                      16.2          15.1   11.7
-//        full     1 x 2048 x 16 / 32 (256 / 512 WGs)           30.9 / 38.9   27.7 / 48.8   33.6 / 62.3
-//   ring shares, 4 ranks, zigzag, d192: 4096 rows x 16 rank 0 / 3   357 / 315   329 / 332   312 / 314   430 / 423
-//                                       2048 rows x 16 rank 1 / 2   149 / 129   125 / 111   116 / 105   117 / 116
+//   d128 causal   1 x 16384 x 8 heads (cached)           454    470    507    515    643
+//                 3 x 1999 x 32 (cached)                 109    107    133    131    187
+//                 1 x 4096 x 8  (256 WGs of 128 rows)   82.1   76.6   61.4   68.2   64.2
+//                 1 x 4096 x 6  (192 WGs)               79.5   71.1   57.0   64.5   50.9
+//                 1 x 8192 x 4  (256 WGs)                150    137    109    123    108
+//                 1 x 2048 x 8  (128 WGs)               43.4   37.8   30.5   33.7   26.4
+//                 1 x 384 x 8 / 320 x 8 (cached)               11.2 / 9.5           10.9 / 10.3
+//   d192 causal   1 x 8192 x 16 (1024 WGs, cached)              298    339    331    430
+//                 1 x 4096 x 16 (512 WGs)                       112    100    110    152
+//                 1 x 4096 x 8  (256 WGs)                      85.6   74.2   84.2   78.2
+//                 1 x 1021 x 16 (128 WGs)                      27.3   25.9   28.8   24.0
+//   d64  causal   1 x 4096 x 20 (640 WGs, cached)              62.4          69.7   78.0
+//                 1 x 4096 x 16 (512 WGs)                      57.2          52.9   65.0
+//                 2 x 2048 x 16 (512 WGs)                      32.0          32.4   44.4
+//                 1 x 4096 x 8  (256 WGs)                      52.4          42.7   43.6
+//                 1 x 1024 x 16 (128 WGs)                      16.4          15.2   11.8
+//        full     1 x 2048 x 16 (256 WGs)                      30.3          27.4   39.9
+//   ring shares, 4 ranks, zigzag: d192 4096 rows x 16 rank 0 / 3    416 / 323   367 / 342   385 / 330   530 / 460
+//                                      2048 rows x 16 rank 0 / 2    180 / 136   142 / 113   149 / 117   130 / 121
+//                                 d128 4096 rows x 8/2 rank 0       281         218         239         195
 // (d192 FULL never won: the register budget of 256 rows forced a tile maximum into every softmax.)
 enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter };
 
-// `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50). At 192 features
-// TEAMS stands in for HALF except on a full (unmasked) chunk, where HALF is 1.5 % faster.
-Split pick_split(const pith_attn_fwd_args* a, int mean, bool full_chunk) {
+// `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50).
+Split pick_split(const pith_attn_fwd_args* a, int mean) {
   const int64_t cus = compute_units_or_default();
   const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B, wgs64 = ((a->Sq + 63) / 64) * a->Hq * a->B;  // of 128 and 64 rows
-  const bool unequal = mean <= 70;
-  const Split key_split = a->Dqk == 64 || (a->Dqk == 192 && !full_chunk) ? Split::kTeams : Split::kHalf;
+  const bool d64 = a->Dqk == 64, unequal = mean <= 70;  // HALF is 3 % slower than DUO at 0.75, 5-10 % above
   // few rows: below 6 tiles (64 features: 5) the merge costs more than the shorter streams save
-  if (wgs64 <= cus && a->Skv > (a->Dqk == 64 ? 256 : 320)) return Split::kQuarter;
-  // two 64-row workgroups per compute unit one after the other, a heavy one and a light one
-  if (unequal && wgs64 <= 2 * cus && a->Skv >= (a->Dqk == 64 ? 2048 : 4096)) return Split::kQuarter;
-  if (wgs <= cus && a->Skv > (a->Dqk == 64 ? 1024 : 512)) return key_split;
-  // at 0.8 (zigzag, last rank) TEAMS still ties with DUO or wins by 3 %, HALF is 5-10 % slower above 0.7
-  if (wgs <= 2 * cus && a->Skv >= 1536 && mean <= (a->Dqk == 192 ? 80 : 70)) return key_split;
+  if (wgs64 <= cus && a->Skv > (d64 ? 256 : 320)) return Split::kQuarter;
+  // more 64-row workgroups than compute units: heavy ones first, then light ones, as long as the streams are long
+  if (!d64 && unequal && ((2 * wgs64 <= 3 * cus && a->Skv >= 2048) || (wgs64 <= 2 * cus && a->Skv >= 6144))) return Split::kQuarter;
+  const Split key_split = d64 ? Split::kTeams : Split::kHalf;
+  if (wgs <= cus && a->Skv > (d64 ? 1024 : 512)) return key_split;
+  if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 1535)) return key_split;
   if (a->Dqk == 128 && (unequal ? a->Sq >= 3072 && wgs > 2 * cus : a->Skv > 1024 && wgs > cus)) return Split::kFull;
   return Split::kDuo;
 }
@@ -149,7 +151,7 @@ int launch(const P& p, const pith_attn_fwd_args* a, Split split, pith_stream_t s
 extern "C" int pith_attn_fwd(const pith_attn_fwd_args* a, pith_stream_t stream) {
   FwdParams p;
   if (const int rc = prepare(a, p)) return rc;
-  return launch(p, a, pick_split(a, a->causal ? 50 : 100, !a->causal), stream, "pith_attn_fwd");
+  return launch(p, a, pick_split(a, a->causal ? 50 : 100), stream, "pith_attn_fwd");
 }
 
 extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
@@ -175,7 +177,7 @@ extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_k
   p.n_chunks = (int)n;
   // The split goes by the whole stream and by how unequal the rows' streams are.
   a.Skv = keys;
-  const Split split = pick_split(&a, (int)(100 * seen / (keys * args->Sq)), false);
+  const Split split = pick_split(&a, (int)(100 * seen / (keys * args->Sq)));
   a.causal = 1;
   if (n == 1) return launch<FwdParams>(p, &a, split, stream, who);
   return launch(p, &a, split, stream, who);

@@ -48,13 +48,13 @@ __device__ __forceinline__ const KeyChunk& chunk_of(const FwdChunkParams& p, int
 __device__ __forceinline__ int chunk_count(const FwdParams&) { return 1; }
 __device__ __forceinline__ int chunk_count(const FwdChunkParams& p) { return p.n_chunks; }
 
-// Forward with one 8-wave workgroup per compute unit: attn_fwd_direct.hip. dqk = 128, or 192 on an unmasked chunk with half;
-// half = workgroups of 128 query rows whose wave pairs split the keys of every tile (see there) instead of 256-row workgroups.
+// Forward with one 8-wave workgroup per compute unit: attn_fwd_direct.hip. dqk = 128, or 192 with half; half = workgroups
+// of 128 query rows whose wave pairs split the keys of every tile (see there) instead of 256-row workgroups.
 void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipStream_t stream);
 void launch_fwd_direct(const FwdChunkParams& p, int dqk, bool causal, bool half, hipStream_t stream);
 
-// attn_fwd_duo.hip. parts = 1: two (64 features: three) 4-wave workgroups of 128 query rows per compute unit; 2 or 4: one
-// 8-wave workgroup of 128 or 64 rows, whose key stream is split in that many parts.
+// attn_fwd_duo.hip. parts = 1: two (64 features: three) 4-wave workgroups of 128 query rows per compute unit; 2 (64
+// features) or 4: one 8-wave workgroup of 128 or 64 rows, whose key stream is split in that many parts.
 void launch_fwd_duo(const FwdParams& p, int dqk, int parts, bool causal, hipStream_t stream);
 void launch_fwd_duo(const FwdChunkParams& p, int dqk, int parts, bool causal, hipStream_t stream);
 

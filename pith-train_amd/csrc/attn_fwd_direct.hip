@@ -511,25 +511,27 @@ void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(kThreads);
   if constexpr (MULTI) {  // the last chunk is seen under the mask
     hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, true>), grid, block, 0, st, p);
-  } else if constexpr (DQK == 192) {
-    hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false, false>), grid, block, 0, st, p);
   } else {
     if (causal) hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, true, false>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((attn_fwd_direct_kernel<DQK, HALF, false, false>), grid, block, 0, st, p);
   }
 }
 
+template <bool MULTI>
+void launch_split(const FwdArgs<MULTI>& p, int dqk, bool causal, bool half, hipStream_t st) {
+  if (dqk == 192) launch_one<192, true, MULTI>(p, causal, st);
+  else if (half) launch_one<128, true, MULTI>(p, causal, st);
+  else launch_one<128, false, MULTI>(p, causal, st);
+}
+
 }  // namespace
 
 void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipStream_t st) {
-  if (dqk == 192) launch_one<192, true, false>(p, false, st);
-  else if (half) launch_one<128, true, false>(p, causal, st);
-  else launch_one<128, false, false>(p, causal, st);
+  launch_split<false>(p, dqk, causal, half, st);
 }
 
-void launch_fwd_direct(const FwdChunkParams& p, int, bool causal, bool half, hipStream_t st) {
-  if (half) launch_one<128, true, true>(p, causal, st);
-  else launch_one<128, false, true>(p, causal, st);
+void launch_fwd_direct(const FwdChunkParams& p, int dqk, bool causal, bool half, hipStream_t st) {
+  launch_split<true>(p, dqk, causal, half, st);
 }
 
 }  // namespace pith

@@ -17,9 +17,10 @@
 // merged through LDS. For grids that leave units idle or a heavy workgroup alone on its unit, where the length of a stream
 // counts. PARTS = 2: 128 rows as above. PARTS = 4: 64 rows, the two waves of a team that share rows take half a tile's keys
 // each: twice the requests per product, on units that have nothing else to do. Measured against the split-key workgroups of
-// attn_fwd_direct.hip (64 features: against one team): 1 x 1021 x 16 heads of 192 23.5 -> 19.2 us, its ring share of 3
-// chunks 55.4 -> 46.6, 1 x 4096 x 4 of 192 69 -> 52, 1 x 2048 x 8 of 128 29.7 -> 25.6, 1 x 8192 x 4 of 64 97 -> 58 (4
-// parts); 4096 x 16 of 192, ring share of 4 ranks 330 -> 314, 1 x 4096 x 16 of 64 61 -> 53 (2 parts). More at pick_split.
+// attn_fwd_direct.hip (64 features: against one team), inputs from memory: 1 x 1021 x 16 heads of 192 25.9 -> 24.0 us, its
+// ring share of 3 chunks 60.0 -> 47.7, 1 x 4096 x 4 of 192 70 -> 62, 1 x 2048 x 8 of 128 30.5 -> 26.4, 1 x 8192 x 4 of 64
+// 98 -> 70 (4 parts); 1 x 4096 x 16 of 64 57 -> 53, 1 x 4096 x 8 of 64 52 -> 43 (2 parts, 64 features only). More at
+// pick_split.
 //
 // LDS: rings of two K and two V tiles; interval i reads V(i) and K(i+1) while V(i+1) and K(i+2) land in the slots that
 // interval i-1 released.
@@ -450,8 +451,8 @@ void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
 template <int DQK, bool MULTI>
 void launch_parts(const FwdArgs<MULTI>& p, int parts, bool causal, hipStream_t st) {
   if (parts == 1) launch_one<DQK, 1, MULTI>(p, causal, st);
-  else if (parts == 2) launch_one<DQK, 2, MULTI>(p, causal, st);
-  else launch_one<DQK, 4, MULTI>(p, causal, st);
+  else if (parts == 4) launch_one<DQK, 4, MULTI>(p, causal, st);
+  else if constexpr (DQK == 64) launch_one<DQK, 2, MULTI>(p, causal, st);
 }
 
 template <bool MULTI>

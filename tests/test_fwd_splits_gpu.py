@@ -49,12 +49,12 @@ def test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     # 64-row workgroups: stream of 256 / 257 and 320 / 321 keys, one tile for one team only, rows that see one key block
     (1, 256, 256, 4, 2, 64, True), (1, 257, 257, 4, 2, 64, True), (1, 320, 320, 2, 2, 128, False), (1, 1, 321, 2, 1, 128, False),
     (1, 33, 1025, 4, 4, 192, False), (2, 449, 449, 2, 1, 192, True), (1, 95, 350, 2, 2, 64, False), (1, 700, 700, 4, 1, 128, True),
-    # 256 / 257 and 512 / 513 of them; a heavy and a light one per compute unit from 2048 (64 features) and 4096 keys on
-    (1, 512, 512, 32, 4, 128, True), (1, 2047, 2047, 16, 4, 64, True), (1, 2048, 2048, 16, 4, 64, True), (1, 4095, 4095, 8, 2, 128, True),
-    (1, 4096, 4096, 8, 8, 192, True), (1, 2112, 2112, 16, 4, 64, True),
-    # 128-row workgroups of two teams: 1024 / 1025 keys, 1535 / 1536 under the mask, ragged, one and two per compute unit
-    (1, 900, 1025, 32, 8, 64, False), (1, 1536, 1536, 42, 2, 64, True), (1, 1535, 1535, 42, 2, 64, True), (1, 4096, 4096, 16, 2, 64, True),
-    (1, 3001, 3001, 21, 3, 192, True), (1, 1100, 1100, 28, 28, 192, True),
+    # 256 / 257 of them; under the mask 384 / 385 from 2048 keys and 512 / 513 from 6144 keys on
+    (1, 512, 512, 32, 4, 128, True), (1, 2047, 2047, 12, 4, 128, True), (1, 2048, 2048, 12, 4, 128, True), (1, 2049, 2049, 12, 4, 192, True),
+    (1, 6143, 6143, 5, 1, 128, True), (1, 6144, 6144, 5, 5, 192, True),
+    # 128-row workgroups of two teams: 1024 / 1025 keys, 2048 / 2049 under the mask, ragged, one and two per compute unit
+    (1, 900, 1025, 32, 8, 64, False), (1, 900, 1024, 32, 8, 64, False), (1, 2048, 2048, 32, 4, 64, True), (1, 2049, 2049, 30, 3, 64, True),
+    (1, 4096, 4096, 16, 2, 64, True), (1, 2111, 2111, 11, 11, 64, True),
 ])  # fmt: skip
 def test_forward_key_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
