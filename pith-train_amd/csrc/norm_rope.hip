@@ -348,10 +348,15 @@ Plan make_plan(int64_t B, int64_t S, int64_t H, int64_t D) {
   return pl;
 }
 
-constexpr int kMaxBwdBlocksX = 1024;
+// Backward: at most three blocks of a tensor per compute unit. Five fit (90 registers), and the two tensors of a pair share
+// them; with up to 1024 blocks for either the pair left a second round of a few blocks. Alone, too, three do better than
+// four: the fewer rows in flight stream closer together. With 1024 and 768 blocks on 256 compute units, both kernels, inputs
+// from memory: 8192 x 32/4 heads of 128 50.6 -> 49.3 us (q alone 47.1 -> 45.0), 16384 x 64/4 175 -> 165, 4096 x 32/4 30.4 ->
+// 28.8, 16384 x 8/2 32.6 -> 30.9; 512 and 640 are slower.
+constexpr int kBwdBlocksPerUnit = 3;
 
 int bwd_blocks_x(const Plan& pl, int64_t B) {
-  int64_t cap = kMaxBwdBlocksX / B;
+  int64_t cap = kBwdBlocksPerUnit * (int64_t)compute_units_or_default() / B;
   if (cap < 1) cap = 1;
   return (int)(pl.n_tiles < cap ? pl.n_tiles : cap);
 }
