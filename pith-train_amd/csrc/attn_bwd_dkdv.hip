@@ -235,15 +235,29 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
 
 // Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
 // split-key ones (the two kernels must agree on the workgroup size), which is what grids of up to one workgroup per compute
-// unit want anyway. With two per unit a chunk pair gains nothing (1 x 4096 x 16 heads of 192 features: 293 us apart, 298 us
-// together), several chunks, whose dK/dV workgroups are more unequal, 1-5 % (2048 x 32/4 of 128, 4 ranks, zigzag, rank 0:
-// 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081); with three it loses (6144 x 16 of 192: 2385 -> 2413). At 64
-// features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only grids of a
-// few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us, 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16 474 -> 483 us).
+// unit want anyway. Beyond, one grid pays where either kernel alone would leave its last round half empty, against what the
+// two-workgroup dQ kernel is faster by; W = dQ workgroups per compute unit, apart -> together, inputs from memory, us:
+//   d128 causal   W 1.5: 1 x 2304 x 16 108 -> 91, 1 x 6144 x 8/2 289 -> 265, 6 x 512 x 16/4 68 -> 61; 1.75: 1 x 1792 x 32/4
+//                 122 -> 121; 2: 1 x 2048 x 32/4 154 -> 150, 1 x 8192 x 8/2 446 -> 449; 2.25-2.5: 1 x 2304 x 32/4 191 -> 181,
+//                 1 x 5120 x 16 377 -> 351, 5 x 1024 x 16/4 127 -> 127
+//        full     W 1.5: 1 x 1536 x 32/4 157 -> 145; 1.7: 1 x 3456 x 16 307 -> 329; 2: 1 x 4096 x 16 412 -> 422;
+//                 2.2: 1 x 4480 x 16 628 -> 520, 1 x 2304 x 32/4 383 -> 289
+//   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186, 3 x 1024 x 16 92 -> 94; 1.7: 1 x 3456 x 16
+//                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
+// Several chunks, whose dK/dV workgroups are more unequal, gain 1-5 % up to two per unit (2048 x 32/4 of 128, 4 ranks,
+// zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081); with three they lose (6144 x 16 of 192: 2385 ->
+// 2413). At 64 features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only
+// grids of a few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us, 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16
+// 474 -> 483 us).
 bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
   if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
+  const int64_t cus = compute_units_or_default();
   const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
-  return q_wgs <= (a->Dqk == 64 ? 4 : chunks ? 2 : 1) * (int64_t)compute_units_or_default();
+  if (a->Dqk == 64) return q_wgs <= 4 * cus;
+  if (chunks) return q_wgs <= 2 * cus;
+  if (q_wgs <= cus) return true;
+  if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;
+  return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));
 }
 
 }  // namespace

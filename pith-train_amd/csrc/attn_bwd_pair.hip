@@ -4,7 +4,7 @@
 // compute units), on grids of a few rounds the tails do. Here a workgroup takes its role from its block id, the dK/dV
 // workgroups first (they carry a third more work), the dQ ones behind them fill every unit that falls free.
 // Measured, dK/dV + dQ, separate launches against one: 1 x 1021 x 16 heads of 192 causal 71 -> 42 us, 1 x 2048 x 16 of 192
-// 122 -> 84 us, 2 x 2048 x 16/4 of 64 114 -> 79 us, 1 x 4096 x 16 of 192 290 -> 280 us.
+// 122 -> 84 us, 2 x 2048 x 16/4 of 64 114 -> 79 us, 1 x 2304 x 32/4 of 128, no mask 383 -> 289 us. Which launches: one_grid.
 #include "attn_bwd_common.h"
 #include "attn_bwd_dkdv_d128.h"
 #include "attn_bwd_dkdv_d192.h"

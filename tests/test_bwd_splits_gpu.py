@@ -58,3 +58,13 @@ def test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     attn_bwd_pair_into(q, k, v, dout, lse, delta, *pair, scale, causal)
     for name, got, want in zip(("dQ", "dK", "dV"), pair, refs):
         check_bf16_result(got, want, name + " of the pair", otol=1e-3)
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D,causal", [
+    # both sides of 1.5 and of 2.5 workgroups per compute unit, above 2 of them, streams of 1023 / 1024 and 1535 / 1536 keys
+    (1, 1536, 1536, 32, 4, 128, False), (1, 1537, 1537, 32, 4, 128, False), (1, 2177, 2177, 30, 2, 128, False), (1, 2100, 700, 32, 4, 128, False),
+    (1, 2560, 2560, 32, 4, 128, True), (1, 2561, 2561, 32, 4, 128, True), (1, 1024, 1024, 64, 8, 128, True), (1, 1023, 1023, 64, 8, 128, True),
+    (1, 1536, 1536, 32, 32, 192, True), (1, 1535, 1535, 32, 32, 192, True), (1, 1500, 1600, 32, 32, 192, False),
+])  # fmt: skip
+def test_backward_pairs_of_a_few_rounds(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+    test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
