@@ -612,7 +612,8 @@ Three mla_assemble_bwd(const Tensor& dqo, const Tensor& dko, const Tensor& dvo, 
 
 // ---------------------------------------------------------------------------------------------
 // Autograd. Each formula calls the ops through the dispatcher, below autograd, so that fake tensors, functionalisation and
-// torch.compile see ordinary ops.
+// torch.compile see ordinary ops. A result carries a node whenever any floating-point input requires grad, the rotary tables
+// too: they receive no gradient, but a program whose tables alone require grad may still call backward().
 
 template <typename Sig>
 auto op_handle(const char* name) { return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>(); }
@@ -679,7 +680,7 @@ struct NormRopeFunction : torch::autograd::Function<NormRopeFunction> {
 };
 Tensor norm_rope_fwd_autograd(const Tensor& x, const OptTensor& w, const Tensor& cos, const Tensor& sin, double eps) {
   const Tensor ww = or_undefined(w);
-  if (any_requires_grad({&x, &ww})) return NormRopeFunction::apply(x, w, cos, sin, eps);
+  if (any_requires_grad({&x, &ww, &cos, &sin})) return NormRopeFunction::apply(x, w, cos, sin, eps);
   at::AutoDispatchBelowADInplaceOrView guard;
   return call_norm_rope_fwd(x, w, cos, sin, eps);
 }
@@ -706,7 +707,7 @@ struct QkNormRopeFunction : torch::autograd::Function<QkNormRopeFunction> {
 };
 Two qk_norm_rope_fwd_autograd(const Tensor& q, const Tensor& k, const OptTensor& qw, const OptTensor& kw, const Tensor& cos, const Tensor& sin, double eps) {
   const Tensor a = or_undefined(qw), b = or_undefined(kw);
-  if (any_requires_grad({&q, &k, &a, &b})) {
+  if (any_requires_grad({&q, &k, &a, &b, &cos, &sin})) {
     auto r = QkNormRopeFunction::apply(q, k, qw, kw, cos, sin, eps);
     return {r[0], r[1]};
   }
@@ -735,7 +736,7 @@ struct MlaAssembleFunction : torch::autograd::Function<MlaAssembleFunction> {
   }
 };
 Three mla_assemble_fwd_autograd(const Tensor& q, const Tensor& kv, const Tensor& k_pe, const Tensor& cos, const Tensor& sin, const OptTensor& pos) {
-  if (any_requires_grad({&q, &kv, &k_pe})) {
+  if (any_requires_grad({&q, &kv, &k_pe, &cos, &sin})) {
     auto r = MlaAssembleFunction::apply(q, kv, k_pe, cos, sin, pos);
     return {r[0], r[1], r[2]};
   }
