@@ -837,15 +837,17 @@ TORCH_LIBRARY_IMPL(pithtrain_amd, Autograd, m) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_bodies", [](py::dict d) { bodies().attr("update")(d); }, "Registers the Python bodies of ops (name -> function).");
-  m.def("attn_fwd_into", &attn_fwd_into);
-  m.def("attn_bwd_delta_into", &attn_bwd_delta_into);
-  m.def("attn_bwd_dkdv_into", &attn_bwd_dkdv_into);
-  m.def("attn_bwd_dq_into", &attn_bwd_dq_into);
-  m.def("attn_bwd_pair_into", &attn_bwd_pair_into);
-  m.def("ring_forward", &ring_forward);
-  m.def("ring_backward", &ring_backward);
-  m.def("combine_into", &combine_into);
-  m.def("combine_new", &combine_new);
-  m.def("cast_f32_bf16_into", &cast_f32_bf16_into);
+  // These allocate and launch, either of which can block (a full queue): other Python threads run meanwhile.
+  using Unlocked = py::call_guard<py::gil_scoped_release>;
+  m.def("attn_fwd_into", &attn_fwd_into, Unlocked());
+  m.def("attn_bwd_delta_into", &attn_bwd_delta_into, Unlocked());
+  m.def("attn_bwd_dkdv_into", &attn_bwd_dkdv_into, Unlocked());
+  m.def("attn_bwd_dq_into", &attn_bwd_dq_into, Unlocked());
+  m.def("attn_bwd_pair_into", &attn_bwd_pair_into, Unlocked());
+  m.def("ring_forward", &ring_forward, Unlocked());
+  m.def("ring_backward", &ring_backward, Unlocked());
+  m.def("combine_into", &combine_into, Unlocked());
+  m.def("combine_new", &combine_new, Unlocked());
+  m.def("cast_f32_bf16_into", &cast_f32_bf16_into, Unlocked());
   m.def("ds_handover_pays", &ds_handover_pays);
 }

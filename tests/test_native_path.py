@@ -1,8 +1,12 @@
 """The operators' native host path on a machine without a GPU."""
 
+import sys
+import threading
+
 import pytest
 import torch
 
+from pithtrain_amd._ext import native
 from pithtrain_amd.operators.mla_assemble import mla_assemble_qkv
 from pithtrain_amd.operators.norm_rope import norm_rope, qk_norm_rope
 
@@ -31,3 +35,45 @@ def test_rotary_tables_that_require_grad(name, which):
     assert outs and all(o.requires_grad for o in outs)
     torch.autograd.backward(outs, [torch.empty_like(o) for o in outs])
     assert tables[which].grad is None
+
+
+def _declined_calls():
+    """One call of every bound function that may launch kernels, on CPU tensors: declined without touching a device."""
+    q, d = torch.empty(1, 2, 2, 128, dtype=torch.bfloat16), torch.empty(1, 2, 2)
+    f = torch.empty(1, 2, 2, 128)
+    n = native
+    return {
+        "attn_fwd_into": lambda: n.attn_fwd_into(q, q, q, q, d, 0.1, True, None, None, None, None, None),
+        "attn_bwd_delta_into": lambda: n.attn_bwd_delta_into(q, q, d),
+        "attn_bwd_dkdv_into": lambda: n.attn_bwd_dkdv_into(q, q, q, q, d, d, q, q, 0.1, True, False, None, None, None, 0),
+        "attn_bwd_dq_into": lambda: n.attn_bwd_dq_into(q, q, q, q, d, d, q, 0.1, True, False, None, None, None, None),
+        "attn_bwd_pair_into": lambda: n.attn_bwd_pair_into(q, q, q, q, d, d, q, q, q, 0.1, True, False, False, None, None, None, 0, None, None),
+        "ring_forward": lambda: n.ring_forward(q, [q, q], [q, q], None, 0.1, 0, 2, True),
+        "ring_backward": lambda: n.ring_backward(q, q, q, d, [q, q], [q, q], None, 0.1, 0, 2, True),
+        "combine_into": lambda: n.combine_into(q, d, q, d, f, d, 0),
+        "combine_new": lambda: n.combine_new(q, d, q, d, 0),
+        "cast_f32_bf16_into": lambda: n.cast_f32_bf16_into(f, q),
+    }
+
+
+@pytest.mark.parametrize("name", _declined_calls())
+def test_bound_functions_release_the_interpreter_lock(name):
+    """A launch can block on a full queue; other Python threads must be able to run meanwhile. The interpreter is told not to
+    take the lock away by itself, so the other thread gets it only from a call that gives it up."""
+    call = _declined_calls()[name]
+    go, ran = threading.Event(), threading.Event()
+    other = threading.Thread(target=lambda: (go.wait(), ran.set()), daemon=True)
+    other.start()
+    before = sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(1000.0)
+        go.set()
+        for _ in range(200000):
+            assert not call()
+            if ran.is_set():
+                break
+        else:
+            raise AssertionError(f"{name} keeps the interpreter lock")
+    finally:
+        sys.setswitchinterval(before)
+        other.join()
