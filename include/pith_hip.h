@@ -49,8 +49,11 @@ enum {
 enum { PITH_BF16 = 0, PITH_F32 = 1 };
 enum { PITH_BASE_2 = 0, PITH_BASE_E = 1 };
 
-/* Library version: major*10000 + minor*100 + patch. */
-int pith_version(void);
+/* Version of this interface: major*10000 + minor*100 + patch. The minor number goes up whenever a struct or a signature below
+ * changes; a program built against another one must not call into the library (its structs have other sizes).
+ * 200: pith_norm_rope_args gained dweight_bf16, and dweight became void*; chunk calls and pith_attn_bwd added. */
+#define PITH_VERSION 200
+int pith_version(void); /* PITH_VERSION of the library that was loaded */
 /* Text of the last error raised on the calling thread ("" if none). Never NULL. */
 const char* pith_last_error(void);
 /* Symbolic name of an error code ("PITH_OK", "PITH_ERR_BAD_SHAPE", ...). Never NULL. */

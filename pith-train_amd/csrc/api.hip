@@ -41,7 +41,7 @@ int check_launch(const char* what) {
 }
 }  // namespace pith
 
-extern "C" int pith_version(void) { return 100; /* 0.1.0 */ }
+extern "C" int pith_version(void) { return PITH_VERSION; }
 
 extern "C" const char* pith_last_error(void) { return pith::g_last_error; }
 

@@ -836,6 +836,8 @@ TORCH_LIBRARY_IMPL(pithtrain_amd, Autograd, m) {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  TORCH_CHECK(pith_version() == PITH_VERSION, "_pith_torch.so was built for interface version ", PITH_VERSION, " of libpith_hip.so, found ",
+              pith_version(), ": build both again");
   m.def("set_bodies", [](py::dict d) { bodies().attr("update")(d); }, "Registers the Python bodies of ops (name -> function).");
   // These allocate and launch, either of which can block (a full queue): other Python threads run meanwhile.
   using Unlocked = py::call_guard<py::gil_scoped_release>;

@@ -13,6 +13,8 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libpith_hip.so")
 
+PITH_VERSION = 200  # of include/pith_hip.h, whose structs are declared below
+
 PITH_BF16, PITH_F32 = 0, 1
 PITH_BASE_2, PITH_BASE_E = 0, 1
 
@@ -170,6 +172,8 @@ def lib() -> ctypes.CDLL:
             fn = getattr(handle, name)
             fn.restype = restype
             fn.argtypes = argtypes
+        if handle.pith_version() != PITH_VERSION:
+            raise ImportError(f"{LIB_PATH} has interface version {handle.pith_version()}, this package needs {PITH_VERSION}: build it again")
         _lib = handle
     return _lib
 

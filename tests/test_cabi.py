@@ -61,6 +61,26 @@ def test_struct_layouts_match_the_header(tmp_path):
             assert int(got[f"{cname}.{fname}"]) == getattr(st, fname).offset, f"{cname}.{fname}"
 
 
+# Struct sizes of a version of the interface: a change here needs a new version (programs built against the old header pass
+# structs of the old size).
+STRUCT_SIZES = {
+    200: {"pith_combine_args": 168, "pith_attn_fwd_args": 248, "pith_attn_delta_args": 88, "pith_attn_bwd_args": 352,
+          "pith_norm_rope_args": 152, "pith_mla_assemble_args": 192, "pith_key_chunk": 72, "pith_device_info_t": 88},
+}  # fmt: skip
+
+
+def test_version_goes_with_the_struct_sizes(tmp_path):
+    src = tmp_path / "sizes.c"
+    names = list(STRUCT_SIZES[_C.PITH_VERSION])
+    src.write_text('#include <stdio.h>\n#include "pith_hip.h"\nint main(void){printf("%d", PITH_VERSION);'
+                   + "".join(f'printf(" %zu", sizeof({n}));' for n in names) + "return 0;}")  # fmt: skip
+    exe = tmp_path / "sizes"
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
+    version, *sizes = map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
+    assert version == _C.PITH_VERSION == _C.lib().pith_version()
+    assert dict(zip(names, sizes)) == STRUCT_SIZES[version]
+
+
 def test_device_info_without_a_device():
     lib = _C.lib()
     assert lib.pith_device_info(0, None) == _C.PITH_ERR_NULL_POINTER
