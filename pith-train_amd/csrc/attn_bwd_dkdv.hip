@@ -267,8 +267,12 @@ extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t str
 }
 
 extern "C" int pith_attn_bwd(const pith_attn_bwd_args* a, pith_stream_t stream) {
-  if (const int rc = validate_bwd(a, "pith_attn_bwd", true, true)) return rc;
-  if (one_grid(a, false)) return bwd_dkdv(a, stream, "pith_attn_bwd", true);
+  const char* who = "pith_attn_bwd";
+  if (const int rc = validate_bwd(a, who, true, true)) return rc;
+  if (one_grid(a, false)) return bwd_dkdv(a, stream, who, true);
+  // what the second call would reject is rejected before the first has written (or added to) anything
+  BwdParams dq;
+  if (const int rc = prepare_dq(a, &dq, who)) return rc;
   if (const int rc = pith_attn_bwd_dkdv(a, stream)) return rc;
   return pith_attn_bwd_dq(a, stream);
 }

@@ -6,8 +6,9 @@
 // therefore works on at::Tensor directly, allocates from torch's caching allocator and enqueues on the current stream.
 //
 // Two layers share each operator. The native one serves the calls of ordinary layout (GPU tensors, the expected dtypes,
-// contiguous per batch element). Whenever a condition fails, or the library rejects the arguments, it has done nothing yet
-// and hands over to the operator's Python body, which accepts every layout (copying where needed) and words the errors.
+// contiguous per batch element). Whenever a condition fails, or the library rejects the arguments, it has launched nothing yet
+// and hands over to the operator's Python body, which accepts every layout (copying where needed) and words the errors. A
+// launch that fails is raised as it is (see accepted()).
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 #include <torch/library.h>
@@ -36,6 +37,13 @@ template <typename R, typename... Args>
 R python_body(const char* name, const Args&... args) {
   py::gil_scoped_acquire gil;
   return bodies()[name](args...).template cast<R>();
+}
+
+// Whether the library took a call. One that it rejected has launched nothing, so the Python body may run it again. After a
+// failed launch that is not so: kernels of the call may be out, and accumulating ones must not run twice. Raises PithError.
+bool accepted(int rc) {
+  if (rc == PITH_ERR_LAUNCH) python_body<bool>("check", rc);
+  return rc == PITH_OK;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -150,7 +158,7 @@ bool attn_fwd_into(const Tensor& q, const Tensor& k, const Tensor& v, const OptT
   a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.lse = lse.data_ptr<float>();
   a.B = b; a.Sq = sq; a.Skv = k.size(1); a.Hq = hq; a.Hkv = k.size(2); a.Dqk = q.size(3); a.Dv = dv;
   a.scale = (float)scale; a.causal = causal;
-  return pith_attn_fwd(&a, stream_of(q)) == PITH_OK;
+  return accepted(pith_attn_fwd(&a, stream_of(q)));
 }
 
 bool attn_bwd_delta_into(const Tensor& out, const Tensor& dout, const Tensor& delta) {
@@ -161,7 +169,7 @@ bool attn_bwd_delta_into(const Tensor& out, const Tensor& dout, const Tensor& de
       !bshd(out, &a.o_bs) || !bshd(dout, &a.dout_bs))
     return false;
   a.o = out.data_ptr(); a.dout = dout.data_ptr(); a.delta = delta.data_ptr<float>();
-  return pith_attn_bwd_delta(&a, stream_of(out)) == PITH_OK;
+  return accepted(pith_attn_bwd_delta(&a, stream_of(out)));
 }
 
 // What both backward calls of a chunk pair share.
@@ -243,7 +251,7 @@ bool attn_bwd_dkdv_into(const Tensor& q, const Tensor& k, const Tensor& v, const
   pith_attn_bwd_args a = {};
   Tensor workspace;
   return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) && dkdv_args(a, q, k, v, dk, dv, accumulate, k_pe, dk_pe, zero_tail, workspace) &&
-         pith_attn_bwd_dkdv(&a, stream_of(q)) == PITH_OK;
+         accepted(pith_attn_bwd_dkdv(&a, stream_of(q)));
 }
 
 bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dout, const Tensor& lse, const Tensor& delta, const Tensor& dq,
@@ -251,7 +259,7 @@ bool attn_bwd_dq_into(const Tensor& q, const Tensor& k, const Tensor& v, const T
                       const Rows& dq_final_rows) {
   pith_attn_bwd_args a = {};
   return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) && dq_args(a, q, dq, accumulate, dq_final, dq_final_rows) &&
-         pith_attn_bwd_dq(&a, stream_of(q)) == PITH_OK;
+         accepted(pith_attn_bwd_dq(&a, stream_of(q)));
 }
 
 // Both of them; `ds` is the hand-over buffer between the two, if any.
@@ -262,7 +270,7 @@ bool attn_bwd_pair_into(const Tensor& q, const Tensor& k, const Tensor& v, const
   Tensor workspace;
   return bwd_args(a, q, k, v, dout, lse, delta, scale, causal, k_pe, ds) &&
          dkdv_args(a, q, k, v, dk, dv, accumulate_dkv, k_pe, dk_pe, zero_tail, workspace) && dq_args(a, q, dq, accumulate_dq, dq_final, dq_final_rows) &&
-         pith_attn_bwd(&a, stream_of(q)) == PITH_OK;
+         accepted(pith_attn_bwd(&a, stream_of(q)));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -321,7 +329,7 @@ std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const st
   a.o = o.data_ptr(); a.lse = lse.data_ptr<float>();
   a.o_bs = a.Sq * a.Hq * a.Dv;
   a.scale = (float)scale;
-  if (pith_attn_fwd_chunks(&a, r.chunk.data(), (int64_t)r.chunk.size(), stream_of(q)) != PITH_OK) return std::nullopt;
+  if (!accepted(pith_attn_fwd_chunks(&a, r.chunk.data(), (int64_t)r.chunk.size(), stream_of(q)))) return std::nullopt;
   return std::make_tuple(o, lse);
 }
 
@@ -366,7 +374,7 @@ std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, c
     a.workspace = workspace.data_ptr();
     a.workspace_bytes = need;
   }
-  if (pith_attn_bwd_chunks(&a, r.chunk.data(), n, stream_of(q)) != PITH_OK) return std::nullopt;
+  if (!accepted(pith_attn_bwd_chunks(&a, r.chunk.data(), n, stream_of(q)))) return std::nullopt;
   return g;
 }
 
@@ -439,7 +447,7 @@ bool combine_into(const Tensor& out1, const Tensor& lse1, const Tensor& out2, co
   a.out1 = out1.data_ptr(); a.out2 = out2.data_ptr(); a.out = out.data_ptr();
   a.lse1 = lse1.data_ptr<float>(); a.lse2 = lse2.data_ptr<float>(); a.lse_out = lse_out.data_ptr<float>();
   a.base = (int32_t)base;
-  return pith_combine(&a, stream_of(out1)) == PITH_OK;
+  return accepted(pith_combine(&a, stream_of(out1)));
 }
 
 // The reference's calling convention: fresh fp32 outputs. None when the Python body has to take the call.
@@ -454,7 +462,7 @@ bool cast_f32_bf16_into(const Tensor& src, const Tensor& dst) {
   if (!src.is_cuda() || dst.device() != src.device() || src.scalar_type() != at::kFloat || dst.scalar_type() != at::kBFloat16 ||
       src.numel() != dst.numel() || !src.is_contiguous() || !dst.is_contiguous())
     return false;
-  return pith_cast_f32_bf16(src.data_ptr<float>(), dst.data_ptr(), src.numel(), stream_of(src)) == PITH_OK;
+  return accepted(pith_cast_f32_bf16(src.data_ptr<float>(), dst.data_ptr(), src.numel(), stream_of(src)));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -509,7 +517,7 @@ Tensor norm_rope_fwd(const Tensor& x, const OptTensor& weight, const Tensor& cos
   if (x.is_cuda()) {
     Tensor out = at::empty_like(x, at::MemoryFormat::Contiguous);
     pith_norm_rope_args a = {};
-    if (norm_rope_args(a, x, weight, cos, sin, out, eps) && pith_norm_rope_fwd(&a, stream_of(x)) == PITH_OK) return out;
+    if (norm_rope_args(a, x, weight, cos, sin, out, eps) && accepted(pith_norm_rope_fwd(&a, stream_of(x)))) return out;
   }
   return python_body<Tensor>("norm_rope_fwd", x, weight, cos, sin, eps);
 }
@@ -519,7 +527,7 @@ Two norm_rope_bwd(const Tensor& x, const OptTensor& weight, const Tensor& cos, c
     Tensor dx = at::empty_like(x, at::MemoryFormat::Contiguous), dw = dweight_for(x, weight), ws;
     pith_norm_rope_args a = {};
     if (norm_rope_args(a, x, weight, cos, sin, dx, eps) && norm_rope_bwd_args(a, x, weight, dout, dw, ws) &&
-        pith_norm_rope_bwd(&a, stream_of(x)) == PITH_OK)
+        accepted(pith_norm_rope_bwd(&a, stream_of(x))))
       return {dx, dw};
   }
   return python_body<Two>("norm_rope_bwd", x, weight, cos, sin, dout, eps);
@@ -530,7 +538,7 @@ Two qk_norm_rope_fwd(const Tensor& q, const Tensor& k, const OptTensor& qw, cons
     Tensor qo = at::empty_like(q, at::MemoryFormat::Contiguous), ko = at::empty_like(k, at::MemoryFormat::Contiguous);
     pith_norm_rope_args a = {}, b = {};
     if (k.device() == q.device() && norm_rope_args(a, q, qw, cos, sin, qo, eps) && norm_rope_args(b, k, kw, cos, sin, ko, eps) &&
-        pith_norm_rope_fwd_pair(&a, &b, stream_of(q)) == PITH_OK)
+        accepted(pith_norm_rope_fwd_pair(&a, &b, stream_of(q))))
       return {qo, ko};
   }
   return python_body<Two>("qk_norm_rope_fwd", q, k, qw, kw, cos, sin, eps);
@@ -544,7 +552,7 @@ Four qk_norm_rope_bwd(const Tensor& q, const Tensor& k, const OptTensor& qw, con
     pith_norm_rope_args a = {}, b = {};
     if (k.device() == q.device() && norm_rope_args(a, q, qw, cos, sin, dq, eps) && norm_rope_args(b, k, kw, cos, sin, dk, eps) &&
         norm_rope_bwd_args(a, q, qw, dqo, dwq, ws_q) && norm_rope_bwd_args(b, k, kw, dko, dwk, ws_k) &&
-        pith_norm_rope_bwd_pair(&a, &b, stream_of(q)) == PITH_OK)
+        accepted(pith_norm_rope_bwd_pair(&a, &b, stream_of(q))))
       return {dq, dk, dwq, dwk};
   }
   return python_body<Four>("qk_norm_rope_bwd", q, k, qw, kw, cos, sin, dqo, dko, eps);
@@ -586,7 +594,7 @@ Three mla_assemble_fwd(const Tensor& q, const Tensor& kv, const Tensor& k_pe, co
       a.kv_bs = a.S * a.H * (a.Dn + a.Dv);
       a.k_pe_rs = a.S > 1 ? k_pe.stride(1) : a.Dr;
       a.k_pe_bs = a.B > 1 ? k_pe.stride(0) : a.S * k_pe.stride(1);
-      if (pith_mla_assemble_fwd(&a, stream_of(q)) == PITH_OK) return {qo, ko, vo};
+      if (accepted(pith_mla_assemble_fwd(&a, stream_of(q)))) return {qo, ko, vo};
     }
   }
   return python_body<Three>("mla_assemble_fwd", q, kv, k_pe, cos, sin, pos);
@@ -604,7 +612,7 @@ Three mla_assemble_bwd(const Tensor& dqo, const Tensor& dko, const Tensor& dvo, 
       Tensor dpe = k_pe_heads ? at::empty({a.B, a.S, 1, a.Dr}, dqo.options()) : at::empty({a.B, a.S, a.Dr}, dqo.options());
       a.dq_out = dqo.data_ptr(); a.dk_out = dko.data_ptr(); a.dv_out = dvo.data_ptr();
       a.q_out = dq.data_ptr(); a.k_out = dkv.data_ptr(); a.v_out = dpe.data_ptr();
-      if (pith_mla_assemble_bwd(&a, stream_of(dqo)) == PITH_OK) return {dq, dkv, dpe};
+      if (accepted(pith_mla_assemble_bwd(&a, stream_of(dqo)))) return {dq, dkv, dpe};
     }
   }
   return python_body<Three>("mla_assemble_bwd", dqo, dko, dvo, cos, sin, pos, k_pe_heads);
@@ -851,5 +859,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("combine_into", &combine_into, Unlocked());
   m.def("combine_new", &combine_new, Unlocked());
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into, Unlocked());
+  m.def("accepted", &accepted);
   m.def("ds_handover_pays", &ds_handover_pays);
 }

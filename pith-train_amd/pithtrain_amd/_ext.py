@@ -3,12 +3,15 @@
 not been built, importing the operators raises.
 
 Every native function returns False (None) when a call is not of ordinary layout or the library rejected it; nothing has
-been launched then, and the caller runs the operator's Python body, which takes every layout and words the errors."""
+been launched then, and the caller runs the operator's Python body, which takes every layout and words the errors. A launch
+that failed raises PithError at once."""
 
 import importlib.util
 import os
 
 import torch  # noqa: F401  (libtorch and the HIP runtime must be in the process first)
+
+from pithtrain_amd import _C
 
 EXT_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_pith_torch.so")
 
@@ -25,6 +28,7 @@ def _load():
 
 
 native = _load()
+native.set_bodies({"check": _C.check})
 
 
 def define_op(name: str, body, fake):

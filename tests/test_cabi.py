@@ -379,3 +379,20 @@ def test_ds_storing_dkdv_kernel_waits_for_its_tile_loads_only(tmp_path_factory):
             elif cur and re.match(r"\s+(global_store|scratch_)", l):
                 in_loop_blocks.append(l.strip())
         assert not in_loop_blocks, f"stores or spills in out-of-line blocks of the loop: {in_loop_blocks}"
+
+
+def test_attn_bwd_rejects_before_its_first_launch():
+    """As two launches (dK/dV, then dQ) the call must find bad arguments of the second before the first goes out. There is no
+    device here, so a launch would show as PITH_ERR_LAUNCH."""
+    n, h = 4096, 16
+    base = dict(q=16, k=16, v=16, dout=16, lse=16, delta=16, dq=16, dk=16, dv=16, B=1, Sq=n, Skv=n, Hq=h, Hkv=h, Dqk=192, Dv=128,
+                q_bs=n * h * 192, k_bs=n * h * 192, v_bs=n * h * 128, dout_bs=n * h * 128, dq_bs=n * h * 192, dk_bs=n * h * 192,
+                dv_bs=n * h * 128, lse_bs=h * n, lse_hs=n, scale=0.07, causal=1, dq_dtype=_C.PITH_F32, dkv_dtype=_C.PITH_BF16,
+                accumulate_dkv=1, dq_final=16, dq_final_bs=n * h * 192)  # fmt: skip
+    for bad, code in (
+        (dict(dq_final_rows=(ctypes.c_int64 * 2)(8, 40)), _C.PITH_ERR_BAD_SHAPE),
+        (dict(dq_final=8), _C.PITH_ERR_MISALIGNED),
+        (dict(dq_dtype=_C.PITH_BF16), _C.PITH_ERR_UNSUPPORTED),
+        (dict(ds=16, ds_bytes=1 << 40, Dqk=128, dq_final_rows=(ctypes.c_int64 * 2)(8, 40)), _C.PITH_ERR_BAD_SHAPE),
+    ):
+        assert _C.lib().pith_attn_bwd(ctypes.byref(_C.AttnBwdArgs(**{**base, **bad})), None) == code, bad

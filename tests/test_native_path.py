@@ -6,6 +6,7 @@ import threading
 import pytest
 import torch
 
+from pithtrain_amd import _C
 from pithtrain_amd._ext import native
 from pithtrain_amd.operators.mla_assemble import mla_assemble_qkv
 from pithtrain_amd.operators.norm_rope import norm_rope, qk_norm_rope
@@ -35,6 +36,14 @@ def test_rotary_tables_that_require_grad(name, which):
     assert outs and all(o.requires_grad for o in outs)
     torch.autograd.backward(outs, [torch.empty_like(o) for o in outs])
     assert tables[which].grad is None
+
+
+def test_failed_launch_is_not_tried_again():
+    """What the library rejects goes to the Python body; a failed launch, whose call may have written something, raises."""
+    assert native.accepted(_C.PITH_OK) and not native.accepted(_C.PITH_ERR_BAD_SHAPE)
+    with pytest.raises(_C.PithError) as e:
+        native.accepted(_C.PITH_ERR_LAUNCH)
+    assert e.value.code == _C.PITH_ERR_LAUNCH
 
 
 def _declined_calls():
