@@ -47,12 +47,6 @@ __global__ __launch_bounds__(dq_duo::kThreads, 2) void attn_bwd_dq_duo_chunks_ke
 }
 
 template <int DQK>
-__global__ __launch_bounds__(dq_direct::kThreads) void attn_bwd_dq_direct_chunks_kernel(BwdChunkParams p) {
-  __shared__ __attribute__((aligned(1024))) char smem[dq_direct::kSmem<DQK>];
-  dq_direct::body<DQK, true, __bf16, true>(p, smem, blockIdx.x);
-}
-
-template <int DQK>
 __global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_pair_chunks_kernel(BwdChunkParams p, int dkdv_blocks, int dq_first) {
   const int dq_blocks = gridDim.x - dkdv_blocks;
   const int block = dq_first ? ((int)blockIdx.x < dq_blocks ? dkdv_blocks + blockIdx.x : blockIdx.x - dq_blocks) : blockIdx.x;
@@ -68,28 +62,22 @@ __global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_pair_chunks_ker
 }
 
 template <int DQK>
-void launch_dim(const BwdChunkParams& p, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
+void launch_dim(const BwdChunkParams& p, bool one_grid, bool dq_first, unsigned dkdv_blocks, hipStream_t st) {
   const unsigned dq_blocks = (unsigned)(p.q_tiles * p.Hq * p.B);
   if (one_grid) {
     hipLaunchKernelGGL((attn_bwd_pair_chunks_kernel<DQK>), dim3(dkdv_blocks + dq_blocks), dim3(kDkdvThreads<DQK>), 0, st, p, (int)dkdv_blocks, (int)dq_first);
     return;
   }
   hipLaunchKernelGGL((attn_bwd_dkdv_chunks_kernel<DQK>), dim3(dkdv_blocks), dim3(kDkdvThreads<DQK>), 0, st, p);
-  if constexpr (DQK != 64) {
-    if (split_keys) {
-      hipLaunchKernelGGL((attn_bwd_dq_direct_chunks_kernel<DQK>), dim3(dq_blocks), dim3(dq_direct::kThreads), 0, st, p);
-      return;
-    }
-  }
   hipLaunchKernelGGL((attn_bwd_dq_duo_chunks_kernel<DQK>), dim3(dq_blocks), dim3(dq_duo::kThreads), 0, st, p);
 }
 
 }  // namespace
 
-void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t st) {
-  if (dqk == 64) launch_dim<64>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
-  else if (dqk == 128) launch_dim<128>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
-  else launch_dim<192>(p, one_grid, dq_first, split_keys, dkdv_blocks, st);
+void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, unsigned dkdv_blocks, hipStream_t st) {
+  if (dqk == 64) launch_dim<64>(p, one_grid, dq_first, dkdv_blocks, st);
+  else if (dqk == 128) launch_dim<128>(p, one_grid, dq_first, dkdv_blocks, st);
+  else launch_dim<192>(p, one_grid, dq_first, dkdv_blocks, st);
 }
 
 }  // namespace pith

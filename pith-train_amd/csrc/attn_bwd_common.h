@@ -253,9 +253,9 @@ void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned gr
 // dQ workgroups. False: no such kernel for these output types.
 bool launch_bwd_pair(const BwdParams& p, int dqk, bool causal, bool dkdv_f32, bool dq_f32, unsigned dkdv_blocks, hipStream_t stream);
 
-// The backward of a chunk call: attn_bwd_chunks.hip. dkdv_blocks = the dK/dV grid; p.q_tiles = 128-row query tiles; split_keys
-// as for launch_dq_direct / launch_dq_duo (one_grid implies it at 128 and 192 features); dq_first: one grid starts with dQ.
-void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, bool split_keys, unsigned dkdv_blocks, hipStream_t stream);
+// The backward of a chunk call: attn_bwd_chunks.hip. dkdv_blocks = the dK/dV grid; p.q_tiles = 128-row query tiles; dq_first:
+// one grid starts with dQ. dQ workgroups: the split-key ones in one grid (128 and 192 features), the two-per-unit ones alone.
+void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, unsigned dkdv_blocks, hipStream_t stream);
 
 // dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
 // split every tile's keys: attn_bwd_dq_direct.hip.
@@ -270,8 +270,7 @@ void launch_dq_from_ds(const BwdParams& p, bool causal, bool f32_out, hipStream_
 // Bytes of dS images for a shape (0: the shape has no hand-over path), and whether the call brings a buffer for them.
 int64_t ds_bytes_for(const pith_attn_bwd_args* a);
 bool ds_usable(const pith_attn_bwd_args* a);
-// Whether a recomputing dQ call uses the split-key workgroups, and its share of the parameters (attn_bwd_dq.hip).
-bool dq_split_keys(const pith_attn_bwd_args* a);
+// What a dQ call adds to the parameters, checked (attn_bwd_dq.hip).
 int prepare_dq(const pith_attn_bwd_args* a, BwdParams* p, const char* who);
 
 // Argument checks common to both entry points; returns PITH_OK or records the error.

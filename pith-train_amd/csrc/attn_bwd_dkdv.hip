@@ -396,7 +396,7 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   // any case (128 and 192 features): 2048 x 32/4 of 128, rank 0: 498 us, dQ first 518; 4096 x 16 of 192, rank 3: 1081 and 1084.
   const bool few = all.Dqk == 64 || ((all.Sq + 127) / 128) * all.Hq * all.B <= (int64_t)compute_units_or_default();
   const bool dq_first = few && 3 * all.Skv > 4 * all.Sq * (all.Hq / all.Hkv / split);
-  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, true), dq_first, dq_split_keys(&all), blocks, st);
+  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, true), dq_first, blocks, st);
   if (all.k_pe || split > 1) {  // (never both: keys in two parts have no head groups to split)
     Reduction<2 * kMaxChunks> r;
     for (int64_t i = 0; i < n; ++i) {

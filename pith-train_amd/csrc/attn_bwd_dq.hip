@@ -4,6 +4,8 @@
 #include "attn_bwd_common.h"
 
 namespace pith {
+namespace {
+
 // Recomputing dQ kernels: 128-row workgroups either way. Two 4-wave workgroups per compute unit (attn_bwd_dq_duo.hip), or
 // one of 8 waves whose pairs split every tile's keys (attn_bwd_dq_direct.hip, "half"). Measured, microseconds:
 //                                              duo    half
@@ -21,6 +23,8 @@ bool dq_split_keys(const pith_attn_bwd_args* a) {
   const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
   return wgs <= cus ? a->Skv > 256 : a->causal && wgs <= 2 * cus && a->Skv >= 1536;
 }
+
+}  // namespace
 
 bool ds_usable(const pith_attn_bwd_args* a) { return a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a); }
 
