@@ -18,6 +18,7 @@ struct FwdParams {
   float* lse;
   int Sq, Skv, Hq, Hkv, group;  // group = Hq / Hkv
   int B, m_tiles;
+  int chunked;  // tiles from which the heads are taken in chunks (decode_block; 128-row workgroups only)
   int64_t q_bs, k_bs, v_bs, o_bs, lse_bs, lse_hs;
   float kappa;  // scale * log2(e)
   // keys in two parts (k_pe != nullptr): k holds the first 128 features per head, k_pe the last 64,
@@ -43,10 +44,10 @@ struct FwdChunkParams : FwdParams {
 
 template <bool MULTI>
 using FwdArgs = std::conditional_t<MULTI, FwdChunkParams, FwdParams>;
-__device__ __forceinline__ KeyChunk chunk_of(const FwdParams& p, int) { return KeyChunk{p.k, p.v, p.k_pe, p.Skv, 0}; }
-__device__ __forceinline__ const KeyChunk& chunk_of(const FwdChunkParams& p, int i) { return p.chunk[i]; }
-__device__ __forceinline__ int chunk_count(const FwdParams&) { return 1; }
-__device__ __forceinline__ int chunk_count(const FwdChunkParams& p) { return p.n_chunks; }
+__host__ __device__ __forceinline__ KeyChunk chunk_of(const FwdParams& p, int) { return KeyChunk{p.k, p.v, p.k_pe, p.Skv, 0}; }
+__host__ __device__ __forceinline__ const KeyChunk& chunk_of(const FwdChunkParams& p, int i) { return p.chunk[i]; }
+__host__ __device__ __forceinline__ int chunk_count(const FwdParams&) { return 1; }
+__host__ __device__ __forceinline__ int chunk_count(const FwdChunkParams& p) { return p.n_chunks; }
 
 // Forward with one 8-wave workgroup per compute unit: attn_fwd_direct.hip. dqk = 128, or 192 with half; half = workgroups
 // of 128 query rows whose wave pairs split the keys of every tile (see there) instead of 256-row workgroups.

@@ -68,7 +68,7 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   const int c = lane & 31, g = lane >> 5;
 
   int m_tile, h, b;
-  decode_block(blockIdx.x, p.Hq, p.B, p.m_tiles, p.group, m_tile, h, b);
+  decode_block(blockIdx.x, p.Hq, p.B, p.m_tiles, p.group, m_tile, h, b, p.chunked);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
   const int q_wave0 = m0 + row_block * 32;
@@ -435,10 +435,38 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
+// Tiles from which the heads are taken in chunks (decode_block). Taken level by level (every head's tile t before any tile
+// t-1), the workgroups in flight stream K and V of all heads, which costs nothing while the last-level cache (256 MB) holds
+// them; once it does not, every level reads them from memory, and with 128-row workgroups half as many rows share a stream as
+// with 256-row ones. So the line is the size of K and V, however many the tiles; under the mask a row sees half of the keys
+// and heaviest-first over the whole grid is worth something, hence a higher one. Level by level / in chunks, us:
+//   d192 full    4096 x 64 heads (160 MiB) 588 / 601     8192 x 40 (200) 1381 / 1432    16384 x 24 (240) 3240 / 3300
+//                4096 x 96 (240) 932 / 899               6144 x 64 (240) 1278 / 1260    8192 x 64 (320) 2484 / 2249
+//                4096 x 128 (320) 1437 / 1189            6144 x 128 (480) 3385 / 2533   1024 x 256 (160) 207 / 179
+//        causal  8192 x 24 (120) 441 / 475               8192 x 40 (200) 718 / 765      9216 x 40 (225) 898 / 947
+//                4096 x 104 (260) 523 / 546              32768 x 16 (320) 4280 / 4319   2 x 16384 x 16 (320) 2230 / 2202
+//                4096 x 128 (320) 682 / 671              4096 x 256 (640) 1679 / 1292   2048 x 224 (280) 366 / 345
+//   d64  full    8192 x 64 (128) 1081 / 1079             8192 x 128 (256) 2266 / 2116   1024 x 512 (128) 173 / 158
+//        causal  8192 x 32 (64) 276 / 303                16384 x 64 (256) 2190 / 2249   16 x 4096 x 32 (512) 1582 / 1243
+// A walk over several chunks of keys has them one after the other: what counts is the size of one, and it takes many heads;
+// otherwise the line of many tiles stands. 4 ranks, d192, level by level / in chunks: 4096 x 128 heads (320 MiB a chunk) 2735 /
+// 2431 and 4830 / 4101; 3072 x 128 (240) 1425 / 1402 and 2533 / 2255; 2048 x 128 (160) 659 / 680 and 1152 / 1060; 4096 x 64
+// (160) 1149 / 1177 and 2004 / 2002; 6144 x 64 (240) 2675 / 2708; 8192 x 32 (160) 2278 / 2234 and 4014 / 3833.
+template <int DQK, bool MULTI>
+int chunked_tiles(const FwdArgs<MULTI>& p, bool causal) {
+  const bool two_part = DQK == 192 && chunk_of(p, 0).k_pe != nullptr;
+  const int64_t keys = chunk_of(p, chunk_count(p) - 1).rows, heads = (int64_t)p.B * p.Hkv;  // (the last chunk is a whole one)
+  const int64_t mib = keys * heads * ((two_part ? 128 : DQK) + (DQK == 64 ? 64 : 128)) * 2 >> 20;
+  if (MULTI) return heads >= 96 && mib >= 200 ? 1 : kChunkedTiles;
+  const int64_t line = causal ? (DQK != 64 && heads >= 208 ? 240 : 288) : heads >= 192 ? 128 : heads >= 64 ? 200 : 256;
+  return mib >= line ? 1 : 0x7fffffff;
+}
+
 template <int DQK, int PARTS, bool MULTI>
 void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
   using L = DuoLayout<DQK, PARTS>;
   p.m_tiles = (p.Sq + L::kBM - 1) / L::kBM;
+  p.chunked = chunked_tiles<DQK, MULTI>(p, causal);
   const dim3 grid((unsigned)(p.m_tiles * p.Hq * p.B)), block(L::kThreads);
   if constexpr (MULTI) {  // the last chunk is seen under the mask
     hipLaunchKernelGGL((attn_fwd_duo_kernel<DQK, PARTS, true, true>), grid, block, 0, st, p);

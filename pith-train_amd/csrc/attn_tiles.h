@@ -61,18 +61,19 @@ __device__ __forceinline__ bf16x8 to_bf16x8(float a0, float a1, float a2, float 
 //   - workgroups are dealt round-robin to the 8 XCDs of the device, each with its own L2: the
 //     heads of one level are permuted so that an XCD keeps a contiguous range of heads, i.e. the
 //     query heads that share a kv head read their K/V through the same L2;
-//   - with more than 8 kv heads per level (`group` = query heads per kv head) and at least kChunkedTiles tiles
+//   - with more than 8 kv heads per level (`group` = query heads per kv head) and at least `chunked` tiles
 //     the heads are taken in chunks of 8 kv heads, all tiles of a chunk before the next chunk: the workgroups an
 //     XCD holds at one time then belong to ONE kv head and stream the same K/V tiles at about the same time,
 //     instead of one stream per head. Each chunk ends with its light tiles, so the order is no longer
 //     heaviest-first over the whole grid: measured 9-14 % faster at 128 heads x 32768 rows, 2-6 % slower at 4096
-//     rows (16-32 tiles), hence the threshold.
+//     rows (16-32 tiles), hence the threshold; the forward with 128-row workgroups goes by the size of K and V instead
+//     (attn_fwd_duo.hip).
 constexpr int kChunkedTiles = 64;
-__device__ __forceinline__ void decode_block(int linear, int heads, int batch, int tiles, int group, int& tile, int& h, int& b) {
+__device__ __forceinline__ void decode_block(int linear, int heads, int batch, int tiles, int group, int& tile, int& h, int& b, int chunked = kChunkedTiles) {
   const int per_level = heads * batch;
   const int chunk = 8 * group;
   int level, pos;
-  if (tiles >= kChunkedTiles && per_level > chunk && per_level % chunk == 0) {
+  if (tiles >= chunked && per_level > chunk && per_level % chunk == 0) {
     const int per_chunk = chunk * tiles;
     const int c = linear / per_chunk;
     const int rem = linear - c * per_chunk;

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from pithtrain_amd.operators.mla import hip as H
+from pithtrain_amd.operators.ring_attention import local as L
 
 pytestmark = pytest.mark.gpu
 
@@ -127,3 +128,43 @@ def test_chunked_order_with_a_batch_dimension(gpu):
         part = run(*(t[b : b + 1] for t in (q, k, v, dout)))
         for name, w, p in zip(("o", "dq", "dk", "dv"), whole, part):
             _close(w[b : b + 1], p, f"{name}, batch element {b}")
+
+
+# K and V large enough for heads in chunks in the forward with small workgroups (attn_fwd_duo.hip, chunked_tiles); the halves of
+# the heads stay below the line. (Dqk, rows, keys, heads, causal): few tiles of 64 and 128 rows, the line without a mask, with
+# one, and for many heads; many tiles below the line.
+@pytest.mark.parametrize("D,Sq,Skv,heads,causal", [(64, 160, 2736, 192, False), (192, 130, 8200, 40, False), (192, 1030, 1030, 336, False),
+                                                   (128, 2304, 2304, 256, True), (64, 8200, 8200, 16, True)])  # fmt: skip
+def test_forward_with_many_heads(gpu, D, Sq, Skv, heads, causal):
+    dv = min(D, 128)
+    g = torch.Generator(device=gpu).manual_seed(11)
+    q, k, v = (torch.randn(1, n, heads, d, generator=g, device=gpu).to(torch.bfloat16) for n, d in ((Sq, D), (Skv, D), (Skv, dv)))
+
+    def run(hs):
+        qs, ks, vs = (t[:, :, hs].contiguous() for t in (q, k, v))
+        o = torch.full((1, Sq, qs.shape[2], dv), float("nan"), dtype=torch.bfloat16, device=gpu)
+        lse = torch.full((1, qs.shape[2], Sq), float("nan"), device=gpu)
+        H.attn_fwd_into(qs, ks, vs, o, lse, D**-0.5, causal)
+        return o, lse
+
+    o, lse = run(slice(0, heads))
+    for hs in (slice(0, heads // 2), slice(heads // 2, heads)):
+        part = run(hs)
+        _close(o[:, :, hs], part[0], "o")
+        assert (lse[:, hs] - part[1]).abs().max().item() < 2e-3
+
+
+def test_share_forward_with_many_heads(gpu):
+    """The same for a walk over several chunks of keys: 2 x 1600 keys x 256 heads of 128 are 400 MiB."""
+    g = torch.Generator(device=gpu).manual_seed(12)
+    q, k0, k1, v0, v1 = (torch.randn(1, 1600, 256, 128, generator=g, device=gpu).to(torch.bfloat16) for _ in range(5))
+
+    def run(hs):
+        qs, ka, kb, va, vb = (t[:, :, hs].contiguous() for t in (q, k0, k1, v0, v1))
+        return L.ring_forward_local(qs, [ka, kb], [va, vb], 128**-0.5, 1, 2, "contiguous")
+
+    o, lse = run(slice(0, 256))
+    for hs in (slice(0, 128), slice(128, 256)):
+        part = run(hs)
+        _close(o[:, :, hs], part[0], "o")
+        assert (lse[:, hs] - part[1]).abs().max().item() < 2e-3
