@@ -132,9 +132,9 @@ def test_chunked_order_with_a_batch_dimension(gpu):
 
 # K and V large enough for heads in chunks in the forward with small workgroups (attn_fwd_duo.hip, chunked_tiles); the halves of
 # the heads stay below the line. (Dqk, rows, keys, heads, causal): few tiles of 64 and 128 rows, the line without a mask, with
-# one, and for many heads; many tiles below the line.
+# one, and for many heads; many tiles below the line. The last: 256-row workgroups (attn_fwd.hip, many_heads).
 @pytest.mark.parametrize("D,Sq,Skv,heads,causal", [(64, 160, 2736, 192, False), (192, 130, 8200, 40, False), (192, 1030, 1030, 336, False),
-                                                   (128, 2304, 2304, 256, True), (64, 8200, 8200, 16, True)])  # fmt: skip
+                                                   (128, 2304, 2304, 256, True), (64, 8200, 8200, 16, True), (128, 1030, 1030, 448, True)])  # fmt: skip
 def test_forward_with_many_heads(gpu, D, Sq, Skv, heads, causal):
     dv = min(D, 128)
     g = torch.Generator(device=gpu).manual_seed(11)
