@@ -245,8 +245,12 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
 //   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186, 3 x 1024 x 16 92 -> 94; 1.7: 1 x 3456 x 16
 //                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
 // Several chunks, whose dK/dV workgroups are more unequal, gain 1-5 % up to two per unit (2048 x 32/4 of 128, 4 ranks,
-// zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081); with three they lose (6144 x 16 of 192: 2385 ->
-// 2413). At 64 features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only
+// zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081). 128 features: up to four, where two launches lost
+// even to one pair of them per ring step (in brackets): 4096 x 32/4, 4 ranks, rank 0 1889 -> 1728 (1724); 9216 x 8/2, 8
+// ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
+// rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
+// 16: 2385 -> 2413).
+// At 64 features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only
 // grids of a few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us, 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16
 // 474 -> 483 us).
 bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
@@ -254,7 +258,7 @@ bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
   const int64_t cus = compute_units_or_default();
   const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
   if (a->Dqk == 64) return q_wgs <= 4 * cus;
-  if (chunks) return q_wgs <= 2 * cus;
+  if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
   if (q_wgs <= cus) return true;
   if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;
   return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));

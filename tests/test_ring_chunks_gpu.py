@@ -6,6 +6,7 @@ import torch
 
 from helpers import check_bf16_result, check_lse
 from oracle import ring_oracle as R
+from pithtrain_amd.operators.mla import hip as H
 from pithtrain_amd.operators.ring_attention import local as L
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +65,15 @@ def test_share(gpu, monkeypatch, one_launch, B, S, Hq, Hkv, D, C, rank, layout, 
 def test_share_of_unequal_rows_64_features(gpu, monkeypatch):
     """The two-team forward over several chunks."""
     test_share(gpu, monkeypatch, True, 1, 1026, 36, 36, 64, 2, 0, "zigzag", False)
+
+
+# Backward of shares with more 128-row query workgroups than one grid of dK/dV and dQ takes (attn_bwd_dkdv.hip, one_grid: two
+# per compute unit at 192 features, four at 64 and 128): two launches, the dQ one with two workgroups per compute unit; and at
+# 128 features the last of the single grids. Chunk ends, half chunks and half rows fall into tiles in all of them.
+@pytest.mark.parametrize("S,Hq,Hkv,D,C,rank,layout,two_part", [
+    (130, 516, 258, 64, 3, 1, "zigzag", False), (130, 516, 516, 128, 3, 1, "zigzag", False), (258, 344, 86, 128, 2, 1, "contiguous", False),
+    (130, 260, 130, 128, 3, 1, "zigzag", False), (130, 260, 260, 192, 3, 1, "zigzag", False), (258, 172, 172, 192, 2, 1, "contiguous", True),
+    (130, 260, 260, 192, 2, 0, "zigzag", True)])  # fmt: skip
+def test_share_with_many_workgroups(gpu, monkeypatch, S, Hq, Hkv, D, C, rank, layout, two_part):
+    monkeypatch.setattr(H, "DS_BUFFER_LIMIT_BYTES", 0)  # no dS hand-over: every kernel recomputes
+    test_share(gpu, monkeypatch, True, 1, S, Hq, Hkv, D, C, rank, layout, two_part)
