@@ -317,6 +317,38 @@ bool ring_chunks(const Tensor& q, const std::vector<OptTensor>& ks, const std::v
   return true;
 }
 
+// Compute units of a device, looked up once.
+int64_t compute_units(int device) {
+  static std::array<std::atomic<int>, 64> cached = {};
+  if (device < 0 || device >= 64) return 0;
+  int n = cached[device].load(std::memory_order_relaxed);
+  if (n == 0) {
+    pith_device_info_t info;
+    if (pith_device_info(device, &info) != PITH_OK) return 0;
+    cached[device].store(n = info.compute_units, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Whether a share's forward goes out as one launch over its chunks, or as one launch per ring step. One launch saves launches
+// and merges; but its loop keeps the state of several walks, and one work split has to serve chunks with and without a mask,
+// where the steps take the best for each. That shows where workgroups are few and streams long. rows = query rows, wgs = 128-row
+// workgroups, mean = mean length of the rows' streams in percent of the longest. One launch against steps, time ratio:
+//   more than two workgroups per compute unit, or 64-row ones fit:  0.85-1.01
+//   up to two    8192 x 8 heads of 128, mean 50 / 57 / 67 / 75      1.00 / 1.02 / 1.07 / 1.07      16384 x 4  1.04 / 1.06 / 1.09 / 1.10
+//                16384 x 4 of 192 1.04 / 1.06 / 1.06 / 1.07         8192 x 8  1.00 / 1.01 / 1.03 / 1.03
+//                3072 x 16 of 128 0.90 / 0.87 / 0.98 / 1.04         4096 x 16 of 192  0.95 / 0.94 / 0.98 / 1.00
+//   up to one    8192 x 4 of 128  0.92 / 0.96 / 1.03 / 1.08         6144 x 4 of 192  0.91 / 0.88 / 1.03 / 1.14
+//                16384 x 2 of 128 0.97 / 1.03 / 1.09 / 1.13         12288 x 2 of 192  0.99 / 0.94 / 1.06 / 1.22
+//   two chunks only: 6144 x 8 of 128 1.04 (mean 50), 1.10 (75); eight chunks: 8192 x 8 of 192 0.96, 16384 x 4 1.06
+bool share_forward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chunks, int64_t mean, int64_t cus) {
+  const int64_t wgs = (rows + 127) / 128 * heads, wgs64 = (rows + 63) / 64 * heads;
+  if (dqk == 64 || chunks == 1 || wgs > 2 * cus || wgs64 <= cus) return true;
+  if (rows >= 12288 || (rows >= 8192 && chunks < 8)) return wgs <= cus && mean <= 60;
+  if (wgs <= cus) return rows < 6144 || mean <= 65;
+  return !(chunks == 2 && (rows >= 6144 || (dqk == 128 && mean > 70 && rows >= 3072)));
+}
+
 // (out, lse), or None when the steps have to run one by one.
 std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs,
                                                        const std::optional<std::vector<OptTensor>>& pes, double scale, int64_t rank, int64_t cp,
@@ -324,6 +356,13 @@ std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const st
   pith_attn_fwd_args a = {};
   RingChunks r;
   if (!ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r)) return std::nullopt;
+  int64_t keys = 0, seen = 0;  // in the chunks; (query row, key) pairs
+  for (const pith_key_chunk& c : r.chunk) {
+    keys += c.rows;
+    seen += &c == &r.chunk.back() ? c.rows * a.Sq / 2 : c.rows * (a.Sq - c.q_row0);
+  }
+  if (keys * a.Sq > 0 && !share_forward_in_one(a.Dqk, a.Sq, a.Hq * a.B, (int64_t)r.chunk.size(), 100 * seen / (keys * a.Sq), compute_units(q.device().index())))
+    return std::nullopt;
   Tensor o = at::empty({a.B, a.Sq, a.Hq, a.Dv}, q.options());
   Tensor lse = empty_like_shape(q, {a.B, a.Hq, a.Sq}, at::kFloat);
   a.o = o.data_ptr(); a.lse = lse.data_ptr<float>();
@@ -389,19 +428,6 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
     if (attn_fwd_into(q, k, v, o, lse, scale, causal, {}, {}, {}, {}, {})) return {o, lse};
   }
   return python_body<Two>("attn_fwd", q, k, v, scale, causal);
-}
-
-// Compute units of a device, looked up once.
-int64_t compute_units(int device) {
-  static std::array<std::atomic<int>, 64> cached = {};
-  if (device < 0 || device >= 64) return 0;
-  int n = cached[device].load(std::memory_order_relaxed);
-  if (n == 0) {
-    pith_device_info_t info;
-    if (pith_device_info(device, &info) != PITH_OK) return 0;
-    cached[device].store(n = info.compute_units, std::memory_order_relaxed);
-  }
-  return n;
 }
 
 // Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill
@@ -860,5 +886,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("combine_new", &combine_new, Unlocked());
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into, Unlocked());
   m.def("accepted", &accepted);
+  m.def("share_forward_in_one", &share_forward_in_one);
   m.def("ds_handover_pays", &ds_handover_pays);
 }

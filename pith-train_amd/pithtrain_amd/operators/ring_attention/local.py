@@ -53,8 +53,9 @@ from pithtrain_amd.operators.mla.hip import (
 from pithtrain_amd.operators.ring_attention.combine import cast_f32_bf16_into, combine_into
 
 LAYOUTS = ("contiguous", "zigzag")
-# A share whose chunks are all at hand runs as one launch over all of them; False restores one launch per step (what a
-# share has to do whose chunks arrive one by one; kept for comparison runs).
+# A share whose chunks are all at hand runs as one launch over all of them where that is faster (csrc/host/torch_ops.cpp);
+# False restores one launch per step everywhere (what a share has to do whose chunks arrive one by one; kept for comparison
+# runs).
 FUSE_CHUNKS = True
 # Ring steps after the first merge inside the forward kernel (one launch per step) where the kernels support it;
 # False restores chunk forward + combine launch per step (kept for comparison runs).

@@ -10,6 +10,7 @@ from pithtrain_amd import _C
 from pithtrain_amd._ext import native
 from pithtrain_amd.operators.mla_assemble import mla_assemble_qkv
 from pithtrain_amd.operators.norm_rope import norm_rope, qk_norm_rope
+from pithtrain_amd.operators.ring_attention.local import ring_schedule
 
 
 def _meta(*shape):
@@ -86,3 +87,18 @@ def test_bound_functions_release_the_interpreter_lock(name):
     finally:
         sys.setswitchinterval(before)
         other.join()
+
+
+@pytest.mark.parametrize("in_one,dqk,rows,heads,cp,rank,layout", [
+    (True, 128, 8192, 32, 4, 1, "zigzag"), (True, 192, 4096, 16, 4, 1, "zigzag"), (True, 192, 1021, 16, 4, 2, "contiguous"),
+    (True, 128, 8192, 4, 4, 0, "zigzag"), (True, 128, 3072, 16, 4, 3, "contiguous"), (True, 64, 16384, 4, 4, 1, "contiguous"),
+    (True, 192, 8192, 2, 2, 1, "contiguous"), (False, 128, 8192, 8, 2, 1, "zigzag"), (False, 128, 6144, 8, 4, 1, "contiguous"),
+    (False, 128, 4096, 16, 2, 1, "contiguous"), (False, 192, 16384, 4, 8, 3, "zigzag"), (False, 192, 6144, 4, 4, 3, "contiguous"),
+    (False, 192, 12288, 4, 4, 0, "zigzag"), (True, 128, 8192, 8, 4, 0, "contiguous"), (True, 192, 8192, 8, 8, 3, "zigzag"),
+    (False, 128, 6144, 8, 2, 0, "zigzag"), (True, 128, 6144, 8, 4, 0, "zigzag")])  # fmt: skip
+def test_share_forward_by_size(in_one, dqk, rows, heads, cp, rank, layout):
+    """One launch over all chunks, or one per ring step: whichever measured faster (256 compute units)."""
+    steps = ring_schedule(rank, cp, rows, layout)
+    keys = sum(st.kv_rows[1] - st.kv_rows[0] for st in steps)
+    seen = sum((st.q_rows[1] - st.q_rows[0]) * (st.kv_rows[1] - st.kv_rows[0]) // (2 if st.causal else 1) for st in steps)
+    assert native.share_forward_in_one(dqk, rows, heads, len(steps), 100 * seen // (keys * rows), 256) == in_one
