@@ -372,6 +372,17 @@ std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const st
   return std::make_tuple(o, lse);
 }
 
+// The same for the backward without a dS hand-over. One grid over all chunks fills the rounds that a step's kernels leave half
+// empty; long streams of whole chunks whose query workgroups come in whole rounds have none, and a step can cut the heads of
+// its chunk finer. One grid against steps, 128 features: 8192 x 8/2 heads, 4 ranks 1850 and 1744 us (rank 0), 8 ranks,
+// contiguous 3790 and 3480, 16384 x 8/2, 2 ranks 3320 and 3130, 16384 x 4 contiguous 5464 and 5377; but 9216 x 8/2, 8 ranks
+// 4593 and 4746, 12288 x 8/2 rank 0 3736 and 3675, rank 1 (half chunks) 3594 and 3747, 8192 x 8/2 rank 1 1705 and 1738.
+bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chunks, int64_t keys, int64_t cus) {
+  const int64_t wgs = (rows + 127) / 128 * heads;
+  const bool whole_rounds = cus > 0 && wgs % (2 * cus) == 0 && wgs <= 4 * cus;
+  return dqk != 128 || chunks == 1 || rows < 8192 || keys < chunks * rows || !whole_rounds;
+}
+
 // (dq, dk list, dv list, dk_pe list or empty); the lists hold a tensor per visited chunk. None as above. The policy for the
 // dS hand-over is the caller's: this call recomputes.
 using RingGrads = std::tuple<Tensor, std::vector<OptTensor>, std::vector<OptTensor>, std::vector<OptTensor>>;
@@ -381,6 +392,9 @@ std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, c
   pith_attn_bwd_args a = {};
   RingChunks r;
   if (!ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r)) return std::nullopt;
+  int64_t keys = 0;
+  for (const pith_key_chunk& c : r.chunk) keys += c.rows;
+  if (!share_backward_in_one(a.Dqk, a.Sq, a.Hq * a.B, (int64_t)r.chunk.size(), keys, compute_units(q.device().index()))) return std::nullopt;
   if (!is_gpu_bf16(dout_in, 4) || !is_gpu_bf16(out, 4) || !out.is_contiguous() || !is_gpu_f32(lse, 3) || !lse.is_contiguous() ||
       dout_in.device() != q.device() || out.device() != q.device() || lse.device() != q.device() || !has_shape(dout_in, {a.B, a.Sq, a.Hq, a.Dv}) ||
       !has_shape(out, {a.B, a.Sq, a.Hq, a.Dv}) || !has_shape(lse, {a.B, a.Hq, a.Sq}))
@@ -887,5 +901,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into, Unlocked());
   m.def("accepted", &accepted);
   m.def("share_forward_in_one", &share_forward_in_one);
+  m.def("share_backward_in_one", &share_backward_in_one);
   m.def("ds_handover_pays", &ds_handover_pays);
 }
