@@ -58,8 +58,9 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   if (wgs <= cus && a->Skv > (d64 ? 1024 : 512)) return key_split;
   if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 1535)) return key_split;
   // FULL under the mask also for shorter rows of many heads whose K and V outgrow the last-level cache (half the streams in
-  // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235)
-  const bool many_heads = a->Skv == a->Sq && a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2 >= 224ll << 20;
+  // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
+  // for rows of a few workgroups: 8 x 512 x 128 155 -> 167)
+  const bool many_heads = a->Sq >= 1024 && a->Skv == a->Sq && a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2 >= 224ll << 20;
   if (a->Dqk == 128 && (unequal ? (a->Sq >= 3072 || many_heads) && wgs > 2 * cus : a->Skv > 1024 && wgs > cus)) return Split::kFull;
   return Split::kDuo;
 }

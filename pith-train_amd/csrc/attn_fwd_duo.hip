@@ -439,10 +439,12 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
 // t-1), the workgroups in flight stream K and V of all heads, which costs nothing while the last-level cache (256 MB) holds
 // them; once it does not, every level reads them from memory, and with 128-row workgroups half as many rows share a stream as
 // with 256-row ones. So the line is the size of K and V, however many the tiles; under the mask a row sees half of the keys
-// and heaviest-first over the whole grid is worth something, hence a higher one. Level by level / in chunks, us:
+// and heaviest-first over the whole grid is worth something, hence a higher one. From 192 heads on a chunk's tiles are in flight
+// together and read its K and V through one L2: without a mask, chunks for any size. Level by level / in chunks, us:
 //   d192 full    4096 x 64 heads (160 MiB) 588 / 601     8192 x 40 (200) 1381 / 1432    16384 x 24 (240) 3240 / 3300
 //                4096 x 96 (240) 932 / 899               6144 x 64 (240) 1278 / 1260    8192 x 64 (320) 2484 / 2249
 //                4096 x 128 (320) 1437 / 1189            6144 x 128 (480) 3385 / 2533   1024 x 256 (160) 207 / 179
+//                768 x 256 (120) 123 / 104               512 x 384 (120) 91 / 80        384 x 512 of 64 features 35.4 / 32.5
 //        causal  8192 x 24 (120) 441 / 475               8192 x 40 (200) 718 / 765      9216 x 40 (225) 898 / 947
 //                4096 x 104 (260) 523 / 546              32768 x 16 (320) 4280 / 4319   2 x 16384 x 16 (320) 2230 / 2202
 //                4096 x 128 (320) 682 / 671              4096 x 256 (640) 1679 / 1292   2048 x 224 (280) 366 / 345
@@ -458,7 +460,7 @@ int chunked_tiles(const FwdArgs<MULTI>& p, bool causal) {
   const int64_t keys = chunk_of(p, chunk_count(p) - 1).rows, heads = (int64_t)p.B * p.Hkv;  // (the last chunk is a whole one)
   const int64_t mib = keys * heads * ((two_part ? 128 : DQK) + (DQK == 64 ? 64 : 128)) * 2 >> 20;
   if (MULTI) return heads >= 96 && mib >= 200 ? 1 : kChunkedTiles;
-  const int64_t line = causal ? (DQK != 64 && heads >= 208 ? 240 : 288) : heads >= 192 ? 128 : heads >= 64 ? 200 : 256;
+  const int64_t line = causal ? (DQK != 64 && heads >= 208 ? 240 : 288) : heads >= 192 ? 0 : heads >= 64 ? 200 : 256;
   return mib >= line ? 1 : 0x7fffffff;
 }
 
