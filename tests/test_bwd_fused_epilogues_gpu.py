@@ -93,8 +93,10 @@ def test_dq_final_rows_equal_accumulate_then_cast(gpu, Sq, Skv, Hq, Hkv, handove
 @pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
 @pytest.mark.parametrize("Hq,Hkv,S,D", [(8, 2, 2048, 128), (32, 4, 4096, 128), (4, 4, 1000, 128), (4, 4, 2048, 192)])
 def test_ring_backward_with_and_without_the_fused_epilogues(gpu, layout, Hq, Hkv, S, D, monkeypatch):
-    """Every rank of a ring of 4: dQ, dK, dV bit for bit the same whether the fill and the cast are separate
-    launches or folded into the dK/dV and dQ launches, and equal to the oracle's ring share."""
+    """Every rank of a ring of 4, step by step as a rank runs it whose chunks arrive one by one: dQ, dK, dV bit for bit the
+    same whether the fill and the cast are separate launches or folded into the dK/dV and dQ launches, and equal to the
+    oracle's ring share."""
+    monkeypatch.setattr(L, "FUSE_CHUNKS", False)  # the one launch over all chunks reads neither switch
     B, C = 1, 4
     g = torch.Generator().manual_seed(13)
     scale = D**-0.5
@@ -104,6 +106,14 @@ def test_ring_backward_with_and_without_the_fused_epilogues(gpu, layout, Hq, Hkv
         pytest.skip("zigzag needs 2 * cp_size blocks")
     qs, ks, vs, dos = (split(t) for t in full)
     kd, vd = [c.to(gpu) for c in ks], [c.to(gpu) for c in vs]
+    fused_calls = []  # per step: whether it finishes dQ rows or clears the rows behind the visible ones itself
+    pair = L.attn_bwd_pair_into
+
+    def counting(*args, **kw):
+        fused_calls.append(kw["dq_final"] is not None or kw["zero_tail"] > 0)
+        return pair(*args, **kw)
+
+    monkeypatch.setattr(L, "attn_bwd_pair_into", counting)
     for r in range(C):
         res = {}
         for fused in (True, False):
@@ -111,7 +121,11 @@ def test_ring_backward_with_and_without_the_fused_epilogues(gpu, layout, Hq, Hkv
             monkeypatch.setattr(L, "FUSE_ZERO_TAIL", fused)
             qd = qs[r].to(gpu)
             out, lse = L.ring_forward_local(qd, kd, vd, scale, r, C, layout)
+            fused_calls.clear()
             res[fused] = L.ring_backward_local(dos[r].to(gpu), qd, out, lse, kd, vd, scale, r, C, layout)
+            # both runs did what their switches say (a share of one chunk has nothing to fold)
+            assert fused or not any(fused_calls)
+            assert not fused or any(fused_calls) or len(L.ring_schedule(r, C, S // C, layout)) == 1
         dq1, dk1, dv1 = res[True]
         dq0, dk0, dv0 = res[False]
         assert torch.equal(dq1, dq0), f"rank {r}: dQ differs"
