@@ -377,10 +377,13 @@ std::optional<std::tuple<Tensor, Tensor>> ring_forward(const Tensor& q, const st
 // its chunk finer. One grid against steps, 128 features: 8192 x 8/2 heads, 4 ranks 1850 and 1744 us (rank 0), 8 ranks,
 // contiguous 3790 and 3480, 16384 x 8/2, 2 ranks 3320 and 3130, 16384 x 4 contiguous 5464 and 5377; but 9216 x 8/2, 8 ranks
 // 4593 and 4746, 12288 x 8/2 rank 0 3736 and 3675, rank 1 (half chunks) 3594 and 3747, 8192 x 8/2 rank 1 1705 and 1738.
+// Beyond the one grid (two launches; a share of that size recomputes only for want of memory) the same holds of half chunks
+// too: 8192 x 32/4 6707 and 6202, rank 1 6702 and 6249, 4096 x 64/4 3715 and 3246, but 6144 x 32/4 rank 3 3574 and 3864.
 bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chunks, int64_t keys, int64_t cus) {
   const int64_t wgs = (rows + 127) / 128 * heads;
-  const bool whole_rounds = cus > 0 && wgs % (2 * cus) == 0 && wgs <= 4 * cus;
-  return dqk != 128 || chunks == 1 || rows < 8192 || keys < chunks * rows || !whole_rounds;
+  if (dqk != 128 || chunks == 1 || cus == 0) return true;
+  if (wgs > 4 * cus) return rows < 4096 || wgs % (4 * cus) != 0;
+  return rows < 8192 || keys < chunks * rows || wgs % (2 * cus) != 0;
 }
 
 // (dq, dk list, dv list, dk_pe list or empty); the lists hold a tensor per visited chunk. None as above. The policy for the

@@ -108,7 +108,7 @@ def test_share_forward_by_size(in_one, dqk, rows, heads, cp, rank, layout):
     (False, 128, 8192, 8, 4, 0, "zigzag"), (False, 128, 8192, 8, 8, 4, "contiguous"), (False, 128, 16384, 8, 2, 0, "zigzag"),
     (True, 128, 8192, 8, 4, 1, "zigzag"), (True, 128, 12288, 8, 4, 0, "zigzag"), (True, 128, 4096, 16, 4, 0, "zigzag"),
     (True, 128, 9216, 8, 8, 4, "contiguous"), (True, 192, 16384, 4, 4, 0, "zigzag"), (True, 64, 8192, 16, 4, 0, "zigzag"),
-    (True, 128, 8192, 8, 4, 0, "contiguous")])  # fmt: skip
+    (True, 128, 8192, 8, 4, 0, "contiguous"), (False, 128, 8192, 32, 4, 1, "zigzag"), (True, 128, 6144, 32, 4, 3, "zigzag")])  # fmt: skip
 def test_share_backward_by_size(in_one, dqk, rows, heads, cp, rank, layout):
     steps = ring_schedule(rank, cp, rows, layout)
     keys = sum(st.kv_rows[1] - st.kv_rows[0] for st in steps)
