@@ -6,7 +6,7 @@
 
 A step is one forward + backward pass of one GPU's share of causal ring attention at the
 Qwen3-30B-A3B shape (32 q heads / 4 kv heads, head dim 128, 32768 tokens as 4 zigzag chunks of 8192,
-rank 1 of 4): 4 chunk-attention forwards, 3 log2 combines, delta, 4 dK/dV and 4 dQ launches.
+rank 1 of 4): one forward launch over the four chunks, delta, 4 dK/dV and 4 dQ launches and the 2 that add partial sums.
 Inputs are synthetic (CPU generator, seed 42; q/k/v ~ N(0,1)/sqrt(Dqk), dO ~ N(0,1)) and resident in
 HBM before the timed region. One JSON line is printed; everything in it is measured in this run except
 `roofline.traffic` (HBM bytes per launch need a rocprofv3 --pmc run: the figure is read from the committed summary
@@ -15,10 +15,10 @@ named beside it in `traffic_from`, null when that summary has none):
   value      algorithmic TFLOP/s of the whole step: 2*(Dqk+Dv)*E*Hq forward + 2*(3Dqk+2Dv)*E*Hq backward
              with E = C*S_l^2/2 score entries per head (5 backward matmuls; recomputation not counted)
   roofline   the dominant kernel (non-causal dK/dV), timed per launch with events on the launch stream
-  fwd_only   the forward alone (the forward-only configuration of the same shape), with its dominant kernel
-             (the non-causal forward launch) and its own CPU baseline
+  fwd_only   the forward alone (the forward-only configuration of the same shape): its one kernel, and its own CPU
+             baseline
   mla16k     the same ring driver at the MLA shape (16 heads, 192/128, 16384 tokens as 4 zigzag chunks), with the
-             roofline of its dominant kernel and the CPU port on the whole workload
+             roofline of its dominant kernel (dK/dV and dQ of all chunks in one grid) and the CPU port on the whole workload
   long131k   the same at the long-context shape (64 q / 4 kv heads, 131072 tokens as 8 zigzag chunks, rank 3);
              CPU port on 4 of the 64 query heads
   mla_op     the reference's own MLA operator benchmark matrix (h in {16,128} x s in {4096,32768}, causal,
@@ -150,7 +150,7 @@ def ring_summary(cfg, ms_step, ms_fwd, ms_bwd):
     step_tf = tf(fwd_flops + bwd_flops, ms_step)
     return {
         "workload": f"{cfg.hq} q / {cfg.hkv} kv heads, head dims {cfg.dqk}/{cfg.dv}, S={cfg.cp * cfg.s_local} as {cfg.cp} zigzag "
-                    f"chunks of {cfg.s_local} looped locally (rank {cfg.rank}), B=1, fwd+bwd incl. combines and delta",
+                    f"chunks of {cfg.s_local} looped locally (rank {cfg.rank}), B=1, fwd+bwd incl. merges and delta",
         "ms_per_step": round(ms_step, 4), "tflops": round(step_tf, 2), "frac_mfma_peak": round(step_tf / MFMA_BF16_PEAK_TFLOPS, 4),
         "fwd": {"ms": round(ms_fwd, 4), "tflops": round(tf(fwd_flops, ms_fwd), 2)},
         "bwd": {"ms": round(ms_bwd, 4), "tflops": round(tf(bwd_flops, ms_bwd), 2)},
@@ -249,47 +249,51 @@ def dominant_dkdv(torch, cfg, dev, out, lse, reps, counter_pass=False):
     return ms, flops, len(launches), (0 if buf is None else buf.numel())
 
 
-def dominant_fwd(torch, cfg, dev, reps):
-    """The non-causal chunk-attention forward launches of one step of `cfg`, timed like dominant_dkdv."""
-    from pithtrain_amd.operators.mla import hip
+def share_forward(torch, cfg, dev, reps):
+    """The forward of a share of `cfg`: one launch over all of its chunks. (ms, FLOPs, launches)."""
+    from pithtrain_amd.operators.ring_attention.local import ring_forward_local
 
     q, ks, vs, _ = dev
-    scale = cfg.dqk**-0.5
-    launches, flops = [], 0
-    for s in noncausal_steps(cfg):
-        kr, qr = slice(*s.kv_rows), slice(*s.q_rows)
-        n_q = qr.stop - qr.start
-        o = torch.empty((1, n_q, cfg.hq, cfg.dv), dtype=torch.bfloat16, device=q.device)
-        l = torch.empty((1, cfg.hq, n_q), dtype=torch.float32, device=q.device)
-        launches.append((q[:, qr], ks[s.kv_rank][:, kr], vs[s.kv_rank][:, kr], o, l))
-        flops = 2 * (cfg.dqk + cfg.dv) * n_q * (kr.stop - kr.start) * cfg.hq
-
-    def run():
-        for a in launches:
-            hip.attn_fwd_into(*a, scale, False)
-
+    run = lambda: ring_forward_local(q, ks, vs, cfg.dqk**-0.5, cfg.rank, cfg.cp, LAYOUT)  # noqa: E731
     run()
-    return time_events(torch, run, reps) / len(launches), flops, len(launches)
+    return time_events(torch, run, reps), cfg.flops()[0], 1
+
+
+def share_backward(torch, cfg, dev, out, lse, reps):
+    """The backward of a share of `cfg` that hands no dS over: dK/dV and dQ of all chunks in one grid, behind the delta
+    launch (8 us of it at 4096 rows x 16 heads). (ms, FLOPs, launches)."""
+    from pithtrain_amd.operators.ring_attention.local import ring_backward_local
+
+    q, ks, vs, dout = dev
+    run = lambda: ring_backward_local(dout, q, out, lse, ks, vs, cfg.dqk**-0.5, cfg.rank, cfg.cp, LAYOUT)  # noqa: E731
+    run()
+    return time_events(torch, run, reps), cfg.flops()[1], 1
 
 
 def bench_other_config(torch, device, cfg, steps, warmup, cpu_heads=None, counter_pass=False):
-    """Step time of another configuration through the same ring driver, its dominant kernel (the non-causal dK/dV
-    launch) against the MFMA roofline, and (cpu_heads = (first, last+1) query heads, or "all") the oracle's CPU port
-    on that sample of the same workload."""
+    """Step time of another configuration through the same ring driver, its dominant kernel (the non-causal dK/dV launch,
+    or the one grid of a share that hands no dS over) against the MFMA roofline, and (cpu_heads = (first, last+1) query
+    heads, or "all") the oracle's CPU port on that sample of the same workload."""
     host, dev = cfg.make_inputs(torch, device, host=cpu_heads is not None)
     ms_step, ms_fwd, ms_bwd, o, lse = time_ring_share(torch, cfg, dev, steps, warmup)
+    scratch = handover_scratch_bytes(cfg, dev)
     if counter_pass:
-        dominant_dkdv(torch, cfg, dev, o, lse, 1, counter_pass=True)
+        if scratch:
+            dominant_dkdv(torch, cfg, dev, o, lse, 1, counter_pass=True)
         return None
     out = ring_summary(cfg, ms_step, ms_fwd, ms_bwd)
-    ms, flops, n, scratch = dominant_dkdv(torch, cfg, dev, o, lse, steps)
-    kname = "attn_bwd_dkdv_d192_kernel" if cfg.dqk == 192 else "attn_bwd_dkdv_d128_kernel"
-    slabs = n // len(noncausal_steps(cfg))
-    out["roofline"] = roofline_entry(
-        f"{kname}<non-causal> (S, dP, dV, dK of one ring step" + (f", one of {slabs} kv-head slabs per launch" if slabs > 1 else "")
-        + ("; also stores its dS tiles for the dQ kernel)" if scratch else ")"),
-        flops, ms, n, profile_figure(HBM_COUNTERS, f"{cfg.name}.dkdv_traffic_bytes_per_launch"), "profiles/" + HBM_COUNTERS)  # fmt: skip
-    out["ds_handover_scratch_bytes_per_ring_step"] = handover_scratch_bytes(cfg, dev)
+    if scratch:
+        ms, flops, n, _ = dominant_dkdv(torch, cfg, dev, o, lse, steps)
+        slabs = n // len(noncausal_steps(cfg))
+        kernel = ("attn_bwd_dkdv_d128_kernel<non-causal> (S, dP, dV, dK of one ring step" + (f", one of {slabs} kv-head slabs per launch" if slabs > 1 else "")
+                  + "; also stores its dS tiles for the dQ kernel)")  # fmt: skip
+        traffic = f"{cfg.name}.dkdv_traffic_bytes_per_launch"
+    else:
+        ms, flops, n = share_backward(torch, cfg, dev, o, lse, steps)
+        kernel = f"attn_bwd_pair_chunks_kernel<{cfg.dqk}> (dK/dV and dQ of all chunks in one grid, with the delta launch before it)"
+        traffic = f"{cfg.name}.bwd_traffic_bytes_per_launch"
+    out["roofline"] = roofline_entry(kernel, flops, ms, n, profile_figure(HBM_COUNTERS, traffic), "profiles/" + HBM_COUNTERS)
+    out["ds_handover_scratch_bytes_per_ring_step"] = scratch
     del dev, o, lse
     torch.cuda.empty_cache()
     if cpu_heads is not None:
@@ -595,7 +599,7 @@ def main():
         print("counter pass done")
         return
     ms_dkdv, dkdv_flops, dkdv_n, scratch = dominant_dkdv(torch, QWEN3, dev_inputs, out, lse, args.steps)
-    ms_fwdk, fwdk_flops, fwdk_n = dominant_fwd(torch, QWEN3, dev_inputs, args.steps)
+    ms_fwdk, fwdk_flops, fwdk_n = share_forward(torch, QWEN3, dev_inputs, args.steps)
     handover_on = scratch > 0
     scratch = handover_scratch_bytes(QWEN3, dev_inputs)
     recompute = None
@@ -648,18 +652,18 @@ def main():
         "data": "synthetic",
         "config": {
             "workload": "GQA ring share fwd+bwd: 32 q / 4 kv heads, head dim 128, S=32768 as 4 zigzag chunks of "
-                        "8192 looped locally (rank 1), B=1, incl. log2 combines and delta",
+                        "8192 looped locally (rank 1), B=1, incl. log2 merges and delta",
             "layout": LAYOUT, "cp_size": CP, "cp_rank": RANK, "s_local": S_LOCAL,
         },  # fmt: skip
         "frac_mfma_peak": round(tflops / MFMA_BF16_PEAK_TFLOPS, 4),
         "fwd": {"ms": round(ms_fwd, 4), "tflops": round(fwd_flops / (ms_fwd * 1e-3) / 1e12, 2)},
         "bwd": {"ms": round(ms_bwd, 4), "tflops": round(bwd_flops / (ms_bwd * 1e-3) / 1e12, 2)},
         "fwd_only": {
-            "workload": "the same share, forward only (4 chunk-attention launches and the log2 merges): O and the base-2 LSE",
+            "workload": "the same share, forward only (one launch over its four chunks): O and the base-2 LSE",
             "ms": round(ms_fwd, 4), "tflops": round(fwd_flops / (ms_fwd * 1e-3) / 1e12, 2),
             "frac_mfma_peak": round(fwd_flops / (ms_fwd * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
             "roofline": roofline_entry(
-                "attn_fwd_direct_kernel<128, non-causal> (S, P, O of one ring step)", fwdk_flops, ms_fwdk, fwdk_n,
+                "attn_fwd_direct_kernel<128, several chunks> (S, P, O of the whole share)", fwdk_flops, ms_fwdk, fwdk_n,
                 profile_figure(HBM_COUNTERS, "qwen3-32k.fwd_traffic_bytes_per_launch"), "profiles/" + HBM_COUNTERS),
             "cpu_baseline": fwd_cpu,
         },  # fmt: skip
