@@ -42,7 +42,12 @@ namespace {
 //   ring shares, 4 ranks, zigzag: d192 4096 rows x 16 rank 0 / 3    416 / 323   367 / 342   385 / 330   530 / 460
 //                                      2048 rows x 16 rank 0 / 2    180 / 136   142 / 113   149 / 117   130 / 121
 //                                 d128 4096 rows x 8/2 rank 0       281         218         239         195
-// (d192 FULL never won: the register budget of 256 rows forced a tile maximum into every softmax.)
+// No FULL at 192 features: its register budget left no room for the row-sum test of the running maximum. Such a kernel, ms,
+// against DUO, tiles from memory; the two are within what one machine differs from the next (32768 x 128 on three of them:
+// 36.0 / 36.4, 35.6 / 35.2, 35.7 / 37.4), and shorter streams are DUO's:
+//   causal   32768 x 128 heads 36.0 / 36.4   x 120 33.9 / 33.3   x 64 18.1 / 17.9   x 16 4.58 / 4.53   16384 x 64  4.67 / 4.59
+//            8192 x 128        2.59 / 2.39   x 16  0.345 / 0.298                    4096 x 128 0.692 / 0.663
+//   full     32768 x 16        8.89 / 8.96   16384 x 64 8.91 / 9.05   8192 x 128 4.87 / 4.58   x 16 0.565 / 0.567   4096 x 128 1.24 / 1.17
 enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter };
 
 // `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50).

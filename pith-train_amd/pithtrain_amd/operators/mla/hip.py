@@ -197,8 +197,9 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
     args.ds, args.ds_bytes = ds.data_ptr(), ds.numel()
 
 
-# The dS hand-over (head dims 128/128) makes the backward of a chunk pair 3-5 % faster at the price of a
-# transient buffer of Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask).
+# The dS hand-over (head dims 128/128) makes the backward of a chunk pair 1-5 % faster (share of 8192 rows, 32/4 heads,
+# four ranks: 6.15 -> 5.92 ms; the gain differs between machines) at the price of a transient buffer of
+# Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask).
 # Policy: the buffer never exceeds DS_BUFFER_LIMIT_BYTES nor DS_BUFFER_FREE_FRACTION of the device memory that is
 # free right now; a chunk pair that needs more is processed one group of kv heads (with their query heads) after
 # the other through one buffer of the bounded size; when not even one kv head fits, or the allocation fails, the

@@ -357,8 +357,8 @@ class RingBackward:
 
 def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunks) -> bool:
     """Whether some step of the share would hand dS from its dK/dV to its dQ kernel: 5 matrix products instead of 7, which is
-    worth more than one launch over all chunks saves (8192 rows x 32 heads, four ranks: 6.1 ms in steps, 6.6 ms in one launch;
-    4096 rows: 1645 and 1705 us)."""
+    worth more than one launch over all chunks saves (8192 rows x 32/4 heads, four ranks: 5.9 ms handing over, 6.2 ms recomputing
+    in steps, 6.7 ms in one launch; 4096 rows: 1645 us handing over, 1705 us in one launch)."""
     if q.shape[-1] != 128:
         return False
     return any(
