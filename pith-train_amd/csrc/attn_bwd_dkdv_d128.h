@@ -37,7 +37,8 @@ constexpr int kTile = kBM * kRowBytes128;        // 16 KB
 constexpr int kStat = 2 * kBM * 4;               // lse[64], delta[64]
 constexpr int kStage = 2 * kTile + kStat;        // Q tile, dO tile, stats
 constexpr int kExchPair = kBM * 32 * 4;          // one 64 x 32 fp32 P tile
-constexpr int kSmem = kStages * kStage + 4 * kExchPair;
+constexpr int kTurn = 8 * kRowsViaLdsBytes<kD / 32>;  // the epilogue's use of it
+constexpr int kSmem = kStages * kStage + 4 * kExchPair > kTurn ? kStages * kStage + 4 * kExchPair : kTurn;
 // dS hand-over: vector-memory stores a B wave issues per interval (one 16-byte store per lane and 16-row step of
 // the 64-row tile). The wait that ends an interval lets exactly this many operations stay in flight, which is
 // right only while they are the LAST vector-memory operations the wave issued (tests/test_cabi.py checks that on
@@ -137,23 +138,13 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     }
     req.advance(m_first, m_end, hq0, hq_end);
   };
-  if (n_iter > 0 && role_b) request(smem);
-
-  // stationary fragments: K rows for wave A, V rows for wave B
+  // stationary fragments: K rows for wave A, V rows for wave B, each wave's staged in ring stages 1 and 2
   bf16x8 stat[KS];
-  {
-    const int row = key < p.Skv ? key : p.Skv - 1;
-    const __bf16* src = (role_b ? p.v + b * p.v_bs : p.k + b * p.k_bs) + row * kv_row_stride + (int64_t)hk * kD + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) stat[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    if (role_b) {
-      // wave B works with -V: its score-type product then starts from delta and yields delta - dP,
-      // i.e. -(dP - delta) without a subtraction per element; the sign is undone with the factor
-      // -scale on the accumulated dK (and by the reader of the dS images)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) stat[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, stat[ks]) ^ 0x80008000u);
-    }
-  }
+  static_assert(8 * 8192 <= (kStages - 1) * kStage, "areas of the stationary rows");
+  char* const stat_area = smem + kStage + wave * 8192;
+  stage_rows32<true>(reinterpret_cast<const char*>((role_b ? p.v + b * p.v_bs : p.k + b * p.k_bs) + (int64_t)hk * kD), kv_pair0, p.Skv,
+                     (int)(kv_row_stride * 2), stat_area, lane);
+  if (n_iter > 0 && role_b) request(smem);
   f32x16 acc[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i)
@@ -338,7 +329,16 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     }
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // everything issued so far: tile 0, stationary fragments
+  wait_staged();  // everything issued so far: tile 0, stationary rows
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) stat[ks] = staged_fragment<true>(stat_area, ks, c, g);
+  if (role_b) {
+    // wave B works with -V: its score-type product then starts from delta and yields delta - dP,
+    // i.e. -(dP - delta) without a subtraction per element; the sign is undone with the factor
+    // -scale on the accumulated dK (and by the reader of the dS images)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) stat[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, stat[ks]) ^ 0x80008000u);
+  }
   __syncthreads();
 
   // Interval i = 0 .. n_iter touches tiles i-1 and i; tile -1 and tile n_iter do not exist, so the
@@ -407,33 +407,20 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     else run(std::true_type{});
   }
 
-  if (role_b) {
-#pragma unroll
-    for (int o = 0; o < DB; ++o)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[o][v] *= -p.scale;  // wave B accumulated -dK / scale
-  }
-  // ---- epilogue: wave A stores dV, wave B stores dK, for key row `key`, features 32*o + 8*b4 + 4*g ..+3
-  if (key < p.Skv) {
-    if (p.split > 1) {
-      // the partials are packed: exactly the Hkv heads of this call per row
-      float* ws = (role_b ? p.ws_dk : p.ws_dv) + (((int64_t)part * p.B + b) * p.Skv + key) * ((int64_t)p.Hkv * kD) + (int64_t)hk * kD;
-#pragma unroll
-      for (int o = 0; o < DB; ++o)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4)
-          store4<float>(ws + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4], acc[o][4 * b4 + 1], acc[o][4 * b4 + 2],
-                        acc[o][4 * b4 + 3], false);
-    } else {
-      OutT* out = reinterpret_cast<OutT*>(role_b ? p.dk : p.dv) + b * (role_b ? p.dk_bs : p.dv_bs) + key * kv_row_stride +
-                  (int64_t)hk * kD;
-#pragma unroll
-      for (int o = 0; o < DB; ++o)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4)
-          store4<OutT>(out + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4], acc[o][4 * b4 + 1], acc[o][4 * b4 + 2],
-                       acc[o][4 * b4 + 3], p.accumulate != 0);
-    }
+  // ---- epilogue: wave A stores dV, wave B stores dK (it accumulated -dK / scale); a lane holds one key row, turned through
+  // LDS so that the stores cover whole rows
+  __syncthreads();  // every wave is done with the ring
+  char* const turn = smem + wave * kRowsViaLdsBytes<DB>;
+  const float factor = role_b ? -p.scale : 1.f;
+  const int rows_valid = p.Skv - kv_pair0;
+  if (p.split > 1) {
+    // the partials are packed: exactly the Hkv heads of this call per row
+    const int64_t row_stride = (int64_t)p.Hkv * kD;
+    float* ws = (role_b ? p.ws_dk : p.ws_dv) + (((int64_t)part * p.B + b) * p.Skv + kv_pair0) * row_stride + (int64_t)hk * kD;
+    store_rows32_via_lds<float, DB>(turn, ws, row_stride, rows_valid, acc, factor, false, lane);
+  } else {
+    OutT* out = reinterpret_cast<OutT*>(role_b ? p.dk : p.dv) + b * (role_b ? p.dk_bs : p.dv_bs) + kv_pair0 * kv_row_stride + (int64_t)hk * kD;
+    store_rows32_via_lds<OutT, DB>(turn, out, kv_row_stride, rows_valid, acc, factor, p.accumulate != 0, lane);
   }
 }
 

@@ -158,28 +158,20 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     }
     req.advance(m_first, m_end);
   };
-  if (n_iter > 0 && role_b) request(smem);
-
-  // stationary fragments: K rows for wave A (12), V rows for wave B (8)
+  // stationary fragments: K rows for wave A (12), V rows for wave B (8), each wave's rows staged in ring stages 1 and 2
   bf16x8 stat[KS];
-  {
-    const int row = key < p.Skv ? key : p.Skv - 1;
-    if (!role_b) {
-      const __bf16* src = p.k + b * p.k_bs + row * k_row_stride + (int64_t)hk * k_head + g * 8;
-      const __bf16* src_pe = two_part ? p.k_pe + b * p.k_pe_bs + row * p.k_pe_rs + g * 8 : src + 128;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        stat[ks] = *reinterpret_cast<const bf16x8*>(ks < 8 ? src + ks * 16 : src_pe + (ks - 8) * 16);
-    } else {
-      const __bf16* src = p.v + b * p.v_bs + row * v_row_stride + (int64_t)hk * kDV + g * 8;
-#pragma unroll
-      for (int ks = 0; ks < VS; ++ks) stat[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-      // wave B works with -V: its score-type product then starts from delta and yields delta - dP,
-      // i.e. -(dP - delta) without a subtraction per element; the factor -scale on the accumulated dK
-      // undoes the sign
-#pragma unroll
-      for (int ks = 0; ks < VS; ++ks) stat[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, stat[ks]) ^ 0x80008000u);
-    }
+  constexpr int kStatPair = 12288 + 8192;  // K, V
+  static_assert(4 * kStatPair <= (kStages - 1) * kStage, "areas of the stationary rows");
+  char* const stat_area = smem + kStage + pair * kStatPair + (role_b ? 12288 : 0);
+  if (!role_b) {
+    const int k_row_bytes = (int)(k_row_stride * 2);
+    const char* const ksrc = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * k_head);
+    stage_rows32<true>(ksrc, kv_pair0, p.Skv, k_row_bytes, stat_area, lane);
+    stage_rows32<false>(two_part ? reinterpret_cast<const char*>(p.k_pe + b * p.k_pe_bs) : ksrc + 256, kv_pair0, p.Skv,
+                        two_part ? (int)p.k_pe_rs * 2 : k_row_bytes, stat_area + 8192, lane);
+  } else {
+    stage_rows32<true>(reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kDV), kv_pair0, p.Skv, (int)(v_row_stride * 2), stat_area, lane);
+    if (n_iter > 0) request(smem);
   }
   f32x16 acc[DB];  // A uses the first DVB of them
 #pragma unroll
@@ -352,7 +344,19 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     }
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // everything issued so far: tile 0, stationary fragments
+  wait_staged();  // everything issued so far: tile 0, stationary rows
+  if (!role_b) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      stat[ks] = ks < 8 ? staged_fragment<true>(stat_area, ks, c, g) : staged_fragment<false>(stat_area + 8192, ks - 8, c, g);
+  } else {
+    // wave B works with -V: its score-type product then starts from delta and yields delta - dP,
+    // i.e. -(dP - delta) without a subtraction per element; the factor -scale on the accumulated dK
+    // undoes the sign
+#pragma unroll
+    for (int ks = 0; ks < VS; ++ks)
+      stat[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, staged_fragment<true>(stat_area, ks, c, g)) ^ 0x80008000u);
+  }
   __syncthreads();
 
   // Interval i = 0 .. n_iter touches tiles i-1 and i; tile -1 and tile n_iter do not exist, so the
@@ -415,42 +419,37 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     else run(std::true_type{});
   }
 
-  // ---- epilogue: wave A stores dV, wave B stores dK (times scale), for key row `key`, features
-  // 32*o + 8*b4 + 4*g ..+3
-  if (key < p.Skv) {
-    const float f = role_b ? -p.scale : 1.f;  // wave B accumulated -dK / scale
-    const int d = role_b ? k_head : kDV;
-    const int nblk = role_b ? k_head / 32 : DVB;
-    const int64_t row_stride = role_b ? k_row_stride : v_row_stride;
-    if (two_part && role_b) {  // this head's gradient of the shared rotary part: [Hkv][B][Skv][64] fp32
-      float* ws = p.ws_dkpe + (((int64_t)hk * p.B + b) * p.Skv + key) * 64;
+  // ---- epilogue: wave A stores dV, wave B stores dK (it accumulated -dK / scale); a lane holds one key row, turned through
+  // LDS so that the stores cover whole rows, 64 features at a time
+  __syncthreads();  // every wave is done with the ring
+  constexpr int NB = 2;
+  char* const turn = smem + wave * kRowsViaLdsBytes<NB>;
+  const int rows_valid = p.Skv - kv_pair0;
+  auto store = [&](auto o0_tag, float factor, float* ws, int64_t ws_stride, OutT* out, int64_t out_stride, bool partial) __attribute__((always_inline)) {
+    constexpr int O0 = decltype(o0_tag)::value;
+    f32x16 part_acc[NB];
 #pragma unroll
-      for (int o = 4; o < DB; ++o)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4)
-          store4<float>(ws + 32 * (o - 4) + 8 * b4 + 4 * g, acc[o][4 * b4] * f, acc[o][4 * b4 + 1] * f, acc[o][4 * b4 + 2] * f,
-                        acc[o][4 * b4 + 3] * f, false);
-    }
-    if (p.split > 1) {
-      // the partials are packed: exactly the Hkv heads of this call per row
-      float* ws = (role_b ? p.ws_dk : p.ws_dv) + (((int64_t)part * p.B + b) * p.Skv + key) * ((int64_t)p.Hkv * d) + (int64_t)hk * d;
-#pragma unroll
-      for (int o = 0; o < DB; ++o)
-        if (o < nblk)
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4)
-            store4<float>(ws + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4] * f, acc[o][4 * b4 + 1] * f, acc[o][4 * b4 + 2] * f,
-                          acc[o][4 * b4 + 3] * f, false);
+    for (int o = 0; o < NB; ++o) part_acc[o] = acc[O0 + o];
+    if (partial) store_rows32_via_lds<float, NB>(turn, ws + 32 * O0, ws_stride, rows_valid, part_acc, factor, false, lane);
+    else store_rows32_via_lds<OutT, NB>(turn, out + 32 * O0, out_stride, rows_valid, part_acc, factor, p.accumulate != 0, lane);
+  };
+  const bool parts = p.split > 1;  // the partials are packed: exactly the Hkv heads of this call per row
+  const int64_t ws_row = ((int64_t)part * p.B + b) * p.Skv + kv_pair0;
+  if (!role_b) {
+    float* const ws = p.ws_dv + ws_row * ((int64_t)p.Hkv * kDV) + (int64_t)hk * kDV;
+    OutT* const out = reinterpret_cast<OutT*>(p.dv) + b * p.dv_bs + kv_pair0 * v_row_stride + (int64_t)hk * kDV;
+    store(std::integral_constant<int, 0>{}, 1.f, ws, (int64_t)p.Hkv * kDV, out, v_row_stride, parts);
+    store(std::integral_constant<int, 2>{}, 1.f, ws, (int64_t)p.Hkv * kDV, out, v_row_stride, parts);
+  } else {
+    float* const ws = p.ws_dk + ws_row * ((int64_t)p.Hkv * k_head) + (int64_t)hk * k_head;
+    OutT* const out = reinterpret_cast<OutT*>(p.dk) + b * p.dk_bs + kv_pair0 * k_row_stride + (int64_t)hk * k_head;
+    store(std::integral_constant<int, 0>{}, -p.scale, ws, (int64_t)p.Hkv * k_head, out, k_row_stride, parts);
+    store(std::integral_constant<int, 2>{}, -p.scale, ws, (int64_t)p.Hkv * k_head, out, k_row_stride, parts);
+    if (two_part) {  // this head's gradient of the shared rotary part: [Hkv][B][Skv][64] fp32
+      float* const pe = p.ws_dkpe + (((int64_t)hk * p.B + b) * p.Skv + kv_pair0) * 64;
+      store(std::integral_constant<int, 4>{}, -p.scale, pe - 128, 64, out, k_row_stride, true);
     } else {
-      OutT* out = reinterpret_cast<OutT*>(role_b ? p.dk : p.dv) + b * (role_b ? p.dk_bs : p.dv_bs) + key * row_stride +
-                  (int64_t)hk * d;
-#pragma unroll
-      for (int o = 0; o < DB; ++o)
-        if (o < nblk)
-#pragma unroll
-          for (int b4 = 0; b4 < 4; ++b4)
-            store4<OutT>(out + 32 * o + 8 * b4 + 4 * g, acc[o][4 * b4] * f, acc[o][4 * b4 + 1] * f, acc[o][4 * b4 + 2] * f,
-                         acc[o][4 * b4 + 3] * f, p.accumulate != 0);
+      store(std::integral_constant<int, 4>{}, -p.scale, ws, (int64_t)p.Hkv * k_head, out, k_row_stride, parts);
     }
   }
 }

@@ -85,22 +85,27 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
       ++req_h;
     }
   };
+  // stationary fragments: K and -V rows as B operands. Every wave stages its own rows in the ring; the first tiles are
+  // requested when all have been read.
+  bf16x8 kf[KS], vf[KS];
+  {
+    static_assert(kWaves * 8192 <= kSmem, "areas of the stationary rows");
+    char* const area = smem + wave * 8192;
+    const int kv_row_bytes = (int)(kv_row_stride * 2);
+    stage_rows32<false>(reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * kD), kv_wave0, p.Skv, kv_row_bytes, area, lane);
+    stage_rows32<false>(reinterpret_cast<const char*>(p.v + b * p.v_bs + (int64_t)hk * kD), kv_wave0, p.Skv, kv_row_bytes, area + 4096, lane);
+    wait_staged();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      kf[ks] = staged_fragment<false>(area, ks, c, g);
+      vf[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, staged_fragment<false>(area + 4096, ks, c, g)) ^ 0x80008000u);
+    }
+    __syncthreads();
+  }
   if (n_iter > 0) request(0);
   if (n_iter > 1) request(1);
   if (n_iter > 2) request(2);
 
-  // stationary fragments: K and -V rows as B operands
-  bf16x8 kf[KS], vf[KS];
-  {
-    const int row = key < p.Skv ? key : p.Skv - 1;
-    const __bf16* ksrc = p.k + b * p.k_bs + row * kv_row_stride + (int64_t)hk * kD + g * 8;
-    const __bf16* vsrc = p.v + b * p.v_bs + row * kv_row_stride + (int64_t)hk * kD + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kf[ks] = *reinterpret_cast<const bf16x8*>(ksrc + ks * 16);
-      vf[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, *reinterpret_cast<const bf16x8*>(vsrc + ks * 16)) ^ 0x80008000u);
-    }
-  }
   f32x16 dk[DB], dv[DB];  // transposed: this lane's key, 32 features per block
 #pragma unroll
   for (int o = 0; o < DB; ++o)
@@ -223,11 +228,15 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     }
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0F70);
+  if (n_iter > 2) wait_staged<2 * kLoads>();
+  else wait_staged();
   __syncthreads();
   if (n_iter > 0) {
     scores(smem);
     make_p_ds(m_first);
+    if (n_iter > 2) wait_staged<kLoads>();
+    else wait_staged();
+    __syncthreads();  // tile 1 is there
     int mt = m_first;
     for (int i = 1; i < n_iter; ++i) {
       if (++mt == m_end) mt = m_first;

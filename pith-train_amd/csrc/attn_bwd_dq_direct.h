@@ -12,14 +12,15 @@
 // waves (4-7) vector then matrix, so that on every SIMD one wave's MFMAs coincide with the other's
 // arithmetic. Q^T and dO^T fragments, lse and delta of a wave's 32 query rows are stationary.
 // A workgroup owns 128 query rows; wave w and w + 4 own the SAME 32 rows, the early wave keys
-// 0-31 and the late wave keys 32-63 of every tile; at the end the late wave hands its partial dQ to
-// the early wave through LDS.
+// 0-31 and the late wave keys 32-63 of every tile; at the end they add up their partial dQ through LDS.
 //
 // With 192-feature queries the stationary fragments alone (Q^T 48 + dO^T 32 registers) push a wave
 // past 256 registers, and spilled fragments are reloaded from scratch memory in every interval. The
 // last four Q^T fragments (features 128..191) and the last four dO^T fragments are therefore kept
 // in LDS (written once, 8 KB per pair of waves) and read as B operands when needed; tiles are
-// requested ONE interval ahead there (K ring of 4, V ring of 2) to make the room.
+// requested ONE interval ahead there (K ring of 4, V ring of 2) to make the room. The tile movers' source
+// offsets are formed anew for every tile: kept across the loop, 6 registers were spilled and reloaded in
+// front of the requests of every interval (4096 x 16 heads causal, with the staged rows: 142 -> 129 us).
 //
 // Why this form: with 192-feature queries a wave that owned all 64 keys of a tile would need more
 // than 256 registers (Q^T 48 + dO^T 32 + dQ 96 + S, dP 64 + dS 16); owning half the keys brings
@@ -116,45 +117,56 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   }
   auto request = [&](int t) __attribute__((always_inline)) {
     char* kslot = kbuf + (t & (kSlots - 1)) * kKTile;
+    char* vslot = vbuf + (t & (kVSlots - 1)) * kTile;
+    const int left = k_src.left(t);
     if constexpr (DQK != kDv) {
-      kmover.issue(k_src.src(t), k_src.left(t), kslot, wave, lane);
-      xmover.issue(kx_src.src(t), k_src.left(t), kslot + kTile, wave, lane);
+      // source offsets formed on the spot: kept across the loop, some end up in scratch memory, and a reload costs each
+      // interval a memory latency (behind the tile loads in flight even those)
+      kmover.issue_clamped(k_src.src(t), left, kslot, wave, lane);
+      xmover.issue_clamped(kx_src.src(t), left, kslot + kTile, wave, lane);
+      mover.issue_clamped(v_src.src(t), left, vslot, wave, lane);
       kx_src.advance(p, range, kx_rows);
     } else {
-      mover.issue(k_src.src(t), k_src.left(t), kslot, wave, lane);
+      mover.issue(k_src.src(t), left, kslot, wave, lane);
+      mover.issue(v_src.src(t), left, vslot, wave, lane);
     }
-    mover.issue(v_src.src(t), k_src.left(t), vbuf + (t & (kVSlots - 1)) * kTile, wave, lane);
     k_src.advance(p, range, k_rows);
     v_src.advance(p, range, v_rows);
   };
-  // tiles of the prologue (0) and of the first kDist intervals
-#pragma unroll
-  for (int t = 0; t <= kDist; ++t)
-    if (t < n_tiles_wg) request(t);
-
-  // stationary side: Q^T and dO^T fragments (B operands), lse and delta of this lane's query row
+  // stationary side: Q^T and dO^T fragments (B operands), lse and delta of this lane's query row. The rows come first: nothing
+  // can start without them. The two waves of a pair share them, Q in K slots 2 and 3 (two pairs each), dO in V slots 2 and 3,
+  // at 192 features in the pair's part of the area for LDS-resident fragments; tiles 0 and 1 are requested behind them.
   constexpr int KSR = KS - kLdsQ, VSR = VS - kLdsDo;  // fragments held in registers
+  constexpr int kQArea = 8192 + (DQK == 192 ? 4096 : 0);
+  static_assert(2 * kQArea <= kKTile && (DQK == 192 ? 8192 <= kStatPair : 2 * 8192 <= kTile), "areas of the query-side rows");
+  char* const q_area = kbuf + (2 + (wave >> 1 & 1)) * kKTile + (wave & 1) * kQArea;
+  char* const do_area = DQK == 192 ? smem + kSlots * kKTile + kVSlots * kTile + (wave & 3) * kStatPair
+                                   : vbuf + (2 + (wave >> 1 & 1)) * kTile + (wave & 1) * 8192;
   bf16x8 qf[KSR], dof[VSR];
   float lse_q, delta_q;
   {
     const int row = qrow < p.Sq ? qrow : p.Sq - 1;
-    const __bf16* src = p.q + b * p.q_bs + (int64_t)h * DQK + row * q_row_stride + g * 8;
-    const __bf16* dsrc = p.dout + b * p.dout_bs + (int64_t)h * kDv + row * do_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KSR; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-#pragma unroll
-    for (int ks = 0; ks < VSR; ++ks) dof[ks] = *reinterpret_cast<const bf16x8*>(dsrc + ks * 16);
-    if (!late) {  // the two waves of a pair hold the same rows: the early one fills the pair's LDS copy
-#pragma unroll
-      for (int ks = 0; ks < kLdsQ; ++ks)
-        *reinterpret_cast<bf16x8*>(const_cast<char*>(stat) + ks * 1024) = *reinterpret_cast<const bf16x8*>(src + (KSR + ks) * 16);
-#pragma unroll
-      for (int ks = 0; ks < kLdsDo; ++ks)
-        *reinterpret_cast<bf16x8*>(const_cast<char*>(stat) + (kLdsQ + ks) * 1024) = *reinterpret_cast<const bf16x8*>(dsrc + (VSR + ks) * 16);
-    }
     lse_q = (p.lse + b * p.lse_bs + (int64_t)h * p.lse_hs)[row];
     delta_q = (p.delta + b * p.lse_bs + (int64_t)h * p.lse_hs)[row];
+    const char* const qsrc = reinterpret_cast<const char*>(p.q + b * p.q_bs + (int64_t)h * DQK);
+    const char* const dsrc = reinterpret_cast<const char*>(p.dout + b * p.dout_bs + (int64_t)h * kDv);
+    const int q_row_bytes = (int)(q_row_stride * 2), do_row_bytes = (int)(do_row_stride * 2);
+    if constexpr (DQK == 192) {
+      if (!late) {
+        stage_rows32<true>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane);
+        stage_rows32<true, 2>(dsrc, q_wave0, p.Sq, do_row_bytes, do_area, lane, 0);
+      } else {
+        stage_rows32<false>(qsrc + 256, q_wave0, p.Sq, q_row_bytes, q_area + 8192, lane);
+        stage_rows32<true, 6>(dsrc, q_wave0, p.Sq, do_row_bytes, do_area, lane, 2);
+      }
+    } else {
+      stage_rows32<true, 4>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane, late ? 4 : 0);
+      stage_rows32<true, 4>(dsrc, q_wave0, p.Sq, do_row_bytes, do_area, lane, late ? 4 : 0);
+    }
   }
+  request(0);
+  if (n_tiles_wg > 1) request(1);
+  constexpr int kTileLoads = 2 * DirectTile128<kBN, kThreads>::kPerThread + (DQK == 192 ? 1 : 0);  // load instructions of a wave per tile
   // B operand of contraction step ks of S / of dP
   auto q_frag = [&](int ks) __attribute__((always_inline)) {
     return ks < KSR ? qf[ks < KSR ? ks : 0] : *reinterpret_cast<const bf16x8*>(stat + (ks - KSR) * 1024);
@@ -348,13 +360,42 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   auto vslot = [&](int t) __attribute__((always_inline)) { return vbuf + (t & (kVSlots - 1)) * kTile; };
 
   // ---- prologue: S(0), dP(0) (and dS(0) in the early waves)
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // everything issued so far, the stationary fragments included
-  __syncthreads();
+  if (n_tiles_wg > 1) wait_staged<kTileLoads>();
+  else wait_staged();
+  __syncthreads();  // the query-side rows and tile 0 are there
+  auto q_row_frag = [&](int ks) __attribute__((always_inline)) {
+    return ks < 8 ? staged_fragment<true>(q_area, ks, c, g) : staged_fragment<false>(q_area + 8192, ks - 8, c, g);
+  };
+#pragma unroll
+  for (int ks = 0; ks < KSR; ++ks) qf[ks] = q_row_frag(ks);
+#pragma unroll
+  for (int ks = 0; ks < VSR; ++ks) dof[ks] = staged_fragment<true>(do_area, ks, c, g);
+  if constexpr (kLdsQ > 0) {  // the early wave fills the pair's LDS-resident fragments, where the dO rows were
+    bf16x8 qt[kLdsQ], dt[kLdsDo];
+#pragma unroll
+    for (int ks = 0; ks < kLdsQ; ++ks) qt[ks] = q_row_frag(KSR + ks);
+#pragma unroll
+    for (int ks = 0; ks < kLdsDo; ++ks) dt[ks] = staged_fragment<true>(do_area, VSR + ks, c, g);
+    __syncthreads();
+    if (!late) {
+#pragma unroll
+      for (int ks = 0; ks < kLdsQ; ++ks) *reinterpret_cast<bf16x8*>(const_cast<char*>(stat) + ks * 1024) = qt[ks];
+#pragma unroll
+      for (int ks = 0; ks < kLdsDo; ++ks) *reinterpret_cast<bf16x8*>(const_cast<char*>(stat) + (kLdsQ + ks) * 1024) = dt[ks];
+    }
+    wait_staged();
+    __syncthreads();  // tile 1 is there as well
+  }
   scores(kslot(0), vslot(0));
   if (!late) make_ds(0, std::true_type{});
+  if constexpr (kLdsQ == 0) {
+    wait_staged();
+    __syncthreads();  // tile 1 is there, the query-side rows have been read
+  }
+  if (kDist > 1 && n_tiles_wg > 2) request(2);
 
   // Interval i = 0 .. n_tiles_wg - 1 reads K(i) (gradient product), K(i+1) and V(i+1) (scores) and
-  // requests tile i + 1 + kDist, whose slots were last read in interval i - 1 (kDist 2: they held
+  // requests tile i + 1 + kDist (kDist 2: tile 2 has been, above), whose slots were last read in interval i - 1 (kDist 2: they held
   // tile i - 1) or hold nothing that is still needed (kDist 1: K slot of tile i - 2, V slot of tile i,
   // read in interval i - 1).
   // FULL: this wave has both a tile to accumulate and a next tile to score.
@@ -401,14 +442,47 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
     for (; i < n_tiles_wg; ++i) interval(i, yes, no, yes);
   }
 
-  // ---- the late wave of a pair hands its partial dQ to the early wave (the tile ring is free: every
-  // wave passed the barrier that ends the last interval)
-  // one area per wave pair; with 128 features it is used twice: for the late wave's partial dQ, then to turn the
-  // early wave's result tile (the 192-feature kernel keeps the direct stores: it has no register to spare, and any
-  // longer epilogue pushes spills into its main loop)
-  constexpr bool kTurn = DQK == 128;
-  constexpr int kExch = kTurn ? kRowsViaLdsBytes<DB> : DB * 4 * 64 * 16;
-  static_assert(kExch >= DB * 4 * 64 * 16 && 4 * kExch <= kSmem<DQK>, "exchange area");
+  // ---- epilogue: the two waves of a pair hold partial sums of the same rows; the tile ring is free (every wave passed the
+  // barrier that ends the last interval)
+  if constexpr (DQK == 128) {
+    // each hands its partner half of the feature blocks, adds up the other half, turns it through LDS and stores whole rows
+    constexpr int NB = DB / 2, kExch = kRowsViaLdsBytes<NB>;  // what a wave has read from its area leaves the area to its rows
+    static_assert(kExch >= NB * 4 * 64 * 16 && kWaves * kExch <= kSmem<DQK>, "exchange area");
+    auto finish = [&](auto late_tag) __attribute__((always_inline)) {
+      constexpr int MINE = decltype(late_tag)::value ? NB : 0, THEIRS = NB - MINE;
+      char* const mine = smem + wave * kExch;
+      char* const theirs = smem + (wave ^ (kWaves / 2)) * kExch;
+#pragma unroll
+      for (int o = 0; o < NB; ++o)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x16& x = acc[THEIRS + o];
+          *reinterpret_cast<f32x4*>(theirs + ((o * 4 + b4) * 64 + lane) * 16) = f32x4{x[4 * b4], x[4 * b4 + 1], x[4 * b4 + 2], x[4 * b4 + 3]};
+        }
+      __syncthreads();
+      f32x16 part[NB];
+#pragma unroll
+      for (int o = 0; o < NB; ++o)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x4 v4 = *reinterpret_cast<const f32x4*>(mine + ((o * 4 + b4) * 64 + lane) * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[o][4 * b4 + e] = acc[MINE + o][4 * b4 + e] + v4[e];
+        }
+      const int64_t at = (int64_t)h * DQK + q_wave0 * q_row_stride + 32 * MINE;
+      __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
+      if (p.dq_final != nullptr && q_wave0 >= p.final_r0 && q_wave0 < p.final_r1) fin = p.dq_final + b * p.dq_final_bs + at;
+      store_rows32_via_lds<OutT, NB>(mine, reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + at, q_row_stride, p.Sq - q_wave0, part, p.scale,
+                                     p.accumulate_dq != 0, lane, fin);
+    };
+    if (!late) finish(std::false_type{});
+    else finish(std::true_type{});
+    return;
+  }
+  // 192 features: the late wave hands over everything and the early one stores from the accumulators. There is no register to
+  // spare, and any longer epilogue pushes spills into the main loop (the form above: 13-26 of them).
+  constexpr int kExch = DB * 4 * 64 * 16;
+  static_assert(4 * kExch <= kSmem<DQK>, "exchange area");
   char* const exch = smem + (wave & 3) * kExch;
   if (late) {
 #pragma unroll
@@ -421,25 +495,8 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   }
   __syncthreads();
   if (late) return;
-
-  OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK;
-  if constexpr (kTurn) {
-    // the pair's dQ^T (a lane owns one query row) is turned through LDS - the same area, once the partner's values
-    // are in registers - so that the epilogue reads and writes whole rows
-#pragma unroll
-    for (int o = 0; o < DB; ++o)
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        const f32x4 v4 = *reinterpret_cast<const f32x4*>(exch + ((o * 4 + b4) * 64 + lane) * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[o][4 * b4 + e] += v4[e];
-      }
-    __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
-    if (p.dq_final != nullptr && q_wave0 >= p.final_r0 && q_wave0 < p.final_r1)
-      fin = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + q_wave0 * q_row_stride;
-    store_rows32_via_lds<OutT, DB>(exch, dqh + q_wave0 * q_row_stride, q_row_stride, p.Sq - q_wave0, acc, p.scale, p.accumulate_dq != 0, lane, fin);
-  } else if (qrow < p.Sq) {
-    OutT* dst = dqh + qrow * q_row_stride;
+  if (qrow < p.Sq) {
+    OutT* dst = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK + qrow * q_row_stride;
     // rows whose gradient is complete with this call go out as bf16 (an fp32 dq only; the same for the whole wave)
     const bool fin = sizeof(OutT) == 4 && p.dq_final != nullptr && q_wave0 >= p.final_r0 && q_wave0 < p.final_r1;
     __bf16* fdst = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + qrow * q_row_stride;

@@ -120,24 +120,35 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
     k_src.advance(p, range, k_rows);
     v_src.advance(p, range, v_rows);
   };
-  request(0);
-  if (n_wg > 1) request(1);
-  if (n_wg > 2) request(2);
-
-  // stationary B operands (column = query row), lse and delta of this lane's row
+  // stationary B operands (column = query row), lse and delta of this lane's row. Every wave stages its own rows in the rings,
+  // which they fill exactly; the first tiles are requested when all have been read.
   bf16x8 qf[KS], dof[VS];
   float lse_q, delta_q;
   {
+    constexpr int kQArea = kPaired ? 4096 : 8192 + (DQK == 192 ? 4096 : 0), kDoArea = kPaired ? 4096 : 8192;
+    static_assert(kWaves * (kQArea + kDoArea) <= L::kSmem, "areas of the query-side rows");
+    char* const q_area = smem + wave * (kQArea + kDoArea);
+    char* const do_area = q_area + kQArea;
     const int row = qrow < p.Sq ? qrow : p.Sq - 1;
-    const __bf16* src = p.q + b * p.q_bs + (int64_t)h * DQK + row * q_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-    const __bf16* dsrc = p.dout + b * p.dout_bs + (int64_t)h * kDv + row * do_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < VS; ++ks) dof[ks] = *reinterpret_cast<const bf16x8*>(dsrc + ks * 16);
     lse_q = p.lse[b * p.lse_bs + (int64_t)h * p.lse_hs + row];
     delta_q = p.delta[b * p.lse_bs + (int64_t)h * p.lse_hs + row];
+    const char* const qsrc = reinterpret_cast<const char*>(p.q + b * p.q_bs + (int64_t)h * DQK);
+    const char* const dsrc = reinterpret_cast<const char*>(p.dout + b * p.dout_bs + (int64_t)h * kDv);
+    const int q_row_bytes = (int)(q_row_stride * 2), do_row_bytes = (int)(do_row_stride * 2);
+    stage_rows32<!kPaired>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane);
+    if constexpr (DQK == 192) stage_rows32<false>(qsrc + 256, q_wave0, p.Sq, q_row_bytes, q_area + 8192, lane);
+    stage_rows32<!kPaired>(dsrc, q_wave0, p.Sq, do_row_bytes, do_area, lane);
+    wait_staged();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = ks < 8 ? staged_fragment<!kPaired>(q_area, ks, c, g) : staged_fragment<false>(q_area + 8192, ks - 8, c, g);
+#pragma unroll
+    for (int ks = 0; ks < VS; ++ks) dof[ks] = staged_fragment<!kPaired>(do_area, ks, c, g);
+    __syncthreads();
   }
+  request(0);
+  if (n_wg > 1) request(1);
+  if (n_wg > 2) request(2);
 
   // per-lane read offsets. Straight fragment of the tile's 32 keys, contraction step ks; transposed fragment of keys
   // 16j..16j+15, feature block i. A 64-feature tile holds key r in pieces 0-7 and key r + 16 in pieces 8-15 of LDS row r.
@@ -250,10 +261,14 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
       dsf[j] = to_bf16x8(s[8 * j], s[8 * j + 1], s[8 * j + 2], s[8 * j + 3], s[8 * j + 4], s[8 * j + 5], s[8 * j + 6], s[8 * j + 7]);
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0F70);
+  if (n_wg > 2) wait_staged<2 * L::kLoads>();
+  else wait_staged();
   __syncthreads();
   scores(kbuf, vbuf);
   make_ds(0);
+  if (n_wg > 2) wait_staged<L::kLoads>();
+  else wait_staged();
+  __syncthreads();  // tile 1 is there
 
   int i = 1;
   for (; i < n_wave; ++i) {

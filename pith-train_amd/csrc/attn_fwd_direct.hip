@@ -51,8 +51,9 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
   constexpr int kBM = HALF ? 128 : 256;      // query rows per workgroup
   constexpr int kKTile = kTile + (DQK == 192 ? kExtraTile : 0);
   static_assert(DQK == 128 || (DQK == 192 && HALF), "head dims");
-  // the tile rings; the epilogue reuses them to turn the output tile (one area per storing wave)
-  constexpr int kRings = kSlots * (kKTile + kTile), kTurn = (HALF ? kWaves / 2 : kWaves) * kRowsViaLdsBytes<DVB>;
+  // the tile rings; the epilogue reuses them to turn the output tile (one area per wave, which stores half of the features
+  // of its rows with HALF)
+  constexpr int kRings = kSlots * (kKTile + kTile), kTurn = kWaves * kRowsViaLdsBytes<HALF ? DVB / 2 : DVB>;
   // 256-row workgroups for 128 features fetch their query block through LDS as well (four 64-row tiles into the three
   // ring slots that are still empty while the first tiles land, and one more tile behind the rings): whole-row direct
   // loads instead of 32-byte pieces of 32 different rows per instruction
@@ -130,20 +131,16 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
     mover.issue(v_src.src(t), v_src.left(t), vbuf + (t & (kSlots - 1)) * kTile, wave, lane);
     v_src.advance(p, range, v_rows);
   };
-  // tiles needed by the prologue (K 0), interval 0 (K 1, V 0) and interval 1 (K 2, V 1)
-  issue_k(0);
-#pragma unroll
-  for (int t = 0; t < kDist; ++t) {
-    if (t + 1 < n_tiles_wg) issue_k(t + 1);
-    if (t < n_tiles_wg) issue_v(t);
-  }
-
-  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features.
-  bf16x8 qf[KS];
-  // LDS homes of the workgroup's four 64-row query tiles (kQViaLds): K slot 3, V slots 2 and 3, behind the rings
+  // Query rows first: nothing can start without them, and the address unit takes the requests of a compute unit in order.
+  // 256-row workgroups: four 64-row tiles in K slot 3, V slots 2 and 3 and behind the rings. 128-row workgroups: per pair of
+  // waves that own the same 32 rows an area in K slot 3 (pairs 0, 1) or V slots 2 and 3 (pairs 2, 3).
+  bf16x8 qf[KS];  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features
+  constexpr int kQArea = 8192 + (DQK == 192 ? 4096 : 0);
+  static_assert(2 * kQArea <= kKTile && 2 * kQArea <= 2 * kTile, "query areas");
   auto q_home = [&](int t) __attribute__((always_inline)) -> char* {
     return t == 0 ? kbuf + 3 * kKTile : t == 1 ? vbuf + 2 * kTile : t == 2 ? vbuf + 3 * kTile : smem + kQSpill;
   };
+  char* const q_area = (wave & 2 ? vbuf + 2 * kTile : kbuf + 3 * kKTile) + (wave & 1) * kQArea;
   if constexpr (kQViaLds) {
     DirectTile128<kBN, kThreads> qmover;
     qmover.init((int)(q_row_stride * 2), wave, lane);
@@ -151,16 +148,29 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       // rows beyond Sq repeat the last row (their results are never stored); a tile wholly beyond Sq is skipped by
-      // clamping its first row, which keeps the number of load instructions per wave fixed
+      // clamping its first row
       const int row0 = min(m0 + t * kBN, p.Sq - 1);
       qmover.issue(qsrc + (int64_t)row0 * q_row_stride * 2, p.Sq - row0, q_home(t), wave, lane);
     }
   } else {
-    const int row = qrow < p.Sq ? qrow : p.Sq - 1;
-    const __bf16* src = qh + row * q_row_stride + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
+    const char* qsrc = reinterpret_cast<const char*>(qh);
+    const int q_row_bytes = (int)(q_row_stride * 2);
+    if constexpr (DQK == 192) {
+      if (!late) stage_rows32<true>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane);
+      else stage_rows32<false>(qsrc + 256, q_wave0, p.Sq, q_row_bytes, q_area + 8192, lane);
+    } else {
+      stage_rows32<true, 4>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane, late ? 4 : 0);
+    }
   }
+  // tiles needed by the prologue (K 0), interval 0 (K 1, V 0) and interval 1 (K 2, V 1)
+  issue_k(0);
+#pragma unroll
+  for (int t = 0; t < kDist; ++t) {
+    if (t + 1 < n_tiles_wg) issue_k(t + 1);
+    if (t < n_tiles_wg) issue_v(t);
+  }
+  // load instructions of a wave behind K tile 0 when all of these tiles exist
+  constexpr int kLaterLoads = kDist * (2 * DirectTile128<kBN, kThreads>::kPerThread + (DQK == 192 ? 1 : 0));
 
   // per-lane read offsets inside a tile. The swizzle is an XOR, so every offset is one base XOR a constant; only the
   // bases live in registers across the loop (refresh_offsets keeps the compiler from hoisting all derived values
@@ -336,16 +346,23 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
   };
 
   // ---- prologue: S(0) (and P(0) in the early waves) from K tile 0
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // everything issued so far, Q fragments included
+  // Q and K tile 0 have landed; the tiles behind them follow while S(0) is formed
+  if (n_tiles_wg > kDist) wait_staged<kLaterLoads>();
+  else wait_staged();
   __syncthreads();
   if constexpr (kQViaLds) {
     // this wave's 32 rows: tile wave / 2, row block wave % 2 (the slots are refilled only after the next barrier)
     const char* qt = q_home(wave >> 1) + (wave & 1) * 32 * kRowBytes128;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qt + straight_offset128(c, 2 * ks + g));
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = ks < 8 ? staged_fragment<true>(q_area, ks, c, g) : staged_fragment<false>(q_area + 8192, ks - 8, c, g);
   }
   scores(kbuf);
-  __syncthreads();  // K tile 0 has been read by every wave: its slot may be refilled
+  wait_staged();
+  __syncthreads();  // K tile 0 has been read by every wave: its slot may be refilled; K 1, V 0 and what else is needed first is there
   if (!late) softmax(0);
 
   // One interval; FULL: this wave has both a tile to accumulate and a next tile to score.
@@ -429,79 +446,94 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
   if (!late) run(std::false_type{});
   else run(std::true_type{});
 
-  // ---- HALF: the late wave of a pair hands its accumulator, maximum and sum to the early wave,
-  // which rescales both to the common maximum and adds them. The tile ring is free by now (every
-  // wave passed the barrier that ends the last interval).
-  if constexpr (HALF) {
-    constexpr int kExch = 16 * 64 * 16 + 64 * 8;  // 64 accumulator values and (m, l) per lane
-    char* const exch = smem + (wave & 3) * kExch;
-    if (late) {
-#pragma unroll
-      for (int i = 0; i < DVB; ++i)
-#pragma unroll
-        for (int b4 = 0; b4 < 4; ++b4) {
-          const f32x4 v4 = {oacc[i][4 * b4], oacc[i][4 * b4 + 1], oacc[i][4 * b4 + 2], oacc[i][4 * b4 + 3]};
-          *reinterpret_cast<f32x4*>(exch + ((i * 4 + b4) * 64 + lane) * 16) = v4;
-        }
-      const f32x2 ml = {m_run, l_run};
-      *reinterpret_cast<f32x2*>(exch + 16 * 64 * 16 + lane * 8) = ml;
-    }
-    __syncthreads();
-    if (late) return;
-    const f32x2 ml = *reinterpret_cast<const f32x2*>(exch + 16 * 64 * 16 + lane * 8);
-    const float m_new = fmaxf(m_run, ml[0]);
-    // a side that saw no key has m = -inf, l = 0 and a zero accumulator: weight 0
-    const float a_e = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
-    const float a_l = (ml[0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((ml[0] - m_new) * p.kappa);
-    m_run = m_new;
-    l_run = l_run * a_e + ml[1] * a_l;
-#pragma unroll
-    for (int i = 0; i < DVB; ++i)
-#pragma unroll
-      for (int b4 = 0; b4 < 4; ++b4) {
-        const f32x4 v4 = *reinterpret_cast<const f32x4*>(exch + ((i * 4 + b4) * 64 + lane) * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) oacc[i][4 * b4 + e] = oacc[i][4 * b4 + e] * a_e + v4[e] * a_l;
-      }
-  }
-
-  // ---- epilogue: normalise, store O (bf16) and LSE2
+  // ---- epilogue: normalise, store O (bf16) and LSE2, feature blocks [B0, B0 + NB) of this wave's rows. The tile rings are
+  // free by now (every wave passed the barrier that ends the last interval).
   __bf16* oh = p.o + b * p.o_bs + (int64_t)h * kDv;
   float* lse = p.lse + b * p.lse_bs + (int64_t)h * p.lse_hs;
-  const float l = pair_sum(l_run);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  if constexpr (!CAUSAL) {
-    if (p.prev_o != nullptr) {  // the same for the whole launch
-      // ---- merging epilogue: the ring's log2-domain online-softmax combine of this chunk's (O, LSE2) with the running
-      // (prev_o, lse) of the rows: M = max(l1, l2), w = 2^(l - M), out = (w1 o1 + w2 o2) / (w1 + w2),
-      // lse = M + log2(w1 + w2). The chunk's O is acc / l, so its weight and 1 / l fold into one factor per row.
-      const float lse_new = l > 0.f ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
-      const float lse_old = qrow < p.Sq ? lse[qrow] : -INFINITY;
-      const float big = fmaxf(lse_old, lse_new);
-      // both sides empty (-inf): weights 0, result (0, -inf); the ring never gets there (it starts from finfo.min)
-      const float w_old = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_old - big);
-      const float w_new = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_new - big);
-      const float den = w_old + w_new;
-      const float rden = den > 0.f ? 1.f / den : 0.f;
-      char* const turn = smem + (HALF ? (wave & 3) : wave) * kRowsViaLdsBytes<DVB>;
-      const int64_t prev_rs = o_row_stride;  // the three tensors share the [.., Hq, 128] row layout
-      const char* prev = reinterpret_cast<const char*>(p.prev_o) +
-                         (b * p.prev_bs + (int64_t)h * kDv + q_wave0 * prev_rs) * (p.prev_f32 ? 4 : 2);
-      // which of the two outputs this wave's 32 rows go to (the ranges lie on multiples of 32 rows)
-      const bool to_o = p.o && q_wave0 >= p.o_r0 && q_wave0 < p.o_r1;
-      const bool to_acc = p.acc_o && q_wave0 >= p.acc_r0 && q_wave0 < p.acc_r1;
-      merge_rows32_via_lds<DVB>(turn, prev, p.prev_f32 != 0, prev_rs, to_o ? oh + q_wave0 * o_row_stride : nullptr, o_row_stride,
-                                to_acc ? p.acc_o + b * p.acc_bs + (int64_t)h * kDv + q_wave0 * o_row_stride : nullptr,
-                                o_row_stride, p.Sq - q_wave0, oacc, w_new * inv * rden, w_old * rden, lane);
-      if (qrow < p.Sq && g == 0) lse[qrow] = den > 0.f ? big + __builtin_amdgcn_logf(den) : -INFINITY;
-      return;
+  const bool merging = !CAUSAL && p.prev_o != nullptr;  // the same for the whole launch
+  float lse_old = -INFINITY;
+  if (merging && qrow < p.Sq) lse_old = lse[qrow];
+  auto finish = [&](auto b0_tag, auto nb_tag, char* turn) __attribute__((always_inline)) {
+    constexpr int B0 = decltype(b0_tag)::value, NB = decltype(nb_tag)::value;
+    f32x16 part[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) part[i] = oacc[B0 + i];
+    const float l = pair_sum(l_run);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    __bf16* const rows = oh + q_wave0 * o_row_stride + 32 * B0;
+    if constexpr (!CAUSAL) {
+      if (merging) {
+        // ---- merging epilogue: the ring's log2-domain online-softmax combine of this chunk's (O, LSE2) with the running
+        // (prev_o, lse) of the rows: M = max(l1, l2), w = 2^(l - M), out = (w1 o1 + w2 o2) / (w1 + w2),
+        // lse = M + log2(w1 + w2). The chunk's O is acc / l, so its weight and 1 / l fold into one factor per row.
+        const float lse_new = l > 0.f ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
+        const float big = fmaxf(lse_old, lse_new);
+        // both sides empty (-inf): weights 0, result (0, -inf); the ring never gets there (it starts from finfo.min)
+        const float w_old = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_old - big);
+        const float w_new = big == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse_new - big);
+        const float den = w_old + w_new;
+        const float rden = den > 0.f ? 1.f / den : 0.f;
+        const int64_t prev_rs = o_row_stride;  // the three tensors share the [.., Hq, 128] row layout
+        const char* prev = reinterpret_cast<const char*>(p.prev_o) +
+                           (b * p.prev_bs + (int64_t)h * kDv + q_wave0 * prev_rs + 32 * B0) * (p.prev_f32 ? 4 : 2);
+        // which of the two outputs this wave's 32 rows go to (the ranges lie on multiples of 32 rows)
+        const bool to_o = p.o && q_wave0 >= p.o_r0 && q_wave0 < p.o_r1;
+        const bool to_acc = p.acc_o && q_wave0 >= p.acc_r0 && q_wave0 < p.acc_r1;
+        merge_rows32_via_lds<NB>(turn, prev, p.prev_f32 != 0, prev_rs, to_o ? rows : nullptr, o_row_stride,
+                                 to_acc ? p.acc_o + b * p.acc_bs + (int64_t)h * kDv + q_wave0 * o_row_stride + 32 * B0 : nullptr,
+                                 o_row_stride, p.Sq - q_wave0, part, w_new * inv * rden, w_old * rden, lane);
+        if (B0 == 0 && qrow < p.Sq && g == 0) lse[qrow] = den > 0.f ? big + __builtin_amdgcn_logf(den) : -INFINITY;
+        return;
+      }
     }
+    // O^T sits in the accumulators (a lane owns one query row): turned through LDS so that the stores cover whole rows
+    store_rows32_via_lds<__bf16, NB>(turn, rows, o_row_stride, p.Sq - q_wave0, part, inv, false, lane);
+    if (B0 == 0 && qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
+  };
+
+  if constexpr (HALF) {
+    // The two waves of a pair hold partial results of the same rows: each hands its partner half of the feature blocks,
+    // with its maximum and sum, and merges and stores the other half (one wave doing it all took twice as long: 2.4 us of
+    // an epilogue, while its partner had left).
+    constexpr int NB = DVB / 2;
+    constexpr int kExch = NB * 4 * 64 * 16 + 64 * 8;  // accumulator values and (m, l) per lane
+    static_assert(kExch == kRowsViaLdsBytes<NB>, "what a wave has read from its area leaves the area to its output rows");
+    auto exchange = [&](auto late_tag) __attribute__((always_inline)) {
+      constexpr int MINE = decltype(late_tag)::value ? NB : 0, THEIRS = NB - MINE;
+      char* const mine = smem + wave * kExch;
+      char* const theirs = smem + (wave ^ (kWaves / 2)) * kExch;
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x16& x = oacc[THEIRS + i];
+          *reinterpret_cast<f32x4*>(theirs + ((i * 4 + b4) * 64 + lane) * 16) = f32x4{x[4 * b4], x[4 * b4 + 1], x[4 * b4 + 2], x[4 * b4 + 3]};
+        }
+      *reinterpret_cast<f32x2*>(theirs + NB * 4 * 64 * 16 + lane * 8) = f32x2{m_run, l_run};
+      __syncthreads();  // (the old LSE of the rows, if any, has been read by both waves before either writes the new one)
+      const f32x2 ml = *reinterpret_cast<const f32x2*>(mine + NB * 4 * 64 * 16 + lane * 8);
+      const float m_new = fmaxf(m_run, ml[0]);
+      // a side that saw no key has m = -inf, l = 0 and a zero accumulator: weight 0
+      const float w = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.kappa);
+      const float w_other = (ml[0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((ml[0] - m_new) * p.kappa);
+      m_run = m_new;
+      l_run = l_run * w + ml[1] * w_other;
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int b4 = 0; b4 < 4; ++b4) {
+          const f32x4 v4 = *reinterpret_cast<const f32x4*>(mine + ((i * 4 + b4) * 64 + lane) * 16);
+          f32x16& x = oacc[MINE + i];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[4 * b4 + e] = x[4 * b4 + e] * w + v4[e] * w_other;
+        }
+      finish(std::integral_constant<int, MINE>{}, std::integral_constant<int, NB>{}, mine);
+    };
+    if (!late) exchange(std::false_type{});
+    else exchange(std::true_type{});
+  } else {
+    finish(std::integral_constant<int, 0>{}, std::integral_constant<int, DVB>{}, smem + wave * kRowsViaLdsBytes<DVB>);
   }
-  // O^T sits in the accumulators (a lane owns one query row): turned through LDS so that the stores
-  // cover whole rows. Every wave is past the barrier behind the last tile read (HALF: past the merge).
-  char* const turn = smem + (HALF ? (wave & 3) : wave) * kRowsViaLdsBytes<DVB>;
-  store_rows32_via_lds<__bf16, DVB>(turn, oh + q_wave0 * o_row_stride, o_row_stride, p.Sq - q_wave0, oacc, inv, false, lane);
-  if (qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
 }
 
 template <int DQK, bool HALF, bool MULTI>

@@ -149,20 +149,42 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     else vmover.issue(v_src.src(at), v_src.left(at), slot, wave, lane);
     for (int n = 0; n < kTeams; ++n) v_src.advance(p, range, v_rows);
   };
+  // Query rows first: nothing can start without them. PARTS = 1: every wave stages its own in slots of tiles that are requested
+  // behind them (K 1 and V 1, two waves each; at 192 features the fourth wave takes V 0). Several parts: the waves of a row
+  // block share the loads and an area in the V 1 slots.
+  constexpr int kQArea = kPaired ? 4096 : 8192 + (DQK == 192 ? 4096 : 0);
+  constexpr bool kDelayV0 = PARTS == 1 && DQK == 192;
+  static_assert(PARTS == 1 ? 2 * kQArea <= L::kKTile && (kDelayV0 ? kQArea : 2 * kQArea) <= L::kVTile
+                           : kQArea * L::kRowBlocks / 2 <= L::kVTile, "query areas");
+  char* const k1 = kbuf + L::kKTile;
+  char* const v0 = vbuf;
+  char* const v1 = vbuf + L::kVTile;
+  char* q_area;
+  if constexpr (PARTS == 1) q_area = wave < 2 ? k1 + wave * kQArea : kDelayV0 ? (wave == 2 ? v1 : v0) : v1 + (wave - 2) * kQArea;
+  else if constexpr (PARTS == 2) q_area = smem + (row_block >> 1) * L::kRings + 2 * L::kKTile + L::kVTile + (row_block & 1) * kQArea;
+  else q_area = smem + row_block * L::kRings + 2 * L::kKTile + L::kVTile;
+  {
+    constexpr int kShare = PARTS;  // waves of a row block
+    const int part = PARTS == 4 ? 2 * team + kvb0 : team;
+    const char* const qsrc = reinterpret_cast<const char*>(qh);
+    const int q_row_bytes = (int)(q_row_stride * 2);
+    if constexpr (!kPaired) stage_rows32<true, 8 / kShare>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane, part * (8 / kShare));
+    if constexpr (DQK != 128)
+      stage_rows32<false, 4 / kShare>(qsrc + (kPaired ? 0 : 256), q_wave0, p.Sq, q_row_bytes, q_area + (kPaired ? 0 : 8192), lane, part * (4 / kShare));
+  }
   if (kTeams == 1 || n_tiles_wg > 0) {
     issue_k(0);
-    issue_v(0);
+    if constexpr (!kDelayV0) issue_v(0);
   }
-  if (n_tiles_wg > 1) issue_k(1);
-
-  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features.
-  bf16x8 qf[KS];
-  {
-    const int row = qrow < p.Sq ? qrow : p.Sq - 1;
-    const __bf16* src = qh + row * q_row_stride + g * 8;
+  if (PARTS > 1 && n_tiles_wg > 1) issue_k(1);
+  constexpr int kLoadsK = kPaired ? 2 : DQK == 192 ? 6 : 4, kLoadsV = kPaired ? 2 : 4;  // load instructions of a wave per tile
+  bf16x8 qf[KS];  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features
+  auto read_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + ks * 16);
-  }
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = kPaired ? staged_fragment<false>(q_area, ks, c, g) : ks < 8 ? staged_fragment<true>(q_area, ks, c, g)
+                                                                           : staged_fragment<false>(q_area + 8192, ks - 8, c, g);
+  };
 
   // per-lane read offsets (see attn_fwd_direct.hip): one base per tile part, the rest by XOR
   // (KVB = 1: the wave's key block sits in the bases)
@@ -315,12 +337,24 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     __builtin_amdgcn_s_setprio(0);
   };
 
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  __syncthreads();
+  if constexpr (PARTS == 1) {
+    wait_staged<kLoadsK + (kDelayV0 ? 0 : kLoadsV)>();
+    read_q();
+    wait_staged<kDelayV0 ? 0 : kLoadsV>();
+    __syncthreads();  // K tile 0 is there, and every wave has read its query rows: their slots may be filled
+    if constexpr (kDelayV0) issue_v(0);
+    if (n_tiles_wg > 1) issue_k(1);
+  } else {
+    if (n_tiles_wg > 1) wait_staged<kLoadsV + kLoadsK>();
+    else wait_staged();
+    __syncthreads();
+    read_q();
+  }
   const bool any = kTeams == 1 || n_tiles_wave > 0;
   if (any) scores(kbuf);
   if (team == 0) softmax(0);
-  __syncthreads();  // K tile 0 has been read: its slot may be refilled
+  wait_staged();
+  __syncthreads();  // K tile 0 (and the query rows) has been read: its slot may be refilled; V 0 and K 1 are there
 
   // interval i: O += V(i)^T P(i), S(i+1) = K(i+1) Q^T, P(i+1); K(i+2) and V(i+1) are requested meanwhile. The second team
   // takes the softmax first (of S(i)): the two waves of a SIMD are in different phases.

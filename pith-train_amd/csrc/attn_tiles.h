@@ -323,7 +323,11 @@ struct DirectExtra64 {
   }
   __device__ __forceinline__ void issue(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
     if (rows_left >= 64) load_lds16(tile_src, src_off, slot + wave * 1024);
-    else load_lds16(tile_src, source(row_bytes, col_bytes, wave, lane, rows_left), slot + wave * 1024);
+    else issue_clamped(tile_src, rows_left, slot, wave, lane);
+  }
+  // source offset formed on the spot, see DirectTile128::issue_clamped
+  __device__ __forceinline__ void issue_clamped(const char* tile_src, int rows_left, char* slot, int wave, int lane) const {
+    load_lds16(tile_src, source(row_bytes, col_bytes, wave, lane, rows_left), slot + wave * 1024);
   }
 };
 
@@ -366,6 +370,49 @@ struct DirectPaired64 {
                  slot + (n * kWaves + wave) * 1024);
   }
 };
+
+// ---------------------------------------------------------------------------------------------
+// A wavefront's 32 stationary rows (Q, dO, K or V) on their way into registers as MFMA B fragments: staged in a wave-private
+// LDS area (tile slots that hold nothing yet) with whole-row direct loads, then read like a tile. Fetched straight into
+// registers, a fragment load touches 32 rows with 32 bytes each: every lane of a quad on a line of its own, which the address
+// unit serves at one lane per cycle (64 cycles per instruction against 16 for contiguous rows). A workgroup of 8 waves then
+// spent 2-5 us only on issuing them, in front of or behind its first tiles. From the start of a workgroup of the second round
+// to its first interval (stamps inside the kernels), before -> now: forward 4096 x 16 heads of 192 5.3 -> 3.6 us, its dQ 5.7 ->
+// 4.0, its dK/dV 4.1 -> 2.6, dK/dV of 4096 x 32/4 of 128 3.8 -> 2.5; fwd + bwd of a layer of 4096 x 16 of 192 (with the spills
+// in dQ and the epilogues of this change) 397 -> 382 us, of 4096 x 32/4 of 128 575 -> 571: there the chip is at its power limit
+// and gives most of the time back as a lower clock.
+//
+// Features [col, col + 128) (WIDE: 8 KB, eight loads) or [col, col + 64) (4 KB, four loads, rows r and r + 16 in one 256-byte
+// LDS row) of rows row0 .. row0 + 31; rows from `rows` on are read from the last one (row0 may lie beyond it). `src` points to
+// row 0, feature `col` of the head. Completion as for tiles (vmcnt); the wave needs no barrier before it reads its own area.
+// Waves that own the same rows share an area and the loads: this one issues the loads n0 .. n0 + N - 1 (wave-uniform).
+template <bool WIDE, int N = WIDE ? 8 : 4>
+__device__ __forceinline__ void stage_rows32(const char* src, int row0, int rows, int row_bytes, char* area, int lane, int n0 = 0) {
+  const int first = min(row0, rows - 1), left = rows - first;
+  const char* const base = src + (int64_t)first * row_bytes;
+  const int sub = lane >> 4, piece = lane & 15;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int n = n0 + i;
+    const int p = piece ^ tile_swizzle(4 * n + sub);
+    int row = 4 * n + sub + (WIDE ? 0 : 16 * (p >> 3));
+    row = row < left ? row : left - 1;
+    load_lds16(base, row * row_bytes + ((WIDE ? p : p & 7) << 4), area + n * 1024);
+  }
+}
+// The fragment of contraction step ks (features 16 ks ..) of the row this lane owns, c = lane % 32.
+template <bool WIDE>
+__device__ __forceinline__ bf16x8 staged_fragment(const char* area, int ks, int c, int g) {
+  const int off = WIDE ? swizzled_offset(c, 2 * ks + g) : swizzled_offset(c & 15, (2 * ks + g) | ((c >> 4) << 3));
+  return *reinterpret_cast<const bf16x8*>(area + off);
+}
+// Waits for the wave's own loads; `later` of them, the last ones issued, may stay in flight.
+template <int LATER = 0>
+__device__ __forceinline__ void wait_staged() {
+  static_assert(LATER < 16, "the immediate has four low bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | LATER);
+  asm volatile("" ::: "memory");
+}
 
 // Per-lane offsets for reading a packed swizzled tile.
 // straight_offset(c, piece): fragment of row c (+ a multiple of 16 rows added by the caller as
