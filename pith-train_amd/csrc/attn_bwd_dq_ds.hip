@@ -5,8 +5,9 @@
 // other dQ kernels repeat are gone; the price is one trip of dS through memory, so this kernel is
 // bound by the rate at which it can stream the images, not by the matrix pipe.
 //
-// Work split: a workgroup of 8 wavefronts owns 512 query rows of one (batch, head), wave w the 64-row
-// query tile 8*m_tile + w of the writer. Keys are visited in steps of 32 (one wave pair of the
+// Work split: a workgroup of 8 wavefronts owns 512 query rows of one (batch, head), a wave one 64-row query tile of the
+// writer (under the mask two blocks of 256 rows, one near the start and one near the end: with 512 consecutive rows the
+// heaviest of 8 workgroups of a 4096-row head carried twice the average and a single round of them did not pay). Keys are visited in steps of 32 (one wave pair of the
 // writer). Per step the K tile (shared, packed and swizzled like everywhere else, 8 KB) and, per
 // wave, the 4 KB image of its tile for that pair (copied verbatim) go global -> LDS directly. What
 // bounds the kernel is how many bytes of dS each compute unit keeps in flight (a compute unit's
@@ -78,8 +79,18 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   int m_tile, h, b;
   decode_block(blockIdx.x, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b);
   const int hk = h / p.group;
-  const int m0 = m_tile * kBM;
-  const int q_wave0 = m0 + wave * QW;
+  // Query tiles of the waves. Without a mask eight consecutive ones. Under it the workgroup takes two 256-row blocks, waves
+  // 0..3 the m_tile-th from the start and waves 4..7 the m_tile-th from the end, so that all workgroups read the same number
+  // of images (the middle one of an odd number of blocks goes to waves 4..7 alone).
+  const int blocks256 = (p.Sq + kBM / 2 - 1) / (kBM / 2);
+  auto rows_of = [&](int w) __attribute__((always_inline)) {
+    if (!CAUSAL) return m_tile * kBM + w * QW;
+    const int late = blocks256 - 1 - m_tile;
+    const int block = w >= 4 ? late : m_tile < late ? m_tile : blocks256;  // blocks256: none
+    return block * (kBM / 2) + (w & 3) * QW;
+  };
+  const int m_end = CAUSAL ? (blocks256 - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
+  const int q_wave0 = rows_of(wave), q_other0 = rows_of(wave & 3);  // q_other0: of the wave whose images waves 4..7 also request
 
   const int kv_row_bytes = p.HkvT * DQK * 2;
   const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * DQK);
@@ -87,7 +98,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   // key steps: all of them, or up to the diagonal; a wave whose query tile does not exist (ragged
   // Sq) has no images and visits nothing. Rows q0 .. q0+QW-1 lie in the writer's 64-row tile q0 >> 6.
   const int n_steps_all = (p.Skv + kBN - 1) / kBN;
-  const int n_steps_wg = CAUSAL ? min(n_steps_all, (m0 + kBM - 1) / kBN + 1) : n_steps_all;
+  const int n_steps_wg = CAUSAL ? min(n_steps_all, (m_end - 1) / kBN + 1) : n_steps_all;
   auto steps_of = [&](int q0) __attribute__((always_inline)) {
     if ((q0 >> 6) >= p.ds_qt) return 0;
     return CAUSAL ? min(n_steps_all, (q0 + QW - 1) / kBN + 1) : n_steps_all;
@@ -104,8 +115,8 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   const bool k_mover = wave < 4;
   DirectTile128<kBN, 256> mover;
   mover.init(kv_row_bytes, wave & 3, lane);
-  const char* ds_src[2] = {images_of(q_wave0 - 4 * QW), images_of(q_wave0)};        // only used by waves 4..7
-  const int ds_steps[2] = {k_mover ? 0 : steps_of(q_wave0 - 4 * QW), k_mover ? 0 : n_steps_wave};
+  const char* ds_src[2] = {images_of(q_other0), images_of(q_wave0)};        // only used by waves 4..7
+  const int ds_steps[2] = {k_mover ? 0 : steps_of(q_other0), k_mover ? 0 : n_steps_wave};
   auto request_k = [&](int s, int slot) __attribute__((always_inline)) {
     char* stage = smem + slot * kKStage;
     const char* k_src = kh + (int64_t)s * kBN * kv_row_bytes;
@@ -143,12 +154,15 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   constexpr int kSteadyDs = (kRingD - 2) * 2 * kLoadsDs;
   static_assert(kRingK == 3 && kSteadyDs < 32, "one K step in flight; dS loads in flight fit the decision tree");
   const int ds_steady_end = min(min(ds_steps[0], ds_steps[1]), n_steps_wg) - (kRingD - 2);  // steps below: steady state
+  const int ds_single_end = min(ds_steps[1], n_steps_wg) - (kRingD - 2);
   auto wait_step = [&](int s) __attribute__((always_inline)) {
     if (k_mover) {
       if (s + 1 < n_steps_wg) wait_vector_loads_but<kLoadsK>();
       else wait_vector_loads_but<0>();
     } else if (s < ds_steady_end) {
       wait_vector_loads_but<kSteadyDs>();
+    } else if (CAUSAL && s >= ds_steps[0] && s < ds_single_end) {  // only the later block's images are left
+      wait_vector_loads_but<kSteadyDs / 2>();
     } else {
       int n = 0;
 #pragma unroll

@@ -447,12 +447,18 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
   return python_body<Two>("attn_fwd", q, k, v, scale, causal);
 }
 
-// Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill
-// the device, and under the mask one round of workgroups will not do, because the heaviest of them carries almost twice
-// the average work (1 x 4096 rows x 32 heads: pair of kernels 445 us handing over, 428 us recomputing; 2 x 2048 x 32: 252
-// and 238 us), unless the sequence is so short (two tiles) that there is nothing to balance.
-bool ds_handover_pays(int64_t workgroups, int64_t row_tiles, bool causal, int64_t cus) {
-  return workgroups >= cus && !(causal && row_tiles > 2 && workgroups <= cus);
+// Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup, all of about the same length) beats recomputing
+// the scores: it has to fill the device, and under the mask, where a workgroup reads half as much and the rounds are short, it
+// must not leave most of its last round empty. W = workgroups per compute unit; forward + backward, handing over / recomputing:
+//   causal  W 1     1 x 4096 x 32/4 heads 578 / 600 us, 2 x 2048 x 32/4 337 / 340, 4 x 1024 x 32/4 208 / 219, 8 x 512 x 32/4 179 / 192
+//           W 1.12  9216 x 16 1469 / 1428, 3 x 1536 x 32/4 332 / 324       W 1.25  5120 x 32/4 936 / 950, 2 x 2560 x 32/4 527 / 525
+//           W 1.5   6144 x 32/4 1265 / 1314, 6 x 1024 x 32/4 318 / 324, 3 x 1999 x 32/4 515 / 507, 2 x 3072 x 32/4 726 / 714
+//           W 1.75  7168 x 32/4 1692 / 1720    W 2  8192 x 32/4 2130 / 2194    W 2.25  9 x 1024 x 32/4 456 / 472, 9216 x 32/4 2863 / 2821
+//           W 0.75  3072 x 32/4 391 / 390
+//   full    W 1.12  4608 x 32/4 1663 / 1730, 9216 x 16 2766 / 2899         W 1.25  5120 x 32/4 1878 / 1930    W 1.5  6144 x 32/4 2487 / 2480
+bool ds_handover_pays(int64_t workgroups, bool causal, int64_t cus) {
+  if (cus <= 0 || workgroups < cus) return false;
+  return !causal || 10 * workgroups >= 7 * cus * ((workgroups + cus - 1) / cus);
 }
 
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
@@ -460,8 +466,7 @@ Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& 
   // kernels outlast its host work many times over.
   bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4;
   if (small && q.size(3) == 128) {
-    const int64_t row_tiles = (q.size(1) + 511) / 512;
-    small = !ds_handover_pays(row_tiles * q.size(2) * q.size(0), row_tiles, causal, compute_units(q.device().index()));
+    small = !ds_handover_pays((q.size(1) + 511) / 512 * q.size(2) * q.size(0), causal, compute_units(q.device().index()));
   }
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);

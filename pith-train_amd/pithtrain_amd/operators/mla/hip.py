@@ -234,12 +234,11 @@ def _ds_budget_bytes(device: torch.device, enough: int) -> int:
 def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = False):
     """How the backward of one chunk pair uses the dS hand-over: (kv heads per slab, bytes of the buffer),
     or None when both kernels should recompute (no hand-over path for these head dims, the dS-reading dQ
-    kernel would have fewer workgroups than the device has compute units, or not even one kv head fits the
-    budget)."""
+    kernel would not fill the device, or not even one kv head fits the budget)."""
     b, sq, hq, _ = q.shape
     hkv = k.shape[2]
     row_tiles = -(-sq // _DS_ROWS_PER_WORKGROUP)
-    if not native.ds_handover_pays(row_tiles * hq * b, row_tiles, causal, _device_compute_units(q.device)):  # nor for any slab
+    if not native.ds_handover_pays(row_tiles * hq * b, causal, _device_compute_units(q.device)):  # nor for any slab
         return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:

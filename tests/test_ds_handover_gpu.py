@@ -83,6 +83,13 @@ def test_causal_dq_from_ds(gpu, shape):
     _run(gpu, True, shape, torch.bfloat16)
 
 
+@pytest.mark.parametrize("S", [255, 257, 511, 513, 767, 769, 1025, 1281, 1537])
+def test_causal_pairs_of_row_blocks(gpu, S):
+    """Under the mask a workgroup takes 256-row blocks in pairs, one from either end: odd and even numbers of blocks, the last
+    one full, of one row or one row short."""
+    _run(gpu, True, (1, S, S, 2, 1), torch.bfloat16)
+
+
 @pytest.mark.parametrize("shape", NONCAUSAL_SHAPES)
 def test_noncausal_dq_from_ds(gpu, shape):
     _run(gpu, False, shape, torch.bfloat16)
@@ -286,3 +293,37 @@ def test_allocation_failure_falls_back_to_recomputation(gpu, monkeypatch):
     rdq, _, _ = R.chunk_bwd(q, k, v, dout, lse.double().cpu(), delta.double().cpu(), scale, False)
     check_bf16_result(out["oom"][0], rdq, "recomputed dQ after allocation failure", otol=1e-3)
     check_bf16_result(out["handover"][0], rdq, "hand-over dQ", otol=1e-3)
+
+
+def test_layer_of_one_round_under_capture(gpu):
+    """A causal layer whose dS-reading dQ kernel just fills the device hands dS over, eagerly and in a captured graph."""
+    import pithtrain_amd.operators.mla.hip as H
+
+    g = torch.Generator(device=gpu).manual_seed(3)
+    mk = lambda h: torch.randn(4, 1024, h, 128, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v, dout, scale = mk(32), mk(4), mk(4), mk(32), 128**-0.5
+    if H._device_compute_units(q.device) == 256:
+        assert H.ds_plan(q, k, v, True) is not None  # 2 x 32 x 4 workgroups of 512 rows
+    fwd, bwd = torch.ops.pithtrain_amd.attn_fwd, torch.ops.pithtrain_amd.attn_bwd
+
+    def step():
+        o, lse = fwd(q, k, v, scale, True)
+        return [o, lse, *bwd(q, k, v, o, lse, dout, scale, True)]
+
+    want = [t.clone() for t in step()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for replay in range(3):
+        for t in captured:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, want)), f"replay {replay}"
+        assert all(torch.equal(a, b) for a, b in zip(step(), want))
