@@ -250,14 +250,14 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
 // ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
 // rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
 // 16: 2385 -> 2413).
-// At 64 features one kernel costs dQ its third workgroup per compute unit (186 instead of 150 registers), which only
-// grids of a few rounds do not miss (1 x 4096 x 16 heads causal 184 -> 130 us, 1 x 4096 x 32 262 -> 259 us, 4 x 4096 x 16
-// 474 -> 483 us).
+// At 64 features both kernels fit two workgroups to a unit, and one grid is never slower: forward + backward, before (apart from
+// more than four workgroups per unit, three of dQ) -> now, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 ->
+// 2359, 16 x 1024 x 32/8 415 -> 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630.
 bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
   if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
   const int64_t cus = compute_units_or_default();
   const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
-  if (a->Dqk == 64) return q_wgs <= 4 * cus;
+  if (a->Dqk == 64) return true;
   if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
   if (q_wgs <= cus) return true;
   if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;

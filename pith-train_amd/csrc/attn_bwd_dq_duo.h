@@ -1,5 +1,5 @@
 // Query-gradient kernel for head dims (64, 64), (128, 128) and (192, 128) on gfx950 with SMALL workgroups: 4 wavefronts,
-// 128 query rows, two of them per compute unit (three at 64 features). Same function and numerics as
+// 128 query rows, two of them per compute unit. Same function and numerics as
 // attn_bwd_dq_direct.hip (pithtrain/operators/mla/triton.py:205-266, :392-441: P = exp2(kappa*s - lse2) in fp32, masked
 // entries 0, dS = P*(dP - delta) rounded to bf16, fp32 accumulation of dQ += dS K, `scale` applied once at the end).
 //
@@ -12,6 +12,8 @@
 // Bound by the matrix pipe (three products executed for the one that counts). Measured, executed products: 8192 x 8192 x
 // 32 heads of 128 features 1284 TFLOP/s (1242 for the 256-row kernel with interleaved halves it replaces), 2 x 4096 x 16 of 64
 // features 1033 (915 register-staged), 4096 x 4096 x 16 of 192 features 1219 (1156 with 128-row workgroups splitting keys).
+// At 64 features the two blocks are woven as in attn_bwd_dkdv_d64.h (229 registers; in blocks it took 150, and three workgroups
+// to a unit: equal alone, slower beside dK/dV workgroups, see one_grid).
 #pragma once
 
 #include "attn_bwd_common.h"
@@ -23,11 +25,12 @@ constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
 constexpr int kBM = 32 * kWaves;  // query rows per workgroup
 constexpr int kBN = 32;           // keys per tile
-constexpr int kSlots = 4;         // tiles i-1 and i (in use), i+1 and i+2 (landing); a power of two
 
 template <int DQK>
 struct DqDuoLayout {
   static constexpr int kDv = DQK == 64 ? 64 : 128;
+  // ring depth: tiles i-1 and i (in use), i+1 and i+2 (landing), at 64 features i-1 to i+1 and i+2, i+3; a power of two
+  static constexpr int kSlots = DQK == 64 ? 8 : 4;
   static constexpr int kPair = kBN / 2 * kRowBytes128, kFull = kBN * kRowBytes128;  // 64- and 128-feature tiles
   static constexpr int kKTile = DQK == 64 ? kPair : DQK == 128 ? kFull : kFull + kPair;
   static constexpr int kVTile = kDv == 64 ? kPair : kFull;
@@ -44,7 +47,7 @@ constexpr int kSmem = DqDuoLayout<DQK>::kSmem;
 template <int DQK, bool CAUSAL, typename OutT, bool MULTI = false>
 __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int block) {
   using L = DqDuoLayout<DQK>;
-  constexpr int kDv = L::kDv, KS = DQK / 16, VS = kDv / 16, DB = DQK / 32;
+  constexpr int kDv = L::kDv, KS = DQK / 16, VS = kDv / 16, DB = DQK / 32, kSlots = L::kSlots;
   constexpr bool kPaired = DQK == 64;
   constexpr int kAhead = DQK == 192 ? 3 : 4;  // fragment reads run this many products ahead in the matrix block
   char* const kbuf = smem;
@@ -99,6 +102,16 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
     kmover.init(k_row_bytes, wave, lane);
     if constexpr (DQK == 192) kpmover.init(kx_row_bytes, two_part ? 0 : 256, wave, lane);
   }
+  // one operand at a time, without a branch: source offsets formed on the spot, and behind the last tile that one again, into a
+  // slot that nobody reads (64 features, one chunk)
+  auto request_k = [&](int t) __attribute__((always_inline)) {
+    const int at = min(t, n_wg - 1);
+    kpmover.issue_clamped(k_src.src(at), k_src.left(at), kbuf + (t & (kSlots - 1)) * L::kKTile, wave, lane);
+  };
+  auto request_v = [&](int t) __attribute__((always_inline)) {
+    const int at = min(t, n_wg - 1);
+    vpmover.issue_clamped(v_src.src(at), k_src.left(at), vbuf + (t & (kSlots - 1)) * L::kVTile, wave, lane);
+  };
   auto request = [&](int t) __attribute__((always_inline)) {
     char* const ks = kbuf + (t & (kSlots - 1)) * L::kKTile;
     char* const vs = vbuf + (t & (kSlots - 1)) * L::kVTile;
@@ -155,10 +168,10 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   int s_base = straight_offset128(c, g);
   int x_base = straight_offset128(c & 15, g + 8 * (c >> 4));
   int t_base[2] = {transposed_offset128(0, 0, 0, lane), transposed_offset128(0, 1, 0, lane)};
-  // 192 features: one base per tile part lives across the loop, the derived offsets are formed anew in every interval
+  // 192 and 64 features: one base per tile part lives across the loop, the derived offsets are formed anew in every interval
   // (hoisted out of it they would push accumulators into scratch memory)
   auto refresh_offsets = [&]() __attribute__((always_inline)) {
-    if constexpr (DQK == 192) asm volatile("" : "+v"(s_base), "+v"(x_base), "+v"(t_base[0]), "+v"(t_base[1]));
+    if constexpr (DQK != 128) asm volatile("" : "+v"(s_base), "+v"(x_base), "+v"(t_base[0]), "+v"(t_base[1]));
   };
   auto k_frag = [&](const char* kt, int ks) __attribute__((always_inline)) {
     const int off = kPaired ? x_base ^ (ks << 5) : ks < 8 ? s_base ^ (ks << 5) : L::kFull + (x_base ^ ((ks - 8) << 5));
@@ -261,36 +274,145 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
       dsf[j] = to_bf16x8(s[8 * j], s[8 * j + 1], s[8 * j + 2], s[8 * j + 3], s[8 * j + 4], s[8 * j + 5], s[8 * j + 6], s[8 * j + 7]);
   };
 
-  if (n_wg > 2) wait_staged<2 * L::kLoads>();
-  else wait_staged();
-  __syncthreads();
-  scores(kbuf, vbuf);
-  make_ds(0);
-  if (n_wg > 2) wait_staged<L::kLoads>();
-  else wait_staged();
-  __syncthreads();  // tile 1 is there
+  if constexpr (kPaired) {
+    // ---- 64 features: the vector work of a tile costs as much issue time as its products, so the two are woven. Step i: the
+    // gradient products of tile i - 1 and S(i + 1) between the exponentials of tile i, then dP(i + 1) between the rest of its
+    // arithmetic. Tile i + 3 is requested; tile i + 2 has landed when the step ends.
+    f32x16 s1, dp1;
+    auto kslot = [&](int t) __attribute__((always_inline)) { return kbuf + (t & (kSlots - 1)) * L::kKTile; };
+    auto vslot = [&](int t) __attribute__((always_inline)) { return vbuf + (t & (kSlots - 1)) * L::kVTile; };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    // product m of the step: gradient products 0..3 (GRAD), then S, 4..7, and dP, 8..11, of the next tile (NEXT)
+    auto step = [&](int i, auto grad_tag, auto next_tag, f32x16& x, f32x16& y, f32x16& nx, f32x16& ny) __attribute__((always_inline)) {
+      constexpr bool GRAD = decltype(grad_tag)::value, NEXT = decltype(next_tag)::value;
+      static_assert(2 * DB == 4 && KS == 4 && VS == 4, "products of a step");
+      refresh_offsets();
+      const char* const kp = kslot(i - 1);
+      const char* const kn = kslot(i + 1);
+      const char* const vn = vslot(i + 1);
+      auto frag = [&](int m) __attribute__((always_inline)) -> bf16x8 {
+        if (m < 4) return GRAD ? kt_frag(kp, m >> 1, m & 1) : bf16x8{};
+        return NEXT ? (m < 8 ? k_frag(kn, m - 4) : v_frag(vn, m - 8)) : bf16x8{};
+      };
+      if constexpr (NEXT && MULTI) request(i + 3);  // (a tile's address takes branches; behind the last tile it is one of the last chunk)
+      bf16x8 a[12];
+#pragma unroll
+      for (int m = 0; m < kAhead; ++m) a[m] = frag(m);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        if (NEXT) nx[v] = 0.f;
+        if (NEXT) ny[v] = -delta_q;  // dS = P * (dP - delta) without a subtraction per element
+      }
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        a[m + kAhead] = frag(m + kAhead);
+        if (GRAD && m < 4) acc[m & 1] = mfma32(a[m], dsf[m >> 1], acc[m & 1]);
+        if (NEXT && m >= 4) nx = mfma32(a[m], qf[m - 4], nx);
+        if constexpr (NEXT && !MULTI) {
+          if (m == 1) request_k(i + 3);
+          if (m == 3) request_v(i + 3);
+        }
+#pragma unroll
+        for (int v = 2 * m; v < 2 * m + 2; ++v) x[v] = __builtin_amdgcn_exp2f(x[v] * p.kappa - lse_q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (mask.partial(range, i, q_wave0)) {  // wave-uniform
+        const int limit = mask.limit(range, qrow), n0 = mask.key0(i);
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (n0 + acc_row(v, g) > limit) x[v] = 0.f;
+      }
+      mask.advance(p, range);
+      u32x4 du[2];
+#pragma unroll
+      for (int m = 8; m < 12; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (NEXT) ny = mfma32(a[m], dof[m - 8], ny);
+#pragma unroll
+        for (int w = 2 * (m - 8); w < 2 * (m - 8) + 2; ++w) {
+          uint32_t dw = pack_bf16x2(x[2 * w] * y[2 * w], x[2 * w + 1] * y[2 * w + 1]);
+          asm volatile("" : "+v"(dw));  // formed here, not where it is used
+          du[w >> 2][w & 3] = dw;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dsf[j] = __builtin_bit_cast(bf16x8, du[j]);
+      if constexpr (NEXT) {  // (a wave's last tile waits for nothing)
+        wait_staged<L::kLoads>();
+        __syncthreads();
+      }
+    };
+    if (n_wg > 2) wait_staged<2 * L::kLoads>();
+    else wait_staged();
+    __syncthreads();
+    scores(kbuf, vbuf);
+    if (n_wg > 2) wait_staged<L::kLoads>();
+    else wait_staged();
+    __syncthreads();  // tile 1 is there
+    if (n_wave == 1) {
+      step(0, no, no, s, dp, s1, dp1);
+    } else {
+      step(0, no, yes, s, dp, s1, dp1);
+      int i = 1;
+      for (; i + 2 < n_wave; i += 2) {
+        step(i, yes, yes, s1, dp1, s, dp);
+        step(i + 1, yes, yes, s, dp, s1, dp1);
+      }
+      if (i + 1 < n_wave) {
+        step(i, yes, yes, s1, dp1, s, dp);
+        step(i + 1, yes, no, s, dp, s1, dp1);
+      } else {
+        step(i, yes, no, s1, dp1, s, dp);
+      }
+    }
+    accumulate(kslot(n_wave - 1));
+    for (int i = n_wave - 1; i + 1 < n_wg; ++i) {  // waves above the workgroup's last diagonal block keep moving tiles for the others
+      if constexpr (MULTI) {
+        request(i + 3);
+      } else {
+        request_k(i + 3);
+        request_v(i + 3);
+      }
+      wait_staged<L::kLoads>();
+      __syncthreads();
+    }
+    wait_staged();
+    __syncthreads();  // every wave is done with the rings, and nothing lands in them any more
+  } else {
+    if (n_wg > 2) wait_staged<2 * L::kLoads>();
+    else wait_staged();
+    __syncthreads();
+    scores(kbuf, vbuf);
+    make_ds(0);
+    if (n_wg > 2) wait_staged<L::kLoads>();
+    else wait_staged();
+    __syncthreads();  // tile 1 is there
 
-  int i = 1;
-  for (; i < n_wave; ++i) {
-    const bool more = i + 2 < n_wg;
-    refresh_offsets();
-    if (more) request(i + 2);
-    matrix_block(kbuf + ((i - 1) & (kSlots - 1)) * L::kKTile, kbuf + (i & (kSlots - 1)) * L::kKTile, vbuf + (i & (kSlots - 1)) * L::kVTile);
-    make_ds(i);
-    // tile i + 1 has landed; the loads just requested may stay in flight (they are the wave's last memory operations)
-    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    int i = 1;
+    for (; i < n_wave; ++i) {
+      const bool more = i + 2 < n_wg;
+      refresh_offsets();
+      if (more) request(i + 2);
+      matrix_block(kbuf + ((i - 1) & (kSlots - 1)) * L::kKTile, kbuf + (i & (kSlots - 1)) * L::kKTile, vbuf + (i & (kSlots - 1)) * L::kVTile);
+      make_ds(i);
+      // tile i + 1 has landed; the loads just requested may stay in flight (they are the wave's last memory operations)
+      if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+    accumulate(kbuf + ((n_wave - 1) & (kSlots - 1)) * L::kKTile);
+    for (; i < n_wg; ++i) {  // waves above the workgroup's last diagonal block keep moving tiles for the others
+      const bool more = i + 2 < n_wg;
+      if (more) request(i + 2);
+      if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+    __syncthreads();  // every wave is done with the rings
   }
-  accumulate(kbuf + ((n_wave - 1) & (kSlots - 1)) * L::kKTile);
-  for (; i < n_wg; ++i) {  // waves above the workgroup's last diagonal block keep moving tiles for the others
-    const bool more = i + 2 < n_wg;
-    if (more) request(i + 2);
-    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | L::kLoads);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  }
-  __syncthreads();  // every wave is done with the rings
 
   OutT* rows = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK + q_wave0 * q_row_stride;
   __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16

@@ -49,3 +49,13 @@ def test_first_tiles_of_larger_grids(gpu, D, H, S):
     for causal in [False, True]:
         o, _ = _mla_fwd(q, k, v, D**-0.5, causal)
         check_bf16_result(o, _forward_reference(q, k, v, D**-0.5, causal), "O", otol=1e-3)
+
+
+@pytest.mark.parametrize("S", [32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 224, 290])
+@pytest.mark.parametrize("Hq,Hkv", [(1, 1), (6, 2)])
+def test_woven_steps_at_64_features(gpu, S, Hq, Hkv):
+    """Gradients of 64 features: streams of one to ten steps of 32 rows, ragged ends, one and several heads to a stream, with
+    waves that leave the workgroup's stream early (causal)."""
+    for causal in [False, True]:
+        check_backward(gpu, 1, S, S, Hq, Hkv, 64, causal)
+    check_backward(gpu, 1, S, 290 - S // 2, Hq, Hkv, 64, False)
