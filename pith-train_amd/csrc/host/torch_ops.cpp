@@ -800,6 +800,90 @@ Three mla_assemble_fwd_autograd(const Tensor& q, const Tensor& kv, const Tensor&
   return call_mla_assemble_fwd(q, kv, k_pe, cos, sin, pos);
 }
 
+// One rank's ring share as one node. What its Python counterpart (RingAttentionLocalFunc) spends on a dozen chunk tensors
+// outlasts the kernels of a short share: forward + backward of 64 rows, 16 heads of 192 in two parts, rank 2 of 4 177 -> 138 us (of
+// which 108 are the engine handing out ten gradients); 1021 rows 165 -> 157 us, now the length of its kernels.
+// Inputs: q, then the visited chunks of K, of V and, if keys come in two parts, of k_pe.
+using OptTensors = std::vector<OptTensor>;
+
+int64_t visited_chunks(int64_t rank, int64_t cp, bool zigzag) { return zigzag ? cp : rank + 1; }  // the first ones, by rank
+
+struct RingFunction : torch::autograd::Function<RingFunction> {
+  // chunk lists of cp entries from the flat inputs, whose first chunk is at `first`
+  static std::vector<OptTensors> chunk_lists(at::TensorList in, size_t first, int64_t cp, int64_t visited) {
+    std::vector<OptTensors> lists((in.size() - first) / visited, OptTensors(cp));
+    for (size_t kind = 0; kind < lists.size(); ++kind)
+      for (int64_t j = 0; j < visited; ++j) lists[kind][j] = in[first + kind * visited + j];
+    return lists;
+  }
+  static std::optional<OptTensors> part_two(const std::vector<OptTensors>& lists) {
+    return lists.size() == 3 ? std::optional<OptTensors>(lists[2]) : std::nullopt;
+  }
+  static Tensor forward(AutogradContext* ctx, at::TensorList in, double scale, int64_t rank, int64_t cp, bool zigzag) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const auto lists = chunk_lists(in, 1, cp, visited_chunks(rank, cp, zigzag));
+    auto done = ring_forward(in[0], lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
+    if (!done) done = python_body<Two>("ring_forward_local", in[0], lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
+    variable_list saved = {std::get<0>(*done), std::get<1>(*done)};
+    saved.insert(saved.end(), in.begin(), in.end());
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["rank"] = rank;
+    ctx->saved_data["cp"] = cp;
+    ctx->saved_data["zigzag"] = zigzag;
+    return std::get<0>(*done);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const auto s = ctx->get_saved_variables();  // out, lse, q, chunks
+    const double scale = ctx->saved_data["scale"].toDouble();
+    const int64_t rank = ctx->saved_data["rank"].toInt(), cp = ctx->saved_data["cp"].toInt();
+    const bool zigzag = ctx->saved_data["zigzag"].toBool();
+    const int64_t visited = visited_chunks(rank, cp, zigzag);
+    const Tensor &out = s[0], &lse = s[1], &q = s[2];
+    const auto lists = chunk_lists(s, 3, cp, visited);
+    std::optional<RingGrads> g;
+    if (!may_hand_over(q, rank, cp, zigzag)) g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
+    if (!g) g = python_body<RingGrads>("ring_backward_local", grads[0], q, out, lse, lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
+    variable_list r = {std::get<0>(*g)};
+    for (const OptTensors* kind : {&std::get<1>(*g), &std::get<2>(*g), &std::get<3>(*g)})
+      for (int64_t j = 0; j < visited && j < (int64_t)kind->size(); ++j) r.push_back(or_undefined((*kind)[j]));
+    r.resize(s.size() - 2 + 4);  // scale, rank, cp, zigzag
+    return r;
+  }
+  // Whether a step of the share may hand dS over, a decision that the Python body makes.
+  static bool may_hand_over(const Tensor& q, int64_t rank, int64_t cp, bool zigzag) {
+    if (q.size(3) != 128) return false;
+    const int64_t cus = compute_units(q.device().index());
+    const auto pays = [&](int64_t rows, bool causal) { return ds_handover_pays((rows + 511) / 512 * q.size(2) * q.size(0), causal, cus); };
+    return pays(q.size(1), true) || (rank > 0 && pays(q.size(1), false)) || (zigzag && rank + 1 < cp && pays(q.size(1) / 2, false));
+  }
+};
+
+// None where the Python function has to do: CPU tensors and missing chunks (it words the errors), and tensors or modes that
+// look at every operation (fake, batched and functional tensors, dispatch modes, tracing, forward-mode gradients).
+OptTensor ring_attention(const Tensor& q, const OptTensors& ks, const OptTensors& vs, const std::optional<OptTensors>& pes, double scale, int64_t rank,
+                         int64_t cp, bool zigzag) {
+  if (!(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty()) return {};
+  if (rank < 0 || rank >= cp || (int64_t)ks.size() != cp || (int64_t)vs.size() != cp || (pes && (int64_t)pes->size() != cp)) return {};
+  constexpr c10::DispatchKeySet watching({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchBatched,
+                                          c10::DispatchKey::BatchedNestedTensor, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Batched});
+  const auto plain = [&](const OptTensor& t) { return t && t->is_cuda() && !t->key_set().has_any(watching) && !t->_fw_grad(0).defined(); };
+  if (!plain(q) || q.dim() != 4) return {};
+  variable_list in = {q};
+  bool recorded = q.requires_grad();
+  for (const OptTensors* kind : {&ks, &vs, pes ? &*pes : nullptr})
+    for (int64_t j = 0; kind && j < visited_chunks(rank, cp, zigzag); ++j) {
+      if (!plain((*kind)[j])) return {};
+      in.push_back(*(*kind)[j]);
+      recorded |= in.back().requires_grad();
+    }
+  if (recorded && at::GradMode::is_enabled()) return RingFunction::apply(at::TensorList(in), scale, rank, cp, zigzag);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  if (auto done = ring_forward(q, ks, vs, pes, scale, rank, cp, zigzag)) return std::get<0>(*done);
+  return std::get<0>(python_body<Two>("ring_forward_local", q, ks, vs, scale, rank, cp, zigzag, pes));
+}
+
 // The backward ops have no derivative of their own: under create_graph their results carry a node that raises when somebody
 // differentiates through it (without one the dispatcher would only warn and leave the second-order part out).
 struct NoSecondDerivative : torch::autograd::Function<NoSecondDerivative> {
@@ -904,6 +988,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_bwd_pair_into", &attn_bwd_pair_into, Unlocked());
   m.def("ring_forward", &ring_forward, Unlocked());
   m.def("ring_backward", &ring_backward, Unlocked());
+  m.def("ring_attention", &ring_attention, Unlocked());
   m.def("combine_into", &combine_into, Unlocked());
   m.def("combine_new", &combine_new, Unlocked());
   m.def("cast_f32_bf16_into", &cast_f32_bf16_into, Unlocked());

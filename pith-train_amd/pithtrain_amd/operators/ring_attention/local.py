@@ -417,8 +417,21 @@ def ring_backward_local(
     return bwd.finish(), dk_list, dv_list, dpe_list
 
 
+def _forward_body(q, ks, vs, scale, rank, cp, zigzag, pes):
+    return ring_forward_local(q, ks, vs, scale, rank, cp, "zigzag" if zigzag else "contiguous", pes)
+
+
+def _backward_body(dout, q, out, lse, ks, vs, scale, rank, cp, zigzag, pes):
+    grads = ring_backward_local(dout, q, out, lse, ks, vs, scale, rank, cp, "zigzag" if zigzag else "contiguous", pes)
+    return grads if pes is not None else (*grads, [])
+
+
+# what the native share (csrc/host/torch_ops.cpp, RingFunction) hands back: step-wise shares and the dS hand-over
+native.set_bodies({"ring_forward_local": _forward_body, "ring_backward_local": _backward_body})
+
+
 class RingAttentionLocalFunc(torch.autograd.Function):
-    """autograd wrapper of one rank's ring share; gradients flow to q and to every visited chunk.
+    """The same in Python, for tensors and modes that look at every operation: autograd wrapper of one rank's ring share; gradients flow to q and to every visited chunk.
     *kv holds cp_size K chunks and cp_size V chunks, optionally followed by cp_size k_pe chunks
     (keys in two parts)."""
 
@@ -462,6 +475,10 @@ def ring_attention_local(
     With k_pe_chunks the keys come in two parts (k_chunks = k_nope, see the module docstring)."""
     assert len(k_chunks) == cp_size and len(v_chunks) == cp_size
     assert k_pe_chunks is None or len(k_pe_chunks) == cp_size
+    if layout in LAYOUTS and FUSE_CHUNKS and not torch.compiler.is_compiling():
+        out = native.ring_attention(q, k_chunks, v_chunks, k_pe_chunks, softmax_scale, cp_rank, cp_size, layout == "zigzag")
+        if out is not None:
+            return out
     # Chunks the schedule never visits may be None; autograd needs tensors, so they are replaced
     # by empty placeholders that receive no gradient.
     visited = {st.kv_rank for st in ring_schedule(cp_rank, cp_size, q.shape[1], layout)}
