@@ -843,20 +843,14 @@ struct RingFunction : torch::autograd::Function<RingFunction> {
     const Tensor &out = s[0], &lse = s[1], &q = s[2];
     const auto lists = chunk_lists(s, 3, cp, visited);
     std::optional<RingGrads> g;
-    if (!may_hand_over(q, rank, cp, zigzag)) g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
+    if (q.size(3) != 128)  // whether steps of 128 features hand dS over is the Python body's decision
+      g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
     if (!g) g = python_body<RingGrads>("ring_backward_local", grads[0], q, out, lse, lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
     variable_list r = {std::get<0>(*g)};
     for (const OptTensors* kind : {&std::get<1>(*g), &std::get<2>(*g), &std::get<3>(*g)})
       for (int64_t j = 0; j < visited && j < (int64_t)kind->size(); ++j) r.push_back(or_undefined((*kind)[j]));
     r.resize(s.size() - 2 + 4);  // scale, rank, cp, zigzag
     return r;
-  }
-  // Whether a step of the share may hand dS over, a decision that the Python body makes.
-  static bool may_hand_over(const Tensor& q, int64_t rank, int64_t cp, bool zigzag) {
-    if (q.size(3) != 128) return false;
-    const int64_t cus = compute_units(q.device().index());
-    const auto pays = [&](int64_t rows, bool causal) { return ds_handover_pays((rows + 511) / 512 * q.size(2) * q.size(0), causal, cus); };
-    return pays(q.size(1), true) || (rank > 0 && pays(q.size(1), false)) || (zigzag && rank + 1 < cp && pays(q.size(1) / 2, false));
   }
 };
 
