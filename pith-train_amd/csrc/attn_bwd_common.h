@@ -239,11 +239,15 @@ __device__ __forceinline__ void decode_dkdv_block(int linear, int per_level, int
 
 // dK/dV kernels: a workgroup owns kDkdvBlockN key rows (the grid and the head split depend on it).
 constexpr int kDkdvBlockN = 128;
+constexpr int kDkdvWideN = 256;  // ... of attn_bwd_dkdv_wide.h
 // dK/dV for head dims (64, 64): attn_bwd_dkdv_d64.hip. Conventions as below.
 void launch_dkdv_d64(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
 
 // dK/dV for head dims (128, 128): attn_bwd_dkdv_d128.hip. p.tiles, p.split, p.ws_* are set by the caller.
 void launch_dkdv_d128(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
+
+// The same with kDkdvWideN key rows per workgroup: attn_bwd_dkdv_wide.hip.
+void launch_dkdv_wide(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);
 
 // dK/dV for head dims (192, 128): attn_bwd_dkdv_d192.hip. Same conventions.
 void launch_dkdv_d192(const BwdParams& p, bool causal, bool f32_out, unsigned grid, hipStream_t stream);

@@ -6,6 +6,7 @@
 // different workgroups (more parallelism when there are few key tiles); the parts leave fp32
 // partial results in a caller-provided workspace and a second kernel adds them in a fixed
 // order, so the result does not depend on scheduling.
+#include <algorithm>
 #include <mutex>
 
 #include "attn_bwd_common.h"
@@ -13,7 +14,7 @@
 namespace pith {
 namespace {
 
-constexpr int kBN = kDkdvBlockN;  // key rows per workgroup
+constexpr int kBN = kDkdvBlockN;  // key rows per workgroup (128 features: or kDkdvWideN)
 
 // out[b, s, h, :] (+)= sum over parts of ws[part][b][s][h][:], parts added in index order; blockIdx.y picks the item (dK and
 // dV of a call, or those of all its chunks).
@@ -87,7 +88,6 @@ int pick_split(const pith_attn_bwd_args* a, int64_t tiles) {
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
   return split;
 }
-int pick_split(const pith_attn_bwd_args* a) { return pick_split(a, (a->Skv + kBN - 1) / kBN); }
 
 // Workspace layout: [head-split partial dK | partial dV] (split > 1), then the per-head gradients of a
 // shared k_pe [Hkv][B][Skv][64] (keys in two parts).
@@ -100,12 +100,46 @@ int64_t dkpe_bytes_for(const pith_attn_bwd_args* a) {
 }
 int64_t workspace_bytes_for(const pith_attn_bwd_args* a, int split) { return split_bytes_for(a, split) + dkpe_bytes_for(a); }
 
+// How a dK/dV call is cut: key rows per workgroup and head parts. A pair in one grid with dQ has workgroups of kBN rows.
+struct Plan {
+  int rows, split;
+};
+Plan plan_for(const pith_attn_bwd_args* a, int rows) { return {rows, pick_split(a, (a->Skv + rows - 1) / rows)}; }
+
+// Whether a call of 128 features, launched alone, goes to the workgroups of kDkdvWideN keys (attn_bwd_dkdv_wide.h), which are
+// 4-7 % faster per product. Half as many workgroups cost
+//   - without a mask, a longer last round: the rounds are compared (5000 x 16 heads, 320 workgroups of 256 keys: +17 %);
+//   - under it, balance, below two workgroups per unit (8192 x 8/8 +34 %, 12288 x 8/8, 1.5 per unit, +5 %), and the products of
+//     256 instead of 128 keys with rows that see none of them, so not for short rows;
+//   - a finer head split, whose partial sums make a round trip: each part needs work for it. dK/dV + sums, 128 -> 256 keys, us,
+//     (mean rows per key) x (heads of a part) behind it: causal 4096 x 32/4 293 -> 311 (2048), 6144 x 32/4 651 -> 668 (3072),
+//     4096 x 64/4 600 -> 585 (4096), 8192 x 32/4 1141 -> 1100 (8192); full 3072 x 32/4 339 -> 344 (3072), 2 x 2048 x 32/4 267 ->
+//     268 (4096 in short rows), 4096 x 32/4 529 -> 514 (8192), 8192 x 4096 x 32/4 1061 -> 1018, 16384 x 8192 x 16/1 2077 -> 1992.
+// Without a finer split: full 16 x 1024 x 16 333 -> 309, 8192 x 16 1064 -> 1013; causal 16 x 1024 x 16 221 -> 215, 2 x 8192 x 8
+// 579 -> 545 (all handing dS over; recomputing 0-7 % faster). A call that fits the built-in scratch of pith_attn_bwd_dkdv_static
+// with 128 keys has to fit it with 256, too: both entry points add up in the same order.
+bool wide(const pith_attn_bwd_args* a, const Plan& n, const Plan& w) {
+  if (a->Dqk != 128 || a->Sq < (a->causal ? 1024 : 512)) return false;
+  const int64_t cus = compute_units_or_default(), heads = a->Hkv * a->B;
+  const int64_t narrow_wgs = (a->Skv + n.rows - 1) / n.rows * heads * n.split, wide_wgs = (a->Skv + w.rows - 1) / w.rows * heads * w.split;
+  const int64_t narrow_heads = a->Hq / a->Hkv / n.split, wide_heads = a->Hq / a->Hkv / w.split;
+  if (w.split > 1 && (a->Sq < 4096 || (a->causal ? a->Sq / 2 : a->Sq) * wide_heads < 4096)) return false;
+  const int64_t fits = PITH_DKDV_STATIC_SCRATCH_BYTES;
+  if (workspace_bytes_for(a, w.split) > fits && workspace_bytes_for(a, n.split) <= fits) return false;
+  if (a->causal) return wide_wgs >= 2 * cus;
+  return (wide_wgs + cus - 1) / cus * 2 * wide_heads <= (narrow_wgs + cus - 1) / cus * narrow_heads;
+}
+Plan pick_plan(const pith_attn_bwd_args* a) {
+  const Plan n = plan_for(a, kBN), w = plan_for(a, kDkdvWideN);
+  return wide(a, n, w) ? w : n;
+}
+
 constexpr int64_t kWalkDescBytes = 192ll << 20;
 
 // with_dq: dQ of the pair in the same grid (p prepared for it)
 template <int DQK, int DV>
-void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, bool with_dq, hipStream_t st) {
-  p.tiles = (int)((a->Skv + kBN - 1) / kBN);
+void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_dq, hipStream_t st) {
+  p.tiles = (int)((a->Skv + rows - 1) / rows);
   p.accumulate = a->accumulate_dkv;
   p.main_blocks = (int)(p.tiles * a->Hkv * a->B * p.split);
   p.zero_tail = a->accumulate_dkv ? 0 : (int)a->dkv_zero_tail;  // rows that are added to keep what they hold
@@ -116,7 +150,8 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, bool with_dq, hipStre
   } else if constexpr (DQK == 128 && DV == 128) {
     // descending walk under the mask when Q and dO together exceed what the last-level cache (256 MB) keeps
     p.walk_desc = a->causal != 0 && (int64_t)a->B * a->Sq * a->Hq * (DQK + DV) * 2 > kWalkDescBytes;
-    launch_dkdv_d128(p, a->causal != 0, f32, grid, st);
+    if (rows == kDkdvWideN) launch_dkdv_wide(p, a->causal != 0, f32, grid, st);
+    else launch_dkdv_d128(p, a->causal != 0, f32, grid, st);
   } else if constexpr (DQK == 192 && DV == 128) {
     launch_dkdv_d192(p, a->causal != 0, f32, grid, st);
   } else {
@@ -142,7 +177,8 @@ using namespace pith;
 
 extern "C" int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* a) {
   if (!a || a->Hkv <= 0 || a->Hq <= 0 || a->Hq % a->Hkv != 0 || a->B <= 0 || a->Skv <= 0) return 0;
-  return workspace_bytes_for(a, pick_split(a));
+  // of the call alone or in one grid with dQ
+  return std::max(workspace_bytes_for(a, pick_plan(a).split), workspace_bytes_for(a, plan_for(a, kBN).split));
 }
 
 namespace {
@@ -158,7 +194,8 @@ int validate_dk_pe(const pith_attn_bwd_args* a, const char* who) {
 }
 
 // Runs the kernels with the head-split partials in `workspace` (NULL: no head split).
-int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_t st, const char* who, bool with_dq = false) {
+int run_dkdv(const pith_attn_bwd_args* a, const Plan& plan, void* workspace, hipStream_t st, const char* who, bool with_dq = false) {
+  const int split = plan.split;
   // the grid of this kernel runs over key tiles (validate_bwd bounded the query-side grid)
   if (((a->Skv + kBN - 1) / kBN) * a->Hkv * a->B * (int64_t)split > 0x7fffffffLL)
     return fail(PITH_ERR_UNSUPPORTED, "%s: Skv=%lld x Hkv=%lld x B=%lld exceeds the launch grid limit", who,
@@ -182,9 +219,9 @@ int run_dkdv(const pith_attn_bwd_args* a, int split, void* workspace, hipStream_
     if ((uintptr_t)a->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
     p.ds = reinterpret_cast<char*>(a->ds);
   }
-  if (a->Dqk == 128) launch_dkdv<128, 128>(p, a, with_dq, st);
-  else if (a->Dqk == 192) launch_dkdv<192, 128>(p, a, with_dq, st);
-  else launch_dkdv<64, 64>(p, a, with_dq, st);
+  if (a->Dqk == 128) launch_dkdv<128, 128>(p, a, plan.rows, with_dq, st);
+  else if (a->Dqk == 192) launch_dkdv<192, 128>(p, a, plan.rows, with_dq, st);
+  else launch_dkdv<64, 64>(p, a, plan.rows, with_dq, st);
   return check_launch(who);
 }
 
@@ -224,13 +261,16 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
   const int rc = validate_bwd(a, who, false, true);
   if (rc != PITH_OK) return rc;
   // Head groups are split only when the caller brought a workspace that is large enough.
-  int split = pick_split(a);
-  if (!(split > 1 && a->workspace && a->workspace_bytes >= workspace_bytes_for(a, split))) split = 1;
+  const Plan narrow = plan_for(a, kBN);
+  const auto fits = [&](const Plan& plan) { return plan.split == 1 || (a->workspace && a->workspace_bytes >= workspace_bytes_for(a, plan.split)); };
+  Plan plan = with_dq ? narrow : pick_plan(a);
+  if (!fits(plan)) plan = narrow;
+  if (!fits(plan)) plan.split = 1;
   if (a->workspace && !aligned16(a->workspace)) return fail(PITH_ERR_MISALIGNED, "%s: workspace must be 16-byte aligned", who);
-  if (a->k_pe && (!a->workspace || a->workspace_bytes < workspace_bytes_for(a, split)))
+  if (a->k_pe && (!a->workspace || a->workspace_bytes < workspace_bytes_for(a, plan.split)))
     return fail(PITH_ERR_BAD_SHAPE, "%s: keys in two parts need a workspace of %lld bytes, %lld given", who,
-                (long long)workspace_bytes_for(a, split), (long long)(a->workspace ? a->workspace_bytes : 0));
-  return run_dkdv(a, split, a->workspace, (hipStream_t)stream, who, with_dq);
+                (long long)workspace_bytes_for(a, plan.split), (long long)(a->workspace ? a->workspace_bytes : 0));
+  return run_dkdv(a, plan, a->workspace, (hipStream_t)stream, who, with_dq);
 }
 
 // Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
@@ -285,8 +325,8 @@ extern "C" int pith_attn_bwd_dkdv_static(const pith_attn_bwd_args* a, pith_strea
   const char* who = "pith_attn_bwd_dkdv_static";
   const int rc = validate_bwd(a, who, false, true);
   if (rc != PITH_OK) return rc;
-  const int split = pick_split(a);
-  const int64_t need = workspace_bytes_for(a, split);
+  const Plan plan = pick_plan(a);
+  const int64_t need = workspace_bytes_for(a, plan.split);
   if (need > kStaticScratchBytes)
     return fail(PITH_ERR_UNSUPPORTED,
                 "%s: the head-split partial sums of this shape need %lld bytes, the built-in scratch holds %lld "
@@ -297,7 +337,7 @@ extern "C" int pith_attn_bwd_dkdv_static(const pith_attn_bwd_args* a, pith_strea
     const int src = static_scratch(&ws, who);
     if (src != PITH_OK) return src;
   }
-  return run_dkdv(a, split, ws, (hipStream_t)stream, who);
+  return run_dkdv(a, plan, ws, (hipStream_t)stream, who);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -21,7 +21,7 @@ OBJ_DIR = os.path.join(LIB_DIR, "obj")
 EXT_SRC = os.path.join(SRC_DIR, "host", "torch_ops.cpp")
 EXT_PATH = os.path.join(LIB_DIR, "_pith_torch.so")
 
-SOURCES = ["api.hip", "combine.hip", "norm_rope.hip", "mla_assemble.hip", "attn_fwd.hip", "attn_fwd_direct.hip", "attn_fwd_duo.hip", "attn_bwd_dq.hip", "attn_bwd_dq_direct.hip", "attn_bwd_dq_duo.hip", "attn_bwd_dq_ds.hip", "attn_bwd_dkdv.hip", "attn_bwd_pair.hip", "attn_bwd_chunks.hip", "attn_bwd_dkdv_d64.hip", "attn_bwd_dkdv_d128.hip", "attn_bwd_dkdv_d192.hip"]
+SOURCES = ["api.hip", "combine.hip", "norm_rope.hip", "mla_assemble.hip", "attn_fwd.hip", "attn_fwd_direct.hip", "attn_fwd_duo.hip", "attn_bwd_dq.hip", "attn_bwd_dq_direct.hip", "attn_bwd_dq_duo.hip", "attn_bwd_dq_ds.hip", "attn_bwd_dkdv.hip", "attn_bwd_pair.hip", "attn_bwd_chunks.hip", "attn_bwd_dkdv_d64.hip", "attn_bwd_dkdv_d128.hip", "attn_bwd_dkdv_wide.hip", "attn_bwd_dkdv_d192.hip"]
 
 # -packed-fp32-ops is switched off on purpose: some packed fp32 forms have produced wrong results
 # on the target machines. Code object v5 is understood by both the ROCm 7.0 runtime bundled with
