@@ -1,6 +1,6 @@
 // Entry points of the key/value-gradient step of one chunk attention backward for gfx950, against an external
 // (ring-combined) base-2 LSE and delta = rowsum(O*dO): argument checks, the head split and its reduction kernel. The
-// kernels are attn_bwd_dkdv_d64.hip, attn_bwd_dkdv_d128.hip and attn_bwd_dkdv_d192.hip.
+// kernels are attn_bwd_dkdv_d64.hip, attn_bwd_dkdv_d128.hip, attn_bwd_dkdv_wide.hip and attn_bwd_dkdv_d192.hip.
 //
 // With grouped-query attention the heads of a group may be cut into `split` parts handled by
 // different workgroups (more parallelism when there are few key tiles); the parts leave fp32
@@ -106,7 +106,7 @@ struct Plan {
 };
 Plan plan_for(const pith_attn_bwd_args* a, int rows) { return {rows, pick_split(a, (a->Skv + rows - 1) / rows)}; }
 
-// Whether a call of 128 features, launched alone, goes to the workgroups of kDkdvWideN keys (attn_bwd_dkdv_wide.h), which are
+// Whether a call of 128 features and not too few rows, launched alone, goes to the workgroups of kDkdvWideN keys (attn_bwd_dkdv_wide.h), which are
 // 4-7 % faster per product. Half as many workgroups cost
 //   - without a mask, a longer last round: the rounds are compared (5000 x 16 heads, 320 workgroups of 256 keys: +17 %);
 //   - under it, balance, below two workgroups per unit (8192 x 8/8 +34 %, 12288 x 8/8, 1.5 per unit, +5 %), and the products of
@@ -119,7 +119,6 @@ Plan plan_for(const pith_attn_bwd_args* a, int rows) { return {rows, pick_split(
 // 579 -> 545 (all handing dS over; recomputing 0-7 % faster). A call that fits the built-in scratch of pith_attn_bwd_dkdv_static
 // with 128 keys has to fit it with 256, too: both entry points add up in the same order.
 bool wide(const pith_attn_bwd_args* a, const Plan& n, const Plan& w) {
-  if (a->Dqk != 128 || a->Sq < (a->causal ? 1024 : 512)) return false;
   const int64_t cus = compute_units_or_default(), heads = a->Hkv * a->B;
   const int64_t narrow_wgs = (a->Skv + n.rows - 1) / n.rows * heads * n.split, wide_wgs = (a->Skv + w.rows - 1) / w.rows * heads * w.split;
   const int64_t narrow_heads = a->Hq / a->Hkv / n.split, wide_heads = a->Hq / a->Hkv / w.split;
@@ -129,8 +128,10 @@ bool wide(const pith_attn_bwd_args* a, const Plan& n, const Plan& w) {
   if (a->causal) return wide_wgs >= 2 * cus;
   return (wide_wgs + cus - 1) / cus * 2 * wide_heads <= (narrow_wgs + cus - 1) / cus * narrow_heads;
 }
-Plan pick_plan(const pith_attn_bwd_args* a) {
-  const Plan n = plan_for(a, kBN), w = plan_for(a, kDkdvWideN);
+// `n`: the plan with kBN rows
+Plan pick_plan(const pith_attn_bwd_args* a, const Plan& n) {
+  if (a->Dqk != 128 || a->Sq < (a->causal ? 1024 : 512)) return n;
+  const Plan w = plan_for(a, kDkdvWideN);
   return wide(a, n, w) ? w : n;
 }
 
@@ -178,7 +179,8 @@ using namespace pith;
 extern "C" int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* a) {
   if (!a || a->Hkv <= 0 || a->Hq <= 0 || a->Hq % a->Hkv != 0 || a->B <= 0 || a->Skv <= 0) return 0;
   // of the call alone or in one grid with dQ
-  return std::max(workspace_bytes_for(a, pick_plan(a).split), workspace_bytes_for(a, plan_for(a, kBN).split));
+  const Plan narrow = plan_for(a, kBN);
+  return workspace_bytes_for(a, std::max(pick_plan(a, narrow).split, narrow.split));
 }
 
 namespace {
@@ -263,7 +265,7 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
   // Head groups are split only when the caller brought a workspace that is large enough.
   const Plan narrow = plan_for(a, kBN);
   const auto fits = [&](const Plan& plan) { return plan.split == 1 || (a->workspace && a->workspace_bytes >= workspace_bytes_for(a, plan.split)); };
-  Plan plan = with_dq ? narrow : pick_plan(a);
+  Plan plan = with_dq ? narrow : pick_plan(a, narrow);
   if (!fits(plan)) plan = narrow;
   if (!fits(plan)) plan.split = 1;
   if (a->workspace && !aligned16(a->workspace)) return fail(PITH_ERR_MISALIGNED, "%s: workspace must be 16-byte aligned", who);
@@ -325,7 +327,7 @@ extern "C" int pith_attn_bwd_dkdv_static(const pith_attn_bwd_args* a, pith_strea
   const char* who = "pith_attn_bwd_dkdv_static";
   const int rc = validate_bwd(a, who, false, true);
   if (rc != PITH_OK) return rc;
-  const Plan plan = pick_plan(a);
+  const Plan plan = pick_plan(a, plan_for(a, kBN));
   const int64_t need = workspace_bytes_for(a, plan.split);
   if (need > kStaticScratchBytes)
     return fail(PITH_ERR_UNSUPPORTED,

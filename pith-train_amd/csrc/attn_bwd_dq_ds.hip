@@ -1,7 +1,7 @@
 // Query-gradient kernel for head dims (128, 128) on gfx950 that reads dS instead of recomputing it:
 // dQ = scale * dS K (pithtrain/operators/mla/triton.py:205-266, the last product of the loop body),
 // with dS = P*(dP - delta) taken, already rounded to bf16 and with its sign flipped, from the images
-// that the dK/dV kernel of attn_bwd_dkdv_d128.hip leaves in p.ds (layout documented there). The two score products that the
+// that the dK/dV kernels of attn_bwd_dkdv_d128.h and attn_bwd_dkdv_wide.h leave in p.ds (layout documented in the former). The two score products that the
 // other dQ kernels repeat are gone; the price is one trip of dS through memory, so this kernel is
 // bound by the rate at which it can stream the images, not by the matrix pipe.
 //
