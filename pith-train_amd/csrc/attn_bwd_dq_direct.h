@@ -388,16 +388,15 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   }
   scores(kslot(0), vslot(0));
   if (!late) make_ds(0, std::true_type{});
-  if constexpr (kLdsQ == 0) {
-    wait_staged();
-    __syncthreads();  // tile 1 is there, the query-side rows have been read
-  }
+  if constexpr (kLdsQ == 0) wait_staged();
+  // Tile 1 is there, and what the next requests write to has been read by every wave: the query-side rows (kDist 2: slots of
+  // tile 2), V(0) (kDist 1: slot of V(2), which the late waves request first thing in interval 0).
+  __syncthreads();
   if (kDist > 1 && n_tiles_wg > 2) request(2);
 
   // Interval i = 0 .. n_tiles_wg - 1 reads K(i) (gradient product), K(i+1) and V(i+1) (scores) and
-  // requests tile i + 1 + kDist (kDist 2: tile 2 has been, above), whose slots were last read in interval i - 1 (kDist 2: they held
-  // tile i - 1) or hold nothing that is still needed (kDist 1: K slot of tile i - 2, V slot of tile i,
-  // read in interval i - 1).
+  // requests tile i + 1 + kDist (kDist 2: tile 2 has been, above), whose slots were last read in interval i - 1 or, for i = 0,
+  // ahead of the barrier above (kDist 2: they held tile i - 1; kDist 1: K slot of tile i - 2, V slot of tile i).
   // FULL: this wave has both a tile to accumulate and a next tile to score.
   // MASKED: the tile whose dS this interval makes (i + 1 in the early waves, i in the late ones) may
   // need the mask.

@@ -381,6 +381,38 @@ def test_ds_storing_dkdv_kernel_waits_for_its_tile_loads_only(tmp_path_factory):
         assert not in_loop_blocks, f"stores or spills in out-of-line blocks of the loop: {in_loop_blocks}"
 
 
+def test_split_key_dq_requests_no_tile_over_one_still_read(tmp_path_factory):
+    """The split-key dQ kernel scores tile 0 ahead of its loop and then requests tiles into slots that other waves read for
+    that (V of tile 2 at 192 features, the staged rows at 128). Followed over the control flow of the compiler's output: between
+    the first product of a path and the first tile load behind it lies a workgroup barrier."""
+    text = _kernel_asm("attn_bwd_dq_direct.hip", tmp_path_factory.getbasetemp())
+    kernels = re.findall(r"^(_Z\w*attn_bwd_dq_direct_kernel\w*):(.*?)^\.Lfunc_end", text, re.M | re.S)
+    assert len(kernels) == 8, "head dims, mask, output type"
+    for name, body in kernels:
+        code = [re.sub(r"\s*;.*", "", l) for l in body.splitlines()]
+        label = {l[:-1]: i for i, l in enumerate(code) if re.match(r"\.LBB\w+:$", l)}
+        assert not any(re.match(r"\s+s_(setpc|swappc|call)", l) for l in code), "the paths below would not be all"
+        BEFORE, SCORED = 0, 1  # no product yet; products, and no barrier behind them
+        todo, seen, scored_then_synced = [(0, BEFORE)], set(), 0
+        while todo:
+            i, state = todo.pop()
+            while (i, state) not in seen:
+                seen.add((i, state))
+                op = code[i].split() or [""]
+                if op[0].startswith("v_mfma"):
+                    state = SCORED
+                elif op[0] == "s_barrier" and state == SCORED:
+                    scored_then_synced += 1
+                    break
+                assert state == BEFORE or "_load_lds" not in op[0], f"{name}: tile request before the barrier, line {i}"
+                if op[0].startswith("s_cbranch"):
+                    todo.append((label[op[1]], state))
+                if op[0] == "s_endpgm":
+                    break
+                i = label[op[1]] if op[0] == "s_branch" else i + 1
+        assert scored_then_synced
+
+
 def test_attn_bwd_rejects_before_its_first_launch():
     """As two launches (dK/dV, then dQ) the call must find bad arguments of the second before the first goes out. There is no
     device here, so a launch would show as PITH_ERR_LAUNCH."""
