@@ -303,6 +303,16 @@ int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* args);
  * behave as before. */
 int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* args);
 
+/* How the backward calls of these shapes are cut on the current device, for tests and profiles: no results depend on it except
+ * by fp32 summation order. Only the shapes and `causal` are read. */
+typedef struct {
+  int32_t dkdv_rows;    /* pith_attn_bwd_dkdv, launched alone: key rows per workgroup */
+  int32_t dkdv_split;   /* and the parts each group of query heads is cut into (given the workspace) */
+  int32_t dq_ds_pairs;  /* pith_attn_bwd_dq from handed-over dS, causal: workgroups take rows from both ends */
+} pith_attn_bwd_plan_t;
+
+int pith_attn_bwd_plan(const pith_attn_bwd_args* args, pith_attn_bwd_plan_t* plan);
+
 /* pith_attn_bwd_dkdv for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). It has no counterpart in the
  * reference. Same arguments and results, bit for bit, as pith_attn_bwd_dkdv called with a

@@ -42,6 +42,7 @@ struct BwdParams {
   char* ds;
   int ds_qt, ds_kb;
   int64_t ds_hs;
+  int ds_pairs;  // dQ from dS under the mask: a workgroup takes 256-row blocks from both ends (dq_ds_pairs)
   // dQ kernels, fp32 dq: query rows [final_r0, final_r1) (multiples of 32, or Sq) receive their result, old
   // contents of dq included when accumulating, as bf16 in dq_final instead of dq (nullptr: none do)
   __bf16* dq_final;
@@ -270,7 +271,9 @@ void launch_dq_duo(const BwdParams& p, int dqk, bool causal, bool f32_out, hipSt
 
 // dQ for head dims (128, 128) from the dS images the dK/dV kernel left in p.ds: attn_bwd_dq_ds.hip.
 // p.q_tiles = number of 512-row query tiles.
-void launch_dq_from_ds(const BwdParams& p, bool causal, bool f32_out, hipStream_t stream);
+// Whether under the mask a grid of that many workgroups takes 256-row blocks from both ends of the rows.
+bool dq_ds_pairs(int64_t workgroups);
+void launch_dq_from_ds(BwdParams p, bool causal, bool f32_out, hipStream_t stream);
 // Bytes of dS images for a shape (0: the shape has no hand-over path), and whether the call brings a buffer for them.
 int64_t ds_bytes_for(const pith_attn_bwd_args* a);
 bool ds_usable(const pith_attn_bwd_args* a);

@@ -183,6 +183,18 @@ extern "C" int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* 
   return workspace_bytes_for(a, std::max(pick_plan(a, narrow).split, narrow.split));
 }
 
+extern "C" int pith_attn_bwd_plan(const pith_attn_bwd_args* a, pith_attn_bwd_plan_t* plan) {
+  const char* who = "pith_attn_bwd_plan";
+  if (!a || !plan) return fail(PITH_ERR_NULL_POINTER, "%s: %s is NULL", who, a ? "plan" : "args");
+  if (a->Hkv <= 0 || a->Hq <= 0 || a->Hq % a->Hkv != 0 || a->B <= 0 || a->Sq <= 0 || a->Skv <= 0)
+    return fail(PITH_ERR_BAD_SHAPE, "%s: bad shape", who);
+  const Plan chosen = pick_plan(a, plan_for(a, kBN));
+  plan->dkdv_rows = chosen.rows;
+  plan->dkdv_split = chosen.split;
+  plan->dq_ds_pairs = a->causal && ds_bytes_for(a) > 0 && dq_ds_pairs((a->Sq + 511) / 512 * a->Hq * a->B);
+  return PITH_OK;
+}
+
 namespace {
 
 // Keys in two parts: what the dK/dV side asks of them.

@@ -6,9 +6,8 @@
 // bound by the rate at which it can stream the images, not by the matrix pipe.
 //
 // Work split: a workgroup of 8 wavefronts owns 512 query rows of one (batch, head), a wave one 64-row query tile of the
-// writer (under the mask two blocks of 256 rows, one near the start and one near the end: with 512 consecutive rows the
-// heaviest of 8 workgroups of a 4096-row head carried twice the average and a single round of them did not pay). Keys are visited in steps of 32 (one wave pair of the
-// writer). Per step the K tile (shared, packed and swizzled like everywhere else, 8 KB) and, per
+// writer (under the mask in a grid of one round two blocks of 256 rows, see dq_ds_pairs). Keys are visited in steps of 32 (one
+// wave pair of the writer). Per step the K tile (shared, packed and swizzled like everywhere else, 8 KB) and, per
 // wave, the 4 KB image of its tile for that pair (copied verbatim) go global -> LDS directly. What
 // bounds the kernel is how many bytes of dS each compute unit keeps in flight (a compute unit's
 // vector cache holds about 64 outstanding 128-byte requests, i.e. ~8 KB per ~650 cycles of latency, so
@@ -79,17 +78,18 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   int m_tile, h, b;
   decode_block(blockIdx.x, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b);
   const int hk = h / p.group;
-  // Query tiles of the waves. Without a mask eight consecutive ones. Under it the workgroup takes two 256-row blocks, waves
-  // 0..3 the m_tile-th from the start and waves 4..7 the m_tile-th from the end, so that all workgroups read the same number
-  // of images (the middle one of an odd number of blocks goes to waves 4..7 alone).
+  // Query tiles of the waves: eight consecutive ones, or, with ds_pairs, two 256-row blocks, waves 0..3 the m_tile-th from the
+  // start and waves 4..7 the m_tile-th from the end, so that all workgroups read the same number of images (the middle one of
+  // an odd number of blocks goes to waves 4..7 alone).
+  const bool pairs = CAUSAL && p.ds_pairs;
   const int blocks256 = (p.Sq + kBM / 2 - 1) / (kBM / 2);
   auto rows_of = [&](int w) __attribute__((always_inline)) {
-    if (!CAUSAL) return m_tile * kBM + w * QW;
+    if (!pairs) return m_tile * kBM + w * QW;
     const int late = blocks256 - 1 - m_tile;
     const int block = w >= 4 ? late : m_tile < late ? m_tile : blocks256;  // blocks256: none
     return block * (kBM / 2) + (w & 3) * QW;
   };
-  const int m_end = CAUSAL ? (blocks256 - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
+  const int m_end = pairs ? (blocks256 - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
   const int q_wave0 = rows_of(wave), q_other0 = rows_of(wave & 3);  // q_other0: of the wave whose images waves 4..7 also request
 
   const int kv_row_bytes = p.HkvT * DQK * 2;
@@ -254,7 +254,19 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
 
 }  // namespace
 
-void launch_dq_from_ds(const BwdParams& p, bool causal, bool f32_out, hipStream_t st) {
+// Under the mask a workgroup of 512 consecutive rows carries up to twice the average work. In a grid of one round the heaviest
+// one is the kernel's time, so there the rows go out as pairs of blocks of equal work. In more rounds consecutive rows, the
+// heaviest first, fill the units by themselves, while pairs, all alike, leave the last round as empty as it is. The kernel
+// alone, consecutive rows / pairs, us:
+//   one round         4096 x 32/4 heads 143 / 118, 8192 x 16 273 / 219, 4 x 1024 x 32/4 38 / 35, 8 x 512 x 32/4 24 / 24
+//   1.125 rounds      9216 x 16 328 / 382, 4608 x 32/4 168 / 204, 3 x 1536 x 32/4 55 / 89
+//   1.25, 1.5, 1.75   5120 x 32/4 196 / 225, 6144 x 32/4 256 / 271, 3 x 1999 x 32/4 102 / 114, 7168 x 32/4 322 / 337
+//   2, 2.25           8192 x 32/4 405 / 409, 2 x 4096 x 32/4 224 / 233, 9216 x 32/4 517 / 599
+//   2.75, 3, 4        11264 x 32/4 785 / 799, 12288 x 32/4 921 / 904, 3 x 4096 x 32/4 341 / 353, 16384 x 32/4 1524 / 1565
+bool dq_ds_pairs(int64_t workgroups) { return workgroups <= compute_units_or_default(); }
+
+void launch_dq_from_ds(BwdParams p, bool causal, bool f32_out, hipStream_t st) {
+  p.ds_pairs = dq_ds_pairs((int64_t)p.q_tiles * p.Hq * p.B);
   const dim3 grid((unsigned)(p.q_tiles * p.Hq * p.B)), block(kThreads);
   if (causal) {
     if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<true, float>), grid, block, 0, st, p);

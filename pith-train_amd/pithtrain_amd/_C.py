@@ -99,6 +99,10 @@ class AttnBwdArgs(Structure):
     ]  # fmt: skip
 
 
+class AttnBwdPlan(Structure):
+    _fields_ = [("dkdv_rows", c_int32), ("dkdv_split", c_int32), ("dq_ds_pairs", c_int32)]
+
+
 class NormRopeArgs(Structure):
     _fields_ = [
         ("x", c_void_p), ("weight", c_void_p), ("cos", c_void_p), ("sin", c_void_p), ("dout", c_void_p),
@@ -145,6 +149,7 @@ SYMBOLS = {
     "pith_attn_bwd_dkdv_static": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dkdv_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
     "pith_attn_bwd_ds_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
+    "pith_attn_bwd_plan": (c_int, [POINTER(AttnBwdArgs), POINTER(AttnBwdPlan)]),
     "pith_cast_f32_bf16": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "pith_norm_rope_fwd": (c_int, [POINTER(NormRopeArgs), c_void_p]),
     "pith_norm_rope_bwd": (c_int, [POINTER(NormRopeArgs), c_void_p]),
@@ -237,6 +242,6 @@ def bhs_strides(t: torch.Tensor, what: str):
 
 
 __all__ = [
-    "lib", "check", "PithError", "CombineArgs", "AttnFwdArgs", "KeyChunk", "AttnDeltaArgs", "AttnBwdArgs", "NormRopeArgs", "MlaAssembleArgs", "DeviceInfo", "SYMBOLS",
+    "lib", "check", "PithError", "CombineArgs", "AttnFwdArgs", "KeyChunk", "AttnDeltaArgs", "AttnBwdArgs", "AttnBwdPlan", "NormRopeArgs", "MlaAssembleArgs", "DeviceInfo", "SYMBOLS",
     "dtype_code", "current_stream", "require_device", "bshd_batch_stride", "bshd_head_range_strides", "bhs_strides", "byref",
 ]  # fmt: skip

@@ -90,6 +90,34 @@ def test_causal_pairs_of_row_blocks(gpu, S):
     _run(gpu, True, (1, S, S, 2, 1), torch.bfloat16)
 
 
+@pytest.mark.parametrize("B,S", [(17, 255), (9, 513), (9, 1024), (6, 1025), (5, 1537), (4, 2049), (4, 2303)])
+def test_consecutive_rows_equal_pairs(gpu, B, S):
+    """More than one round of workgroups takes consecutive rows, a batch element alone pairs of blocks: the same sums."""
+    from pithtrain_amd import _C
+
+    g = torch.Generator(device=gpu).manual_seed(S)
+    t = lambda h: torch.randn(B, S, h, 128, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v, dout = t(16), t(2), t(2), t(16)
+    o, lse = _mla_fwd(q, k, v, 0.09, True)
+    delta = _mla_bwd_preprocess(o, dout)
+
+    def dq_of(*x):
+        args, plan = _C.AttnBwdArgs(B=x[0].shape[0], Sq=S, Skv=S, Hq=16, Hkv=2, Dqk=128, Dv=128, causal=1), _C.AttnBwdPlan()
+        _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+        ds = torch.full((attn_bwd_ds_bytes(*x[:3], True),), 0x7F, dtype=torch.uint8, device=gpu)
+        dk, dv, dq = torch.empty_like(x[1]), torch.empty_like(x[2]), torch.full_like(x[0], float("nan"))
+        attn_bwd_dkdv_into(*x, dk, dv, 0.09, True, ds=ds)
+        attn_bwd_dq_into(*x, dq, 0.09, True, ds=ds)
+        return dq, plan.dq_ds_pairs
+
+    whole, pairs = dq_of(q, k, v, dout, lse, delta)
+    if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
+        assert not pairs
+    for b in range(B):
+        one, pairs = dq_of(*[x[b : b + 1] for x in (q, k, v, dout, lse, delta)])
+        assert pairs and torch.equal(whole[b : b + 1], one), f"batch element {b}"
+
+
 @pytest.mark.parametrize("shape", NONCAUSAL_SHAPES)
 def test_noncausal_dq_from_ds(gpu, shape):
     _run(gpu, False, shape, torch.bfloat16)
