@@ -447,26 +447,25 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
   return python_body<Two>("attn_fwd", q, k, v, scale, causal);
 }
 
-// Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup, all of about the same length) beats recomputing
-// the scores: it has to fill the device, and under the mask, where a workgroup reads half as much and the rounds are short, it
-// must not leave most of its last round empty. W = workgroups per compute unit; forward + backward, handing over / recomputing:
-//   causal  W 1     1 x 4096 x 32/4 heads 578 / 600 us, 2 x 2048 x 32/4 337 / 340, 4 x 1024 x 32/4 208 / 219, 8 x 512 x 32/4 179 / 192
-//           W 1.12  9216 x 16 1469 / 1428, 3 x 1536 x 32/4 332 / 324       W 1.25  5120 x 32/4 936 / 950, 2 x 2560 x 32/4 527 / 525
-//           W 1.5   6144 x 32/4 1265 / 1314, 6 x 1024 x 32/4 318 / 324, 3 x 1999 x 32/4 515 / 507, 2 x 3072 x 32/4 726 / 714
-//           W 1.75  7168 x 32/4 1692 / 1720    W 2  8192 x 32/4 2130 / 2194    W 2.25  9 x 1024 x 32/4 456 / 472, 9216 x 32/4 2863 / 2821
-//           W 0.75  3072 x 32/4 391 / 390
-//   full    W 1.12  4608 x 32/4 1663 / 1730, 9216 x 16 2766 / 2899         W 1.25  5120 x 32/4 1878 / 1930    W 1.5  6144 x 32/4 2487 / 2480
-bool ds_handover_pays(int64_t workgroups, bool causal, int64_t cus) {
-  if (cus <= 0 || workgroups < cus) return false;
-  return !causal || 10 * workgroups >= 7 * cus * ((workgroups + cus - 1) / cus);
-}
+// Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill the
+// device. W = workgroups per compute unit; forward + backward, inputs changing, handing over / recomputing, us:
+//   causal  W 1     4096 x 32/4 heads 561 / 576, 8192 x 16 1030 / 1059, 2 x 2048 x 32/4 323 / 332, 4 x 1024 x 32/4 204 / 215, 8 x 512 x 32/4 148 / 162
+//           W 1.12  9216 x 16 1378 / 1392, 3 x 1536 x 32/4 305 / 312, 9 x 512 x 32/4 189 / 190       W 1.03  2 x 1536 x 44/4 507 / 480 (the one
+//                   shape found that loses: eleven heads to a group)
+//           W 1.25  5120 x 32/4 891 / 914, 2 x 2560 x 32/4 496 / 502       W 1.5   6144 x 32/4 1229 / 1265, 6 x 1024 x 32/4 310 / 317,
+//                   3 x 1999 x 32/4 487 / 500, 2 x 3072 x 32/4 677 / 693   W 1.75  7168 x 32/4 1600 / 1651
+//           W 2     8192 x 32/4 2055 / 2103, 16 x 512 x 32/4 262 / 276     W 2.25  9216 x 32/4 2611 / 2721, 9 x 1024 x 32/4 443 / 461
+//           W 3     12288 x 32/4 4524 / 4756                               W 4     16384 x 32/4 7929 / 8004, 16 x 1024 x 32/4 718 / 736
+//   full    W 1     2 x 2048 x 32/4 534 / 539    W 1.12  4608 x 32/4 1625 / 1670, 9216 x 16 2716 / 2798
+//           W 1.25  5120 x 32/4 1833 / 1887      W 1.5   6144 x 32/4 2367 / 2426
+bool ds_handover_pays(int64_t workgroups, int64_t cus) { return cus > 0 && workgroups >= cus; }
 
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
   // Calls large enough for the dS hand-over belong to the Python body, which owns the policy for the hand-over buffer: their
   // kernels outlast its host work many times over.
   bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4;
   if (small && q.size(3) == 128) {
-    small = !ds_handover_pays((q.size(1) + 511) / 512 * q.size(2) * q.size(0), causal, compute_units(q.device().index()));
+    small = !ds_handover_pays((q.size(1) + 511) / 512 * q.size(2) * q.size(0), compute_units(q.device().index()));
   }
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);

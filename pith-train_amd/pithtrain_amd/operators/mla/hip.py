@@ -199,7 +199,8 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
 
 # The dS hand-over (head dims 128/128) makes the backward of a chunk pair 1-5 % faster (share of 8192 rows, 32/4 heads,
 # four ranks: 6.15 -> 5.92 ms; the gain differs between machines) at the price of a transient buffer of
-# Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask).
+# Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask: a layer of 4096 rows, 32/4 heads,
+# takes 0.55 GB for 3 % of its forward + backward).
 # Policy: the buffer never exceeds DS_BUFFER_LIMIT_BYTES nor DS_BUFFER_FREE_FRACTION of the device memory that is
 # free right now; a chunk pair that needs more is processed one group of kv heads (with their query heads) after
 # the other through one buffer of the bounded size; when not even one kv head fits, or the allocation fails, the
@@ -238,7 +239,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
     b, sq, hq, _ = q.shape
     hkv = k.shape[2]
     row_tiles = -(-sq // _DS_ROWS_PER_WORKGROUP)
-    if not native.ds_handover_pays(row_tiles * hq * b, causal, _device_compute_units(q.device)):  # nor for any slab
+    if not native.ds_handover_pays(row_tiles * hq * b, _device_compute_units(q.device)):  # nor for any slab
         return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:

@@ -5,6 +5,7 @@ import heapq
 import pytest
 
 from pithtrain_amd import _C
+from pithtrain_amd._ext import native
 
 UNITS = 256
 
@@ -44,3 +45,14 @@ def test_dq_from_ds_goes_out_in_the_order_that_ends_first(tiles, heads):
     assert chosen <= 1.1 * min(consecutive, pairs)
     if tiles * heads <= UNITS:
         assert chosen == pairs
+
+
+@pytest.mark.parametrize("b,s,hq", [(1, 4096, 32), (2, 2048, 32), (8, 512, 32), (1, 8192, 16), (1, 9216, 16), (3, 1536, 32), (2, 2560, 32), (1, 5120, 32),
+                                    (6, 1024, 32), (3, 1999, 32), (2, 3072, 32), (1, 7168, 32), (1, 9216, 32), (1, 10240, 32)])  # fmt: skip
+def test_layers_that_gain_hand_ds_over(b, s, hq):
+    """Causal layers measured faster with the hand-over than without (table at ds_handover_pays)."""
+    assert native.ds_handover_pays(-(-s // 512) * hq * b, UNITS)
+
+
+def test_grids_that_do_not_fill_the_device_recompute():
+    assert not native.ds_handover_pays(UNITS - 1, UNITS) and not native.ds_handover_pays(10 * UNITS, 0)
