@@ -253,7 +253,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
             heads -= 1
     if per_kv_head * heads > budget:
         return None
-    if row_tiles * (hq // hkv) * heads * b < _device_compute_units(q.device):
+    if heads < hkv and not native.ds_handover_pays(row_tiles * (hq // hkv) * heads * b, _device_compute_units(q.device)):
         return None
     return heads, per_kv_head * heads
 

@@ -3,9 +3,11 @@
 import heapq
 
 import pytest
+import torch
 
 from pithtrain_amd import _C
 from pithtrain_amd._ext import native
+from pithtrain_amd.operators.mla import hip as H
 
 UNITS = 256
 
@@ -56,3 +58,23 @@ def test_layers_that_gain_hand_ds_over(b, s, hq):
 
 def test_grids_that_do_not_fill_the_device_recompute():
     assert not native.ds_handover_pays(UNITS - 1, UNITS) and not native.ds_handover_pays(10 * UNITS, 0)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_slabs_are_asked_for_by_the_rule_of_whole_calls(monkeypatch, causal):
+    """A budget for one of two halves of the kv heads: the grid of a slab has to pass the same rule as that of the whole pair."""
+    q = torch.empty(1, 10240, 32, 128, dtype=torch.bfloat16, device="meta")
+    k = torch.empty(1, 10240, 4, 128, dtype=torch.bfloat16, device="meta")
+    monkeypatch.setattr(H, "_device_compute_units", lambda device: UNITS)
+    monkeypatch.setattr(H, "attn_bwd_ds_bytes", lambda *a: 4 << 20)
+    monkeypatch.setattr(H, "_ds_budget_bytes", lambda device, enough: 2 << 20)
+    asked = []
+
+    def rule(workgroups, units, refuse=None):
+        asked.append(workgroups)
+        return workgroups != refuse
+
+    monkeypatch.setattr(native, "ds_handover_pays", rule)
+    assert H.ds_plan(q, k, k, causal) == (2, 2 << 20) and asked == [20 * 32, 20 * 16]
+    monkeypatch.setattr(native, "ds_handover_pays", lambda *a: rule(*a, refuse=20 * 16))
+    assert H.ds_plan(q, k, k, causal) is None
