@@ -1,6 +1,6 @@
 """dK/dV of 128 features with 256 key rows per workgroup against the 128-key kernel: both add up the rows in the same steps of 16,
 so for the same head split the results are equal bit for bit. The large call takes the one, each of its batch elements or kv
-heads alone, whose grid is too small for it, the other. Sizes: keys and rows at, before and behind the edges of blocks (32, 64,
+heads alone, whose grid is too small for it, the other (asked of the plan each time). Sizes: keys and rows at, before and behind the edges of blocks (32, 64,
 128, 256), two query walks, every output type and the dS images (through dQ)."""
 
 import re
@@ -8,9 +8,17 @@ import re
 import pytest
 import torch
 
+from pithtrain_amd import _C
 from pithtrain_amd.operators.mla.hip import attn_bwd_dkdv_into, attn_bwd_dq_into, attn_bwd_ds_bytes
 
 gpu_only = pytest.mark.gpu
+
+
+def _key_rows(q, k, causal):
+    """Key rows per workgroup that dK/dV of such a call takes."""
+    args, plan = _C.AttnBwdArgs(B=q.shape[0], Sq=q.shape[1], Skv=k.shape[1], Hq=q.shape[2], Hkv=k.shape[2], Dqk=128, Dv=128, causal=causal), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+    return plan.dkdv_rows
 
 
 def _grads(q, k, v, dout, lse, delta, causal, handover, dtype, old, tail):
@@ -47,6 +55,7 @@ def test_equal_to_the_128_key_kernel(gpu, B, Sq, Skv, H, causal, handover, dtype
     q, k, v, dout = (t(B, s, H, 128).to(torch.bfloat16) for s in (Sq, Skv, Skv, Sq))
     lse, delta = t(B, H, Sq) + 8.0, t(B, H, Sq)
     old = t(B, Skv, H, 128).to(dtype) if accumulate else None
+    assert _key_rows(q, k, causal) == 256 and _key_rows(q[:1], k[:1], causal) == 128
     got = _grads(q, k, v, dout, lse, delta, causal, handover, dtype, old, tail)
     for b in range(0, B, 5):
         one = [x[b : b + 1] for x in (q, k, v, dout, lse, delta)]
@@ -57,29 +66,43 @@ def test_equal_to_the_128_key_kernel(gpu, B, Sq, Skv, H, causal, handover, dtype
             assert not got[0][b, Skv:].any() and not got[1][b, Skv:].any()
 
 
-@gpu_only
-@pytest.mark.parametrize("Sq,Skv,Hq,Hkv,causal", [(4096, 520, 64, 16, False), (4100, 4100, 64, 4, True), (16400, 16400, 24, 8, True)])
-def test_head_parts_and_descending_walk(gpu, Sq, Skv, Hq, Hkv, causal):
-    """Grouped heads: parts of a group in several workgroups. The last one walks the query tiles from the end
-    (its Q and dO outgrow the last-level cache)."""
+def _heads(gpu, Sq, Skv, Hq, Hkv, causal, handover):
+    """A grouped call against its first and last kv head, query head by query head, in fp32 (sums of sums in another order)."""
     g = torch.Generator(device=gpu).manual_seed(5)
     t = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
     q, dout = (t(1, Sq, Hq, 128).to(torch.bfloat16) for _ in range(2))
     k, v = (t(1, Skv, Hkv, 128).to(torch.bfloat16) for _ in range(2))
     lse, delta = t(1, Hq, Sq) + 10.0, t(1, Hq, Sq)
-    dk, dv, _ = _grads(q, k, v, dout, lse, delta, causal, False, torch.float32, None, 0)
+    assert _key_rows(q, k, causal) == 256 and _key_rows(q[:, :, :1], k[:, :, :1], causal) == 128
+    dk, dv, dq = _grads(q, k, v, dout, lse, delta, causal, handover, torch.float32, None, 0)
     group = Hq // Hkv
-    for h in (0, Hkv - 1):  # by query head, in fp32: sums of sums in another order
+    for h in (0, Hkv - 1):
         want = [0.0, 0.0]
         for j in range(h * group, (h + 1) * group):
             part = _grads(q[:, :, j : j + 1].contiguous(), k[:, :, h : h + 1].contiguous(), v[:, :, h : h + 1].contiguous(),
                           dout[:, :, j : j + 1].contiguous(), lse[:, j : j + 1].contiguous(), delta[:, j : j + 1].contiguous(),
-                          causal, False, torch.float32, None, 0)  # fmt: skip
+                          causal, handover, torch.float32, None, 0)  # fmt: skip
             want = [w + x.double() for w, x in zip(want, part)]
+            if handover:
+                assert torch.equal(dq[:, :, j : j + 1], part[2])  # dS has the same bits from either kernel
         for x, w in zip((dk, dv), want):
             # fp32 accumulation of up to group * Sq terms in two orders: 2^-24 a step, a random walk of them
             bound = 2.0**-24 * (group * Sq) ** 0.5 * 4
             assert (x[:, :, h : h + 1].double() - w).norm() <= bound * w.norm()
+
+
+@gpu_only
+@pytest.mark.parametrize("Sq,Skv,Hq,Hkv,causal", [(4096, 520, 64, 16, False), (4100, 4100, 64, 4, True), (16400, 16400, 24, 8, True)])
+def test_head_parts_and_descending_walk(gpu, Sq, Skv, Hq, Hkv, causal):
+    """Grouped heads: parts of a group in several workgroups. The last one walks the query tiles from the end
+    (its Q and dO outgrow the last-level cache)."""
+    _heads(gpu, Sq, Skv, Hq, Hkv, causal, False)
+
+
+@gpu_only
+def test_descending_walk_hands_ds_over(gpu):
+    assert 2 * 16400 * 24 * 128 * 2 > 192 << 20  # bytes of Q and dO from which on the walk descends
+    _heads(gpu, 16400, 16400, 24, 8, True, True)
 
 
 def test_waits_for_its_tile_loads_only(tmp_path):
