@@ -450,22 +450,39 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
 // Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill the
 // device. W = workgroups per compute unit; forward + backward, inputs changing, handing over / recomputing, us:
 //   causal  W 1     4096 x 32/4 heads 561 / 576, 8192 x 16 1030 / 1059, 2 x 2048 x 32/4 323 / 332, 4 x 1024 x 32/4 204 / 215, 8 x 512 x 32/4 148 / 162
-//           W 1.12  9216 x 16 1378 / 1392, 3 x 1536 x 32/4 305 / 312, 9 x 512 x 32/4 189 / 190       W 1.03  2 x 1536 x 44/4 507 / 480 (the one
-//                   shape found that loses: eleven heads to a group)
+//           W 1.12  9216 x 16 1378 / 1392, 3 x 1536 x 32/4 305 / 312, 9 x 512 x 32/4 189 / 190
 //           W 1.25  5120 x 32/4 891 / 914, 2 x 2560 x 32/4 496 / 502       W 1.5   6144 x 32/4 1229 / 1265, 6 x 1024 x 32/4 310 / 317,
 //                   3 x 1999 x 32/4 487 / 500, 2 x 3072 x 32/4 677 / 693   W 1.75  7168 x 32/4 1600 / 1651
 //           W 2     8192 x 32/4 2055 / 2103, 16 x 512 x 32/4 262 / 276     W 2.25  9216 x 32/4 2611 / 2721, 9 x 1024 x 32/4 443 / 461
 //           W 3     12288 x 32/4 4524 / 4756                               W 4     16384 x 32/4 7929 / 8004, 16 x 1024 x 32/4 718 / 736
 //   full    W 1     2 x 2048 x 32/4 534 / 539    W 1.12  4608 x 32/4 1625 / 1670, 9216 x 16 2716 / 2798
 //           W 1.25  5120 x 32/4 1833 / 1887      W 1.5   6144 x 32/4 2367 / 2426
-bool ds_handover_pays(int64_t workgroups, int64_t cus) { return cus > 0 && workgroups >= cus; }
+// And dK/dV, whose stores wait for memory, must not leave units idle that the recomputing dQ of one grid would take: a group
+// of an odd number of heads is not split, and a slab of few heads is a small grid. F = its 128-key workgroups per unit; backward
+// alone, causal and full unless one is named:
+//   F 0.25-0.5  2 x 1536 x 44/4 452 / 430 and 550 / 518, 8 x 512 x 33/3 198 / 184 and 216 / 198, 4096 x 33/3 causal 1111 / 1057, 2048 x 36/4 x 2
+//               505 / 485 and 639 / 612, 12288 x 11/1 3238 / 3084 and 3916 / 3863, 4096 x 76/4 1964 / 1947 and 2432 / 2353, 4096 x 52/4 0-1 % slower;
+//               8192 x 4096 in slabs, full: 66/6 in two 5452 / 3615, 88/8 in two 5636 / 4428
+//   F 0.62      4096 x 35/5 causal 786 / 776, 2 x 2048 x 35/5 full 575 / 547, 4096 x 55/5 1191 / 1200 and 1612 / 1597
+//   F 0.75      4096 x 66/6 1256 / 1282 and 1796 / 1868, 4 x 1536 x 44/4 528 / 536 and 718 / 726, 2 x 3072 x 44/4 causal 957 / 978
+//   F 0.85      2 x 1536 x 45/9 275 / 274 and 384 / 387, 2 x 2048 x 35/7 344 / 345 and 498 / 510
+//   F 1, 1.4    4096 x 40/8 causal 666 / 690, 2 x 2048 x 33/11 282 / 284 and 508 / 549
+bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
+  if (cus <= 0 || (sq + 511) / 512 * hq * b < cus) return false;
+  pith_attn_bwd_args a = {};
+  a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = a.Dv = 128; a.causal = causal;
+  pith_attn_bwd_plan_t plan;
+  if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
+  const int64_t key_tiles = (skv + plan.dkdv_rows - 1) / plan.dkdv_rows * plan.dkdv_rows / 128;
+  return 4 * key_tiles * hkv * b * plan.dkdv_split >= 3 * cus;
+}
 
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
   // Calls large enough for the dS hand-over belong to the Python body, which owns the policy for the hand-over buffer: their
   // kernels outlast its host work many times over.
   bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4;
-  if (small && q.size(3) == 128) {
-    small = !ds_handover_pays((q.size(1) + 511) / 512 * q.size(2) * q.size(0), compute_units(q.device().index()));
+  if (small && q.size(3) == 128 && k.dim() == 4) {
+    small = !ds_handover_pays(q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), causal, compute_units(q.device().index()));
   }
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);

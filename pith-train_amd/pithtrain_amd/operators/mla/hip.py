@@ -208,7 +208,6 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
 # no scratch at all.
 DS_BUFFER_LIMIT_BYTES = int(float(os.environ.get("PITHTRAIN_AMD_DS_BUFFER_LIMIT_GB", "4")) * (1 << 30))
 DS_BUFFER_FREE_FRACTION = 0.5
-_DS_ROWS_PER_WORKGROUP = 512  # query rows a workgroup of the dS-reading dQ kernel owns
 _compute_units = {}
 
 
@@ -234,12 +233,12 @@ def _ds_budget_bytes(device: torch.device, enough: int) -> int:
 
 def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = False):
     """How the backward of one chunk pair uses the dS hand-over: (kv heads per slab, bytes of the buffer),
-    or None when both kernels should recompute (no hand-over path for these head dims, the dS-reading dQ
-    kernel would not fill the device, or not even one kv head fits the budget)."""
+    or None when both kernels should recompute (no hand-over path for these head dims, one of the kernels
+    would not fill the device, or not even one kv head fits the budget)."""
     b, sq, hq, _ = q.shape
-    hkv = k.shape[2]
-    row_tiles = -(-sq // _DS_ROWS_PER_WORKGROUP)
-    if not native.ds_handover_pays(row_tiles * hq * b, _device_compute_units(q.device)):  # nor for any slab
+    skv, hkv = k.shape[1:3]
+    units = _device_compute_units(q.device)
+    if not native.ds_handover_pays(b, sq, skv, hq, hkv, causal, units):  # nor for any slab
         return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:
@@ -253,7 +252,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
             heads -= 1
     if per_kv_head * heads > budget:
         return None
-    if heads < hkv and not native.ds_handover_pays(row_tiles * (hq // hkv) * heads * b, _device_compute_units(q.device)):
+    if heads < hkv and not native.ds_handover_pays(b, sq, skv, hq // hkv * heads, heads, causal, units):
         return None
     return heads, per_kv_head * heads
 

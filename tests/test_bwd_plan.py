@@ -53,11 +53,22 @@ def test_dq_from_ds_goes_out_in_the_order_that_ends_first(tiles, heads):
                                     (6, 1024, 32), (3, 1999, 32), (2, 3072, 32), (1, 7168, 32), (1, 9216, 32), (1, 10240, 32)])  # fmt: skip
 def test_layers_that_gain_hand_ds_over(b, s, hq):
     """Causal layers measured faster with the hand-over than without (table at ds_handover_pays)."""
-    assert native.ds_handover_pays(-(-s // 512) * hq * b, UNITS)
+    assert native.ds_handover_pays(b, s, s, hq, 16 if hq == 16 else 4, True, UNITS)
 
 
 def test_grids_that_do_not_fill_the_device_recompute():
-    assert not native.ds_handover_pays(UNITS - 1, UNITS) and not native.ds_handover_pays(10 * UNITS, 0)
+    assert not native.ds_handover_pays(1, 255 * 512, 255 * 512, 1, 1, True, UNITS) and native.ds_handover_pays(1, 256 * 512, 256 * 512, 1, 1, True, UNITS)
+    assert not native.ds_handover_pays(1, 8192, 8192, 32, 4, True, 0) and not native.ds_handover_pays(1, 8192, 8192, 32, 3, True, UNITS)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("pays,b,sq,skv,hq,hkv", [
+    (False, 2, 1536, 1536, 44, 4), (False, 8, 512, 512, 33, 3), (False, 1, 12288, 12288, 11, 1), (False, 2, 2048, 2048, 36, 4), (False, 1, 8192, 4096, 44, 4),
+    (True, 4, 1536, 1536, 44, 4), (True, 2, 1536, 1536, 48, 4), (True, 2, 2048, 2048, 33, 11), (True, 1, 4096, 4096, 40, 8), (True, 1, 12288, 12288, 12, 1),
+])  # fmt: skip
+def test_grids_of_unsplit_groups(pays, b, sq, skv, hq, hkv, causal):
+    """Groups of an odd number of heads are not split: too few dK/dV workgroups to hand dS over, as measured."""
+    assert native.ds_handover_pays(b, sq, skv, hq, hkv, causal, UNITS) == pays
 
 
 @pytest.mark.parametrize("causal", [False, True])
@@ -68,13 +79,26 @@ def test_slabs_are_asked_for_by_the_rule_of_whole_calls(monkeypatch, causal):
     monkeypatch.setattr(H, "_device_compute_units", lambda device: UNITS)
     monkeypatch.setattr(H, "attn_bwd_ds_bytes", lambda *a: 4 << 20)
     monkeypatch.setattr(H, "_ds_budget_bytes", lambda device, enough: 2 << 20)
-    asked = []
+    real, asked = native.ds_handover_pays, []
 
-    def rule(workgroups, units, refuse=None):
-        asked.append(workgroups)
-        return workgroups != refuse
+    def rule(*call, refuse=None):
+        asked.append(call)
+        return real(*call) and call[3] != refuse
 
     monkeypatch.setattr(native, "ds_handover_pays", rule)
-    assert H.ds_plan(q, k, k, causal) == (2, 2 << 20) and asked == [20 * 32, 20 * 16]
-    monkeypatch.setattr(native, "ds_handover_pays", lambda *a: rule(*a, refuse=20 * 16))
+    assert H.ds_plan(q, k, k, causal) == (2, 2 << 20)
+    assert asked == [(1, 10240, 10240, heads, heads // 8, causal, UNITS) for heads in (32, 16)]
+    monkeypatch.setattr(native, "ds_handover_pays", lambda *a: rule(*a, refuse=16))
     assert H.ds_plan(q, k, k, causal) is None
+
+
+def test_slabs_that_leave_units_idle_recompute(monkeypatch):
+    """8192 x 4096 rows, 88/8 heads: 256 dK/dV workgroups as a whole, 128 in either of two slabs (measured 27 % slower)."""
+    q = torch.empty(1, 8192, 88, 128, dtype=torch.bfloat16, device="meta")
+    k = torch.empty(1, 4096, 8, 128, dtype=torch.bfloat16, device="meta")
+    monkeypatch.setattr(H, "_device_compute_units", lambda device: UNITS)
+    monkeypatch.setattr(H, "attn_bwd_ds_bytes", lambda *a: 8 << 20)
+    monkeypatch.setattr(H, "_ds_budget_bytes", lambda device, enough: 8 << 20)
+    assert H.ds_plan(q, k, k) == (8, 8 << 20)
+    monkeypatch.setattr(H, "_ds_budget_bytes", lambda device, enough: 4 << 20)
+    assert H.ds_plan(q, k, k) is None
