@@ -105,6 +105,7 @@ struct Plan {
   int rows, split;
 };
 Plan plan_for(const pith_attn_bwd_args* a, int rows) { return {rows, pick_split(a, (a->Skv + rows - 1) / rows)}; }
+int64_t workgroups(const pith_attn_bwd_args* a, const Plan& p) { return (a->Skv + p.rows - 1) / p.rows * a->Hkv * a->B * p.split; }
 
 // Whether a call of 128 features and not too few rows, launched alone, goes to the workgroups of kDkdvWideN keys (attn_bwd_dkdv_wide.h), which are
 // 4-7 % faster per product. Half as many workgroups cost
@@ -119,8 +120,7 @@ Plan plan_for(const pith_attn_bwd_args* a, int rows) { return {rows, pick_split(
 // 579 -> 545 (all handing dS over; recomputing 0-7 % faster). A call that fits the built-in scratch of pith_attn_bwd_dkdv_static
 // with 128 keys has to fit it with 256, too: both entry points add up in the same order.
 bool wide(const pith_attn_bwd_args* a, const Plan& n, const Plan& w) {
-  const int64_t cus = compute_units_or_default(), heads = a->Hkv * a->B;
-  const int64_t narrow_wgs = (a->Skv + n.rows - 1) / n.rows * heads * n.split, wide_wgs = (a->Skv + w.rows - 1) / w.rows * heads * w.split;
+  const int64_t cus = compute_units_or_default(), narrow_wgs = workgroups(a, n), wide_wgs = workgroups(a, w);
   const int64_t narrow_heads = a->Hq / a->Hkv / n.split, wide_heads = a->Hq / a->Hkv / w.split;
   if (w.split > 1 && (a->Sq < 4096 || (a->causal ? a->Sq / 2 : a->Sq) * wide_heads < 4096)) return false;
   const int64_t fits = PITH_DKDV_STATIC_SCRATCH_BYTES;
@@ -171,6 +171,38 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_d
   }
 }
 
+// Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
+// split-key ones (the two kernels must agree on the workgroup size), which is what grids of up to one workgroup per compute
+// unit want anyway. Beyond, one grid pays where either kernel alone would leave its last round half empty, against what the
+// two-workgroup dQ kernel is faster by; W = dQ workgroups per compute unit, apart -> together, inputs from memory, us:
+//   d128 causal   W 1.5: 1 x 2304 x 16 108 -> 91, 1 x 6144 x 8/2 289 -> 265, 6 x 512 x 16/4 68 -> 61; 1.75: 1 x 1792 x 32/4
+//                 122 -> 121; 2: 1 x 2048 x 32/4 154 -> 150, 1 x 8192 x 8/2 446 -> 449; 2.25-2.5: 1 x 2304 x 32/4 191 -> 181,
+//                 1 x 5120 x 16 377 -> 351, 5 x 1024 x 16/4 127 -> 127
+//        full     W 1.5: 1 x 1536 x 32/4 157 -> 145; 1.7: 1 x 3456 x 16 307 -> 329; 2: 1 x 4096 x 16 412 -> 422;
+//                 2.2: 1 x 4480 x 16 628 -> 520, 1 x 2304 x 32/4 383 -> 289
+//   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186, 3 x 1024 x 16 92 -> 94; 1.7: 1 x 3456 x 16
+//                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
+// Several chunks, whose dK/dV workgroups are more unequal, gain 1-5 % up to two per unit (2048 x 32/4 of 128, 4 ranks,
+// zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081). 128 features: up to four, where two launches lost
+// even to one pair of them per ring step (in brackets): 4096 x 32/4, 4 ranks, rank 0 1889 -> 1728 (1724); 9216 x 8/2, 8
+// ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
+// rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
+// 16: 2385 -> 2413).
+// At 64 features both kernels fit two workgroups to a unit, and one grid is never slower: forward + backward, before (apart from
+// more than four workgroups per unit, three of dQ) -> now, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 ->
+// 2359, 16 x 1024 x 32/8 415 -> 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630. Together they have to be a grid that the
+// runtime launches (2^32 threads are refused), which either of them may be where both are not (65535 x 1 row x 130 heads).
+bool one_grid(const pith_attn_bwd_args* a, int64_t dkdv_wgs, bool chunks) {
+  if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
+  const int64_t cus = compute_units_or_default();
+  const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
+  if (a->Dqk == 64) return (q_wgs + dkdv_wgs) * 256 < (1ll << 32);
+  if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
+  if (q_wgs <= cus) return true;
+  if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;
+  return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));
+}
+
 }  // namespace
 }  // namespace pith
 
@@ -192,6 +224,10 @@ extern "C" int pith_attn_bwd_plan(const pith_attn_bwd_args* a, pith_attn_bwd_pla
   plan->dkdv_rows = chosen.rows;
   plan->dkdv_split = chosen.split;
   plan->dq_ds_pairs = a->causal && ds_bytes_for(a) > 0 && dq_ds_pairs((a->Sq + 511) / 512 * a->Hq * a->B);
+  pith_attn_bwd_args bf16 = *a;
+  bf16.ds = nullptr;
+  bf16.dq_dtype = bf16.dkv_dtype = PITH_BF16;
+  plan->one_grid = one_grid(&bf16, workgroups(a, plan_for(a, kBN)), false);
   return PITH_OK;
 }
 
@@ -287,37 +323,6 @@ int bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream, const char* who,
   return run_dkdv(a, plan, a->workspace, (hipStream_t)stream, who, with_dq);
 }
 
-// Whether dK/dV and dQ go out as one grid (no dS handed over). At 128 and 192 features the dQ workgroups are then the
-// split-key ones (the two kernels must agree on the workgroup size), which is what grids of up to one workgroup per compute
-// unit want anyway. Beyond, one grid pays where either kernel alone would leave its last round half empty, against what the
-// two-workgroup dQ kernel is faster by; W = dQ workgroups per compute unit, apart -> together, inputs from memory, us:
-//   d128 causal   W 1.5: 1 x 2304 x 16 108 -> 91, 1 x 6144 x 8/2 289 -> 265, 6 x 512 x 16/4 68 -> 61; 1.75: 1 x 1792 x 32/4
-//                 122 -> 121; 2: 1 x 2048 x 32/4 154 -> 150, 1 x 8192 x 8/2 446 -> 449; 2.25-2.5: 1 x 2304 x 32/4 191 -> 181,
-//                 1 x 5120 x 16 377 -> 351, 5 x 1024 x 16/4 127 -> 127
-//        full     W 1.5: 1 x 1536 x 32/4 157 -> 145; 1.7: 1 x 3456 x 16 307 -> 329; 2: 1 x 4096 x 16 412 -> 422;
-//                 2.2: 1 x 4480 x 16 628 -> 520, 1 x 2304 x 32/4 383 -> 289
-//   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186, 3 x 1024 x 16 92 -> 94; 1.7: 1 x 3456 x 16
-//                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
-// Several chunks, whose dK/dV workgroups are more unequal, gain 1-5 % up to two per unit (2048 x 32/4 of 128, 4 ranks,
-// zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081). 128 features: up to four, where two launches lost
-// even to one pair of them per ring step (in brackets): 4096 x 32/4, 4 ranks, rank 0 1889 -> 1728 (1724); 9216 x 8/2, 8
-// ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
-// rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
-// 16: 2385 -> 2413).
-// At 64 features both kernels fit two workgroups to a unit, and one grid is never slower: forward + backward, before (apart from
-// more than four workgroups per unit, three of dQ) -> now, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 ->
-// 2359, 16 x 1024 x 32/8 415 -> 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630.
-bool one_grid(const pith_attn_bwd_args* a, bool chunks) {
-  if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
-  const int64_t cus = compute_units_or_default();
-  const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
-  if (a->Dqk == 64) return true;
-  if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
-  if (q_wgs <= cus) return true;
-  if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;
-  return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));
-}
-
 }  // namespace
 
 extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t stream) {
@@ -327,7 +332,7 @@ extern "C" int pith_attn_bwd_dkdv(const pith_attn_bwd_args* a, pith_stream_t str
 extern "C" int pith_attn_bwd(const pith_attn_bwd_args* a, pith_stream_t stream) {
   const char* who = "pith_attn_bwd";
   if (const int rc = validate_bwd(a, who, true, true)) return rc;
-  if (one_grid(a, false)) return bwd_dkdv(a, stream, who, true);
+  if (one_grid(a, workgroups(a, plan_for(a, kBN)), false)) return bwd_dkdv(a, stream, who, true);
   // what the second call would reject is rejected before the first has written (or added to) anything
   BwdParams dq;
   if (const int rc = prepare_dq(a, &dq, who)) return rc;
@@ -454,7 +459,7 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   // any case (128 and 192 features): 2048 x 32/4 of 128, rank 0: 498 us, dQ first 518; 4096 x 16 of 192, rank 3: 1081 and 1084.
   const bool few = all.Dqk == 64 || ((all.Sq + 127) / 128) * all.Hq * all.B <= (int64_t)compute_units_or_default();
   const bool dq_first = few && 3 * all.Skv > 4 * all.Sq * (all.Hq / all.Hkv / split);
-  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, true), dq_first, blocks, st);
+  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, blocks, true), dq_first, blocks, st);
   if (all.k_pe || split > 1) {  // (never both: keys in two parts have no head groups to split)
     Reduction<2 * kMaxChunks> r;
     for (int64_t i = 0; i < n; ++i) {

@@ -100,7 +100,7 @@ class AttnBwdArgs(Structure):
 
 
 class AttnBwdPlan(Structure):
-    _fields_ = [("dkdv_rows", c_int32), ("dkdv_split", c_int32), ("dq_ds_pairs", c_int32)]
+    _fields_ = [("dkdv_rows", c_int32), ("dkdv_split", c_int32), ("dq_ds_pairs", c_int32), ("one_grid", c_int32)]
 
 
 class NormRopeArgs(Structure):

@@ -27,6 +27,14 @@ def test_plan_query():
     assert _C.lib().pith_attn_bwd_plan(None, None) == -1
 
 
+@pytest.mark.parametrize("b,s,hq,hkv", [(65535, 1, 130, 130), (65535, 129, 120, 8), (60000, 1, 270, 30), (65535, 1, 256, 1)])
+def test_one_grid_is_one_that_can_be_launched(b, s, hq, hkv):
+    """64 features: two grids of fewer than 2^32 threads each may make a grid of more, which the runtime refuses."""
+    dq, dkdv = -(-s // 128) * b * hq, -(-s // 128) * b * hkv
+    assert _plan(b, s, s, hq, hkv, 0, 64).one_grid == ((dq + dkdv) * 256 < 2**32)
+    assert _plan(64, s, s, hq, hkv, 0, 64).one_grid
+
+
 def _makespan(jobs):
     """Jobs handed out in order, each to the compute unit that is free first."""
     free = [0.0] * UNITS
@@ -102,3 +110,18 @@ def test_slabs_that_leave_units_idle_recompute(monkeypatch):
     assert H.ds_plan(q, k, k) == (8, 8 << 20)
     monkeypatch.setattr(H, "_ds_budget_bytes", lambda device, enough: 4 << 20)
     assert H.ds_plan(q, k, k) is None
+
+
+@pytest.mark.gpu
+def test_more_workgroups_than_one_launch_takes(gpu):
+    """One row attends to itself: O = V, dV = dO, dQ = dK = 0. 8.5 M workgroups of either kernel."""
+    b, h, d = 65535, 130, 64
+    assert not _plan(b, 1, 1, h, h, 0, d).one_grid
+    g = torch.Generator(device=gpu).manual_seed(1)
+    q, k, v, dout = (torch.randn(b, 1, h, d, generator=g, device=gpu, dtype=torch.bfloat16) for _ in range(4))
+    o, lse = torch.ops.pithtrain_amd.attn_fwd(q, k, v, d**-0.5, False)
+    assert torch.equal(o, v)
+    dq, dk, dv = torch.ops.pithtrain_amd.attn_bwd(q, k, v, o, lse, dout, d**-0.5, False)
+    assert torch.equal(dv, dout)
+    # dS is the difference of two fp32 sums of 64 products |x y| < 36 in two orders: below 64 * 2^-24 * 64 * 36 = 0.0088; times |k| < 6, scale 1/8
+    assert dq.abs().max() < 0.0067 and dk.abs().max() < 0.0067

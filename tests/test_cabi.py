@@ -65,7 +65,7 @@ def test_struct_layouts_match_the_header(tmp_path):
 # Struct sizes of a version of the interface: a change here needs a new version (programs built against the old header pass
 # structs of the old size).
 STRUCT_SIZES = {
-    200: {"pith_combine_args": 168, "pith_attn_fwd_args": 248, "pith_attn_delta_args": 88, "pith_attn_bwd_args": 352, "pith_attn_bwd_plan_t": 12,
+    200: {"pith_combine_args": 168, "pith_attn_fwd_args": 248, "pith_attn_delta_args": 88, "pith_attn_bwd_args": 352, "pith_attn_bwd_plan_t": 16,
           "pith_norm_rope_args": 152, "pith_mla_assemble_args": 192, "pith_key_chunk": 72, "pith_device_info_t": 88},
 }  # fmt: skip
 
