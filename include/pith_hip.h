@@ -313,6 +313,8 @@ typedef struct {
 } pith_attn_bwd_plan_t;
 
 int pith_attn_bwd_plan(const pith_attn_bwd_args* args, pith_attn_bwd_plan_t* plan);
+/* The same for pith_attn_bwd_chunks; the rows and q_row0 of the chunks are read, too. */
+int pith_attn_bwd_chunks_plan(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_attn_bwd_plan_t* plan);
 
 /* pith_attn_bwd_dkdv for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). It has no counterpart in the

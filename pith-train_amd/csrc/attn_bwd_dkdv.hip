@@ -188,10 +188,16 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_d
 // ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
 // rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
 // 16: 2385 -> 2413).
-// At 64 features both kernels fit two workgroups to a unit, and one grid is never slower: forward + backward, before (apart from
-// more than four workgroups per unit, three of dQ) -> now, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 ->
-// 2359, 16 x 1024 x 32/8 415 -> 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630. Together they have to be a grid that the
-// runtime launches (2^32 threads are refused), which either of them may be where both are not (65535 x 1 row x 130 heads).
+// At 64 features both kernels fit two workgroups to a unit, and one grid is faster for chunk pairs and most shares: forward +
+// backward, apart -> together, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 -> 2359, 16 x 1024 x 32/8 415 ->
+// 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630; shares, zigzag, 4096 x 64/8, 4 ranks, rank 0 2740 -> 2543, 8192 x 32/8 rank 1
+// 5084 -> 4972, 5120 x 32/8 rank 0 2284 -> 2135, 12288 x 16/4 rank 1 5771 -> 5615, 32768 x 8/2, 2 ranks, rank 0 10660 -> 10224, 16384 x
+// 32/8, 2 ranks 10091 -> 9983. Not where few long dQ walks start beside the last dK/dV workgroups and either kernel is whole
+// rounds (three or more of dK/dV, up to four of dQ, from 12288 rows on), so that nothing is left to fill: 12288 x 16/4, 4 ranks, rank 0
+// 5805 -> 5994, 16384 x 16/4 10106 -> 10295, 24576 x 8/2 11896 -> 12077, contiguous 16384 x 16/4 rank 2 12525 -> 12699, 12288 x 16/4 rank 3
+// 9957 -> 10027. Whole rounds of more or shorter ones: 10240, 12288, 16384 x 32/8 7642 -> 7543, 10879 -> 10763, 19213 -> 18984, 3 x 4096 x
+// 16/4 1983 -> 1964; dQ first: 16384 x 16 10221 -> 10018. Together they have to be a grid that the runtime launches (2^32 threads
+// are refused), which either of them may be where both are not (65535 x 1 row x 130 heads).
 bool one_grid(const pith_attn_bwd_args* a, int64_t dkdv_wgs, bool chunks) {
   if (ds_usable(a) || (a->dkv_dtype == PITH_F32 && a->dq_dtype != PITH_F32)) return false;
   const int64_t cus = compute_units_or_default();
@@ -389,7 +395,42 @@ int pick_chunks_split(pith_attn_bwd_args a, int64_t tiles) {
   return pick_split(&a, tiles);
 }
 
+// The launches of a call of several chunks: one grid or two, and which kind goes first in one.
+struct ChunkGrids {
+  bool one, dq_first;
+};
+ChunkGrids chunk_grids(const pith_attn_bwd_args* all, int64_t tiles, int split, int64_t dkdv_blocks) {
+  const int64_t cus = compute_units_or_default(), q_wgs = ((all->Sq + 127) / 128) * all->Hq * all->B;
+  // In one grid the longer workgroups go first: dQ's cost 3 products per key of all chunks, dK/dV's 4 per query row and head
+  // of the part. With more than a workgroup of either per compute unit the dK/dV ones, unequal over the chunks, come first in
+  // any case (128 and 192 features): 2048 x 32/4 of 128, rank 0: 498 us, dQ first 518; 4096 x 16 of 192, rank 3: 1081 and 1084.
+  const bool few = all->Dqk == 64 || q_wgs <= cus;
+  const bool dq_first = few && 3 * all->Skv > 4 * all->Sq * (all->Hq / all->Hkv / split);
+  // (64 features: see one_grid)
+  const int64_t round = 2 * cus, dkdv_wgs = tiles * all->Hkv * all->B * split;
+  const bool whole = q_wgs > 2 * round && q_wgs <= 4 * round && q_wgs % round == 0 && dkdv_wgs >= 3 * round && dkdv_wgs % round == 0;
+  return {one_grid(all, dkdv_blocks, true) && !(all->Dqk == 64 && !dq_first && all->Sq >= 12288 && whole), dq_first};
+}
+
 }  // namespace
+
+extern "C" int pith_attn_bwd_chunks_plan(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_attn_bwd_plan_t* plan) {
+  const char* who = "pith_attn_bwd_chunks_plan";
+  pith_attn_bwd_args all;
+  int64_t tiles;
+  if (!plan || !merged_call(args, chunks, n, &all, &tiles)) return fail(PITH_ERR_BAD_SHAPE, "%s: plan is NULL or bad shape", who);
+  if (n == 1) {
+    all.Skv = chunks[0].rows;
+    all.causal = 1;
+    return pith_attn_bwd_plan(&all, plan);
+  }
+  all.dq_dtype = all.dkv_dtype = PITH_BF16;
+  plan->dkdv_rows = kBN;
+  plan->dkdv_split = pick_chunks_split(all, tiles);
+  plan->dq_ds_pairs = 0;
+  plan->one_grid = chunk_grids(&all, tiles, plan->dkdv_split, tiles * all.Hkv * all.B * plan->dkdv_split).one;
+  return PITH_OK;
+}
 
 extern "C" int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n) {
   pith_attn_bwd_args a;
@@ -454,12 +495,8 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));
   hipStream_t st = (hipStream_t)stream;
   begin_launch();
-  // In one grid the longer workgroups go first: dQ's cost 3 products per key of all chunks, dK/dV's 4 per query row and head
-  // of the part. With more than a workgroup of either per compute unit the dK/dV ones, unequal over the chunks, come first in
-  // any case (128 and 192 features): 2048 x 32/4 of 128, rank 0: 498 us, dQ first 518; 4096 x 16 of 192, rank 3: 1081 and 1084.
-  const bool few = all.Dqk == 64 || ((all.Sq + 127) / 128) * all.Hq * all.B <= (int64_t)compute_units_or_default();
-  const bool dq_first = few && 3 * all.Skv > 4 * all.Sq * (all.Hq / all.Hkv / split);
-  launch_bwd_chunks(p, (int)all.Dqk, one_grid(&all, blocks, true), dq_first, blocks, st);
+  const ChunkGrids grids = chunk_grids(&all, tiles, split, blocks);
+  launch_bwd_chunks(p, (int)all.Dqk, grids.one, grids.dq_first, blocks, st);
   if (all.k_pe || split > 1) {  // (never both: keys in two parts have no head groups to split)
     Reduction<2 * kMaxChunks> r;
     for (int64_t i = 0; i < n; ++i) {

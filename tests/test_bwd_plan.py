@@ -8,6 +8,7 @@ import torch
 from pithtrain_amd import _C
 from pithtrain_amd._ext import native
 from pithtrain_amd.operators.mla import hip as H
+from pithtrain_amd.operators.ring_attention.local import ring_schedule
 
 UNITS = 256
 
@@ -15,6 +16,14 @@ UNITS = 256
 def _plan(b, sq, skv, hq, hkv, causal, d=128):
     args, plan = _C.AttnBwdArgs(B=b, Sq=sq, Skv=skv, Hq=hq, Hkv=hkv, Dqk=d, Dv=min(d, 128), causal=causal), _C.AttnBwdPlan()
     _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+    return plan
+
+
+def _share_plan(b, s, hq, hkv, cp, rank, layout):
+    steps = sorted(ring_schedule(rank, cp, s, layout), key=lambda st: (st.kv_rank == rank, st.q_rows[0]))
+    chunks = (_C.KeyChunk * len(steps))(*(_C.KeyChunk(rows=st.kv_rows[1] - st.kv_rows[0], q_row0=st.q_rows[0]) for st in steps))
+    args, plan = _C.AttnBwdArgs(B=b, Sq=s, Skv=s, Hq=hq, Hkv=hkv, Dqk=64, Dv=64), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_chunks_plan(_C.byref(args), chunks, len(steps), _C.byref(plan)))
     return plan
 
 
@@ -33,6 +42,18 @@ def test_one_grid_is_one_that_can_be_launched(b, s, hq, hkv):
     dq, dkdv = -(-s // 128) * b * hq, -(-s // 128) * b * hkv
     assert _plan(b, s, s, hq, hkv, 0, 64).one_grid == ((dq + dkdv) * 256 < 2**32)
     assert _plan(64, s, s, hq, hkv, 0, 64).one_grid
+
+
+@pytest.mark.parametrize("one,b,s,hq,hkv,cp,rank,layout", [
+    (0, 1, 12288, 16, 4, 4, 0, "zigzag"), (0, 1, 16384, 16, 4, 4, 0, "zigzag"), (0, 1, 24576, 8, 2, 4, 0, "zigzag"), (0, 1, 16384, 16, 4, 4, 2, "contiguous"),
+    (0, 1, 12288, 16, 4, 4, 3, "contiguous"),
+    (1, 1, 12288, 16, 4, 4, 1, "zigzag"), (1, 1, 4096, 64, 8, 4, 0, "zigzag"), (1, 1, 8192, 32, 8, 4, 1, "zigzag"), (1, 1, 5120, 32, 8, 4, 0, "zigzag"),
+    (1, 1, 32768, 8, 2, 2, 0, "zigzag"), (1, 1, 16384, 16, 16, 4, 0, "zigzag"), (1, 3, 3001, 16, 4, 2, 1, "contiguous"), (1, 2, 8192, 16, 16, 4, 2, "zigzag"),
+    (1, 1, 16384, 32, 8, 4, 0, "zigzag"), (1, 1, 10240, 32, 8, 4, 0, "zigzag"), (1, 1, 12288, 32, 8, 4, 0, "zigzag"), (1, 3, 4096, 16, 4, 4, 0, "zigzag"),
+])  # fmt: skip
+def test_shares_of_64_features(one, b, s, hq, hkv, cp, rank, layout):
+    """Both gradients in one grid unless either kernel alone is whole rounds of long walks, as measured (table at one_grid)."""
+    assert _share_plan(b, s, hq, hkv, cp, rank, layout).one_grid == one
 
 
 def _makespan(jobs):
@@ -125,3 +146,22 @@ def test_more_workgroups_than_one_launch_takes(gpu):
     assert torch.equal(dv, dout)
     # dS is the difference of two fp32 sums of 64 products |x y| < 36 in two orders: below 64 * 2^-24 * 64 * 36 = 0.0088; times |k| < 6, scale 1/8
     assert dq.abs().max() < 0.0067 and dk.abs().max() < 0.0067
+
+
+@pytest.mark.gpu
+def test_share_of_64_features_in_two_launches(gpu):
+    """Whole rounds of workgroups go out as two launches, those of one kv head as one: equal bit for bit."""
+    s, hq, hkv, cp = 16384, 12, 4, 4
+    assert not _share_plan(1, s, hq, hkv, cp, 0, "zigzag").one_grid and _share_plan(1, s, 3, 1, cp, 0, "zigzag").one_grid
+    g = torch.Generator(device=gpu).manual_seed(1)
+    mk = lambda h: torch.randn(1, s, h, 64, generator=g, device=gpu, dtype=torch.bfloat16)  # noqa: E731
+    q, ks, vs, dout = mk(hq), [mk(hkv) for _ in range(cp)], [mk(hkv) for _ in range(cp)], mk(hq)
+    out, lse = mk(hq), torch.randn(1, hq, s, generator=g, device=gpu) + 12.0
+    whole = native.ring_backward(dout, q, out, lse, ks, vs, None, 0.125, 0, cp, True)
+    for h in (0, 3):
+        qh, kh = slice(3 * h, 3 * h + 3), slice(h, h + 1)
+        dout_h, q_h, out_h, lse_h = dout[:, :, qh].contiguous(), q[:, :, qh].contiguous(), out[:, :, qh].contiguous(), lse[:, qh].contiguous()
+        one = native.ring_backward(dout_h, q_h, out_h, lse_h, [k[:, :, kh].contiguous() for k in ks], [v[:, :, kh].contiguous() for v in vs], None, 0.125, 0, cp, True)
+        assert torch.equal(whole[0][:, :, qh], one[0])
+        for j in range(cp):
+            assert torch.equal(whole[1][j][:, :, kh], one[1][j]) and torch.equal(whole[2][j][:, :, kh], one[2][j])
