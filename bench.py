@@ -66,7 +66,7 @@ def profile_figure(name, key):
     return None
 
 
-HBM_COUNTERS = "attn_bwd_dkdv_d128_qwen3_step_hbm_counters.txt"
+HBM_COUNTERS = "attn_qwen3_step_hbm_counters.txt"
 STREAM_COUNTERS = "combine_norm_rope_mla_assemble_hbm_counters.txt"
 
 
@@ -203,6 +203,15 @@ def roofline_entry(kernel, flops_per_launch, ms_per_launch, launches, traffic=No
     return out
 
 
+def dkdv_kernel(b, sq, skv, hq, hkv):
+    """Name of the kernel a non-causal dK/dV launch of 128 features runs."""
+    from pithtrain_amd import _C
+
+    args, plan = _C.AttnBwdArgs(B=b, Sq=sq, Skv=skv, Hq=hq, Hkv=hkv, Dqk=128, Dv=128, causal=0), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+    return "attn_bwd_dkdv_wide_kernel" if plan.dkdv_rows == 256 else "attn_bwd_dkdv_d128_kernel"
+
+
 def noncausal_steps(cfg):
     from pithtrain_amd.operators.ring_attention.local import ring_schedule
 
@@ -213,14 +222,14 @@ def dominant_dkdv(torch, cfg, dev, out, lse, reps, counter_pass=False):
     """The non-causal dK/dV launches of one step of `cfg`, launched exactly as the ring backward launches them
     (with the dS hand-over buffer, whole or one slab of kv heads at a time, whenever its policy takes one) and
     timed with events on the launch stream. Returns (ms per launch, FLOP per launch, launches per step, bytes of
-    hand-over scratch)."""
+    hand-over scratch, kernel names)."""
     from pithtrain_amd.operators.mla import hip
 
     q, ks, vs, dout = dev
     scale = cfg.dqk**-0.5
     delta = torch.empty_like(lse)
     hip.attn_bwd_delta_into(out, dout, delta)
-    launches, buf, flops = [], None, 0
+    launches, buf, flops, kernels = [], None, 0, set()
     for s in noncausal_steps(cfg):
         kr, qr = slice(*s.kv_rows), slice(*s.q_rows)
         k_j, v_j = ks[s.kv_rank][:, kr], vs[s.kv_rank][:, kr]
@@ -234,6 +243,7 @@ def dominant_dkdv(torch, cfg, dev, out, lse, reps, counter_pass=False):
             kv_h, q_h = slice(h0, h0 + heads), slice(h0 * g, (h0 + heads) * g)
             launches.append((q[:, qr, q_h], k_j[:, :, kv_h], v_j[:, :, kv_h], dout[:, qr, q_h], lse[:, q_h, qr],
                              delta[:, q_h, qr], dk[:, :, kv_h], dv[:, :, kv_h]))  # fmt: skip
+        kernels.add(dkdv_kernel(1, qr.stop - qr.start, kr.stop - kr.start, heads * g, heads))
         flops = 2 * (2 * cfg.dqk + 2 * cfg.dv) * (qr.stop - qr.start) * (kr.stop - kr.start) * heads * g
 
     def run():
@@ -246,7 +256,7 @@ def dominant_dkdv(torch, cfg, dev, out, lse, reps, counter_pass=False):
         torch.cuda.synchronize()
         return None
     ms = time_events(torch, run, reps) / len(launches)
-    return ms, flops, len(launches), (0 if buf is None else buf.numel())
+    return ms, flops, len(launches), (0 if buf is None else buf.numel()), " / ".join(sorted(kernels))
 
 
 def share_forward(torch, cfg, dev, reps):
@@ -283,9 +293,9 @@ def bench_other_config(torch, device, cfg, steps, warmup, cpu_heads=None, counte
         return None
     out = ring_summary(cfg, ms_step, ms_fwd, ms_bwd)
     if scratch:
-        ms, flops, n, _ = dominant_dkdv(torch, cfg, dev, o, lse, steps)
+        ms, flops, n, _, name = dominant_dkdv(torch, cfg, dev, o, lse, steps)
         slabs = n // len(noncausal_steps(cfg))
-        kernel = ("attn_bwd_dkdv_d128_kernel<non-causal> (S, dP, dV, dK of one ring step" + (f", one of {slabs} kv-head slabs per launch" if slabs > 1 else "")
+        kernel = (f"{name}<non-causal> (S, dP, dV, dK of one ring step" + (f", one of {slabs} kv-head slabs per launch" if slabs > 1 else "")
                   + "; also stores its dS tiles for the dQ kernel)")  # fmt: skip
         traffic = f"{cfg.name}.dkdv_traffic_bytes_per_launch"
     else:
@@ -598,7 +608,7 @@ def main():
         bench_mla_assemble(torch, device, reps=3)
         print("counter pass done")
         return
-    ms_dkdv, dkdv_flops, dkdv_n, scratch = dominant_dkdv(torch, QWEN3, dev_inputs, out, lse, args.steps)
+    ms_dkdv, dkdv_flops, dkdv_n, scratch, dkdv_name = dominant_dkdv(torch, QWEN3, dev_inputs, out, lse, args.steps)
     ms_fwdk, fwdk_flops, fwdk_n = share_forward(torch, QWEN3, dev_inputs, args.steps)
     handover_on = scratch > 0
     scratch = handover_scratch_bytes(QWEN3, dev_inputs)
@@ -668,7 +678,7 @@ def main():
             "cpu_baseline": fwd_cpu,
         },  # fmt: skip
         "roofline": roofline_entry(
-            "attn_bwd_dkdv_d128_kernel<non-causal> (S, dP, dV, dK of one ring step"
+            f"{dkdv_name}<non-causal> (S, dP, dV, dK of one ring step"
             + ("; also stores its dS tiles for the dQ kernel)" if handover_on else ")"), dkdv_flops, ms_dkdv, dkdv_n,
             profile_figure(HBM_COUNTERS, "qwen3-32k.dkdv_traffic_bytes_per_launch" if handover_on
                            else "qwen3-32k.dkdv_traffic_bytes_per_launch_without_ds_stores"), "profiles/" + HBM_COUNTERS),  # fmt: skip

@@ -8,7 +8,7 @@ import subprocess
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 BIN_DIR = os.path.join(HERE, "bin")
-PROBES = ("mfma_rate_probe", "atomic_rate_probe", "wide_wave_probe")
+PROBES = ("mfma_rate_probe", "atomic_rate_probe", "wide_wave_probe", "lds_fragment_rate_probe")
 CSRC = os.path.join(os.path.dirname(os.path.dirname(HERE)), "pith-train_amd", "csrc")  # attn_tiles.h (wide_wave_probe)
 
 

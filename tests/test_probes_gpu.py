@@ -1,8 +1,8 @@
 """Runs the device probes of tests/probes/ (built ahead of time by __graft_entry__.build()) and checks what the
 design argues from: the full-chip rate of bf16 matrix instructions depends on the operand data and stays below the
 nominal peak with random operands, and fp32 global atomic adds are far too slow to accumulate dQ in a single backward
-kernel; and a forward loop with one 64-row wave per SIMD (half the LDS fragment reads) is issue-bound below the
-shipped loop. The probes print their tables; profiles/ holds a copy with hardware counters beside it."""
+kernel; a forward loop with one 64-row wave per SIMD (half the LDS fragment reads) is issue-bound below the
+shipped loop; and products fed from LDS run faster the more of them share a fragment read. The probes print their tables; profiles/ holds a copy with hardware counters beside it."""
 
 import os
 import re
@@ -68,3 +68,14 @@ def test_one_wide_wave_per_simd_does_not_beat_the_shipped_forward_loop(gpu):
     # barriers; this loop has neither and still stays below that: a single wave cannot issue the softmax of 64 rows
     # next to 64 matrix instructions per tile fast enough
     assert all(700 < r < 1400 for r in rates), rates
+
+
+def test_products_that_share_a_fragment_read_run_faster(gpu):
+    rates = {1: [], 2: [], 4: []}
+    for line in _run("lds_fragment_rate_probe"):
+        m = re.match(r"products per fragment read (\d) rep \d+:\s+([\d.]+) ms\s+(\d+) TFLOP/s", line)
+        if m:
+            rates[int(m.group(1))].append(float(m.group(3)))
+    assert all(len(r) == 5 and 700 < min(r) and max(r) < 2500 for r in rates.values()), rates
+    one, two, four = (sorted(rates[n])[2] for n in (1, 2, 4))  # 1.65, 1.77, 1.80 PFLOP/s; 1.53, 1.65, 1.71 on another machine
+    assert one < two < 1.03 * four, rates
