@@ -118,7 +118,9 @@ int64_t workgroups(const pith_attn_bwd_args* a, const Plan& p) { return (a->Skv 
 //     268 (4096 in short rows), 4096 x 32/4 529 -> 514 (8192), 8192 x 4096 x 32/4 1061 -> 1018, 16384 x 8192 x 16/1 2077 -> 1992.
 // Without a finer split: full 16 x 1024 x 16 333 -> 309, 8192 x 16 1064 -> 1013; causal 16 x 1024 x 16 221 -> 215, 2 x 8192 x 8
 // 579 -> 545 (all handing dS over; recomputing 0-7 % faster). A call that fits the built-in scratch of pith_attn_bwd_dkdv_static
-// with 128 keys has to fit it with 256, too: both entry points add up in the same order.
+// with 128 keys has to fit it with 256, too, so that both entry points add up in the same order. This keeps two of the measured
+// calls above on 128 keys, causal 4096 x 64/4 and 8192 x 32/4 (64 MB of partial sums, 128 with 256 keys), and the causal steps of
+// shares of 16384 x 64/4 (none, 128 MB).
 bool wide(const pith_attn_bwd_args* a, const Plan& n, const Plan& w) {
   const int64_t cus = compute_units_or_default(), narrow_wgs = workgroups(a, n), wide_wgs = workgroups(a, w);
   const int64_t narrow_heads = a->Hq / a->Hkv / n.split, wide_heads = a->Hq / a->Hkv / w.split;

@@ -2,15 +2,18 @@
 // (wave A of a pair: S, P, dV; wave B one tile behind: dP, dS, dK) and dS images as attn_bwd_dkdv_d128.h, and the same bits for
 // the same head split: rows are added up in the same steps of 16.
 //
-// What bounds the 128-key kernel on long calls is power: the chip lowers its clock to 1.7 GHz. A fragment read from LDS feeds one
-// product there, 1 KB per 32-cycle product and wave, all that LDS can deliver, and in a loop of nothing but reads and products
-// 1, 2 and 4 products per read run at 1.53, 1.65 and 1.71 PFLOP/s. Here a wave owns two 32-key blocks, so that every fragment
+// What bounds the 128-key kernel on long calls is power: the chip lowers its clock to 1.66-1.71 GHz. A fragment read from LDS feeds
+// one product there, 1 KB per 32-cycle product and wave, all that LDS can deliver, and in a loop of nothing but reads and products
+// (tests/probes/lds_fragment_rate_probe.hip) 1, 2 and 4 products per read run at 1.65, 1.77 and 1.80 PFLOP/s, at 1.64, 1.76 and 1.79
+// GHz. Here a wave owns two 32-key blocks, so that every fragment
 // of Q and dO feeds two products, and a tile requested serves twice as many keys. The accumulators (128 registers) and the
 // stationary fragments (64) then leave room for tiles of 32 query rows, two fragments read ahead and five of eight steps'
 // stationary fragments; the other three stay in LDS (22 reads per 32 products instead of 32; 24 with a third fragment ahead
 // were 1 % slower, and one step more in registers spills without a mask: 8-12 % slower).
 // Measured, dK/dV with the sums over head parts, dS handed over, 128 -> 256 keys, us: 8192 x 4096 x 32/4 heads 1084 -> 1034, 16384 x
 // 8192 x 16/1 2110 -> 2040, 8192 x 16 1096 -> 1029, causal 4 x 4096 x 16 631 -> 606, 8 x 2048 x 16 376 -> 351. Which calls: wide().
+// Counters of the kernel alone at 8192 x 4096 x 32/4: 6.72e7 -> 4.42e7 LDS instructions, 1.71 -> 1.79 GHz, pipe busy 58 -> 60 %, 1055 ->
+// 976 us; no dS 1.66 -> 1.77 GHz, 68 -> 65 % of 4 % more cycles, 929 -> 907 us.
 // Tried: the first fragments of a matrix block read before the barrier that starts it, 0.5 % slower; no s_setprio, 20 % slower.
 #pragma once
 
