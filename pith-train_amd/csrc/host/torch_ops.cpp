@@ -467,8 +467,18 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
 //   F 0.75      4096 x 66/6 1256 / 1282 and 1796 / 1868, 4 x 1536 x 44/4 528 / 536 and 718 / 726, 2 x 3072 x 44/4 causal 957 / 978
 //   F 0.85      2 x 1536 x 45/9 275 / 274 and 384 / 387, 2 x 2048 x 35/7 344 / 345 and 498 / 510
 //   F 1, 1.4    4096 x 40/8 causal 666 / 690, 2 x 2048 x 33/11 282 / 284 and 508 / 549
+// And few workgroups may be mostly empty:
+//   up to 256 rows         8 x 64 x 32/4 51 / 29 and 44 / 35 (64/4 heads), 8 x 128 x 32/4 48 / 39 and 44 / 38, 64 x 64 x 32/4 113 / 91 and 91 / 70, 1024 x
+//                          100 x 4/1 258 / 220, 32 x 192 x 8 49.2 / 48.5 and 52.4 / 52.1, 8 x 256 x 32/4 76 / 74 and 65 / 64, 64 x 256 x 16/4 158 / 159 and
+//                          175 / 179 (and such calls spend more time in Python than on the device)
+//   257 to 512             8 x 257 x 32/4 90 / 94 and 88 / 91, 32 x 320 x 8 78 / 84 and 92 / 101, 64 x 384 x 16/4 257 / 264 and 319 / 340; worst 16 x 288 x 32/4
+//                          full 157 / 155
+//   full, 513 to 639 rows  4 x 513 x 32/4 127 / 108, 4 x 600 x 32/4 138 / 119, 4 x 513 x 64/4 222 / 211, 16 x 540 x 32/4 410 / 391, 8 x 600 x 16 129 / 123;
+//                          640 and more 8 x 640 x 32/8 232 / 233, 16 x 640 x 32/4 439 / 441, 8 x 720 x 16 155 / 164
+//   causal, from 513 on    4 x 513 x 32/4 98 / 99, 4 x 600 x 32/4 113 / 110, 8 x 600 x 32/4 167 / 173, 4 x 600 x 64/4 168 / 174, 8 x 1025 x 32/4 333 / 354
 bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
   if (cus <= 0 || (sq + 511) / 512 * hq * b < cus) return false;
+  if (sq <= 256 || (!causal && sq > 512 && sq < 640)) return false;
   pith_attn_bwd_args a = {};
   a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = a.Dv = 128; a.causal = causal;
   pith_attn_bwd_plan_t plan;

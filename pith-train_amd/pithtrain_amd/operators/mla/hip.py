@@ -234,7 +234,7 @@ def _ds_budget_bytes(device: torch.device, enough: int) -> int:
 def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = False):
     """How the backward of one chunk pair uses the dS hand-over: (kv heads per slab, bytes of the buffer),
     or None when both kernels should recompute (no hand-over path for these head dims, one of the kernels
-    would not fill the device, or not even one kv head fits the budget)."""
+    would not fill the device with work, or not even one kv head fits the budget)."""
     b, sq, hq, _ = q.shape
     skv, hkv = k.shape[1:3]
     units = _device_compute_units(q.device)

@@ -100,6 +100,16 @@ def test_grids_of_unsplit_groups(pays, b, sq, skv, hq, hkv, causal):
     assert native.ds_handover_pays(b, sq, skv, hq, hkv, causal, UNITS) == pays
 
 
+@pytest.mark.parametrize("pays,b,s,hq,hkv", [
+    ("no", 8, 64, 64, 4), ("no", 8, 128, 32, 4), ("no", 64, 64, 32, 4), ("no", 8, 256, 32, 4), ("yes", 8, 257, 32, 4), ("yes", 32, 320, 8, 8), ("yes", 8, 512, 32, 4),
+    ("causal", 4, 513, 32, 4), ("causal", 8, 600, 32, 4), ("causal", 16, 639, 32, 4), ("yes", 8, 640, 32, 8), ("yes", 8, 720, 16, 16), ("yes", 2, 1100, 64, 4),
+    ("yes", 1, 4095, 32, 4), ("yes", 1, 2100, 64, 4), ("yes", 1, 3600, 32, 4),
+])  # fmt: skip
+def test_rows_that_fill_their_workgroups(pays, b, s, hq, hkv):
+    """512-row workgroups that are mostly empty do not fill the device, as measured."""
+    assert [native.ds_handover_pays(b, s, s, hq, hkv, c, UNITS) for c in (True, False)] == {"no": [False] * 2, "yes": [True] * 2, "causal": [True, False]}[pays]
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_slabs_are_asked_for_by_the_rule_of_whole_calls(monkeypatch, causal):
     """A budget for one of two halves of the kv heads: the grid of a slab has to pass the same rule as that of the whole pair."""
