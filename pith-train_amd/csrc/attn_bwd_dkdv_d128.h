@@ -79,7 +79,7 @@ struct TileCursor {
 // order (under the causal mask only the key blocks a query tile can see: ds_tile_start); an image is the four bf16x8 fragments of the pair's B wave as they sit in registers,
 // 1 KB per 16-row step j, the 16 bytes of lane (g, c) at g*512 + ((c ^ 8g ^ 4(j&1)) << 4) (the
 // XOR terms make the reader's transposing LDS reads conflict-free). Keys at or beyond Skv hold 0
-// (their P is masked to 0).
+// (their P is masked to 0), in images of attn_bwd_dkdv_wide.h those of the last 32 that are read.
 template <bool CAUSAL, typename OutT, bool EMIT_DS, bool DESC = false>
 __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, int key_shift = 0) {
   constexpr int KS = kD / 16, DB = kD / 32;

@@ -250,14 +250,18 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(0);
   };
+  // Where dS is handed on, the nonexistent keys of a 32-key block that also holds real ones must read 0: dQ's last step reads them.
+  // Nobody reads what lies behind (such keys have accumulator columns of their own, which are not stored), and a workgroup that masks
+  // them in every tile is what a grid of one round ends on. Backward against 128 keys per workgroup, before -> now: 1664 x 32 heads, full,
+  // +7 -> 0 %, 1920 x 32 +5 -> 0 %, 8064 x 8 +5 -> -1 %, 2432 x 24 +5 -> 0 %, 2 x 3000 x 896 x 32 +1 -> -4 %.
+  const bool mask_keys = p.ds != nullptr && (p.Skv & 31) != 0 && kv_pair0 < p.Skv && kv_pair0 + 32 * KB > p.Skv;
   // A: x = S of query tile mt -> P, left in the exchange buffer (fp32) and in frag (bf16).
   // Rows of the tile are queries q0 + acc_row(v, g); this lane's columns are keys kv_pair0 + 32*kb + c.
   auto make_p = [&](const char* stage, int mt) __attribute__((always_inline)) {
     const float* lse_s = reinterpret_cast<const float*>(stage + 2 * kTile);
     const int q0 = mt * kBM;
-    // tile on the diagonal, ragged last tile, or ragged last key block, whose nonexistent keys must read 0 where dS is handed
-    // on (wave-uniform)
-    const bool masked = (CAUSAL && q0 < kv_pair0 + 32 * KB - 1) || q0 + kBM > p.Sq || kv_pair0 + 32 * KB > p.Skv;
+    // tile on the diagonal, ragged last tile, or mask_keys (wave-uniform)
+    const bool masked = (CAUSAL && q0 < kv_pair0 + 32 * KB - 1) || q0 + kBM > p.Sq || mask_keys;
     f32x4 l4[4];
 #pragma unroll
     for (int b4 = 0; b4 < 4; ++b4) l4[b4] = *reinterpret_cast<const f32x4*>(lse_s + 8 * b4 + 4 * g);
