@@ -14,6 +14,7 @@
 #include <torch/library.h>
 
 #include <array>
+#include <array>
 #include <atomic>
 #include <cstdlib>
 
@@ -485,6 +486,55 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
   if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
   const int64_t key_tiles = (skv + plan.dkdv_rows - 1) / plan.dkdv_rows * plan.dkdv_rows / 128;
   return 4 * key_tiles * hkv * b * plan.dkdv_split >= 3 * cus;
+}
+
+// Whether a share that could be one launch over all chunks goes out step by step instead, because steps hand dS over; `steps`:
+// (rows, keys, causal, kv heads of a slab that hands over at once, 0: recomputes). A step is a grid of its own for either kernel, and the last
+// round of each is lost, which one launch does not know; handing over saves a fifth of the time where the grids are whole rounds. L =
+// rounds of the unmasked steps that hand over against what their workgroups would fill, 0.7 for dK/dV and 0.3 for dQ as their times are;
+// backward, steps / one launch, four ranks, rank 2 zigzag and contiguous unless another is named, us:
+//   L 1          4096 x 64/4 heads 3208 / 3262 and 3779 / 3923, 8192 x 16 3028 / 3209 and 3643 / 3865, 16384 x 8 5864 / 6309 and 7072 / 7493, 8000 x 32/4 5879 / 6432
+//                and 6980 / 7797
+//   L 1.05-1.2   7680 x 32/4 5544 / 5988 and 6683 / 7265, 7168 x 32/4 5048 / 5330 and 6066 / 6328, 2 x 7168 x 32/4 9665 / 9372 and 11836 / 11701, 8192 x 40/8
+//                7793 / 7664 and 9775 / 9485, 6000 x 32 3645 / 3502 and 4216 / 4223
+//   L 1.2-1.4    6144 x 64/4 7452 / 7585 and 9372 / 9466, 3 x 4096 x 32/4 5248 / 5169 and 6285 / 6453, 6144 x 32/4 3979 / 3883 and 4737 / 4352, 11264 x 32/4 12720 /
+//                11931 and 15956 / 14840, 5632 x 64/8 6604 / 5941 and 8074 / 7450, 4 x 3000 x 32/4 4005 / 3511 and 4796 / 4330
+//   L 1.4-1.8    9216 x 32/4 9779 / 8198 and 12376 / 9958, 10240 x 32/4 11186 / 9970 and 14109 / 12097, 5120 x 32/4 2860 / 2531 and 3594 / 3132, 4608 x 32/4
+//                2500 / 2134 and 3201 / 2614, 4 x 1100 x 64/4 1592 / 1152 and 1780 / 1329
+// With short rows the fp32 dQ and the launches of every step weigh more: L 1, 2 x 2048 x 64/4 1783 / 1774 and 2103 / 2130 (two ranks 880 / 987
+// and 1292 / 1381), 2 x 2048 x 32/4 two ranks, rank 0 502 / 475, 8 x 1024 x 32/4 1058 / 904 and 1139 / 1095, 16 x 512 x 32/4 720 / 508 and 700 / 594. Where
+// only the masked step hands over (it has no half-empty round): half of the work, two ranks, rank 0 8192 x 16 1535 / 1582, 6144 x 32/4 1913 /
+// 1867, 1792 x 64/4 448 / 394; less of it, 12288 x 16/2 contiguous 9341 / 8613, 1792 x 64/4 four ranks, rank 0 832 / 715. One launch means two from
+// four dQ workgroups per unit on, and where dQ, two workgroups to a unit, leaves its last round half empty, the steps are faster from a
+// quarter of the work on: two ranks, rank 0 4352 x 32/4 1058 / 1183, 20480 x 8/2 4975 / 5452, 2560 x 64/4 720 / 748, four ranks 1413 / 1555, 5120 x 32/4 2629 /
+// 3013, 2304 x 64/4 1231 / 1303, 2 x 2304 x 32 1253 / 1259; whole rounds 3072 x 64/4 1021 / 977, four ranks 2067 / 2031.
+bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const std::vector<std::array<int64_t, 4>>& steps, int64_t cus) {
+  if (cus <= 0 || hkv <= 0) return false;
+  const auto lost = [&](int64_t wgs, int per_unit = 1) {
+    const int64_t round = per_unit * cus;
+    return (double)((wgs + round - 1) / round * round) / (double)wgs;
+  };
+  double all = 0, handed = 0, full = 0, full_lost = 0;
+  for (const auto& [sq, skv, causal, heads] : steps) {
+    const double work = (double)sq * (double)skv * (causal ? 0.5 : 1.0);
+    all += work;
+    if (heads == 0) continue;
+    handed += work;
+    if (causal) continue;
+    pith_attn_bwd_args a = {};
+    a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq / hkv * heads; a.Hkv = heads; a.Dqk = a.Dv = 128;
+    pith_attn_bwd_plan_t plan;
+    if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
+    full += work;
+    full_lost += work * (0.7 * lost((skv + plan.dkdv_rows - 1) / plan.dkdv_rows * heads * b * plan.dkdv_split) + 0.3 * lost((sq + 511) / 512 * a.Hq * b));
+  }
+  if (handed == 0) return false;
+  if (steps.size() == 1) return true;  // a call like any other
+  const int64_t q_wgs = (rows + 127) / 128 * hq * b;
+  if (full == 0 && q_wgs > 4 * cus && rows >= 2304 && 4 * handed >= all && lost(q_wgs, 2) >= 1.1) return true;
+  if (2 * handed < all) return false;
+  if (rows >= 4096) return full_lost < 1.2 * full || full == 0;
+  return rows >= 2048 && handed == all && (rows + 511) / 512 * hq * b >= 2 * cus && full_lost <= 1.05 * full;
 }
 
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
@@ -1016,4 +1066,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("share_forward_in_one", &share_forward_in_one);
   m.def("share_backward_in_one", &share_backward_in_one);
   m.def("ds_handover_pays", &ds_handover_pays);
+  m.def("share_hands_over", &share_hands_over);
 }

@@ -355,16 +355,22 @@ class RingBackward:
         return self.dq
 
 
+def _steps_beat_one_launch(q: torch.Tensor, hkv: int, steps: Sequence[Tuple[int, int, bool, int]]) -> bool:
+    """steps: (rows, keys, causal, kv heads of a slab that hands dS over at once or 0). Both sides are measured beside the rule."""
+    b, s, hq, _ = q.shape
+    return native.share_hands_over(b, s, hq, hkv, steps, hip._device_compute_units(q.device))
+
+
 def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunks) -> bool:
-    """Whether some step of the share would hand dS from its dK/dV to its dQ kernel: 5 matrix products instead of 7, which is
-    worth more than one launch over all chunks saves (8192 rows x 32/4 heads, four ranks: 5.9 ms handing over, 6.2 ms recomputing
-    in steps, 6.7 ms in one launch; 4096 rows: 1645 us handing over, 1705 us in one launch)."""
+    """Whether enough steps of the share hand dS from their dK/dV to their dQ kernel (5 matrix products instead of 7) to be worth
+    more than one launch over all chunks saves."""
     if q.shape[-1] != 128:
         return False
-    return any(
-        hip.ds_plan(_rows(q, st.q_rows), _rows(k_chunks[st.kv_rank], st.kv_rows), _rows(v_chunks[st.kv_rank], st.kv_rows), st.causal) is not None
-        for st in steps
-    )
+    plans = [hip.ds_plan(_rows(q, st.q_rows), _rows(k_chunks[st.kv_rank], st.kv_rows), _rows(v_chunks[st.kv_rank], st.kv_rows), st.causal) for st in steps]
+    if not any(plans):
+        return False
+    sizes = [(st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0], st.causal, plan[0] if plan else 0) for st, plan in zip(steps, plans)]
+    return _steps_beat_one_launch(q, k_chunks[steps[0].kv_rank].shape[2], sizes)
 
 
 def ring_forward_local(

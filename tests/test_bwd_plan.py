@@ -143,6 +143,30 @@ def test_slabs_that_leave_units_idle_recompute(monkeypatch):
     assert H.ds_plan(q, k, k) is None
 
 
+@pytest.mark.parametrize("steps,b,s,hq,hkv,cp,rank,layout", [
+    (1, 1, 8192, 32, 4, 4, 1, "zigzag"), (1, 1, 4096, 32, 4, 2, 1, "zigzag"), (1, 1, 8192, 16, 16, 4, 2, "contiguous"), (1, 1, 7168, 32, 4, 4, 2, "zigzag"),
+    (1, 1, 7680, 32, 4, 4, 2, "contiguous"), (1, 2, 2048, 64, 4, 2, 1, "contiguous"), (1, 1, 4352, 32, 4, 2, 0, "zigzag"), (1, 1, 20480, 8, 2, 2, 0, "zigzag"),
+    (1, 2, 1536, 64, 4, 4, 0, "contiguous"), (1, 1, 4608, 32, 4, 2, 0, "contiguous"),
+    (1, 1, 2560, 64, 4, 2, 0, "zigzag"), (1, 1, 2304, 64, 4, 4, 0, "zigzag"), (1, 1, 5120, 32, 4, 4, 0, "zigzag"), (0, 1, 3072, 64, 4, 4, 0, "zigzag"),
+    (0, 1, 9216, 32, 4, 4, 2, "zigzag"), (0, 1, 4608, 32, 4, 4, 2, "contiguous"), (0, 1, 5120, 64, 4, 4, 2, "zigzag"), (0, 1, 10240, 16, 4, 4, 2, "zigzag"),
+    (0, 2, 1536, 64, 4, 4, 2, "zigzag"), (0, 16, 512, 32, 4, 4, 2, "zigzag"), (0, 4, 1100, 64, 4, 2, 1, "contiguous"), (0, 4, 3000, 32, 4, 4, 2, "zigzag"),
+    (0, 1, 1792, 64, 4, 4, 0, "zigzag"), (0, 1, 1792, 64, 4, 4, 3, "zigzag"), (0, 1, 2048, 64, 4, 2, 0, "zigzag"), (0, 1, 1024, 8, 2, 4, 2, "zigzag"),
+])  # fmt: skip
+def test_shares_that_hand_over_go_out_step_by_step_where_that_is_faster(steps, b, s, hq, hkv, cp, rank, layout):
+    """As measured (table at share_hands_over), with the steps that hand over by the rule of calls."""
+    sizes = [(st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0], st.causal) for st in ring_schedule(rank, cp, s, layout)]
+    sizes = [(m, n, c, hkv if native.ds_handover_pays(b, m, n, hq, hkv, c, UNITS) else 0) for m, n, c in sizes]
+    assert native.share_hands_over(b, s, hq, hkv, sizes, UNITS) == bool(steps)
+
+
+def test_share_of_slabs_counts_their_grids():
+    """131072 tokens, 64/4 heads: a slab of one kv head at a time fills the device; a quarter of its heads would not."""
+    sizes = lambda heads: [(16384, 8192, False, heads)] * 3 + [(8192, 16384, False, heads)] * 4 + [(16384, 16384, True, 0)]  # noqa: E731
+    assert native.share_hands_over(1, 16384, 64, 4, sizes(1), UNITS) and native.share_hands_over(1, 16384, 64, 4, sizes(4), UNITS)
+    small = [(16384, 8192, False, 1)] * 3
+    assert not native.share_hands_over(1, 16384, 16, 4, small, UNITS) and not native.share_hands_over(1, 16384, 64, 4, [], UNITS)
+
+
 @pytest.mark.gpu
 def test_more_workgroups_than_one_launch_takes(gpu):
     """One row attends to itself: O = V, dV = dO, dQ = dK = 0. 8.5 M workgroups of either kernel."""

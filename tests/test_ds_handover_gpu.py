@@ -190,6 +190,19 @@ def test_ring_share_uses_the_handover(gpu, layout, monkeypatch):
     check_bf16_result(dq1, dq_ref, "ring dQ", otol=1e-3)
 
 
+@pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
+def test_small_ring_share_step_by_step_uses_the_handover(gpu, layout, monkeypatch):
+    """The same with the rule that would send a share this small out as one launch switched off."""
+    from pithtrain_amd.operators.mla import hip as H
+    from pithtrain_amd.operators.ring_attention import local as L
+
+    buffers, real = [], H._try_alloc
+    monkeypatch.setattr(L, "_steps_beat_one_launch", lambda *a: True)
+    monkeypatch.setattr(H, "_try_alloc", lambda *a: buffers.append(real(*a)) or buffers[-1])
+    test_ring_share_uses_the_handover(gpu, layout, monkeypatch)
+    assert buffers, "no step handed dS over"
+
+
 def _shaped(gpu, b, s, hq, hkv):
     q = torch.empty(b, s, hq, 128, dtype=torch.bfloat16, device=gpu)
     k = torch.empty(b, s, hkv, 128, dtype=torch.bfloat16, device=gpu)
