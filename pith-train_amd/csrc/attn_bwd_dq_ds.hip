@@ -22,6 +22,11 @@
 // from transposing reads of the image, in the same key slot order. The accumulators therefore hold
 // dQ untransposed (a lane owns one feature column of 16 rows) and the epilogue reads and writes whole
 // 128-byte lines (store_rows32).
+// The images are read once, by one workgroup, and all of them exceed every cache: loaded non-temporally they leave the caches to K
+// and to what the dK/dV launch wrote last. The kernel alone over 4096 x 32/4 heads, plain / non-temporal: under the mask 118 / 99
+// us, without 196 / 169 (6.4 TB/s); with the dK/dV launch before it (the same rows) 436 / 422, 8192 x 32/4 1584 / 1559, 3 x 1999 x 32/4
+// 363 / 348, 4 x 1024 x 32/4 152.5 / 151.6. Past the vector cache only (sc1), or past more than that (sc0 nt, sc1 nt, sc0 sc1 nt): 0-3 %
+// slower than nt.
 // With 192-feature keys the same scheme was measured not to pay: a workgroup then holds accumulators
 // for 256 rows only, K is 43 % of the bytes a compute unit requests, and the kernel is no faster than
 // recomputing the scores.
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
         const char* src = ds_src[r] + (int64_t)s * 4096;
         char* dst = smem + kOffDs + slot * kDsStage + (wave - 4 + 4 * r) * kDsWave;
 #pragma unroll
-        for (int j = 0; j < kLoadsDs; ++j) load_lds16(src + j * 1024, off, dst + j * 1024);
+        for (int j = 0; j < kLoadsDs; ++j) load_lds16_once(src + j * 1024, off, dst + j * 1024);
       }
   };
   // loads this wave issued for step t

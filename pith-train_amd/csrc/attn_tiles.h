@@ -233,6 +233,15 @@ __device__ __forceinline__ void load_lds16(const char* base, int offset, char* d
                : "memory");
 }
 
+// The same for bytes that nobody reads again: they pass through the caches without displacing what is read later.
+__device__ __forceinline__ void load_lds16_once(const char* base, int offset, char* dst_wave) {
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_char*)dst_wave;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+               :
+               : "s"(lds_addr), "v"(offset), "s"(base)
+               : "memory");
+}
+
 // 4 bytes per lane from the per-lane global address `src` to LDS at `dst_wave` + 4 * lane (same
 // conventions as load_lds16).
 __device__ __forceinline__ void load_lds4(const void* src, char* dst_wave) {
