@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kDeltaThreads) void delta_kernel(DeltaParams p) {
     float acc = 0.f;
     if (c < chunks) {
       Vec8<__bf16> x, y;
-      x.load(o + (int64_t)c * 8);
+      x.load_nt(o + (int64_t)c * 8);  // (dO is read again by the gradient kernels, O by nobody)
       y.load(g + (int64_t)c * 8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc += x.get(j) * y.get(j);
