@@ -325,7 +325,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
       asm volatile("" : "+v"(off));
 #pragma unroll
       for (int j = 0; j < kDsStoresPerInterval; ++j)
-        __builtin_nontemporal_store(frag[j], reinterpret_cast<bf16x8*>(img + j * 1024 + (off ^ ((j & 1) << 6))));
+        store16_through(img + j * 1024, off ^ ((j & 1) << 6), frag[j]);
     }
   };
 

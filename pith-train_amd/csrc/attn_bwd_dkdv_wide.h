@@ -315,7 +315,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block) 
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        __builtin_nontemporal_store(frag[kb][j], reinterpret_cast<bf16x8*>(img + kb * 4096 + j * 1024 + (off ^ (j << 6))));
+        store16_through(img + kb * 4096 + j * 1024, off ^ (j << 6), frag[kb][j]);
     return true;
   };
 

@@ -242,6 +242,14 @@ __device__ __forceinline__ void load_lds16_once(const char* base, int offset, ch
                : "memory");
 }
 
+// 16 bytes per lane to `base` (wave-uniform) + `offset`, written through the second-level cache (sc1) and kept by none (nt): for what
+// another launch reads, while this one shares tiles through that cache. dS images, plain / nt / sc1 nt / sc0 sc1 nt, forward + backward of
+// 4096 x 32/4 heads of 128 569 / 533 / 525 / 527 us, share of 8192 x 32/4 7820 / 7440 / 7353 / 7352 us. The wait states are those
+// that a VALU write of the data registers needs behind a store of more than 8 bytes; the compiler does not see the store.
+__device__ __forceinline__ void store16_through(char* base, int offset, bf16x8 value) {
+  asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" : : "v"(offset), "v"(__builtin_bit_cast(u32x4, value)), "s"(base) : "memory");
+}
+
 // 4 bytes per lane from the per-lane global address `src` to LDS at `dst_wave` + 4 * lane (same
 // conventions as load_lds16).
 __device__ __forceinline__ void load_lds4(const void* src, char* dst_wave) {
