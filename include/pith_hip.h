@@ -299,7 +299,7 @@ int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* args);
  * diagonal: about half). Results agree with the recomputing dQ kernel up to
  * fp32 summation order (the dS values are the same bf16 numbers). The buffer holds nothing of
  * value after the dQ call. Returns the bytes needed, or 0 when the shape has no hand-over path
- * (head dims other than (128,128)); with ds == NULL or a buffer that is too small both calls
+ * (head dims other than (128,128) and (192,128), the latter up to 128 rows, keys in two parts); with ds == NULL or a buffer that is too small both calls
  * behave as before. */
 int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* args);
 
@@ -308,7 +308,7 @@ int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* args);
 typedef struct {
   int32_t dkdv_rows;    /* pith_attn_bwd_dkdv, launched alone: key rows per workgroup */
   int32_t dkdv_split;   /* and the parts each group of query heads is cut into (given the workspace) */
-  int32_t dq_ds_pairs;  /* pith_attn_bwd_dq from handed-over dS, causal: workgroups take rows from both ends */
+  int32_t dq_ds_pairs;  /* pith_attn_bwd_dq from handed-over dS, 128 features, causal: workgroups take rows from both ends */
   int32_t one_grid;     /* pith_attn_bwd with bf16 gradients and without ds: both kernels in one launch */
 } pith_attn_bwd_plan_t;
 

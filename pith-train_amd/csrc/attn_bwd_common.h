@@ -34,7 +34,7 @@ struct BwdParams {
   const __bf16* k_pe;
   int64_t k_pe_bs, k_pe_rs;
   float* ws_dkpe;
-  // dS hand-over from the dK/dV kernel to the dQ kernel (head dims 128/128): bf16 images, 16 KB per
+  // dS hand-over from the dK/dV kernel to the dQ kernel (head dims 128/128 and 192/128): bf16 images, 16 KB per
   // (batch, query head, 64-row query tile, 128-key block); ds_qt / ds_kb = number of such tiles / blocks.
   // Without a causal mask a head holds ds_qt x ds_kb of them, query tile by query tile; under the mask
   // only the blocks a tile can see are kept (tile t: its first t/2 + 1 key blocks, see ds_tile_start).
@@ -42,7 +42,7 @@ struct BwdParams {
   char* ds;
   int ds_qt, ds_kb;
   int64_t ds_hs;
-  int ds_pairs;  // dQ from dS under the mask: a workgroup takes 256-row blocks from both ends (dq_ds_pairs)
+  int ds_pairs;  // dQ from dS under the mask: a workgroup takes half tiles from both ends (dq_ds_pairs)
   // dQ kernels, fp32 dq: query rows [final_r0, final_r1) (multiples of 32, or Sq) receive their result, old
   // contents of dq included when accumulating, as bf16 in dq_final instead of dq (nullptr: none do)
   __bf16* dq_final;
@@ -269,11 +269,12 @@ void launch_dq_direct(const BwdParams& p, int dqk, bool causal, bool f32_out, hi
 // dQ with two 4-wave workgroups of 128 query rows per compute unit, all head dims: attn_bwd_dq_duo.hip.
 void launch_dq_duo(const BwdParams& p, int dqk, bool causal, bool f32_out, hipStream_t stream);
 
-// dQ for head dims (128, 128) from the dS images the dK/dV kernel left in p.ds: attn_bwd_dq_ds.hip.
-// p.q_tiles = number of 512-row query tiles.
-// Whether under the mask a grid of that many workgroups takes 256-row blocks from both ends of the rows.
+// dQ for head dims (128, 128) and (192, 128) from the dS images the dK/dV kernel left in p.ds: attn_bwd_dq_ds.hip.
+// p.q_tiles = number of tiles of dq_ds_rows query rows.
+constexpr int dq_ds_rows(int dqk) { return dqk == 192 ? 256 : 512; }
+// Whether under the mask a grid of that many workgroups takes blocks of half a tile from both ends of the rows.
 bool dq_ds_pairs(int64_t workgroups);
-void launch_dq_from_ds(BwdParams p, bool causal, bool f32_out, hipStream_t stream);
+void launch_dq_from_ds(BwdParams p, int dqk, bool causal, bool f32_out, hipStream_t stream);
 // Bytes of dS images for a shape (0: the shape has no hand-over path), and whether the call brings a buffer for them.
 int64_t ds_bytes_for(const pith_attn_bwd_args* a);
 bool ds_usable(const pith_attn_bwd_args* a);

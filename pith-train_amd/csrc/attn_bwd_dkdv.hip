@@ -231,7 +231,7 @@ extern "C" int pith_attn_bwd_plan(const pith_attn_bwd_args* a, pith_attn_bwd_pla
   const Plan chosen = pick_plan(a, plan_for(a, kBN));
   plan->dkdv_rows = chosen.rows;
   plan->dkdv_split = chosen.split;
-  plan->dq_ds_pairs = a->causal && ds_bytes_for(a) > 0 && dq_ds_pairs((a->Sq + 511) / 512 * a->Hq * a->B);
+  plan->dq_ds_pairs = a->causal && a->Dqk == 128 && ds_bytes_for(a) > 0 && dq_ds_pairs((a->Sq + 511) / 512 * a->Hq * a->B);
   pith_attn_bwd_args bf16 = *a;
   bf16.ds = nullptr;
   bf16.dq_dtype = bf16.dkv_dtype = PITH_BF16;

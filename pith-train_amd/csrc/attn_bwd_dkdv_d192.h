@@ -88,7 +88,8 @@ struct DirectExtra {
 constexpr int kTB = 2;  // 64-row query tiles (32-row tiles, 1, measured 3 % slower)
 constexpr int kSmem = Layout<kTB>::kSmem;
 
-template <bool CAUSAL, typename OutT, int TB = kTB>
+// EMIT_DS: wave B also stores every dS tile it forms to p.ds, in the layout and with the waits of attn_bwd_dkdv_d128.h.
+template <bool CAUSAL, typename OutT, bool EMIT_DS = false, int TB = kTB>
 __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, int key_shift = 0) {
   using L = Layout<TB>;
   constexpr int kBM = L::kBM, kStage = L::kStage, kOffExtra = L::kOffExtra, kOffO = L::kOffO, kOffStat = L::kOffStat;
@@ -301,7 +302,8 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
   auto make_p = [&](const char* stage, int mt) __attribute__((always_inline)) {
     const float* lse_s = reinterpret_cast<const float*>(stage + kOffStat);
     const int q0 = mt * kBM;
-    const bool masked = (CAUSAL && q0 < kv_pair0 - key_shift + 31) || (q0 + kBM > p.Sq);  // wave-uniform: diagonal or ragged tile
+    const bool masked = (CAUSAL && q0 < kv_pair0 - key_shift + 31) || (q0 + kBM > p.Sq) ||
+                        (EMIT_DS && kv_pair0 + 32 > p.Skv);  // wave-uniform: diagonal or ragged tile, nonexistent keys whose dS is read
 #pragma unroll
     for (int rb = 0; rb < TB; ++rb) {
       f32x4 l4[4];
@@ -313,7 +315,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int qrow = q0 + 32 * rb + acc_row(v, g);
-          if ((CAUSAL && key - key_shift > qrow) || qrow >= p.Sq) x[rb][v] = 0.f;
+          if ((CAUSAL && key - key_shift > qrow) || qrow >= p.Sq || (EMIT_DS && key >= p.Skv)) x[rb][v] = 0.f;
         }
       }
 #pragma unroll
@@ -329,7 +331,9 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
   };
   // B: x = delta - dP of the tile in `stage`, P from the exchange buffer -> -dS / scale in frag (bf16),
   // one 32-row block at a time (the temporaries of a block are dead before the next one is read).
-  auto make_ds = [&](const char* stage) __attribute__((always_inline)) {
+  // With EMIT_DS each block's two fragments are also stored, into the image of `tile`, the (query head, tile) that the stage holds.
+  char* const ds_wg = EMIT_DS ? p.ds + ((int64_t)n_tile * 4 + pair) * 4096 : nullptr;
+  auto make_ds = [&](const char* stage, const TileCursor& tile) __attribute__((always_inline)) {
 #pragma unroll
     for (int rb = 0; rb < TB; ++rb) {
       f32x4 pr[4];
@@ -341,6 +345,13 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
       for (int jj = 0; jj < 2; ++jj)
         frag[2 * rb + jj] = to_bf16x8(x[rb][8 * jj], x[rb][8 * jj + 1], x[rb][8 * jj + 2], x[rb][8 * jj + 3],
                                       x[rb][8 * jj + 4], x[rb][8 * jj + 5], x[rb][8 * jj + 6], x[rb][8 * jj + 7]);
+    }
+    if constexpr (EMIT_DS) {
+      char* img = ds_wg + (int64_t)(b * p.Hq + tile.hq) * p.ds_hs + ds_tile_start<CAUSAL>(tile.mt, p.ds_kb) * kDsBlockBytes;
+      int off = (g << 9) + ((c ^ (g << 3)) << 4);  // recomputed per tile: no register is held across the interval
+      asm volatile("" : "+v"(off));
+#pragma unroll
+      for (int j = 0; j < 2 * TB; ++j) store16_through(img + j * 1024, off ^ ((j & 1) << 6), frag[j]);
     }
   };
 
@@ -365,11 +376,14 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
   // other: its P is all zeros. Ring stages rotate: prev <- cur <- next <- (the stage prev used to be).
   auto run = [&](auto role_tag) __attribute__((always_inline)) {
     constexpr bool ROLE_B = decltype(role_tag)::value;
-    TileCursor cur = {hq0, m_first};
+    TileCursor cur = {hq0, m_first}, done = cur;  // tiles i and i-1 of interval i
     int off_prev = 2 * kStage, off_cur = 0, off_next = kStage;
-    auto end_interval = [&]() __attribute__((always_inline)) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // the tile requested in this interval has landed
+    auto end_interval = [&](bool stored) __attribute__((always_inline)) {
+      // the tile requested in this interval has landed; the dS stores that wave B issued behind the request may stay in flight
+      if (ROLE_B && EMIT_DS && stored) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * TB));
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
       __syncthreads();
+      done = cur;
       cur.advance(m_first, m_end);
       const int t = off_prev;
       off_prev = off_cur;
@@ -386,7 +400,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
       __syncthreads();
       straight_product(smem + off_cur, role_tag);
     }
-    end_interval();
+    end_interval(false);
     for (int i = 1; i < n_iter; ++i) {
       const char* stage_cur = smem + off_cur;
       const char* stage_prev = smem + off_prev;
@@ -397,18 +411,18 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
         make_p(stage_cur, cur.mt);
       } else {
         if (will_request) request(smem + off_next);
-        make_ds(stage_prev);
+        make_ds(stage_prev, done);
         __syncthreads();
         matrix_block(stage_prev, stage_cur, role_tag);
       }
-      end_interval();
+      end_interval(true);
     }
     // interval n_iter
     if (!ROLE_B) {
       transposed_product(smem + off_prev, role_tag);
       __syncthreads();
     } else {
-      make_ds(smem + off_prev);
+      make_ds(smem + off_prev, done);
       __syncthreads();
       transposed_product(smem + off_prev, role_tag);
     }

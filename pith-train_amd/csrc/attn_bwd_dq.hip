@@ -105,7 +105,8 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
 }
 
 int64_t ds_bytes_for(const pith_attn_bwd_args* a) {
-  if (!a || a->Dqk != 128 || a->Dv != 128 || a->k_pe || a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || a->Skv <= 0) return 0;
+  if (!a || (a->Dqk != 128 && a->Dqk != 192) || a->Dv != 128 || a->k_pe || a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || a->Skv <= 0) return 0;
+  if (a->Dqk == 192 && a->Sq <= dq_ds_rows(192) / 2) return 0;  // half of every dQ workgroup would be empty
   const int qt = (int)((a->Sq + 63) / 64), kb = (int)((a->Skv + kDkdvBlockN - 1) / kDkdvBlockN);
   // a causal call (Sq == Skv) keeps only the key blocks at or below the diagonal of every query tile
   const int64_t blocks = a->causal ? ds_tile_start<true>(qt, kb) : ds_tile_start<false>(qt, kb);
@@ -154,8 +155,9 @@ extern "C" int pith_attn_bwd_dq(const pith_attn_bwd_args* a, pith_stream_t strea
     // dS was left by the dK/dV call of the same chunk: one product instead of three
     if ((uintptr_t)a->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
     p.ds = reinterpret_cast<char*>(a->ds);
-    p.q_tiles = (int)((a->Sq + 511) / 512);
-    launch_dq_from_ds(p, a->causal != 0, f32, st);
+    const int rows = dq_ds_rows((int)a->Dqk);
+    p.q_tiles = (int)((a->Sq + rows - 1) / rows);
+    launch_dq_from_ds(p, (int)a->Dqk, a->causal != 0, f32, st);
   } else if (dq_split_keys(a)) {
     launch_dq_direct(p, (int)a->Dqk, a->causal != 0, f32, st);
   } else {

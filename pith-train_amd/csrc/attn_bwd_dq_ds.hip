@@ -1,11 +1,11 @@
-// Query-gradient kernel for head dims (128, 128) on gfx950 that reads dS instead of recomputing it:
+// Query-gradient kernel for head dims (128, 128) and (192, 128) on gfx950 that reads dS instead of recomputing it:
 // dQ = scale * dS K (pithtrain/operators/mla/triton.py:205-266, the last product of the loop body),
 // with dS = P*(dP - delta) taken, already rounded to bf16 and with its sign flipped, from the images
-// that the dK/dV kernels of attn_bwd_dkdv_d128.h and attn_bwd_dkdv_wide.h leave in p.ds (layout documented in the former). The two score products that the
+// that the dK/dV kernels of attn_bwd_dkdv_d128.h, attn_bwd_dkdv_wide.h and attn_bwd_dkdv_d192.h leave in p.ds (layout documented in the former). The two score products that the
 // other dQ kernels repeat are gone; the price is one trip of dS through memory, so this kernel is
 // bound by the rate at which it can stream the images, not by the matrix pipe.
 //
-// Work split: a workgroup of 8 wavefronts owns 512 query rows of one (batch, head), a wave one 64-row query tile of the
+// Work split (128 features; 192 below): a workgroup of 8 wavefronts owns 512 query rows of one (batch, head), a wave one 64-row query tile of the
 // writer (under the mask in a grid of one round two blocks of 256 rows, see dq_ds_pairs). Keys are visited in steps of 32 (one
 // wave pair of the writer). Per step the K tile (shared, packed and swizzled like everywhere else, 8 KB) and, per
 // wave, the 4 KB image of its tile for that pair (copied verbatim) go global -> LDS directly. What
@@ -27,12 +27,15 @@
 // us, without 196 / 169 (6.4 TB/s); with the dK/dV launch before it (the same rows) 436 / 422, 8192 x 32/4 1584 / 1559, 3 x 1999 x 32/4
 // 363 / 348, 4 x 1024 x 32/4 152.5 / 151.6. Past the vector cache only (sc1), or past more than that (sc0 nt, sc1 nt, sc0 sc1 nt): 0-3 %
 // slower than nt.
-// With 192-feature keys the same scheme was measured not to pay: a workgroup then holds accumulators
-// for 256 rows only, K is 43 % of the bytes a compute unit requests, and the kernel is no faster than
-// recomputing the scores.
+// (192, 128): accumulators for 512 rows do not fit, so a workgroup owns 256 rows (under the mask in one round two blocks of 128), and
+// two waves share a 64-row tile, each with 96 of the features: a wave reads 2 + 3 KB of fragments per 6 products, and neither its images
+// nor K are requested twice. K is 43 % of what a unit requests, so the images get the deeper ring: 7 stages of 16 KB beside 3 of 12.
+// dQ from dS / the recomputing kernels, us (dK/dV with / without the stores): 4096 x 16 causal 95 / 130 (166 / 160), 8192 x 16 251 / 438
+// (660 / 578), 4096 x 2048 x 16 68 / 114 (150 / 145), 4096 x 128 causal 570 / 936 (1468 / 1280).
 #include <type_traits>
 
 #include "attn_bwd_common.h"
+#include "attn_bwd_dkdv_d192.h"
 
 namespace pith {
 namespace {
@@ -61,19 +64,22 @@ __device__ __forceinline__ void wait_vector_loads_but(int n) {
   }
 }
 
-template <bool CAUSAL, typename OutT>
+template <int DQK, bool CAUSAL, typename OutT>
 __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
-  constexpr int DQK = 128, DB = DQK / 32;
+  constexpr int FS = DQK == 192 ? 2 : 1;    // waves that share 64 query rows, a part of the features each
+  constexpr int RG = 8 / FS;                // 64-row groups of a workgroup
+  constexpr int DB = DQK / 32 / FS;         // feature blocks per wave
   constexpr int QW = 64;                    // query rows per wave
   constexpr int RBW = QW / 32;              // 32-row blocks per wave
-  constexpr int kBM = 8 * QW;               // query rows per workgroup
-  constexpr int kKStage = kBN * kRowBytes128;                        // 8 KB
-  constexpr int kDsWave = RBW * 2048;                                // per wave and step
-  constexpr int kDsStage = 8 * kDsWave;                              // 32 KB
-  constexpr int kRingD = 4;                                          // images: step s in use, the next three requested
+  constexpr int kBM = RG * QW;              // query rows per workgroup
+  constexpr int kKStage = kBN * DQK * 2;                             // 8 KB, 12 KB
+  constexpr int kDsWave = RBW * 2048;                                // per row group and step
+  constexpr int kDsStage = RG * kDsWave;                             // 32 KB, 16 KB
+  constexpr int kRingD = DQK == 192 ? 7 : 4;                         // images: step s in use, the next ones requested
   constexpr int kOffDs = kRingK * kKStage;
   constexpr int kLoadsDs = 2 * RBW;                                  // per image
-  constexpr int kLoadsK = 2;                                         // per K-moving wave and step
+  constexpr int kImages = RG / 4;                                    // per image-moving wave and step
+  constexpr int kLoadsK = DQK / 64;                                  // per K-moving wave and step
   static_assert(kOffDs + kRingD * kDsStage <= 160 * 1024, "the rings must fit the LDS");
   __shared__ __attribute__((aligned(1024))) char smem[kOffDs + kRingD * kDsStage];
 
@@ -86,16 +92,17 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   // Query tiles of the waves: eight consecutive ones, or, with ds_pairs, two 256-row blocks, waves 0..3 the m_tile-th from the
   // start and waves 4..7 the m_tile-th from the end, so that all workgroups read the same number of images (the middle one of
   // an odd number of blocks goes to waves 4..7 alone).
+  const int rg = wave & (RG - 1), fh = wave / RG;
   const bool pairs = CAUSAL && p.ds_pairs;
-  const int blocks256 = (p.Sq + kBM / 2 - 1) / (kBM / 2);
+  const int half_blocks = (p.Sq + kBM / 2 - 1) / (kBM / 2);
   auto rows_of = [&](int w) __attribute__((always_inline)) {
     if (!pairs) return m_tile * kBM + w * QW;
-    const int late = blocks256 - 1 - m_tile;
-    const int block = w >= 4 ? late : m_tile < late ? m_tile : blocks256;  // blocks256: none
-    return block * (kBM / 2) + (w & 3) * QW;
+    const int late = half_blocks - 1 - m_tile;
+    const int block = w >= RG / 2 ? late : m_tile < late ? m_tile : half_blocks;  // half_blocks: none
+    return block * (kBM / 2) + (w & (RG / 2 - 1)) * QW;
   };
-  const int m_end = pairs ? (blocks256 - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
-  const int q_wave0 = rows_of(wave), q_other0 = rows_of(wave & 3);  // q_other0: of the wave whose images waves 4..7 also request
+  const int m_end = pairs ? (half_blocks - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
+  const int q_wave0 = rows_of(rg);
 
   const int kv_row_bytes = p.HkvT * DQK * 2;
   const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * DQK);
@@ -116,22 +123,31 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
     return p.ds + (int64_t)(b * p.Hq + h) * p.ds_hs + ds_tile_start<CAUSAL>(mt, p.ds_kb) * kDsBlockBytes + (q0 & 63) * 64;
   };
 
-  // ---- requests. Waves 0..3: K tiles. Waves 4..7: the dS parts of waves w-4 and w.
+  // ---- requests. Waves 0..3: K tiles. Waves 4..7: the images of row groups w-4 and, with 8 of them, w.
   const bool k_mover = wave < 4;
   DirectTile128<kBN, 256> mover;
   mover.init(kv_row_bytes, wave & 3, lane);
-  const char* ds_src[2] = {images_of(q_other0), images_of(q_wave0)};        // only used by waves 4..7
-  const int ds_steps[2] = {k_mover ? 0 : steps_of(q_other0), k_mover ? 0 : n_steps_wave};
+  dkdv_d192::DirectExtra<kBN / 2> extra;  // features 128..191
+  if constexpr (DQK == 192) extra.init(kv_row_bytes, wave & 3, lane);
+  const char* ds_src[kImages];  // only used by waves 4..7
+  int ds_steps[kImages];
+#pragma unroll
+  for (int r = 0; r < kImages; ++r) {
+    const int q0 = rows_of((wave & 3) + 4 * r);
+    ds_src[r] = images_of(q0);
+    ds_steps[r] = k_mover ? 0 : steps_of(q0);
+  }
   auto request_k = [&](int s, int slot) __attribute__((always_inline)) {
     char* stage = smem + slot * kKStage;
     const char* k_src = kh + (int64_t)s * kBN * kv_row_bytes;
     mover.issue(k_src, p.Skv - s * kBN, stage, wave & 3, lane);
+    if constexpr (DQK == 192) extra.issue(k_src, p.Skv - s * kBN, stage + kBN * kRowBytes128, wave & 3, lane);
   };
   auto request_ds = [&](int s, int slot) __attribute__((always_inline)) {
     int off = lane << 4;
     asm volatile("" : "+v"(off));
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < kImages; ++r)
       if (s < ds_steps[r]) {
         const char* src = ds_src[r] + (int64_t)s * 4096;
         char* dst = smem + kOffDs + slot * kDsStage + (wave - 4 + 4 * r) * kDsWave;
@@ -143,7 +159,10 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   auto loads_of = [&](int t) __attribute__((always_inline)) {
     if (t >= n_steps_wg) return 0;
     if (k_mover) return kLoadsK;
-    return (t < ds_steps[0] ? kLoadsDs : 0) + (t < ds_steps[1] ? kLoadsDs : 0);
+    int n = 0;
+#pragma unroll
+    for (int r = 0; r < kImages; ++r) n += t < ds_steps[r] ? kLoadsDs : 0;
+    return n;
   };
   // ring slots of step s (K tiles, dS parts) and of the steps to request next; advanced by one per step
   int k_slot = 0, k_next = kRingK - 1, d_slot = 0, d_next = kRingD - 1;
@@ -156,17 +175,17 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   // waits until this wave's loads for step s have landed: the steps requested after it (all but the
   // last of the ring, which follows after the barrier) may stay in flight. Away from the end of the key
   // range that is a constant number of loads.
-  constexpr int kSteadyDs = (kRingD - 2) * 2 * kLoadsDs;
+  constexpr int kSteadyDs = (kRingD - 2) * kImages * kLoadsDs;
   static_assert(kRingK == 3 && kSteadyDs < 32, "one K step in flight; dS loads in flight fit the decision tree");
-  const int ds_steady_end = min(min(ds_steps[0], ds_steps[1]), n_steps_wg) - (kRingD - 2);  // steps below: steady state
-  const int ds_single_end = min(ds_steps[1], n_steps_wg) - (kRingD - 2);
+  const int ds_steady_end = min(min(ds_steps[0], ds_steps[kImages - 1]), n_steps_wg) - (kRingD - 2);  // steps below: steady state
+  const int ds_single_end = min(ds_steps[kImages - 1], n_steps_wg) - (kRingD - 2);
   auto wait_step = [&](int s) __attribute__((always_inline)) {
     if (k_mover) {
       if (s + 1 < n_steps_wg) wait_vector_loads_but<kLoadsK>();
       else wait_vector_loads_but<0>();
     } else if (s < ds_steady_end) {
       wait_vector_loads_but<kSteadyDs>();
-    } else if (CAUSAL && s >= ds_steps[0] && s < ds_single_end) {  // only the later block's images are left
+    } else if (CAUSAL && kImages == 2 && s >= ds_steps[0] && s < ds_single_end) {  // only the later block's images are left
       wait_vector_loads_but<kSteadyDs / 2>();
     } else {
       int n = 0;
@@ -190,6 +209,20 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   // key 4g + i (+ 8 for the upper read) at queries 16*chalf + 4m .. +3 of a 32-row block: 16-row step
   // chalf of the block, writer lane group m&1, fragment half m>>1.
   const int t_base[2] = {transposed_offset128(0, 0, 0, lane), transposed_offset128(0, 1, 0, lane)};
+  // with 192 features per 16-key step and block of this wave, blocks 4 and 5 in the extra tile (its two 16-key steps side by side)
+  int k_off[DQK == 192 ? 2 : 1][DB][2];
+  if constexpr (DQK == 192) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int o = 0; o < DB; ++o) {
+        const int fb = DB * fh + o;
+        const int tile = fb < 4 ? ks * 16 * kRowBytes128 : kBN * kRowBytes128;
+        const int piece_bits = fb < 4 ? fb << 6 : (8 * ks + 4 * (fb - 4)) << 4;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) k_off[ks][o][hh] = tile + (t_base[hh] ^ piece_bits);
+      }
+  }
   int ds_off[2];
   {
     const int r = lane & 15, chalf = (lane >> 4) & 1;
@@ -210,8 +243,13 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
       }
 #pragma unroll
       for (int o = 0; o < DB; ++o) {
-        const char* kt = stage + ks * 16 * kRowBytes128;
-        const bf16x8 a = lds_read_transposed_at(kt + (t_base[0] ^ (o << 6)), kt + (t_base[1] ^ (o << 6)));
+        bf16x8 a;
+        if constexpr (DQK == 192) {
+          a = lds_read_transposed_at(stage + k_off[ks][o][0], stage + k_off[ks][o][1]);
+        } else {
+          const char* kt = stage + ks * 16 * kRowBytes128;
+          a = lds_read_transposed_at(kt + (t_base[0] ^ (o << 6)), kt + (t_base[1] ^ (o << 6)));
+        }
 #pragma unroll
         for (int rb = 0; rb < RBW; ++rb) acc[rb][o] = mfma32(dsf[rb], a, acc[rb][o]);
       }
@@ -236,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
       if (s + kRingD - 1 < n_steps_wg) request_ds(s + kRingD - 1, d_next);
     }
     if constexpr (decltype(compute_tag)::value)
-      compute(smem + k_slot * kKStage, smem + kOffDs + d_slot * kDsStage + wave * kDsWave);
+      compute(smem + k_slot * kKStage, smem + kOffDs + d_slot * kDsStage + rg * kDsWave);
     advance();
   };
   int s = 0;
@@ -244,7 +282,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   // other waves of the workgroup may still have steps to visit: keep moving tiles, keep in step
   for (; s < n_steps_wg; ++s) step(s, std::false_type{});
 
-  OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK;
+  OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK + fh * (32 * DB);
   const float sc = -p.scale;  // the images hold -dS (the writer forms delta - dP)
   const int64_t row_stride = (int64_t)p.HqT * DQK;
 #pragma unroll
@@ -252,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
     const int row0 = q_wave0 + 32 * rb;
     __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
     if (p.dq_final != nullptr && row0 >= p.final_r0 && row0 < p.final_r1)
-      fin = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + row0 * row_stride;
+      fin = p.dq_final + b * p.dq_final_bs + (int64_t)h * DQK + fh * (32 * DB) + row0 * row_stride;
     store_rows32<OutT, DB>(dqh + row0 * row_stride, row_stride, p.Sq - row0, acc[rb], sc, p.accumulate_dq != 0, c, g, fin);
   }
 }
@@ -270,16 +308,21 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
 //   2.75, 3, 4        11264 x 32/4 785 / 799, 12288 x 32/4 921 / 904, 3 x 4096 x 32/4 341 / 353, 16384 x 32/4 1524 / 1565
 bool dq_ds_pairs(int64_t workgroups) { return workgroups <= compute_units_or_default(); }
 
-void launch_dq_from_ds(BwdParams p, bool causal, bool f32_out, hipStream_t st) {
+void launch_dq_from_ds(BwdParams p, int dqk, bool causal, bool f32_out, hipStream_t st) {
   p.ds_pairs = dq_ds_pairs((int64_t)p.q_tiles * p.Hq * p.B);
   const dim3 grid((unsigned)(p.q_tiles * p.Hq * p.B)), block(kThreads);
-  if (causal) {
-    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<true, float>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<true, __bf16>), grid, block, 0, st, p);
-  } else {
-    if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<false, float>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<false, __bf16>), grid, block, 0, st, p);
-  }
+  auto launch = [&](auto dqk) {
+    constexpr int D = decltype(dqk)::value;
+    if (causal) {
+      if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<D, true, float>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<D, true, __bf16>), grid, block, 0, st, p);
+    } else {
+      if (f32_out) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<D, false, float>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<D, false, __bf16>), grid, block, 0, st, p);
+    }
+  };
+  if (dqk == 192) launch(std::integral_constant<int, 192>{});
+  else launch(std::integral_constant<int, 128>{});
 }
 
 }  // namespace pith

@@ -488,6 +488,25 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
   return 4 * key_tiles * hkv * b * plan.dkdv_split >= 3 * cus;
 }
 
+// The same for (192, 128): its dQ kernel takes 256 rows per workgroup.
+// W = 256-row workgroups per compute unit, F as above; backward alone, inputs changing, handing over / recomputing, us (16 heads unless
+// others are named):
+//   causal  W 0.5         2048 110 / 86, 1024 x 32 65 / 52, 8192 x 4 371 / 289    W 0.75  3072 169 / 170, 12288 x 4 619 / 600, 3 x 1021 75 / 85
+//           W 1           4096 253 / 281, 2 x 2048 142 / 161, 4 x 1024 88 / 101, 8 x 512 65 / 71, 512 x 128 66 / 71, 16384 x 4 943 / 1007, 4096 x 16/4 269 / 298
+//           W 1.12-2.25   4608 325 / 376, 5120 392 / 450, 6144 533 / 604, 3 x 1999 210 / 230, 7168 692 / 769, 1024 x 128 178 / 193, 9216 1145 / 1277
+//   full    F below 0.75  2048 x 1024 84 / 73, 8192 x 4096 x 4 289 / 261, 2731 x 1366 129 / 143    W 0.25  1024 x 2048 88 / 86, 4096 x 8192 x 4 299 / 286
+//           W 0.5         2048 x 2048 124 / 135, 2 x 1024 x 2048 132 / 144, 8192 x 16384 x 4 917 / 959
+//           W 0.6-1.25    2560 x 5120 375 / 420, 3072 x 1536 141 / 153, 3072 x 6144 499 / 598, 2 x 2048 x 1024 120 / 138, 5120 x 2560 441 / 503
+// Below 512 rows the device still gains 4-7 % (16 x 300 77 / 81, 32 x 192 82 / 85), less than the time such a call spends in Python.
+bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
+  if (cus <= 0 || sq < 512 || (sq + 255) / 256 * hq * b * (causal ? 1 : 2) < cus) return false;
+  pith_attn_bwd_args a = {};
+  a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = 192; a.Dv = 128; a.causal = causal;
+  pith_attn_bwd_plan_t plan;
+  if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
+  return 4 * ((skv + 127) / 128) * hkv * b * plan.dkdv_split >= 3 * cus;
+}
+
 // Whether a share that could be one launch over all chunks goes out step by step instead, because steps hand dS over; `steps`:
 // (rows, keys, causal, kv heads of a slab that hands over at once, 0: recomputes). A step is a grid of its own for either kernel, and the last
 // round of each is lost, which one launch does not know; handing over saves a fifth of the time where the grids are whole rounds. L =
@@ -508,7 +527,7 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
 // four dQ workgroups per unit on, and where dQ, two workgroups to a unit, leaves its last round half empty, the steps are faster from a
 // quarter of the work on: two ranks, rank 0 4352 x 32/4 1058 / 1183, 20480 x 8/2 4975 / 5452, 2560 x 64/4 720 / 748, four ranks 1413 / 1555, 5120 x 32/4 2629 /
 // 3013, 2304 x 64/4 1231 / 1303, 2 x 2304 x 32 1253 / 1259; whole rounds 3072 x 64/4 1021 / 977, four ranks 2067 / 2031.
-bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const std::vector<std::array<int64_t, 4>>& steps, int64_t cus) {
+bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const std::vector<std::array<int64_t, 4>>& steps, int64_t cus, int64_t dqk) {
   if (cus <= 0 || hkv <= 0) return false;
   const auto lost = [&](int64_t wgs, int per_unit = 1) {
     const int64_t round = per_unit * cus;
@@ -522,11 +541,12 @@ bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const st
     handed += work;
     if (causal) continue;
     pith_attn_bwd_args a = {};
-    a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq / hkv * heads; a.Hkv = heads; a.Dqk = a.Dv = 128;
+    a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq / hkv * heads; a.Hkv = heads; a.Dqk = dqk; a.Dv = 128;
     pith_attn_bwd_plan_t plan;
     if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
     full += work;
-    full_lost += work * (0.7 * lost((skv + plan.dkdv_rows - 1) / plan.dkdv_rows * heads * b * plan.dkdv_split) + 0.3 * lost((sq + 511) / 512 * a.Hq * b));
+    const int64_t dq_rows = dqk == 192 ? 256 : 512;
+    full_lost += work * (0.7 * lost((skv + plan.dkdv_rows - 1) / plan.dkdv_rows * heads * b * plan.dkdv_split) + 0.3 * lost((sq + dq_rows - 1) / dq_rows * a.Hq * b));
   }
   if (handed == 0) return false;
   if (steps.size() == 1) return true;  // a call like any other
@@ -537,12 +557,20 @@ bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const st
   return rows >= 2048 && handed == all && (rows + 511) / 512 * hq * b >= 2 * cus && full_lost <= 1.05 * full;
 }
 
+// Whether any step of a share of (192, 128) could hand dS over, by its grids (steps: a chunk under the mask, whole, half its keys, half the rows).
+bool step_of_192_hands_over(const Tensor& q, int64_t hkv) {
+  const int64_t b = q.size(0), s = q.size(1), hq = q.size(2), cus = compute_units(q.device().index());
+  return ds_handover_pays_192(b, s, s, hq, hkv, true, cus) || ds_handover_pays_192(b, s, s, hq, hkv, false, cus) ||
+         ds_handover_pays_192(b, s, s / 2, hq, hkv, false, cus) || ds_handover_pays_192(b, s / 2, s, hq, hkv, false, cus);
+}
+
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
   // Calls large enough for the dS hand-over belong to the Python body, which owns the policy for the hand-over buffer: their
   // kernels outlast its host work many times over.
   bool small = q.is_cuda() && q.dim() == 4 && v.dim() == 4;
-  if (small && q.size(3) == 128 && k.dim() == 4) {
-    small = !ds_handover_pays(q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), causal, compute_units(q.device().index()));
+  if (small && (q.size(3) == 128 || q.size(3) == 192) && k.dim() == 4) {
+    const auto pays = q.size(3) == 128 ? ds_handover_pays : ds_handover_pays_192;
+    small = !pays(q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), causal, compute_units(q.device().index()));
   }
   if (small && q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) {
     Tensor delta = empty_like_shape(q, {q.size(0), q.size(2), q.size(1)}, at::kFloat);
@@ -919,7 +947,9 @@ struct RingFunction : torch::autograd::Function<RingFunction> {
     const Tensor &out = s[0], &lse = s[1], &q = s[2];
     const auto lists = chunk_lists(s, 3, cp, visited);
     std::optional<RingGrads> g;
-    if (q.size(3) != 128)  // whether steps of 128 features hand dS over is the Python body's decision
+    // Whether steps hand dS over is the Python body's decision where a step could.
+    const bool whole_keys = q.size(3) == 128 || (q.size(3) == 192 && !part_two(lists));
+    if (!whole_keys || (q.size(3) == 192 && !step_of_192_hands_over(q, lists[0][0]->size(2))))
       g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
     if (!g) g = python_body<RingGrads>("ring_backward_local", grads[0], q, out, lse, lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
     variable_list r = {std::get<0>(*g)};
@@ -1066,5 +1096,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("share_forward_in_one", &share_forward_in_one);
   m.def("share_backward_in_one", &share_backward_in_one);
   m.def("ds_handover_pays", &ds_handover_pays);
-  m.def("share_hands_over", &share_hands_over);
+  m.def("ds_handover_pays_192", &ds_handover_pays_192);
+  m.def("share_hands_over", &share_hands_over, py::arg("b"), py::arg("rows"), py::arg("hq"), py::arg("hkv"), py::arg("steps"), py::arg("cus"),
+        py::arg("dqk") = 128);
 }

@@ -197,7 +197,7 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
     args.ds, args.ds_bytes = ds.data_ptr(), ds.numel()
 
 
-# The dS hand-over (head dims 128/128) makes the backward of a chunk pair 1-5 % faster (share of 8192 rows, 32/4 heads,
+# The dS hand-over (head dims 128/128 and 192/128) makes the backward of a chunk pair 1-5 % faster (share of 8192 rows, 32/4 heads,
 # four ranks: 6.15 -> 5.92 ms; the gain differs between machines) at the price of a transient buffer of
 # Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask: a layer of 4096 rows, 32/4 heads,
 # takes 0.55 GB for 3 % of its forward + backward).
@@ -235,10 +235,11 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
     """How the backward of one chunk pair uses the dS hand-over: (kv heads per slab, bytes of the buffer),
     or None when both kernels should recompute (no hand-over path for these head dims, one of the kernels
     would not fill the device with work, or not even one kv head fits the budget)."""
-    b, sq, hq, _ = q.shape
+    b, sq, hq, d_q = q.shape
     skv, hkv = k.shape[1:3]
+    pays = native.ds_handover_pays_192 if d_q == 192 else native.ds_handover_pays
     units = _device_compute_units(q.device)
-    if not native.ds_handover_pays(b, sq, skv, hq, hkv, causal, units):  # nor for any slab
+    if not pays(b, sq, skv, hq, hkv, causal, units):  # nor for any slab
         return None
     need = attn_bwd_ds_bytes(q, k, v, causal)
     if need == 0:
@@ -252,7 +253,7 @@ def ds_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
             heads -= 1
     if per_kv_head * heads > budget:
         return None
-    if heads < hkv and not native.ds_handover_pays(b, sq, skv, hq // hkv * heads, heads, causal, units):
+    if heads < hkv and not pays(b, sq, skv, hq // hkv * heads, heads, causal, units):
         return None
     return heads, per_kv_head * heads
 

@@ -319,7 +319,7 @@ class RingBackward:
         ls, dl = _lse_rows(self.lse, st.q_rows), _lse_rows(self.delta, st.q_rows)
         pes = _pe_rows(k_pe_j, st.kv_rows)
         # dK/dV, then dQ; the pair helper decides whether the dK/dV kernel leaves its dS tiles for the dQ
-        # kernel (head dims 128/128, bounded scratch) or both kernels recompute the scores.
+        # kernel (bounded scratch) or both kernels recompute the scores.
         # Step 0 covers every row and initialises the dQ accumulator; later steps add to their rows.
         covered = [r for r in self.dq_ranges if st.q_rows[0] <= r[0] and r[1] <= st.q_rows[1]]
         for r in covered:
@@ -358,13 +358,13 @@ class RingBackward:
 def _steps_beat_one_launch(q: torch.Tensor, hkv: int, steps: Sequence[Tuple[int, int, bool, int]]) -> bool:
     """steps: (rows, keys, causal, kv heads of a slab that hands dS over at once or 0). Both sides are measured beside the rule."""
     b, s, hq, _ = q.shape
-    return native.share_hands_over(b, s, hq, hkv, steps, hip._device_compute_units(q.device))
+    return native.share_hands_over(b, s, hq, hkv, steps, hip._device_compute_units(q.device), q.shape[-1])
 
 
 def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunks) -> bool:
     """Whether enough steps of the share hand dS from their dK/dV to their dQ kernel (5 matrix products instead of 7) to be worth
     more than one launch over all chunks saves."""
-    if q.shape[-1] != 128:
+    if q.shape[-1] not in (128, 192) or k_chunks[steps[0].kv_rank].shape[-1] != q.shape[-1]:  # (nor keys in two parts)
         return False
     plans = [hip.ds_plan(_rows(q, st.q_rows), _rows(k_chunks[st.kv_rank], st.kv_rows), _rows(v_chunks[st.kv_rank], st.kv_rows), st.causal) for st in steps]
     if not any(plans):

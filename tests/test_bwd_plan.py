@@ -110,6 +110,17 @@ def test_rows_that_fill_their_workgroups(pays, b, s, hq, hkv):
     assert [native.ds_handover_pays(b, s, s, hq, hkv, c, UNITS) for c in (True, False)] == {"no": [False] * 2, "yes": [True] * 2, "causal": [True, False]}[pays]
 
 
+@pytest.mark.parametrize("causal,b,sq,skv,h,pays", [
+    (True, 1, 4096, 4096, 16, True), (True, 4, 1024, 1024, 16, True), (True, 1, 4608, 4608, 16, True), (True, 1, 16384, 16384, 4, True),
+    (True, 1, 3072, 3072, 16, False), (True, 1, 2048, 2048, 16, False), (True, 1, 12288, 12288, 4, False), (True, 16, 256, 256, 16, False),
+    (False, 1, 4096, 2048, 16, True), (False, 1, 2048, 4096, 16, True), (False, 1, 2048, 1024, 16, False), (False, 1, 1024, 2048, 16, False),
+    (False, 1, 8192, 4096, 4, False), (False, 1, 4096, 8192, 4, False),
+])  # fmt: skip
+def test_calls_of_192_that_hand_over(causal, b, sq, skv, h, pays):
+    """As measured (table at ds_handover_pays_192)."""
+    assert native.ds_handover_pays_192(b, sq, skv, h, h, causal, UNITS) == pays and not native.ds_handover_pays_192(b, sq, skv, h, h, causal, 0)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_slabs_are_asked_for_by_the_rule_of_whole_calls(monkeypatch, causal):
     """A budget for one of two halves of the kv heads: the grid of a slab has to pass the same rule as that of the whole pair."""

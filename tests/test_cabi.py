@@ -382,6 +382,18 @@ def test_ds_storing_dkdv_kernel_waits_for_its_tile_loads_only(tmp_path_factory):
         assert not in_loop_blocks, f"stores or spills in out-of-line blocks of the loop: {in_loop_blocks}"
 
 
+def test_ds_storing_dkdv_kernel_of_192_waits_for_its_tile_loads_only(tmp_path_factory):
+    """The same of (192, 128), straight-line from the interval's requests to its wait."""
+    lines = _kernel_asm("attn_bwd_dkdv_d192.hip", tmp_path_factory.getbasetemp()).splitlines()
+    assert not [l for l in lines if re.match(r"\s+scratch_", l)], "registers are spilled"
+    waits = [i for i, l in enumerate(lines) if re.search(r"s_waitcnt vmcnt\(4\)\s*$", l) and "s_barrier" in lines[i + 1]]
+    assert len(waits) == 4, "one steady-state wait per storing instance"
+    for w in waits:
+        ops = [l.split()[0] for l in lines[max(i for i in range(w) if "Inner Loop Header" in lines[i]) : w] if re.match(r"\s+(global_|buffer_|flat_)", l)]
+        assert ops[-4:] == ["global_store_dwordx4"] * 4 and ops[-5].startswith("global_load_lds"), ops[-6:]
+        assert sum(o.startswith("global_store") for o in ops) == 4
+
+
 def test_split_key_dq_requests_no_tile_over_one_still_read(tmp_path_factory):
     """The split-key dQ kernel scores tile 0 ahead of its loop and then requests tiles into slots that other waves read for
     that (V of tile 2 at 192 features, the staged rows at 128). Followed over the control flow of the compiler's output: between

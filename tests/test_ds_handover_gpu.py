@@ -1,4 +1,4 @@
-"""dS hand-over between the two backward kernels of one chunk pair (head dims 128/128): with a `ds`
+"""dS hand-over between the two backward kernels of one chunk pair (head dims 128/128 and 192/128): with a `ds`
 buffer the dK/dV kernel stores the dS tiles it forms and the dQ kernel computes dQ = scale * dS K from
 them instead of recomputing S and dP (pithtrain/operators/mla/triton.py:205-266 recomputes). Expected
 values come from the fp64 oracle; the recomputing dQ kernel is compared as well (the same bf16 dS values
@@ -83,6 +83,40 @@ def test_causal_dq_from_ds(gpu, shape):
     _run(gpu, True, shape, torch.bfloat16)
 
 
+SHAPES_192 = [(1, 129, 129, 4, 1), (1, 256, 256, 4, 4), (1, 257, 257, 2, 1), (2, 333, 333, 4, 2), (2, 777, 777, 8, 2), (1, 1025, 1025, 2, 2),
+              (1, 2048, 2048, 4, 4), (17, 255, 255, 16, 16)]  # fmt: skip
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("causal,shape", [(True, s) for s in SHAPES_192] + [(False, s) for s in [*SHAPES_192[:4], (1, 512, 256, 8, 2), (1, 200, 450, 4, 2), (1, 257, 129, 2, 2)]])
+def test_dq_from_ds_192(gpu, causal, shape, dtype):
+    """(192, 128): 256 rows per dQ workgroup, two waves to 64 of them with half of the features each (the last quarter from the tile of
+    trailing features); pairs of 128-row blocks under the mask, consecutive rows where the grid exceeds a round."""
+    _run(gpu, causal, shape, dtype, dqk=192)
+
+
+@pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
+def test_ring_share_of_192_with_and_without_handover(gpu, layout, monkeypatch):
+    """Steps that hand dS over (fp32 dQ added to and finished by their kernels) against one launch that recomputes: the same bf16 dS
+    values summed in other orders, up to one bf16 step (2^-8) of the largest element."""
+    from pithtrain_amd.operators.mla import hip as H
+    from pithtrain_amd.operators.ring_attention import local as L
+
+    g = torch.Generator(device=gpu).manual_seed(5)
+    t = lambda h, d: torch.randn(1, 2050, h, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, dout, ks, vs = t(16, 192), t(16, 128), [t(16, 192) for _ in range(3)], [t(16, 128) for _ in range(3)]
+    ks, vs = (ks, vs) if layout == "zigzag" else ([*ks[:2], None], [*vs[:2], None])
+    out, lse = L.ring_forward_local(q, ks, vs, 0.07, 1, 3, layout)
+    monkeypatch.setattr(L, "_handover_pays", lambda *a: True)
+    monkeypatch.setattr(H, "ds_plan", lambda q, k, v, causal=False: (16, attn_bwd_ds_bytes(q, k, v, causal)))
+    steps = L.ring_backward_local(dout, q, out, lse, ks, vs, 0.07, 1, 3, layout)
+    monkeypatch.setattr(L, "_handover_pays", lambda *a: False)
+    one = L.ring_backward_local(dout, q, out, lse, ks, vs, 0.07, 1, 3, layout)
+    flat = lambda r: [r[0], *(x for l in r[1:3] for x in l if x is not None)]  # noqa: E731
+    for a, b in zip(flat(steps), flat(one), strict=True):
+        assert norm_max_err(a.float(), b.float()) < 6e-3
+
+
 @pytest.mark.parametrize("S", [255, 257, 511, 513, 767, 769, 1025, 1281, 1537])
 def test_causal_pairs_of_row_blocks(gpu, S):
     """Under the mask a workgroup takes 256-row blocks in pairs, one from either end: odd and even numbers of blocks, the last
@@ -141,7 +175,7 @@ def test_small_buffer_falls_back_to_recomputation(gpu):
     small = torch.zeros(attn_bwd_ds_bytes(qd, kd, vd, True) - 1024, dtype=torch.uint8, device=gpu)
     attn_bwd_dq_into(qd, kd, vd, dod, lse, delta, dq1, scale, True, ds=small)
     assert torch.equal(dq0, dq1)
-    # head dims without a hand-over path report 0 bytes and get no buffer
+    # head dims without a hand-over path, and rows that leave half of the 192-feature workgroups empty, report 0 bytes and get no buffer
     for d in (64, 192):
         qx = torch.empty(1, 128, 4, d, dtype=torch.bfloat16, device=gpu)
         vx = torch.empty(1, 128, 4, min(d, 128), dtype=torch.bfloat16, device=gpu)
