@@ -276,9 +276,11 @@ int pith_attn_bwd(const pith_attn_bwd_args* args, pith_stream_t stream);
 
 /* The same against several chunks at once (pith_key_chunk, conventions of pith_attn_fwd_chunks): dq is written once, over
  * all chunks, and dk, dv (dk_pe) of every chunk. args describes the query side and what the chunks share; its k, v, k_pe,
- * Skv, causal, dk, dv, dk_pe, dkv_zero_tail and ds are ignored. Gradients are bf16, nothing is accumulated. The workspace is
- * required wherever pith_attn_bwd_chunks_workspace_bytes is not 0. */
+ * Skv, causal, dk, dv, dk_pe and dkv_zero_tail are ignored. Gradients are bf16, nothing is accumulated. The workspace is
+ * required wherever pith_attn_bwd_chunks_workspace_bytes is not 0. With a `ds` buffer of at least pith_attn_bwd_chunks_ds_bytes (0:
+ * no hand-over path; head dims (192,128), keys in one part or two, every q_row0 a multiple of 64) dS is handed over as described below. */
 int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n);
+int64_t pith_attn_bwd_chunks_ds_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n);
 int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream);
 
 /* Scratch size with which pith_attn_bwd_dkdv runs fastest for these shapes (0 = none needed).

@@ -25,19 +25,19 @@ constexpr int kDkdvSmem = DQK == 64 ? dkdv_d64::kSmem : DQK == 128 ? dkdv_d128::
 template <int DQK>
 constexpr int kDkdvThreads = DQK == 64 ? dkdv_d64::kThreads : 512;
 
-template <int DQK>
+template <int DQK, bool EMIT_DS = false>
 __device__ __forceinline__ void dkdv_body(const BwdChunkParams& p, char* smem, int block) {
   int key_shift;
   const BwdParams r = dkdv_chunk_params<DQK, DQK == 64 ? 64 : 128>(p, block, key_shift);
   if constexpr (DQK == 64) dkdv_d64::body<true, __bf16>(r, smem, block, key_shift);
   else if constexpr (DQK == 128) dkdv_d128::body<true, __bf16, false>(r, smem, block, key_shift);
-  else dkdv_d192::body<true, __bf16>(r, smem, block, key_shift);
+  else dkdv_d192::body<true, __bf16, EMIT_DS>(r, smem, block, key_shift);
 }
 
-template <int DQK>
+template <int DQK, bool EMIT_DS = false>
 __global__ __launch_bounds__(kDkdvThreads<DQK>, 2) void attn_bwd_dkdv_chunks_kernel(BwdChunkParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[kDkdvSmem<DQK>];
-  dkdv_body<DQK>(p, smem, blockIdx.x);
+  dkdv_body<DQK, EMIT_DS>(p, smem, blockIdx.x);
 }
 
 template <int DQK>
@@ -75,6 +75,11 @@ void launch_dim(const BwdChunkParams& p, bool one_grid, bool dq_first, unsigned 
 }  // namespace
 
 void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, unsigned dkdv_blocks, hipStream_t st) {
+  if (p.ds != nullptr) {
+    hipLaunchKernelGGL((attn_bwd_dkdv_chunks_kernel<192, true>), dim3(dkdv_blocks), dim3(kDkdvThreads<192>), 0, st, p);
+    launch_dq_from_ds_chunks(p, st);
+    return;
+  }
   if (dqk == 64) launch_dim<64>(p, one_grid, dq_first, dkdv_blocks, st);
   else if (dqk == 128) launch_dim<128>(p, one_grid, dq_first, dkdv_blocks, st);
   else launch_dim<192>(p, one_grid, dq_first, dkdv_blocks, st);

@@ -67,6 +67,8 @@ struct BwdChunk {
   int tiles, zero_tail;   // as in BwdParams
   int first_block;        // of the dK/dV grid
   int rows_before;        // keys of the chunks in front: where the chunk's part of the workspaces lies
+  int64_t ds_off, ds_hs;  // dS hand-over: the chunk's images within p.ds, bytes per (batch, query head), 128-key blocks; its query
+  int ds_kb;              // tiles count from q_row0
 };
 struct BwdChunkParams : BwdParams {
   int n_chunks;
@@ -106,6 +108,7 @@ __device__ __forceinline__ BwdParams dkdv_chunk_params(const BwdChunkParams& p, 
   r.ws_dk += row_parts * p.split * DQK;
   r.ws_dv += row_parts * p.split * DV;
   r.ws_dkpe += row_parts * 64;
+  r.ds += ch.ds_off; r.ds_hs = ch.ds_hs; r.ds_kb = ch.ds_kb;
   return r;
 }
 
@@ -260,6 +263,7 @@ bool launch_bwd_pair(const BwdParams& p, int dqk, bool causal, bool dkdv_f32, bo
 
 // The backward of a chunk call: attn_bwd_chunks.hip. dkdv_blocks = the dK/dV grid; p.q_tiles = 128-row query tiles; dq_first:
 // one grid starts with dQ. dQ workgroups: the split-key ones in one grid (128 and 192 features), the two-per-unit ones alone.
+// With p.ds (192 features) two launches, dS handed over; p.q_tiles = tiles of dq_ds_rows.
 void launch_bwd_chunks(const BwdChunkParams& p, int dqk, bool one_grid, bool dq_first, unsigned dkdv_blocks, hipStream_t stream);
 
 // dQ for head dims (128, 128) and (192, 128) with one 8-wave workgroup of 128 query rows per compute unit whose wave pairs
@@ -275,6 +279,7 @@ constexpr int dq_ds_rows(int dqk) { return dqk == 192 ? 256 : 512; }
 // Whether under the mask a grid of that many workgroups takes blocks of half a tile from both ends of the rows.
 bool dq_ds_pairs(int64_t workgroups);
 void launch_dq_from_ds(BwdParams p, int dqk, bool causal, bool f32_out, hipStream_t stream);
+void launch_dq_from_ds_chunks(BwdChunkParams p, hipStream_t stream);  // (192, 128)
 // Bytes of dS images for a shape (0: the shape has no hand-over path), and whether the call brings a buffer for them.
 int64_t ds_bytes_for(const pith_attn_bwd_args* a);
 bool ds_usable(const pith_attn_bwd_args* a);

@@ -392,6 +392,12 @@ bool merged_call(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, i
   return a->B > 0 && a->Hkv > 0 && a->Hq > 0 && a->Hq % a->Hkv == 0;
 }
 
+// Bytes of a chunk's dS images per (batch, query head).
+int64_t chunk_ds_head_bytes(int64_t sq, const pith_key_chunk& c, bool diagonal) {
+  const int qt = (int)((sq - c.q_row0 + 63) / 64), kb = (int)((c.rows + kBN - 1) / kBN);
+  return (diagonal ? ds_tile_start<true>(qt, kb) : ds_tile_start<false>(qt, kb)) * kDsBlockBytes;
+}
+
 int pick_chunks_split(pith_attn_bwd_args a, int64_t tiles) {
   a.causal = 1;  // the chunks' workgroups are unequal in any case
   return pick_split(&a, tiles);
@@ -441,6 +447,17 @@ extern "C" int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args
   return workspace_bytes_for(&a, pick_chunks_split(a, tiles));
 }
 
+extern "C" int64_t pith_attn_bwd_chunks_ds_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n) {
+  pith_attn_bwd_args a;
+  int64_t tiles, bytes = 0;
+  if (n < 2 || !merged_call(args, chunks, n, &a, &tiles) || a.Dqk != 192 || a.Dv != 128 || a.Sq <= dq_ds_rows(192) / 2) return 0;
+  for (int64_t i = 0; i < n; ++i) {
+    if (chunks[i].q_row0 % 64) return 0;  // a 64-row tile that sees the chunk in part would lie across two of its images
+    bytes += a.B * a.Hq * chunk_ds_head_bytes(a.Sq, chunks[i], i == n - 1);
+  }
+  return bytes;
+}
+
 extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
   const char* who = "pith_attn_bwd_chunks";
   if (!args || !chunks) return fail(PITH_ERR_NULL_POINTER, "%s: args or chunks is NULL", who);
@@ -461,9 +478,12 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   const int64_t need = workspace_bytes_for(&all, split);
   if (need > 0 && (!args->workspace || args->workspace_bytes < need || !aligned16(args->workspace)))
     return fail(PITH_ERR_BAD_SHAPE, "%s: a 16-byte aligned workspace of %lld bytes is needed", who, (long long)need);
+  const int64_t ds_need = pith_attn_bwd_chunks_ds_bytes(args, chunks, n);
+  const bool hand_over = args->ds && ds_need > 0 && args->ds_bytes >= ds_need;
+  if (hand_over && (uintptr_t)args->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
   BwdChunkParams p;
   unsigned blocks = 0;
-  int64_t rows_before = 0;
+  int64_t rows_before = 0, ds_off = 0;
   for (int64_t i = 0; i < n; ++i) {
     const pith_key_chunk& c = chunks[i];
     const bool diagonal = i == n - 1;
@@ -483,6 +503,10 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
     ch.zero_tail = (int)c.zero_tail;
     ch.first_block = (int)blocks;
     ch.rows_before = (int)rows_before;
+    ch.ds_off = ds_off;
+    ch.ds_hs = chunk_ds_head_bytes(a.Sq, c, diagonal);
+    ch.ds_kb = ch.tiles;
+    ds_off += a.B * a.Hq * ch.ds_hs;
     const int64_t next = blocks + (int64_t)ch.tiles * a.Hkv * a.B * split + (c.zero_tail + kZeroTailRows - 1) / kZeroTailRows;
     rows_before += c.rows;
     if (next > 0x3fffffff || rows_before > 0x3fffffff) return fail(PITH_ERR_UNSUPPORTED, "%s: the chunks exceed the launch grid limit", who);
@@ -491,7 +515,9 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   p.n_chunks = (int)n;
   p.dk_pe_bs = args->dk_pe_bs;
   p.split = split;
-  p.q_tiles = (p.Sq + 127) / 128;
+  const int dq_rows = hand_over ? dq_ds_rows(192) : 128;
+  p.q_tiles = (p.Sq + dq_rows - 1) / dq_rows;
+  if (hand_over) p.ds = reinterpret_cast<char*>(args->ds);
   p.ws_dk = reinterpret_cast<float*>(need > 0 ? args->workspace : nullptr);
   p.ws_dv = p.ws_dk + (split > 1 ? (int64_t)split * all.B * all.Skv * all.Hkv * all.Dqk : 0);
   p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));

@@ -347,7 +347,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
                                       x[rb][8 * jj + 4], x[rb][8 * jj + 5], x[rb][8 * jj + 6], x[rb][8 * jj + 7]);
     }
     if constexpr (EMIT_DS) {
-      char* img = ds_wg + (int64_t)(b * p.Hq + tile.hq) * p.ds_hs + ds_tile_start<CAUSAL>(tile.mt, p.ds_kb) * kDsBlockBytes;
+      char* img = ds_wg + (int64_t)(b * p.Hq + tile.hq) * p.ds_hs + (CAUSAL && key_shift == 0 ? ds_tile_start<true>(tile.mt, p.ds_kb) : ds_tile_start<false>(tile.mt, p.ds_kb)) * kDsBlockBytes;
       int off = (g << 9) + ((c ^ (g << 3)) << 4);  // recomputed per tile: no register is held across the interval
       asm volatile("" : "+v"(off));
 #pragma unroll

@@ -64,8 +64,9 @@ __device__ __forceinline__ void wait_vector_loads_but(int n) {
   }
 }
 
-template <int DQK, bool CAUSAL, typename OutT>
-__global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
+// MULTI: over several chunks, whose steps are one stream; dQ is written once.
+template <int DQK, bool CAUSAL, typename OutT, bool MULTI = false>
+__global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdArgs<MULTI> p) {
   constexpr int FS = DQK == 192 ? 2 : 1;    // waves that share 64 query rows, a part of the features each
   constexpr int RG = 8 / FS;                // 64-row groups of a workgroup
   constexpr int DB = DQK / 32 / FS;         // feature blocks per wave
@@ -104,7 +105,9 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   const int m_end = pairs ? (half_blocks - m_tile) * (kBM / 2) : (m_tile + 1) * kBM;  // behind the workgroup's last row
   const int q_wave0 = rows_of(rg);
 
-  const int kv_row_bytes = p.HkvT * DQK * 2;
+  const bool two_part = MULTI && p.k_pe != nullptr;  // keys in two parts
+  const int k_head = two_part ? 128 : DQK;
+  const int kv_row_bytes = p.HkvT * k_head * 2, extra_row_bytes = two_part ? (int)p.k_pe_rs * 2 : kv_row_bytes;
   const char* kh = reinterpret_cast<const char*>(p.k + b * p.k_bs + (int64_t)hk * DQK);
 
   // key steps: all of them, or up to the diagonal; a wave whose query tile does not exist (ragged
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
   DirectTile128<kBN, 256> mover;
   mover.init(kv_row_bytes, wave & 3, lane);
   dkdv_d192::DirectExtra<kBN / 2> extra;  // features 128..191
-  if constexpr (DQK == 192) extra.init(kv_row_bytes, wave & 3, lane);
+  if constexpr (DQK == 192) extra.init(extra_row_bytes, wave & 3, lane);
   const char* ds_src[kImages];  // only used by waves 4..7
   int ds_steps[kImages];
 #pragma unroll
@@ -256,31 +259,119 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdParams p) {
     }
   };
 
-  if (k_mover) {
+  if constexpr (MULTI) {
+    static_assert(!MULTI || (CAUSAL && kImages == 1 && DQK == 192), "one image per mover and step");
+    // Every wave walks the same steps: chunk by chunk those that any row of the workgroup sees, in the last chunk up to the diagonal.
+    const int last = chunk_count(p) - 1;
+    auto chunk_steps = [&](int i) __attribute__((always_inline)) {
+      const KeyChunk& ch = chunk_of(p, i);
+      const int all = (ch.rows + kBN - 1) / kBN;
+      return i == last ? min(all, (m_end - 1) / kBN + 1) : ch.q_row0 < m_end ? all : 0;
+    };
+    auto group_steps = [&](int i, int q0) __attribute__((always_inline)) {
+      const KeyChunk& ch = chunk_of(p, i);
+      const int all = (ch.rows + kBN - 1) / kBN;
+      if ((q0 >> 6) >= p.ds_qt) return 0;
+      return i == last ? min(all, (q0 + QW - 1) / kBN + 1) : q0 >= ch.q_row0 ? all : 0;
+    };
+    // The mover's place in the stream, ahead of the products, and what it needs of that chunk.
+    int req_i = -1, req_s = 0, req_n = 0, keys_left = 0, image_steps = 0;
+    const char *k_src = nullptr, *extra_src = nullptr, *image = nullptr;
+    const int q_image0 = rows_of(wave & 3);
+    auto next_chunk = [&]() __attribute__((always_inline)) {
+      do ++req_i;
+      while (req_i <= last && chunk_steps(req_i) == 0);
+      if (req_i > last) return;
+      req_s = 0;
+      req_n = chunk_steps(req_i);
+      const KeyChunk& ch = chunk_of(p, req_i);
+      keys_left = ch.rows;
+      k_src = reinterpret_cast<const char*>(ch.k + b * p.k_bs + (int64_t)hk * k_head);
+      extra_src = two_part ? reinterpret_cast<const char*>(ch.k_pe + b * p.k_pe_bs) - 256 : k_src;  // (the mover adds the first part's 256 bytes)
+      image_steps = k_mover ? 0 : group_steps(req_i, q_image0);
+      if (image_steps > 0) {
+        const BwdChunk& c = p.chunk[req_i];
+        const int64_t tile = req_i == last ? ds_tile_start<true>(q_image0 >> 6, c.ds_kb) : ds_tile_start<false>((q_image0 - ch.q_row0) >> 6, c.ds_kb);
+        image = p.ds + c.ds_off + (int64_t)(b * p.Hq + h) * c.ds_hs + tile * kDsBlockBytes;
+      }
+    };
+    unsigned issued = 0;  // bit j: loads were issued for the step j before the last one requested
+    auto request_next = [&](int slot) __attribute__((always_inline)) {
+      issued <<= 1;
+      if (req_i > last) return;
+      if (k_mover) {
+        char* const stage = smem + slot * kKStage;
+        mover.issue(k_src, keys_left, stage, wave & 3, lane);
+        extra.issue(extra_src, keys_left, stage + kBN * kRowBytes128, wave & 3, lane);
+        k_src += (int64_t)kBN * kv_row_bytes;
+        extra_src += (int64_t)kBN * extra_row_bytes;
+        keys_left -= kBN;
+        issued |= 1;
+      } else if (req_s < image_steps) {
+        int off = lane << 4;
+        asm volatile("" : "+v"(off));
+        char* const dst = smem + kOffDs + slot * kDsStage + (wave - 4) * kDsWave;
 #pragma unroll
-    for (int d = 0; d < kRingK - 1; ++d)
-      if (d < n_steps_wg) request_k(d, d);
-  } else {
-#pragma unroll
-    for (int d = 0; d < kRingD - 1; ++d)
-      if (d < n_steps_wg) request_ds(d, d);
-  }
-  auto step = [&](int s, auto compute_tag) __attribute__((always_inline)) {
-    wait_step(s);
-    __syncthreads();  // every wave's requests for step s have landed; everyone is done with step s-1
+        for (int j = 0; j < kLoadsDs; ++j) load_lds16_once(image + j * 1024, off, dst + j * 1024);
+        image += 4096;
+        issued |= 1;
+      }
+      if (++req_s == req_n) next_chunk();
+    };
+    next_chunk();
     if (k_mover) {
-      if (s + kRingK - 1 < n_steps_wg) request_k(s + kRingK - 1, k_next);
+      for (int d = 0; d < kRingK - 1; ++d) request_next(d);
     } else {
-      if (s + kRingD - 1 < n_steps_wg) request_ds(s + kRingD - 1, d_next);
+      for (int d = 0; d < kRingD - 1; ++d) request_next(d);
     }
-    if constexpr (decltype(compute_tag)::value)
-      compute(smem + k_slot * kKStage, smem + kOffDs + d_slot * kDsStage + rg * kDsWave);
-    advance();
-  };
-  int s = 0;
-  for (; s < n_steps_wave; ++s) step(s, std::true_type{});
-  // other waves of the workgroup may still have steps to visit: keep moving tiles, keep in step
-  for (; s < n_steps_wg; ++s) step(s, std::false_type{});
+    auto step = [&](auto compute_tag) __attribute__((always_inline)) {
+      if (k_mover) {
+        if (issued & 1) wait_vector_loads_but<kLoadsK>();
+        else wait_vector_loads_but<0>();
+      } else {
+        constexpr unsigned kLater = (1u << (kRingD - 2)) - 1;  // the steps requested after this one
+        if ((issued & kLater) == kLater) wait_vector_loads_but<kSteadyDs>();
+        else wait_vector_loads_but<0, 31>(kLoadsDs * __builtin_popcount(issued & kLater));
+      }
+      __syncthreads();  // every wave's requests for this step have landed; everyone is done with the one before
+      request_next(k_mover ? k_next : d_next);
+      if constexpr (decltype(compute_tag)::value)
+        compute(smem + k_slot * kKStage, smem + kOffDs + d_slot * kDsStage + rg * kDsWave);
+      advance();
+    };
+    for (int i = 0; i <= last; ++i) {
+      const int n_wg = chunk_steps(i), n_own = group_steps(i, q_wave0);
+      int s = 0;
+      for (; s < n_own; ++s) step(std::true_type{});
+      for (; s < n_wg; ++s) step(std::false_type{});
+    }
+  } else {
+    if (k_mover) {
+#pragma unroll
+      for (int d = 0; d < kRingK - 1; ++d)
+        if (d < n_steps_wg) request_k(d, d);
+    } else {
+#pragma unroll
+      for (int d = 0; d < kRingD - 1; ++d)
+        if (d < n_steps_wg) request_ds(d, d);
+    }
+    auto step = [&](int s, auto compute_tag) __attribute__((always_inline)) {
+      wait_step(s);
+      __syncthreads();  // every wave's requests for step s have landed; everyone is done with step s-1
+      if (k_mover) {
+        if (s + kRingK - 1 < n_steps_wg) request_k(s + kRingK - 1, k_next);
+      } else {
+        if (s + kRingD - 1 < n_steps_wg) request_ds(s + kRingD - 1, d_next);
+      }
+      if constexpr (decltype(compute_tag)::value)
+        compute(smem + k_slot * kKStage, smem + kOffDs + d_slot * kDsStage + rg * kDsWave);
+      advance();
+    };
+    int s = 0;
+    for (; s < n_steps_wave; ++s) step(s, std::true_type{});
+    // other waves of the workgroup may still have steps to visit: keep moving tiles, keep in step
+    for (; s < n_steps_wg; ++s) step(s, std::false_type{});
+  }
 
   OutT* dqh = reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + (int64_t)h * DQK + fh * (32 * DB);
   const float sc = -p.scale;  // the images hold -dS (the writer forms delta - dP)
@@ -323,6 +414,12 @@ void launch_dq_from_ds(BwdParams p, int dqk, bool causal, bool f32_out, hipStrea
   };
   if (dqk == 192) launch(std::integral_constant<int, 192>{});
   else launch(std::integral_constant<int, 128>{});
+}
+
+void launch_dq_from_ds_chunks(BwdChunkParams p, hipStream_t st) {
+  const unsigned workgroups = (unsigned)(p.q_tiles * p.Hq * p.B);
+  p.ds_pairs = dq_ds_pairs(workgroups);
+  hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<192, true, __bf16, true>), dim3(workgroups), dim3(kThreads), 0, st, p);
 }
 
 }  // namespace pith

@@ -387,12 +387,30 @@ bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chu
   return rows < 8192 || keys < chunks * rows || wgs % (2 * cus) != 0;
 }
 
+// Bytes of the buffer through which a share's one dK/dV launch hands dS to its one dQ launch, 0 where it recomputes.
+// Against one grid of both kinds (two recomputing launches from W 1 on) that loses the last round of either launch and wins two products
+// of seven. W = its 256-row dQ workgroups per compute unit; backward, handing over / recomputing, us, four ranks unless named, zigzag rank 1
+// and contiguous rank 1:
+//   W 0.25  1024 x 16 130 / 88 and 146 / 106               W 0.5   2048 x 16 323 / 288 and 232 / 217, 8192 x 4 1177 / 1061 and 826 / 791, 4 x 512 x 16 119 / 102
+//   W 0.75  3072 x 16 569 / 638 and 683 / 775, 12032 x 4 2080 / 2312 and 2499 / 2886, 2 x 1536 x 16 315 / 344 and 358 / 412
+//   W 1     4096 x 16 974 / 1070 and 684 / 798, 8 ranks 1856 / 2064 and 2427 / 2794, 2 x 2048 x 16 532 / 573 and 373 / 429, 4 x 1024 x 16 324 / 342 and
+//           218 / 248, 16384 x 4 3734 / 4036 and 2636 / 3024    W 1.25-2   5120 x 16, 2 ranks 737 / 839, 6144 x 16 2034 / 2325, 8192 x 16, 2 ranks 1771 / 2027
+// Keys in two parts the same: 4096 x 16 986 / 1072, 4 x 1024 x 16 331 / 348.
+bool share_of_192_pays(int64_t b, int64_t rows, int64_t hq, int64_t cus) { return cus > 0 && rows >= 512 && 10 * ((rows + 255) / 256 * hq * b) >= 7 * cus; }
+int64_t share_ds_bytes(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes,
+                       int64_t rank, int64_t cp, bool zigzag) {
+  if (!q.is_cuda() || q.dim() != 4 || q.size(3) != 192 || !share_of_192_pays(q.size(0), q.size(1), q.size(2), compute_units(q.device().index()))) return 0;
+  pith_attn_bwd_args a = {};
+  RingChunks r;
+  return ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r) ? pith_attn_bwd_chunks_ds_bytes(&a, r.chunk.data(), (int64_t)r.chunk.size()) : 0;
+}
+
 // (dq, dk list, dv list, dk_pe list or empty); the lists hold a tensor per visited chunk. None as above. The policy for the
-// dS hand-over is the caller's: this call recomputes.
+// dS hand-over is the caller's: without its buffer of share_ds_bytes this call recomputes.
 using RingGrads = std::tuple<Tensor, std::vector<OptTensor>, std::vector<OptTensor>, std::vector<OptTensor>>;
 std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, const Tensor& out, const Tensor& lse, const std::vector<OptTensor>& ks,
                                        const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes, double scale, int64_t rank,
-                                       int64_t cp, bool zigzag) {
+                                       int64_t cp, bool zigzag, const OptTensor& ds) {
   pith_attn_bwd_args a = {};
   RingChunks r;
   if (!ring_chunks(q, ks, vs, pes, rank, cp, zigzag, a, r)) return std::nullopt;
@@ -412,6 +430,11 @@ std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, c
   a.dk_pe_bs = a.Sq * 64;
   a.dq_dtype = a.dkv_dtype = PITH_BF16;
   a.scale = (float)scale;
+  if (ds) {
+    if (!ds->is_cuda() || ds->device() != q.device() || ds->scalar_type() != at::kByte || !ds->is_contiguous() || (uintptr_t)ds->data_ptr() % 256) return std::nullopt;
+    a.ds = ds->data_ptr();
+    a.ds_bytes = ds->numel();
+  }
   RingGrads g = {dq, std::vector<OptTensor>(cp), std::vector<OptTensor>(cp), std::vector<OptTensor>(pes ? cp : 0)};
   for (size_t i = 0; i < r.chunk.size(); ++i) {
     const int64_t j = r.rank[i];
@@ -947,10 +970,11 @@ struct RingFunction : torch::autograd::Function<RingFunction> {
     const Tensor &out = s[0], &lse = s[1], &q = s[2];
     const auto lists = chunk_lists(s, 3, cp, visited);
     std::optional<RingGrads> g;
-    // Whether steps hand dS over is the Python body's decision where a step could.
+    // Whether a share or its steps hand dS over is the Python body's decision where they could.
     const bool whole_keys = q.size(3) == 128 || (q.size(3) == 192 && !part_two(lists));
-    if (!whole_keys || (q.size(3) == 192 && !step_of_192_hands_over(q, lists[0][0]->size(2))))
-      g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag);
+    if (share_ds_bytes(q, lists[0], lists[1], part_two(lists), rank, cp, zigzag) == 0 &&
+        (!whole_keys || (q.size(3) == 192 && !step_of_192_hands_over(q, lists[0][0]->size(2)))))
+      g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag, {});
     if (!g) g = python_body<RingGrads>("ring_backward_local", grads[0], q, out, lse, lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
     variable_list r = {std::get<0>(*g)};
     for (const OptTensors* kind : {&std::get<1>(*g), &std::get<2>(*g), &std::get<3>(*g)})
@@ -1087,7 +1111,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_bwd_dq_into", &attn_bwd_dq_into, Unlocked());
   m.def("attn_bwd_pair_into", &attn_bwd_pair_into, Unlocked());
   m.def("ring_forward", &ring_forward, Unlocked());
-  m.def("ring_backward", &ring_backward, Unlocked());
+  m.def("ring_backward", &ring_backward, py::arg("dout"), py::arg("q"), py::arg("out"), py::arg("lse"), py::arg("ks"), py::arg("vs"), py::arg("pes"),
+        py::arg("scale"), py::arg("rank"), py::arg("cp"), py::arg("zigzag"), py::arg("ds") = py::none(), Unlocked());
+  m.def("share_ds_bytes", &share_ds_bytes);
+  m.def("share_of_192_pays", &share_of_192_pays);
   m.def("ring_attention", &ring_attention, Unlocked());
   m.def("combine_into", &combine_into, Unlocked());
   m.def("combine_new", &combine_new, Unlocked());

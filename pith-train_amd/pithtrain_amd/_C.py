@@ -150,6 +150,7 @@ SYMBOLS = {
     "pith_attn_bwd_dkdv_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
     "pith_attn_bwd_ds_bytes": (c_int64, [POINTER(AttnBwdArgs)]),
     "pith_attn_bwd_plan": (c_int, [POINTER(AttnBwdArgs), POINTER(AttnBwdPlan)]),
+    "pith_attn_bwd_chunks_ds_bytes": (c_int64, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64]),
     "pith_attn_bwd_chunks_plan": (c_int, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64, POINTER(AttnBwdPlan)]),
     "pith_cast_f32_bf16": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "pith_norm_rope_fwd": (c_int, [POINTER(NormRopeArgs), c_void_p]),

@@ -373,6 +373,15 @@ def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunk
     return _steps_beat_one_launch(q, k_chunks[steps[0].kv_rank].shape[2], sizes)
 
 
+def _share_ds(q: torch.Tensor, k_chunks, v_chunks, k_pe_chunks, cp_rank: int, cp_size: int, layout: str):
+    """The buffer for a share that hands dS over between one dK/dV and one dQ launch over all chunks (192 features, where that is
+    faster), within the limits of a chunk pair's (operators/mla/hip.py); None: not such a share, or not that much memory."""
+    need = native.share_ds_bytes(q, k_chunks, v_chunks, k_pe_chunks, cp_rank, cp_size, layout == "zigzag")
+    if need == 0 or hip._ds_budget_bytes(q.device, need) < need:
+        return None
+    return hip._try_alloc(need, q.device)
+
+
 def ring_forward_local(
     q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
     softmax_scale: float, cp_rank: int, cp_size: int, layout: str = "contiguous",
@@ -404,8 +413,9 @@ def ring_backward_local(
     dv_list[j] are this rank's contribution to the gradients of chunk j (None if never visited).
     With k_pe_chunks (keys in two parts) a fourth list holds the contributions to every k_pe chunk."""
     steps = ring_schedule(cp_rank, cp_size, q.shape[1], layout)
-    if FUSE_CHUNKS and not _handover_pays(steps, q, k_chunks, v_chunks):
-        done = native.ring_backward(dout, q, out, lse, k_chunks, v_chunks, k_pe_chunks, softmax_scale, cp_rank, cp_size, layout == "zigzag")
+    ds = _share_ds(q, k_chunks, v_chunks, k_pe_chunks, cp_rank, cp_size, layout) if FUSE_CHUNKS else None
+    if FUSE_CHUNKS and (ds is not None or not _handover_pays(steps, q, k_chunks, v_chunks)):
+        done = native.ring_backward(dout, q, out, lse, k_chunks, v_chunks, k_pe_chunks, softmax_scale, cp_rank, cp_size, layout == "zigzag", ds)
         if done is not None:
             return done if k_pe_chunks is not None else done[:3]
     bwd = RingBackward(dout, q, out, lse, softmax_scale, steps)

@@ -121,6 +121,26 @@ def test_calls_of_192_that_hand_over(causal, b, sq, skv, h, pays):
     assert native.ds_handover_pays_192(b, sq, skv, h, h, causal, UNITS) == pays and not native.ds_handover_pays_192(b, sq, skv, h, h, causal, 0)
 
 
+@pytest.mark.parametrize("b,s,h,pays", [(1, 1024, 16, 0), (1, 2048, 16, 0), (1, 8192, 4, 0), (4, 512, 16, 0), (8, 256, 32, 0), (1, 3072, 16, 1), (1, 12032, 4, 1),
+                                        (2, 1536, 16, 1), (1, 4096, 16, 1), (4, 1024, 16, 1), (1, 16384, 4, 1), (1, 6144, 16, 1)])  # fmt: skip
+def test_shares_of_192_that_hand_over(b, s, h, pays):
+    """As measured (table at share_of_192_pays)."""
+    assert native.share_of_192_pays(b, s, h, UNITS) == bool(pays) and not native.share_of_192_pays(b, s, h, 0)
+
+
+def test_bytes_of_a_share_that_hands_over():
+    """All chunks, a query tile of one lying within its images: 128 rows and keys of a half, their own chunk under the mask last."""
+    def need(sq, chunks, dqk=192):
+        args = _C.AttnBwdArgs(B=2, Sq=sq, Hq=4, Hkv=4, Dqk=dqk, Dv=128)
+        given = (_C.KeyChunk * len(chunks))(*[_C.KeyChunk(rows=rows, q_row0=row0) for rows, row0 in chunks])
+        return _C.lib().pith_attn_bwd_chunks_ds_bytes(_C.byref(args), given, len(chunks))
+
+    assert need(256, [(128, 0), (256, 128), (256, 0)]) == 2 * 4 * 16384 * (4 * 1 + 2 * 2 + 6)
+    assert need(258, [(129, 0), (258, 0)]) == 2 * 4 * 16384 * (5 * 2 + 1 + 1 + 2 + 2 + 3)
+    assert need(258, [(129, 0), (258, 129), (258, 0)]) == 0 and need(128, [(128, 0), (128, 0)]) == 0
+    assert need(256, [(256, 0)]) == 0 and need(256, [(128, 0), (256, 0)], 128) == 0
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_slabs_are_asked_for_by_the_rule_of_whole_calls(monkeypatch, causal):
     """A budget for one of two halves of the kv heads: the grid of a slab has to pass the same rule as that of the whole pair."""

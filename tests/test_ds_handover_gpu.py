@@ -117,6 +117,74 @@ def test_ring_share_of_192_with_and_without_handover(gpu, layout, monkeypatch):
         assert norm_max_err(a.float(), b.float()) < 6e-3
 
 
+@pytest.mark.parametrize("b,s,h,cp,rank,layout,two_parts", [
+    (1, 256, 2, 2, 0, "zigzag", False), (2, 640, 2, 3, 1, "zigzag", True), (1, 333, 2, 3, 2, "contiguous", False), (1, 1021, 4, 4, 2, "contiguous", True),
+    (3, 1100, 48, 2, 1, "contiguous", False), (5, 1024, 16, 4, 2, "zigzag", False), (1, 1152, 3, 4, 1, "zigzag", True),
+])  # fmt: skip
+def test_share_of_192_in_two_launches(gpu, b, s, h, cp, rank, layout, two_parts):
+    """All chunks' images in one buffer (poisoned), one dK/dV and one dQ launch: dK and dV bit for bit as without, dQ of the same bf16 dS
+    values summed in another order (one bf16 step, 2^-8, of the largest element). Half and whole chunks, an empty middle block of
+    rows, both orders of workgroups, ragged rows and keys."""
+    from pithtrain_amd._ext import native
+    from pithtrain_amd.operators.ring_attention import local as L
+
+    g = torch.Generator(device=gpu).manual_seed(s)
+    t = lambda *n: torch.randn(*n, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    of = lambda *n: [t(b, s, *n) if layout == "zigzag" or j <= rank else None for j in range(cp)]  # noqa: E731
+    q, dout, ks, vs, pes = t(b, s, h, 192), t(b, s, h, 128), of(h, 128 if two_parts else 192), of(h, 128), of(64) if two_parts else None
+    out, lse = L.ring_forward_local(q, ks, vs, 0.07, rank, cp, layout, pes)
+    blocks = 0
+    for st in L.ring_schedule(rank, cp, s, layout):
+        qt, kb = -((st.q_rows[0] - st.q_rows[1]) // 64), -((st.kv_rows[0] - st.kv_rows[1]) // 128)
+        blocks += sum(i // 2 + 1 for i in range(qt)) if st.causal else qt * kb
+    ds = torch.full((b * h * blocks * 16384,), 0x7F, dtype=torch.uint8, device=gpu)
+    args = (dout, q, out, lse, ks, vs, pes, 0.07, rank, cp, layout == "zigzag")
+    want, got, small = native.ring_backward(*args), native.ring_backward(*args, ds), native.ring_backward(*args, ds[:-256])
+    for a, x, y in zip((l for r in want[1:] for l in r), (l for r in got[1:] for l in r), (l for r in small[1:] for l in r), strict=True):
+        assert a is None and x is None or torch.equal(a, x) and torch.equal(a, y)
+    assert torch.equal(small[0], want[0]), "a buffer that is too small must not be used"
+    assert not torch.equal(got[0], want[0]) and norm_max_err(got[0].float(), want[0].float()) < 6e-3
+
+
+def test_share_of_192_hands_over_within_the_limits(gpu, monkeypatch):
+    """Also in a captured graph, every replay; above the memory limit and where the allocation fails the share recomputes."""
+    from pithtrain_amd._ext import native
+    from pithtrain_amd.operators.mla import hip as H
+
+    units = torch.cuda.get_device_properties(gpu).multi_processor_count
+    t = lambda d, grad: torch.randn(1, 3072, 16, d, device=gpu).to(torch.bfloat16).requires_grad_(grad)  # noqa: E731
+    q, ks, vs, dout = t(192, True), [t(192, True) for _ in range(2)], [t(128, True) for _ in range(2)], t(128, False)
+    need = native.share_ds_bytes(q, ks, vs, None, 1, 2, True)
+    assert (need > 0) == native.share_of_192_pays(1, 3072, 16, units)
+    buffers, real = [], H._try_alloc
+    monkeypatch.setattr(H, "_try_alloc", lambda *a: buffers.append(a[0]) or real(*a))
+
+    def step():
+        return torch.autograd.grad(ring_attention_local(q, ks, vs, 0.07, 1, 2, "zigzag"), [q, *ks, *vs], dout)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = step()
+    torch.cuda.current_stream().wait_stream(side)
+    assert buffers == ([need] if need else [])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for replay in range(3):
+        for x in captured:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, want)), f"replay {replay}"
+        assert all(torch.equal(a, b) for a, b in zip(step(), want))
+    monkeypatch.setattr(H, "_try_alloc", lambda *a: None)
+    failed = step()
+    monkeypatch.setattr(H, "DS_BUFFER_LIMIT_BYTES", 0)
+    limited = step()
+    assert all(torch.equal(a, b) for a, b in zip(failed, limited)) and norm_max_err(limited[0].float(), want[0].float()) < 6e-3
+
+
 @pytest.mark.parametrize("S", [255, 257, 511, 513, 767, 769, 1025, 1281, 1537])
 def test_causal_pairs_of_row_blocks(gpu, S):
     """Under the mask a workgroup takes 256-row blocks in pairs, one from either end: odd and even numbers of blocks, the last
