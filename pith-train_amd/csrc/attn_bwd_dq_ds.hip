@@ -28,9 +28,10 @@
 // 363 / 348, 4 x 1024 x 32/4 152.5 / 151.6. Past the vector cache only (sc1), or past more than that (sc0 nt, sc1 nt, sc0 sc1 nt): 0-3 %
 // slower than nt.
 // (192, 128): accumulators for 512 rows do not fit, so a workgroup owns 256 rows (under the mask in one round two blocks of 128), and
-// two waves share a 64-row tile, each with 96 of the features: a wave reads 2 + 3 KB of fragments per 6 products, and neither its images
+// two neighbouring waves share a 64-row tile, each with 96 of the features (either block's four waves lie on four SIMDs: with a tile's
+// waves four apart the late block, alone for most of the longest walk, had two; 4096 x 16 causal 83 -> 72 us): a wave reads 2 + 3 KB of fragments per 6 products, and neither its images
 // nor K are requested twice. K is 43 % of what a unit requests, so the images get the deeper ring: 7 stages of 16 KB beside 3 of 12.
-// dQ from dS / the recomputing kernels, us (dK/dV with / without the stores): 4096 x 16 causal 95 / 130 (166 / 160), 8192 x 16 251 / 438
+// dQ from dS / the recomputing kernels, us (dK/dV with / without the stores): 4096 x 16 causal 72 / 130 (166 / 160), 8192 x 16 251 / 438
 // (660 / 578), 4096 x 2048 x 16 68 / 114 (150 / 145), 4096 x 128 causal 570 / 936 (1468 / 1280).
 #include <type_traits>
 
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdArgs<MULTI>
   // Query tiles of the waves: eight consecutive ones, or, with ds_pairs, two 256-row blocks, waves 0..3 the m_tile-th from the
   // start and waves 4..7 the m_tile-th from the end, so that all workgroups read the same number of images (the middle one of
   // an odd number of blocks goes to waves 4..7 alone).
-  const int rg = wave & (RG - 1), fh = wave / RG;
+  const int rg = wave / FS, fh = wave % FS;
   const bool pairs = CAUSAL && p.ds_pairs;
   const int half_blocks = (p.Sq + kBM / 2 - 1) / (kBM / 2);
   auto rows_of = [&](int w) __attribute__((always_inline)) {
