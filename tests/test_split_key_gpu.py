@@ -122,3 +122,25 @@ def test_public_wrapper_with_keys_in_two_parts(gpu, rerotate):
     check_bf16_result(vd.grad, dv_ref, "dV", otol=1e-3)
     check_bf16_result(knd.grad, dk_ref[..., :128], "dK nope", otol=1e-3)
     check_bf16_result(kpd.grad[:, :, 0], dk_ref[..., 128:].sum(2), "dK pe", otol=1e-3)
+
+
+@pytest.mark.parametrize("heads", [1, 2, 3, 4, 5, 6, 7, 8, 13])
+def test_sum_over_heads_in_head_order(gpu, heads):
+    """dk_pe adds its heads' fp32 gradients one after the other, however many are loaded at a time: what the call with whole keys
+    leaves per head, summed in that order and rounded once."""
+    from pithtrain_amd.operators.mla import hip as H
+
+    g = torch.Generator(device=gpu).manual_seed(heads)
+    t = lambda *n: torch.randn(2, 130, *n, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, pe, v, dout = t(heads, 192), t(heads, 128), t(64), t(heads, 128), t(heads, 128)
+    whole = torch.cat([k, pe[:, :, None].expand(-1, -1, heads, -1)], dim=-1).contiguous()
+    o, lse = H._mla_fwd(q, whole, v, 0.07, True)
+    delta = H._mla_bwd_preprocess(o, dout)
+    dk32, dv32 = torch.empty(whole.shape, device=gpu), torch.empty(v.shape, device=gpu)
+    H.attn_bwd_dkdv_into(q, whole, v, dout, lse, delta, dk32, dv32, 0.07, True)
+    dk, dv, dpe = torch.empty_like(k), torch.empty_like(v), torch.empty_like(pe)
+    H.attn_bwd_dkdv_into(q, k, v, dout, lse, delta, dk, dv, 0.07, True, k_pe=pe, dk_pe=dpe)
+    want = dk32[:, :, 0, 128:].clone()
+    for h in range(1, heads):
+        want += dk32[:, :, h, 128:]
+    assert torch.equal(dpe, want.to(torch.bfloat16)) and torch.equal(dk, dk32[..., :128].to(torch.bfloat16))
