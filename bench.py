@@ -178,11 +178,15 @@ def bench_recompute(torch, dev_inputs, steps, warmup):
 
 
 def handover_scratch_bytes(cfg, dev):
-    """Largest dS hand-over scratch the ring backward takes in a ring step of `cfg` (0: it recomputes in all of them)."""
+    """Largest dS hand-over scratch the ring backward takes in a ring step of `cfg` (0: it recomputes in all of them); of a share
+    that hands over between two launches over all chunks, that of the share."""
     from pithtrain_amd.operators.mla import hip
-    from pithtrain_amd.operators.ring_attention.local import ring_schedule
+    from pithtrain_amd.operators.ring_attention.local import _share_ds, ring_schedule
 
     q, ks, vs, _ = dev
+    share = _share_ds(q, ks, vs, None, cfg.rank, cfg.cp, LAYOUT)
+    if share is not None:
+        return share.numel()
     most = 0
     for s in ring_schedule(cfg.rank, cfg.cp, cfg.s_local, LAYOUT):
         rows = slice(s.kv_rows[0], s.kv_rows[1])
@@ -270,8 +274,8 @@ def share_forward(torch, cfg, dev, reps):
 
 
 def share_backward(torch, cfg, dev, out, lse, reps):
-    """The backward of a share of `cfg` that hands no dS over: dK/dV and dQ of all chunks in one grid, behind the delta
-    launch (8 us of it at 4096 rows x 16 heads). (ms, FLOPs, launches)."""
+    """The backward of a share of `cfg` whose chunks go out together, dK/dV and dQ of all of them in one grid or, handing dS over, in
+    two, behind the delta launch (8 us of it at 4096 rows x 16 heads). (ms, FLOPs, launches)."""
     from pithtrain_amd.operators.ring_attention.local import ring_backward_local
 
     q, ks, vs, dout = dev
@@ -282,17 +286,18 @@ def share_backward(torch, cfg, dev, out, lse, reps):
 
 def bench_other_config(torch, device, cfg, steps, warmup, cpu_heads=None, counter_pass=False):
     """Step time of another configuration through the same ring driver, its dominant kernel (the non-causal dK/dV launch,
-    or the one grid of a share that hands no dS over) against the MFMA roofline, and (cpu_heads = (first, last+1) query
+    or all of a backward whose chunks go out together) against the MFMA roofline, and (cpu_heads = (first, last+1) query
     heads, or "all") the oracle's CPU port on that sample of the same workload."""
     host, dev = cfg.make_inputs(torch, device, host=cpu_heads is not None)
     ms_step, ms_fwd, ms_bwd, o, lse = time_ring_share(torch, cfg, dev, steps, warmup)
     scratch = handover_scratch_bytes(cfg, dev)
+    by_step = scratch and cfg.dqk == 128
     if counter_pass:
-        if scratch:
+        if by_step:
             dominant_dkdv(torch, cfg, dev, o, lse, 1, counter_pass=True)
         return None
     out = ring_summary(cfg, ms_step, ms_fwd, ms_bwd)
-    if scratch:
+    if by_step:
         ms, flops, n, _, name = dominant_dkdv(torch, cfg, dev, o, lse, steps)
         slabs = n // len(noncausal_steps(cfg))
         kernel = (f"{name}<non-causal> (S, dP, dV, dK of one ring step" + (f", one of {slabs} kv-head slabs per launch" if slabs > 1 else "")
@@ -300,8 +305,11 @@ def bench_other_config(torch, device, cfg, steps, warmup, cpu_heads=None, counte
         traffic = f"{cfg.name}.dkdv_traffic_bytes_per_launch"
     else:
         ms, flops, n = share_backward(torch, cfg, dev, o, lse, steps)
-        kernel = f"attn_bwd_pair_chunks_kernel<{cfg.dqk}> (dK/dV and dQ of all chunks in one grid, with the delta launch before it)"
-        traffic = f"{cfg.name}.bwd_traffic_bytes_per_launch"
+        if scratch:
+            kernel = f"attn_bwd_dkdv_chunks_kernel<{cfg.dqk}>, attn_bwd_dq_ds_kernel<{cfg.dqk}> (all chunks, dS handed over, with the delta launch before them)"
+        else:
+            kernel = f"attn_bwd_pair_chunks_kernel<{cfg.dqk}> (dK/dV and dQ of all chunks in one grid, with the delta launch before it)"
+        traffic = f"{cfg.name}.bwd_{'handover_' if scratch else ''}traffic_bytes_per_launch"
     out["roofline"] = roofline_entry(kernel, flops, ms, n, profile_figure(HBM_COUNTERS, traffic), "profiles/" + HBM_COUNTERS)
     out["ds_handover_scratch_bytes_per_ring_step"] = scratch
     del dev, o, lse
