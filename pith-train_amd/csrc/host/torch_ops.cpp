@@ -391,11 +391,11 @@ bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chu
 // Against one grid of both kinds (two recomputing launches from W 1 on) that loses the last round of either launch and wins two products
 // of seven. W = its 256-row dQ workgroups per compute unit; backward, handing over / recomputing, us, four ranks unless named, zigzag rank 1
 // and contiguous rank 1:
-//   W 0.25  1024 x 16 130 / 88 and 146 / 106               W 0.5   2048 x 16 323 / 288 and 232 / 217, 8192 x 4 1177 / 1061 and 826 / 791, 4 x 512 x 16 119 / 102
-//   W 0.75  3072 x 16 569 / 638 and 683 / 775, 12032 x 4 2080 / 2312 and 2499 / 2886, 2 x 1536 x 16 315 / 344 and 358 / 412
-//   W 1     4096 x 16 974 / 1070 and 684 / 798, 8 ranks 1856 / 2064 and 2427 / 2794, 2 x 2048 x 16 532 / 573 and 373 / 429, 4 x 1024 x 16 324 / 342 and
-//           218 / 248, 16384 x 4 3734 / 4036 and 2636 / 3024    W 1.25-2   5120 x 16, 2 ranks 737 / 839, 6144 x 16 2034 / 2325, 8192 x 16, 2 ranks 1771 / 2027
-// Keys in two parts the same: 4096 x 16 986 / 1072, 4 x 1024 x 16 331 / 348.
+//   W 0.25  1024 x 16 123 / 88 and 143 / 106               W 0.5   2048 x 16 300 / 287 and 224 / 216, 8192 x 4 1077 / 1055 and 800 / 788, 4 x 512 x 16 110 / 101
+//   W 0.75  3072 x 16 567 / 640 and 679 / 777, 12032 x 4 2055 / 2326 and 2466 / 2873, 2 x 1536 x 16 313 / 349 and 361 / 418
+//   W 1     4096 x 16 948 / 1052 and 678 / 790, 8 ranks 1825 / 2066 and 2444 / 2801, 2 x 2048 x 16 519 / 568 and 361 / 422, 4 x 1024 x 16 310 / 336 and
+//           209 / 244, 16384 x 4 3575 / 4007 and 2630 / 3008    W 1.25-2   5120 x 16, 2 ranks 740 / 838, 6144 x 16 2054 / 2322, 8192 x 16, 2 ranks 1776 / 2017
+// Keys in two parts the same: 4096 x 16 969 / 1063, 4 x 1024 x 16 316 / 344.
 bool share_of_192_pays(int64_t b, int64_t rows, int64_t hq, int64_t cus) { return cus > 0 && rows >= 512 && 10 * ((rows + 255) / 256 * hq * b) >= 7 * cus; }
 int64_t share_ds_bytes(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes,
                        int64_t rank, int64_t cp, bool zigzag) {
@@ -514,15 +514,15 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
 // The same for (192, 128): its dQ kernel takes 256 rows per workgroup.
 // W = 256-row workgroups per compute unit, F as above; backward alone, inputs changing, handing over / recomputing, us (16 heads unless
 // others are named):
-//   causal  W 0.5         2048 110 / 86, 1024 x 32 65 / 52, 8192 x 4 371 / 289    W 0.75  3072 169 / 170, 12288 x 4 619 / 600, 3 x 1021 75 / 85
-//           W 1           4096 253 / 281, 2 x 2048 142 / 161, 4 x 1024 88 / 101, 8 x 512 65 / 71, 512 x 128 66 / 71, 16384 x 4 943 / 1007, 4096 x 16/4 269 / 298
-//           W 1.12-2.25   4608 325 / 376, 5120 392 / 450, 6144 533 / 604, 3 x 1999 210 / 230, 7168 692 / 769, 1024 x 128 178 / 193, 9216 1145 / 1277
-//   full    F below 0.75  2048 x 1024 84 / 73, 8192 x 4096 x 4 289 / 261, 2731 x 1366 129 / 143    W 0.25  1024 x 2048 88 / 86, 4096 x 8192 x 4 299 / 286
-//           W 0.5         2048 x 2048 124 / 135, 2 x 1024 x 2048 132 / 144, 8192 x 16384 x 4 917 / 959
-//           W 0.6-1.25    2560 x 5120 375 / 420, 3072 x 1536 141 / 153, 3072 x 6144 499 / 598, 2 x 2048 x 1024 120 / 138, 5120 x 2560 441 / 503
-// Below 512 rows the device still gains 4-7 % (16 x 300 77 / 81, 32 x 192 82 / 85), less than the time such a call spends in Python.
+//   causal  W 0.5         2048 104 / 88, 1024 x 32 61 / 52, 8192 x 4 336 / 287    W 0.75  3072 156 / 170, 12288 x 4 581 / 610, 3 x 1021 69 / 82
+//           W 1           4096 243 / 282, 2 x 2048 135 / 161, 4 x 1024 82 / 98, 8 x 512 60 / 66, 512 x 128 59 / 65, 16384 x 4 917 / 1036, 4096 x 16/4 265 / 301
+//           W 1.12-2.25   4608 326 / 379, 5120 396 / 454, 6144 542 / 614, 3 x 1999 204 / 229, 7168 706 / 790, 1024 x 128 171 / 189, 9216 1176 / 1308
+//   full    F below 0.75  2048 x 1024 85 / 74, 8192 x 4096 x 4 292 / 268, 2731 x 1366 127 / 140    W 0.25  1024 x 2048 91 / 84, 4096 x 8192 x 4 313 / 290
+//           W 0.5         2048 x 2048 128 / 139, 2 x 1024 x 2048 134 / 144, 8192 x 16384 x 4 942 / 994
+//           W 0.6-1.25    2560 x 5120 391 / 428, 3072 x 1536 138 / 155, 3072 x 6144 507 / 604, 2 x 2048 x 1024 117 / 139, 5120 x 2560 426 / 503
+// Below 512 rows the device still gains 2-11 % (16 x 300 69 / 75, 32 x 192 81 / 83), less than the time such a call spends in Python.
 bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
-  if (cus <= 0 || sq < 512 || (sq + 255) / 256 * hq * b * (causal ? 1 : 2) < cus) return false;
+  if (cus <= 0 || sq < 512 || 10 * ((sq + 255) / 256 * hq * b) < (causal ? 7 : 5) * cus) return false;
   pith_attn_bwd_args a = {};
   a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = 192; a.Dv = 128; a.causal = causal;
   pith_attn_bwd_plan_t plan;
