@@ -395,8 +395,8 @@ bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chu
 //   W 0.75  3072 x 16 567 / 640 and 679 / 777, 12032 x 4 2055 / 2326 and 2466 / 2873, 2 x 1536 x 16 313 / 349 and 361 / 418
 //   W 1     4096 x 16 948 / 1052 and 678 / 790, 8 ranks 1825 / 2066 and 2444 / 2801, 2 x 2048 x 16 519 / 568 and 361 / 422, 4 x 1024 x 16 310 / 336 and
 //           209 / 244, 16384 x 4 3575 / 4007 and 2630 / 3008    W 1.25-2   5120 x 16, 2 ranks 740 / 838, 6144 x 16 2054 / 2322, 8192 x 16, 2 ranks 1776 / 2017
-// Keys in two parts the same: 4096 x 16 969 / 1063, 4 x 1024 x 16 316 / 344.
-bool share_of_192_pays(int64_t b, int64_t rows, int64_t hq, int64_t cus) { return cus > 0 && rows >= 512 && 10 * ((rows + 255) / 256 * hq * b) >= 7 * cus; }
+// Keys in two parts the same: 4096 x 16 969 / 1063, 4 x 1024 x 16 316 / 344. Shorter rows were not measured at W 0.7 and more.
+bool share_of_192_pays(int64_t b, int64_t rows, int64_t hq, int64_t cus) { return cus > 0 && rows >= 1024 && 10 * ((rows + 255) / 256 * hq * b) >= 7 * cus; }
 int64_t share_ds_bytes(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes,
                        int64_t rank, int64_t cp, bool zigzag) {
   if (!q.is_cuda() || q.dim() != 4 || q.size(3) != 192 || !share_of_192_pays(q.size(0), q.size(1), q.size(2), compute_units(q.device().index()))) return 0;
@@ -520,9 +520,10 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
 //   full    F below 0.75  2048 x 1024 85 / 74, 8192 x 4096 x 4 292 / 268, 2731 x 1366 127 / 140    W 0.25  1024 x 2048 91 / 84, 4096 x 8192 x 4 313 / 290
 //           W 0.5         2048 x 2048 128 / 139, 2 x 1024 x 2048 134 / 144, 8192 x 16384 x 4 942 / 994
 //           W 0.6-1.25    2560 x 5120 391 / 428, 3072 x 1536 138 / 155, 3072 x 6144 507 / 604, 2 x 2048 x 1024 117 / 139, 5120 x 2560 426 / 503
-// Below 512 rows the device still gains 2-11 % (16 x 300 69 / 75, 32 x 192 81 / 83), less than the time such a call spends in Python.
+// Below 2^25 visible pairs of rows and heads the device gains as much, but the Python body of such a call takes longer than its kernels:
+// forward + backward with the host's time 8 x 512 causal 93-120 / 102, 512 x 128 99-123 / 111; 4 x 1024 127 / 140.
 bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
-  if (cus <= 0 || sq < 512 || 10 * ((sq + 255) / 256 * hq * b) < (causal ? 7 : 5) * cus) return false;
+  if (cus <= 0 || b * hq * sq * skv < (int64_t)(causal ? 64 : 32) << 20 || 10 * ((sq + 255) / 256 * hq * b) < (causal ? 7 : 5) * cus) return false;
   pith_attn_bwd_args a = {};
   a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = 192; a.Dv = 128; a.causal = causal;
   pith_attn_bwd_plan_t plan;

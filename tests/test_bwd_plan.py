@@ -112,7 +112,7 @@ def test_rows_that_fill_their_workgroups(pays, b, s, hq, hkv):
 
 @pytest.mark.parametrize("causal,b,sq,skv,h,pays", [
     (True, 1, 4096, 4096, 16, True), (True, 4, 1024, 1024, 16, True), (True, 1, 4608, 4608, 16, True), (True, 1, 16384, 16384, 4, True),
-    (True, 1, 3072, 3072, 16, True), (True, 1, 2048, 2048, 16, False), (True, 1, 12288, 12288, 4, True), (True, 1, 8192, 8192, 4, False), (True, 16, 256, 256, 16, False),
+    (True, 1, 3072, 3072, 16, True), (True, 1, 2048, 2048, 16, False), (True, 1, 12288, 12288, 4, True), (True, 1, 8192, 8192, 4, False), (True, 8, 512, 512, 16, False), (True, 16, 512, 512, 16, True), (True, 16, 256, 256, 16, False),
     (False, 1, 4096, 2048, 16, True), (False, 1, 2048, 4096, 16, True), (False, 1, 2048, 1024, 16, False), (False, 1, 1024, 2048, 16, False),
     (False, 1, 8192, 4096, 4, False), (False, 1, 4096, 8192, 4, False),
 ])  # fmt: skip
