@@ -50,9 +50,11 @@ enum { PITH_BF16 = 0, PITH_F32 = 1 };
 enum { PITH_BASE_2 = 0, PITH_BASE_E = 1 };
 
 /* Version of this interface: major*10000 + minor*100 + patch. The minor number goes up whenever a struct or a signature below
- * changes; a program built against another one must not call into the library (its structs have other sizes).
+ * changes; a program built against another one must not call into the library (its structs have other sizes). The patch number
+ * goes up when functions are added.
+ * 201: pith_attn_bwd_chunks_handover, pith_attn_bwd_chunks_ds_bytes and the plan functions added.
  * 200: pith_norm_rope_args gained dweight_bf16, and dweight became void*; chunk calls and pith_attn_bwd added. */
-#define PITH_VERSION 200
+#define PITH_VERSION 201
 int pith_version(void); /* PITH_VERSION of the library that was loaded */
 /* Text of the last error raised on the calling thread ("" if none). Never NULL. */
 const char* pith_last_error(void);
@@ -276,12 +278,15 @@ int pith_attn_bwd(const pith_attn_bwd_args* args, pith_stream_t stream);
 
 /* The same against several chunks at once (pith_key_chunk, conventions of pith_attn_fwd_chunks): dq is written once, over
  * all chunks, and dk, dv (dk_pe) of every chunk. args describes the query side and what the chunks share; its k, v, k_pe,
- * Skv, causal, dk, dv, dk_pe and dkv_zero_tail are ignored. Gradients are bf16, nothing is accumulated. The workspace is
- * required wherever pith_attn_bwd_chunks_workspace_bytes is not 0. With a `ds` buffer of at least pith_attn_bwd_chunks_ds_bytes (0:
- * no hand-over path; head dims (192,128), keys in one part or two, every q_row0 a multiple of 64) dS is handed over as described below. */
+ * Skv, causal, dk, dv, dk_pe, dkv_zero_tail and ds are ignored. Gradients are bf16, nothing is accumulated. The workspace is
+ * required wherever pith_attn_bwd_chunks_workspace_bytes is not 0.
+ * pith_attn_bwd_chunks_handover is the same call with a buffer of its own, 256-byte aligned, of pith_attn_bwd_chunks_ds_bytes bytes, through which
+ * dS is handed over as described below; with `ds` NULL or a buffer that is too small it does what pith_attn_bwd_chunks does. The size is 0
+ * where there is no hand-over path: head dims other than (192,128), a single chunk, up to 128 rows, a q_row0 that is no multiple of 64. */
 int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n);
 int64_t pith_attn_bwd_chunks_ds_bytes(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n);
 int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream);
+int pith_attn_bwd_chunks_handover(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, void* ds, int64_t ds_bytes, pith_stream_t stream);
 
 /* Scratch size with which pith_attn_bwd_dkdv runs fastest for these shapes (0 = none needed).
  * With grouped-query attention and few key rows the kernel spreads the query heads of a group

@@ -478,8 +478,9 @@ extern "C" int64_t pith_attn_bwd_chunks_ds_bytes(const pith_attn_bwd_args* args,
   return bytes;
 }
 
-extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
-  const char* who = "pith_attn_bwd_chunks";
+namespace {
+
+int run_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, void* ds, int64_t ds_bytes, pith_stream_t stream, const char* who) {
   if (!args || !chunks) return fail(PITH_ERR_NULL_POINTER, "%s: args or chunks is NULL", who);
   pith_attn_bwd_args all;
   int64_t tiles;
@@ -499,8 +500,8 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   if (need > 0 && (!args->workspace || args->workspace_bytes < need || !aligned16(args->workspace)))
     return fail(PITH_ERR_BAD_SHAPE, "%s: a 16-byte aligned workspace of %lld bytes is needed", who, (long long)need);
   const int64_t ds_need = pith_attn_bwd_chunks_ds_bytes(args, chunks, n);
-  const bool hand_over = args->ds && ds_need > 0 && args->ds_bytes >= ds_need;
-  if (hand_over && (uintptr_t)args->ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
+  const bool hand_over = ds && ds_need > 0 && ds_bytes >= ds_need;
+  if (hand_over && (uintptr_t)ds % 256) return fail(PITH_ERR_MISALIGNED, "%s: ds must be 256-byte aligned", who);
   BwdChunkParams p;
   unsigned blocks = 0;
   int64_t rows_before = 0, ds_off = 0;
@@ -537,7 +538,7 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
   p.split = split;
   const int dq_rows = hand_over ? dq_ds_rows(192) : 128;
   p.q_tiles = (p.Sq + dq_rows - 1) / dq_rows;
-  if (hand_over) p.ds = reinterpret_cast<char*>(args->ds);
+  if (hand_over) p.ds = reinterpret_cast<char*>(ds);
   p.ws_dk = reinterpret_cast<float*>(need > 0 ? args->workspace : nullptr);
   p.ws_dv = p.ws_dk + (split > 1 ? (int64_t)split * all.B * all.Skv * all.Hkv * all.Dqk : 0);
   p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));
@@ -560,4 +561,15 @@ extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_k
     r.launch(all.k_pe ? (int)all.Hkv : split, false, false, st);
   }
   return check_launch(who);
+}
+
+}  // namespace
+
+extern "C" int pith_attn_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream) {
+  return run_bwd_chunks(args, chunks, n, nullptr, 0, stream, "pith_attn_bwd_chunks");
+}
+
+extern "C" int pith_attn_bwd_chunks_handover(const pith_attn_bwd_args* args, const pith_key_chunk* chunks, int64_t n, void* ds, int64_t ds_bytes,
+                                             pith_stream_t stream) {
+  return run_bwd_chunks(args, chunks, n, ds, ds_bytes, stream, "pith_attn_bwd_chunks_handover");
 }

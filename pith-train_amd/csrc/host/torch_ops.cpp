@@ -430,11 +430,7 @@ std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, c
   a.dk_pe_bs = a.Sq * 64;
   a.dq_dtype = a.dkv_dtype = PITH_BF16;
   a.scale = (float)scale;
-  if (ds) {
-    if (!ds->is_cuda() || ds->device() != q.device() || ds->scalar_type() != at::kByte || !ds->is_contiguous() || (uintptr_t)ds->data_ptr() % 256) return std::nullopt;
-    a.ds = ds->data_ptr();
-    a.ds_bytes = ds->numel();
-  }
+  if (ds && (!ds->is_cuda() || ds->device() != q.device() || ds->scalar_type() != at::kByte || !ds->is_contiguous() || (uintptr_t)ds->data_ptr() % 256)) return std::nullopt;
   RingGrads g = {dq, std::vector<OptTensor>(cp), std::vector<OptTensor>(cp), std::vector<OptTensor>(pes ? cp : 0)};
   for (size_t i = 0; i < r.chunk.size(); ++i) {
     const int64_t j = r.rank[i];
@@ -454,7 +450,7 @@ std::optional<RingGrads> ring_backward(const Tensor& dout_in, const Tensor& q, c
     a.workspace = workspace.data_ptr();
     a.workspace_bytes = need;
   }
-  if (!accepted(pith_attn_bwd_chunks(&a, r.chunk.data(), n, stream_of(q)))) return std::nullopt;
+  if (!accepted(pith_attn_bwd_chunks_handover(&a, r.chunk.data(), n, ds ? ds->data_ptr() : nullptr, ds ? ds->numel() : 0, stream_of(q)))) return std::nullopt;
   return g;
 }
 

@@ -13,7 +13,7 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libpith_hip.so")
 
-PITH_VERSION = 200  # of include/pith_hip.h, whose structs are declared below
+PITH_VERSION = 201  # of include/pith_hip.h, whose structs are declared below
 
 PITH_BF16, PITH_F32 = 0, 1
 PITH_BASE_2, PITH_BASE_E = 0, 1
@@ -145,6 +145,7 @@ SYMBOLS = {
     "pith_attn_bwd_dq": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_chunks": (c_int, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64, c_void_p]),
+    "pith_attn_bwd_chunks_handover": (c_int, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64, c_void_p, c_int64, c_void_p]),
     "pith_attn_bwd_chunks_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs), POINTER(KeyChunk), c_int64]),
     "pith_attn_bwd_dkdv_static": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dkdv_workspace_bytes": (c_int64, [POINTER(AttnBwdArgs)]),

@@ -470,3 +470,40 @@ def test_layer_of_one_round_under_capture(gpu):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(captured, want)), f"replay {replay}"
         assert all(torch.equal(a, b) for a, b in zip(step(), want))
+
+
+@pytest.mark.parametrize("head_dim", [128, 192])
+def test_chunk_call_leaves_the_ds_of_its_arguments_alone(gpu, head_dim):
+    """pith_attn_bwd_chunks ignores args.ds, which may hold a chunk pair's tiles: nothing is written there, no result depends on it and
+    an odd address is none of its business. The buffer of the hand-over is an argument of its own call."""
+    from pithtrain_amd import _C
+
+    S, H, scale = 256, 2, 0.07
+    g = torch.Generator(device=gpu).manual_seed(3)
+    t = lambda d: torch.randn(1, S, H, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, dout, out, ks, vs = t(head_dim), t(128), t(128), [t(head_dim) for _ in range(2)], [t(128) for _ in range(2)]
+    lse, delta = torch.full((1, H, S), 12.0, device=gpu), _mla_bwd_preprocess(out, dout)
+    grads = [torch.empty_like(q), *(torch.empty_like(x) for x in (*ks, *vs))]
+    chunks = (_C.KeyChunk * 2)(*[_C.KeyChunk(k=ks[i].data_ptr(), v=vs[i].data_ptr(), rows=S, dk=grads[1 + i].data_ptr(), dv=grads[3 + i].data_ptr())
+                                 for i in range(2)])  # fmt: skip
+
+    def run(ds=None, offset=0, call="pith_attn_bwd_chunks", *more):
+        for x in grads:
+            x.fill_(float("nan"))
+        a = _C.AttnBwdArgs(q=q.data_ptr(), dout=dout.data_ptr(), lse=lse.data_ptr(), delta=delta.data_ptr(), dq=grads[0].data_ptr(), B=1, Sq=S, Hq=H, Hkv=H,
+                           Dqk=head_dim, Dv=128, q_bs=q.stride(0), k_bs=q.stride(0), v_bs=dout.stride(0), dout_bs=dout.stride(0), dq_bs=q.stride(0),
+                           dk_bs=q.stride(0), dv_bs=dout.stride(0), lse_bs=H * S, lse_hs=S, scale=scale)  # fmt: skip
+        if ds is not None and not more:
+            a.ds, a.ds_bytes = ds.data_ptr() + offset, ds.numel() - offset
+        _C.check(getattr(_C.lib(), call)(_C.byref(a), chunks, 2, *more, torch.cuda.current_stream().cuda_stream))
+        return [x.clone() for x in grads]
+
+    want = run()
+    ds = torch.full((1 << 20,), 0x7F, dtype=torch.uint8, device=gpu)
+    for offset in (0, 8):
+        assert all(torch.equal(a, b) for a, b in zip(run(ds, offset), want))
+        assert (ds == 0x7F).all(), "written through args.ds"
+    handed = run(ds, 0, "pith_attn_bwd_chunks_handover", ds.data_ptr(), ds.numel())
+    assert (ds == 0x7F).all() == (head_dim == 128) and torch.equal(handed[0], want[0]) == (head_dim == 128)
+    assert all(torch.equal(a, b) for a, b in zip(handed[1:], want[1:])) and norm_max_err(handed[0].float(), want[0].float()) < 6e-3
+    assert all(torch.equal(a, b) for a, b in zip(run(ds, 0, "pith_attn_bwd_chunks_handover", None, 0), want))
