@@ -51,8 +51,8 @@ enum { PITH_BASE_2 = 0, PITH_BASE_E = 1 };
 
 /* Version of this interface: major*10000 + minor*100 + patch. The minor number goes up whenever a struct or a signature below
  * changes; a program built against another one must not call into the library (its structs have other sizes). The patch number
- * goes up when functions are added.
- * 201: pith_attn_bwd_chunks_handover, pith_attn_bwd_chunks_ds_bytes and the plan functions added.
+ * goes up when functions are added or a call takes up a field that it ignored.
+ * 201: pith_attn_bwd_chunks_handover, pith_attn_bwd_chunks_ds_bytes and the plan functions added; `ds` used at head dims (192,128).
  * 200: pith_norm_rope_args gained dweight_bf16, and dweight became void*; chunk calls and pith_attn_bwd added. */
 #define PITH_VERSION 201
 int pith_version(void); /* PITH_VERSION of the library that was loaded */
@@ -306,8 +306,9 @@ int64_t pith_attn_bwd_dkdv_workspace_bytes(const pith_attn_bwd_args* args);
  * diagonal: about half). Results agree with the recomputing dQ kernel up to
  * fp32 summation order (the dS values are the same bf16 numbers). The buffer holds nothing of
  * value after the dQ call. Returns the bytes needed, or 0 when the shape has no hand-over path
- * (head dims other than (128,128) and (192,128), the latter up to 128 rows, keys in two parts); with ds == NULL or a buffer that is too small both calls
- * behave as before. */
+ * (head dims other than (128,128) and (192,128), the latter up to 128 rows, keys in two parts). With ds == NULL or a buffer that is too
+ * small both calls recompute. A buffer that is not 256-byte aligned is an error at (128,128) and counts as none at (192,128), where
+ * interface 200 ignored the field. */
 int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* args);
 
 /* How the backward calls of these shapes are cut on the current device, for tests and profiles: no results depend on it except

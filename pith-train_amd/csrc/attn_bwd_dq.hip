@@ -26,7 +26,10 @@ bool dq_split_keys(const pith_attn_bwd_args* a) {
 
 }  // namespace
 
-bool ds_usable(const pith_attn_bwd_args* a) { return a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a); }
+bool ds_usable(const pith_attn_bwd_args* a) {
+  // (192 features: the field was ignored before there was a hand-over, so what callers left in it is no error)
+  return a->ds && ds_bytes_for(a) > 0 && a->ds_bytes >= ds_bytes_for(a) && (a->Dqk != 192 || (uintptr_t)a->ds % 256 == 0);
+}
 
 int validate_bwd(const pith_attn_bwd_args* a, const char* who, bool need_dq, bool need_dkv) {
   if (!a) return fail(PITH_ERR_NULL_POINTER, "%s: args is NULL", who);

@@ -507,3 +507,41 @@ def test_chunk_call_leaves_the_ds_of_its_arguments_alone(gpu, head_dim):
     assert (ds == 0x7F).all() == (head_dim == 128) and torch.equal(handed[0], want[0]) == (head_dim == 128)
     assert all(torch.equal(a, b) for a, b in zip(handed[1:], want[1:])) and norm_max_err(handed[0].float(), want[0].float()) < 6e-3
     assert all(torch.equal(a, b) for a, b in zip(run(ds, 0, "pith_attn_bwd_chunks_handover", None, 0), want))
+
+
+@pytest.mark.parametrize("head_dim", [128, 192])
+def test_misaligned_buffer(gpu, head_dim):
+    """A buffer off 256 bytes: refused at 128 features, where it always was; at 192, where the field used to be ignored, both calls
+    recompute and leave it alone."""
+    from pithtrain_amd import _C
+
+    S, H, scale = 256, 2, 0.07
+    g = torch.Generator(device=gpu).manual_seed(4)
+    t = lambda d: torch.randn(1, S, H, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v, dout = t(head_dim), t(head_dim), t(128), t(128)
+    o, lse = _mla_fwd(q, k, v, scale, True)
+    delta = _mla_bwd_preprocess(o, dout)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    a = _C.AttnBwdArgs(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), dout=dout.data_ptr(), lse=lse.data_ptr(), delta=delta.data_ptr(), dq=dq.data_ptr(),
+                       dk=dk.data_ptr(), dv=dv.data_ptr(), B=1, Sq=S, Skv=S, Hq=H, Hkv=H, Dqk=head_dim, Dv=128, q_bs=q.stride(0), k_bs=k.stride(0),
+                       v_bs=v.stride(0), dout_bs=v.stride(0), dq_bs=q.stride(0), dk_bs=k.stride(0), dv_bs=v.stride(0), lse_bs=H * S, lse_hs=S,
+                       scale=scale, causal=1)  # fmt: skip
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(*calls):
+        for x in (dq, dk, dv):
+            x.fill_(float("nan"))
+        codes = [getattr(_C.lib(), c)(_C.byref(a), stream) for c in calls]
+        return codes, [x.clone() for x in (dq, dk, dv)]
+
+    forms = [("pith_attn_bwd_dkdv", "pith_attn_bwd_dq"), ("pith_attn_bwd",)]
+    want = [run(*calls)[1] for calls in forms]
+    ds = torch.full((1 << 20,), 0x7F, dtype=torch.uint8, device=gpu)
+    a.ds, a.ds_bytes = ds.data_ptr() + 16, ds.numel() - 16
+    for calls, results in zip(forms, want):
+        codes, got = run(*calls)
+        if head_dim == 128:
+            assert codes == [_C.PITH_ERR_MISALIGNED] * len(calls)
+        else:
+            assert codes == [_C.PITH_OK] * len(calls) and all(torch.equal(x, y) for x, y in zip(got, results))
+    assert (ds == 0x7F).all()
