@@ -316,8 +316,8 @@ int64_t pith_attn_bwd_ds_bytes(const pith_attn_bwd_args* args);
 typedef struct {
   int32_t dkdv_rows;    /* pith_attn_bwd_dkdv, launched alone: key rows per workgroup */
   int32_t dkdv_split;   /* and the parts each group of query heads is cut into (given the workspace) */
-  int32_t dq_ds_pairs;  /* pith_attn_bwd_dq from handed-over dS, 128 features, causal: workgroups take rows from both ends */
-  int32_t one_grid;     /* pith_attn_bwd with bf16 gradients and without ds: both kernels in one launch */
+  int32_t dq_ds_pairs;  /* dQ from handed-over dS, causal or of several chunks: workgroups take rows from both ends */
+  int32_t one_grid;     /* pith_attn_bwd (_chunks) with bf16 gradients and without ds: both kernels in one launch */
 } pith_attn_bwd_plan_t;
 
 int pith_attn_bwd_plan(const pith_attn_bwd_args* args, pith_attn_bwd_plan_t* plan);

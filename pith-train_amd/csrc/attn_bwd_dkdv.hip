@@ -231,6 +231,12 @@ bool one_grid(const pith_attn_bwd_args* a, int64_t dkdv_wgs, bool chunks) {
   return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));
 }
 
+// Workgroups of the dQ kernel that reads handed-over dS.
+int64_t dq_ds_workgroups(const pith_attn_bwd_args* a) {
+  const int rows = dq_ds_rows((int)a->Dqk);
+  return (a->Sq + rows - 1) / rows * a->Hq * a->B;
+}
+
 }  // namespace
 }  // namespace pith
 
@@ -251,7 +257,7 @@ extern "C" int pith_attn_bwd_plan(const pith_attn_bwd_args* a, pith_attn_bwd_pla
   const Plan chosen = pick_plan(a, plan_for(a, kBN));
   plan->dkdv_rows = chosen.rows;
   plan->dkdv_split = chosen.split;
-  plan->dq_ds_pairs = a->causal && a->Dqk == 128 && ds_bytes_for(a) > 0 && dq_ds_pairs((a->Sq + 511) / 512 * a->Hq * a->B);
+  plan->dq_ds_pairs = a->causal && ds_bytes_for(a) > 0 && dq_ds_pairs(dq_ds_workgroups(a));
   pith_attn_bwd_args bf16 = *a;
   bf16.ds = nullptr;
   bf16.dq_dtype = bf16.dkv_dtype = PITH_BF16;
@@ -455,7 +461,7 @@ extern "C" int pith_attn_bwd_chunks_plan(const pith_attn_bwd_args* args, const p
   all.dq_dtype = all.dkv_dtype = PITH_BF16;
   plan->dkdv_rows = kBN;
   plan->dkdv_split = pick_chunks_split(all, tiles);
-  plan->dq_ds_pairs = 0;
+  plan->dq_ds_pairs = pith_attn_bwd_chunks_ds_bytes(args, chunks, n) > 0 && dq_ds_pairs(dq_ds_workgroups(args));
   plan->one_grid = chunk_grids(&all, tiles, plan->dkdv_split, tiles * all.Hkv * all.B * plan->dkdv_split).one;
   return PITH_OK;
 }

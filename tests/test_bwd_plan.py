@@ -19,10 +19,10 @@ def _plan(b, sq, skv, hq, hkv, causal, d=128):
     return plan
 
 
-def _share_plan(b, s, hq, hkv, cp, rank, layout):
+def _share_plan(b, s, hq, hkv, cp, rank, layout, d=64):
     steps = sorted(ring_schedule(rank, cp, s, layout), key=lambda st: (st.kv_rank == rank, st.q_rows[0]))
     chunks = (_C.KeyChunk * len(steps))(*(_C.KeyChunk(rows=st.kv_rows[1] - st.kv_rows[0], q_row0=st.q_rows[0]) for st in steps))
-    args, plan = _C.AttnBwdArgs(B=b, Sq=s, Skv=s, Hq=hq, Hkv=hkv, Dqk=64, Dv=64), _C.AttnBwdPlan()
+    args, plan = _C.AttnBwdArgs(B=b, Sq=s, Skv=s, Hq=hq, Hkv=hkv, Dqk=d, Dv=min(d, 128)), _C.AttnBwdPlan()
     _C.check(_C.lib().pith_attn_bwd_chunks_plan(_C.byref(args), chunks, len(steps), _C.byref(plan)))
     return plan
 
@@ -30,7 +30,7 @@ def _share_plan(b, s, hq, hkv, cp, rank, layout):
 def test_plan_query():
     assert (_plan(1, 8192, 4096, 32, 4, 0).dkdv_rows, _plan(1, 256, 256, 8, 2, 1).dkdv_rows, _plan(1, 8192, 8192, 16, 16, 1, 192).dkdv_rows) == (256, 128, 128)
     assert _plan(1, 256, 256, 8, 2, 1).dkdv_split == 4
-    assert not _plan(1, 4096, 4096, 32, 4, 0).dq_ds_pairs and not _plan(1, 4096, 4096, 16, 16, 1, 192).dq_ds_pairs
+    assert not _plan(1, 4096, 4096, 32, 4, 0).dq_ds_pairs and _plan(1, 4096, 4096, 16, 16, 1, 192).dq_ds_pairs
     for bad in (dict(B=1, Sq=1, Skv=1, Hq=3, Hkv=2), dict(B=0, Sq=1, Skv=1, Hq=1, Hkv=1)):
         assert _C.lib().pith_attn_bwd_plan(_C.byref(_C.AttnBwdArgs(**bad)), _C.byref(_C.AttnBwdPlan())) == -2
     assert _C.lib().pith_attn_bwd_plan(None, None) == -1
@@ -76,6 +76,14 @@ def test_dq_from_ds_goes_out_in_the_order_that_ends_first(tiles, heads):
     assert chosen <= 1.1 * min(consecutive, pairs)
     if tiles * heads <= UNITS:
         assert chosen == pairs
+
+
+@pytest.mark.parametrize("pairs,b,s,h", [(1, 1, 4096, 16), (1, 1, 3072, 16), (1, 4, 1024, 16), (1, 1, 16384, 4), (1, 1, 129, 1), (0, 1, 4097, 16), (0, 1, 4608, 16),
+                                         (0, 3, 1999, 16), (0, 1, 8192, 16), (0, 17, 255, 16), (0, 1, 128, 16)])  # fmt: skip
+def test_order_of_dq_from_ds_at_192(pairs, b, s, h):
+    """256-row workgroups, one round of which takes pairs of 128-row blocks; 128 rows have no hand-over. A share orders its rows alike."""
+    assert _plan(b, s, s, h, h, 1, 192).dq_ds_pairs == pairs and not _plan(b, s, s, h, h, 0, 192).dq_ds_pairs
+    assert _share_plan(b, s, h, h, 4, 2, "contiguous", 192).dq_ds_pairs == pairs and not _share_plan(b, s, h, h, 4, 2, "contiguous").dq_ds_pairs
 
 
 @pytest.mark.parametrize("b,s,hq", [(1, 4096, 32), (2, 2048, 32), (8, 512, 32), (1, 8192, 16), (1, 9216, 16), (3, 1536, 32), (2, 2560, 32), (1, 5120, 32),

@@ -220,6 +220,36 @@ def test_consecutive_rows_equal_pairs(gpu, B, S):
         assert pairs and torch.equal(whole[b : b + 1], one), f"batch element {b}"
 
 
+@pytest.mark.parametrize("heads", [1, 3])
+@pytest.mark.parametrize("S", [129, 255, 513, 1024, 1100])
+def test_consecutive_rows_equal_pairs_192(gpu, S, heads):
+    """The same of 192 features, at either side of one round of this device's units (256-row workgroups, pairs of 128-row blocks)."""
+    from pithtrain_amd import _C
+
+    units = torch.cuda.get_device_properties(gpu).multi_processor_count
+    B = units // (heads * -(-S // 256)) + 1
+    g = torch.Generator(device=gpu).manual_seed(S)
+    t = lambda d: torch.randn(B, S, heads, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v, dout = t(192), t(192), t(128), t(128)
+    o, lse = _mla_fwd(q, k, v, 0.07, True)
+    delta = _mla_bwd_preprocess(o, dout)
+
+    def dq_of(*x):
+        args, plan = _C.AttnBwdArgs(B=x[0].shape[0], Sq=S, Skv=S, Hq=heads, Hkv=heads, Dqk=192, Dv=128, causal=1), _C.AttnBwdPlan()
+        _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+        ds = torch.full((attn_bwd_ds_bytes(*x[:3], True),), 0x7F, dtype=torch.uint8, device=gpu)
+        dk, dv, dq = torch.empty_like(x[1]), torch.empty_like(x[2]), torch.full_like(x[0], float("nan"))
+        attn_bwd_dkdv_into(*x, dk, dv, 0.07, True, ds=ds)
+        attn_bwd_dq_into(*x, dq, 0.07, True, ds=ds)
+        return dq, plan.dq_ds_pairs
+
+    whole, pairs = dq_of(q, k, v, dout, lse, delta)
+    assert not pairs
+    most, pairs = dq_of(*[x[1:] for x in (q, k, v, dout, lse, delta)])
+    one, pairs_one = dq_of(*[x[:1] for x in (q, k, v, dout, lse, delta)])
+    assert pairs and pairs_one and torch.equal(whole[1:], most) and torch.equal(whole[:1], one)
+
+
 @pytest.mark.parametrize("shape", NONCAUSAL_SHAPES)
 def test_noncausal_dq_from_ds(gpu, shape):
     _run(gpu, False, shape, torch.bfloat16)
