@@ -577,11 +577,13 @@ bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const st
   return rows >= 2048 && handed == all && (rows + 511) / 512 * hq * b >= 2 * cus && full_lost <= 1.05 * full;
 }
 
-// Whether any step of a share of (192, 128) could hand dS over, by its grids (steps: a chunk under the mask, whole, half its keys, half the rows).
-bool step_of_192_hands_over(const Tensor& q, int64_t hkv) {
-  const int64_t b = q.size(0), s = q.size(1), hq = q.size(2), cus = compute_units(q.device().index());
-  return ds_handover_pays_192(b, s, s, hq, hkv, true, cus) || ds_handover_pays_192(b, s, s, hq, hkv, false, cus) ||
-         ds_handover_pays_192(b, s, s / 2, hq, hkv, false, cus) || ds_handover_pays_192(b, s / 2, s, hq, hkv, false, cus);
+// Whether any step of a share of (192, 128) could hand dS over, by its grids: its own chunk under the mask, and of the others whole chunks
+// (contiguous), half the keys of those in front and half the rows against those behind (zigzag).
+bool step_of_192_hands_over(int64_t b, int64_t s, int64_t hq, int64_t hkv, int64_t rank, int64_t cp, bool zigzag, int64_t cus) {
+  const auto pays = [&](int64_t rows, int64_t keys, bool causal) { return ds_handover_pays_192(b, rows, keys, hq, hkv, causal, cus); };
+  if (pays(s, s, true)) return true;
+  if (!zigzag) return rank > 0 && pays(s, s, false);
+  return (rank > 0 && pays(s, s / 2, false)) || (rank < cp - 1 && pays(s / 2, s, false));
 }
 
 Three attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& dout, double scale, bool causal) {
@@ -970,7 +972,7 @@ struct RingFunction : torch::autograd::Function<RingFunction> {
     // Whether a share or its steps hand dS over is the Python body's decision where they could.
     const bool whole_keys = q.size(3) == 128 || (q.size(3) == 192 && !part_two(lists));
     if (share_ds_bytes(q, lists[0], lists[1], part_two(lists), rank, cp, zigzag) == 0 &&
-        (!whole_keys || (q.size(3) == 192 && !step_of_192_hands_over(q, lists[0][0]->size(2)))))
+        (!whole_keys || (q.size(3) == 192 && !step_of_192_hands_over(q.size(0), q.size(1), q.size(2), lists[0][0]->size(2), rank, cp, zigzag, compute_units(q.device().index())))))
       g = ring_backward(grads[0], q, out, lse, lists[0], lists[1], part_two(lists), scale, rank, cp, zigzag, {});
     if (!g) g = python_body<RingGrads>("ring_backward_local", grads[0], q, out, lse, lists[0], lists[1], scale, rank, cp, zigzag, part_two(lists));
     variable_list r = {std::get<0>(*g)};
@@ -1121,6 +1123,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("share_backward_in_one", &share_backward_in_one);
   m.def("ds_handover_pays", &ds_handover_pays);
   m.def("ds_handover_pays_192", &ds_handover_pays_192);
+  m.def("step_of_192_hands_over", &step_of_192_hands_over);
   m.def("share_hands_over", &share_hands_over, py::arg("b"), py::arg("rows"), py::arg("hq"), py::arg("hkv"), py::arg("steps"), py::arg("cus"),
         py::arg("dqk") = 128);
 }

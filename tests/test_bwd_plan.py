@@ -136,6 +136,19 @@ def test_shares_of_192_that_hand_over(b, s, h, pays):
     assert native.share_of_192_pays(b, s, h, UNITS) == bool(pays) and not native.share_of_192_pays(b, s, h, 0)
 
 
+@pytest.mark.parametrize("layout", ["zigzag", "contiguous"])
+@pytest.mark.parametrize("b,s,h", [(1, 2048, 16), (1, 2176, 16), (1, 2560, 16), (1, 4096, 16), (1, 4098, 16), (1, 8194, 16), (1, 1024, 16), (1, 8192, 4), (4, 512, 16), (2, 2050, 64)])
+def test_share_of_192_is_looked_at_in_python_where_one_of_its_steps_hands_over(b, s, h, layout):
+    """2048 and 2176 rows x 16 heads: whole chunks would, the half chunks of a zigzag share do not."""
+    for cp in (1, 2, 4):
+        for rank in range(cp):
+            sizes = [(st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0], st.causal) for st in ring_schedule(rank, cp, s, layout)]
+            want = any(native.ds_handover_pays_192(b, m, n, h, h, c, UNITS) for m, n, c in sizes)
+            assert native.step_of_192_hands_over(b, s, h, h, rank, cp, layout == "zigzag", UNITS) == want, (cp, rank)
+            if s in (2048, 2176):
+                assert want == (layout == "contiguous" and rank > 0)
+
+
 def test_bytes_of_a_share_that_hands_over():
     """All chunks, a query tile of one lying within its images: 128 rows and keys of a half, their own chunk under the mask last."""
     def need(sq, chunks, dqk=192):
