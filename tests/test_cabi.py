@@ -395,6 +395,19 @@ def test_ds_storing_dkdv_kernel_of_192_waits_for_its_tile_loads_only(tmp_path_fa
         assert sum(o.startswith("global_store") for o in ops) == 4
 
 
+def test_results_leave_by_both_kinds_of_stores(tmp_path_factory):
+    """bf16 rows are stored plainly or non-temporally by the size of the result: every kernel has as many stores of either kind (the
+    compiler would make one plain store of the two)."""
+    for src in ("attn_fwd_direct.hip", "attn_fwd_duo.hip", "attn_bwd_dkdv_d192.hip", "attn_bwd_dkdv_d128.hip", "attn_bwd_dkdv_wide.hip"):
+        text = _kernel_asm(src, tmp_path_factory.getbasetemp())
+        for name, body in re.findall(r"^(_Z\w+kernel\w*):(.*?)^\.Lfunc_end", text, re.M | re.S):
+            if "dkdv" in src and not re.search(r"kernelILb[01]EDF16b", name):
+                continue  # fp32 results
+            through = len(re.findall(r"\tglobal_store_dwordx2 .* nt$", body, re.M))
+            plain = len(re.findall(r"\tglobal_store_dwordx2 (?!.* nt$)", body, re.M))
+            assert through and plain >= through, (name, plain, through)
+
+
 def test_split_key_dq_requests_no_tile_over_one_still_read(tmp_path_factory):
     """The split-key dQ kernel scores tile 0 ahead of its loop and then requests tiles into slots that other waves read for
     that (V of tile 2 at 192 features, the staged rows at 128). Followed over the control flow of the compiler's output: between
