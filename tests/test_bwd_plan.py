@@ -211,6 +211,20 @@ def test_shares_that_hand_over_go_out_step_by_step_where_that_is_faster(steps, b
     assert native.share_hands_over(b, s, hq, hkv, sizes, UNITS) == bool(steps)
 
 
+@pytest.mark.parametrize("steps,b,s,h,cp,rank,layout", [
+    (1, 1, 8192, 16, 4, 2, "zigzag"), (1, 1, 10240, 16, 4, 2, "zigzag"), (1, 1, 9216, 16, 4, 2, "contiguous"), (1, 1, 12288, 16, 2, 0, "zigzag"),
+    (1, 1, 7170, 16, 4, 1, "zigzag"), (1, 2, 4098, 32, 4, 3, "zigzag"), (1, 16, 2048, 16, 4, 1, "zigzag"), (1, 16, 2050, 16, 4, 1, "zigzag"),
+    (1, 8, 3072, 16, 4, 2, "contiguous"), (1, 8, 2306, 16, 4, 2, "zigzag"), (1, 4, 4096, 16, 4, 3, "contiguous"), (1, 1, 16384, 8, 4, 2, "zigzag"),
+    (0, 1, 4098, 16, 4, 2, "zigzag"), (0, 1, 3074, 16, 4, 2, "zigzag"), (0, 1, 3074, 16, 2, 0, "zigzag"), (0, 64, 1024, 16, 4, 2, "zigzag"), (0, 1, 2560, 32, 4, 2, "zigzag"),
+    (0, 1, 8194, 16, 4, 2, "zigzag"), (0, 1, 9216, 16, 4, 2, "zigzag"), (0, 1, 5122, 16, 4, 1, "zigzag"),
+])  # fmt: skip
+def test_shares_of_192_that_go_out_step_by_step(steps, b, s, h, cp, rank, layout):
+    """The same at 192 features (asked where the share as a whole does not hand over): step by step only where that measured faster."""
+    sizes = [(st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0], st.causal) for st in ring_schedule(rank, cp, s, layout)]
+    sizes = [(m, n, c, h if native.ds_handover_pays_192(b, m, n, h, h, c, UNITS) else 0) for m, n, c in sizes]
+    assert native.share_hands_over(b, s, h, h, sizes, UNITS, 192) == bool(steps)
+
+
 def test_share_of_slabs_counts_their_grids():
     """131072 tokens, 64/4 heads: a slab of one kv head at a time fills the device; a quarter of its heads would not."""
     sizes = lambda heads: [(16384, 8192, False, heads)] * 3 + [(8192, 16384, False, heads)] * 4 + [(16384, 16384, True, 0)]  # noqa: E731

@@ -395,6 +395,28 @@ def test_ds_storing_dkdv_kernel_of_192_waits_for_its_tile_loads_only(tmp_path_fa
         assert sum(o.startswith("global_store") for o in ops) == 4
 
 
+def test_ds_storing_dkdv_kernel_of_chunks_waits_for_its_tile_loads_only(tmp_path_factory):
+    """The same of the chunk kernel, which spills a register: outside the loop, where its traffic does not count in the wait."""
+    text = _kernel_asm("attn_bwd_chunks.hip", tmp_path_factory.getbasetemp())
+    (body,) = re.findall(r"^_Z\w*attn_bwd_dkdv_chunks_kernelILi192ELb1EE\w*:(.*?)^\.Lfunc_end", text, re.M | re.S)
+    lines = body.splitlines()
+    (wait,) = [i for i, l in enumerate(lines) if re.search(r"s_waitcnt vmcnt\(4\)\s*$", l) and "s_barrier" in lines[i + 1]]
+    head = max(i for i in range(wait) if "Inner Loop Header" in lines[i])
+    label = re.match(r"\.L(BB\d+_\d+):", lines[head]).group(1)
+    memory = r"\s+(global_|scratch_|buffer_|flat_)"
+    ops = [l.split()[0] for l in lines[head:wait] if re.match(memory, l)]
+    assert ops[-4:] == ["global_store_dwordx4"] * 4 and all(o.startswith("global_load_lds") for o in ops[:-4]) and len(ops) > 4, ops
+    # behind the wait: the branch back, and blocks of the loop that the compiler placed out of line (requests of ragged tiles)
+    inside = True
+    for l in lines[wait + 1 :]:
+        if re.match(r"\.LBB\d+_\d+:|; %bb", l):
+            inside = f"Loop: Header={label} " in l
+        elif inside and re.match(memory, l):
+            assert "global_load_lds" in l, l
+        elif inside and re.match(rf"\s+s_c?branch\w* \.L{label}$", l):
+            inside = False
+
+
 def test_results_leave_by_both_kinds_of_stores(tmp_path_factory):
     """bf16 rows are stored plainly or non-temporally by the size of the result: every kernel has as many stores of either kind (the
     compiler would make one plain store of the two)."""

@@ -98,23 +98,34 @@ def test_dq_from_ds_192(gpu, causal, shape, dtype):
 @pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
 def test_ring_share_of_192_with_and_without_handover(gpu, layout, monkeypatch):
     """Steps that hand dS over (fp32 dQ added to and finished by their kernels) against one launch that recomputes: the same bf16 dS
-    values summed in other orders, up to one bf16 step (2^-8) of the largest element."""
+    values summed in other orders, up to one bf16 step (2^-8) of the largest element; and two heads against the oracle."""
     from pithtrain_amd.operators.mla import hip as H
     from pithtrain_amd.operators.ring_attention import local as L
 
     g = torch.Generator(device=gpu).manual_seed(5)
     t = lambda h, d: torch.randn(1, 2050, h, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
     q, dout, ks, vs = t(16, 192), t(16, 128), [t(16, 192) for _ in range(3)], [t(16, 128) for _ in range(3)]
+    visited = len(L.ring_schedule(1, 3, 2050, layout))
     ks, vs = (ks, vs) if layout == "zigzag" else ([*ks[:2], None], [*vs[:2], None])
     out, lse = L.ring_forward_local(q, ks, vs, 0.07, 1, 3, layout)
     monkeypatch.setattr(L, "_handover_pays", lambda *a: True)
     monkeypatch.setattr(H, "ds_plan", lambda q, k, v, causal=False: (16, attn_bwd_ds_bytes(q, k, v, causal)))
+    used, pair = [], H.attn_bwd_pair_into
+    monkeypatch.setattr(L, "attn_bwd_pair_into", lambda *a, **kw: used.append(pair(*a, **kw)) or used[-1])
     steps = L.ring_backward_local(dout, q, out, lse, ks, vs, 0.07, 1, 3, layout)
+    assert len(used) == visited and all(used), "every step hands its dS over"
     monkeypatch.setattr(L, "_handover_pays", lambda *a: False)
     one = L.ring_backward_local(dout, q, out, lse, ks, vs, 0.07, 1, 3, layout)
+    assert len(used) == visited and not torch.equal(steps[0], one[0])
     flat = lambda r: [r[0], *(x for l in r[1:3] for x in l if x is not None)]  # noqa: E731
     for a, b in zip(flat(steps), flat(one), strict=True):
         assert norm_max_err(a.float(), b.float()) < 6e-3
+    two = lambda x: None if x is None else x[:, :, 6:8].cpu()  # noqa: E731
+    host = two(q), [two(x) for x in ks], [two(x) for x in vs]
+    o_ref, lse_ref = R.ring_forward(*host, 0.07, 1, 3, layout)
+    want = R.ring_backward(two(dout), host[0], o_ref, lse_ref, *host[1:], 0.07, 1, 3, layout)
+    for name, a, b in zip(["dQ", *[f"{n}{j}" for n in ("dK", "dV") for j in range(visited)]], flat(steps), flat(want), strict=True):
+        check_bf16_result(a[:, :, 6:8], b, f"ring {name}", otol=1e-3)
 
 
 @pytest.mark.parametrize("b,s,h,cp,rank,layout,two_parts", [
@@ -381,15 +392,16 @@ def test_default_policy_of_the_buffer(gpu, monkeypatch):
     assert H.ds_plan(q, k, k) == (1, 4 << 30)
 
 
+@pytest.mark.parametrize("dqk", [128, 192])
 @pytest.mark.parametrize("causal", [False, True])
-def test_slabs_of_kv_heads_equal_the_whole_call(gpu, causal, monkeypatch):
+def test_slabs_of_kv_heads_equal_the_whole_call(gpu, causal, dqk, monkeypatch):
     """attn_bwd_pair_into through a buffer that holds one or two kv heads at a time (head ranges of the full
     tensors, passed in place) gives dK/dV bit for bit and dQ bit for bit what the whole-pair hand-over gives."""
     from pithtrain_amd.operators.mla import hip as H
 
     B, Sq, Hq, Hkv = 2, 1024, 16, 4
     Skv = Sq if causal else 640
-    q, k, v, dout, scale = _inputs(B, Sq, Skv, Hq, Hkv, seed=11)
+    q, k, v, dout, scale = _inputs(B, Sq, Skv, Hq, Hkv, seed=11, dqk=dqk)
     qd, kd, vd, dod = (t.to(gpu) for t in (q, k, v, dout))
     o, lse = _mla_fwd(qd, kd, vd, scale, causal)
     delta = _mla_bwd_preprocess(o, dod)
@@ -402,6 +414,12 @@ def test_slabs_of_kv_heads_equal_the_whole_call(gpu, causal, monkeypatch):
         used = H.attn_bwd_pair_into(qd, kd, vd, dod, lse, delta, dq, dk, dv, scale, causal, accumulate_dq=True)
         assert used == need // Hkv * heads
         results.append((dq, dk, dv))
+        # rows that are finished by the call go out as bf16, the others stay in fp32
+        part, final = torch.full_like(dq, 0.25), torch.full_like(qd, 7.0)
+        H.attn_bwd_pair_into(qd, kd, vd, dod, lse, delta, part, dk, dv, scale, causal, accumulate_dq=True, dq_final=final, dq_final_rows=(320, 992))
+        assert torch.equal(final[:, 320:992], dq[:, 320:992].to(torch.bfloat16)) and (part[:, 320:992] == 0.25).all()
+        for rows in (slice(0, 320), slice(992, Sq)):
+            assert torch.equal(part[:, rows], dq[:, rows]) and (final[:, rows] == 7).all()
     for dq, dk, dv in results[1:]:
         assert torch.equal(dq, results[0][0]) and torch.equal(dk, results[0][1]) and torch.equal(dv, results[0][2])
     rdq, rdk, rdv = R.chunk_bwd(q, k, v, dout, lse.double().cpu(), delta.double().cpu(), scale, causal)
@@ -575,3 +593,46 @@ def test_misaligned_buffer(gpu, head_dim):
         else:
             assert codes == [_C.PITH_OK] * len(calls) and all(torch.equal(x, y) for x, y in zip(got, results))
     assert (ds == 0x7F).all()
+
+
+@pytest.mark.parametrize("S", [1024, 1000])
+@pytest.mark.parametrize("head_dim", [128, 192])
+def test_infinity_reaches_the_rows_that_it_reaches_without_handover(gpu, head_dim, S):
+    """An infinity in K or V of one key (LSE and delta are those of finite ones): rows before the key's 64-row tile do not see it, and dQ
+    from dS is not finite exactly where the recomputing kernel's is not. dK and dV bit for bit."""
+    q, k, v, dout, scale = (t.to(gpu) if torch.is_tensor(t) else t for t in _inputs(1, S, S, 2, 2, dqk=head_dim))
+    o, lse = _mla_fwd(q, k, v, scale, True)
+    delta = _mla_bwd_preprocess(o, dout)
+    for which in (1, 2):
+        for key in (0, 33, 64, 95, 127, 128, 300, 999):
+            x = [q, k.clone(), v.clone(), dout, lse, delta]
+            x[which][:, key, :, 5] = float("inf")
+            runs = []
+            for ds in (None, torch.full((attn_bwd_ds_bytes(*x[:3], True),), 0x7F, dtype=torch.uint8, device=gpu)):
+                dk, dv, dq = torch.empty_like(k), torch.empty_like(v), torch.empty_like(q)
+                attn_bwd_dkdv_into(*x, dk, dv, scale, True, ds=ds)
+                attn_bwd_dq_into(*x, dq, scale, True, ds=ds)
+                runs.append((dq, dk, dv))
+            finite = [r[0].isfinite().all(-1) for r in runs]
+            assert torch.equal(*finite) and finite[0][:, : key // 64 * 64].all() and not finite[0][:, key:].all(), (which, key)
+            assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(runs[0][1:], runs[1][1:])), (which, key)
+
+
+@pytest.mark.parametrize("magnitude", [1e4, 1e18])
+def test_large_values_at_masked_keys(gpu, magnitude):
+    """Rows of one 64-row tile see none of the next tile's keys, however large their scores and values are."""
+    S = 512
+    q, k, v, dout, scale = (t.to(gpu) if torch.is_tensor(t) else t for t in _inputs(1, S, S, 2, 2, dqk=192))
+    dqs = []
+    for factor in (1.0, magnitude):
+        kx, vx = k.clone(), v.clone()
+        kx[:, 320:] *= factor
+        vx[:, 320:] *= factor
+        o, lse = _mla_fwd(q, kx, vx, scale, True)
+        delta = _mla_bwd_preprocess(o, dout)
+        ds = torch.full((attn_bwd_ds_bytes(q, kx, vx, True),), 0x7F, dtype=torch.uint8, device=gpu)
+        dk, dv, dq = torch.empty_like(k), torch.empty_like(v), torch.empty_like(q)
+        attn_bwd_dkdv_into(q, kx, vx, dout, lse, delta, dk, dv, scale, True, ds=ds)
+        attn_bwd_dq_into(q, kx, vx, dout, lse, delta, dq, scale, True, ds=ds)
+        dqs.append(dq)
+    assert torch.equal(dqs[0][:, :320], dqs[1][:, :320])
