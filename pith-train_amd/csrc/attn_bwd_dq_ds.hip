@@ -22,10 +22,11 @@
 // from transposing reads of the image, in the same key slot order. The accumulators therefore hold
 // dQ untransposed (a lane owns one feature column of 16 rows) and the epilogue reads and writes whole
 // 128-byte lines (store_rows32).
-// The images are read once, by one workgroup, and all of them exceed every cache: loaded non-temporally they leave the caches to K
-// and to what the dK/dV launch wrote last. The kernel alone over 4096 x 32/4 heads, plain / non-temporal: under the mask 118 / 99
+// The images are read once, by one workgroup: loaded non-temporally they leave the caches to K and to what the dK/dV launch wrote last.
+// The kernel alone over 4096 x 32/4 heads, plain / non-temporal: under the mask 118 / 99
 // us, without 196 / 169 (6.4 TB/s); with the dK/dV launch before it (the same rows) 436 / 422, 8192 x 32/4 1584 / 1559, 3 x 1999 x 32/4
-// 363 / 348, 4 x 1024 x 32/4 152.5 / 151.6. Past the vector cache only (sc1), or past more than that (sc0 nt, sc1 nt, sc0 sc1 nt): 0-3 %
+// 363 / 348, 4 x 1024 x 32/4 152.5 / 151.6. So where all images fit the 256 MB last-level cache: backward of 16 heads of 192/128, 8 x 512 (40 MiB)
+// 68.5 / 67.2, 3 x 1021 (54) 77.9 / 73.2, 4 x 1024 (72) 95.5 / 93.3, 2 x 2048 (136) 151 / 146. Past the vector cache only (sc1), or past more than that (sc0 nt, sc1 nt, sc0 sc1 nt): 0-3 %
 // slower than nt.
 // (192, 128): accumulators for 512 rows do not fit, so a workgroup owns 256 rows (under the mask in one round two blocks of 128), and
 // two neighbouring waves share a 64-row tile, each with 96 of the features (either block's four waves lie on four SIMDs: with a tile's
@@ -398,6 +399,13 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dq_ds_kernel(BwdArgs<MULTI>
 //   1.25, 1.5, 1.75   5120 x 32/4 196 / 225, 6144 x 32/4 256 / 271, 3 x 1999 x 32/4 102 / 114, 7168 x 32/4 322 / 337
 //   2, 2.25           8192 x 32/4 405 / 409, 2 x 4096 x 32/4 224 / 233, 9216 x 32/4 517 / 599
 //   2.75, 3, 4        11264 x 32/4 785 / 799, 12288 x 32/4 921 / 904, 3 x 4096 x 32/4 341 / 353, 16384 x 32/4 1524 / 1565
+// 256 rows of 192 features, 16 heads unless others are named, the same:
+//   up to one round   3072 71 / 54, 4096 100 / 80, 2 x 2048 55 / 45, 4 x 1024 33 / 29, 8 x 512 22 / 20, 16384 x 4 368 / 283
+//   1.12-2            4608 114 / 142, 5120 129 / 159, 3 x 1999 62 / 79, 6144 160 / 194, 8192 248 / 279, 1024 x 128 51 / 56
+//   2.25-8            9216 328 / 412, 12288 568 / 608, 4096 x 64 266 / 300, 4096 x 128 564 / 609
+// and shares of four ranks, rank 1, whose rows walk the other chunks at equal length (backward without delta, zigzag and contiguous):
+//   up to one round   3072 620 / 571 and 431 / 418, 4096 1004 / 948 and 697 / 680, in two parts 1015 / 958, 4 x 1024 329 / 314 and 224 / 220
+//   1.12-2            4608 1234 / 1363 and 902 / 974, 5120 1481 / 1620 and 1088 / 1152, 6144 2042 / 2190 and 1538 / 1587, 8192 3520 / 3646 and 2644 / 2660
 bool dq_ds_pairs(int64_t workgroups) { return workgroups <= compute_units_or_default(); }
 
 void launch_dq_from_ds(BwdParams p, int dqk, bool causal, bool f32_out, hipStream_t st) {

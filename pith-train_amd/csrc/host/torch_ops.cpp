@@ -395,7 +395,12 @@ bool share_backward_in_one(int64_t dqk, int64_t rows, int64_t heads, int64_t chu
 //   W 0.75  3072 x 16 567 / 640 and 679 / 777, 12032 x 4 2055 / 2326 and 2466 / 2873, 2 x 1536 x 16 313 / 349 and 361 / 418
 //   W 1     4096 x 16 948 / 1052 and 678 / 790, 8 ranks 1825 / 2066 and 2444 / 2801, 2 x 2048 x 16 519 / 568 and 361 / 422, 4 x 1024 x 16 310 / 336 and
 //           209 / 244, 16384 x 4 3575 / 4007 and 2630 / 3008    W 1.25-2   5120 x 16, 2 ranks 740 / 838, 6144 x 16 2054 / 2322, 8192 x 16, 2 ranks 1776 / 2017
-// Keys in two parts the same: 4096 x 16 969 / 1063, 4 x 1024 x 16 316 / 344. Shorter rows were not measured at W 0.7 and more.
+// Keys in two parts the same: 4096 x 16 969 / 1063, 4 x 1024 x 16 316 / 344. Rows below 1024 gain on the device as well, W 1-2, zigzag and contiguous: 4 x
+// 896 x 16 257 / 280 and 180 / 203, 8 x 640 x 16 295 / 321 and 207 / 233, 8 x 512 x 16 212 / 225 and 146 / 165, 512 x 128 213 / 226 and 152 / 170 (16 x 256 x 16
+// zigzag loses, 194 / 190). The line was drawn before these were measured and has not been weighed against the host: the Python body, which owns the
+// buffer, takes 136 us of its time, the native one 108, about as long as the shorter of these kernels. A zigzag share whose half chunk is no multiple of 64 rows has no such hand-over (a 64-row tile would
+// lie across two images, pith_attn_bwd_chunks_ds_bytes) and pays 13 % of its backward: 4160 x 16 1198, recomputing, where 4224 x 16 takes
+// 1040 (1220 recomputing); 6146 x 16 2355 beside 1988 for 6144, 2 x 2050 x 16 660 beside 508 for 2 x 2048 (both with a further round).
 bool share_of_192_pays(int64_t b, int64_t rows, int64_t hq, int64_t cus) { return cus > 0 && rows >= 1024 && 10 * ((rows + 255) / 256 * hq * b) >= 7 * cus; }
 int64_t share_ds_bytes(const Tensor& q, const std::vector<OptTensor>& ks, const std::vector<OptTensor>& vs, const std::optional<std::vector<OptTensor>>& pes,
                        int64_t rank, int64_t cp, bool zigzag) {
@@ -516,8 +521,8 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
 //   full    F below 0.75  2048 x 1024 85 / 74, 8192 x 4096 x 4 292 / 268, 2731 x 1366 127 / 140    W 0.25  1024 x 2048 91 / 84, 4096 x 8192 x 4 313 / 290
 //           W 0.5         2048 x 2048 128 / 139, 2 x 1024 x 2048 134 / 144, 8192 x 16384 x 4 942 / 994
 //           W 0.6-1.25    2560 x 5120 391 / 428, 3072 x 1536 138 / 155, 3072 x 6144 507 / 604, 2 x 2048 x 1024 117 / 139, 5120 x 2560 426 / 503
-// Below 2^25 visible pairs of rows and heads the device gains as much, but the Python body of such a call takes longer than its kernels:
-// forward + backward with the host's time 8 x 512 causal 93-120 / 102, 512 x 128 99-123 / 111; 4 x 1024 127 / 140.
+// Below 2^25 visible pairs of rows and heads the device gains as much, but the Python body of such a call takes longer than its kernels, on the
+// host of one machine: forward + backward with the host's time 8 x 512 causal 93-120 / 102, 512 x 128 99-123 / 111; 4 x 1024 127 / 140.
 bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
   if (cus <= 0 || b * hq * sq * skv < (int64_t)(causal ? 64 : 32) << 20 || 10 * ((sq + 255) / 256 * hq * b) < (causal ? 7 : 5) * cus) return false;
   pith_attn_bwd_args a = {};
@@ -547,6 +552,14 @@ bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_
 // four dQ workgroups per unit on, and where dQ, two workgroups to a unit, leaves its last round half empty, the steps are faster from a
 // quarter of the work on: two ranks, rank 0 4352 x 32/4 1058 / 1183, 20480 x 8/2 4975 / 5452, 2560 x 64/4 720 / 748, four ranks 1413 / 1555, 5120 x 32/4 2629 /
 // 3013, 2304 x 64/4 1231 / 1303, 2 x 2304 x 32 1253 / 1259; whole rounds 3072 x 64/4 1021 / 977, four ranks 2067 / 2031.
+// 192 features are asked only where the share as a whole does not hand over (share_of_192_pays, images beyond the buffer's limit, half chunks
+// off the 64-row grid). The limits are those of 128 features: wherever they choose the steps these are faster, and what they leave out is mostly
+// even. 16 heads, four ranks, rank 2 zigzag and contiguous unless others are named:
+//   chosen     8192 3510 / 3798 and 4298 / 4692, 10240 5738 / 5993 and 6823 / 7755, 16384 x 8 6743 / 7422 and 8350 / 9251, 9216 contiguous 5796 / 6460, 12288 in slabs
+//              of 8 heads contiguous 9822 / 10598, 8192 x 64/4 in slabs of 2 kv heads 14300 / 16940, 16 x 2048 4907 / 5001 and 5994 / 6372, 8 x 3072 4715 / 4944 and
+//              5589 / 6000; half chunks off the grid: 7170 2935 / 3125, 2 x 4098 x 32 4307 / 4485, 16 x 2050 5408 / 5567, 8 x 2306 3111 / 3142
+//   left out   4098 1332 / 1115, 3074 703 / 670, 64 x 1024 7357 / 6247, 2560 x 32 950 / 840, 9216 4903 / 4971, 5122 1724 / 1766, 8194 4148 / 4198; two ranks, rank 0, 3074 368 /
+//              342, 4098 604 / 622, 8194 1972 / 2270
 bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const std::vector<std::array<int64_t, 4>>& steps, int64_t cus, int64_t dqk) {
   if (cus <= 0 || hkv <= 0) return false;
   const auto lost = [&](int64_t wgs, int per_unit = 1) {

@@ -197,10 +197,11 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
     args.ds, args.ds_bytes = ds.data_ptr(), ds.numel()
 
 
-# The dS hand-over (head dims 128/128 and 192/128) makes the backward of a chunk pair 1-5 % faster (share of 8192 rows, 32/4 heads,
-# four ranks: 6.15 -> 5.92 ms; the gain differs between machines) at the price of a transient buffer of
-# Sq*Skv*Hq*B*2 bytes while the pair's two kernels run (about half under the causal mask: a layer of 4096 rows, 32/4 heads,
-# takes 0.55 GB for 3 % of its forward + backward).
+# The dS hand-over makes a backward faster (128 features 1-8 %: share of 8192 rows, 32/4 heads, four ranks 6.08 -> 5.59 ms; 192 features
+# 5-14 %: layer of 4096 rows, 16 heads, 282 -> 243 us; the gain differs between machines) at the price of a transient buffer of
+# Sq*Skv*Hq*B*2 bytes while the pair's two kernels run, about half under the causal mask: a layer of 4096 rows, 32/4 heads of 128
+# takes 0.55 GB, of 16 heads of 192/128 0.28 GB. A share of 192 features that goes out as one dK/dV and one dQ launch holds the images of all
+# its chunks at once: 4096 rows, 16 heads, four ranks, zigzag 1.08 GB.
 # Policy: the buffer never exceeds DS_BUFFER_LIMIT_BYTES nor DS_BUFFER_FREE_FRACTION of the device memory that is
 # free right now; a chunk pair that needs more is processed one group of kv heads (with their query heads) after
 # the other through one buffer of the bounded size; when not even one kv head fits, or the allocation fails, the
