@@ -25,7 +25,7 @@ struct BwdParams {
   int64_t q_bs, k_bs, v_bs, dout_bs, dq_bs, dk_bs, dv_bs, lse_bs, lse_hs;
   float kappa, scale;
   int accumulate, accumulate_dq;  // dK/dV and dQ kernels: add to what the outputs hold
-  int keep_dkv, keep_dq;          // bf16 results stay in the caches (keep_results)
+  int through_dkv, through_dq;    // bf16 results are written through (through_results)
   int split;        // dK/dV kernel: query-head groups are cut into `split` parts handled by different workgroups
   float* ws_dk;     // dK/dV kernel, split > 1: fp32 partial results [split][B][Skv][Hkv][D]
   float* ws_dv;

@@ -540,6 +540,7 @@ int run_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks,
     blocks = (unsigned)next;
   }
   p.n_chunks = (int)n;
+  p.through_dkv = through_results(rows_before * all.B * all.Hkv * (all.Dqk + all.Dv) * 2);
   p.dk_pe_bs = args->dk_pe_bs;
   p.split = split;
   const int dq_rows = hand_over ? dq_ds_rows(192) : 128;

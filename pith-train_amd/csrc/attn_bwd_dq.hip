@@ -93,8 +93,8 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
   p.scale = a->scale;
   p.kappa = a->scale * 1.44269504088896340736f;
   p.accumulate = p.accumulate_dq = 0;
-  p.keep_dkv = keep_results(a->B * a->Skv * a->Hkv * a->Dqk * 2);
-  p.keep_dq = keep_results(a->B * a->Sq * a->Hq * a->Dqk * 2);
+  p.through_dkv = through_results(a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2);
+  p.through_dq = through_results(a->B * a->Sq * a->Hq * a->Dqk * 2);
   p.split = 1;
   p.ws_dk = nullptr;
   p.ws_dv = nullptr;

@@ -472,7 +472,7 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
       __bf16* fin = nullptr;  // rows whose gradient is complete with this call go out as bf16
       if (p.dq_final != nullptr && q_wave0 >= p.final_r0 && q_wave0 < p.final_r1) fin = p.dq_final + b * p.dq_final_bs + at;
       store_rows32_via_lds<OutT, NB>(mine, reinterpret_cast<OutT*>(p.dq) + b * p.dq_bs + at, q_row_stride, p.Sq - q_wave0, part, p.scale,
-                                     p.accumulate_dq != 0, lane, p.keep_dq, fin);
+                                     p.accumulate_dq != 0, lane, p.through_dq, fin);
     };
     if (!late) finish(std::false_type{});
     else finish(std::true_type{});

@@ -425,7 +425,7 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
 #pragma unroll
     for (int o = 0; o < L::kTurnBlocks; ++o) part[o] = acc[o0 + o];
     store_rows32_via_lds<OutT, L::kTurnBlocks>(turn, rows + 32 * o0, q_row_stride, p.Sq - q_wave0, part, p.scale, p.accumulate_dq != 0, lane,
-                                               p.keep_dq, fin == nullptr ? nullptr : fin + 32 * o0);
+                                               p.through_dq, fin == nullptr ? nullptr : fin + 32 * o0);
   }
 }
 

@@ -103,7 +103,7 @@ int prepare(const pith_attn_fwd_args* a, FwdParams& p) {
   p.q = (const __bf16*)a->q; p.k = (const __bf16*)a->k; p.v = (const __bf16*)a->v;
   p.o = (__bf16*)a->o; p.lse = a->lse;
   p.Sq = (int)a->Sq; p.Skv = (int)a->Skv; p.Hq = (int)a->Hq; p.Hkv = (int)a->Hkv; p.group = (int)(a->Hq / a->Hkv);
-  p.B = (int)a->B; p.m_tiles = 0; p.keep_o = keep_results(a->B * a->Sq * a->Hq * a->Dv * 2); p.chunked = kChunkedTiles;
+  p.B = (int)a->B; p.m_tiles = 0; p.through_o = through_results(a->B * a->Sq * a->Hq * a->Dv * 2); p.chunked = kChunkedTiles;
   p.q_bs = a->q_bs; p.k_bs = a->k_bs; p.v_bs = a->v_bs; p.o_bs = a->o_bs; p.lse_bs = a->lse_bs; p.lse_hs = a->lse_hs;
   p.kappa = a->scale * 1.44269504088896340736f;
   p.k_pe = (const __bf16*)a->k_pe; p.k_pe_bs = a->k_pe_bs; p.k_pe_rs = a->k_pe_rs;

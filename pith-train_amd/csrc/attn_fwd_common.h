@@ -18,7 +18,7 @@ struct FwdParams {
   float* lse;
   int Sq, Skv, Hq, Hkv, group;  // group = Hq / Hkv
   int B, m_tiles;
-  int keep_o;   // O stays in the caches (keep_results)
+  int through_o;  // O is written through (through_results)
   int chunked;  // tiles from which the heads are taken in chunks (decode_block; 128-row workgroups only)
   int64_t q_bs, k_bs, v_bs, o_bs, lse_bs, lse_hs;
   float kappa;  // scale * log2(e)

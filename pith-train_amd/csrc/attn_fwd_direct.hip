@@ -487,7 +487,7 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
       }
     }
     // O^T sits in the accumulators (a lane owns one query row): turned through LDS so that the stores cover whole rows
-    store_rows32_via_lds<__bf16, NB>(turn, rows, o_row_stride, p.Sq - q_wave0, part, inv, false, lane, p.keep_o);
+    store_rows32_via_lds<__bf16, NB>(turn, rows, o_row_stride, p.Sq - q_wave0, part, inv, false, lane, p.through_o);
     if (B0 == 0 && qrow < p.Sq && g == 0) lse[qrow] = (l > 0.f) ? __builtin_amdgcn_logf(l) + m_run * p.kappa : -INFINITY;
   };
 

@@ -469,27 +469,29 @@ __device__ __forceinline__ bf16x8 lds_read_transposed_at(const char* lo_addr, co
 // With `accumulate` all old values are read before the first store. With `final_block` (wave-uniform; the same rows of
 // a bf16 tensor laid out like `block`) the result, old values included, is rounded to bf16 and written there, and
 // `block` keeps what it held.
-// bf16 rows are stored plainly with `keep` (keep_results), else non-temporally: workgroups that are still in their loops share K and V (Q
-// and dO) through the second-level cache; but whoever reads the result next would find it there. Through that cache (sc1 nt) as nt within
-// 0.3 %. fp32 rows are read again soon, by the sums over head parts or the next ring step: nt 0.3 % slower.
+// bf16 rows leave in one of two ways (through_results): workgroups that are still in their loops share K and V (Q and dO) through the
+// second-level cache, which plain stores fill with rows that wait there to be written. fp32 rows are read again soon, by the sums over
+// head parts or the next ring step: plain, nt 0.3 % slower.
 template <int NB>
 constexpr int kRowsViaLdsBytes = 32 * (NB * 128 + 16);
 
-// Whether a result of that many bytes is left to the second-level caches (8 x 4 MB) for its next reader. A launch alone is faster with nt, what
-// follows it slower, and the sum turns at about 16 MiB. Plain / nt with the projections that read the results next, us: forward, by the size of O
-//   2-4 MiB   1024 x 16/4 heads of 64 20.3 / 21.5, 2048 x 16/4 36.8 / 37.1, 512 x 32/4 of 128 31.2 / 32.2
-//   8 MiB     1024 x 32/4 of 128 44.7 / 45.4, 2 x 512 x 32/4 40.2 / 41.0, 2048 x 16 of 192/128 59.3 / 61.6, 4096 x 16/4 of 64 64.6 / 65.2; but
-//             2 x 2048 x 16/4 of 64 47.6 / 46.0, 8 x 512 x 16/4 28.9 / 25.9
-//   16 MiB    4 x 512 x 32/4 of 128 53.9 / 53.3, 2048 x 32/4 79.6 / 80.2, 4096 x 16 of 192/128 126.2 / 127.1
-//   32-47     8 x 512 x 32/4 of 128 93.0 / 91.2, 4096 x 32/4 187.7 / 187.8, 3 x 1999 x 32/4 186.6 / 186.3
-// backward 2048 x 16 of 192/128 184.8 / 186.8, 1024 x 32/4 of 128 105.3 / 105.1, 4096 x 32/4 523 / 523. The launch alone: forward 2 x 512 x 32/4
-// 14.5 / 13.6, 8 x 512 x 32/4 33.7 / 30.7, 4096 x 16 of 192/128 93.2 / 92.1, 3 x 1999 x 32/4 of 128 110.5 / 106.5.
-inline bool keep_results(int64_t bytes) { return bytes < (int64_t)16 << 20; }
+// Whether results of that many bytes (O, dQ, or dK and dV of a launch together) are written through the second-level caches (sc1) rather than
+// non-temporally: as long as the 8 x 4 MB of them could hold it. Either keeps the tiles of the other workgroups cached, but what went out non-temporally its next reader fetches from
+// memory. Plain / sc1 / nt, us, the forward alone and with the projection that reads O:
+//   2-4 MiB   1024 x 16/4 heads of 64 10.8 / 10.7 / 10.7 and 20.3 / 20.4 / 21.8, 512 x 32/4 of 128 11.1 / 10.7 / 10.8 and 31.8 / 29.9 / 32.5
+//   8 MiB     2 x 512 x 32/4 of 128 14.7 / 13.8 / 13.8 and 39.9 / 38.5 / 40.1, 2048 x 16 of 192/128 40.3 / 39.7 / 40.0 and 59.6 / 59.3 / 61.9, 2 x 2048 x 16/4 of 64
+//             31.2 / 30.7 / 30.5 and 47.7 / 44.8 / 45.1
+//   16 MiB    4 x 512 x 32/4 of 128 18.1 / 17.8 / 16.9 and 53.1 / 51.9 / 52.5, 4096 x 16 of 192/128 91.3 / 90.7 / 89.9 and 123.7 / 123.1 / 125.0
+//   32 MiB    8 x 512 x 32/4 of 128 33.4 / 30.3 / 30.2 and 91.2 / 88.5 / 89.7, 4096 x 32/4 126.0 / 124.3 / 124.8 and 183.9 / 181.4 / 183.9
+//   47 MiB    3 x 1999 x 32/4 of 128 106.3 / 105.2 / 102.8 and 183.8 / 183.6 / 183.2
+// and the backward with the products that read dQ, dK and dV: 512 x 32/4 of 128 71.2 / 71.0 / 72.3, 2048 x 16 of 192/128 181.0 / 181.1 / 182.7, the others within
+// 0.5 %. sc1 nt as nt, sc0 sc1 as sc1.
+inline bool through_results(int64_t bytes) { return bytes <= (int64_t)32 << 20; }
 
 template <typename OutT, int NB>
 __device__ __forceinline__ void store_rows32_via_lds(char* lds, OutT* block, int64_t row_stride, int rows_valid,
                                                      const f32x16 (&accT)[NB], float factor, bool accumulate, int lane,
-                                                     bool keep, __bf16* final_block = nullptr) {
+                                                     bool through, __bf16* final_block = nullptr) {
 #pragma clang fp contract(off)  // product rounded, then added: what accumulating into a separate tensor gives
   constexpr int kPitch = NB * 128 + 16;  // bytes; the 16 spread the 32 rows of a column over the banks
   constexpr int kPieces = NB * 8;        // 16-byte pieces (4 features) per row
@@ -554,19 +556,15 @@ __device__ __forceinline__ void store_rows32_via_lds(char* lds, OutT* block, int
           u32x2 w;
           w[0] = pack_bf16x2(val[it][0], val[it][1]);
           w[1] = pack_bf16x2(val[it][2], val[it][3]);
-          if constexpr (decltype(through_tag)::value) __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(dst));
-          else *reinterpret_cast<u32x2*>(dst) = w;
+          if constexpr (decltype(through_tag)::value)  // (a store of device scope is what writes through)
+            __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), __builtin_bit_cast(uint64_t, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(dst));
         }
       }
     }
   };
-  if (sizeof(OutT) == 4 || keep) {
-    store(std::false_type{});
-  } else {
-    asm volatile("");  // at either end: or the compiler makes one plain store of the two
-    store(std::true_type{});
-    asm volatile("");
-  }
+  if (sizeof(OutT) == 4 || !through) store(std::false_type{});
+  else store(std::true_type{});
 }
 
 // The same turn through LDS for the forward kernel's merging epilogue: row r of the block becomes

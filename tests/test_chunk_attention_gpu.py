@@ -296,16 +296,16 @@ def test_forward_when_the_running_maximum_moves(gpu, Dqk, Hq, Hkv, Sq, causal, r
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("D,Dv", [(64, 64), (128, 128), (192, 128)])
 def test_large_results_equal_small_ones(gpu, D, Dv, causal):
-    """Results of 16 MiB and more are stored in another way than smaller ones: every batch element of such a call against the call of
+    """Results of more than 32 MiB are stored in another way than smaller ones: every batch element of such a call against the call of
     that element alone, whose sums may run in another order: results may round to neighbouring bf16 numbers, which lie 2^(e-7) apart
     in [2^e, 2^(e+1)), i.e. at most 2^-7 of the largest element. Ragged rows."""
-    B, S, H = 9, 1000, 1024 // Dv
+    B, S, H = 17, 1000, 1024 // Dv
     g = torch.Generator(device=gpu).manual_seed(D)
     t = lambda d: torch.randn(B, S, H, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
     q, k, v, dout = t(D), t(D), t(Dv), t(Dv)
     fwd, bwd = torch.ops.pithtrain_amd.attn_fwd, torch.ops.pithtrain_amd.attn_bwd
     o, lse = fwd(q, k, v, 0.07, causal)
-    assert o.numel() * 2 >= 16 << 20 > o[:1].numel() * 2
+    assert o.numel() * 2 > 32 << 20 > o[:1].numel() * 2
     whole = (o, *bwd(q, k, v, o, lse, dout, 0.07, causal))
     for b in range(B):
         x = [y[b : b + 1] for y in (q, k, v)]
