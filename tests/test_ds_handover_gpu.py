@@ -95,6 +95,13 @@ def test_dq_from_ds_192(gpu, causal, shape, dtype):
     _run(gpu, causal, shape, dtype, dqk=192)
 
 
+@pytest.mark.parametrize("dqk", [128, 192])
+@pytest.mark.parametrize("keys", [2, 32, 33, 65])  # (of a single key P is 1 and dS = dP - delta nothing but rounding)
+def test_dq_from_ds_of_few_key_steps(gpu, keys, dqk):
+    """Walks of one, two and three 32-key steps: shorter than the rings, and than what is read ahead of the products."""
+    _run(gpu, False, (1, 321, keys, 4, 2), torch.bfloat16, dqk=dqk)
+
+
 @pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
 def test_ring_share_of_192_with_and_without_handover(gpu, layout, monkeypatch):
     """Steps that hand dS over (fp32 dQ added to and finished by their kernels) against one launch that recomputes: the same bf16 dS
