@@ -20,7 +20,8 @@ namespace {
 // FULL and DUO when every compute unit has work for its whole time; the others when workgroups are few or (under the mask)
 // so unequal that a heavy one would run alone on its unit. Kernels measured on one box, microseconds, with inputs that
 // rotate over 500 MB (the tiles come from memory, as in a training step; the prefetch depth counts then: TEAMS at 192
-// features, two tiles per ring, beat HALF by 2-8 % on inputs in the last-level cache and lost 4-9 % here):
+// features, two tiles per ring, beat HALF by 2-8 % on inputs in the last-level cache and lost 4-9 % here)
+// (QUARTER before its teams took turns on streams of 1024 keys and more, 3-17 % faster since: kHalvesFrom in attn_fwd_duo.hip):
 //                                                       FULL    DUO   HALF  TEAMS QUARTER
 //   d128 causal   1 x 16384 x 8 heads (cached)           454    470    507    515    643
 //                 3 x 1999 x 32 (cached)                 109    107    133    131    187
@@ -57,8 +58,12 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   const bool d64 = a->Dqk == 64, unequal = mean <= 70;  // HALF is 3 % slower than DUO at 0.75, 5-10 % above
   // few rows: below 6 tiles (64 features: 5) the merge costs more than the shorter streams save
   if (wgs64 <= cus && a->Skv > (d64 ? 256 : 320)) return Split::kQuarter;
-  // more 64-row workgroups than compute units: heavy ones first, then light ones, as long as the streams are long
-  if (!d64 && unequal && ((2 * wgs64 <= 3 * cus && a->Skv >= 2048) || (wgs64 <= 2 * cus && a->Skv >= 6144))) return Split::kQuarter;
+  // more 64-row workgroups than compute units: heavy ones first, then light ones, as long as the streams are long. HALF / QUARTER, causal,
+  // us, inputs from memory, rounds of 64-row workgroups: 192 features, 1.1 1024 x 18 21.7 / 17.5, 1536 x 12 28.6 / 21.1; 1.5 1024 x 24 23.5 / 23.0, 1536 x
+  // 16 31.0 / 27.0; 1.75-2 1536 x 20 32.2 / 32.5, 2048 x 14 38.8 / 36.1, x 16 40.6 / 39.7, 3072 x 10 54.2 / 49.4, 4096 x 7 69.0 / 58.8, x 8 71.2 /
+  // 64.0; 128, 1.1 1024 x 18 18.0 / 16.1, 1536 x 12 23.4 / 19.5; 1.5 1024 x 24 18.2 / 19.3, 1536 x 16 23.6 / 22.4; 1.75-2 1536 x 20 26.8 / 28.3, 2048 x 14
+  // 31.0 / 30.6, x 16 33.7 / 34.6, 3072 x 10 43.8 / 40.7, 4096 x 7 53.6 / 46.9, x 8 57.8 / 53.6. Without a mask HALF, 1024 x 2048 x 32 45.8 / 62.0 and 37.6 / 52.9.
+  if (!d64 && unequal && wgs64 <= 2 * cus && a->Skv >= (4 * wgs64 <= 5 * cus ? 1024 : 2 * wgs64 <= 3 * cus ? 1536 : a->Dqk == 192 ? 2048 : 3072)) return Split::kQuarter;
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;
   if (wgs <= cus && a->Skv > (d64 ? 1024 : 512)) return key_split;
   if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 1535)) return key_split;

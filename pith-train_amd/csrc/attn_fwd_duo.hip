@@ -33,6 +33,14 @@ constexpr int kTeamWaves = 4;                 // waves that share a stream of ti
 constexpr int kTeamThreads = kTeamWaves * 64;
 constexpr int kBN = kFwdBlockN;   // keys per tile
 constexpr int kAhead = 4;         // fragment reads run this many products ahead in the matrix block
+// Intervals of a workgroup from which the two teams of 64-row workgroups (128 and 192 features) take turns (run_halves). The tiles of such a workgroup, 40 KB
+// per team and interval at 192 features, are what bounds it: without its loads 1021 x 3063 keys x 16 heads takes 33 us, loads alone 45, and with everything
+// landed at the end of each interval 54. Rows of few tiles lose the half interval by which the second team ends later. One
+// barrier an interval / turns, us, inputs from memory, full: 512 x 512 x 16 of 192 (4 intervals) 12.4 / 12.9, 768 (6) 15.3 / 15.2, 1024 18.1 / 17.2, 2048 32.6 /
+// 28.6, 3063 53.2 / 45.6, 1021 x 3063 54.1 / 47.5; of 128 512 11.0 / 11.7, 1024 15.6 / 15.3, 2048 24.5 / 22.2, 3063 45.3 / 37.9; causal 1021 x 16 of
+// 192 17.9 / 17.1, 2048 x 8 28.4 / 25.1, 4096 x 4 47.8 / 41.1, 8192 x 4 122 / 110, of 128 1021 x 16 15.3 / 15.1, 4096 x 4 41.0 / 36.2, 8192 x 4 104 / 91;
+// shares, 4 ranks: 1021 x 16 of 192 in two parts 44.3 / 41.4, 2048 x 16 115.6 / 107.0, 1024 x 16 55.0 / 48.6. 64 features lose at any length (4096 x 16 48.8 / 49.7).
+constexpr int kHalvesFrom = 8;
 
 template <int DQK, int PARTS>
 struct DuoLayout {
@@ -56,6 +64,7 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   constexpr int KVB = PARTS == 4 ? 1 : 2;  // 32-key blocks of a tile this wave owns
   constexpr bool kPaired = DQK == 64;  // tiles hold two rows per 256-byte LDS row
   constexpr int kTile = kBN * kRowBytes128;
+  constexpr bool kHalves = PARTS == 4 && DQK != 64;  // see kHalvesFrom
   __shared__ __attribute__((aligned(1024))) char smem[L::kSmem];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wg_wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -384,7 +393,43 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
       __syncthreads();
     }
   };
-  if (kTeams == 1 || team == 0) run(std::false_type{});
+  // Long streams (kHalvesFrom): a team's interval is its products of V(i) and K(i+1), a barrier, the softmax of tile i+1, a barrier, and
+  // the second team is half an interval behind. Slots are requested anew as soon as the products have read them, V(i+2) and K(i+3),
+  // which then have the softmax and a whole interval to land, instead of one interval that ends with everything landed.
+  auto run_halves = [&]() __attribute__((always_inline)) {
+    auto request = [&](int i) __attribute__((always_inline)) {
+      if (i + 2 < n_tiles_wg) issue_v(i + 2);
+      if (i + 3 < n_tiles_wg) issue_k(i + 3);
+    };
+    request(-1);
+    if (team == 1) {
+      if (any) softmax(0);
+      __syncthreads();
+    }
+    int i = 0;
+    for (; i + 3 < n_tiles_wg && i + 1 < n_tiles_wave; ++i) {
+      matrix_block(vbuf + (i & 1) * L::kVTile, kbuf + ((i + 1) & 1) * L::kKTile);
+      __syncthreads();
+      request(i);
+      softmax(i + 1);
+      wait_staged<kLoadsV + kLoadsK>();  // V(i+1) and K(i+2) are there, what has just been requested may be on its way
+      __syncthreads();
+    }
+    for (; i < intervals; ++i) {
+      if (i + 1 < n_tiles_wave) matrix_block(vbuf + (i & 1) * L::kVTile, kbuf + ((i + 1) & 1) * L::kKTile);
+      else if (i < n_tiles_wave) accumulate(vbuf + (i & 1) * L::kVTile);
+      __syncthreads();
+      request(i);
+      if (i + 1 < n_tiles_wave) softmax(i + 1);
+      if (i + 3 < n_tiles_wg) wait_staged<kLoadsV + kLoadsK>();
+      else if (i + 2 < n_tiles_wg) wait_staged<kLoadsV>();
+      else wait_staged();
+      __syncthreads();
+    }
+    if (team == 0) __syncthreads();
+  };
+  if (kHalves && intervals >= kHalvesFrom) run_halves();
+  else if (kTeams == 1 || team == 0) run(std::false_type{});
   else run(std::true_type{});
 
   // ---- several parts: the other waves of a row block hand accumulator, maximum and sum to its first one, which rescales

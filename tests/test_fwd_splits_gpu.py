@@ -58,3 +58,38 @@ def test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
 ])  # fmt: skip
 def test_forward_key_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D,causal", [
+    # 64-row workgroups whose teams take turns: 7 / 8 / 9 intervals, an odd tile, one ragged key, waves that end before their workgroup
+    (1, 64, 896, 2, 1, 128, False), (1, 64, 897, 2, 1, 128, False), (1, 70, 1024, 2, 2, 192, False), (2, 33, 1025, 4, 2, 192, False),
+    (1, 961, 961, 2, 2, 192, True), (1, 1023, 1023, 4, 1, 128, True), (1, 1089, 1089, 2, 1, 128, True),
+    # as many of them as one and a quarter, one and a half or two per unit, from 1024, 1536 and 2048 (128 features: 3072) keys on
+    (1, 1023, 1023, 20, 20, 192, True), (1, 1024, 1024, 20, 4, 128, True), (1, 1535, 1535, 16, 4, 128, True), (1, 1536, 1536, 16, 16, 192, True),
+    (1, 2048, 2048, 16, 16, 192, True), (1, 2050, 2050, 16, 16, 192, True), (1, 3072, 3072, 10, 2, 128, True),
+])  # fmt: skip
+def test_forward_teams_in_turns(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+    test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
+@pytest.mark.parametrize("rows,D", [(510, 192), (514, 128), (258, 192)])
+def test_shares_of_teams_in_turns(gpu, rows, D, layout):
+    """Streams over several chunks, whose tiles the teams take in turns: each row against all keys it sees."""
+    from pithtrain_amd.operators.ring_attention.local import ring_forward_local
+
+    rank, cp, h = 1, 4, 2
+    g = torch.Generator(device=gpu).manual_seed(4)
+    mk = lambda s, d: torch.randn(1, s, h, d, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    half = rows // 2
+    # positions of a chunk's rows in the sequence
+    at = lambda j: torch.cat([torch.arange(half) + half * j, torch.arange(half) + half * (2 * cp - 1 - j)]) if layout == "zigzag" else torch.arange(rows) + rows * j  # noqa: E731
+    seen = range(cp) if layout == "zigzag" else range(rank + 1)
+    q, ks, vs = mk(rows, D), [mk(rows, D) if j in seen else None for j in range(cp)], [mk(rows, 128) if j in seen else None for j in range(cp)]
+    o, lse = ring_forward_local(q, ks, vs, D**-0.5, rank, cp, layout)
+    k, v = (torch.cat([x for x in t if x is not None], 1) for t in (ks, vs))
+    hidden = torch.cat([at(j) for j in seen])[None, :] > at(rank)[:, None]
+    s = (q[0].transpose(0, 1).float() @ k[0].permute(1, 2, 0).float().contiguous()) * D**-0.5
+    s = s.masked_fill(hidden.to(gpu), float("-inf"))
+    check_lse(lse, torch.logsumexp(s, -1)[None] / 0.6931471805599453, "LSE2")
+    check_bf16_result(o, (torch.softmax(s, -1) @ v[0].transpose(0, 1).float().contiguous()).transpose(0, 1)[None], "O")
