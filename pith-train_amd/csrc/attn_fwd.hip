@@ -16,7 +16,9 @@ namespace {
 //          tiles overlap the other's loop, and the diagonal wastes half as much;
 //   HALF   one 128-row workgroup of 8 waves per compute unit, wave pairs splitting the keys of every tile;
 //   TEAMS  one 128-row workgroup of 8 waves per compute unit, two teams of 4 waves taking every second tile (64 features);
-//   QUARTER  one 64-row workgroup of 8 waves: two teams, and wave pairs of a team splitting the keys of its tile.
+//   QUARTER  one 64-row workgroup of 8 waves: two teams, and wave pairs of a team splitting the keys of its tile;
+//   SMALL  two (64 features: five) 64-row workgroups of 4 waves, wave pairs splitting the keys of every tile: an interval of half the length, and
+//          more workgroups than any other split that hide each other's first tiles and epilogues.
 // FULL and DUO when every compute unit has work for its whole time; the others when workgroups are few or (under the mask)
 // so unequal that a heavy one would run alone on its unit. Kernels measured on one box, microseconds, with inputs that
 // rotate over 500 MB (the tiles come from memory, as in a training step; the prefetch depth counts then: TEAMS at 192
@@ -49,24 +51,60 @@ namespace {
 //   causal   32768 x 128 heads 36.0 / 36.4   x 120 33.9 / 33.3   x 64 18.1 / 17.9   x 16 4.58 / 4.53   16384 x 64  4.67 / 4.59
 //            8192 x 128        2.59 / 2.39   x 16  0.345 / 0.298                    4096 x 128 0.692 / 0.663
 //   full     32768 x 16        8.89 / 8.96   16384 x 64 8.91 / 9.05   8192 x 128 4.87 / 4.58   x 16 0.565 / 0.567   4096 x 128 1.24 / 1.17
-enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter };
+// Where workgroups are few, by W = 64-row workgroups per compute unit, us, DUO / HALF (64 features: TEAMS) / QUARTER / SMALL, inputs from memory:
+//   d64 causal   W 1         2 x 256 x 32 7.3 / 7.6 / 6.7 / 6.2, 1024 x 16 15.9 / 14.1 / 10.8 / 12.1, 4096 x 4 50.4 / 39.8 / 27.3 / 35.4
+//                W 2         4 x 256 x 32 7.6 / 7.9 / 9.8 / 6.4, 1024 x 32 16.4 / 14.5 / 13.8 / 12.5, 2048 x 16 27.6 / 23.0 / 19.7 / 20.6,
+//                            4096 x 8 50.4 / 40.0 / 31.1 / 36.9
+//                W 3 - 4     8 x 256 x 24 7.7 / 12.9 / 13.1 / 7.2, 2 x 1024 x 32 17.7 / 19.9 / 24.7 / 14.9, 2048 x 24 28.7 / 24.2 / 29.0 / 22.6,
+//                            2048 x 32 30.1 / 28.6 / 35.3 / 25.1, 2 x 2048 x 16 30.1 / 28.6 / 35.1 / 25.0, 4096 x 16 55.9 / 47.8 / 57.8 / 47.1
+//                W 4.1 - 6   3 x 1346 x 16 22.4 / 28.2 / 31.3 / 19.0, 3 x 1596 x 16 26.5 / 34.1 / 36.6 / 25.5, 4404 x 16 61.8 / 60.8 / 68.2 / 52.2,
+//                            4 x 1024 x 20 18.5 / 27.3 / 30.4 / 20.3, 2 x 2048 x 20 33.3 / 40.6 / 44.5 / 32.4, 12 x 512 x 16 14.4 / 23.4 / 28.2 / 15.9
+//   d64 full     W 1         2 x 256 x 32 6.9 / 7.8 / 6.8 / 6.2, 1024 x 16 15.8 / 14.6 / 11.2 / 12.2
+//                W 2         4 x 192 x 43 8.1 / 14.4 / 14.7 / 8.1, 1024 x 32 16.6 / 15.4 / 19.2 / 13.9, 2 x 512 x 32 10.3 / 10.3 / 13.3 / 9.1
+//                W 3 - 4     2048 x 24 33.6 / 45.3 / 43.3 / 35.0
+//   d128 causal  W 1         4 x 128 x 32 7.1 / 7.9 / 7.9 / 6.7, 2 x 256 x 32 9.0 / 9.1 / 9.0 / 8.1, 512 x 32 13.0 / 12.1 / 11.0 / 10.8,
+//                            1024 x 16 20.9 / 17.7 / 15.3 / 16.2
+//                W 1.1 - 1.5 1024 x 18 21.2 / 18.2 / 16.0 / 16.7, 1536 x 12 28.9 / 23.5 / 19.2 / 22.1, 2 x 512 x 24 13.3 / 12.4 / 16.0 / 11.3,
+//                            1024 x 24 21.3 / 18.0 / 19.1 / 16.9, 1536 x 16 29.0 / 23.4 / 21.7 / 22.3
+//                W 2         2 x 512 x 32 13.6 / 12.6 / 16.8 / 11.7, 1024 x 32 21.8 / 18.7 / 21.2 / 17.8, 2048 x 16 37.5 / 30.0 / 30.1 / 29.5,
+//                            3072 x 10 53.6 / 42.0 / 39.0 / 42.1, 4096 x 8 69.4 / 53.2 / 47.1 / 53.4
+//                W 2.5 - 3   8 x 256 x 20 10.1 / 15.1 / 20.5 / 13.2, 2 x 1024 x 20 23.2 / 19.9 / 29.8 / 19.1, 2 x 1024 x 24 23.6 / 22.6 / 31.6 / 22.7
+//   d128 full    W 1         2 x 256 x 32 9.2 / 9.0 / 9.4 / 8.2, 512 x 32 13.4 / 11.8 / 11.6 / 10.9
+//                W 2         4 x 256 x 32 10.5 / 10.1 / 17.3 / 10.3, 2 x 512 x 32 14.8 / 13.1 / 21.1 / 13.7, 1024 x 2048 x 32 40.8 / 35.4 / 47.1 / 37.9
+//   d192 causal  W 1         2 x 256 x 32 10.5 / 10.4 / 10.2 / 9.2, 512 x 32 15.2 / 14.0 / 12.6 / 12.4, 1024 x 16 24.6 / 21.6 / 17.2 / 18.5
+//                W 1.1 - 1.5 8 x 128 x 24 9.9 / 11.3 / 16.7 / 10.4, 2 x 512 x 24 16.7 / 16.1 / 19.4 / 15.2, 1024 x 24 25.8 / 23.6 / 23.2 / 22.2,
+//                            1409 x 16 32.7 / 28.5 / 24.8 / 26.6
+//                W 2         2 x 512 x 32 17.0 / 16.1 / 20.4 / 15.3, 2048 x 16 45.3 / 38.5 / 36.3 / 37.7, 4096 x 8 82.3 / 69.7 / 58.3 / 67.5
+//                W 2.5 - 3   2 x 1024 x 20 27.5 / 24.4 / 35.6 / 24.6
+//   d192 full    W 1         2 x 256 x 32 10.5 / 10.4 / 10.7 / 9.5, 512 x 32 15.3 / 13.9 / 13.3 / 12.9
+//                W 2         4 x 256 x 32 12.8 / 14.4 / 21.2 / 14.0, 2 x 512 x 32 18.2 / 17.2 / 26.5 / 19.3, 1024 x 2048 x 32 50.5 / 44.6 / 60.5 / 54.9
+// Shares whose rows are short beside their streams gain nothing from a second round of QUARTER: rank 1 of 4, 1022 x 32/4 of 128,
+// 67.1 / 51.7 / 73.2 / 56.6.
+enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter, kSmall };
 
 // `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50).
 Split pick_split(const pith_attn_fwd_args* a, int mean) {
   const int64_t cus = compute_units_or_default();
   const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B, wgs64 = ((a->Sq + 63) / 64) * a->Hq * a->B;  // of 128 and 64 rows
   const bool d64 = a->Dqk == 64, unequal = mean <= 70;  // HALF is 3 % slower than DUO at 0.75, 5-10 % above
-  // few rows: below 6 tiles (64 features: 5) the merge costs more than the shorter streams save
-  if (wgs64 <= cus && a->Skv > (d64 ? 256 : 320)) return Split::kQuarter;
-  // more 64-row workgroups than compute units: heavy ones first, then light ones, as long as the streams are long. HALF / QUARTER, causal,
-  // us, inputs from memory, rounds of 64-row workgroups: 192 features, 1.1 1024 x 18 21.7 / 17.5, 1536 x 12 28.6 / 21.1; 1.5 1024 x 24 23.5 / 23.0, 1536 x
-  // 16 31.0 / 27.0; 1.75-2 1536 x 20 32.2 / 32.5, 2048 x 14 38.8 / 36.1, x 16 40.6 / 39.7, 3072 x 10 54.2 / 49.4, 4096 x 7 69.0 / 58.8, x 8 71.2 /
-  // 64.0; 128, 1.1 1024 x 18 18.0 / 16.1, 1536 x 12 23.4 / 19.5; 1.5 1024 x 24 18.2 / 19.3, 1536 x 16 23.6 / 22.4; 1.75-2 1536 x 20 26.8 / 28.3, 2048 x 14
-  // 31.0 / 30.6, x 16 33.7 / 34.6, 3072 x 10 43.8 / 40.7, 4096 x 7 53.6 / 46.9, x 8 57.8 / 53.6. Without a mask HALF, 1024 x 2048 x 32 45.8 / 62.0 and 37.6 / 52.9.
-  if (!d64 && unequal && wgs64 <= 2 * cus && a->Skv >= (4 * wgs64 <= 5 * cus ? 1024 : 2 * wgs64 <= 3 * cus ? 1536 : a->Dqk == 192 ? 2048 : 3072)) return Split::kQuarter;
+  if (a->Skv > 64) {  // (64 features to 6144 keys: 4404 x 16 61.8 -> 52.2, 4998 x 16 75 -> 67, 5938 x 16 95 -> 91)
+    if (wgs64 <= cus) return a->Skv > 512 ? Split::kQuarter : Split::kSmall;
+    if (unequal) {
+      if (wgs64 <= 2 * cus) {
+        const bool quarter_more = 4 * wgs64 > 5 * cus, half_more = 2 * wgs64 > 3 * cus;  // workgroups than one round of QUARTER
+        const int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
+        if (a->Skv >= from && (!half_more || a->Sq >= 1536)) return Split::kQuarter;
+        if (a->Skv >= (a->Dqk == 192 ? 129 : 128) && a->Skv < 1536) return Split::kSmall;
+      } else if (d64 && 2 * wgs64 <= (a->Skv < 1536 ? 9 : 10) * cus && a->Skv >= 128 && a->Skv <= 6144) {
+        return Split::kSmall;
+      }
+    } else if (d64 && wgs64 <= 2 * cus && a->Skv >= 192) {
+      return Split::kSmall;
+    }
+  }
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;
-  if (wgs <= cus && a->Skv > (d64 ? 1024 : 512)) return key_split;
-  if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 1535)) return key_split;
+  if (wgs <= cus && a->Skv > (d64 ? 1024 : a->Dqk == 192 ? 383 : 255)) return key_split;
+  if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 2 * wgs <= 3 * cus ? 1023 : 1535)) return key_split;
   // FULL under the mask also for shorter rows of many heads whose K and V outgrow the last-level cache (half the streams in
   // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
   // for rows of a few workgroups: 8 x 512 x 128 155 -> 167)
@@ -156,7 +194,7 @@ int launch(const P& p, const pith_attn_fwd_args* a, Split split, pith_stream_t s
   const int dqk = (int)a->Dqk;
   const bool causal = a->causal != 0;
   if (split == Split::kFull || split == Split::kHalf) launch_fwd_direct(p, dqk, causal, split == Split::kHalf, st);
-  else launch_fwd_duo(p, dqk, split == Split::kDuo ? 1 : split == Split::kTeams ? 2 : 4, causal, st);
+  else launch_fwd_duo(p, dqk, split == Split::kDuo ? 1 : split == Split::kTeams ? 2 : split == Split::kSmall ? 3 : 4, causal, st);
   return check_launch(who);
 }
 

@@ -56,7 +56,8 @@ void launch_fwd_direct(const FwdParams& p, int dqk, bool causal, bool half, hipS
 void launch_fwd_direct(const FwdChunkParams& p, int dqk, bool causal, bool half, hipStream_t stream);
 
 // attn_fwd_duo.hip. parts = 1: two (64 features: three) 4-wave workgroups of 128 query rows per compute unit; 2 (64
-// features) or 4: one 8-wave workgroup of 128 or 64 rows, whose key stream is split in that many parts.
+// features) or 4: one 8-wave workgroup of 128 or 64 rows, whose key stream is split in that many parts; 3: two or more 4-wave
+// workgroups of 64 rows, whose key stream is split in two.
 void launch_fwd_duo(const FwdParams& p, int dqk, int parts, bool causal, hipStream_t stream);
 void launch_fwd_duo(const FwdChunkParams& p, int dqk, int parts, bool causal, hipStream_t stream);
 

@@ -13,7 +13,11 @@
 // 64 features: a K or V tile packs two rows per 256-byte LDS row (see DirectPaired64), and the softmax of 32 x 64 scores
 // costs as much vector time as its products cost matrix time, so three workgroups per compute unit share the pipes.
 //
-// PARTS > 1: two such teams of 4 waves in one workgroup, each with its own rings, taking every second tile; the results are
+// PARTS = 3 (SMALL): 64 rows; the two waves that share 32 rows take half a tile's keys each and merge through LDS. An interval has
+// half the products and half the vector work of a wave, and the grid twice the workgroups, where those of 128 rows leave a SIMD little more
+// than one wave that does one thing at a time (2 x 2048 x 16/4 heads of 64: 0.97 waves per SIMD, matrix pipe 18 % busy): 33.3 -> 27.3
+// us, 2 x 1024 x 16/4 16.5 -> 13.1, 256 x 8/2 of 128 8.5 -> 7.3, 2 x 512 x 32/4 13.9 -> 11.6.
+// PARTS = 2, 4: two such teams of 4 waves in one workgroup, each with its own rings, taking every second tile; the results are
 // merged through LDS. For grids that leave units idle or a heavy workgroup alone on its unit, where the length of a stream
 // counts. PARTS = 2: 128 rows as above. PARTS = 4: 64 rows, the two waves of a team that share rows take half a tile's keys
 // each: twice the requests per product, on units that have nothing else to do. Measured against the split-key workgroups of
@@ -44,16 +48,17 @@ constexpr int kHalvesFrom = 8;
 
 template <int DQK, int PARTS>
 struct DuoLayout {
-  static constexpr int kTeams = PARTS == 1 ? 1 : 2;
+  static constexpr int kTeams = PARTS == 1 || PARTS == 3 ? 1 : 2;
+  static constexpr int kParts = PARTS == 3 ? 2 : PARTS;  // waves that share 32 query rows
   static constexpr int kThreads = kTeams * kTeamThreads;
-  static constexpr int kRowBlocks = PARTS == 4 ? 2 : 4;  // of 32 query rows
+  static constexpr int kRowBlocks = PARTS >= 3 ? 2 : 4;  // of 32 query rows
   static constexpr int kBM = 32 * kRowBlocks;            // query rows per workgroup
   static constexpr int kDv = DQK == 64 ? 64 : 128;
   static constexpr int kKTile = DQK == 64 ? kExtraTileBytes : DQK == 128 ? kBN * kRowBytes128 : kBN * kRowBytes128 + kExtraTileBytes;
   static constexpr int kVTile = kDv == 64 ? kExtraTileBytes : kBN * kRowBytes128;
   static constexpr int kRings = 2 * (kKTile + kVTile);   // of one team
   static constexpr int kTurn = kRowsViaLdsBytes<kDv / 32>;
-  static constexpr int kAfter = kRowBlocks * (PARTS == 1 ? 1 : PARTS - 1) * kTurn;  // the epilogue's use of the rings
+  static constexpr int kAfter = kRowBlocks * (PARTS == 1 ? 1 : kParts - 1) * kTurn;  // the epilogue's use of the rings
   static constexpr int kSmem = kTeams * kRings > kAfter ? kTeams * kRings : kAfter;
 };
 
@@ -61,7 +66,7 @@ template <int DQK, int PARTS, bool CAUSAL, bool MULTI>
 __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd_duo_kernel(FwdArgs<MULTI> p) {
   using L = DuoLayout<DQK, PARTS>;
   constexpr int kDv = L::kDv, KS = DQK / 16, DVB = kDv / 32, kBM = L::kBM, kTeams = L::kTeams;
-  constexpr int KVB = PARTS == 4 ? 1 : 2;  // 32-key blocks of a tile this wave owns
+  constexpr int KVB = PARTS >= 3 ? 1 : 2;  // 32-key blocks of a tile this wave owns
   constexpr bool kPaired = DQK == 64;  // tiles hold two rows per 256-byte LDS row
   constexpr int kTile = kBN * kRowBytes128;
   constexpr bool kHalves = PARTS == 4 && DQK != 64;  // see kHalvesFrom
@@ -71,7 +76,8 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   const int wave = wg_wave & (kTeamWaves - 1);              // within its team
   const int team = kTeams == 1 ? 0 : wg_wave / kTeamWaves;  // takes the tiles t with t % kTeams == team
   const int row_block = wave & (L::kRowBlocks - 1);
-  const int kvb0 = PARTS == 4 ? wave >> 1 : 0;              // first 32-key block of a tile this wave owns
+  const int kvb0 = PARTS >= 3 ? wave >> 1 : 0;              // first 32-key block of a tile this wave owns
+  const int part = PARTS == 4 ? 2 * team + kvb0 : PARTS == 3 ? kvb0 : team;  // of its 32 rows' keys
   char* const kbuf = smem + team * L::kRings;
   char* const vbuf = kbuf + 2 * L::kKTile;
   const int c = lane & 31, g = lane >> 5;
@@ -160,21 +166,22 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   };
   // Query rows first: nothing can start without them. PARTS = 1: every wave stages its own in slots of tiles that are requested
   // behind them (K 1 and V 1, two waves each; at 192 features the fourth wave takes V 0). Several parts: the waves of a row
-  // block share the loads and an area in the V 1 slots.
+  // block share the loads and an area in the V 1 slots (small workgroups of 192 features: in V 1 and K 1).
   constexpr int kQArea = kPaired ? 4096 : 8192 + (DQK == 192 ? 4096 : 0);
-  constexpr bool kDelayV0 = PARTS == 1 && DQK == 192;
-  static_assert(PARTS == 1 ? 2 * kQArea <= L::kKTile && (kDelayV0 ? kQArea : 2 * kQArea) <= L::kVTile
-                           : kQArea * L::kRowBlocks / 2 <= L::kVTile, "query areas");
+  constexpr bool kDelayV0 = PARTS == 1 && DQK == 192, kDelayK1 = PARTS == 3 && DQK == 192;
+  static_assert(PARTS == 1   ? 2 * kQArea <= L::kKTile && (kDelayV0 ? kQArea : 2 * kQArea) <= L::kVTile
+                : PARTS == 3 ? (kDelayK1 ? kQArea <= L::kKTile && kQArea <= L::kVTile : 2 * kQArea <= L::kVTile)
+                             : kQArea * L::kRowBlocks / 2 <= L::kVTile, "query areas");
   char* const k1 = kbuf + L::kKTile;
   char* const v0 = vbuf;
   char* const v1 = vbuf + L::kVTile;
   char* q_area;
   if constexpr (PARTS == 1) q_area = wave < 2 ? k1 + wave * kQArea : kDelayV0 ? (wave == 2 ? v1 : v0) : v1 + (wave - 2) * kQArea;
+  else if constexpr (PARTS == 3) q_area = row_block == 0 ? v1 : kDelayK1 ? k1 : v1 + kQArea;
   else if constexpr (PARTS == 2) q_area = smem + (row_block >> 1) * L::kRings + 2 * L::kKTile + L::kVTile + (row_block & 1) * kQArea;
   else q_area = smem + row_block * L::kRings + 2 * L::kKTile + L::kVTile;
   {
-    constexpr int kShare = PARTS;  // waves of a row block
-    const int part = PARTS == 4 ? 2 * team + kvb0 : team;
+    constexpr int kShare = L::kParts;
     const char* const qsrc = reinterpret_cast<const char*>(qh);
     const int q_row_bytes = (int)(q_row_stride * 2);
     if constexpr (!kPaired) stage_rows32<true, 8 / kShare>(qsrc, q_wave0, p.Sq, q_row_bytes, q_area, lane, part * (8 / kShare));
@@ -185,7 +192,7 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     issue_k(0);
     if constexpr (!kDelayV0) issue_v(0);
   }
-  if (PARTS > 1 && n_tiles_wg > 1) issue_k(1);
+  if (PARTS > 1 && !kDelayK1 && n_tiles_wg > 1) issue_k(1);
   constexpr int kLoadsK = kPaired ? 2 : DQK == 192 ? 6 : 4, kLoadsV = kPaired ? 2 : 4;  // load instructions of a wave per tile
   bf16x8 qf[KS];  // Q^T fragments (B operand): column = query row, slots = 8 consecutive features
   auto read_q = [&]() __attribute__((always_inline)) {
@@ -354,10 +361,15 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     if constexpr (kDelayV0) issue_v(0);
     if (n_tiles_wg > 1) issue_k(1);
   } else {
-    if (n_tiles_wg > 1) wait_staged<kLoadsV + kLoadsK>();
+    if (kDelayK1) wait_staged<kLoadsV>();
+    else if (n_tiles_wg > 1) wait_staged<kLoadsV + kLoadsK>();
     else wait_staged();
     __syncthreads();
     read_q();
+    if constexpr (kDelayK1) {
+      __syncthreads();
+      if (n_tiles_wg > 1) issue_k(1);
+    }
   }
   const bool any = kTeams == 1 || n_tiles_wave > 0;
   if (any) scores(kbuf);
@@ -437,7 +449,6 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
   if constexpr (PARTS > 1) {
     constexpr int kExch = L::kTurn;  // DVB * 16 accumulator values and (m, l) per lane
     static_assert(kExch == DVB * 4 * 64 * 16 + 64 * 8, "exchange area");
-    const int part = PARTS == 4 ? 2 * team + kvb0 : team;
     auto area = [&](int from) __attribute__((always_inline)) { return smem + ((from - 1) * L::kRowBlocks + row_block) * kExch; };
     if (part > 0) {
       char* const exch = area(part);
@@ -453,10 +464,10 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     }
     __syncthreads();
     if (part > 0) return;
-    f32x2 ml[PARTS - 1];
+    f32x2 ml[L::kParts - 1];
     float m_new = m_run;
 #pragma unroll
-    for (int n = 0; n < PARTS - 1; ++n) {
+    for (int n = 0; n < L::kParts - 1; ++n) {
       ml[n] = *reinterpret_cast<const f32x2*>(area(n + 1) + DVB * 4 * 64 * 16 + lane * 8);
       m_new = fmaxf(m_new, ml[n][0]);
     }
@@ -469,7 +480,7 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
 #pragma unroll
       for (int v = 0; v < 16; ++v) oacc[i][v] *= w0;
 #pragma unroll
-    for (int n = 0; n < PARTS - 1; ++n) {
+    for (int n = 0; n < L::kParts - 1; ++n) {
       const float w = (ml[n][0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((ml[n][0] - m_new) * p.kappa);
       l_run += ml[n][1] * w;
 #pragma unroll
@@ -560,6 +571,7 @@ void launch_one(FwdArgs<MULTI> p, bool causal, hipStream_t st) {
 template <int DQK, bool MULTI>
 void launch_parts(const FwdArgs<MULTI>& p, int parts, bool causal, hipStream_t st) {
   if (parts == 1) launch_one<DQK, 1, MULTI>(p, causal, st);
+  else if (parts == 3) launch_one<DQK, 3, MULTI>(p, causal, st);
   else if (parts == 4) launch_one<DQK, 4, MULTI>(p, causal, st);
   else if constexpr (DQK == 64) launch_one<DQK, 2, MULTI>(p, causal, st);
 }

@@ -85,7 +85,7 @@ def test_shares_of_teams_in_turns(gpu, rows, D, layout):
     # positions of a chunk's rows in the sequence
     at = lambda j: torch.cat([torch.arange(half) + half * j, torch.arange(half) + half * (2 * cp - 1 - j)]) if layout == "zigzag" else torch.arange(rows) + rows * j  # noqa: E731
     seen = range(cp) if layout == "zigzag" else range(rank + 1)
-    q, ks, vs = mk(rows, D), [mk(rows, D) if j in seen else None for j in range(cp)], [mk(rows, 128) if j in seen else None for j in range(cp)]
+    q, ks, vs = mk(rows, D), [mk(rows, D) if j in seen else None for j in range(cp)], [mk(rows, min(D, 128)) if j in seen else None for j in range(cp)]
     o, lse = ring_forward_local(q, ks, vs, D**-0.5, rank, cp, layout)
     k, v = (torch.cat([x for x in t if x is not None], 1) for t in (ks, vs))
     hidden = torch.cat([at(j) for j in seen])[None, :] > at(rank)[:, None]
@@ -93,3 +93,23 @@ def test_shares_of_teams_in_turns(gpu, rows, D, layout):
     s = s.masked_fill(hidden.to(gpu), float("-inf"))
     check_lse(lse, torch.logsumexp(s, -1)[None] / 0.6931471805599453, "LSE2")
     check_bf16_result(o, (torch.softmax(s, -1) @ v[0].transpose(0, 1).float().contiguous()).transpose(0, 1)[None], "O")
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D,causal", [
+    # 64-row workgroups of 4 waves: one ragged row, key halves that do not exist or end early, 64 / 65 and 512 / 513 keys
+    *[(1, sq, skv, 2, 1, d, sq == skv) for d in (64, 128, 192) for sq, skv in ((65, 65), (1, 65), (64, 96), (33, 97), (127, 128), (95, 350), (300, 300), (512, 512))],
+    (1, 70, 513, 2, 1, 64, False), (2, 257, 257, 3, 3, 192, True),
+    # one and two of them per unit (192 features: from 129 keys on), at 64 features four and a half, five from 1536 keys on
+    (2, 512, 512, 16, 4, 128, True), (4, 320, 320, 25, 25, 128, True), (8, 128, 128, 32, 32, 192, True), (8, 129, 129, 21, 21, 192, True),
+    (4, 192, 192, 43, 43, 64, False), (4, 576, 576, 32, 8, 64, True), (4, 577, 577, 32, 8, 64, True), (2, 1535, 1535, 26, 13, 64, True), (2, 1536, 1536, 26, 13, 64, True),
+    # wave pairs of 128-row workgroups from 256 (192 features: 384) keys on
+    (2, 255, 300, 70, 70, 128, False), (4, 256, 256, 32, 8, 128, False), (2, 384, 384, 33, 33, 192, False), (2, 1024, 1024, 20, 20, 192, True),
+])  # fmt: skip
+def test_forward_small_workgroups(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+    test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
+@pytest.mark.parametrize("rows,D", [(66, 64), (100, 128), (130, 192)])
+def test_shares_of_small_workgroups(gpu, rows, D, layout):
+    test_shares_of_teams_in_turns(gpu, rows, D, layout)
