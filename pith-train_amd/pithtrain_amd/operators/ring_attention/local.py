@@ -36,7 +36,7 @@ backward returns dk_nope and the head-summed dk_pe per chunk.
 """
 
 from dataclasses import dataclass
-from typing import List, Sequence, Tuple
+from typing import List, NamedTuple, Sequence, Tuple
 
 import torch
 
@@ -361,15 +361,30 @@ def _steps_beat_one_launch(q: torch.Tensor, hkv: int, steps: Sequence[Tuple[int,
     return native.share_hands_over(b, s, hq, hkv, steps, hip._device_compute_units(q.device), q.shape[-1])
 
 
+class _Sizes(NamedTuple):
+    """A row range of a [B, S, H, D] tensor as hip.ds_plan looks at it."""
+
+    shape: Tuple[int, int, int, int]
+    device: torch.device
+
+
 def _handover_pays(steps: Sequence[RingStep], q: torch.Tensor, k_chunks, v_chunks) -> bool:
     """Whether enough steps of the share hand dS from their dK/dV to their dQ kernel (5 matrix products instead of 7) to be worth
-    more than one launch over all chunks saves."""
-    if q.shape[-1] not in (128, 192) or k_chunks[steps[0].kv_rank].shape[-1] != q.shape[-1]:  # (nor keys in two parts)
+    more than one launch over all chunks saves. Asked for sizes alone, and once for steps alike: with views of every step's tensors
+    this was 15 (two chunks) to 40 us (eight) of the host's time, beside 30 to 60 us of kernels where rows are short."""
+    b, _, hq, d = q.shape
+    if d not in (128, 192) or k_chunks[steps[0].kv_rank].shape[-1] != d:  # (nor keys in two parts)
         return False
-    plans = [hip.ds_plan(_rows(q, st.q_rows), _rows(k_chunks[st.kv_rank], st.kv_rows), _rows(v_chunks[st.kv_rank], st.kv_rows), st.causal) for st in steps]
-    if not any(plans):
+    plans, sizes = {}, []
+    for st in steps:
+        m, n = st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0]
+        hkv, dv = k_chunks[st.kv_rank].shape[2], v_chunks[st.kv_rank].shape[3]
+        key = (m, n, st.causal, hkv, dv)
+        if key not in plans:
+            plans[key] = hip.ds_plan(_Sizes((b, m, hq, d), q.device), _Sizes((b, n, hkv, d), q.device), _Sizes((b, n, hkv, dv), q.device), st.causal)
+        sizes.append((m, n, st.causal, plans[key][0] if plans[key] else 0))
+    if not any(plans.values()):
         return False
-    sizes = [(st.q_rows[1] - st.q_rows[0], st.kv_rows[1] - st.kv_rows[0], st.causal, plan[0] if plan else 0) for st, plan in zip(steps, plans)]
     return _steps_beat_one_launch(q, k_chunks[steps[0].kv_rank].shape[2], sizes)
 
 
