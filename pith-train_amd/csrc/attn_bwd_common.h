@@ -26,6 +26,7 @@ struct BwdParams {
   float kappa, scale;
   int accumulate, accumulate_dq;  // dK/dV and dQ kernels: add to what the outputs hold
   int through_dkv, through_dq;    // bf16 results are written through (through_results)
+  int through_parts;  // and so are the fp32 partial results below
   int split;        // dK/dV kernel: query-head groups are cut into `split` parts handled by different workgroups
   float* ws_dk;     // dK/dV kernel, split > 1: fp32 partial results [split][B][Skv][Hkv][D]
   float* ws_dv;

@@ -417,7 +417,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     // the partials are packed: exactly the Hkv heads of this call per row
     const int64_t row_stride = (int64_t)p.Hkv * kD;
     float* ws = (role_b ? p.ws_dk : p.ws_dv) + (((int64_t)part * p.B + b) * p.Skv + kv_pair0) * row_stride + (int64_t)hk * kD;
-    store_rows32_via_lds<float, DB>(turn, ws, row_stride, rows_valid, acc, factor, false, lane, p.through_dkv);
+    store_rows32_via_lds<float, DB>(turn, ws, row_stride, rows_valid, acc, factor, false, lane, p.through_parts);
   } else {
     OutT* out = reinterpret_cast<OutT*>(role_b ? p.dk : p.dv) + b * (role_b ? p.dk_bs : p.dv_bs) + kv_pair0 * kv_row_stride + (int64_t)hk * kD;
     store_rows32_via_lds<OutT, DB>(turn, out, kv_row_stride, rows_valid, acc, factor, p.accumulate != 0, lane, p.through_dkv);

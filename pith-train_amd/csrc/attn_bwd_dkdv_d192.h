@@ -444,7 +444,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
     f32x16 part_acc[NB];
 #pragma unroll
     for (int o = 0; o < NB; ++o) part_acc[o] = acc[O0 + o];
-    if (partial) store_rows32_via_lds<float, NB>(turn, ws + 32 * O0, ws_stride, rows_valid, part_acc, factor, false, lane, p.through_dkv);
+    if (partial) store_rows32_via_lds<float, NB>(turn, ws + 32 * O0, ws_stride, rows_valid, part_acc, factor, false, lane, p.through_parts);
     else store_rows32_via_lds<OutT, NB>(turn, out + 32 * O0, out_stride, rows_valid, part_acc, factor, p.accumulate != 0, lane, p.through_dkv);
   };
   const bool parts = p.split > 1;  // the partials are packed: exactly the Hkv heads of this call per row

@@ -316,8 +316,8 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
   if (p.split > 1) {  // packed fp32 partials
     const int64_t row_stride = (int64_t)p.Hkv * kD;
     const int64_t at = (((int64_t)part * p.B + b) * p.Skv + kv_wave0) * row_stride + (int64_t)hk * kD;
-    store_rows32_via_lds<float, DB>(turn, p.ws_dv + at, row_stride, p.Skv - kv_wave0, dv, 1.f, false, lane, p.through_dkv);
-    store_rows32_via_lds<float, DB>(turn, p.ws_dk + at, row_stride, p.Skv - kv_wave0, dk, -p.scale, false, lane, p.through_dkv);
+    store_rows32_via_lds<float, DB>(turn, p.ws_dv + at, row_stride, p.Skv - kv_wave0, dv, 1.f, false, lane, p.through_parts);
+    store_rows32_via_lds<float, DB>(turn, p.ws_dk + at, row_stride, p.Skv - kv_wave0, dk, -p.scale, false, lane, p.through_parts);
   } else {
     const int64_t at = kv_wave0 * kv_row_stride + (int64_t)hk * kD;
     store_rows32_via_lds<OutT, DB>(turn, reinterpret_cast<OutT*>(p.dv) + b * p.dv_bs + at, kv_row_stride, p.Skv - kv_wave0, dv, 1.f, p.accumulate != 0, lane, p.through_dkv);

@@ -93,8 +93,10 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
   p.scale = a->scale;
   p.kappa = a->scale * 1.44269504088896340736f;
   p.accumulate = p.accumulate_dq = 0;
-  p.through_dkv = through_results(a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2);
-  p.through_dq = through_results(a->B * a->Sq * a->Hq * a->Dqk * 2);
+  // (fp32 results are updated by later steps)
+  p.through_dkv = a->dkv_dtype == PITH_BF16 && through_results(a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2);
+  p.through_dq = a->dq_dtype == PITH_BF16 && through_results(a->B * a->Sq * a->Hq * a->Dqk * 2);
+  p.through_parts = 0;
   p.split = 1;
   p.ws_dk = nullptr;
   p.ws_dv = nullptr;

@@ -475,6 +475,10 @@ __device__ __forceinline__ bf16x8 lds_read_transposed_at(const char* lo_addr, co
 template <int NB>
 constexpr int kRowsViaLdsBytes = 32 * (NB * 128 + 16);
 
+// The fp32 partial sums of the head split follow the same line, plain stores instead of nt beyond it (their reader is the next launch, and what
+// they leave in the second-level caches is written back at the end of the launch). Forward + backward, plain / sc1 / nt, us: 32 MiB 1024 x 32/4 of
+// 128 without a mask 94.7 / 92.0 / 93.6, 2 x 2048 x 16/4 of 64 105.0 / 104.3 / 105.7; 56 to 78 MiB 8 x 512 x 32/4 142.3 / 140.8 / 142.5, 3 x 768 x 32/4
+// 123.1 / 121.5 / 123.2, but 4 x 947 x 64/4 330 / 332 / 334, 4096 x 32/4 523 / 528 / 532, 4992 x 32/8 of 64 472.5 / 472.9 / 475.3.
 // Whether results of that many bytes (O, dQ, or dK and dV of a launch together) are written through the second-level caches (sc1) rather than
 // non-temporally: as long as the 8 x 4 MB of them could hold it. Either keeps the tiles of the other workgroups cached, but what went out non-temporally its next reader fetches from
 // memory. Plain / sc1 / nt, us, the forward alone and with the projection that reads O:
@@ -551,7 +555,9 @@ __device__ __forceinline__ void store_rows32_via_lds(char* lds, OutT* block, int
       if (row[it] < rows_valid) {
         OutT* dst = block + row[it] * row_stride + 4 * piece[it];
         if constexpr (sizeof(OutT) == 4) {
-          *reinterpret_cast<f32x4*>(dst) = val[it];
+          const u32x4 bits = __builtin_bit_cast(u32x4, val[it]);
+          if constexpr (decltype(through_tag)::value) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(dst), "v"(bits) : "memory");
+          else *reinterpret_cast<u32x4*>(dst) = bits;
         } else {
           u32x2 w;
           w[0] = pack_bf16x2(val[it][0], val[it][1]);
@@ -563,7 +569,7 @@ __device__ __forceinline__ void store_rows32_via_lds(char* lds, OutT* block, int
       }
     }
   };
-  if (sizeof(OutT) == 4 || !through) store(std::false_type{});
+  if (!through) store(std::false_type{});
   else store(std::true_type{});
 }
 

@@ -68,3 +68,11 @@ def test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
 ])  # fmt: skip
 def test_backward_pairs_of_a_few_rounds(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D", [
+    # eight head parts: 32 MiB of partial sums, written through, and a row of keys more; ragged keys, the last of 32 missing; four parts of 64 features
+    (1, 129, 1024, 32, 4, 128), (1, 129, 1025, 32, 4, 128), (1, 70, 95, 16, 2, 128), (2, 100, 1000, 16, 4, 64),
+])  # fmt: skip
+def test_backward_of_split_head_groups(gpu, B, Sq, Skv, Hq, Hkv, D):
+    test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, False)
