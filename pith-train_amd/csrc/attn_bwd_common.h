@@ -22,6 +22,7 @@ struct BwdParams {
   // tensors that hold exactly the heads of this call, larger when the call works on a head range of wider tensors
   int HqT, HkvT;
   int tiles, q_tiles;  // key tiles of the dK/dV kernels' grid, query tiles of the dQ kernels'
+  int chunked;  // tiles from which either takes its heads in chunks (bwd_chunked_tiles)
   int64_t q_bs, k_bs, v_bs, dout_bs, dq_bs, dk_bs, dv_bs, lse_bs, lse_hs;
   float kappa, scale;
   int accumulate, accumulate_dq;  // dK/dV and dQ kernels: add to what the outputs hold
@@ -229,9 +230,9 @@ __device__ __forceinline__ void store_rows32(OutT* block, int64_t row_stride, in
 // query tiles. Each combination streams its own Q / dO tiles. With more than 8 of them and at least kChunkedTiles
 // key tiles they are taken in chunks of 8, all key tiles of a chunk before the next chunk, so that the workgroups
 // one XCD holds at a time (block id mod 8) belong to one combination and share its Q / dO stream through that
-// XCD's L2 (see decode_block for the measurements behind the threshold).
-__device__ __forceinline__ void decode_dkdv_block(int linear, int per_level, int tiles, int& n_tile, int& pos) {
-  if (tiles >= kChunkedTiles && per_level > 8 && (per_level & 7) == 0) {
+// XCD's L2 (see decode_block for the measurements behind the threshold, bwd_chunked_tiles for `chunked`).
+__device__ __forceinline__ void decode_dkdv_block(int linear, int per_level, int tiles, int chunked, int& n_tile, int& pos) {
+  if (tiles >= chunked && per_level > 8 && (per_level & 7) == 0) {
     const int per_chunk = 8 * tiles;
     const int c = linear / per_chunk;
     const int rem = linear - c * per_chunk;
@@ -242,6 +243,16 @@ __device__ __forceinline__ void decode_dkdv_block(int linear, int per_level, int
     pos = linear - n_tile * per_level;
   }
 }
+
+// Tiles from which a backward launch takes its heads in chunks. Under the mask heaviest-first over the whole grid is worth more than
+// the caches below many tiles: in chunks 8 x 512 x 32/4 heads of 128 105 -> 116 us, 2 x 414 x 128 of 192 119 -> 137. Without one all
+// workgroups are alike, and those of a head started together read its rows through one L2, where level by level every tile fetches
+// them again. dK/dV + dQ, level by level / in chunks, us: 128 features 32 x 256 x 16 105.9 / 100.3, 8 x 512 x 16 67.9 / 65.4, 4 x 1024 x 16
+// 111.3 / 108.5, 2 x 2048 x 16 200.2 / 197.8, 8192 x 16 and 16384 x 16 equal; 64 features 32 x 300 x 16 77.4 / 74.2, 16 x
+// 512 x 16 74.1 / 71.6, 5 x 900 x 16 75.7 / 71.8, 8 x 2048 x 16 464.8 / 447.3, 2 x 1664 x 16 equal; 192 features 8 x 256 x 128 242.9 / 232.6.
+// Not for grouped heads, whose parts share keys, not rows (8 x 300 x 32/4 118 / 120), nor for calls that hand dS over, whose two
+// launches go through the images in the same order: 192 features 4096 x 16 422 / 433.
+constexpr int bwd_chunked_tiles(bool causal, bool grouped, bool hands_over) { return causal || grouped || hands_over ? kChunkedTiles : 1; }
 
 // dK/dV kernels: a workgroup owns kDkdvBlockN key rows (the grid and the head split depend on it).
 constexpr int kDkdvBlockN = 128;

@@ -541,6 +541,7 @@ int run_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks,
     blocks = (unsigned)next;
   }
   p.n_chunks = (int)n;
+  p.chunked = kChunkedTiles;  // (rows unequal, as under the mask)
   p.through_dkv = through_results(rows_before * all.B * all.Hkv * (all.Dqk + all.Dv) * 2);
   p.dk_pe_bs = args->dk_pe_bs;
   p.split = split;

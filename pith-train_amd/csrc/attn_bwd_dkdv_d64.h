@@ -55,7 +55,7 @@ __device__ __forceinline__ void body(const BwdParams& p, char* smem, int block, 
   // linear block id -> (key tile, kv head, batch, head part)
   const int per_level = p.Hkv * p.B * p.split;
   int n_tile, pos;
-  decode_dkdv_block(block, per_level, p.tiles, n_tile, pos);
+  decode_dkdv_block(block, per_level, p.tiles, p.chunked, n_tile, pos);
   const int part = pos % p.split;
   pos /= p.split;
   const int hk = pos % p.Hkv, b = pos / p.Hkv;

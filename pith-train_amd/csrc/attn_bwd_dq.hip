@@ -97,6 +97,7 @@ BwdParams make_bwd_params(const pith_attn_bwd_args* a) {
   p.through_dkv = a->dkv_dtype == PITH_BF16 && through_results(a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2);
   p.through_dq = a->dq_dtype == PITH_BF16 && through_results(a->B * a->Sq * a->Hq * a->Dqk * 2);
   p.through_parts = 0;
+  p.chunked = bwd_chunked_tiles(a->causal != 0, a->Hq != a->Hkv, ds_usable(a));
   p.split = 1;
   p.ws_dk = nullptr;
   p.ws_dv = nullptr;

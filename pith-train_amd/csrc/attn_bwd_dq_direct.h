@@ -74,7 +74,7 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   const int kvb0 = wave >> 2;  // the 32-key block of every tile this wave owns
 
   int m_tile, h, b;
-  decode_block(block, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b);
+  decode_block(block, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b, p.chunked);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
   const int q_wave0 = m0 + (wave & 3) * 32;

@@ -58,7 +58,7 @@ __device__ __forceinline__ void body(const BwdArgs<MULTI>& p, char* smem, int bl
   const int c = lane & 31, g = lane >> 5;
 
   int m_tile, h, b;
-  decode_block(block, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b);
+  decode_block(block, p.Hq, p.B, p.q_tiles, p.group, m_tile, h, b, p.chunked);
   const int hk = h / p.group;
   const int m0 = m_tile * kBM;
   const int q_wave0 = m0 + wave * 32;

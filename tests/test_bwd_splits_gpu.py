@@ -76,3 +76,9 @@ def test_backward_pairs_of_a_few_rounds(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
 ])  # fmt: skip
 def test_backward_of_split_head_groups(gpu, B, Sq, Skv, Hq, Hkv, D):
     test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, False)
+
+
+@pytest.mark.parametrize("B,Sq,Skv,H,D", [(2, 200, 300, 8, 64), (1, 130, 257, 16, 128), (3, 300, 130, 16, 192), (2, 64, 2, 8, 128), (1, 513, 513, 24, 128)])
+def test_backward_in_chunks_of_heads(gpu, B, Sq, Skv, H, D):
+    """Without a mask more than eight heads (over the batch), a multiple of eight, are taken eight at a time."""
+    test_backward_splits(gpu, B, Sq, Skv, H, H, D, False)
