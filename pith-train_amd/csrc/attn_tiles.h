@@ -197,6 +197,16 @@ struct TileMask {
   }
 };
 
+// Key tiles of a wave of a query-stationary workgroup: a wave whose 32 rows all lie beyond the last one (ragged Sq) is done with the first
+// tile and only moves tiles for the others. It used to multiply to the end for nothing, under the mask in the longest workgroup. us, before /
+// after: forward 8 x 643 x 64/4 heads of 128 causal 95.1 / 90.6 (27 % of the work was padding), 8200 x 16 246 / 237, 4100 x 32/4 136.7 / 131.0, 3 x
+// 1999 x 32/4 100.7 / 99.4, 4 x 1030 x 16 of 192 32.5 / 31.0, 8 x 1290 x 16/4 of 64 39.7 / 38.0; forward + backward 2 x 414 x 128 of 192 171.1 / 166.1, 5
+// x 400 x 32/4 of 128 110.3 / 105.8; shares 4120 x 16 of 192 1609 / 1535, 4100 x 32/4 2605 / 2551. Without a mask only in the forward of small
+// workgroups (8 x 643 x 64/4 147 / 140, 6 x 530 x 32/4 42.0 / 39.8, 8 x 1290 x 32/8 of 64 129 / 126): the others know there that all waves walk as far
+// as their workgroup, and lose more in the loops without it (256-row forward 8200 x 16 570 / 638, 4 x 1564 x 16 85 / 89; dQ 4100 x 8/2 362 / 371,
+// 3 x 3457 x 4 of 64 206 / 211).
+__device__ __forceinline__ int tiles_of_wave(int tiles, int q_wave0, int sq) { return q_wave0 < sq ? tiles : min(tiles, 1); }
+
 // ---------------------------------------------------------------------------------------------
 // 128-feature tiles moved global memory -> LDS directly (global_load_lds_dwordx4), without
 // passing through registers. One wavefront instruction moves 64 pieces of 16 bytes to 1 KB of

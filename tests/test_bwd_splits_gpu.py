@@ -82,3 +82,13 @@ def test_backward_of_split_head_groups(gpu, B, Sq, Skv, Hq, Hkv, D):
 def test_backward_in_chunks_of_heads(gpu, B, Sq, Skv, H, D):
     """Without a mask more than eight heads (over the batch), a multiple of eight, are taken eight at a time."""
     test_backward_splits(gpu, B, Sq, Skv, H, H, D, False)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,S,Hq,Hkv,D", [
+    # one, 32, 33, 64, 65 and 97 rows in the last workgroup of 128: three to no waves without any, as one grid and as two launches
+    (1, 257, 4, 2, 128), (1, 288, 4, 4, 64), (2, 161, 6, 3, 64), (1, 192, 4, 2, 192), (2, 193, 2, 2, 192), (1, 225, 4, 1, 128),
+    (6, 385, 40, 40, 192), (4, 1025, 32, 8, 128), (8, 643, 16, 4, 128),
+])  # fmt: skip
+def test_waves_without_rows(gpu, B, S, Hq, Hkv, D, causal):
+    test_backward_splits(gpu, B, S, S, Hq, Hkv, D, causal)
