@@ -82,10 +82,52 @@ namespace {
 // 67.1 / 51.7 / 73.2 / 56.6.
 enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter, kSmall };
 
+// Calls against one chunk a little above a whole round of 128-row workgroups, W of them per compute unit (a ragged length is enough): the
+// last round of FULL, DUO or HALF would hold few of them, which a split with more or shorter ones spreads. us, by W:
+//   causal d128  HALF / QUARTER   8448 x 4 (1.03) 100.6 / 91.6, 9000 x 4 (1.11) 115.7 / 106.3, 9984 x 4 (1.22) 124.6 / 128.6, 4224 x 8 (1.03) 53.9 / 54.0
+//                FULL / HALF      4220 x 16 (2.06) 88.9 / 80.6, 4400 x 16 (2.19) 94.6 / 88.4, 4700 x 16 (2.31) 102.4 / 99.3, 5100 x 16 (2.5) 116.4 / 114.9,
+//                                 8400 x 8 (2.06) 169.7 / 145.0, 16640 x 4 (2.03) 327.7 / 267.5, 10200 x 8 (2.5) 222.9 / 215.8, 20900 x 4 (2.56) 450.9 /
+//                                 435.7, 12300 x 8 (3.03) 292.6 / 300.8; 2100 x 32 (2.12) DUO 46.4 / 49.1
+//          d192  HALF / QUARTER   4224 x 8 (1.03) 71.4 / 62.3, 4600 x 8 (1.12) 78.2 / 74.1, 5000 x 8 (1.25) 86.1 / 85.4, 5400 x 8 (1.34) 93.9 / 95.8, 8448 x 4 (1.03)
+//                                 134.0 / 108.6, 9984 x 4 (1.22) 165.4 / 152.7, 10700 x 4 (1.31) 179.0 / 171.1, 2112 x 16 (1.06) 37.9 / 40.5
+//                HALF / SMALL     1100 x 32 (1.12) 24.7 / 23.5, 1250 x 32 (1.25) 27.8 / 27.1, 2300 x 16 (1.12) 42.6 / 41.2, 2560 x 16 (1.25) 47.7 / 46.9
+//                DUO / HALF       4220 x 16 (2.06) 106.3 / 100.6, 4400 x 16 (2.19) 111.4 / 111.0, 8400 x 8 (2.06) 201.9 / 180.5, 8900 x 8 (2.19) 219.5 / 206.5,
+//                                 16640 x 4 (2.03) 390.4 / 340.4, 18400 x 4 (2.25) 450.3 / 426.6, 9500 x 8 (2.34) 240.6 / 237.5, 2100 x 32 (2.12) 56.9 / 59.0
+//          d64   TEAMS, to 6144 keys SMALL / QUARTER  4224 x 8 (1.03) 39.5 / 36.2, 4600 x 8 (1.12) 42.3 / 42.3, 8448 x 4 (1.03) 77.7 / 62.3, 9984 x 4 (1.22) 91.6 / 85.8,
+//                                 10700 x 4 (1.31) 98.3 / 97.3, 2112 x 16 (1.06) 21.6 / 22.9
+//                DUO / SMALL      8400 x 8 (2.06) 112.4 / 93.3, 10200 x 8 (2.5) 144.9 / 126.9, 20900 x 4 (2.56) 295.6 / 258.6, 3 x 8064 x 4 (2.95) 126.1 / 119.9,
+//                                 12300 x 8 (3.03) 188.5 / 179.9, 6200 x 16 (3.06) 96.9 / 95.4
+//   full   d128  FULL / HALF      2100 x 32 (2.12) 101.0 / 94.5, 2400 x 32 (2.38) 116.1 / 108.3, 2700 x 32 (2.75) 129.1 / 125.3, 3000 x 32 (3) 142.0 / 142.7, 4400 x
+//                                 16 (2.19) 198.4 / 183.8, 5300 x 16 (2.62) 237.4 / 226.3, 17500 x 4 (2.14) 749.8 / 692.9; 2 x 1400 x 32 (2.75) DUO 70.3 / 72.3
+bool above_a_round(const pith_attn_fwd_args* a, int64_t wgs, int64_t cus, Split* split) {
+  const auto at_most = [&](int64_t n, int64_t d) { return d * wgs <= n * cus; };  // W <= n / d
+  const int64_t keys = a->Skv;
+  if (wgs <= cus) return false;
+  if (!a->causal) {
+    *split = Split::kHalf;
+    return a->Dqk == 128 && wgs > 2 * cus && at_most(11, 4) && keys >= 2048;
+  }
+  if (keys != a->Sq) return false;  // several chunks
+  if (a->Dqk == 64) {
+    *split = wgs > 2 * cus ? Split::kSmall : Split::kQuarter;
+    return wgs > 2 * cus ? at_most(25, 8) && keys > 6144 : (at_most(17, 16) && keys >= 4096) || (at_most(5, 4) && keys >= 8192);
+  }
+  const bool d192 = a->Dqk == 192;
+  if (wgs > 2 * cus) {
+    *split = Split::kHalf;
+    return d192 ? (at_most(17, 8) && keys >= 4096) || (at_most(9, 4) && keys >= 8192) : at_most(5, 2) && keys >= 4096;
+  }
+  *split = d192 && keys < 2600 ? Split::kSmall : Split::kQuarter;
+  if (*split == Split::kSmall) return at_most(5, 4) && keys >= 1024;
+  return d192 ? (at_most(9, 8) && keys >= 4096) || (at_most(4, 3) && keys >= 8192) : at_most(23, 20) && keys >= 8192;
+}
+
 // `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50).
 Split pick_split(const pith_attn_fwd_args* a, int mean) {
   const int64_t cus = compute_units_or_default();
   const int64_t wgs = ((a->Sq + 127) / 128) * a->Hq * a->B, wgs64 = ((a->Sq + 63) / 64) * a->Hq * a->B;  // of 128 and 64 rows
+  Split above;
+  if (above_a_round(a, wgs, cus, &above) && wgs64 > 2 * cus) return above;
   const bool d64 = a->Dqk == 64, unequal = mean <= 70;  // HALF is 3 % slower than DUO at 0.75, 5-10 % above
   if (a->Skv > 64) {  // (64 features to 6144 keys: 4404 x 16 61.8 -> 52.2, 4998 x 16 75 -> 67, 5938 x 16 95 -> 91)
     if (wgs64 <= cus) return a->Skv > 512 ? Split::kQuarter : Split::kSmall;
@@ -109,7 +151,9 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
   // for rows of a few workgroups: 8 x 512 x 128 155 -> 167)
   const bool many_heads = a->Sq >= 1024 && a->Skv == a->Sq && a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2 >= 224ll << 20;
-  if (a->Dqk == 128 && (unequal ? (a->Sq >= 3072 || many_heads) && wgs > 2 * cus : a->Skv > 1024 && wgs > cus)) return Split::kFull;
+  // (without a mask, FULL / DUO: 1100 x 32/4 30.0 / 28.4, 8 x 1100 x 16 104.3 / 97.4, 2 x 1400 x 32/4 73.2 / 70.3, 1500 x 32/4 39.7 / 40.0, 1999 x 32/4 60.9 /
+  // 61.1, 3457 x 32/4 176 / 183)
+  if (a->Dqk == 128 && (unequal ? (a->Sq >= 3072 || many_heads) && wgs > 2 * cus : a->Skv > (a->causal ? 1024 : 1408) && wgs > cus)) return Split::kFull;
   return Split::kDuo;
 }
 

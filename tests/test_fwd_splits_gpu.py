@@ -113,3 +113,14 @@ def test_forward_small_workgroups(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
 @pytest.mark.parametrize("rows,D", [(66, 64), (100, 128), (130, 192)])
 def test_shares_of_small_workgroups(gpu, rows, D, layout):
     test_shares_of_teams_in_turns(gpu, rows, D, layout)
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,causal", [
+    # a row above one and two whole rounds of 128-row workgroups on 256 compute units, and on both sides of the lines above them
+    (1, 8193, 4, 1, 128, True), (1, 9473, 4, 1, 128, True), (1, 4097, 16, 2, 128, True), (1, 5121, 16, 2, 128, True), (1, 4097, 8, 8, 192, True),
+    (1, 4609, 8, 8, 192, True), (1, 2113, 16, 16, 192, True), (1, 2599, 16, 16, 192, True), (1, 4097, 16, 16, 192, True), (1, 4353, 16, 16, 192, True),
+    (1, 4097, 8, 2, 64, True), (1, 4353, 8, 2, 64, True), (1, 8193, 8, 2, 64, True), (2, 6145, 8, 2, 64, True), (1, 2049, 32, 4, 128, False),
+    (1, 2817, 32, 4, 128, False), (1, 1408, 24, 3, 128, False), (1, 1409, 24, 3, 128, False),
+])  # fmt: skip
+def test_forward_above_whole_rounds(gpu, B, S, Hq, Hkv, D, causal):
+    test_forward_splits(gpu, B, S, S, Hq, Hkv, D, causal)
