@@ -95,8 +95,37 @@ struct Reduction {
   }
 };
 
+// The head split doubles until the workgroups wanted are there, which leaves up to twice as many. Whether half of those do better, a
+// round of them without a mask, one to two (workgroups per unit below) under it: they leave half of the partial sums, which make a round
+// trip through memory, and spend half as often what a workgroup spends around its products (7 us). Long walks lose: the wanted number
+// balanced them, and in a call that hands dS over nothing else fills the units. Forward + backward, more / half, us, 32/4 heads
+// unless others are named:
+//   causal d128  1.6 - 1.9   3 x 1100 210 / 185, 3 x 1200 230 / 204, 2 x 1700 261 / 235, 5 x 700 183 / 156, 1790 x 64/4 274 / 249, 5 x 1500 x 16/4
+//                            275 / 253, 3600 446 / 428, 3900 502 / 483, 5 x 2600 x 8/2 339 / 328
+//                1.4 - 1.5   2 x 700 x 64/4 145 / 127, 9 x 1200 x 8/2 185 / 169, 9 x 600 231 / 220, 1300 x 64/4 181 / 172, 2900 338 / 333, 3000 x 64/4
+//                            600 / 617
+//                1.0 - 1.3   no hand-over: 3 x 768 127 / 116, 2 x 1100 147 / 131, 5 x 400 104 / 90, 2200 218 / 204, 4 x 2200 x 8/2 224 / 211; handing
+//                            over: 9 x 512 186 / 175, 7 x 700 210 / 201, 5 x 900 234 / 236, 4 x 1152 x 64/4 454 / 484, 3 x 1500 303 / 321, 2 x 2100
+//                            353 / 396, 3 x 2900 846 / 944, 4300 632 / 738
+//                short rows  24 x 128 112 / 92, 20 x 160 111 / 97, 10 x 200 x 64/4 143 / 125
+//   full   d128  1100 134.7 / 119.6, 1300 162 / 150, 1790 253 / 242, 4 x 520 138 / 126, 3 x 700 155 / 145, 3 x 1408 x 8/2 153 / 140, 2 x 2100 x 8/2
+//                209 / 188, 2700 566 / 530, 20 x 160 118 / 102; 5000 x 8/2 442 / 462, 3500 x 64/4 1509 / 1523. Calls that hand dS over leave at most
+//                a quarter of the units idle (ds_handover_pays).
+//   d64          causal 9 x 1100 x 32/8 303 / 280, 5 x 1290 x 32/8 236 / 216, 4300 x 32/8 369 / 361, 20 x 250 x 32/8 95 / 84, 3 x 2200 x 16/4 equal;
+//                full 10 x 600 x 16/4 114 / 106, 4 x 1290 x 32/8 305 / 295, 2600 x 32/8 281 / 274, 2200 x 32/8 equal
+// Not for several chunks, whose workgroups are unequal: 2 x 1314 x 8/2, zigzag 188 / 195, 2300 x 64/4 1838 / 1939, but 1100 contiguous 405 / 384.
+bool half_as_many(const pith_attn_bwd_args* a, int64_t wgs) {
+  const int64_t cus = compute_units_or_default();
+  if (a->Dqk == 192) return false;
+  if (a->Dqk == 64) return a->Sq <= 5120;
+  const bool hands_over = (a->Sq + 511) / 512 * a->Hq * a->B >= cus;  // (512 query rows per workgroup of its dQ)
+  if (!a->causal) return a->Sq <= 2816 && (!hands_over || 4 * wgs >= 3 * cus);
+  if (5 * wgs >= 8 * cus) return a->Sq <= 4096;
+  return a->Sq <= (hands_over && 8 * wgs < 11 * cus ? 768 : 2304);
+}
+
 // tiles: key tiles of the launch, over all of its chunks
-int pick_split(const pith_attn_bwd_args* a, int64_t tiles) {
+int pick_split(const pith_attn_bwd_args* a, int64_t tiles, bool chunks = false) {
   const int64_t group = a->Hq / a->Hkv;
   const int64_t base = tiles * a->Hkv * a->B;
   int split = 1;
@@ -106,6 +135,7 @@ int pick_split(const pith_attn_bwd_args* a, int64_t tiles) {
   // within 2 %).
   const int64_t want = (a->causal ? 2 : 1) * (a->Dqk == 64 ? 2 : 1) * (int64_t)compute_units_or_default();
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
+  if (!chunks && split > 1 && base * split > want && half_as_many(a, base * split / 2)) split /= 2;
   return split;
 }
 
@@ -427,7 +457,7 @@ int64_t chunk_ds_head_bytes(int64_t sq, const pith_key_chunk& c, bool diagonal) 
 
 int pick_chunks_split(pith_attn_bwd_args a, int64_t tiles) {
   a.causal = 1;  // the chunks' workgroups are unequal in any case
-  return pick_split(&a, tiles);
+  return pick_split(&a, tiles, true);
 }
 
 // The launches of a call of several chunks: one grid or two, and which kind goes first in one.

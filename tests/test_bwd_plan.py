@@ -265,3 +265,15 @@ def test_share_of_64_features_in_two_launches(gpu):
         assert torch.equal(whole[0][:, :, qh], one[0])
         for j in range(cp):
             assert torch.equal(whole[1][j][:, :, kh], one[1][j]) and torch.equal(whole[2][j][:, :, kh], one[2][j])
+
+
+@pytest.mark.parametrize("causal,b,s,hq,hkv,d,split", [
+    # wanted 512 workgroups under the mask and 256 without: half of what doubling leaves, on either side of the lines
+    (1, 3, 768, 32, 4, 128, 4), (1, 2, 2304, 16, 4, 128, 2), (1, 1, 2304, 32, 4, 128, 4), (1, 1, 2305, 32, 4, 128, 8), (1, 3, 1200, 32, 4, 128, 4),
+    (1, 3, 1500, 32, 4, 128, 4), (1, 1, 4096, 32, 4, 128, 4), (1, 1, 4097, 32, 4, 128, 4), (1, 1, 3900, 32, 4, 128, 4), (1, 9, 768, 32, 4, 128, 2),
+    (1, 9, 769, 32, 4, 128, 2), (1, 24, 128, 32, 4, 128, 4), (0, 1, 1100, 32, 4, 128, 4), (0, 2, 1100, 64, 4, 128, 4), (0, 1, 2816, 32, 4, 128, 2),
+    (0, 1, 2817, 32, 4, 128, 4), (1, 9, 1100, 32, 8, 64, 1), (1, 1, 5120, 32, 8, 64, 2), (1, 1, 5121, 32, 8, 64, 4), (0, 4, 1290, 32, 8, 64, 1), (1, 3, 768, 32, 4, 192, 8),
+])  # fmt: skip
+def test_head_split_is_halved_where_that_is_faster(causal, b, s, hq, hkv, d, split):
+    """As measured (table at half_as_many)."""
+    assert _plan(b, s, s, hq, hkv, causal, d).dkdv_split == split
