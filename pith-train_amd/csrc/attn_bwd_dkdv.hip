@@ -113,9 +113,15 @@ struct Reduction {
 //                a quarter of the units idle (ds_handover_pays).
 //   d64          causal 9 x 1100 x 32/8 303 / 280, 5 x 1290 x 32/8 236 / 216, 4300 x 32/8 369 / 361, 20 x 250 x 32/8 95 / 84, 3 x 2200 x 16/4 equal;
 //                full 10 x 600 x 16/4 114 / 106, 4 x 1290 x 32/8 305 / 295, 2600 x 32/8 281 / 274, 2200 x 32/8 equal
-// Not for several chunks, whose workgroups are unequal: 2 x 1314 x 8/2, zigzag 188 / 195, 2300 x 64/4 1838 / 1939, but 1100 contiguous 405 / 384.
-bool half_as_many(const pith_attn_bwd_args* a, int64_t wgs) {
+// Several chunks, whose workgroups are unequal, in one grid with more than one dQ workgroup per unit to even them out: four ranks, 1100 contiguous
+// rank 3 392 / 371, 2 x 900 zigzag 328 / 310, 600 x 64/4 173 / 163, 2 x 2400 x 8/2 500 / 459, 5000 x 8/2 contiguous 1177 / 1117, 8200 x 8/2 2497 / 2430, 3300
+// equal. Not with fewer (2 x 1314 x 8/2 188 / 195, eight ranks 900 335 / 342) nor in two launches (2300 x 64/4 1838 / 1939, 2 x 1371 x 64/4 836 / 865).
+bool half_as_many(const pith_attn_bwd_args* a, int64_t wgs, bool chunks) {
   const int64_t cus = compute_units_or_default();
+  if (chunks) {
+    const int64_t q_wgs = (a->Sq + 127) / 128 * a->Hq * a->B;
+    return a->Dqk == 128 && q_wgs > cus && q_wgs <= 4 * cus;
+  }
   if (a->Dqk == 192) return false;
   if (a->Dqk == 64) return a->Sq <= 5120;
   const bool hands_over = (a->Sq + 511) / 512 * a->Hq * a->B >= cus;  // (512 query rows per workgroup of its dQ)
@@ -135,7 +141,7 @@ int pick_split(const pith_attn_bwd_args* a, int64_t tiles, bool chunks = false) 
   // within 2 %).
   const int64_t want = (a->causal ? 2 : 1) * (a->Dqk == 64 ? 2 : 1) * (int64_t)compute_units_or_default();
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
-  if (!chunks && split > 1 && base * split > want && half_as_many(a, base * split / 2)) split /= 2;
+  if (split > 1 && base * split > want && half_as_many(a, base * split / 2, chunks)) split /= 2;
   return split;
 }
 

@@ -277,3 +277,12 @@ def test_share_of_64_features_in_two_launches(gpu):
 def test_head_split_is_halved_where_that_is_faster(causal, b, s, hq, hkv, d, split):
     """As measured (table at half_as_many)."""
     assert _plan(b, s, s, hq, hkv, causal, d).dkdv_split == split
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,cp,rank,layout,d,split", [
+    # more than 512 workgroups of all chunks; dQ workgroups of 128 rows: 257 to 1024 in the one grid, 256, more
+    (1, 1100, 32, 4, 4, 3, "contiguous", 128, 2), (2, 2400, 8, 2, 4, 3, "zigzag", 128, 2), (1, 1024, 32, 4, 4, 3, "contiguous", 128, 4), (1, 900, 32, 4, 8, 4, "zigzag", 128, 4),
+    (1, 2300, 64, 4, 4, 2, "contiguous", 128, 4), (1, 2048, 64, 4, 4, 2, "contiguous", 128, 2), (1, 4352, 16, 4, 4, 2, "contiguous", 64, 4),
+])  # fmt: skip
+def test_head_split_of_shares(b, s, hq, hkv, cp, rank, layout, d, split):
+    assert _share_plan(b, s, hq, hkv, cp, rank, layout, d).dkdv_split == split
