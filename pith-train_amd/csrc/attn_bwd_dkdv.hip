@@ -234,12 +234,20 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_d
 // unit want anyway. Beyond, one grid pays where either kernel alone would leave its last round half empty, against what the
 // two-workgroup dQ kernel is faster by; W = dQ workgroups per compute unit, apart -> together, inputs from memory, us:
 //   d128 causal   W 1.5: 1 x 2304 x 16 108 -> 91, 1 x 6144 x 8/2 289 -> 265, 6 x 512 x 16/4 68 -> 61; 1.75: 1 x 1792 x 32/4
-//                 122 -> 121; 2: 1 x 2048 x 32/4 154 -> 150, 1 x 8192 x 8/2 446 -> 449; 2.25-2.5: 1 x 2304 x 32/4 191 -> 181,
-//                 1 x 5120 x 16 377 -> 351, 5 x 1024 x 16/4 127 -> 127
+//                 122 -> 121; 2: 1 x 2048 x 32/4 154 -> 150, 1 x 8192 x 8/2 446 -> 449; 2.25: 1 x 2304 x 32/4 191 -> 181
 //        full     W 1.5: 1 x 1536 x 32/4 157 -> 145; 1.7: 1 x 3456 x 16 307 -> 329; 2: 1 x 4096 x 16 412 -> 422;
 //                 2.2: 1 x 4480 x 16 628 -> 520, 1 x 2304 x 32/4 383 -> 289
-//   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186, 3 x 1024 x 16 92 -> 94; 1.7: 1 x 3456 x 16
+//   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186; 1.7: 1 x 3456 x 16
 //                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
+// and with the forward, since the head split halves (half_as_many):
+//   d128 causal   W 1.6: 13 x 500 x 8/2 86.5 -> 80.7; 2: 2 x 1000 x 32/4 128 -> 125, 4 x 500 x 32/4 96 -> 98; 2.25-2.8: 3 x 768 x 32/4 116.4 ->
+//                 107.4, 3 x 700 108.4 -> 100.3, 6 x 384 89 -> 86, 5 x 450 101 -> 98, 1 x 2700 322 -> 309, 1 x 1500 x 60/4 546 -> 505, 3 x 1000 x 30/2 386 ->
+//                 352, 3 x 1900 x 16 234 -> 231; 2.9-3.3: 1 x 6000 x 16 652 -> 629, 1 x 3000 x 32/4 369 -> 361, 1 x 3300 423 -> 410, 1 x 13000 x 8/2 1461
+//                 -> 1429, 1 x 3100 x 34/2 1209 -> 1121; 3.5: 1 x 3500 x 32/4 456 -> 459, 7 x 900 x 16 equal; 5: 20 x 160 x 32/4 99 -> 107
+//        full     W 1.75-2: 1 x 1700 x 32/4 227 -> 235, 2 x 900 148 -> 153; 2.6-3.1: 3 x 900 x 28/4 257 -> 214, 1 x 1400 x 62/2 989 -> 917, 1 x 2816 x 32/4 578
+//                 -> 561, 1 x 6000 x 16 and 1 x 12500 x 8/2 equal; 3.25-3.5: 1 x 3300 x 32/4 763 -> 772, 7 x 900 x 16 263 -> 267
+//   d192 causal   W 1.1-1.4: 2 x 1100 x 16 109.6 -> 95.6, 2 x 1400 x 16 139 -> 128, 1 x 1300 x 32 129 -> 119, 3 x 800 x 16 92.7 -> 89.2, 3 x 384 x 32 81 -> 78;
+//                 1.5: 3 x 1024 x 16 120 -> 116, 1 x 1500 x 32 equal; 2.25: 9 x 400 x 16 99 -> 105
 // Several chunks, whose dK/dV workgroups are more unequal, gain 1-5 % up to two per unit (2048 x 32/4 of 128, 4 ranks,
 // zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081). 128 features: up to four, where two launches lost
 // even to one pair of them per ring step (in brackets): 4096 x 32/4, 4 ranks, rank 0 1889 -> 1728 (1724); 9216 x 8/2, 8
@@ -263,8 +271,9 @@ bool one_grid(const pith_attn_bwd_args* a, int64_t dkdv_wgs, bool chunks) {
   if (a->Dqk == 64) return (q_wgs + dkdv_wgs) * 256 < (1ll << 32);
   if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
   if (q_wgs <= cus) return true;
-  if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= 1536;
-  return 2 * q_wgs <= 3 * cus || (2 * q_wgs <= 5 * cus && (a->causal ? a->Skv >= 1024 : q_wgs > 2 * cus));
+  if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= (a->causal ? 256 : 1536);
+  if (2 * q_wgs <= 3 * cus) return true;
+  return a->causal ? 3 * q_wgs <= 10 * cus && a->Skv >= 384 : q_wgs > 2 * cus && 10 * q_wgs <= 31 * cus;
 }
 
 // Workgroups of the dQ kernel that reads handed-over dS.

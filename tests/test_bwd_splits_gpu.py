@@ -92,3 +92,12 @@ def test_backward_in_chunks_of_heads(gpu, B, Sq, Skv, H, D):
 ])  # fmt: skip
 def test_waves_without_rows(gpu, B, S, Hq, Hkv, D, causal):
     test_backward_splits(gpu, B, S, S, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("B,S,H,D,causal", [
+    # 3.32 and 3.34 dQ workgroups per compute unit under the mask, 383 and 384 keys; 3.09 and 3.11 without; 192 features from 256 keys on
+    (1, 640, 170, 128, True), (1, 640, 171, 128, True), (1, 383, 171, 128, True), (1, 384, 171, 128, True), (1, 513, 158, 128, False),
+    (1, 513, 159, 128, False), (1, 255, 150, 192, True), (1, 256, 150, 192, True), (1, 300, 128, 192, True),
+])  # fmt: skip
+def test_backward_pairs_at_the_lines_of_one_grid(gpu, B, S, H, D, causal):
+    test_backward_splits(gpu, B, S, S, H, H, D, causal)
