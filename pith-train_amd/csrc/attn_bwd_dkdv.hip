@@ -124,7 +124,8 @@ bool half_as_many(const pith_attn_bwd_args* a, int64_t wgs, bool chunks) {
   }
   if (a->Dqk == 192) return false;
   if (a->Dqk == 64) return a->Sq <= 5120;
-  const bool hands_over = (a->Sq + 511) / 512 * a->Hq * a->B >= cus;  // (512 query rows per workgroup of its dQ)
+  // (ds_handover_pays, 512 query rows per workgroup of its dQ)
+  const bool hands_over = (a->Sq + 511) / 512 * a->Hq * a->B >= cus || 100 * a->Sq * a->Hq * a->B >= 69 * 512 * cus;
   if (!a->causal) return a->Sq <= 2816 && (!hands_over || 4 * wgs >= 3 * cus);
   if (5 * wgs >= 8 * cus) return a->Sq <= 4096;
   return a->Sq <= (hands_over && 8 * wgs < 11 * cus ? 768 : 2304);

@@ -473,7 +473,14 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
 }
 
 // Whether a dQ kernel that reads handed-over dS (512 query rows per workgroup) beats recomputing the scores: it has to fill the
-// device. W = workgroups per compute unit; forward + backward, inputs changing, handing over / recomputing, us:
+// device, or two thirds of it with rows. By those rows in 512 per compute unit, forward + backward, handing over / recomputing, us (to 16384 rows):
+//   causal  0.5-0.65   2100 x 32/4 heads 214 / 193, 3 x 768 x 32/4 117 / 105, 2 x 1200 x 32/4 151 / 144, 2 x 1300 x 32/4 168 / 164, 2500 x 32/4 264 / 270, 5 x 512 x 32
+//                      112 / 107, 5 x 1000 x 16/4 138 / 137    0.68   7 x 400 x 32/4 119 / 116
+//           0.69-0.75  2816 x 32/4 305 / 318, 3 x 1900 x 16 219 / 229, 3 x 960 x 32/4 140 / 147, 3000 x 32/4 335 / 357, 1500 x 64/4 194 / 202, 6000 x 16 588 / 615
+//           0.8-0.95   13 x 512 x 16 131 / 139, 7 x 500 x 32/4 132 / 139, 13000 x 8/2 1298 / 1396, 3500 x 32/4 415 / 445, 7 x 1024 x 16 182 / 193, 15000 x 8/2 1644 / 1795
+//   full    0.69-0.75  3 x 1900 x 16 376 / 404, 3 x 1000 x 32/4 231 / 237, 1500 x 64/4 325 / 342, 6000 x 16 1067 / 1173
+//           0.8-0.95   13 x 512 x 16 160 / 179, 3500 x 32/4 772 / 829, 7 x 512 x 32/4 155 / 167, 15000 x 8/2 3202 / 3478
+// From a full device on, W = workgroups per compute unit; forward + backward, inputs changing, handing over / recomputing, us:
 //   causal  W 1     4096 x 32/4 heads 561 / 576, 8192 x 16 1030 / 1059, 2 x 2048 x 32/4 323 / 332, 4 x 1024 x 32/4 204 / 215, 8 x 512 x 32/4 148 / 162
 //           W 1.12  9216 x 16 1378 / 1392, 3 x 1536 x 32/4 305 / 312, 9 x 512 x 32/4 189 / 190
 //           W 1.25  5120 x 32/4 891 / 914, 2 x 2560 x 32/4 496 / 502       W 1.5   6144 x 32/4 1229 / 1265, 6 x 1024 x 32/4 310 / 317,
@@ -502,14 +509,18 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
 //                          640 and more 8 x 640 x 32/8 232 / 233, 16 x 640 x 32/4 439 / 441, 8 x 720 x 16 155 / 164
 //   causal, from 513 on    4 x 513 x 32/4 98 / 99, 4 x 600 x 32/4 113 / 110, 8 x 600 x 32/4 167 / 173, 4 x 600 x 64/4 168 / 174, 8 x 1025 x 32/4 333 / 354
 bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
-  if (cus <= 0 || (sq + 511) / 512 * hq * b < cus) return false;
+  const bool fills = (sq + 511) / 512 * hq * b >= cus;
+  if (cus <= 0 || (!fills && (sq > 16384 || 100 * sq * hq * b < 69 * 512 * cus))) return false;
   if (sq <= 256 || (!causal && sq > 512 && sq < 640)) return false;
   pith_attn_bwd_args a = {};
   a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = a.Dv = 128; a.causal = causal;
   pith_attn_bwd_plan_t plan;
   if (pith_attn_bwd_plan(&a, &plan) != PITH_OK) return false;
   const int64_t key_tiles = (skv + plan.dkdv_rows - 1) / plan.dkdv_rows * plan.dkdv_rows / 128;
-  return 4 * key_tiles * hkv * b * plan.dkdv_split >= 3 * cus;
+  const int64_t dkdv_wgs = key_tiles * hkv * b * plan.dkdv_split;
+  // (causal 7900 x 12/4, 248 of them: 887 / 837)
+  if (!fills && causal && 2 * dkdv_wgs < 3 * cus) return false;
+  return 4 * dkdv_wgs >= 3 * cus;
 }
 
 // The same for (192, 128): its dQ kernel takes 256 rows per workgroup.
@@ -570,7 +581,8 @@ bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const st
   for (const auto& [sq, skv, causal, heads] : steps) {
     const double work = (double)sq * (double)skv * (causal ? 0.5 : 1.0);
     all += work;
-    if (heads == 0) continue;
+    // (the measured shares handed over in steps that fill the device)
+    if (heads == 0 || (dqk == 128 && (sq + 511) / 512 * (hq / hkv * heads) * b < cus)) continue;
     handed += work;
     if (causal) continue;
     pith_attn_bwd_args a = {};

@@ -286,3 +286,13 @@ def test_head_split_is_halved_where_that_is_faster(causal, b, s, hq, hkv, d, spl
 ])  # fmt: skip
 def test_head_split_of_shares(b, s, hq, hkv, cp, rank, layout, d, split):
     assert _share_plan(b, s, hq, hkv, cp, rank, layout, d).dkdv_split == split
+
+
+@pytest.mark.parametrize("causal,b,s,hq,hkv,pays", [
+    # 0.687 / 0.69 of the device filled with rows, to 16384 of them; enough dK/dV workgroups under the mask
+    (True, 1, 2816, 32, 4, False), (True, 1, 2827, 32, 4, True), (False, 1, 2827, 32, 4, True), (True, 3, 768, 32, 4, False), (True, 1, 1450, 64, 4, True),
+    (True, 1, 16384, 7, 7, True), (True, 1, 16385, 7, 7, False), (True, 1, 7900, 12, 4, False), (False, 1, 7900, 12, 4, True),
+])  # fmt: skip
+def test_handover_of_grids_that_two_thirds_fill_the_device(causal, b, s, hq, hkv, pays):
+    """As measured (table at ds_handover_pays)."""
+    assert native.ds_handover_pays(b, s, s, hq, hkv, causal, UNITS) == pays
