@@ -253,8 +253,10 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_d
 // zigzag, rank 0: 525 -> 498 us; 4096 x 16 of 192, rank 3: 1099 -> 1081). 128 features: up to four, where two launches lost
 // even to one pair of them per ring step (in brackets): 4096 x 32/4, 4 ranks, rank 0 1889 -> 1728 (1724); 9216 x 8/2, 8
 // ranks, contiguous 5439 -> 4593 (4746); 12288 x 8/2, rank 0 4120 -> 3875 (3878), rank 1 4040 -> 3721 (3930); 3584 x 32/4,
-// rank 3 1286 -> 1295 (1417); above four dS is handed over wherever memory allows it. 192 features with three lose (6144 x
-// 16: 2385 -> 2413).
+// rank 3 1286 -> 1295 (1417). 192 features with three lose (6144 x 16: 2385 -> 2413). 128 features also up to eight where a share
+// is more than a whole chunk beside its own (forward + backward, 4 ranks, apart -> together): 4.2 17000 x 8/2 10670 -> 9880; 4.5 2300 x 64/4
+// 1588 -> 1488; 5 2 x 1200 x 64/4 974 -> 882, 5120 x 32/4 3272 -> 3232; 6 6144 x 32/4 4866 -> 4590; 7 2 x 1700 x 64/4 contiguous 1994 -> 1928; 8 8 x 1024 x 32/4
+// equal; 9 to 11 9216 x 32/4 10400 -> 10540, 11264 x 32/4 15150 -> 15480; two ranks 2 x 3000 x 32/4 contiguous 1733 -> 1749.
 // At 64 features both kernels fit two workgroups to a unit, and one grid is faster for chunk pairs and most shares: forward +
 // backward, apart -> together, 1 x 32768 x 8/2 heads causal 4808 -> 4660 us, 1 x 16384 x 16/4 2423 -> 2359, 16 x 1024 x 32/8 415 ->
 // 404, 1 x 16384 x 16/4 without a mask 4684 -> 4630; shares, zigzag, 4096 x 64/8, 4 ranks, rank 0 2740 -> 2543, 8192 x 32/8 rank 1
@@ -270,7 +272,7 @@ bool one_grid(const pith_attn_bwd_args* a, int64_t dkdv_wgs, bool chunks) {
   const int64_t cus = compute_units_or_default();
   const int64_t q_wgs = ((a->Sq + 127) / 128) * a->Hq * a->B;
   if (a->Dqk == 64) return (q_wgs + dkdv_wgs) * 256 < (1ll << 32);
-  if (chunks) return q_wgs <= (a->Dqk == 128 ? 4 : 2) * cus;
+  if (chunks) return q_wgs <= (a->Dqk == 128 ? (a->Skv > 2 * a->Sq ? 8 : 4) : 2) * cus;
   if (q_wgs <= cus) return true;
   if (a->Dqk == 192) return 2 * q_wgs <= 3 * cus && a->Skv >= (a->causal ? 256 : 1536);
   if (2 * q_wgs <= 3 * cus) return true;

@@ -296,3 +296,9 @@ def test_head_split_of_shares(b, s, hq, hkv, cp, rank, layout, d, split):
 def test_handover_of_grids_that_two_thirds_fill_the_device(causal, b, s, hq, hkv, pays):
     """As measured (table at ds_handover_pays)."""
     assert native.ds_handover_pays(b, s, s, hq, hkv, causal, UNITS) == pays
+
+
+@pytest.mark.parametrize("one,s,hq,cp,rank,layout", [(1, 2048, 64, 2, 1, "contiguous"), (0, 2176, 64, 2, 1, "contiguous"), (1, 4096, 64, 4, 1, "zigzag"), (0, 4224, 64, 4, 1, "zigzag")])
+def test_shares_of_128_features_in_one_grid(one, s, hq, cp, rank, layout):
+    """Up to four dQ workgroups per compute unit, up to eight against more than two chunks' keys, as measured (table at one_grid)."""
+    assert _share_plan(1, s, hq, 4, cp, rank, layout, 128).one_grid == one
