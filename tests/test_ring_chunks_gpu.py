@@ -77,3 +77,17 @@ def test_share_of_unequal_rows_64_features(gpu, monkeypatch):
 def test_share_with_many_workgroups(gpu, monkeypatch, S, Hq, Hkv, D, C, rank, layout, two_part):
     monkeypatch.setattr(H, "DS_BUFFER_LIMIT_BYTES", 0)  # no dS hand-over: every kernel recomputes
     test_share(gpu, monkeypatch, True, 1, S, Hq, Hkv, D, C, rank, layout, two_part)
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,rank", [(1100, 56, 2, 1), (1100, 58, 2, 1), (1100, 120, 4, 0), (1090, 58, 2, 2), (1278, 52, 2, 2)])
+def test_forward_a_little_above_whole_rounds(gpu, monkeypatch, S, Hq, Hkv, rank):
+    """On 256 compute units 128-row workgroups for just below and above two rounds (256-row ones there) and above four, against a launch per
+    ring step; either rounds P and the result to bf16, and a merge rounds once more: two steps (2^-8 each) of the largest element."""
+    g = torch.Generator(device=gpu).manual_seed(7)
+    mk = lambda h: torch.randn(1, S, h, 128, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, ks, vs = mk(Hq), [mk(Hkv) for _ in range(3)], [mk(Hkv) for _ in range(3)]
+    out, lse = L.ring_forward_local(q, ks, vs, 128**-0.5, rank, 3, "zigzag")
+    monkeypatch.setattr(L, "FUSE_CHUNKS", False)
+    steps, lse_steps = L.ring_forward_local(q, ks, vs, 128**-0.5, rank, 3, "zigzag")
+    assert (out.float() - steps.float()).abs().max() <= 2**-7 * steps.float().abs().max()
+    assert (lse - lse_steps).abs().max() < 1e-3
