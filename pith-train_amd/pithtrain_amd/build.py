@@ -37,6 +37,13 @@ HIPCC_FLAGS = [
     "-Wno-unused-function",
 ]
 
+# Backward over several chunks: a share of few workgroups is as long as its longest walk, one wave to a SIMD, which fetches its loop anew at every
+# turn. Three scalar instructions in front of it (tiles_of_wave) moved it off the fetch lines; forward + backward of 64 features, us, before
+# them / after / with loops on 64 bytes: 2146 x 4 heads, 8 ranks, rank 3 358 / 368 / 356, 848 x 16, rank 0 221 / 225 / 220, 3 x 1856 x 4, rank 6
+# contiguous 401 / 410 / 401; 95 such shares 0.7 % faster, 205 of 128 and 192 features equal. Not the forward (all files aligned: 2884 x 8/2 of 128
+# without a mask 43.8 / 47.8).
+SOURCE_FLAGS = {"attn_bwd_chunks.hip": ["-falign-loops=64"]}
+
 
 def _hipcc() -> str:
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -47,7 +54,7 @@ def _hipcc() -> str:
 
 def _compile(src: str, extra: list) -> str:
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [_hipcc(), *HIPCC_FLAGS, *extra, "-I", INCLUDE_DIR, "-I", SRC_DIR, "-c", os.path.join(SRC_DIR, src), "-o", obj]
+    cmd = [_hipcc(), *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), *extra, "-I", INCLUDE_DIR, "-I", SRC_DIR, "-c", os.path.join(SRC_DIR, src), "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     err = "\n".join(line for line in proc.stderr.splitlines() if noise not in line)

@@ -305,12 +305,19 @@ def _kernel_asm(src, tmp_dir):
 
     if src not in _ASM_CACHE:
         out = os.path.join(str(tmp_dir), src + ".s")
-        cmd = [B._hipcc(), *B.HIPCC_FLAGS, "-I", B.INCLUDE_DIR, "-I", B.SRC_DIR, "--cuda-device-only", "-S",
+        cmd = [B._hipcc(), *B.HIPCC_FLAGS, *B.SOURCE_FLAGS.get(src, []), "-I", B.INCLUDE_DIR, "-I", B.SRC_DIR, "--cuda-device-only", "-S",
                os.path.join(B.SRC_DIR, src), "-o", out]  # fmt: skip
         subprocess.run(cmd, check=True, capture_output=True)
         with open(out) as f:
             _ASM_CACHE[src] = f.read()
     return _ASM_CACHE[src]
+
+
+def test_loops_of_the_chunk_backward_begin_on_fetch_lines(tmp_path_factory):
+    """Its longest walk is one wave per SIMD, 2-3 % longer where a few instructions in front of the loop move it (build.py, SOURCE_FLAGS)."""
+    text = _kernel_asm("attn_bwd_chunks.hip", tmp_path_factory.getbasetemp())
+    headers = re.findall(r"(\.p2align\t6\n)?\.LBB\d+_\d+:[^\n]*(?:\n +; [^\n]*)*Inner Loop Header", text)
+    assert 2 * sum(map(bool, headers)) > len(headers) > 0  # (loops entered in the middle have another block first)
 
 
 def test_m0_is_touched_only_by_the_direct_load_statements(tmp_path_factory):
