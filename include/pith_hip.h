@@ -52,9 +52,10 @@ enum { PITH_BASE_2 = 0, PITH_BASE_E = 1 };
 /* Version of this interface: major*10000 + minor*100 + patch. The minor number goes up whenever a struct or a signature below
  * changes; a program built against another one must not call into the library (its structs have other sizes). The patch number
  * goes up when functions are added or a call takes up a field that it ignored.
+ * 202: pith_attn_fwd_split added.
  * 201: pith_attn_bwd_chunks_handover, pith_attn_bwd_chunks_ds_bytes and the plan functions added; `ds` used at head dims (192,128).
  * 200: pith_norm_rope_args gained dweight_bf16, and dweight became void*; chunk calls and pith_attn_bwd added. */
-#define PITH_VERSION 201
+#define PITH_VERSION 202
 int pith_version(void); /* PITH_VERSION of the library that was loaded */
 /* Text of the last error raised on the calling thread ("" if none). Never NULL. */
 const char* pith_last_error(void);
@@ -181,6 +182,12 @@ typedef struct {
 } pith_key_chunk;
 
 int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, pith_stream_t stream);
+
+/* How the forward of these shapes is cut on the current device, for tests and profiles: pith_attn_fwd with chunks == NULL, else
+ * pith_attn_fwd_chunks. Only the shapes, `causal`, and the rows and q_row0 of the chunks are read. 0: 256 query rows per workgroup,
+ * 1: 128 rows, two workgroups per compute unit, 2: 128 rows, key halves, 3: 128 rows, two teams, 4: 64 rows, two teams of key halves,
+ * 5: 64 rows, four waves, key halves. */
+int pith_attn_fwd_split(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, int32_t* split);
 
 /* ------------------------------------------------------------------------------------------
  * delta[b,h,s] = sum_d fp32(o[b,s,h,d]) * fp32(dout[b,s,h,d]).

@@ -17,34 +17,32 @@ namespace {
 //   HALF   one 128-row workgroup of 8 waves per compute unit, wave pairs splitting the keys of every tile;
 //   TEAMS  one 128-row workgroup of 8 waves per compute unit, two teams of 4 waves taking every second tile (64 features);
 //   QUARTER  one 64-row workgroup of 8 waves: two teams, and wave pairs of a team splitting the keys of its tile;
-//   SMALL  two (64 features: five) 64-row workgroups of 4 waves, wave pairs splitting the keys of every tile: an interval of half the length, and
+//   SMALL  two (64 features: four) 64-row workgroups of 4 waves, wave pairs splitting the keys of every tile: an interval of half the length, and
 //          more workgroups than any other split that hide each other's first tiles and epilogues.
 // FULL and DUO when every compute unit has work for its whole time; the others when workgroups are few or (under the mask)
 // so unequal that a heavy one would run alone on its unit. Kernels measured on one box, microseconds, with inputs that
 // rotate over 500 MB (the tiles come from memory, as in a training step; the prefetch depth counts then: TEAMS at 192
 // features, two tiles per ring, beat HALF by 2-8 % on inputs in the last-level cache and lost 4-9 % here)
-// (QUARTER before its teams took turns on streams of 1024 keys and more, 3-17 % faster since: kHalvesFrom in attn_fwd_duo.hip):
-//                                                       FULL    DUO   HALF  TEAMS QUARTER
-//   d128 causal   1 x 16384 x 8 heads (cached)           454    470    507    515    643
-//                 3 x 1999 x 32 (cached)                 109    107    133    131    187
-//                 1 x 4096 x 8  (256 WGs of 128 rows)   82.1   76.6   61.4   68.2   64.2
-//                 1 x 4096 x 6  (192 WGs)               79.5   71.1   57.0   64.5   50.9
-//                 1 x 8192 x 4  (256 WGs)                150    137    109    123    108
-//                 1 x 2048 x 8  (128 WGs)               43.4   37.8   30.5   33.7   26.4
-//                 1 x 384 x 8 / 320 x 8 (cached)               11.2 / 9.5           10.9 / 10.3
-//   d192 causal   1 x 8192 x 16 (1024 WGs, cached)              298    339    331    430
-//                 1 x 4096 x 16 (512 WGs)                       112    100    110    152
-//                 1 x 4096 x 8  (256 WGs)                      85.6   74.2   84.2   78.2
-//                 1 x 1021 x 16 (128 WGs)                      27.3   25.9   28.8   24.0
-//   d64  causal   1 x 4096 x 20 (640 WGs, cached)              62.4          69.7   78.0
-//                 1 x 4096 x 16 (512 WGs)                      57.2          52.9   65.0
-//                 2 x 2048 x 16 (512 WGs)                      32.0          32.4   44.4
-//                 1 x 4096 x 8  (256 WGs)                      52.4          42.7   43.6
-//                 1 x 1024 x 16 (128 WGs)                      16.4          15.2   11.8
-//        full     1 x 2048 x 16 (256 WGs)                      30.3          27.4   39.9
-//   ring shares, 4 ranks, zigzag: d192 4096 rows x 16 rank 0 / 3    416 / 323   367 / 342   385 / 330   530 / 460
-//                                      2048 rows x 16 rank 0 / 2    180 / 136   142 / 113   149 / 117   130 / 121
-//                                 d128 4096 rows x 8/2 rank 0       281         218         239         195
+//                                                       FULL    DUO   HALF  TEAMS QUARTER  SMALL
+//   d128 causal   1 x 16384 x 8 heads                    451    461    494            597    544
+//                 3 x 1999 x 32                          108    106    126            187    130
+//                 1 x 4096 x 8  (256 WGs of 128 rows)   83.6   76.9   57.4           52.6   60.0
+//                 1 x 4096 x 6  (192 WGs)               82.0   74.5   55.1           42.9   57.2
+//                 1 x 8192 x 4  (256 WGs)                159    147    106           88.7    113
+//                 1 x 2048 x 8  (128 WGs)               44.2   39.1   30.7           25.0   30.0
+//   d192 causal   1 x 8192 x 16 (1024 WGs)                      291    333            380    344
+//                 1 x 4096 x 16 (512 WGs)                       103   90.9            112   94.1
+//                 1 x 4096 x 8  (256 WGs)                      89.0   74.7           59.8   70.6
+//                 1 x 1021 x 16 (128 WGs)                      26.1   23.1           19.7   20.7
+//   d64  causal   1 x 4096 x 20 (640 WGs)                      63.8          74.4    84.1   56.2
+//                 1 x 4096 x 16 (512 WGs)                      60.5          54.9    68.9   49.5
+//                 2 x 2048 x 16 (512 WGs)                      33.7          32.8    42.1   27.5
+//                 1 x 4096 x 8  (256 WGs)                      55.4          44.8    37.7   44.0
+//                 1 x 1024 x 16 (128 WGs)                      16.8          15.0    11.9   13.8
+//        full     1 x 2048 x 16 (256 WGs)                      32.0          27.9    35.6   27.6
+//   ring shares, 4 ranks, zigzag: d192 4096 rows x 16 rank 0 / 3    371 / 313   323 / 322           442 / 393   368 / 363
+//                                      2048 rows x 16 rank 0 / 2    180 / 142   142 / 114           126 / 112   149 / 112
+//                                 d128 4096 rows x 8/2 rank 0       299         216                 175         222
 // No FULL at 192 features: its register budget left no room for the row-sum test of the running maximum. Such a kernel, ms,
 // against DUO, tiles from memory; the two are within what one machine differs from the next (32768 x 128 on three of them:
 // 36.0 / 36.4, 35.6 / 35.2, 35.7 / 37.4), and shorter streams are DUO's:
@@ -122,6 +120,33 @@ bool above_a_round(const pith_attn_fwd_args* a, int64_t wgs, int64_t cus, Split*
   return d192 ? (at_most(9, 8) && keys >= 4096) || (at_most(4, 3) && keys >= 8192) : at_most(23, 20) && keys >= 8192;
 }
 
+// More 64-row workgroups than units: where SMALL pays. By W = those workgroups per unit, us, SMALL / the best other:
+//   64 features, rows unequal, two and more per unit
+//     to 959 keys    SMALL is ahead while all of its workgroups run at once and 128 rows pad (192, 320 rows) or the tiles are many: W 3 512 x 96 heads
+//                    10.6 / 11.9, 768 x 64 12.8 / 14.9; W 3.5-4 320 x 180 10.1 / 11.3, 600 x 90 13.1 / 14.1, 900 x 60 15.2 / 17.4, 768 x 84 14.3 / 16.1, 512 x 128
+//                    12.2 / 12.6; but 256 rows W 3.3 x 210 10.7 / 9.4, 4 x 256 10.2 / 9.7, more than at once (4.2-4.5) 192 x 360 11.9 / 10.4, 370 x 192 15.4 /
+//                    12.8, 768 x 96 17.6 / 16.7, and an odd number of heads, whose tiles wander over the XCDs, 448 x 135 14.2 / 13.4, 768 x 81 18.3 / 16.5
+//     960 to 1535    W 4 1000 x 64 17.1 / 19.4, 1024 x 64 17.1 / 19.3, 4.3 1024 x 69 22.9 / 21.2, 1200 x 58 21.9 / 22.6, 4.5 1400 x 52 23.4 / 25.7
+//     1536 on        W 4.5 2 x 2048 x 18 31.9 / 35.9, 5 1 x 2048 x 40 35.2 / 36.2. With the backward behind it TEAMS is ahead from 2561 keys on while W is 3.25 at
+//                    most: 4 x 2855 x 4 114.9 / 110.8, 2914 x 16 117.9 / 114.8, 2688 x 16 109.0 / 105.6, 5120 x 10 193.7 / 189.6, 6144 x 8 220.7 / 216.1, not 2560 x 20
+//                    106.2 / 106.8, 4096 x 16 (W 4) equal, its forward alone 49.4 / 53.3
+//   64 features without a mask, up to two per unit: to 384 keys from W 1.7 on (320 keys 1.35 9.1 / 8.6, 1.5 9.2 / 8.7, 1.75 9.6 / 10.2; 256 keys equal at best), 384 keys 44 to
+//                    84 heads 8.7-9.6 / 9.0-9.9, but 75 heads 11.0 / 9.8; 1024 x 32 16.2 / 17.0; TEAMS above 2048 keys (2304 x 14 30.4 / 30.1, 6144 x 5 69.8 / 67.0)
+//   128 and 192 features, rows unequal, up to two per unit: not for 128 rows, which one DUO workgroup holds (8.6 / 7.9, 9.2 / 8.9), nor up to 192 at W 1.05 (8.7 / 8.0
+//                    and 9.9 / 9.2; 1.2: 8.1 / 8.4)
+bool small_workgroups(const pith_attn_fwd_args* a, int64_t wgs64, int64_t cus, bool unequal) {
+  const int64_t keys = a->Skv, heads = a->Hq * a->B;
+  const auto at_most = [&](int64_t n, int64_t d) { return d * wgs64 <= n * cus; };  // W <= n / d
+  if (a->Dqk != 64) return unequal && at_most(2, 1) && keys >= 129 && keys < 1536 && (keys > 192 || !at_most(6, 5));
+  if (!unequal) return at_most(2, 1) && keys >= 192 && keys <= 2048 && (keys >= 448 || (keys >= 384 ? heads % 4 == 0 : !at_most(17, 10)));
+  if (at_most(2, 1)) return keys >= 128 && keys < 1536;
+  if (keys < 128 || keys > 6144) return false;
+  if (keys >= 1536) return at_most(5, 1) && (keys <= 2560 || !at_most(13, 4));
+  if (keys >= 960) return keys >= 1200 ? at_most(9, 2) : at_most(4, 1);
+  const bool pads = (a->Sq + 63) / 64 % 2 != 0;  // half of a 128-row workgroup
+  return heads % 2 == 0 && (keys >= 384 || pads) ? at_most(4, 1) : at_most(3, 1);
+}
+
 // `mean` = mean length of the rows' key streams in percent of the longest (a masked chunk: 50).
 Split pick_split(const pith_attn_fwd_args* a, int mean) {
   const int64_t cus = compute_units_or_default();
@@ -129,23 +154,15 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   Split above;
   if (above_a_round(a, wgs, cus, &above) && wgs64 > 2 * cus) return above;
   const bool d64 = a->Dqk == 64, unequal = mean <= 70;  // HALF is 3 % slower than DUO at 0.75, 5-10 % above
-  if (a->Skv > 64) {  // (64 features to 6144 keys: 4404 x 16 61.8 -> 52.2, 4998 x 16 75 -> 67, 5938 x 16 95 -> 91)
-    if (wgs64 <= cus) return a->Skv > 512 ? Split::kQuarter : Split::kSmall;
-    if (unequal) {
-      if (wgs64 <= 2 * cus) {
-        const bool quarter_more = 4 * wgs64 > 5 * cus, half_more = 2 * wgs64 > 3 * cus;  // workgroups than one round of QUARTER
-        const int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
-        if (a->Skv >= from && (!half_more || a->Sq >= 1536)) return Split::kQuarter;
-        if (a->Skv >= (a->Dqk == 192 ? 129 : 128) && a->Skv < 1536) return Split::kSmall;
-      } else if (d64 && 2 * wgs64 <= (a->Skv < 1536 ? 9 : 10) * cus && a->Skv >= 128 && a->Skv <= 6144) {
-        return Split::kSmall;
-      }
-    } else if (d64 && wgs64 <= 2 * cus && a->Skv >= 192) {
-      return Split::kSmall;
-    }
+  if (a->Skv > 64 && wgs64 <= cus) return a->Skv > (d64 ? 384 : 512) ? Split::kQuarter : Split::kSmall;
+  if (unequal && wgs64 <= 2 * cus) {
+    const bool quarter_more = 4 * wgs64 > 5 * cus, half_more = 2 * wgs64 > 3 * cus;  // workgroups than one round of QUARTER
+    const int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
+    if (a->Skv >= from && (!half_more || a->Sq >= 1536)) return Split::kQuarter;
   }
+  if (small_workgroups(a, wgs64, cus, unequal)) return Split::kSmall;
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;
-  if (wgs <= cus && a->Skv > (d64 ? 1024 : a->Dqk == 192 ? 383 : 255)) return key_split;
+  if (wgs <= cus && a->Skv > (d64 ? 1024 : a->Dqk == 192 ? 383 : 256)) return key_split;  // (128 features without a mask, 256 keys: 4 x 27 heads 11.7 / 12.4)
   if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 2 * wgs <= 3 * cus ? 1023 : 1535)) return key_split;
   // FULL under the mask also for shorter rows of many heads whose K and V outgrow the last-level cache (half the streams in
   // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
@@ -250,7 +267,32 @@ int launch(const P& p, const pith_attn_fwd_args* a, Split split, pith_stream_t s
   return check_launch(who);
 }
 
+// (query row, key) pairs of a chunk
+int64_t pairs_seen(const pith_attn_fwd_args* a, const pith_key_chunk& c, bool diagonal) { return diagonal ? c.rows * a->Sq / 2 : c.rows * (a->Sq - c.q_row0); }
+
+// Of several chunks: by the whole stream (a->Skv) and by how unequal the rows' streams are.
+Split pick_chunks_split(const pith_attn_fwd_args* a, int64_t seen) { return pick_split(a, (int)(100 * seen / (a->Skv * a->Sq))); }
+
 }  // namespace
+
+extern "C" int pith_attn_fwd_split(const pith_attn_fwd_args* args, const pith_key_chunk* chunks, int64_t n, int32_t* split) {
+  const char* who = "pith_attn_fwd_split";
+  if (!args || !split) return fail(PITH_ERR_NULL_POINTER, "%s: %s is NULL", who, args ? "split" : "args");
+  pith_attn_fwd_args a = *args;
+  int64_t seen = 0;
+  if (chunks) {
+    if (n < 1 || n > kMaxChunks) return fail(PITH_ERR_BAD_SHAPE, "%s: %lld chunks, not 1..%d", who, (long long)n, kMaxChunks);
+    a.Skv = 0;
+    for (int64_t i = 0; i < n; ++i) {
+      a.Skv += chunks[i].rows;
+      seen += pairs_seen(&a, chunks[i], i == n - 1);
+    }
+    a.causal = 1;
+  }
+  if (a.B <= 0 || a.Sq <= 0 || a.Skv <= 0 || a.Hq <= 0 || a.Hkv <= 0) return fail(PITH_ERR_BAD_SHAPE, "%s: bad shape", who);
+  *split = (int32_t)(chunks ? pick_chunks_split(&a, seen) : pick_split(&a, a.causal ? 50 : 100));
+  return PITH_OK;
+}
 
 extern "C" int pith_attn_fwd(const pith_attn_fwd_args* a, pith_stream_t stream) {
   FwdParams p;
@@ -276,13 +318,11 @@ extern "C" int pith_attn_fwd_chunks(const pith_attn_fwd_args* args, const pith_k
     if (const int rc = prepare(&a, p)) return rc;
     p.chunk[i] = KeyChunk{(const __bf16*)c.k, (const __bf16*)c.v, (const __bf16*)c.k_pe, (int)c.rows, (int)c.q_row0};
     keys += c.rows;
-    seen += diagonal ? c.rows * args->Sq / 2 : c.rows * (args->Sq - c.q_row0);
+    seen += pairs_seen(args, c, diagonal);
   }
   p.n_chunks = (int)n;
-  // The split goes by the whole stream and by how unequal the rows' streams are.
   a.Skv = keys;
-  const Split split = pick_split(&a, (int)(100 * seen / (keys * args->Sq)));
-  a.causal = 1;
+  const Split split = pick_chunks_split(&a, seen);
   if (n == 1) return launch<FwdParams>(p, &a, split, stream, who);
   return launch(p, &a, split, stream, who);
 }

@@ -13,7 +13,7 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libpith_hip.so")
 
-PITH_VERSION = 201  # of include/pith_hip.h, whose structs are declared below
+PITH_VERSION = 202  # of include/pith_hip.h, whose structs are declared below
 
 PITH_BF16, PITH_F32 = 0, 1
 PITH_BASE_2, PITH_BASE_E = 0, 1
@@ -140,6 +140,7 @@ SYMBOLS = {
     "pith_combine": (c_int, [POINTER(CombineArgs), c_void_p]),
     "pith_attn_fwd": (c_int, [POINTER(AttnFwdArgs), c_void_p]),
     "pith_attn_fwd_chunks": (c_int, [POINTER(AttnFwdArgs), POINTER(KeyChunk), c_int64, c_void_p]),
+    "pith_attn_fwd_split": (c_int, [POINTER(AttnFwdArgs), POINTER(KeyChunk), c_int64, POINTER(c_int32)]),
     "pith_attn_bwd_delta": (c_int, [POINTER(AttnDeltaArgs), c_void_p]),
     "pith_attn_bwd_dkdv": (c_int, [POINTER(AttnBwdArgs), c_void_p]),
     "pith_attn_bwd_dq": (c_int, [POINTER(AttnBwdArgs), c_void_p]),

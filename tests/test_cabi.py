@@ -68,7 +68,7 @@ STRUCT_SIZES = {
     200: {"pith_combine_args": 168, "pith_attn_fwd_args": 248, "pith_attn_delta_args": 88, "pith_attn_bwd_args": 352, "pith_attn_bwd_plan_t": 16,
           "pith_norm_rope_args": 152, "pith_mla_assemble_args": 192, "pith_key_chunk": 72, "pith_device_info_t": 88},
 }  # fmt: skip
-STRUCT_SIZES[201] = STRUCT_SIZES[200]
+STRUCT_SIZES[201] = STRUCT_SIZES[202] = STRUCT_SIZES[200]
 
 
 def test_version_goes_with_the_struct_sizes(tmp_path):

@@ -99,11 +99,12 @@ def test_shares_of_teams_in_turns(gpu, rows, D, layout):
     # 64-row workgroups of 4 waves: one ragged row, key halves that do not exist or end early, 64 / 65 and 512 / 513 keys
     *[(1, sq, skv, 2, 1, d, sq == skv) for d in (64, 128, 192) for sq, skv in ((65, 65), (1, 65), (64, 96), (33, 97), (127, 128), (95, 350), (300, 300), (512, 512))],
     (1, 70, 513, 2, 1, 64, False), (2, 257, 257, 3, 3, 192, True),
-    # one and two of them per unit (192 features: from 129 keys on), at 64 features four and a half, five from 1536 keys on
+    # one and two of them per unit (from 129 keys on), at 64 features three and four, five from 1536 keys on; and on the other side of these lines
     (2, 512, 512, 16, 4, 128, True), (4, 320, 320, 25, 25, 128, True), (8, 128, 128, 32, 32, 192, True), (8, 129, 129, 21, 21, 192, True),
     (4, 192, 192, 43, 43, 64, False), (4, 576, 576, 32, 8, 64, True), (4, 577, 577, 32, 8, 64, True), (2, 1535, 1535, 26, 13, 64, True), (2, 1536, 1536, 26, 13, 64, True),
-    # wave pairs of 128-row workgroups from 256 (192 features: 384) keys on
-    (2, 255, 300, 70, 70, 128, False), (4, 256, 256, 32, 8, 128, False), (2, 384, 384, 33, 33, 192, False), (2, 1024, 1024, 20, 20, 192, True),
+    (4, 512, 512, 32, 8, 64, True), (5, 512, 512, 27, 9, 64, True), (2, 2048, 2048, 18, 6, 64, True), (1, 2561, 2561, 16, 4, 64, True), (1, 2049, 2049, 12, 4, 64, False), (4, 129, 129, 32, 8, 128, True),
+    # wave pairs of 128-row workgroups from 257 (192 features: 384) keys on
+    (2, 255, 300, 70, 70, 128, False), (4, 256, 256, 32, 8, 128, False), (4, 256, 257, 32, 8, 128, False), (2, 384, 384, 33, 33, 192, False), (2, 1024, 1024, 20, 20, 192, True),
 ])  # fmt: skip
 def test_forward_small_workgroups(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     test_forward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
