@@ -168,13 +168,17 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
   // for rows of a few workgroups: 8 x 512 x 128 155 -> 167)
   const bool many_heads = a->Sq >= 1024 && a->Skv == a->Sq && a->B * a->Skv * a->Hkv * (a->Dqk + a->Dv) * 2 >= 224ll << 20;
-  // Several chunks of unequal rows (zigzag) a little above two or four 128-row workgroups per unit, W, which are one or two rounds of FULL, DUO / FULL: four
-  // ranks, 2.1 2100 x 32/4 180 / 157, 2 x 2100 x 16/4 179 / 155, rank 0 2176 x 32/4 240 / 213, eight ranks 2200 x 32/4 380 / 322; 2.25 1100 x 64/4 105 / 94.5;
-  // 2.4 2400 x 32/4 217 / 214; 4.5 2 x 1100 x 64/4 188 / 180, 4 x 1100 x 32/4 186 / 174; not at 3 and 4 (1500 x 64/4 158 / 162, 3 x 900 x 32/4 98 / 156, 2 x 2000 x
-  // 32/4 319 / 338), nor where 256 rows waste a fifth (with the backward 2 x 1040 x 32/4 375 / 377, 1090 x 64/4, two ranks, 218 /
-  // 225) or every head has keys of its own (4 x 2100 x 16 1350 / 1374)
-  if (a->Dqk == 128 && a->causal && a->Skv != a->Sq && unequal && a->Hq > a->Hkv && a->Sq >= 1024 && 100 * ((a->Sq + 255) / 256 * 256) <= 117 * a->Sq &&
-      ((wgs > 2 * cus && 20 * wgs <= 47 * cus) || (wgs > 4 * cus && 5 * wgs <= 23 * cus)))
+  // Several chunks of unequal rows (zigzag) a little above two or four 128-row workgroups per unit, which are 1.15 (long rows against more than two chunks: 2.25)
+  // of FULL at most, an odd number of them to a head: where the longer half of the rows begins within the middle one, and not at the end of one that then walks
+  // as far. DUO / FULL, forward of four ranks unless others are named, by FULL workgroups per unit: 1.1 2100 x 32/4 161 / 153, rank 0 253 / 231, 2 x 2100 x 16/4 193 /
+  // 173, rank 0 2176 x 32/4 264 / 239, 2200 x 32/8 173 / 164, 2200 x 32/4, eight ranks, 392 / 345, 1664 x 40/8 130 / 120, 1792 x 40/8 148 / 151; 2.25 2200 x 64/4 323
+  // / 305, rank 0 2300 x 64/4 501 / 456, 4 x 2168 x 16/4 332 / 322. Even: 2944 x 24/3 221 / 212, but rank 0 2862 x 24/3 341 / 376, 1364 x 48/8 177 / 196,
+  // 1920 x 40/8 155 / 178, 2 x 2944 x 24/3, two ranks, 262 / 284. Less than two chunks' keys: 1588 x 40/5, two ranks, 66.6 / 73.3. More workgroups: 2.25 with
+  // short rows 2 x 1408 x 48/8 228 / 238, 2.5 2 x 1100 x 64/4 172 / 177. Nor where 256 rows waste a fifth (with the backward 2 x 1040 x 32/4 375 / 377, 1090
+  // x 64/4, two ranks, 218 / 225) or every head has keys of its own (4 x 2100 x 16 1350 / 1374)
+  const int64_t tiles256 = (a->Sq + 255) / 256, wgs256 = tiles256 * a->Hq * a->B;
+  if (a->Dqk == 128 && a->causal && a->Skv >= 2 * a->Sq && unequal && a->Hq > a->Hkv && a->Sq >= 1024 && 25600 * tiles256 <= 117 * a->Sq && tiles256 % 2 == 1 &&
+      ((wgs > 2 * cus && 20 * wgs256 <= 23 * cus) || (wgs > 4 * cus && 4 * wgs256 <= 9 * cus && a->Sq >= 2048 && a->Skv > 2 * a->Sq)))
     return Split::kFull;
   // (without a mask, FULL / DUO: 1100 x 32/4 30.0 / 28.4, 8 x 1100 x 16 104.3 / 97.4, 2 x 1400 x 32/4 73.2 / 70.3, 1500 x 32/4 39.7 / 40.0, 1999 x 32/4 60.9 /
   // 61.1, 3457 x 32/4 176 / 183)

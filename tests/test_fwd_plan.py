@@ -62,3 +62,14 @@ def test_few_rows():
 def test_shares_of_64_features_of_long_streams():
     """Nearly equal rows, two teams above 2048 keys."""
     assert _share_split(2, 2240, 4, 4, 64, 4, 3, "contiguous") == TEAMS and _share_split(1, 500, 40, 40, 64, 4, 3, "contiguous") == SMALL
+
+
+@pytest.mark.parametrize("full,b,s,hq,hkv,cp,rank", [
+    (1, 1, 2100, 32, 4, 4, 2), (1, 2, 2100, 16, 4, 4, 1), (1, 1, 2176, 32, 4, 4, 0), (1, 1, 2200, 32, 8, 4, 2), (1, 1, 1664, 40, 8, 4, 2), (1, 1, 2100, 32, 4, 2, 0),
+    (0, 1, 2944, 24, 3, 4, 2), (0, 1, 1920, 40, 8, 4, 2), (0, 1, 2862, 24, 3, 4, 0), (0, 1, 1364, 48, 8, 4, 0), (0, 1, 1588, 40, 5, 2, 1),
+    (0, 1, 1100, 64, 4, 4, 2), (1, 1, 1100, 58, 2, 4, 2), (0, 1, 1100, 56, 2, 4, 2), (0, 1, 2400, 32, 4, 4, 1), (1, 1, 2300, 64, 4, 4, 0), (1, 1, 2200, 64, 4, 4, 2),
+    (0, 2, 2944, 24, 3, 2, 0), (0, 2, 1408, 48, 8, 4, 1), (0, 2, 1100, 64, 4, 4, 2), (0, 2, 2100, 16, 16, 4, 1),
+])  # fmt: skip
+def test_zigzag_shares_of_256_row_workgroups(full, b, s, hq, hkv, cp, rank):
+    """As measured (comment at pick_split)."""
+    assert (_share_split(b, s, hq, hkv, 128, cp, rank, "zigzag") == FULL) == bool(full)
