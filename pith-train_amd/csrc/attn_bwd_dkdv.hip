@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "attn_bwd_common.h"
+#include "handover_rows.h"
 
 namespace pith {
 namespace {
@@ -96,39 +97,42 @@ struct Reduction {
 };
 
 // The head split doubles until the workgroups wanted are there, which leaves up to twice as many. Whether half of those do better, a
-// round of them without a mask, one to two (workgroups per unit below) under it: they leave half of the partial sums, which make a round
-// trip through memory, and spend half as often what a workgroup spends around its products (7 us). Long walks lose: the wanted number
-// balanced them, and in a call that hands dS over nothing else fills the units. Forward + backward, more / half, us, 32/4 heads
-// unless others are named:
-//   causal d128  1.6 - 1.9   3 x 1100 210 / 185, 3 x 1200 230 / 204, 2 x 1700 261 / 235, 5 x 700 183 / 156, 1790 x 64/4 274 / 249, 5 x 1500 x 16/4
-//                            275 / 253, 3600 446 / 428, 3900 502 / 483, 5 x 2600 x 8/2 339 / 328
-//                1.4 - 1.5   2 x 700 x 64/4 145 / 127, 9 x 1200 x 8/2 185 / 169, 9 x 600 231 / 220, 1300 x 64/4 181 / 172, 2900 338 / 333, 3000 x 64/4
-//                            600 / 617
-//                1.0 - 1.3   no hand-over: 3 x 768 127 / 116, 2 x 1100 147 / 131, 5 x 400 104 / 90, 2200 218 / 204, 4 x 2200 x 8/2 224 / 211; handing
-//                            over: 9 x 512 186 / 175, 7 x 700 210 / 201, 5 x 900 234 / 236, 4 x 1152 x 64/4 454 / 484, 3 x 1500 303 / 321, 2 x 2100
-//                            353 / 396, 3 x 2900 846 / 944, 4300 632 / 738
+// round of them without a mask, one to two (W workgroups per unit) under it: they leave half of the partial sums, which make a round
+// trip through memory, and spend half as often what a workgroup spends around its products (7 us). Long walks (rows x heads of a part) lose, the
+// sooner the fewer workgroups are there to even them out: in a call that hands dS over nothing else fills the units. Forward + backward, more / half,
+// us, 32/4 heads unless others are named:
+//   causal d128, handing over, by W and walk
+//                1.0         2080 13 x 520 x 16/4 155 / 147, 3072 11 x 768 x 16/4 198 / 187; 4160 13 x 520 265 / 273, 5472 3 x 1368 254 / 278, 12288 11 x 768 x 64/4 647 / 692
+//                1.12-1.17   4096 9 x 1024 x 16/4 235 / 225, 5120 15 x 640 350 / 331; 6000 3 x 1500 294 / 313, 10624 12 x 664 x 64/4 603 / 648
+//                1.2-1.3     6000 7 x 1500 x 16/4 335 / 325, 6144 13 x 768 394 / 375, 3600 5 x 900 231 / 234; 7200 5 x 900 x 64/4 411 / 424, 11344 13 x 709 x 64/4 744 / 752
+//                1.38-1.5    7200 11 x 900 456 / 439, 9216 5 x 1152 x 64/4 557 / 551, 12288 15 x 768 x 64/4 858 / 836; 7200 3 x 1800 392 / 399, 14400 3 x 1800 x 64/4 746 / 763,
+//                            21888 8 x 1368 x 64/4 1223 / 1256
+//                1.55-1.9    3600 2 x 1800 281 / 258, 9216 11 x 1152 616 / 593, 16384 13 x 1024 x 64/4 1151 / 1119, 18432 11 x 1152 x 64/4 1199 / 1186, 28800 equal
+//                not         1.0 11 x 709 x 8/2 118 / 107, 1.12 2304 239 / 224, 9 x 400 x 16/4 104 / 89, 1.4 2 x 1368 201 / 185, 1.5 3 x 900 172 / 157; 3000 x 64/4 600 / 617
 //                short rows  24 x 128 112 / 92, 20 x 160 111 / 97, 10 x 200 x 64/4 143 / 125
-//   full   d128  1100 134.7 / 119.6, 1300 162 / 150, 1790 253 / 242, 4 x 520 138 / 126, 3 x 700 155 / 145, 3 x 1408 x 8/2 153 / 140, 2 x 2100 x 8/2
-//                209 / 188, 2700 566 / 530, 20 x 160 118 / 102; 5000 x 8/2 442 / 462, 3500 x 64/4 1509 / 1523. Calls that hand dS over leave at most
-//                a quarter of the units idle (ds_handover_pays).
+//   full   d128  1100 134.7 / 119.6, 1300 162 / 150, 1790 253 / 242, 3 x 700 155 / 145, 3 x 1408 x 8/2 153 / 140, 2 x 2100 x 8/2 209 / 188, 2700 566 / 530; rows that
+//                do not hand over 4 x 520 133.7 / 125.8, 4 x 600 x 64/4 290 / 268, 9 x 560 x 16/4 154 / 135, 20 x 160 119.6 / 103.8, 40 x 100 113 / 96, 33 x 100 110 /
+//                91; 5000 x 8/2 442 / 462, 3500 x 64/4 1509 / 1523. Calls that hand dS over leave at most a quarter of the units idle (ds_handover_pays).
 //   d64          causal 9 x 1100 x 32/8 303 / 280, 5 x 1290 x 32/8 236 / 216, 4300 x 32/8 369 / 361, 20 x 250 x 32/8 95 / 84, 3 x 2200 x 16/4 equal;
 //                full 10 x 600 x 16/4 114 / 106, 4 x 1290 x 32/8 305 / 295, 2600 x 32/8 281 / 274, 2200 x 32/8 equal
 // Several chunks, whose workgroups are unequal, in one grid with more than one dQ workgroup per unit to even them out: four ranks, 1100 contiguous
 // rank 3 392 / 371, 2 x 900 zigzag 328 / 310, 600 x 64/4 173 / 163, 2 x 2400 x 8/2 500 / 459, 5000 x 8/2 contiguous 1177 / 1117, 8200 x 8/2 2497 / 2430, 3300
-// equal. Not with fewer (2 x 1314 x 8/2 188 / 195, eight ranks 900 335 / 342) nor in two launches (2300 x 64/4 1838 / 1939, 2 x 1371 x 64/4 836 / 865).
-bool half_as_many(const pith_attn_bwd_args* a, int64_t wgs, bool chunks) {
-  const int64_t cus = compute_units_or_default();
+// equal. Not with fewer (2 x 1314 x 8/2 188 / 195, eight ranks 900 335 / 342) nor with more than four, where the two differ by -2 to +2 % (one grid 2300 x 64/4
+// 1439 / 1426, 2 x 1200 x 64/4 887 / 885, 2500 x 64/4 contiguous 2894 / 2847, 2050 x 64/4 2058 / 2100), two ranks 3348 x 64/4 1529 / 1689.
+// half: the parts there would be
+bool half_as_many(const pith_attn_bwd_args* a, int64_t tiles, int half, bool chunks) {
+  const int64_t cus = compute_units_or_default(), wgs = tiles * a->Hkv * a->B * half;
   if (chunks) {
     const int64_t q_wgs = (a->Sq + 127) / 128 * a->Hq * a->B;
     return a->Dqk == 128 && q_wgs > cus && q_wgs <= 4 * cus;
   }
   if (a->Dqk == 192) return false;
   if (a->Dqk == 64) return a->Sq <= 5120;
-  // (ds_handover_pays, 512 query rows per workgroup of its dQ)
-  const bool hands_over = (a->Sq + 511) / 512 * a->Hq * a->B >= cus || 100 * a->Sq * a->Hq * a->B >= 69 * 512 * cus;
+  const bool hands_over = handover_rows_pay(a->B, a->Sq, a->Hq, a->causal != 0, cus);
   if (!a->causal) return a->Sq <= 2816 && (!hands_over || 4 * wgs >= 3 * cus);
-  if (5 * wgs >= 8 * cus) return a->Sq <= 4096;
-  return a->Sq <= (hands_over && 8 * wgs < 11 * cus ? 768 : 2304);
+  if (a->Sq > (5 * wgs >= 8 * cus ? 4096 : 2304)) return false;
+  const int64_t walk = a->Sq * (a->Hq / a->Hkv / half);
+  return !hands_over || walk <= (8 * wgs <= 9 * cus ? 4096 : 8 * wgs < 11 * cus ? 6144 : 2 * wgs <= 3 * cus ? 12288 : 24576);
 }
 
 // tiles: key tiles of the launch, over all of its chunks
@@ -142,7 +146,7 @@ int pick_split(const pith_attn_bwd_args* a, int64_t tiles, bool chunks = false) 
   // within 2 %).
   const int64_t want = (a->causal ? 2 : 1) * (a->Dqk == 64 ? 2 : 1) * (int64_t)compute_units_or_default();
   while (split < group && base * split < want && group % (split * 2) == 0) split *= 2;
-  if (split > 1 && base * split > want && half_as_many(a, base * split / 2, chunks)) split /= 2;
+  if (split > 1 && base * split > want && half_as_many(a, tiles, split / 2, chunks)) split /= 2;
   return split;
 }
 

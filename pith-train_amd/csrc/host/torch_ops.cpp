@@ -19,6 +19,7 @@
 #include <cstdlib>
 
 #include "pith_hip.h"
+#include "../handover_rows.h"
 
 namespace {
 
@@ -509,9 +510,7 @@ Two attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bo
 //                          640 and more 8 x 640 x 32/8 232 / 233, 16 x 640 x 32/4 439 / 441, 8 x 720 x 16 155 / 164
 //   causal, from 513 on    4 x 513 x 32/4 98 / 99, 4 x 600 x 32/4 113 / 110, 8 x 600 x 32/4 167 / 173, 4 x 600 x 64/4 168 / 174, 8 x 1025 x 32/4 333 / 354
 bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hkv, bool causal, int64_t cus) {
-  const bool fills = (sq + 511) / 512 * hq * b >= cus;
-  if (cus <= 0 || (!fills && (sq > 16384 || 100 * sq * hq * b < 69 * 512 * cus))) return false;
-  if (sq <= 256 || (!causal && sq > 512 && sq < 640)) return false;
+  if (cus <= 0 || !pith::handover_rows_pay(b, sq, hq, causal, cus)) return false;
   pith_attn_bwd_args a = {};
   a.B = b; a.Sq = sq; a.Skv = skv; a.Hq = hq; a.Hkv = hkv; a.Dqk = a.Dv = 128; a.causal = causal;
   pith_attn_bwd_plan_t plan;
@@ -519,7 +518,7 @@ bool ds_handover_pays(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_t hk
   const int64_t key_tiles = (skv + plan.dkdv_rows - 1) / plan.dkdv_rows * plan.dkdv_rows / 128;
   const int64_t dkdv_wgs = key_tiles * hkv * b * plan.dkdv_split;
   // (causal 7900 x 12/4, 248 of them: 887 / 837)
-  if (!fills && causal && 2 * dkdv_wgs < 3 * cus) return false;
+  if (causal && 2 * dkdv_wgs < 3 * cus && !pith::handover_fills_device(b, sq, hq, cus)) return false;
   return 4 * dkdv_wgs >= 3 * cus;
 }
 

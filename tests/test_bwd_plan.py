@@ -273,6 +273,12 @@ def test_share_of_64_features_in_two_launches(gpu):
     (1, 3, 1500, 32, 4, 128, 4), (1, 1, 4096, 32, 4, 128, 4), (1, 1, 4097, 32, 4, 128, 4), (1, 1, 3900, 32, 4, 128, 4), (1, 9, 768, 32, 4, 128, 2),
     (1, 9, 769, 32, 4, 128, 2), (1, 24, 128, 32, 4, 128, 4), (0, 1, 1100, 32, 4, 128, 4), (0, 2, 1100, 64, 4, 128, 4), (0, 1, 2816, 32, 4, 128, 2),
     (0, 1, 2817, 32, 4, 128, 4), (1, 9, 1100, 32, 8, 64, 1), (1, 1, 5120, 32, 8, 64, 2), (1, 1, 5121, 32, 8, 64, 4), (0, 4, 1290, 32, 8, 64, 1), (1, 3, 768, 32, 4, 192, 8),
+    # rows that do not hand dS over without a mask: up to 256, 513 to 639
+    (0, 4, 520, 32, 4, 128, 2), (0, 4, 600, 64, 4, 128, 2), (0, 20, 160, 32, 4, 128, 1), (0, 33, 100, 32, 4, 128, 1), (0, 8, 640, 16, 4, 128, 2), (0, 10, 400, 32, 4, 128, 2),
+    # handing over under the mask: rows x heads of a part up to 4096, 6144, 12288, 24576 at 1.125, 1.375, 1.5 workgroups per unit and more
+    (1, 11, 768, 16, 4, 128, 1), (1, 13, 520, 32, 4, 128, 2), (1, 11, 768, 64, 4, 128, 2), (1, 9, 1024, 16, 4, 128, 1), (1, 9, 1025, 16, 4, 128, 1), (1, 12, 664, 64, 4, 128, 2),
+    (1, 13, 768, 32, 4, 128, 1), (1, 13, 709, 64, 4, 128, 2), (1, 7, 1500, 16, 4, 128, 1), (1, 7, 1500, 32, 4, 128, 2), (1, 15, 768, 64, 4, 128, 1), (1, 5, 2304, 64, 4, 128, 2),
+    (1, 8, 1368, 64, 4, 128, 2), (1, 11, 1152, 64, 4, 128, 1), (1, 7, 1800, 64, 4, 128, 2), (1, 3, 2048, 64, 4, 128, 4),
 ])  # fmt: skip
 def test_head_split_is_halved_where_that_is_faster(causal, b, s, hq, hkv, d, split):
     """As measured (table at half_as_many)."""
