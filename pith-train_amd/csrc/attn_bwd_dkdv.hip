@@ -523,6 +523,10 @@ extern "C" int64_t pith_attn_bwd_chunks_workspace_bytes(const pith_attn_bwd_args
   pith_attn_bwd_args a;
   int64_t tiles;
   if (!merged_call(args, chunks, n, &a, &tiles)) return 0;
+  if (n == 1) {  // goes out as pith_attn_bwd, whose head split is another one (with less than it asks for there is none: 1 x 3200 x 32/4 399 -> 617 us)
+    a.causal = 1;
+    return pith_attn_bwd_dkdv_workspace_bytes(&a);
+  }
   return workspace_bytes_for(&a, pick_chunks_split(a, tiles));
 }
 

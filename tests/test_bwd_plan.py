@@ -294,6 +294,19 @@ def test_head_split_of_shares(b, s, hq, hkv, cp, rank, layout, d, split):
     assert _share_plan(b, s, hq, hkv, cp, rank, layout, d).dkdv_split == split
 
 
+@pytest.mark.parametrize("two_part", [False, True])
+@pytest.mark.parametrize("b,s,hq,hkv,d", [(1, 3200, 32, 4, 128), (1, 3600, 32, 4, 128), (2, 1700, 32, 4, 128), (1, 4300, 32, 8, 64), (1, 8192, 32, 4, 128), (3, 1100, 32, 4, 128),
+                                          (1, 256, 8, 2, 128), (1, 2304, 64, 4, 128), (1, 2305, 64, 4, 128), (2, 1024, 16, 16, 192), (3, 768, 32, 4, 192)])  # fmt: skip
+def test_share_of_one_chunk_asks_for_the_workspace_of_the_call_it_is(b, s, hq, hkv, d, two_part):
+    if two_part and (d != 192 or hq != hkv):
+        return
+    dv, pe = min(d, 128), 256 if two_part else None
+    share = _C.AttnBwdArgs(B=b, Sq=s, Hq=hq, Hkv=hkv, Dqk=d, Dv=dv)
+    chunk = (_C.KeyChunk * 1)(_C.KeyChunk(rows=s, q_row0=0, k_pe=pe))
+    call = _C.AttnBwdArgs(B=b, Sq=s, Skv=s, Hq=hq, Hkv=hkv, Dqk=d, Dv=dv, causal=1, k_pe=pe)
+    assert _C.lib().pith_attn_bwd_chunks_workspace_bytes(_C.byref(share), chunk, 1) == _C.lib().pith_attn_bwd_dkdv_workspace_bytes(_C.byref(call))
+
+
 @pytest.mark.parametrize("causal,b,s,hq,hkv,pays", [
     # 0.687 / 0.69 of the device filled with rows, to 16384 of them; enough dK/dV workgroups under the mask
     (True, 1, 2816, 32, 4, False), (True, 1, 2827, 32, 4, True), (False, 1, 2827, 32, 4, True), (True, 3, 768, 32, 4, False), (True, 1, 1450, 64, 4, True),
