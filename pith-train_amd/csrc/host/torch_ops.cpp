@@ -572,6 +572,7 @@ bool ds_handover_pays_192(int64_t b, int64_t sq, int64_t skv, int64_t hq, int64_
 //              342, 4098 604 / 622, 8194 1972 / 2270
 bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const std::vector<std::array<int64_t, 4>>& steps, int64_t cus, int64_t dqk) {
   if (cus <= 0 || hkv <= 0) return false;
+  if (steps.size() == 1) return steps[0][3] != 0;  // a call like any other
   const auto lost = [&](int64_t wgs, int per_unit = 1) {
     const int64_t round = per_unit * cus;
     return (double)((wgs + round - 1) / round * round) / (double)wgs;
@@ -593,7 +594,6 @@ bool share_hands_over(int64_t b, int64_t rows, int64_t hq, int64_t hkv, const st
     full_lost += work * (0.7 * lost((skv + plan.dkdv_rows - 1) / plan.dkdv_rows * heads * b * plan.dkdv_split) + 0.3 * lost((sq + dq_rows - 1) / dq_rows * a.Hq * b));
   }
   if (handed == 0) return false;
-  if (steps.size() == 1) return true;  // a call like any other
   const int64_t q_wgs = (rows + 127) / 128 * hq * b;
   if (full == 0 && q_wgs > 4 * cus && rows >= 2304 && 4 * handed >= all && lost(q_wgs, 2) >= 1.1) return true;
   if (2 * handed < all) return false;

@@ -225,6 +225,13 @@ def test_shares_of_192_that_go_out_step_by_step(steps, b, s, h, cp, rank, layout
     assert native.share_hands_over(b, s, h, h, sizes, UNITS, 192) == bool(steps)
 
 
+def test_share_of_one_step_hands_over_as_the_call_it_is():
+    """Also where its rows are less than a full device's."""
+    for s, pays in ((3200, True), (2816, False), (4096, True)):
+        assert native.ds_handover_pays(1, s, s, 32, 4, True, UNITS) == pays
+        assert native.share_hands_over(1, s, 32, 4, [(s, s, True, 4 if pays else 0)], UNITS) == pays
+
+
 def test_share_of_slabs_counts_their_grids():
     """131072 tokens, 64/4 heads: a slab of one kv head at a time fills the device; a quarter of its heads would not."""
     sizes = lambda heads: [(16384, 8192, False, heads)] * 3 + [(8192, 16384, False, heads)] * 4 + [(16384, 16384, True, 0)]  # noqa: E731
