@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_direct_kernel(FwdArgs<MULTI
     n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
     n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
-  if (CAUSAL) n_tiles_wave = tiles_of_wave(n_tiles_wave, q_wave0, p.Sq);
+  if (CAUSAL && !(HALF && MULTI)) n_tiles_wave = tiles_of_wave(n_tiles_wave, q_wave0, p.Sq);
   TileSource<MULTI, CAUSAL, kBN> k_src(p, range, k_row_bytes, k_rows), kx_src(p, range, kx_row_bytes, kx_rows),
       v_src(p, range, v_row_bytes, v_rows);
   TileMask<MULTI, CAUSAL, kBN> mask(p, range);
