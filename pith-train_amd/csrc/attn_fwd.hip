@@ -76,8 +76,9 @@ namespace {
 //                W 2.5 - 3   2 x 1024 x 20 27.5 / 24.4 / 35.6 / 24.6
 //   d192 full    W 1         2 x 256 x 32 10.5 / 10.4 / 10.7 / 9.5, 512 x 32 15.3 / 13.9 / 13.3 / 12.9
 //                W 2         4 x 256 x 32 12.8 / 14.4 / 21.2 / 14.0, 2 x 512 x 32 18.2 / 17.2 / 26.5 / 19.3, 1024 x 2048 x 32 50.5 / 44.6 / 60.5 / 54.9
-// Shares whose rows are short beside their streams gain nothing from a second round of QUARTER: rank 1 of 4, 1022 x 32/4 of 128,
-// 67.1 / 51.7 / 73.2 / 56.6.
+// Zigzag shares above W 1.5 take QUARTER while the workgroups of their longer half are one round, HALF / QUARTER: 224 to 256 of them 896 x 32/4 of 128, eight ranks,
+// rank 0 164 / 81, four 78 / 49, 960 x 32/4 rank 2 116 / 95, 2 x 1024 x 16/4 117 / 98, 3 x 1204 x 8/2 143 / 115, 960 x 32 of 192 194 / 138; 260 to 288 1022 x 32/4 rank
+// 2 124 / 156, 1530 x 20/5 179 / 219, 3 x 1270 x 8/2 148 / 187, 1300 x 24/3 240 / 260, 1022 x 32 of 192 144 / 185.
 enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter, kSmall };
 
 // Calls against one chunk a little above a whole round of 128-row workgroups, W of them per compute unit (a ragged length is enough): the
@@ -158,7 +159,9 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   if (unequal && wgs64 <= 2 * cus) {
     const bool quarter_more = 4 * wgs64 > 5 * cus, half_more = 2 * wgs64 > 3 * cus;  // workgroups than one round of QUARTER
     const int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
-    if (a->Skv >= from && (!half_more || a->Sq >= 1536)) return Split::kQuarter;
+    // 64-row workgroups of the longer half of a zigzag share's rows; what a second round holds besides is short
+    const int64_t longer = ((a->Sq + 63) / 64 - a->Sq / 2 / 64) * a->Hq * a->B;
+    if (a->Skv >= from && (!half_more || (a->Skv == a->Sq ? a->Sq >= 1536 : longer <= cus))) return Split::kQuarter;
   }
   if (small_workgroups(a, wgs64, cus, unequal)) return Split::kSmall;
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;

@@ -116,7 +116,7 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
     n_tiles_wg += min(tiles, (m0 + kBM - 1) / kBN + 1);
     n_tiles_wave += min(tiles, (q_wave0 + 31) / kBN + 1);
   }
-  n_tiles_wave = tiles_of_wave(n_tiles_wave, q_wave0, p.Sq);
+  if constexpr (PARTS != 2) n_tiles_wave = tiles_of_wave(n_tiles_wave, q_wave0, p.Sq);
   const int intervals = (n_tiles_wg + kTeams - 1) / kTeams;  // of the workgroup
   if constexpr (kTeams > 1) {  // from here on a team's own tiles (the second team of a single tile has none)
     n_tiles_wg = (n_tiles_wg + 1 - team) >> 1;

@@ -205,7 +205,8 @@ struct TileMask {
 // workgroups (8 x 643 x 64/4 147 / 140, 6 x 530 x 32/4 42.0 / 39.8, 8 x 1290 x 32/8 of 64 129 / 126): the others know there that all waves walk as far
 // as their workgroup, and lose more in the loops without it (256-row forward 8200 x 16 570 / 638, 4 x 1564 x 16 85 / 89; dQ 4100 x 8/2 362 / 371,
 // 3 x 3457 x 4 of 64 206 / 211). Nor in the forward of several chunks by wave pairs, which loses with and without such waves: without / with it 4200 x 8/2,
-// eight ranks, 397 / 421, 5000 x 8/2 537 / 566, 1262 x 32/4 149 / 155, 4096 x 16 of 192, four ranks, rank 0 322 / 330; 4100 x 8/2 contiguous 262 / 259.
+// eight ranks, 397 / 421, 5000 x 8/2 537 / 566, 1262 x 32/4 149 / 155, 4096 x 16 of 192, four ranks, rank 0 322 / 330; 4100 x 8/2 contiguous 262 / 259; nor in
+// that of two teams (64 features: 7790 x 8 90.1 / 92.0, 3072 x 16 36.5 / 37.3).
 __device__ __forceinline__ int tiles_of_wave(int tiles, int q_wave0, int sq) { return q_wave0 < sq ? tiles : min(tiles, 1); }
 
 // ---------------------------------------------------------------------------------------------

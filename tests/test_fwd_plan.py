@@ -73,3 +73,14 @@ def test_shares_of_64_features_of_long_streams():
 def test_zigzag_shares_of_256_row_workgroups(full, b, s, hq, hkv, cp, rank):
     """As measured (comment at pick_split)."""
     assert (_share_split(b, s, hq, hkv, 128, cp, rank, "zigzag") == FULL) == bool(full)
+
+
+@pytest.mark.parametrize("quarter,b,s,hq,hkv,d,cp,rank", [
+    # the longer half in up to 256 workgroups of 64 rows or in more
+    (1, 1, 896, 32, 4, 128, 8, 0), (1, 1, 960, 32, 4, 128, 8, 2), (1, 2, 1024, 16, 4, 128, 8, 0), (1, 3, 1204, 8, 2, 128, 8, 2), (1, 1, 896, 32, 4, 128, 4, 0), (1, 1, 960, 32, 32, 192, 8, 0),
+    (1, 3, 1280, 8, 8, 192, 8, 0), (0, 1, 1022, 32, 4, 128, 8, 2), (0, 1, 1530, 20, 5, 128, 8, 0), (0, 3, 1270, 8, 2, 128, 8, 2), (0, 1, 1300, 24, 3, 128, 8, 0), (0, 1, 1022, 32, 32, 192, 8, 0),
+    (0, 1, 768, 40, 8, 128, 2, 0), (1, 1, 1850, 16, 4, 64, 4, 0), (1, 2, 788, 16, 16, 64, 2, 0), (1, 1, 1062, 16, 16, 128, 4, 2),
+])  # fmt: skip
+def test_zigzag_shares_of_64_row_workgroups_in_teams(quarter, b, s, hq, hkv, d, cp, rank):
+    """As measured (in front of Split)."""
+    assert (_share_split(b, s, hq, hkv, d, cp, rank, "zigzag") == QUARTER) == bool(quarter)
