@@ -228,6 +228,12 @@ __global__ __launch_bounds__((DuoLayout<DQK, PARTS>::kThreads), 2) void attn_fwd
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
   float m_run = -INFINITY;
+  // A row that sees nothing of the first chunks has no maximum until its own, and would have the whole workgroup take that of every tile anew: in a zigzag share's
+  // 64-row workgroup across the first row that sees the other chunks, whose teams it made wait for each other. Any finite start below all scores spares that (the
+  // first key that a row sees exceeds the limit and sets its maximum; nothing has been added up by then). Rank 0 of four, 1514 x 16/4 heads of 128 85.5 us before the teams took
+  // turns, 89.4 since, 72.4 without these maxima, of eight 960 x 32/4 116 / 123 / 96, 2260 x 8/2 255 / 265 / 205, 1008 x 16 of 192 67.8 / 68.0 / 58.2.
+  if constexpr (MULTI && PARTS == 4)
+    if (qrow < chunk_of(p, range.first()).q_row0) m_run = -1e38f / fmaxf(p.kappa, 1.f);  // (times kappa finite, too)
   float l_run = 0.f;  // this lane's share of the row sum (the partner lane holds the rest)
   f32x16 s[KVB];       // S^T of one tile: 32 x 32 tiles [keys] x [queries]
   bf16x8 pf[2 * KVB];  // P^T as B operand, one fragment per 16 keys

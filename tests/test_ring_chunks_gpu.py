@@ -62,6 +62,30 @@ def test_share(gpu, monkeypatch, one_launch, B, S, Hq, Hkv, D, C, rank, layout, 
             check_bf16_result(dpe[0][j], ref_dk[j][..., 128:].sum(2), f"chunk {j} dk_pe", otol=1e-3)
 
 
+@pytest.mark.parametrize("S,Hq,Hkv,D,C", [(1030, 2, 1, 128, 4), (1030, 2, 2, 192, 4), (1030, 2, 1, 64, 4), (650, 2, 2, 192, 8), (98, 4, 2, 128, 2), (130, 260, 130, 64, 2)])
+def test_share_of_rows_that_see_nothing_at_first(gpu, monkeypatch, S, Hq, Hkv, D, C):
+    """Rank 0, zigzag: the first half of the rows sees only its own chunk, which comes last; a workgroup across the halves walks all of them."""
+    test_share(gpu, monkeypatch, True, 1, S, Hq, Hkv, D, C, 0, "zigzag", False)
+
+
+@pytest.mark.parametrize("scale,size", [(4.0, 1.0), (1e-3, 1.0), (128**-0.5, 30.0), (30.0, 3.0)])
+def test_share_of_rows_that_see_nothing_at_first_at_other_scales(gpu, scale, size):
+    """Scores of up to some 10^4 either way; each row against all keys it sees."""
+    g = torch.Generator(device=gpu).manual_seed(8)
+    mk = lambda: (size * torch.randn(1, 1030, 2, 128, generator=g, device=gpu)).to(torch.bfloat16)  # noqa: E731
+    q, ks, vs = mk(), [mk() for _ in range(3)], [mk() / size for _ in range(3)]
+    out, lse = L.ring_forward_local(q, ks, vs, scale, 0, 3, "zigzag")
+    at = lambda j: torch.cat([torch.arange(515) + 515 * j, torch.arange(515) + 515 * (5 - j)])  # noqa: E731
+    hidden = (torch.cat([at(j) for j in range(3)])[None, :] > at(0)[:, None]).to(gpu)
+    s = q[0].transpose(0, 1).double() @ torch.cat(ks, 1)[0].permute(1, 2, 0).double().contiguous() * scale
+    s = s.masked_fill(hidden, float("-inf"))
+    # fp32 scores and LSE of size x: 2^-23 x log2(e) each, over some dozen roundings
+    bound = 1e-3 + 16 * 2**-23 * 1.4427 * s[s > -1e30].abs().max().item()
+    check_lse(lse, torch.logsumexp(s, -1)[None] / 0.6931471805599453, "LSE2", tol=bound)
+    if scale * size**2 <= 128:  # (beyond, scores close to each other are rounded apart: P is another function)
+        check_bf16_result(out, (torch.softmax(s, -1) @ torch.cat(vs, 1)[0].transpose(0, 1).double().contiguous()).transpose(0, 1)[None], "O")
+
+
 def test_share_of_unequal_rows_64_features(gpu, monkeypatch):
     """The two-team forward over several chunks."""
     test_share(gpu, monkeypatch, True, 1, 1026, 36, 36, 64, 2, 0, "zigzag", False)
