@@ -79,6 +79,10 @@ namespace {
 // Zigzag shares above W 1.5 take QUARTER while the workgroups of their longer half are one round, HALF / QUARTER: 224 to 256 of them 896 x 32/4 of 128, eight ranks,
 // rank 0 164 / 81, four 78 / 49, 960 x 32/4 rank 2 116 / 95, 2 x 1024 x 16/4 117 / 98, 3 x 1204 x 8/2 143 / 115, 960 x 32 of 192 194 / 138; 260 to 288 1022 x 32/4 rank
 // 2 124 / 156, 1530 x 20/5 179 / 219, 3 x 1270 x 8/2 148 / 187, 1300 x 24/3 240 / 260, 1022 x 32 of 192 144 / 185.
+// Where the other half is not short (mean 2/3) 128 and 192 features wait for 3072 keys from W 1.2 and for 6144 from W 1.3 on: 1024 x 20 of 192, two ranks, rank 1, 33.3 / 35.7, 1280 x
+// 16/4 of 128 32.6 / 33.6; 678 x 32 of 192 rank 2 46 / 50, 3 x 2510 x 4 74 / 78, 4 x 1504 x 4/1 of 128 40.6 / 41.7, but W 1.25 1240 x 16 of 192 rank 2 70 / 58, W 1.5 3 x 2074 x 4
+// 118 / 110, eight ranks, rank 4 1352 x 16 156 / 137. 64 features for 2048 from W 1.4, and above 1.5 for 1536 rows: 3 x 256 x 32/8 24.7 / 26.4, 3 x 552 x 16/4
+// 26.8 / 29.0, 1280 x 24/6 27.8 / 29.1, 3 x 2152 x 4 39.9 / 37.3.
 enum class Split { kFull, kDuo, kHalf, kTeams, kQuarter, kSmall };
 
 // Calls against one chunk a little above a whole round of 128-row workgroups, W of them per compute unit (a ragged length is enough): the
@@ -158,10 +162,14 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
   if (a->Skv > 64 && wgs64 <= cus) return a->Skv > (d64 ? 384 : 512) ? Split::kQuarter : Split::kSmall;
   if (unequal && wgs64 <= 2 * cus) {
     const bool quarter_more = 4 * wgs64 > 5 * cus, half_more = 2 * wgs64 > 3 * cus;  // workgroups than one round of QUARTER
-    const int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
+    int64_t from = d64 ? 1536 : half_more ? (a->Dqk == 192 ? 2048 : 3072) : quarter_more ? (a->Dqk == 192 ? 1400 : 1536) : 1024;
+    const bool one_chunk = a->Skv == a->Sq, both_long = mean > 64;  // (of several chunks: the half that sees less, too)
+    if (both_long && d64 && 5 * wgs64 > 7 * cus) from = 2048;
+    if (both_long && !d64 && 5 * wgs64 > 6 * cus) from = 10 * wgs64 > 13 * cus ? 6144 : 3072;
     // 64-row workgroups of the longer half of a zigzag share's rows; what a second round holds besides is short
     const int64_t longer = ((a->Sq + 63) / 64 - a->Sq / 2 / 64) * a->Hq * a->B;
-    if (a->Skv >= from && (!half_more || (a->Skv == a->Sq ? a->Sq >= 1536 : longer <= cus))) return Split::kQuarter;
+    const bool second_round = (one_chunk || longer <= cus) && (a->Sq >= 1536 || !(one_chunk || (d64 && both_long)));
+    if (a->Skv >= from && (!half_more || second_round)) return Split::kQuarter;
   }
   if (small_workgroups(a, wgs64, cus, unequal)) return Split::kSmall;
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;

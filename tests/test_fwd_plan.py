@@ -79,7 +79,8 @@ def test_zigzag_shares_of_256_row_workgroups(full, b, s, hq, hkv, cp, rank):
     # the longer half in up to 256 workgroups of 64 rows or in more
     (1, 1, 896, 32, 4, 128, 8, 0), (1, 1, 960, 32, 4, 128, 8, 2), (1, 2, 1024, 16, 4, 128, 8, 0), (1, 3, 1204, 8, 2, 128, 8, 2), (1, 1, 896, 32, 4, 128, 4, 0), (1, 1, 960, 32, 32, 192, 8, 0),
     (1, 3, 1280, 8, 8, 192, 8, 0), (0, 1, 1022, 32, 4, 128, 8, 2), (0, 1, 1530, 20, 5, 128, 8, 0), (0, 3, 1270, 8, 2, 128, 8, 2), (0, 1, 1300, 24, 3, 128, 8, 0), (0, 1, 1022, 32, 32, 192, 8, 0),
-    (0, 1, 768, 40, 8, 128, 2, 0), (1, 1, 1850, 16, 4, 64, 4, 0), (1, 2, 788, 16, 16, 64, 2, 0), (1, 1, 1062, 16, 16, 128, 4, 2),
+    (0, 1, 768, 40, 8, 128, 2, 0), (1, 1, 1850, 16, 4, 64, 4, 0), (1, 2, 788, 16, 16, 64, 2, 0), (1, 1, 1062, 16, 16, 128, 4, 2), (0, 3, 2510, 4, 4, 192, 2, 1), (1, 3, 2074, 4, 4, 192, 4, 2), (0, 1, 678, 32, 32, 192, 4, 2), (1, 1, 2370, 8, 8, 192, 2, 1), (1, 1, 1782, 16, 16, 192, 8, 3),
+    (1, 1, 1240, 16, 16, 192, 4, 2), (1, 2, 636, 16, 4, 128, 8, 4), (0, 3, 552, 16, 4, 64, 4, 2), (0, 1, 1280, 24, 6, 64, 2, 1), (0, 3, 256, 32, 8, 64, 8, 4), (0, 1, 1024, 20, 20, 192, 2, 1), (1, 1, 1290, 16, 4, 64, 2, 1), (1, 3, 2152, 4, 4, 64, 2, 1),
 ])  # fmt: skip
 def test_zigzag_shares_of_64_row_workgroups_in_teams(quarter, b, s, hq, hkv, d, cp, rank):
     """As measured (in front of Split)."""
