@@ -37,7 +37,7 @@ def test_split_query():
     # 64 features, unequal rows, more than two 64-row workgroups per unit: all at once and rows that pad 128, many tiles, whole rounds
     (1, 12, 128, 32, 64, 1), (0, 14, 128, 32, 64, 1), (0, 16, 128, 32, 64, 1), (1, 10, 192, 32, 64, 1), (0, 12, 192, 32, 64, 1), (0, 8, 256, 32, 64, 1),
     (1, 6, 320, 32, 64, 1), (0, 7, 320, 29, 64, 1), (0, 3, 370, 64, 64, 1), (1, 3, 512, 32, 64, 1), (0, 5, 512, 27, 64, 1), (0, 5, 448, 27, 64, 1),
-    (1, 2, 768, 32, 64, 1), (1, 3, 768, 28, 64, 1), (0, 3, 768, 27, 64, 1), (1, 2, 900, 30, 64, 1), (0, 3, 900, 24, 64, 1), (1, 4, 512, 32, 64, 1), (0, 7, 256, 30, 64, 1), (0, 3, 768, 32, 64, 1), (1, 2, 1000, 32, 64, 1), (0, 3, 1024, 23, 64, 1), (1, 2, 1200, 29, 64, 1),
+    (1, 2, 768, 32, 64, 1), (1, 3, 768, 28, 64, 1), (0, 3, 768, 27, 64, 1), (1, 2, 900, 30, 64, 1), (0, 3, 900, 24, 64, 1), (1, 4, 512, 32, 64, 1), (0, 7, 256, 30, 64, 1), (0, 3, 768, 32, 64, 1), (1, 2, 1000, 32, 64, 1), (0, 3, 1024, 23, 64, 1), (1, 1, 1088, 64, 64, 1), (1, 2, 1200, 29, 64, 1),
     (1, 2, 2048, 18, 64, 1), (1, 2, 2048, 16, 64, 1), (1, 1, 2560, 20, 64, 1), (0, 4, 2855, 4, 64, 1), (0, 1, 2914, 16, 64, 1), (0, 1, 6144, 8, 64, 1),
     (1, 1, 4096, 16, 64, 1), (1, 1, 4404, 16, 64, 1),
     # without a mask, up to two per unit
@@ -62,6 +62,7 @@ def test_few_rows():
 def test_shares_of_64_features_of_long_streams():
     """Nearly equal rows, two teams above 2048 keys."""
     assert _share_split(2, 2240, 4, 4, 64, 4, 3, "contiguous") == TEAMS and _share_split(1, 500, 40, 40, 64, 4, 3, "contiguous") == SMALL
+    assert _share_split(1, 1152, 32, 8, 64, 4, 0, "zigzag") == SMALL  # (unequal ones stay at four waves)
 
 
 @pytest.mark.parametrize("full,b,s,hq,hkv,cp,rank", [
