@@ -345,11 +345,11 @@ int run_dkdv(const pith_attn_bwd_args* a, const Plan& plan, void* workspace, hip
     p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + split_bytes_for(a, split));
   }
   begin_launch();
+  p.through_parts = through_results(workspace_bytes_for(a, workspace ? split : 1));
   if (split > 1 && workspace) {
     p.split = split;
     p.ws_dk = reinterpret_cast<float*>(workspace);
     p.ws_dv = p.ws_dk + (int64_t)split * a->B * a->Skv * a->Hkv * a->Dqk;
-    p.through_parts = through_results(split_bytes_for(a, split));
   }
   // dS hand-over to the dQ call: only when the buffer is usable (otherwise the call behaves as without it)
   if (ds_usable(a)) {
@@ -607,7 +607,7 @@ int run_bwd_chunks(const pith_attn_bwd_args* args, const pith_key_chunk* chunks,
   p.ws_dk = reinterpret_cast<float*>(need > 0 ? args->workspace : nullptr);
   p.ws_dv = p.ws_dk + (split > 1 ? (int64_t)split * all.B * all.Skv * all.Hkv * all.Dqk : 0);
   p.ws_dkpe = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws_dk) + split_bytes_for(&all, split));
-  p.through_parts = through_results(split_bytes_for(&all, split));
+  p.through_parts = through_results(need);
   hipStream_t st = (hipStream_t)stream;
   begin_launch();
   const ChunkGrids grids = chunk_grids(&all, tiles, split, blocks);

@@ -482,15 +482,11 @@ __device__ __forceinline__ bf16x8 lds_read_transposed_at(const char* lo_addr, co
 // a bf16 tensor laid out like `block`) the result, old values included, is rounded to bf16 and written there, and
 // `block` keeps what it held.
 // bf16 rows leave in one of two ways (through_results): workgroups that are still in their loops share K and V (Q and dO) through the
-// second-level cache, which plain stores fill with rows that wait there to be written. fp32 rows are read again soon, by the sums over
-// head parts or the next ring step: plain, nt 0.3 % slower.
+// second-level cache, which plain stores fill with rows that wait there to be written. fp32 rows are read again soon, by the sums over head parts
+// (written through or plain, see there) or the next ring step (plain, nt 0.3 % slower).
 template <int NB>
 constexpr int kRowsViaLdsBytes = 32 * (NB * 128 + 16);
 
-// The fp32 partial sums of the head split follow the same line, plain stores instead of nt beyond it (their reader is the next launch, and what
-// they leave in the second-level caches is written back at the end of the launch). Forward + backward, plain / sc1 / nt, us: 32 MiB 1024 x 32/4 of
-// 128 without a mask 94.7 / 92.0 / 93.6, 2 x 2048 x 16/4 of 64 105.0 / 104.3 / 105.7; 56 to 78 MiB 8 x 512 x 32/4 142.3 / 140.8 / 142.5, 3 x 768 x 32/4
-// 123.1 / 121.5 / 123.2, but 4 x 947 x 64/4 330 / 332 / 334, 4096 x 32/4 523 / 528 / 532, 4992 x 32/8 of 64 472.5 / 472.9 / 475.3.
 // Whether results of that many bytes (O, dQ, or dK and dV of a launch together) are written through the second-level caches (sc1) rather than
 // non-temporally: as long as the 8 x 4 MB of them could hold it. Either keeps the tiles of the other workgroups cached, but what went out non-temporally its next reader fetches from
 // memory. Plain / sc1 / nt, us, the forward alone and with the projection that reads O:
@@ -502,6 +498,11 @@ constexpr int kRowsViaLdsBytes = 32 * (NB * 128 + 16);
 //   47 MiB    3 x 1999 x 32/4 of 128 106.3 / 105.2 / 102.8 and 183.8 / 183.6 / 183.2
 // and the backward with the products that read dQ, dK and dV: 512 x 32/4 of 128 71.2 / 71.0 / 72.3, 2048 x 16 of 192/128 181.0 / 181.1 / 182.7, the others within
 // 0.5 %. sc1 nt as nt, sc0 sc1 as sc1.
+// The fp32 partial sums of a launch (head parts, k_pe per head) follow the same line by the bytes of all of them, with plain stores instead of nt beyond it: their reader is the
+// next launch, and what they leave in the second-level caches is written back at the end of the launch. Forward + backward, plain / sc1 / nt, us: 32 MiB 1024 x 32/4 of
+// 128 without a mask 94.7 / 92.0 / 93.6, 2 x 2048 x 16/4 of 64 105.0 / 104.3 / 105.7; 56 to 78 MiB 8 x 512 x 32/4 142.3 / 140.8 / 142.5, 3 x 768 x 32/4
+// 123.1 / 121.5 / 123.2, but 4 x 947 x 64/4 330 / 332 / 334, 4096 x 32/4 523 / 528 / 532, 4992 x 32/8 of 64 472.5 / 472.9 / 475.3. Per-head k_pe, plain / sc1, equal: 12 MiB
+// 1021 x 16, four ranks, 157.5 / 157.5, 32 MiB 4096 x 16, two ranks, 912 / 913, 128 MiB 2 x 4096 x 16 4034 / 4048, 8192 x 16 5073 / 5074.
 inline bool through_results(int64_t bytes) { return bytes <= (int64_t)32 << 20; }
 
 template <typename OutT, int NB>
