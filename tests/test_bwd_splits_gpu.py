@@ -4,6 +4,8 @@ import pytest
 import torch
 
 from helpers import check_bf16_result
+from pithtrain_amd import _C
+from pithtrain_amd.operators.mla import hip
 from pithtrain_amd.operators.mla.hip import _mla_bwd_dk_dv, _mla_bwd_dq, _mla_bwd_preprocess, _mla_fwd, attn_bwd_pair_into
 
 pytestmark = pytest.mark.gpu
@@ -66,16 +68,26 @@ def test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
     (1, 2560, 2560, 32, 4, 128, True), (1, 2561, 2561, 32, 4, 128, True), (1, 1024, 1024, 64, 8, 128, True), (1, 1023, 1023, 64, 8, 128, True),
     (1, 1536, 1536, 32, 32, 192, True), (1, 1535, 1535, 32, 32, 192, True), (1, 1500, 1600, 32, 32, 192, False),
 ])  # fmt: skip
-def test_backward_pairs_of_a_few_rounds(gpu, B, Sq, Skv, Hq, Hkv, D, causal):
+def test_backward_pairs_of_a_few_rounds(gpu, monkeypatch, B, Sq, Skv, Hq, Hkv, D, causal):
+    monkeypatch.setattr(hip, "DS_BUFFER_LIMIT_BYTES", 0)  # (192 features would hand dS over)
     test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, causal)
 
 
 @pytest.mark.parametrize("B,Sq,Skv,Hq,Hkv,D", [
-    # eight head parts: 32 MiB of partial sums, written through, and a row of keys more; ragged keys, the last of 32 missing; four parts of 64 features
+    # eight head parts: 32 MiB of partial sums, written through, and a row of keys more, for which there are four; ragged keys, the last of 32 missing; four
+    # parts of 64 features
     (1, 129, 1024, 32, 4, 128), (1, 129, 1025, 32, 4, 128), (1, 70, 95, 16, 2, 128), (2, 100, 1000, 16, 4, 64),
 ])  # fmt: skip
 def test_backward_of_split_head_groups(gpu, B, Sq, Skv, Hq, Hkv, D):
     test_backward_splits(gpu, B, Sq, Skv, Hq, Hkv, D, False)
+
+
+def test_partial_sums_beyond_the_caches(gpu):
+    """64 MiB of them, stored plainly."""
+    args, plan = _C.AttnBwdArgs(B=4, Sq=1024, Skv=1024, Hq=16, Hkv=4, Dqk=128, Dv=128, causal=1), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+    assert plan.dkdv_split == 4 and _C.lib().pith_attn_bwd_dkdv_workspace_bytes(_C.byref(args)) == 64 << 20
+    test_backward_splits(gpu, 4, 1024, 1024, 16, 4, 128, True)
 
 
 @pytest.mark.parametrize("B,Sq,Skv,H,D", [(2, 200, 300, 8, 64), (1, 130, 257, 16, 128), (3, 300, 130, 16, 192), (2, 64, 2, 8, 128), (1, 513, 513, 24, 128)])
@@ -94,10 +106,14 @@ def test_waves_without_rows(gpu, B, S, Hq, Hkv, D, causal):
     test_backward_splits(gpu, B, S, S, Hq, Hkv, D, causal)
 
 
-@pytest.mark.parametrize("B,S,H,D,causal", [
+@pytest.mark.parametrize("one_grid,B,S,H,D,causal", [
     # 3.32 and 3.34 dQ workgroups per compute unit under the mask, 383 and 384 keys; 3.09 and 3.11 without; 192 features from 256 keys on
-    (1, 640, 170, 128, True), (1, 640, 171, 128, True), (1, 383, 171, 128, True), (1, 384, 171, 128, True), (1, 513, 158, 128, False),
-    (1, 513, 159, 128, False), (1, 255, 150, 192, True), (1, 256, 150, 192, True), (1, 300, 128, 192, True),
+    (1, 1, 640, 170, 128, True), (0, 1, 640, 171, 128, True), (0, 1, 383, 171, 128, True), (1, 1, 384, 171, 128, True), (1, 1, 513, 158, 128, False),
+    (0, 1, 513, 159, 128, False), (0, 1, 255, 150, 192, True), (1, 1, 256, 150, 192, True), (1, 1, 300, 128, 192, True),
 ])  # fmt: skip
-def test_backward_pairs_at_the_lines_of_one_grid(gpu, B, S, H, D, causal):
+def test_backward_pairs_at_the_lines_of_one_grid(gpu, monkeypatch, one_grid, B, S, H, D, causal):
+    monkeypatch.setattr(hip, "DS_BUFFER_LIMIT_BYTES", 0)  # (the first two would hand dS over)
+    args, plan = _C.AttnBwdArgs(B=B, Sq=S, Skv=S, Hq=H, Hkv=H, Dqk=D, Dv=min(D, 128), causal=causal), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_plan(_C.byref(args), _C.byref(plan)))
+    assert plan.one_grid == one_grid
     test_backward_splits(gpu, B, S, S, H, H, D, causal)

@@ -1,11 +1,14 @@
 """A ring share as one launch over all of its chunks: every work split of the kernels, at row counts where a tile or a wave
 straddles the first row that sees a chunk, the end of a chunk or the diagonal, against the float64 oracle."""
 
+import ctypes
+
 import pytest
 import torch
 
 from helpers import check_bf16_result, check_lse
 from oracle import ring_oracle as R
+from pithtrain_amd import _C
 from pithtrain_amd.operators.mla import hip as H
 from pithtrain_amd.operators.ring_attention import local as L
 
@@ -91,27 +94,48 @@ def test_share_of_unequal_rows_64_features(gpu, monkeypatch):
     test_share(gpu, monkeypatch, True, 1, 1026, 36, 36, 64, 2, 0, "zigzag", False)
 
 
-# Backward of shares with more 128-row query workgroups than one grid of dK/dV and dQ takes (attn_bwd_dkdv.hip, one_grid: two
-# per compute unit at 192 features, four at 64 and 128): two launches, the dQ one with two workgroups per compute unit; and at
-# 128 features the last of the single grids. Chunk ends, half chunks and half rows fall into tiles in all of them.
-@pytest.mark.parametrize("S,Hq,Hkv,D,C,rank,layout,two_part", [
-    (130, 516, 258, 64, 3, 1, "zigzag", False), (130, 516, 516, 128, 3, 1, "zigzag", False), (258, 344, 86, 128, 2, 1, "contiguous", False),
-    (130, 260, 130, 128, 3, 1, "zigzag", False), (130, 260, 260, 192, 3, 1, "zigzag", False), (258, 172, 172, 192, 2, 1, "contiguous", True),
-    (130, 260, 260, 192, 2, 0, "zigzag", True)])  # fmt: skip
-def test_share_with_many_workgroups(gpu, monkeypatch, S, Hq, Hkv, D, C, rank, layout, two_part):
+# Backward of shares with more 128-row query workgroups than one grid of dK/dV and dQ takes (attn_bwd_dkdv.hip, one_grid: two per
+# compute unit at 192 features, four at 128, eight against more than two chunks' keys): two launches, the dQ one with two workgroups per
+# compute unit; and the last of the single grids (64 features: all of these). Chunk ends, half chunks and half rows fall into tiles in all of them. Keys in two parts
+# with 16 and 33 MiB of per-head gradients of the shared part, written through and not.
+@pytest.mark.parametrize("one_grid,S,Hq,Hkv,D,C,rank,layout,two_part", [
+    (1, 130, 516, 258, 64, 3, 1, "zigzag", False), (1, 130, 516, 516, 128, 3, 1, "zigzag", False), (0, 258, 344, 86, 128, 2, 1, "contiguous", False),
+    (1, 130, 260, 130, 128, 3, 1, "zigzag", False), (0, 130, 516, 258, 128, 2, 0, "zigzag", False), (0, 130, 516, 516, 128, 2, 1, "zigzag", False),
+    (0, 130, 1028, 514, 128, 3, 1, "zigzag", False), (0, 130, 260, 260, 192, 3, 1, "zigzag", False), (0, 258, 172, 172, 192, 2, 1, "contiguous", True),
+    (0, 130, 260, 260, 192, 2, 0, "zigzag", True), (0, 130, 516, 516, 192, 2, 1, "contiguous", True)])  # fmt: skip
+def test_share_with_many_workgroups(gpu, monkeypatch, one_grid, S, Hq, Hkv, D, C, rank, layout, two_part):
     monkeypatch.setattr(H, "DS_BUFFER_LIMIT_BYTES", 0)  # no dS hand-over: every kernel recomputes
+    steps = sorted(L.ring_schedule(rank, C, S, layout), key=lambda st: (st.kv_rank == rank, st.q_rows[0]))
+    chunks = (_C.KeyChunk * len(steps))(*(_C.KeyChunk(rows=st.kv_rows[1] - st.kv_rows[0], q_row0=st.q_rows[0]) for st in steps))
+    args, plan = _C.AttnBwdArgs(B=1, Sq=S, Skv=S, Hq=Hq, Hkv=Hkv, Dqk=D, Dv=min(D, 128)), _C.AttnBwdPlan()
+    _C.check(_C.lib().pith_attn_bwd_chunks_plan(_C.byref(args), chunks, len(steps), _C.byref(plan)))
+    assert plan.one_grid == one_grid
     test_share(gpu, monkeypatch, True, 1, S, Hq, Hkv, D, C, rank, layout, two_part)
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,rank", [(1100, 56, 2, 1), (1100, 58, 2, 1), (1100, 120, 4, 0), (1090, 58, 2, 2), (1278, 52, 2, 2)])
-def test_forward_a_little_above_whole_rounds(gpu, monkeypatch, S, Hq, Hkv, rank):
-    """On 256 compute units 128-row workgroups for just below and above two rounds (256-row ones there) and above four, against a launch per
-    ring step; either rounds P and the result to bf16, and a merge rounds once more: two steps (2^-8 each) of the largest element."""
+@pytest.mark.parametrize("full,S,Hq,Hkv,rank", [(0, 1100, 56, 2, 1), (1, 1100, 58, 2, 1), (0, 1100, 120, 4, 0), (1, 1090, 58, 2, 2), (1, 1278, 52, 2, 2), (1, 2100, 62, 2, 0), (0, 1400, 48, 2, 0)])
+def test_forward_a_little_above_whole_rounds(gpu, monkeypatch, full, S, Hq, Hkv, rank):
+    """On 256 compute units 128-row workgroups for just below and above two rounds (256-row ones there, up to 1.15 per unit and an odd number to a head; rank 2, whose rows are nearly equal, in any case) and above four,
+    against float32 and against a launch per ring step; either rounds P and the result to bf16, and a merge rounds once more: two steps (2^-8
+    each) of the largest element."""
+    steps = sorted(L.ring_schedule(rank, 3, S, "zigzag"), key=lambda st: (st.kv_rank == rank, st.q_rows[0]))
+    chunks = (_C.KeyChunk * len(steps))(*(_C.KeyChunk(rows=st.kv_rows[1] - st.kv_rows[0], q_row0=st.q_rows[0]) for st in steps))
+    split = ctypes.c_int32(-1)
+    _C.check(_C.lib().pith_attn_fwd_split(_C.byref(_C.AttnFwdArgs(B=1, Sq=S, Hq=Hq, Hkv=Hkv, Dqk=128, Dv=128)), chunks, len(steps), _C.byref(split)))
+    assert (split.value == 0) == bool(full)
     g = torch.Generator(device=gpu).manual_seed(7)
     mk = lambda h: torch.randn(1, S, h, 128, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
     q, ks, vs = mk(Hq), [mk(Hkv) for _ in range(3)], [mk(Hkv) for _ in range(3)]
     out, lse = L.ring_forward_local(q, ks, vs, 128**-0.5, rank, 3, "zigzag")
+    at = lambda j: torch.cat([torch.arange(S // 2) + S // 2 * j, torch.arange(S // 2) + S // 2 * (5 - j)])  # noqa: E731
+    hidden = (torch.cat([at(j) for j in range(3)])[None, :] > at(rank)[:, None]).to(gpu)
+    k, v = torch.cat(ks, 1)[0].float(), torch.cat(vs, 1)[0].float()
+    for h in range(0, Hq, 7):  # (heads of every group)
+        s = (q[0, :, h].float() @ k[:, h * Hkv // Hq].t().contiguous()) * 128**-0.5
+        s = s.masked_fill(hidden, float("-inf"))
+        check_bf16_result(out[0, :, h], torch.softmax(s, -1) @ v[:, h * Hkv // Hq], f"O, head {h}")
+        check_lse(lse[0, h], torch.logsumexp(s, -1) / 0.6931471805599453, f"LSE2, head {h}")
     monkeypatch.setattr(L, "FUSE_CHUNKS", False)
-    steps, lse_steps = L.ring_forward_local(q, ks, vs, 128**-0.5, rank, 3, "zigzag")
-    assert (out.float() - steps.float()).abs().max() <= 2**-7 * steps.float().abs().max()
+    stepwise, lse_steps = L.ring_forward_local(q, ks, vs, 128**-0.5, rank, 3, "zigzag")
+    assert (out.float() - stepwise.float()).abs().max() <= 2**-7 * stepwise.float().abs().max()
     assert (lse - lse_steps).abs().max() < 1e-3
