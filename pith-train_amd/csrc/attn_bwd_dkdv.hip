@@ -244,8 +244,10 @@ void launch_dkdv(BwdParams p, const pith_attn_bwd_args* a, int rows, bool with_d
 //                 2.2: 1 x 4480 x 16 628 -> 520, 1 x 2304 x 32/4 383 -> 289
 //   d192 causal   W 1.1: 1 x 4608 x 8 246 -> 198; 1.5: 1 x 3072 x 16 193 -> 186; 1.7: 1 x 3456 x 16
 //                 227 -> 227; 2: 1 x 2048 x 32 171 -> 175; 2.2: 1 x 2560 x 28 233 -> 242
-// and with the forward, since the head split halves (half_as_many):
-//   d128 causal   W 1.6: 13 x 500 x 8/2 86.5 -> 80.7; 2: 2 x 1000 x 32/4 128 -> 125, 4 x 500 x 32/4 96 -> 98; 2.25-2.8: 3 x 768 x 32/4 116.4 ->
+// and with the forward, since the head split halves (half_as_many). These calls recompute; from two thirds of a device of query rows on (about W 2.8) most hand dS over and have
+// two launches in any case, so that the upper lines hold for those which do not: up to 256 rows, unmasked 513 to 639, more than 16384 of few heads, groups of an odd number of
+// heads, fp32 results, no room for the buffer.
+//   d128 causal   W 1.6: 13 x 500 x 8/2 86.5 -> 80.7; 2: 2 x 1000 x 32/4 128 -> 125, 4 x 500 x 32/4 97.6 -> 96.3, 4 x 512 98.4 -> 97.5, 2 x 900 117.2 -> 111.5; 2.25-2.8: 3 x 768 x 32/4 116.4 ->
 //                 107.4, 3 x 700 108.4 -> 100.3, 6 x 384 89 -> 86, 5 x 450 101 -> 98, 1 x 2700 322 -> 309, 1 x 1500 x 60/4 546 -> 505, 3 x 1000 x 30/2 386 ->
 //                 352, 3 x 1900 x 16 234 -> 231; 2.9-3.3: 1 x 6000 x 16 652 -> 629, 1 x 3000 x 32/4 369 -> 361, 1 x 3300 423 -> 410, 1 x 13000 x 8/2 1461
 //                 -> 1429, 1 x 3100 x 34/2 1209 -> 1121; 3.5: 1 x 3500 x 32/4 456 -> 459, 7 x 900 x 16 equal; 5: 20 x 160 x 32/4 99 -> 107

@@ -202,6 +202,8 @@ def _set_ds(args, ds: torch.Tensor, like: torch.Tensor) -> None:
 # Sq*Skv*Hq*B*2 bytes while the pair's two kernels run, about half under the causal mask: a layer of 4096 rows, 32/4 heads of 128
 # takes 0.55 GB, of 16 heads of 192/128 0.28 GB. A share of 192 features that goes out as one dK/dV and one dQ launch holds the images of all
 # its chunks at once: 4096 rows, 16 heads, four ranks, zigzag 1.08 GB.
+# Calls whose 512-row workgroups are between two thirds of a device and a full one hold such a buffer, too (up to 16384 rows):
+# 3000 rows, 32/4 heads 0.30 GB, 15000 rows, 8/2 heads without a mask 3.6 GB.
 # Policy: the buffer never exceeds DS_BUFFER_LIMIT_BYTES nor DS_BUFFER_FREE_FRACTION of the device memory that is
 # free right now; a chunk pair that needs more is processed one group of kv heads (with their query heads) after
 # the other through one buffer of the bounded size; when not even one kv head fits, or the allocation fails, the
