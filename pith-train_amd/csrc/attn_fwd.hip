@@ -132,22 +132,24 @@ bool above_a_round(const pith_attn_fwd_args* a, int64_t wgs, int64_t cus, Split*
 //                    12.2 / 12.6; but 256 rows W 3.3 x 210 10.7 / 9.4, 4 x 256 10.2 / 9.7, more than at once (4.2-4.5) 192 x 360 11.9 / 10.4, 370 x 192 15.4 /
 //                    12.8, 768 x 96 17.6 / 16.7, and an odd number of heads, whose tiles wander over the XCDs, 448 x 135 14.2 / 13.4, 768 x 81 18.3 / 16.5
 //     960 to 1535    W 4 1000 x 64 17.1 / 19.4, 1024 x 64 17.1 / 19.3, 4.25 1088 x 64 18.6 / 20.3, an odd number of heads 4.3 1024 x 69 22.9 / 21.2, 1200 x 58 21.9 / 22.6, 4.5 1400 x 52 23.4 / 25.7
-//     1536 on        W 4.5 2 x 2048 x 18 31.9 / 35.9, 5 1 x 2048 x 40 35.2 / 36.2. With the backward behind it TEAMS is ahead from 2561 keys on while W is 3.25 at
+//     1536 on        W 4.5 2 x 2048 x 18 31.9 / 35.9, 5 1 x 2048 x 40 35.2 / 36.2, but in several chunks with less unequal rows 2048 x 40/10 rank 2 118 / 111 (and 4.5 2 x 756 x 48/12, two
+//                    ranks, rank 1 28.9 / 26.2; rank 0 2 x 582 x 64/16 56 / 71). With the backward behind it TEAMS is ahead from 2561 keys on while W is 3.25 at
 //                    most: 4 x 2855 x 4 114.9 / 110.8, 2914 x 16 117.9 / 114.8, 2688 x 16 109.0 / 105.6, 5120 x 10 193.7 / 189.6, 6144 x 8 220.7 / 216.1, not 2560 x 20
 //                    106.2 / 106.8, nor several chunks (1152 x 32/8, four ranks, rank 0 178 / 196), 4096 x 16 (W 4) equal, its forward alone 49.4 / 53.3
 //   64 features without a mask, up to two per unit: to 384 keys from W 1.7 on (320 keys 1.35 9.1 / 8.6, 1.5 9.2 / 8.7, 1.75 9.6 / 10.2; 256 keys equal at best), 384 keys 44 to
 //                    84 heads 8.7-9.6 / 9.0-9.9, but 75 heads 11.0 / 9.8; 1024 x 32 16.2 / 17.0; TEAMS above 2048 keys (2304 x 14 30.4 / 30.1, 6144 x 5 69.8 / 67.0)
 //   128 and 192 features, rows unequal, up to two per unit: not for 128 rows, which one DUO workgroup holds (8.6 / 7.9, 9.2 / 8.9), nor up to 192 at W 1.05 (8.7 / 8.0
 //                    and 9.9 / 9.2; 1.2: 8.1 / 8.4)
-bool small_workgroups(const pith_attn_fwd_args* a, int64_t wgs64, int64_t cus, bool unequal) {
+bool small_workgroups(const pith_attn_fwd_args* a, int64_t wgs64, int64_t cus, int mean) {
   const int64_t keys = a->Skv, heads = a->Hq * a->B;
+  const bool unequal = mean <= 70, half = mean <= 52;  // half: one chunk, and rank 0 of a zigzag share
   const auto at_most = [&](int64_t n, int64_t d) { return d * wgs64 <= n * cus; };  // W <= n / d
   if (a->Dqk != 64) return unequal && at_most(2, 1) && keys >= 129 && keys < 1536 && (keys > 192 || !at_most(6, 5));
   if (!unequal) return at_most(2, 1) && keys >= 192 && keys <= 2048 && (keys >= 448 || (keys >= 384 ? heads % 4 == 0 : !at_most(17, 10)));
   if (at_most(2, 1)) return keys >= 128 && keys < 1536;
   if (keys < 128 || keys > 6144) return false;
-  if (keys >= 1536) return at_most(5, 1) && (keys <= 2560 || keys != a->Sq || !at_most(13, 4));
-  if (keys >= 960) return keys >= 1200 || heads % 2 == 0 ? at_most(9, 2) : at_most(4, 1);
+  if (keys >= 1536) return (half ? at_most(5, 1) : at_most(9, 2)) && (keys <= 2560 || keys != a->Sq || !at_most(13, 4));
+  if (keys >= 960) return half && (keys >= 1200 || heads % 2 == 0) ? at_most(9, 2) : at_most(4, 1);
   const bool pads = (a->Sq + 63) / 64 % 2 != 0;  // half of a 128-row workgroup
   return heads % 2 == 0 && (keys >= 384 || pads) ? at_most(4, 1) : at_most(3, 1);
 }
@@ -171,10 +173,11 @@ Split pick_split(const pith_attn_fwd_args* a, int mean) {
     const bool second_round = (one_chunk || longer <= cus) && (a->Sq >= 1536 || !(one_chunk || (d64 && both_long)));
     if (a->Skv >= from && (!half_more || second_round)) return Split::kQuarter;
   }
-  if (small_workgroups(a, wgs64, cus, unequal)) return Split::kSmall;
+  if (small_workgroups(a, wgs64, cus, mean)) return Split::kSmall;
   const Split key_split = d64 ? Split::kTeams : Split::kHalf;
   if (wgs <= cus && a->Skv > (d64 ? 1024 : a->Dqk == 192 ? 383 : 256)) return key_split;  // (128 features without a mask, 256 keys: 4 x 27 heads 11.7 / 12.4)
-  if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 2 * wgs <= 3 * cus ? 1023 : 1535)) return key_split;
+  // (mean 1/2: one chunk, and rank 0 of a zigzag share; short rows that are less unequal, DUO / HALF: rank 2 of four, 2 x 396 x 40/8 of 128 36.7 / 42.9)
+  if (unequal && wgs <= 2 * cus && a->Skv > (d64 ? 2048 : 2 * wgs <= 3 * cus && mean <= 52 ? 1023 : 1535)) return key_split;
   // FULL under the mask also for shorter rows of many heads whose K and V outgrow the last-level cache (half the streams in
   // flight; 2048 x 256 heads 355 -> 314 us, 2048 x 224 293 -> 276, 1024 x 512 221 -> 207, 2048 x 192 (192 MiB) 231 -> 235; not
   // for rows of a few workgroups: 8 x 512 x 128 155 -> 167)

@@ -59,6 +59,14 @@ def test_few_rows():
     assert [_split(4, s, 20, 20, 128, 0) for s in (256, 257)] == [DUO, HALF]
 
 
+def test_short_rows_against_several_chunks():
+    """Key halves from 1024 keys on for one chunk and in rank 0, from 1536 in others, as measured."""
+    assert [_split(1, s, 44, 44, 192) for s in (1023, 1024)] == [DUO, HALF] and _share_split(2, 640, 32, 32, 192, 2, 0, "zigzag") == HALF
+    assert _share_split(1, 2048, 40, 10, 64, 4, 2, "zigzag") == DUO and _split(1, 2048, 40, 10, 64) == SMALL
+    assert _share_split(2, 582, 64, 16, 64, 4, 0, "zigzag") == SMALL and _share_split(2, 756, 48, 12, 64, 2, 1, "zigzag") == DUO
+    assert [_share_split(2, s, 40, 8, 128, 4, 2, "zigzag") for s in (396, 510, 512)] == [DUO, DUO, HALF]
+
+
 def test_shares_of_64_features_of_long_streams():
     """Nearly equal rows, two teams above 2048 keys."""
     assert _share_split(2, 2240, 4, 4, 64, 4, 3, "contiguous") == TEAMS and _share_split(1, 500, 40, 40, 64, 4, 3, "contiguous") == SMALL
